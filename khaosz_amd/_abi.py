@@ -90,6 +90,7 @@ LAB_SYMBOLS = {
 
 _lib = None
 _lab = None
+_host = None
 
 
 def load() -> ctypes.CDLL:
@@ -109,6 +110,20 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def host():
+    """The native host path (csrc/host.cpp), bound to the library ``load()`` hands out; raises if it has not been built."""
+    global _host
+    if _host is None:
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError("khaosz_amd/_host.so is missing or does not load: build it with `python -m khaosz_amd.build`. "
+                               "There is no fallback path.") from e
+        module.bind(load()._handle)
+        _host = module
+    return _host
 
 
 def load_lab() -> ctypes.CDLL:
@@ -134,14 +149,16 @@ class lab_library:
 
     def __enter__(self):
         global _lib
-        self._saved = _lib
+        self._saved = load()
         _lib = load_lab()
+        host().bind(_lib._handle)
         return _lib
 
     def __exit__(self, *exc):
         global _lib
         _lib.aq_lab_set_gemm_tile(0)
         _lib = self._saved
+        host().bind(_lib._handle)
         return False
 
 

@@ -20,7 +20,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
 
-from . import ops
+from . import _abi, ops
 from .linear import Linear, QuantLinear
 
 
@@ -432,6 +432,11 @@ class DecoderBlock(nn.Module):
 
     def forward(self, x: Tensor, rotary_emb: Tensor, attention_mask: Optional[Tensor] = None,
                 cache=None) -> Tensor:
+        if self._norm_quant and self._residual_adds and attention_mask is None and cache is not None:
+            # everything fused, over a paged cache: the same launches, queued by native code in one call
+            y = (_host or _native())(self, x, rotary_emb, cache)
+            if y is not None:
+                return y
         if self._residual_adds:  # each branch's last projection adds the stream it is given
             kw = lambda r: {"residual": r}
             add = lambda y, r: y
@@ -445,6 +450,26 @@ class DecoderBlock(nn.Module):
             return add(self.mlp(x, norm=(n2.weight, n2.norm_eps), **kw(x)), x)
         x = add(self.attention(self.input_norm(x), rotary_emb, attention_mask, cache, **kw(x)), x)
         return add(self.mlp(self.post_attention_norm(x), **kw(x)), x)
+
+
+# The operators a fused block's step consists of, as defined.  While a program has one of them replaced (to count or
+# trace calls), blocks go operator by operator, through its replacement.
+_OPERATORS = {name: getattr(ops, name) for name in (
+    "quant_rowwise_i8", "rmsnorm_quant_rowwise_i8", "swiglu_quant_rowwise_i8", "linear_w8a8", "gemv_w8a8_decode", "gemv_swiglu_ok",
+    "gemv_w8a8_decode_swiglu", "gemv_w8a8_codes", "rope_kv_write", "attn_gemv_fusable", "rope_paged_attn_decode", "gemv_w8a8_attn",
+    "prefill_attn_causal", "prefill_attn_paged")}
+_host = None  # the native block step once it is loaded
+
+
+def _native():
+    global _host
+    if _host is None:
+        h, m = _abi.host(), torch.nn.modules.module
+        h.set_block_types(QuantLinear, RMSNorm, GQA, MLP, PagedKV,
+                          (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
+                           m._global_backward_pre_hooks), ops.__dict__, _OPERATORS)
+        _host = h.block_forward
+    return _host
 
 
 def decode_mask(batch: int, total_len: int, device, dtype) -> Tensor:

@@ -1,11 +1,13 @@
 """Compile the HIP sources in csrc/ for gfx950 into
 
   khaosz_amd/lib/libastrai_q.so      the product: the C ABI declared in include/astrai_q.h, nothing else;
+  khaosz_amd/_host.so                the native host path (csrc/host.cpp: tensors in, launches out), a Python extension
+                                     against torch's C++ API that calls the C ABI above;
   khaosz_amd/lib/libastrai_q_lab.so  the same objects plus the measurement probes and the tile-forcing hook
                                      of csrc/aq_lab.h (the GEMM and GEMV sources rebuilt with -DAQ_LAB), for the
                                      benchmark's ceilings and for tests that pin a tile shape.
 
-hipcc cross-compiles without a GPU.  Both depend on the HIP runtime only (no torch, no Python).
+hipcc cross-compiles without a GPU.  The two libraries depend on the HIP runtime only (no torch, no Python).
 
     python -m khaosz_amd.build [--if-stale] [--stall-counters]
 
@@ -16,6 +18,7 @@ reads per K step, so the default lab build leaves them out; the product library 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -23,6 +26,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "lib", "obj")
 LIB = os.path.join(HERE, "lib", "libastrai_q.so")
 LAB_LIB = os.path.join(HERE, "lib", "libastrai_q_lab.so")
+HOST_EXT = os.path.join(HERE, "_host.so")
 SOURCES = ["abi.hip", "quant.hip", "gemm_mfma.hip", "gemv.hip", "attn_decode.hip", "attn_prefill.hip"]
 # (source, object, extra flags) of the lab library's own objects; the other product objects are shared
 LAB_SOURCES = [("gemm_mfma.hip", "gemm_mfma_lab.o", ["-DAQ_LAB"]), ("gemv.hip", "gemv_lab.o", ["-DAQ_LAB"]),
@@ -44,6 +48,24 @@ def _stale(out, deps):
         return True
     t = os.path.getmtime(out)
     return any(os.path.getmtime(d) > t for d in deps)
+
+
+def _build_host(force: bool) -> None:
+    """csrc/host.cpp holds no device code: the host compiler, torch's headers and libraries."""
+    import torch
+
+    src = os.path.join(CSRC, "host.cpp")
+    if not (force or _stale(HOST_EXT, [src, os.path.join(HERE, "..", "include", "astrai_q.h")])):
+        return
+    t = os.path.dirname(torch.__file__)
+    inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           *(x for d in inc for x in ("-isystem", d)), src, "-o", HOST_EXT, "-L" + os.path.join(t, "lib"), "-ltorch_python", "-ltorch_cpu",
+           "-ltorch_hip", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"the host compiler failed for host.cpp:\n{r.stderr}")
 
 
 def build(force: bool = True, verbose: bool = False, stall_counters: bool = False) -> str:
@@ -68,7 +90,9 @@ def build(force: bool = True, verbose: bool = False, stall_counters: bool = Fals
         return o
 
     with ThreadPoolExecutor(max_workers=4) as ex:
+        host = ex.submit(_build_host, force)
         all_objs = list(ex.map(compile_one, SOURCES + lab_sources))
+        host.result()
     objs, lab_only = all_objs[:len(SOURCES)], all_objs[len(SOURCES):]
     lab_objs = [o for o in objs if not o.endswith(("gemm_mfma.o", "gemv.o"))] + lab_only
     for lib, members in ((LIB, objs), (LAB_LIB, lab_objs)):

@@ -54,21 +54,20 @@ class Linear(nn.Module):
 
 
 class _PerStream:
-    """Scratch tensors a module keeps per (device, stream): the decode workspace, the one-launch quantiser's state.
+    """Tensors a module keeps per (device, stream): the one-launch quantiser's state.
     Bounded: the most recently used ``keep`` streams stay, older entries are dropped (a module called from ever
-    new side or capture streams would otherwise grow by a workspace per stream for the life of the model).
-    Keys are raw stream handles, which the runtime may hand out again for a new stream: harmless for a stateless
-    workspace, and for the quantiser's state too, because what it needs is only that calls sharing it do not
-    overlap in time -- which launches on one stream never do -- and every call leaves it in the state the next
-    one accepts."""
+    new side or capture streams would otherwise grow by a state per stream for the life of the model).
+    Keys are raw stream handles, which the runtime may hand out again for a new stream: harmless for the quantiser's
+    state, because what it needs is only that calls sharing it do not overlap in time -- which launches on one stream
+    never do -- and every call leaves it in the state the next one accepts."""
 
     def __init__(self, keep: int = 8):
         self._keep, self._items = keep, {}
 
-    def get(self, device, make, fits=lambda t: True):
-        key = (device, torch.cuda.current_stream(device).cuda_stream)
+    def get(self, device, make):
+        key = (device, ops.current_stream(device))
         t = self._items.pop(key, None)
-        if t is None or not fits(t):
+        if t is None:
             t = make()
         self._items[key] = t  # most recently used last
         while len(self._items) > self._keep:
@@ -82,6 +81,12 @@ class _PerStream:
 def _no_grad_guard(x: Tensor) -> None:
     if torch.is_grad_enabled() and x.requires_grad:
         raise RuntimeError("the quantized Linear is forward-only; call it under torch.no_grad()/inference_mode()")
+
+
+def _bias_of(m: nn.Module) -> Optional[Tensor]:
+    """``m.bias``: a registered parameter, or the plain attribute None."""
+    b = m._parameters.get("bias")
+    return b if b is not None else m.__dict__.get("bias")
 
 
 class _SharedInput:
@@ -139,9 +144,6 @@ class QuantLinear(Linear):
         self.register_buffer("qweight", torch.zeros((out_dim, in_dim), dtype=torch.int8, device=device))
         self.register_buffer("w_scale", torch.ones((out_dim,), dtype=torch.float32, device=device))
         self.bias = nn.Parameter(torch.zeros(out_dim, device=device), requires_grad=False) if bias else None
-        # decode workspaces (activation codes between the row quantiser and the GEMV), one per (device, stream):
-        # the same module called from two streams or threads must not share one
-        self._workspaces = _PerStream()
         self._shared: Optional[Tuple[_SharedInput, int]] = None  # set by share_inputs(): (group, index in it)
 
     # -- construction -----------------------------------------------------
@@ -233,27 +235,24 @@ class QuantLinear(Linear):
         ``norm = (gain [in_dim], eps)``: returns ``linear(rms_norm(x) * gain)`` with the norm fused
         into the activation quantisation (the normalised activations are never written; see
         ``ops.rmsnorm_quant_rowwise_i8``)."""
-        _no_grad_guard(x)
+        if x.requires_grad:
+            _no_grad_guard(x)
         if self._shared is not None and residual is None and norm is None:
             return self._shared[0].output(x, self._shared[1])
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
-        M = x2.shape[0]
-        if x2.shape[1] != self.qweight.shape[1]:
-            raise ValueError(f"expected last dim {self.qweight.shape[1]}, got {x2.shape[1]}")
-        if x2.dtype not in (torch.float32, torch.bfloat16):
-            raise ValueError(f"activation dtype {x2.dtype} is not supported (float32 or bfloat16)")
-        if M <= self.DECODE_MAX_ROWS:
-            ops._need_gpu(x, self.qweight)
-            need = 16 * self.qweight.shape[1] + 512
-            ws = self._workspaces.get(x.device, lambda: torch.empty((need,), dtype=torch.uint8, device=x.device),
-                                      lambda t: t.numel() >= need)
-            y = ops.gemv_w8a8_decode(x2, self.qweight, self.w_scale, self.bias, out_dtype=x.dtype, workspace=ws,
-                                     residual=residual, norm=norm)
+        # straight from where nn.Module keeps them: its __getattr__ costs half a microsecond a name
+        wq, sw, bias = self._buffers["qweight"], self._buffers["w_scale"], _bias_of(self)
+        n, k = wq.shape
+        if x.size(-1) != k:
+            raise ValueError(f"expected last dim {k}, got {x.size(-1)}")
+        if x.dtype is not torch.bfloat16 and x.dtype is not torch.float32:
+            raise ValueError(f"activation dtype {x.dtype} is not supported (float32 or bfloat16)")
+        x2 = x if x.dim() == 2 else x.reshape(-1, k)
+        if x2.size(0) <= self.DECODE_MAX_ROWS:
+            y = ops.gemv_w8a8_decode(x2, wq, sw, bias, out_dtype=x.dtype, residual=residual, norm=norm)
         else:
             xq, sx = ops.quant_rowwise_i8(x2) if norm is None else ops.rmsnorm_quant_rowwise_i8(x2, norm[0], norm[1])
-            y = ops.linear_w8a8(xq, sx, self.qweight, self.w_scale, self.bias, out_dtype=x.dtype, residual=residual)
-        return y.reshape(*lead, self.qweight.shape[0])
+            y = ops.linear_w8a8(xq, sx, wq, sw, bias, out_dtype=x.dtype, residual=residual)
+        return y if x2 is x else y.view(x.shape[:-1] + (n,))
 
     def forward_codes(self, xq: Tensor, sx: Tensor, out_dtype: torch.dtype,
                       residual: Optional[Tensor] = None) -> Tensor:
@@ -286,7 +285,6 @@ class Fp8Linear(Linear):
         self.register_buffer("qweight", torch.zeros((out_dim, in_dim), dtype=torch.uint8, device=device))
         self.register_buffer("w_scale", torch.ones((1,), dtype=torch.float32, device=device))
         self.bias = nn.Parameter(torch.zeros(out_dim, device=device), requires_grad=False) if bias else None
-        self._workspaces = _PerStream()    # decode workspaces, one per (device, stream), as in QuantLinear
         self._quant_states = _PerStream()  # the one-launch activation quantiser's state, one per (device, stream)
 
     DECODE_MAX_ROWS = 16
@@ -323,24 +321,23 @@ class Fp8Linear(Linear):
 
     def forward(self, x: Tensor, residual: Optional[Tensor] = None) -> Tensor:
         """``residual`` (shape and dtype of the output): added in the kernel's epilogue, the bits of a separate add."""
-        _no_grad_guard(x)
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
-        if x2.shape[1] != self.qweight.shape[1]:
-            raise ValueError(f"expected last dim {self.qweight.shape[1]}, got {x2.shape[1]}")
-        if x2.shape[0] <= self.DECODE_MAX_ROWS:  # decode step: the weight-streaming GEMV
-            ops._need_gpu(x, self.qweight)
-            need = 16 * self.qweight.shape[1] + 2048
-            ws = self._workspaces.get(x.device, lambda: torch.empty((need,), dtype=torch.uint8, device=x.device),
-                                      lambda t: t.numel() >= need)
-            y = ops.gemv_fp8_decode(x2, self.qweight, self.w_scale, self.bias, out_dtype=x.dtype, workspace=ws,
-                                    residual=residual)
+        if x.requires_grad:
+            _no_grad_guard(x)
+        wq, sw, bias = self._buffers["qweight"], self._buffers["w_scale"], _bias_of(self)
+        n, k = wq.shape
+        if x.size(-1) != k:
+            raise ValueError(f"expected last dim {k}, got {x.size(-1)}")
+        x2 = x if x.dim() == 2 else x.reshape(-1, k)
+        if x2.size(0) <= self.DECODE_MAX_ROWS:  # decode step: the weight-streaming GEMV
+            y = ops.gemv_fp8_decode(x2, wq, sw, bias, out_dtype=x.dtype, residual=residual)
         else:
-            ops._need_gpu(x, self.qweight)
-            state = self._quant_states.get(x.device, lambda: ops.fp8_onepass_state(x.device))
-            xq, sx = ops.quant_tensor_fp8(x2, state=state)  # one launch for large inputs
-            y = ops.linear_fp8(xq, sx, self.qweight, self.w_scale, self.bias, out_dtype=x.dtype, residual=residual)
-        return y.reshape(*lead, self.qweight.shape[0])
+            state = None
+            if x2.numel() * x2.element_size() >= ops.FP8_ONEPASS_MIN_BYTES:  # quantised in one launch
+                ops._need_gpu(x, wq)
+                state = self._quant_states.get(x.device, lambda: ops.fp8_onepass_state(x.device))
+            xq, sx = ops.quant_tensor_fp8(x2, state=state)
+            y = ops.linear_fp8(xq, sx, wq, sw, bias, out_dtype=x.dtype, residual=residual)
+        return y if x2 is x else y.view(x.shape[:-1] + (n,))
 
 
 # Child names quantized by default: the projections of GQA (attention.py:57-67, `gate` is its optional output

@@ -14,6 +14,18 @@ import torch
 
 from . import _abi
 
+_host = None  # the native host path once it is loaded
+
+
+def _native():
+    """The native host path (csrc/host.cpp).  Its functions serve the plain case -- contiguous tensors of the right
+    types on the current device -- and return None for any other, which the general code below then takes."""
+    global _host
+    if _host is None:
+        _host = _abi.host()
+    return _host
+
+
 _DT = {torch.float32: _abi.AQ_F32, torch.bfloat16: _abi.AQ_BF16}
 
 
@@ -21,11 +33,15 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _cur_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
-def _stream(t: torch.Tensor) -> int:
-    """torch's current HIP stream on the tensor's device, as the raw handle the C ABI takes."""
+def current_stream(device: torch.device) -> int:
+    """torch's current HIP stream on ``device``, as the raw handle the C ABI takes."""
     if _raw_stream is not None:
-        return _raw_stream(t.device.index if t.device.index is not None else torch.cuda.current_device())
-    return torch.cuda.current_stream(t.device).cuda_stream
+        return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+def _stream(t: torch.Tensor) -> int:
+    return current_stream(t.device)
 
 
 class _OnDevice:
@@ -85,6 +101,9 @@ def _check_k(K: int) -> None:
 
 def quant_rowwise_i8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """Symmetric absmax int8 per row of ``x [..., K]`` -> (codes int8 [M, K], scale f32 [M])."""
+    r = (_host or _native()).quant_rowwise_i8(x)
+    if r is not None:
+        return r
     _need_gpu(x)
     x2 = _rows(x, "quant_rowwise_i8")
     M, K = x2.shape
@@ -107,6 +126,9 @@ SWIGLU_QUANT_MAX_F = {torch.bfloat16: 8192, torch.float32: 4096}
 def rmsnorm_quant_rowwise_i8(x: torch.Tensor, gamma: torch.Tensor, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """RMSNorm (gain ``gamma``, same dtype as ``x``) fused with the per-token quantisation of its
     output: ``[..., K]`` -> (codes int8 ``[M, K]``, scales float32 ``[M]``)."""
+    r = (_host or _native()).rmsnorm_quant_rowwise_i8(x, gamma, eps)
+    if r is not None:
+        return r
     _need_gpu(x, gamma)
     x2 = _rows(x, "x")
     M, K = x2.shape
@@ -128,6 +150,9 @@ def rmsnorm_quant_rowwise_i8(x: torch.Tensor, gamma: torch.Tensor, eps: float) -
 def swiglu_quant_rowwise_i8(ug: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """``ug [..., 2F] = [up | gate]`` -> codes and scales of ``up * silu(gate)`` per row
     (int8 ``[M, F]``, float32 ``[M]``), without writing the product."""
+    r = (_host or _native()).swiglu_quant_rowwise_i8(ug)
+    if r is not None:
+        return r
     _need_gpu(ug)
     u2 = _rows(ug, "ug")
     M, F2 = u2.shape
@@ -162,6 +187,12 @@ def quant_tensor_fp8(x: torch.Tensor, state: Optional[torch.Tensor] = None,
     """Per-tensor OCP e4m3fn -> (codes uint8 with x's shape, scale f32 [1]).
     ``state`` (from ``fp8_onepass_state``): allows the one-launch form, which reads x from HBM once instead of
     twice -- same codes and scale; taken for tensors of ``FP8_ONEPASS_MIN_BYTES`` and more, or as ``onepass`` says."""
+    if onepass is None:
+        onepass = state is not None and x.numel() * x.element_size() >= FP8_ONEPASS_MIN_BYTES
+    if state is not None or not onepass:
+        r = (_host or _native()).quant_tensor_fp8(x, state if onepass else None)
+        if r is not None:
+            return r
     _need_gpu(x)
     xc = x.contiguous()
     n = xc.numel()
@@ -169,8 +200,6 @@ def quant_tensor_fp8(x: torch.Tensor, state: Optional[torch.Tensor] = None,
         raise ValueError(f"numel must be a multiple of 16, got {n}")
     q = torch.empty(xc.shape, dtype=torch.uint8, device=x.device)
     s = torch.empty((1,), dtype=torch.float32, device=x.device)
-    if onepass is None:
-        onepass = state is not None and n * xc.element_size() >= FP8_ONEPASS_MIN_BYTES
     if onepass:
         if state is None:
             raise ValueError("the one-launch form needs the state tensor of fp8_onepass_state()")
@@ -234,6 +263,9 @@ def _residual_arg(residual, M, N, out_dtype, dev):
 
 def linear_w8a8(xq, sx, wq, sw, bias=None, out_dtype=torch.bfloat16, residual=None) -> torch.Tensor:
     """MFMA GEMM with the fused epilogue y = (acc * sx[m]) * sw[n] (+ bias[n]) (+ residual[m, n])."""
+    y = (_host or _native()).linear_w8a8(xq, sx, wq, sw, bias, out_dtype, residual)
+    if y is not None:
+        return y
     _need_gpu(xq, sx, wq, sw, bias, residual)
     if xq.dtype != torch.int8 or wq.dtype != torch.int8:
         raise ValueError("linear_w8a8 takes int8 codes")
@@ -267,6 +299,11 @@ def gemv_w8a8_decode(x, wq, sw, bias=None, out_dtype=None, workspace: Optional[t
     """Decode path for at most 16 rows of ``x [M, K]``: fused per-token quantise + int8 GEMV + epilogue.
     ``norm = (gamma [K], eps)``: RMS-normalise the rows first (the codes ``rmsnorm_quant_rowwise_i8``
     gives), in the same launch for up to 8 bfloat16 rows of at most 2048 elements."""
+    if workspace is None:
+        gamma, eps = norm if norm is not None else (None, 0.0)
+        y = (_host or _native()).gemv_w8a8_decode(x, wq, sw, bias, out_dtype, residual, gamma, eps)
+        if y is not None:
+            return y
     _need_gpu(x, wq, sw, bias, workspace, residual, norm[0] if norm is not None else None)
     x2 = _rows(x, "gemv_w8a8_decode")
     M, K = x2.shape
@@ -366,6 +403,9 @@ def gemv_w8a8_decode_swiglu(x, wq, sw, bias=None, out_dtype=None, norm=None) -> 
 
 def gemv_w8a8_codes(xq, sx, wq, sw, bias=None, out_dtype=torch.bfloat16, residual=None) -> torch.Tensor:
     """The decode GEMV on activation codes the caller already holds (at most 16 rows)."""
+    y = (_host or _native()).gemv_w8a8_codes(xq, sx, wq, sw, bias, out_dtype, residual)
+    if y is not None:
+        return y
     _need_gpu(xq, sx, wq, sw, bias, residual)
     if xq.dtype != torch.int8 or wq.dtype != torch.int8:
         raise ValueError("gemv_w8a8_codes takes int8 codes")
@@ -726,6 +766,9 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
 
 def linear_fp8(xq, sx, wq, sw, bias=None, out_dtype=torch.bfloat16, residual=None) -> torch.Tensor:
     """FP8 e4m3fn GEMM with fp32 accumulation: y = (acc * sx[0]) * sw[0] (+ bias), cast, (+ residual)."""
+    y = (_host or _native()).linear_fp8(xq, sx, wq, sw, bias, out_dtype, residual)
+    if y is not None:
+        return y
     _need_gpu(xq, sx, wq, sw, bias, residual)
     if xq.dtype != torch.uint8 or wq.dtype != torch.uint8:
         raise ValueError("linear_fp8 takes e4m3fn codes as uint8")
@@ -788,6 +831,10 @@ def gemv_fp8_decode(x, wq, sw, bias=None, out_dtype=None, workspace: Optional[to
                     residual=None) -> torch.Tensor:
     """FP8 decode path for at most 16 rows of ``x [M, K]``: per-tensor e4m3 cast + GEMV + epilogue, one launch for
     bfloat16 rows of at most 2048 elements."""
+    if workspace is None:
+        y = (_host or _native()).gemv_fp8_decode(x, wq, sw, bias, out_dtype, residual)
+        if y is not None:
+            return y
     _need_gpu(x, wq, sw, bias, workspace, residual)
     x2 = _rows(x, "gemv_fp8_decode")
     M, K = x2.shape

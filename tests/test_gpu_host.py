@@ -1,0 +1,98 @@
+"""The native host path (csrc/host.cpp): a fused block queued in one call gives the bits of the step-by-step path, keeps out of
+the way of hooks and replaced operators, and operators fed with what the native functions do not take still answer."""
+import pytest
+import torch
+
+from khaosz_amd import QuantLinear, fuse_shared_inputs, ops, quantize_model
+from khaosz_amd.block import DecoderBlock, PagedKV, rotary_table
+
+pytestmark = pytest.mark.gpu
+DEV, DT = "cuda:0", torch.bfloat16
+
+
+def _block(hidden=512, heads=8, kv=2, ffn=1408, **kw):
+    torch.manual_seed(3)
+    b = DecoderBlock(hidden, heads, ffn, kv, **kw)
+    b.reset_parameters()
+    b = b.to(DEV).to(DT)
+    quantize_model(b)
+    fuse_shared_inputs(b, norms=True, decode_attention=True, residuals=True)
+    return b
+
+
+def _case(b, B, S, cached, kv=2, d=64, page=32, unmapped=False):
+    P = (cached + S + page - 1) // page
+    table = torch.randperm(B * P, device=DEV).view(B, P)
+    if unmapped:
+        table[0, 0] = -1
+    cache = PagedKV(B * P, page, kv, d, DEV, DT)
+    cache.k_layers.normal_()
+    cache.v_layers.normal_()
+    fr = rotary_table(d, 4096, device=DEV)[cached:cached + S].unsqueeze(0).expand(B, -1, -1)
+    return torch.randn(B, S, kv * 4 * d, device=DEV).to(DT), fr, cache, table
+
+
+@pytest.mark.parametrize("qk_norm", [False, True])
+@pytest.mark.parametrize("B,S,cached,unmapped", [
+    (1, 1, 0, False), (4, 1, 299, False), (8, 1, 1100, False), (16, 1, 40, False), (17, 1, 70, False),  # decode rows
+    (1, 2, 0, False), (3, 5, 0, False), (2, 45, 0, False), (2, 33, 51, False), (1, 3, 9, False), (2, 20, 0, True)])
+def test_block_in_one_call_is_the_step_by_step_path(monkeypatch, qk_norm, B, S, cached, unmapped):
+    b = _block(use_qk_norm=qk_norm)
+    x, fr, cache, table = _case(b, B, S, cached, unmapped=unmapped)
+    k0, v0 = cache.k_layers.clone(), cache.v_layers.clone()
+    cache.bind(table, cached + S)
+    lens = (cached + 1 - torch.arange(B, device=DEV).clamp(max=cached)) if S == 1 else None
+    got = []
+    with torch.inference_mode():
+        for stepwise in (False, True):
+            cache.k_layers.copy_(k0)
+            cache.v_layers.copy_(v0)
+            cache.seq_lens = lens
+            if stepwise:  # a replaced operator: every call goes through it
+                calls = []
+                real = ops.rmsnorm_quant_rowwise_i8, ops.gemv_w8a8_decode
+                monkeypatch.setattr(ops, "rmsnorm_quant_rowwise_i8", lambda *a: (calls.append(1), real[0](*a))[1])
+                monkeypatch.setattr(ops, "gemv_w8a8_decode", lambda *a, **k: (calls.append(1), real[1](*a, **k))[1])
+            y = b(x, fr, None, cache)
+            got.append((y, cache.k_layers.clone(), cache.v_layers.clone()))
+        assert calls
+    for a, c in zip(*got):
+        assert torch.equal(a, c)
+
+
+def test_hooks_on_a_fused_blocks_children_still_run():
+    b = _block()
+    x, fr, cache, table = _case(b, 2, 1, 30)
+    cache.bind(table, 31)
+    seen = []
+    with torch.inference_mode():
+        want = b(x, fr, None, cache)
+        h = b.mlp.down.register_forward_hook(lambda m, a, y: seen.append(tuple(y.shape)))
+        assert torch.equal(b(x, fr, None, cache), want) and len(seen) == 1
+        h.remove()
+        assert torch.equal(b(x, fr, None, cache), want) and len(seen) == 1
+
+
+@pytest.mark.parametrize("rows", [3, 40])
+def test_what_the_native_functions_do_not_take_goes_the_general_way(rows):
+    torch.manual_seed(1)
+    q = QuantLinear(256, 96, bias=True, device=DEV)
+    q.load_float_weight(torch.randn(96, 256, device=DEV) * 0.02)
+    wide = torch.randn(rows, 512, device=DEV).to(DT)
+    res = torch.randn(96, rows, device=DEV).to(DT)
+    with torch.inference_mode():
+        want = q(wide[:, :256].contiguous(), residual=res.t().contiguous())
+        assert torch.equal(q(wide[:, :256], residual=res.t()), want)               # strided rows and residual
+        assert torch.equal(q(wide[:, :256].reshape(1, rows, 256), residual=res.t()), want.view(1, rows, 96))
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            y = q(wide[:, :256].contiguous(), residual=res.t().contiguous())
+        side.synchronize()
+        assert torch.equal(y, want)
+        with pytest.raises(ValueError):
+            q(wide)
+        with pytest.raises(ValueError):
+            q(wide[:, :256].double())
+        with pytest.raises(RuntimeError, match="GPU only"):
+            q(wide[:, :256].cpu())
