@@ -20,8 +20,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
 
-from . import _abi, ops
-from .linear import Linear, QuantLinear
+from . import ops
+from .linear import Linear, QuantLinear, linear_native
 
 
 class RMSNorm(nn.Module):
@@ -464,10 +464,8 @@ _host = None  # the native block step once it is loaded
 def _native():
     global _host
     if _host is None:
-        h, m = _abi.host(), torch.nn.modules.module
-        h.set_block_types(QuantLinear, RMSNorm, GQA, MLP, PagedKV,
-                          (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
-                           m._global_backward_pre_hooks), ops.__dict__, _OPERATORS)
+        h = linear_native()
+        h.set_block_types(RMSNorm, GQA, MLP, PagedKV, _OPERATORS)
         _host = h.block_forward
     return _host
 

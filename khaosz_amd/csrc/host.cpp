@@ -389,7 +389,7 @@ PyObject *k_modules, *k_buffers, *k_parameters, *k_qweight, *k_w_scale, *k_bias,
     *k_fwd_pre_hooks, *k_compiled, *k_attention, *k_mlp, *k_input_norm, *k_post_norm, *k_qkv, *k_upgate, *k_o_proj, *k_down, *k_q_norm,
     *k_k_norm, *k_decode_attention, *k_use_qk_norm, *k_use_gate, *k_n_heads, *k_n_kv_heads, *k_head_dim, *k_layer_id, *k_swiglu_quant,
     *k_norm_quant, *k_residual_adds, *k_k_layers, *k_v_layers, *k_page_table, *k_total_len, *k_seq_lens, *k_invalid, *k_page_size,
-    *k_shared;
+    *k_shared, *k_residual, *k_norm;
 
 PyObject* dict_of(PyObject* o) {  // borrowed; null if it has none
   PyObject** d = _PyObject_GetDictPtr(o);
@@ -407,12 +407,13 @@ bool integer(PyObject* d, PyObject* key, int64_t* v) {
   return true;
 }
 
-// What block_forward() is told about the Python side, once (set_block_types).
+// What the functions that stand for a module's call are told about the Python side, once (set_linear_types, set_block_types).
 struct Types {
-  PyObject *quant_linear = nullptr, *rms_norm = nullptr, *gqa = nullptr, *mlp = nullptr, *paged_kv = nullptr;
+  PyObject *quant_linear = nullptr, *fp8_linear = nullptr;
   PyObject* global_hooks = nullptr;  // tuple of the dicts of hooks that run for every module
   PyObject* ops_dict = nullptr;      // the operators' module and, by name, the operators as they were defined
-  PyObject* ops_own = nullptr;
+  PyObject *linear_ops = nullptr, *block_ops = nullptr;
+  PyObject *rms_norm = nullptr, *gqa = nullptr, *mlp = nullptr, *paged_kv = nullptr;
 } types;
 
 // A module whose forward may be replaced by what it is known to do: exactly the class, nothing hooked, nothing wrapped.
@@ -429,12 +430,12 @@ bool ordinary(PyObject* m, PyObject* type, bool called) {
 
 // Nothing watches module calls globally, and the operators are the package's own: a program that replaces one (to
 // count or trace calls) has every call go through its replacement, on the step-by-step path.
-bool unobserved() {
+bool unobserved(PyObject* operators) {
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(types.global_hooks); ++i)
     if (PyDict_GET_SIZE(PyTuple_GET_ITEM(types.global_hooks, i))) return false;
   PyObject *name, *own;
   Py_ssize_t at = 0;
-  while (PyDict_Next(types.ops_own, &at, &name, &own))
+  while (PyDict_Next(operators, &at, &name, &own))
     if (PyDict_GetItem(types.ops_dict, name) != own) return false;
   return true;
 }
@@ -483,6 +484,108 @@ bool gain_of(PyObject* m, int64_t K, int dev, Gain* g) {
   return true;
 }
 
+constexpr int64_t DECODE_ROWS = 16;                  // QuantLinear.DECODE_MAX_ROWS, Fp8Linear.DECODE_MAX_ROWS
+constexpr int64_t FP8_ONEPASS_MIN_BYTES = 16 << 20;  // ops.FP8_ONEPASS_MIN_BYTES
+
+// linear_call(layer, args, kwargs) -> what calling the QuantLinear or Fp8Linear gives, or None where nn.Module's own call has
+// to serve: hooks, a shared input, FP8 inputs that are quantised in one launch with a state the module keeps.
+PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  AQ_TRY AQ_ARGS(3);
+  PyObject *layer = args[0], *given = args[1], *named = args[2];
+  const bool fp8 = reinterpret_cast<PyObject*>(Py_TYPE(layer)) == types.fp8_linear;
+  if (!types.linear_ops || PyTuple_GET_SIZE(given) != 1 || !ordinary(layer, fp8 ? types.fp8_linear : types.quant_linear, true) ||
+      !unobserved(types.linear_ops))
+    return none();
+  PyObject *residual = nullptr, *norm = nullptr;
+  if (const Py_ssize_t n = PyDict_GET_SIZE(named)) {
+    residual = PyDict_GetItem(named, k_residual);
+    norm = fp8 ? nullptr : PyDict_GetItem(named, k_norm);
+    if (n != (residual != nullptr) + (norm != nullptr)) return none();
+    if (norm == Py_None) norm = nullptr;
+  }
+  PyObject* d = dict_of(layer);
+  if (!fp8 && get(d, k_shared) != Py_None) return none();
+  const Tensor *x = unpack(PyTuple_GET_ITEM(given, 0)), *w, *s;
+  Call c;
+  Rows r;
+  Bias b;
+  const void* res;
+  if (!x || x->requires_grad() || !c.at(*x) || !rows_of(*x, &r) ||
+      !weight_of(nested(d, k_buffers, k_qweight), nested(d, k_buffers, k_w_scale), r.K, c.dev, fp8, &w, &s))
+    return none();
+  const int64_t N = w->size(0);
+  const ScalarType type = x->scalar_type();
+  PyObject* bias = nested(d, k_parameters, k_bias);
+  if (!bias_of(bias ? bias : get(d, k_bias), N, c.dev, &b) || !residual_of(residual, r.M, N, type, c.dev, &res)) return none();
+  const void* gain = nullptr;
+  float eps = 0.f;
+  if (norm) {
+    if (!PyTuple_CheckExact(norm) || PyTuple_GET_SIZE(norm) != 2 || !PyFloat_CheckExact(PyTuple_GET_ITEM(norm, 1))) return none();
+    const Tensor* g = unpack(PyTuple_GET_ITEM(norm, 0));
+    if (!g || !plain(*g, type, c.dev) || g->numel() != r.K) return none();
+    gain = g->const_data_ptr();
+    eps = static_cast<float>(PyFloat_AS_DOUBLE(PyTuple_GET_ITEM(norm, 1)));
+  }
+  const int64_t x_bytes = x->numel() * x->element_size();
+  if (fp8 && r.M > DECODE_ROWS && x_bytes >= FP8_ONEPASS_MIN_BYTES) return none();
+  c.current_stream();
+  c10::DimVector shape(x->sizes());
+  shape.back() = N;
+  Tensor y = c.empty(shape, type);
+  // codes and scales of the tokens (and, for FP8, the partial maxima)
+  const int64_t codes = r.M > DECODE_ROWS ? (r.M * r.K + 255) & ~int64_t(255)
+                        : fp8             ? static_cast<int64_t>(lib.aq_gemv_fp8_workspace_bytes(r.M, r.K))
+                                          : static_cast<int64_t>(lib.aq_gemv_w8a8_workspace_bytes(r.M, r.K));
+  const int64_t room = codes + (r.M > DECODE_ROWS ? (fp8 ? 256 + AQ_FP8_AMAX_WS_BYTES : 4 * r.M) : 0);
+  Tensor ws = c.empty({room}, ScalarType::Byte);
+  char* base = static_cast<char*>(ws.mutable_data_ptr());
+  auto* sx = reinterpret_cast<float*>(base + codes);
+  void* yp = y.mutable_data_ptr();
+  const void* wp = w->const_data_ptr();
+  const auto* sp = static_cast<const float*>(s->const_data_ptr());
+  const char* what = "";
+  const int rc = queued([&]() -> int {
+    if (r.M <= DECODE_ROWS) {
+      what = fp8 ? "aq_gemv_fp8_decode" : "aq_gemv_w8a8_decode";
+      if (fp8)
+        return lib.aq_gemv_fp8_decode_residual(r.p, r.code, static_cast<const uint8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K,
+                                               base, codes, c.stream);
+      if (gain)
+        return lib.aq_gemv_w8a8_decode_rmsnorm(r.p, r.code, gain, eps, static_cast<const int8_t*>(wp), sp, b.p, b.code, res, yp, r.code,
+                                               r.M, N, r.K, base, codes, c.stream);
+      return lib.aq_gemv_w8a8_decode_residual(r.p, r.code, static_cast<const int8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K,
+                                              base, codes, c.stream);
+    }
+    if (fp8) {
+      auto* q = reinterpret_cast<uint8_t*>(base);
+      what = "aq_quant_tensor_fp8";
+      if (int e = lib.aq_quant_tensor_fp8(r.p, r.code, x->numel(), q, sx, reinterpret_cast<uint32_t*>(base + codes + 256),
+                                          AQ_FP8_AMAX_WS_BYTES, c.stream))
+        return e;
+      what = "aq_linear_fp8";
+      return lib.aq_linear_fp8_residual(q, sx, static_cast<const uint8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
+    }
+    auto* q = reinterpret_cast<int8_t*>(base);
+    what = gain ? "aq_rmsnorm_quant_rowwise_i8" : "aq_quant_rowwise_i8";
+    if (int e = gain ? lib.aq_rmsnorm_quant_rowwise_i8(r.p, r.code, gain, r.code, eps, r.M, r.K, r.K, q, sx, c.stream)
+                     : lib.aq_quant_rowwise_i8(r.p, r.code, r.M, r.K, r.K, q, sx, c.stream))
+      return e;
+    what = "aq_linear_w8a8";
+    return lib.aq_linear_w8a8_residual(q, sx, static_cast<const int8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
+  });
+  return rc ? fail(rc, what) : THPVariable_Wrap(y);
+  AQ_CATCH
+}
+
+// set_linear_types(QuantLinear, Fp8Linear, hook dicts, ops.__dict__, {name: operator as defined})
+PyObject* set_linear_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  AQ_ARGS(5);
+  if (!PyTuple_Check(args[2]) || !PyDict_Check(args[3]) || !PyDict_Check(args[4])) return PyErr_Format(PyExc_TypeError, "set_linear_types");
+  for (Py_ssize_t i = 0; i < 5; ++i) Py_INCREF(args[i]);  // for the life of the process
+  types.quant_linear = args[0], types.fp8_linear = args[1], types.global_hooks = args[2], types.ops_dict = args[3], types.linear_ops = args[4];
+  Py_RETURN_NONE;
+}
+
 // One stretch of device memory that a block's intermediate results are cut from.
 struct Scratch {
   char* base = nullptr;
@@ -503,7 +606,6 @@ bool merge_in_projection(int64_t B, int64_t width, int64_t total) {
   return B * width * ((total + SLICE - 1) / SLICE) <= 32768;
 }
 
-constexpr int64_t DECODE_ROWS = 16;     // QuantLinear.DECODE_MAX_ROWS
 constexpr int64_t NORM_MAX_K = 12288;   // ops.RMSNORM_QUANT_MAX_K, bf16
 constexpr int64_t SWIGLU_MAX_F = 8192;  // ops.SWIGLU_QUANT_MAX_F, bf16
 
@@ -716,7 +818,7 @@ int Block::queue(const void* in, void* out, const char** what) const {
 // block_forward(block, x, rotary, cache) -> the block's output, or None where the step-by-step path has to serve
 PyObject* block_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   AQ_TRY AQ_ARGS(4);
-  if (!types.ops_own || !unobserved()) return none();
+  if (!types.block_ops || !unobserved(types.block_ops)) return none();
   Block b;
   if (!b.read(args[0], args[1], args[2], args[3])) return none();
   Tensor y = b.c.empty({b.B, b.S, b.dim}, ScalarType::BFloat16);
@@ -726,12 +828,12 @@ PyObject* block_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   AQ_CATCH
 }
 
-// set_block_types(QuantLinear, RMSNorm, GQA, MLP, PagedKV, hook dicts, ops.__dict__, {name: operator as defined})
+// set_block_types(RMSNorm, GQA, MLP, PagedKV, {name: operator as defined})
 PyObject* set_block_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_ARGS(8);
-  if (!PyTuple_Check(args[5]) || !PyDict_Check(args[6]) || !PyDict_Check(args[7])) return PyErr_Format(PyExc_TypeError, "set_block_types");
-  for (Py_ssize_t i = 0; i < 8; ++i) Py_INCREF(args[i]);  // for the life of the process
-  types = Types{args[0], args[1], args[2], args[3], args[4], args[5], args[6], args[7]};
+  AQ_ARGS(5);
+  if (!PyDict_Check(args[4])) return PyErr_Format(PyExc_TypeError, "set_block_types");
+  for (Py_ssize_t i = 0; i < 5; ++i) Py_INCREF(args[i]);  // for the life of the process
+  types.rms_norm = args[0], types.gqa = args[1], types.mlp = args[2], types.paged_kv = args[3], types.block_ops = args[4];
   Py_RETURN_NONE;
 }
 
@@ -752,7 +854,9 @@ PyObject* bind(PyObject*, PyObject* handle) {
 #define AQ_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
+    AQ_METHOD(set_linear_types),
     AQ_METHOD(set_block_types),
+    AQ_METHOD(linear_call),
     AQ_METHOD(quant_rowwise_i8),
     AQ_METHOD(rmsnorm_quant_rowwise_i8),
     AQ_METHOD(swiglu_quant_rowwise_i8),
@@ -786,7 +890,7 @@ PyMODINIT_FUNC PyInit__host() {
               {&k_norm_quant, "_norm_quant"}, {&k_residual_adds, "_residual_adds"}, {&k_k_layers, "k_layers"},
               {&k_v_layers, "v_layers"},      {&k_page_table, "page_table"},    {&k_total_len, "total_len"},
               {&k_seq_lens, "seq_lens"},      {&k_invalid, "_invalid"},         {&k_page_size, "page_size"},
-              {&k_shared, "_shared"}};
+              {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"}};
   for (const auto& k : keys)
     if (!(*k.key = PyUnicode_InternFromString(k.name))) return nullptr;
   return PyModule_Create(&module);

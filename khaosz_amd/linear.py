@@ -126,7 +126,39 @@ class _SharedInput:
         return y
 
 
-class QuantLinear(Linear):
+_linear_call = None  # the native call of a quantized layer once it is loaded
+
+
+def linear_native():
+    """The native host path, told about the layers' classes, the hooks that run for every module, and the operators as
+    defined: while a program has one of those replaced (to count or trace calls), calls go through its replacement."""
+    global _linear_call
+    h = ops._native()
+    if _linear_call is None:
+        m = torch.nn.modules.module
+        h.set_linear_types(QuantLinear, Fp8Linear, (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
+                                                    m._global_backward_pre_hooks), ops.__dict__, _OPERATORS)
+        _linear_call = h.linear_call
+    return h
+
+
+_OPERATORS = {name: getattr(ops, name) for name in (
+    "quant_rowwise_i8", "rmsnorm_quant_rowwise_i8", "linear_w8a8", "gemv_w8a8_decode", "quant_tensor_fp8", "linear_fp8",
+    "gemv_fp8_decode")}
+
+
+class _NativeCall(Linear):
+    """A quantized Linear's call: natively in one step where nothing observes it (no hooks, plain tensors), through
+    ``nn.Module.__call__`` and ``forward`` otherwise -- the same launches and bits."""
+
+    def __call__(self, *args, **kwargs):
+        if _linear_call is None:
+            linear_native()
+        y = _linear_call(self, args, kwargs)
+        return super().__call__(*args, **kwargs) if y is None else y
+
+
+class QuantLinear(_NativeCall):
     """W8A8 Linear: per-channel int8 weight, per-token int8 activation.
 
     Buffers: ``qweight int8 [out, in]``, ``w_scale float32 [out]``; ``bias`` stays a
@@ -277,7 +309,7 @@ class QuantLinear(Linear):
         return f"in_dim={self.in_dim}, out_dim={self.out_dim}, bias={self.bias is not None}, w8a8"
 
 
-class Fp8Linear(Linear):
+class Fp8Linear(_NativeCall):
     """FP8 (OCP e4m3fn) Linear with per-tensor scales and fp32 accumulation."""
 
     def __init__(self, in_dim: int, out_dim: int, bias: bool = False, device=None):
