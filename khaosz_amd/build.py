@@ -4,7 +4,7 @@
   khaosz_amd/_host.so                the native host path (csrc/host.cpp: tensors in, launches out), a Python extension
                                      against torch's C++ API that calls the C ABI above;
   khaosz_amd/lib/libastrai_q_lab.so  the same objects plus the measurement probes and the tile-forcing hook
-                                     of csrc/aq_lab.h (the GEMM and GEMV sources rebuilt with -DAQ_LAB), for the
+                                     of csrc/aq_lab.h (the GEMM and decode-row GEMV sources rebuilt with -DAQ_LAB), for the
                                      benchmark's ceilings and for tests that pin a tile shape.
 
 hipcc cross-compiles without a GPU.  The two libraries depend on the HIP runtime only (no torch, no Python).
@@ -27,9 +27,9 @@ OBJ_DIR = os.path.join(HERE, "lib", "obj")
 LIB = os.path.join(HERE, "lib", "libastrai_q.so")
 LAB_LIB = os.path.join(HERE, "lib", "libastrai_q_lab.so")
 HOST_EXT = os.path.join(HERE, "_host.so")
-SOURCES = ["abi.hip", "quant.hip", "gemm_mfma.hip", "gemv.hip", "attn_decode.hip", "attn_prefill.hip"]
+SOURCES = ["abi.hip", "quant.hip", "gemm_mfma.hip", "gemv.hip", "gemv_rows.hip", "attn_decode.hip", "attn_prefill.hip"]
 # (source, object, extra flags) of the lab library's own objects; the other product objects are shared
-LAB_SOURCES = [("gemm_mfma.hip", "gemm_mfma_lab.o", ["-DAQ_LAB"]), ("gemv.hip", "gemv_lab.o", ["-DAQ_LAB"]),
+LAB_SOURCES = [("gemm_mfma.hip", "gemm_mfma_lab.o", ["-DAQ_LAB"]), ("gemv_rows.hip", "gemv_rows_lab.o", ["-DAQ_LAB"]),
                ("lab.hip", "lab.o", [])]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -72,7 +72,7 @@ def build(force: bool = True, verbose: bool = False, stall_counters: bool = Fals
     os.makedirs(OBJ_DIR, exist_ok=True)
     lab_sources = [(src, obj, extra + (["-DAQ_LAB_STALL"] if stall_counters and src == "gemm_mfma.hip" else []))
                    for src, obj, extra in LAB_SOURCES]
-    headers = [os.path.join(CSRC, "aq_common.h"), os.path.join(CSRC, "aq_rows.h"), os.path.join(CSRC, "aq_lab.h"),
+    headers = [os.path.join(CSRC, "aq_common.h"), os.path.join(CSRC, "aq_rows.h"), os.path.join(CSRC, "aq_gemv.h"), os.path.join(CSRC, "aq_lab.h"),
                os.path.join(HERE, "..", "include", "astrai_q.h")]
 
     def compile_one(job):
@@ -94,7 +94,7 @@ def build(force: bool = True, verbose: bool = False, stall_counters: bool = Fals
         all_objs = list(ex.map(compile_one, SOURCES + lab_sources))
         host.result()
     objs, lab_only = all_objs[:len(SOURCES)], all_objs[len(SOURCES):]
-    lab_objs = [o for o in objs if not o.endswith(("gemm_mfma.o", "gemv.o"))] + lab_only
+    lab_objs = [o for o in objs if not o.endswith(("gemm_mfma.o", "gemv_rows.o"))] + lab_only
     for lib, members in ((LIB, objs), (LAB_LIB, lab_objs)):
         if force or _stale(lib, members):
             cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib, *members]

@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "aq_common.h"
+#include "aq_gemv.h"
 #include "aq_rows.h"
 
 namespace aq {
@@ -71,78 +72,6 @@ struct Butterfly {
 };
 
 constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v / 2); }
-
-struct GemvArgs {
-  const void* x;      // [M, K] bf16 activations (fused-quantise kernels), row stride K
-  const int8_t* xq;   // [M, K] codes (kernels that take codes)
-  const float* sx;    // [M]
-  const int8_t* wq;   // [N, K]
-  const float* sw;    // [N]
-  const void* bias;   // [N] or null
-  const void* res;    // [M, N] residual in y's dtype (row stride ldr), or null; may be y itself
-  void* y;            // [M, N]
-  int64_t ldr;
-  int M, N, K;
-  int bias_dtype, y_dtype;
-  int ksplit, groups;  // matrix-core variant: wavefronts sharing a row group, row groups per workgroup
-  const void* gamma;   // NORM kernels: RMSNorm gain [K] in x's dtype
-  float eps;
-  const float* parts;  // MERGE kernels: attention partial results in place of x
-  int parts_ns, parts_d;
-};
-
-// y (+ residual): the projection is rounded to the output type first and the
-// sum rounded again, the bits a separate elementwise add of the two tensors gives.
-__device__ __forceinline__ float add_residual_bf16(float y, uint32_t res_bits) {
-  return __fadd_rn(bf16_bits_to_f32((uint16_t)f32_to_bf16_bits(y)), bf16_bits_to_f32((uint16_t)res_bits));
-}
-
-// Epilogue operands (activation scale, weight scale, bias, residual) are requested at the very start of a
-// kernel through buffer descriptors, without a branch: a descriptor of size 0 (no bias, no residual, a
-// wavefront or lane that stores nothing) makes the load return 0 without touching memory.  Written as
-// `if (bias) load`, the compiler waited for the loads at every join of those branches -- a full memory
-// round trip in front of the weight stream whenever a bf16 bias was given.
-struct EpiOperands {
-  __amdgpu_buffer_rsrc_t sx, sw, bias_f32, bias_bf16, res_f32, res_bf16;
-  __device__ __forceinline__ EpiOperands(const GemvArgs& p, bool live, bool want_sx, bool want_res) {
-    const bool has_bias = p.bias != nullptr;
-    const bool bias_is_bf16 = p.bias_dtype == AQ_BF16, res_is_bf16 = p.y_dtype == AQ_BF16;
-    const uint32_t n = (uint32_t)p.N;
-    sx = make_rsrc(want_sx ? (const void*)p.sx : (const void*)p.sw, live && want_sx ? (uint32_t)p.M * 4u : 0u);
-    sw = make_rsrc(p.sw, live ? n * 4u : 0u);
-    bias_f32 = make_rsrc(has_bias ? p.bias : (const void*)p.sw, live && has_bias && !bias_is_bf16 ? n * 4u : 0u);
-    bias_bf16 = make_rsrc(has_bias ? p.bias : (const void*)p.sw, live && has_bias && bias_is_bf16 ? n * 2u : 0u);
-    const bool has_res = want_res && p.res != nullptr;
-    const uint32_t res_elems = (uint32_t)p.M * (uint32_t)p.ldr;
-    res_f32 = make_rsrc(has_res ? p.res : (const void*)p.sw, live && has_res && !res_is_bf16 ? res_elems * 4u : 0u);
-    res_bf16 = make_rsrc(has_res ? p.res : (const void*)p.sw, live && has_res && res_is_bf16 ? res_elems * 2u : 0u);
-  }
-  __device__ __forceinline__ float load_sx(int m, bool ok) const {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(sx, ok ? m * 4 : (int)OOB_OFFSET, 0, 0));
-  }
-  __device__ __forceinline__ float load_sw(int n, bool ok) const {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(sw, ok ? n * 4 : (int)OOB_OFFSET, 0, 0));
-  }
-  // Both element sizes are requested; only the descriptor of the operand's own type has a size, the other
-  // load returns 0, and the two results are OR-ed: no select on the type (which the compiler turns back
-  // into a branch around each load, with a wait at its join).
-  __device__ __forceinline__ float load_bias(int n, bool ok) const {
-    const uint32_t f = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(bias_f32, ok ? n * 4 : (int)OOB_OFFSET, 0, 0);
-    const uint32_t h = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(bias_bf16, ok ? n * 2 : (int)OOB_OFFSET, 0, 0);
-    return __uint_as_float(f | (h << 16));
-  }
-  __device__ __forceinline__ uint32_t load_res(int m, int n, bool ok, int ldr) const {  // raw bits of one element
-    const int e = m * ldr + n;
-    const uint32_t f = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(res_f32, ok ? e * 4 : (int)OOB_OFFSET, 0, 0);
-    const uint32_t h = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(res_bf16, ok ? e * 2 : (int)OOB_OFFSET, 0, 0);
-    return f | (h & 0xffffu);
-  }
-};
-
-// Weight loads are marked as streaming (nt): every byte is read exactly once per launch.  Measured 0.05 - 0.35 us
-// per launch against plain loads (M = 1: 5.50 -> 5.15 us; a one-shot 16 MiB read: 4.4 -> 4.0 us).
-#define GV_WLOAD buffer_load_16_stream
-#define GV_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((n) & 15) | (((n) >> 4) << 14))
 
 // FUSED: the kernel quantises the bf16 activation rows itself (VPL 16-byte vectors
 // per lane per row) instead of copying codes a separate launch produced.
@@ -338,21 +267,6 @@ struct GemvShape {
   int waves, ksplit;
 };
 
-// A kernel whose dynamic LDS may exceed 64 KiB is opted in to the whole 160 KiB of a compute unit the first
-// time a launch on a device needs it (one attribute call per kernel and device instead of one per launch).
-// Two threads racing here both make the idempotent call.
-struct LdsOptIn {
-  bool done[64] = {};
-  int ensure(const void* fn) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
-    if (dev >= 0 && done[dev]) return 0;
-    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e != hipSuccess) return (int)e;
-    if (dev >= 0) done[dev] = true;
-    return 0;
-  }
-};
 static GemvShape gemv_shape(int N, int K, bool fused, int mt) {
   GemvShape sh{GV_WAVES, 1};
   if (fused) return sh;
@@ -402,7 +316,6 @@ static int launch_gemv(GemvArgs a, hipStream_t st) {
   return launch_gemv_fw<MT, FUSED, VPL, NORM, MERGE, GV_WAVES>(a, st);
 }
 
-constexpr int64_t GV_MAX_LDS = 160 * 1024;  // LDS of one gfx950 CU
 #ifndef AQ_GV_MFMA_MIN_M
 #define AQ_GV_MFMA_MIN_M 8
 #endif
@@ -424,21 +337,6 @@ constexpr int GV_MFMA_MIN_M = AQ_GV_MFMA_MIN_M;  // more tokens than this take t
 // summed through LDS (exact int32).  A workgroup holds `groups` row groups:
 // 2 x 2 wavefronts when N fills the device that way, fewer rows per workgroup
 // and more K parts when it does not.
-#ifdef AQ_LAB
-// Lab build only (csrc/aq_lab.h, aq_lab_set_gemv_timeline): where the wavefronts of the matrix-core GEMV leave
-// time stamps of the 100 MHz counter, 8 per wavefront.  Expands to nothing in the product library.
-__device__ long long* gv_timeline = nullptr;
-__device__ int gv_skip_weights = 0;  // != 0: the kernel that quantises its rows requests no weight bytes (products of zeros)
-#define GV_STAMP(slot)                                                                                          \
-  do {                                                                                                          \
-    if (gv_timeline && lane == 0) gv_timeline[((size_t)blockIdx.x * 16 + wave) * 8 + (slot)] = wall_clock64(); \
-  } while (0)
-#else
-#define GV_STAMP(slot) \
-  do {                 \
-  } while (0)
-#endif
-
 constexpr int GM_ROWS = 16;    // weight rows per wavefront
 constexpr int GM_MAX_WAVES = 8;
 constexpr int GM_BATCH = 8;    // MFMA steps (64 K bytes each) per register batch
@@ -448,25 +346,11 @@ constexpr int GM_BATCH = 8;    // MFMA steps (64 K bytes each) per register batc
 // compiler drain the weight loads at the join, 0.4 us of a 6.5 us launch).
 // XR: rounds of token-code vectors (8 per thread each) requested ahead of the weight stream; rows too long for
 // XR rounds copy the rest afterwards, which waits for the weight loads in flight.
-// FQ > 0: the kernel quantises up to FQ (8 or 16) bf16 token rows of at most 2048 elements itself, one or two
-// rows per wavefront of a KS x GR = 8 wavefront workgroup, while its weight loads are in flight (the row
-// arithmetic of the stand-alone quantiser, shared through aq_rows.h: same codes and scales); NORM: after
-// RMS-normalising them with the gain p.gamma.  One launch per decode step instead of two.
 // FP8: weights and tokens are OCP e4m3fn codes with one scale per tensor (p.sx, p.sw point to scalars) and the
 // products run on v_mfma_f32_16x16x128_f8f6f4 -- one instruction per 128-byte line instead of two -- with fp32
-// accumulation; with FQ the kernel casts its bf16 rows itself, after the maximum over ALL rows (the per-tensor
-// scale of aq_quant_tensor_fp8: s = amax / 448, codes = e4m3(clamp(x / s))) has gone round the workgroup.
-// SWI: the weight is an MLP's up and gate projections stacked, rows [0, F) up and [F, 2F) gate with F = N / 2 (what
-// QuantLinear.concat([up, gate]) builds), and the kernel writes h = up * silu(gate), [M, F], instead of the 2F
-// projections: the first half of a workgroup's row groups takes 16-row blocks of up, the second half the same
-// blocks of gate, the gate sums cross to the up wavefronts through LDS, and the up wavefronts apply the activation
-// (the fixed-sequence exponential and correctly rounded divide of the stand-alone SwiGLU kernel) to the two
-// projections as the separate launch would have stored them (rounded to the output type first).
-template <int KS, int GR, bool RES, int XR, int FQ = 0, bool NORM = false, bool FP8 = false, bool SWI = false>
+// accumulation.
+template <int KS, int GR, bool RES, int XR, bool FP8 = false>
 __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p) {
-  static_assert(FQ == 0 || (KS > 0 && GR > 0), "the in-kernel quantiser deals rows to a fixed number of wavefronts");
-  static_assert(!(FP8 && NORM), "no fused norm in front of the FP8 cast");
-  static_assert(!SWI || (FQ > 0 && !RES && !FP8 && GR % 2 == 0), "the SwiGLU epilogue exists for the int8 kernels that quantise their rows");
   extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [16][K + 16] token codes, [16] scales, 16 spare bytes; later the partial sums
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -474,12 +358,8 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
   const int nthreads = ksplit * groups * 64;
   const int grp = wave / ksplit, kh = wave % ksplit;
   const int K = p.K, N = p.N, M = p.M;
-  // first weight row of this wavefront's group, and the end of the rows it may touch
-  const int FH = N >> 1;  // SWI: rows per half
-  const int hgroups = SWI ? groups >> 1 : groups;
-  const int ghalf = SWI ? grp / hgroups : 0, gsub = SWI ? grp - ghalf * hgroups : grp;
-  const int n0 = __builtin_amdgcn_readfirstlane((SWI ? ghalf * FH : 0) + (blockIdx.x * hgroups + gsub) * GM_ROWS);
-  const int nlim = SWI ? (ghalf + 1) * FH : N;
+  // first weight row of this wavefront's group
+  const int n0 = __builtin_amdgcn_readfirstlane((blockIdx.x * groups + grp) * GM_ROWS);
   const int pitch = K + 16;  // 16 token rows then start 4 banks apart: conflict-free 16-byte reads
   const int khalf = K / ksplit;  // a multiple of 128 (checked by the launcher)
   const int nline = khalf / 128;  // 128-byte lines of a row's K part: two MFMA steps each
@@ -495,28 +375,23 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
   // no other workgroup shares and which therefore come from HBM, hold back the token rows that every workgroup
   // reads and the caches serve (M = 16, N = 8192: 7.45 -> 7.2 us with the rows quantised here, 5.85 -> 5.65 us on
   // codes).
-  const EpiOperands epi(p, kh == 0, FQ == 0, RES);
+  const EpiOperands epi(p, kh == 0, true, RES);
   float sxv = 0.0f;
   auto load_epi = [&]() {
     sxv = epi.load_sx(FP8 ? 0 : tok, FP8 || tok < M);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int n = rbase + r;
-      swv[r] = epi.load_sw(FP8 ? 0 : n, FP8 || n < nlim);
-      bv[r] = epi.load_bias(n, n < nlim);
-      rv[r] = RES ? epi.load_res(tok, n, tok < M && n < nlim, (int)p.ldr) : 0u;
+      swv[r] = epi.load_sw(FP8 ? 0 : n, FP8 || n < N);
+      bv[r] = epi.load_bias(n, n < N);
+      rv[r] = RES ? epi.load_res(tok, n, tok < M && n < N, (int)p.ldr) : 0u;
     }
   };
 
   // weight stream: descriptor over this wavefront's 16 rows; rows past N read as zero
-  const int rows = n0 < nlim ? ((nlim - n0) < GM_ROWS ? (nlim - n0) : GM_ROWS) : 0;
-#ifdef AQ_LAB
-  const __amdgpu_buffer_rsrc_t Wr = make_rsrc(p.wq + (int64_t)(n0 < nlim ? n0 : 0) * K,
-                                              FQ > 0 && gv_skip_weights ? 0u : (uint32_t)rows * (uint32_t)K);
-#else
+  const int rows = n0 < N ? ((N - n0) < GM_ROWS ? (N - n0) : GM_ROWS) : 0;
   const __amdgpu_buffer_rsrc_t Wr =
-      make_rsrc(p.wq + (int64_t)(n0 < nlim ? n0 : 0) * K, (uint32_t)rows * (uint32_t)K);
-#endif
+      make_rsrc(p.wq + (int64_t)(n0 < N ? n0 : 0) * K, (uint32_t)rows * (uint32_t)K);
   // Whole 128-byte lines per load: an instruction covers one line of 8 rows (lane l: row l % 8, 16-byte piece
   // l / 8), two instructions (rows 0..7 and 8..15) per line index.  In the MFMA's own operand order (lane l: row
   // l % 16, piece l / 16 of a 64-byte step) an instruction would cover 16 half lines, and a one-shot read of
@@ -539,132 +414,50 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
   // token codes -> LDS (padded rows; tokens >= M are zero).  Their loads are
   // issued before the weight loads, so they return first and the LDS fill
   // overlaps the weight stream's flight time.
-  float* const sx_lds = reinterpret_cast<float*>(xs + 16 * pitch);
-  if constexpr (FQ > 0) {
-    // produced here: every wavefront requests its bf16 rows, then its weights, then rounds the rows while the
-    // weights are in flight.  Rows >= M are not written: the lanes of those tokens read row 0 and their
-    // products are never stored.
-    constexpr int WAVES = KS * GR, RPW = (FQ + WAVES - 1) / WAVES;
-    RowsToLds<true, RPW, 4> xrows;
-    xrows.issue(p.x, M, K, K, wave, WAVES, lane);
-    if constexpr (NORM) xrows.issue_gamma(p.gamma, K, lane);
-    asm volatile("" ::: "memory");  // request order: token rows, epilogue operands, the weight stream
-    load_epi();
-    asm volatile("" ::: "memory");
-    GV_STAMP(0);
-    wload(0, wa);
-    wload(GM_LINES, wb);
-    asm volatile("" ::: "memory");
-    if constexpr (!FP8) {
-      xrows.template finish<NORM>(M, M, K, xs, pitch, sx_lds, wave, WAVES, lane, p.eps);
-      GV_STAMP(3);
-    } else {
-      // the tensor's maximum: every wavefront's share through LDS (a maximum has no order), then the cast
-      float amax = 0.0f;
+  const __amdgpu_buffer_rsrc_t Xr = make_rsrc(p.xq, (uint32_t)M * (uint32_t)K);
+  const int nvec_row = K / 16;
+  const int nvec = 16 * nvec_row;
+  constexpr int XV = 8;  // vectors per thread per round: 16 x 2048 codes in one round of 256 threads
+  uint4 xvr[XR][XV];
+  auto xload = [&](int v0, uint4 (&xv)[XV]) {
 #pragma unroll
-      for (int j = 0; j < RPW; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float f[8];
-          RowIn<true>::unpack(xrows.c[j][i], f);  // rows >= M and vectors past K were loaded as zeros
-          amax = fmaxf(amax, vec_amax<8>(f));
-        }
-      amax = wave_max(amax);
-      if (lane == 0) sx_lds[wave] = amax;
-      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();  // no memory fence: the weight loads stay in flight
-      asm volatile("" ::: "memory");
-      float all = 0.0f;
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w) all = fmaxf(all, sx_lds[w]);
-      float sc = __fdiv_rn(all, 448.0f);
-      if (all == 0.0f) sc = 1.0f;
-      sxv = sc;
-      const float rsc = __fdiv_rn(1.0f, sc);  // correctly rounded: what the one-step sequence below needs
-      const bool lean_ok = sc >= 5.421010862427522e-20f && sc <= 1.8446744073709552e19f;  // [2^-64, 2^64]
-      const int nvec = K / 8;
-#pragma unroll
-      for (int j = 0; j < RPW; ++j) {
-        const int m = wave + j * WAVES;
-        if (m >= M) continue;  // uniform
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int v = i * 64 + lane;
-          if (v < nvec) {
-            float f[8];
-            RowIn<true>::unpack(xrows.c[j][i], f);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              // x / s: the one-correction sequence that gives a bf16 number's e4m3 code exactly for in-range
-              // scales (see quant_codes; a -0.0 comes out as +0.0, which no product can tell apart), the
-              // divide itself otherwise; then the clamp to the e4m3 range
-              float q;
-              if (__builtin_expect(lean_ok, 1)) {
-                q = f[e] * rsc;
-                q = __builtin_fmaf(__builtin_fmaf(-sc, q, f[e]), rsc, q);
-              } else {
-                q = __fdiv_rn(f[e], sc);
-              }
-              f[e] = fminf(fmaxf(q, -448.0f), 448.0f);
-            }
-            int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
-            w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w0, true);
-            int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], 0, false);
-            w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], w1, true);
-            *reinterpret_cast<uint2*>(xs + m * pitch + v * 8) = make_uint2((uint32_t)w0, (uint32_t)w1);
-          }
-        }
-      }
+    for (int i = 0; i < XV; ++i) {
+      const int v = v0 + i * nthreads + tid;
+      xv[i] = buffer_load_16(Xr, v < nvec ? (uint32_t)v * 16u : OOB_OFFSET);
     }
-  } else {
-    const __amdgpu_buffer_rsrc_t Xr = make_rsrc(p.xq, (uint32_t)M * (uint32_t)K);
-    const int nvec_row = K / 16;
-    const int nvec = 16 * nvec_row;
-    constexpr int XV = 8;  // vectors per thread per round: 16 x 2048 codes in one round of 256 threads
-    uint4 xvr[XR][XV];
-    auto xload = [&](int v0, uint4 (&xv)[XV]) {
+  };
+  // Stores without a branch: vectors past the end go to the spare slot behind the scales.  (With the
+  // store under `if (v < nvec)` the compiler sank a vector's load into that branch, behind the weight
+  // loads, and then waited for every load of the wavefront before the first LDS store: the matrix
+  // products started only after the whole weight stream had landed.)
+  uint8_t* const spare = xs + 16 * pitch + 16 * sizeof(float);
+  auto xstore = [&](int v0, const uint4 (&xv)[XV]) {
 #pragma unroll
-      for (int i = 0; i < XV; ++i) {
-        const int v = v0 + i * nthreads + tid;
-        xv[i] = buffer_load_16(Xr, v < nvec ? (uint32_t)v * 16u : OOB_OFFSET);
-      }
-    };
-    // Stores without a branch: vectors past the end go to the spare slot behind the scales.  (With the
-    // store under `if (v < nvec)` the compiler sank a vector's load into that branch, behind the weight
-    // loads, and then waited for every load of the wavefront before the first LDS store: the matrix
-    // products started only after the whole weight stream had landed.)
-    uint8_t* const spare = xs + 16 * pitch + 16 * sizeof(float);
-    auto xstore = [&](int v0, const uint4 (&xv)[XV]) {
-#pragma unroll
-      for (int i = 0; i < XV; ++i) {
-        const int v = v0 + i * nthreads + tid;
-        const int m = v / nvec_row, c = v - m * nvec_row;
-        *reinterpret_cast<uint4*>(v < nvec ? xs + m * pitch + c * 16 : spare) = xv[i];
-      }
-    };
-#pragma unroll
-    for (int r = 0; r < XR; ++r) xload(r * XV * nthreads, xvr[r]);
-    asm volatile("" ::: "memory");  // request order: token codes, epilogue operands, the weight stream
-    load_epi();
-    asm volatile("" ::: "memory");
-    wload(0, wa);
-    wload(GM_LINES, wb);
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int r = 0; r < XR; ++r) xstore(r * XV * nthreads, xvr[r]);  // waits for the token codes only: the oldest requests
-    for (int v0 = XR * XV * nthreads; v0 < nvec; v0 += XV * nthreads) {  // still longer rows
-      xload(v0, xvr[0]);
-      xstore(v0, xvr[0]);
+    for (int i = 0; i < XV; ++i) {
+      const int v = v0 + i * nthreads + tid;
+      const int m = v / nvec_row, c = v - m * nvec_row;
+      *reinterpret_cast<uint4*>(v < nvec ? xs + m * pitch + c * 16 : spare) = xv[i];
     }
+  };
+#pragma unroll
+  for (int r = 0; r < XR; ++r) xload(r * XV * nthreads, xvr[r]);
+  asm volatile("" ::: "memory");  // request order: token codes, epilogue operands, the weight stream
+  load_epi();
+  asm volatile("" ::: "memory");
+  wload(0, wa);
+  wload(GM_LINES, wb);
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int r = 0; r < XR; ++r) xstore(r * XV * nthreads, xvr[r]);  // waits for the token codes only: the oldest requests
+  for (int v0 = XR * XV * nthreads; v0 < nvec; v0 += XV * nthreads) {  // still longer rows
+    xload(v0, xvr[0]);
+    xstore(v0, xvr[0]);
   }
   // LDS writes done, then a barrier without a memory fence: the weight loads stay in flight
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  if constexpr (FQ > 0 && !FP8) sxv = sx_lds[tok < M ? tok : 0];
-  GV_STAMP(4);
 
   // Four independent accumulators (summed at the end: int32, exact in any order) and a batch's token
   // fragments read from LDS up front: one chain of 16 dependent read -> MFMA steps took 0.6 us after the
@@ -679,7 +472,7 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
   // row l % 8 (register lo) and of row 8 + l % 8 (register hi), so lanes 0..7 of each row of 16 lanes have
   // their operand of step e = 0 in lo, and lanes 8..15 find theirs in hi of lane l - 8; for e = 1 it is lo of
   // lane l + 8 and the own hi: one rotation by 8 within the row of 16 lanes, written into half of the lanes.
-  const uint8_t* xl = xs + (FQ > 0 && tok >= M ? 0 : tok) * pitch + kh * khalf + (lane >> 4) * 32;
+  const uint8_t* xl = xs + tok * pitch + kh * khalf + (lane >> 4) * 32;
   auto consume = [&](int line0, const uint4 (&wc)[GM_BATCH]) {
     v4i x[GM_BATCH];
 #pragma unroll
@@ -722,7 +515,6 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
   }
 
   accv acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
-  GV_STAMP(5);
   // sum the K parts: all but the first wavefront of each group park their 4 sums in LDS
   __syncthreads();  // everyone is done reading the token codes: the buffer is reused
   int* part = reinterpret_cast<int*>(xs) + grp * (ksplit - 1) * 256;
@@ -730,49 +522,6 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
     *reinterpret_cast<accv*>(part + (kh - 1) * 256 + lane * 4) = acc;
   }
   __syncthreads();
-  if constexpr (SWI) {
-    // every wavefront stays for the exchange: gate sums -> LDS (behind the K-part area) -> the up wavefronts
-    float* const ex = reinterpret_cast<float*>(xs) + groups * (ksplit - 1) * 256 + (gsub * 64 + lane) * 4;
-    const bool live = kh == 0;
-    float u[4];
-    if (live) {
-      for (int k = 0; k < ksplit - 1; ++k) acc += *reinterpret_cast<const accv*>(part + k * 256 + lane * 4);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        u[r] = __fmul_rn(__fmul_rn((float)acc[r], sxv), swv[r]);
-        if (p.bias) u[r] = __fadd_rn(u[r], bv[r]);
-        if (p.y_dtype == AQ_BF16) u[r] = bf16_bits_to_f32(f32_to_bf16_bits(u[r]));  // as the projection would be stored
-      }
-      if (ghalf == 1) *reinterpret_cast<float4*>(ex) = make_float4(u[0], u[1], u[2], u[3]);
-    }
-    __syncthreads();
-    if (!live || ghalf == 1 || tok >= M) return;
-    const float4 g4 = *reinterpret_cast<const float4*>(ex);
-    const float g[4] = {g4.x, g4.y, g4.z, g4.w};
-    float h[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) h[r] = swiglu_repro(u[r], g[r]);
-    const int64_t o = (int64_t)tok * FH + rbase;  // rbase lies in the up half: the column of h
-    if (p.y_dtype == AQ_BF16) {
-      uint16_t* dst = reinterpret_cast<uint16_t*>(p.y) + o;
-      if ((FH & 3) == 0 && rbase + 3 < FH) {
-        uint2 pk;
-        pk.x = pack_bf16x2(h[0], h[1]);
-        pk.y = pack_bf16x2(h[2], h[3]);
-        *reinterpret_cast<uint2*>(dst) = pk;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (rbase + r < FH) dst[r] = (uint16_t)f32_to_bf16_bits(h[r]);
-      }
-    } else {
-      float* dst = reinterpret_cast<float*>(p.y) + o;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (rbase + r < FH) dst[r] = h[r];
-    }
-    return;
-  }
   if (kh != 0) return;
   for (int k = 0; k < ksplit - 1; ++k) acc += *reinterpret_cast<const accv*>(part + k * 256 + lane * 4);  // fp32: a fixed order
 
@@ -807,7 +556,6 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
         if (rbase + r < N) dst[r] = y[r];
     }
   }
-  GV_STAMP(6);
 }
 
 // the streaming MFMA variant needs K in whole 256-byte steps (two K parts of whole 128-byte lines)
@@ -839,10 +587,10 @@ static int launch_gemv_mfma(GemvArgs a, hipStream_t st, bool fp8 = false) {
         {gemv_mfma_kernel<0, 0, true, 1>, gemv_mfma_kernel<0, 0, true, 3>}},
        {{gemv_mfma_kernel<2, 2, false, 1>, gemv_mfma_kernel<2, 2, false, 3>},
         {gemv_mfma_kernel<2, 2, true, 1>, gemv_mfma_kernel<2, 2, true, 3>}}},
-      {{{gemv_mfma_kernel<0, 0, false, 1, 0, false, true>, gemv_mfma_kernel<0, 0, false, 3, 0, false, true>},
-        {gemv_mfma_kernel<0, 0, true, 1, 0, false, true>, gemv_mfma_kernel<0, 0, true, 3, 0, false, true>}},
-       {{gemv_mfma_kernel<2, 2, false, 1, 0, false, true>, gemv_mfma_kernel<2, 2, false, 3, 0, false, true>},
-        {gemv_mfma_kernel<2, 2, true, 1, 0, false, true>, gemv_mfma_kernel<2, 2, true, 3, 0, false, true>}}}};
+      {{{gemv_mfma_kernel<0, 0, false, 1, true>, gemv_mfma_kernel<0, 0, false, 3, true>},
+        {gemv_mfma_kernel<0, 0, true, 1, true>, gemv_mfma_kernel<0, 0, true, 3, true>}},
+       {{gemv_mfma_kernel<2, 2, false, 1, true>, gemv_mfma_kernel<2, 2, false, 3, true>},
+        {gemv_mfma_kernel<2, 2, true, 1, true>, gemv_mfma_kernel<2, 2, true, 3, true>}}}};
   const kern_t fn = table[fp8][fixed][res][long_rows];
   if (lds > 64 * 1024) {
     static LdsOptIn opted[16];
@@ -853,72 +601,9 @@ static int launch_gemv_mfma(GemvArgs a, hipStream_t st, bool fp8 = false) {
   return (int)hipGetLastError();
 }
 
-// The matrix-core variant that quantises its token rows itself (8 wavefronts per workgroup, a row -- two above
-// 8 tokens -- per wavefront), where it measured faster than the alternatives (bf16 rows of K = 2048, one launch):
-//   9..16 tokens: always (N = 8192: 7.6 us against 8.4 us for row quantiser + GEMV; N = 2048: 6.6 against 7.1);
-//   5..8 tokens: from N = 8192 on (6.45 us against 7.4 us for the dot-product kernel, which is bound by its
-//                vector ALU there; at N = 4096 the dot-product kernel still wins, 4.8 against 5.2 us);
-//                with the norm folded in, whose arithmetic weighs on the dot-product kernel's fewer wavefronts,
-//                from N = 6144 on (7.2 -> 6.5 us there; level at N = 3072);
-//   3..4 tokens: only for matrices with more 32-row blocks than compute units (N = 11264: 7.0 against 7.6 us).
-static bool gemv_mfma_fq_ok(int64_t M, int64_t N, int64_t K, bool norm = false) {
-  if (K > 2048 || (K % 512) != 0) return false;
-  const bool wide = (N + 31) / 32 > device_cus();
-  return M >= 9 || (M >= 5 && N >= (norm ? 6144 : 8192)) || (M >= 3 && wide);
-}
-
-static int launch_gemv_mfma_fq(GemvArgs a, hipStream_t st, bool fp8 = false) {
-  // 32 weight rows per workgroup (2 row groups x 4 K parts) while that gives every workgroup a compute unit
-  // of its own; beyond that 64 rows (4 row groups x 2 K parts): a second round of workgroups would repeat
-  // the row quantisation behind the first (N = 11264, 8 tokens: 9.9 -> 7.1 us).
-  const bool wide = (a.N + 31) / 32 > device_cus();
-  a.ksplit = wide ? 2 : 4;
-  a.groups = wide ? 4 : 2;
-  const unsigned grid = (unsigned)((a.N + GM_ROWS * a.groups - 1) / (GM_ROWS * a.groups));
-  const size_t lds = (size_t)16 * (a.K + 16) + 16 * sizeof(float) + 16;
-  const bool res = a.res != nullptr, many = a.M > 8, norm = a.gamma != nullptr;
-  using kern_t = void (*)(GemvArgs);
-#define AQ_FQ_TABLE(KS, GR)                                                                                  \
-  {{{gemv_mfma_kernel<KS, GR, false, 1, 8, false>, gemv_mfma_kernel<KS, GR, false, 1, 8, true>},             \
-    {gemv_mfma_kernel<KS, GR, false, 1, 16, false>, gemv_mfma_kernel<KS, GR, false, 1, 16, true>}},          \
-   {{gemv_mfma_kernel<KS, GR, true, 1, 8, false>, gemv_mfma_kernel<KS, GR, true, 1, 8, true>},               \
-    {gemv_mfma_kernel<KS, GR, true, 1, 16, false>, gemv_mfma_kernel<KS, GR, true, 1, 16, true>}}}
-  static const kern_t table[2][2][2][2] = {AQ_FQ_TABLE(4, 2), AQ_FQ_TABLE(2, 4)};
-#undef AQ_FQ_TABLE
-#define AQ_FQ8_TABLE(KS, GR)                                                                                       \
-  {{gemv_mfma_kernel<KS, GR, false, 1, 8, false, true>, gemv_mfma_kernel<KS, GR, false, 1, 16, false, true>},      \
-   {gemv_mfma_kernel<KS, GR, true, 1, 8, false, true>, gemv_mfma_kernel<KS, GR, true, 1, 16, false, true>}}
-  static const kern_t table8[2][2][2] = {AQ_FQ8_TABLE(4, 2), AQ_FQ8_TABLE(2, 4)};
-#undef AQ_FQ8_TABLE
-  const kern_t fn = fp8 ? table8[wide][res][many] : table[wide][res][many][norm];
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(8 * 64), lds, st, a);
-  return (int)hipGetLastError();
-}
-
-// up/gate + SwiGLU in one launch: bf16 rows of K <= 2048 in whole 512-byte steps, F a multiple of 16.
-static bool gemv_mfma_swiglu_ok(int64_t M, int64_t F, int64_t K) {
+// up/gate + SwiGLU in one launch (gemv_rows.hip): bf16 rows of K <= 2048 in whole 512-byte steps, F a multiple of 16.
+static bool gemv_swiglu_ok(int64_t M, int64_t F, int64_t K) {
   return M >= 1 && M <= 16 && F > 0 && (F % 16) == 0 && K <= 2048 && (K % 512) == 0;
-}
-
-// a.N = 2 F.  A workgroup holds 16 (2 x 4 wavefronts: up block, gate block) or, once F has more 16-row blocks than the
-// device has compute units, 32 columns of h (4 x 2 wavefronts).
-static int launch_gemv_mfma_swiglu(GemvArgs a, hipStream_t st) {
-  const int F = a.N / 2;
-  const bool wide = (F + 15) / 16 > device_cus();
-  a.ksplit = wide ? 2 : 4;
-  a.groups = wide ? 4 : 2;
-  const int per_wg = GM_ROWS * (a.groups / 2);
-  const unsigned grid = (unsigned)((F + per_wg - 1) / per_wg);
-  const size_t lds = (size_t)16 * (a.K + 16) + 16 * sizeof(float) + 16;
-  const bool many = a.M > 8, norm = a.gamma != nullptr;
-  using kern_t = void (*)(GemvArgs);
-#define AQ_SWI_TABLE(KS, GR)                                                                                   \
-  {{gemv_mfma_kernel<KS, GR, false, 1, 8, false, false, true>, gemv_mfma_kernel<KS, GR, false, 1, 8, true, false, true>},   \
-   {gemv_mfma_kernel<KS, GR, false, 1, 16, false, false, true>, gemv_mfma_kernel<KS, GR, false, 1, 16, true, false, true>}}
-  static const kern_t table[2][2][2] = {AQ_SWI_TABLE(4, 2), AQ_SWI_TABLE(2, 4)};
-#undef AQ_SWI_TABLE
-  hipLaunchKernelGGL(table[wide][many][norm], dim3(grid), dim3(8 * 64), lds, st, a);
-  return (int)hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -1232,44 +917,51 @@ static int gemv_dispatch(const aq::GemvArgs& a, int mt, hipStream_t st) {
   }
 }
 
-// One launch for up to 8 bf16 rows that fit the in-kernel quantiser's register
-// budget; returns -1 when the shape has to take the two-launch path.  With more
-// than 8 rows every workgroup would repeat 2+ row quantisations per wavefront
-// on its critical path, which measures no faster than the separate launch.
-static int gemv_dispatch_fused(const aq::GemvArgs& a, int mt, hipStream_t st) {
-  if (aq::gemv_mfma_fq_ok(a.M, a.N, a.K, a.gamma != nullptr)) return aq::launch_gemv_mfma_fq(a, st);
+// One launch where a kernel quantises (and normalises) the rows itself; -1 when the shape takes two.
+// Up to 4 bf16 rows, the dot-product kernel: one wavefront rounds a row, the others start on their weights, and the few
+// products per weight dword are no load on the vector ALU (1 x 2048 -> 8192: 5.1 us against 5.8, 4 x 5712 -> 4832 9.6
+// against 10.7).  gemv_rows.hip for everything else: more rows; fp32 rows; 3 or 4 rows of a matrix of at most 2048 rows
+// (4 x 1536 -> 1536 3.44 -> 3.28) or of more than 8192, which the dot-product kernel walks in two and more rounds of
+// workgroups that repeat the rounding (4 x 1840 -> 9152 6.9 -> 6.6), any number of long ones there (1 x 8192 -> 11264
+// 23.8 -> 19.3), and the norm in front of a matrix of at most 4096 rows (4 x 1536 -> 2048 4.07 -> 3.70).
+static bool dot_kernel_better(int64_t M, int64_t N, int64_t K, bool norm) {
+  if (M > 4) return false;
+  if (norm) return N > 4096 && (M < 3 || N <= 8192);
+  if (N > 8192) return M < 3 && K <= 4096;
+  return M < 3 || N > 2048;
+}
+
+static int gemv_dispatch_fused(const aq::GemvArgs& a, int x_dtype, int mt, hipStream_t st) {
+  const bool norm = a.gamma != nullptr, bf16 = x_dtype == AQ_BF16;
   const int64_t vpl = (a.K / 8 + 63) / 64;  // 16-byte vectors per lane per bf16 row
-  if (mt > 8 || vpl > 16) return -1;
+  const bool dot = bf16 && a.M <= 4 && mt > 0 && vpl <= (norm ? 4 : 16);
+  const aq::RowsKind kind = norm ? aq::ROWS_I8_NORM : bf16 ? aq::ROWS_I8 : aq::ROWS_I8_F32;
+  if ((bf16 || !norm) && aq::gemv_rows_ok(kind, a.M, a.K) && !(dot && dot_kernel_better(a.M, a.N, a.K, norm)))
+    return aq::launch_gemv_rows(a, kind, st);
+  if (!dot) return -1;
   // A short matrix with long rows (an MLP's down projection): with whole rows per wavefront its N / 32 workgroups
-  // would leave most compute units without loads in flight (N = 2048, K = 5632, 8 rows: 11.0 us against 9.1 for
-  // the separate row quantiser + the K-split GEMV on codes).  The fused kernel with 4 K parts -- 8 weight rows per
-  // workgroup, every wavefront rounding one token row first -- is the fastest form: 8.6 -> 7.15 us for that shape,
-  // 8.0 -> 5.7 us for 4 rows of 6912 against 1536 weight rows, 7.0 -> 4.8 us for one row of 5632 (2 parts: 8.0,
-  // 8 parts: 12.1 us).  With the norm in front (rows stay short there) the two launches remain.
-  if ((a.N + 31) / 32 * 4 <= aq::device_cus() && (a.K > 4096 || (a.M > 4 && a.K >= 4096))) {
-    if (a.gamma) return -1;
+  // would leave most compute units without loads in flight.  4 K parts -- 8 weight rows per workgroup, every wavefront
+  // rounding one token row first: 7.0 -> 4.8 us for one row of 5632 against 2048 weight rows (2 parts: 8.0, 8 parts:
+  // 12.1 us for 8 rows).
+  if (!norm && (a.N + 31) / 32 * 4 <= aq::device_cus() && a.K > 4096) {
     switch (mt) {
       case 1: return aq::launch_gemv_fw<1, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
       case 2: return aq::launch_gemv_fw<2, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
-      case 4: return aq::launch_gemv_fw<4, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
-      default: return aq::launch_gemv_fw<8, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
+      default: return aq::launch_gemv_fw<4, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
     }
   }
   const bool small = vpl <= 4;
-  if (a.gamma) {  // with the norm in front: short rows only (the gain's vectors stay in registers too)
-    if (!small) return -1;
+  if (norm) {
     switch (mt) {
       case 1: return aq::launch_gemv<1, true, 4, true>(a, st);
       case 2: return aq::launch_gemv<2, true, 4, true>(a, st);
-      case 4: return aq::launch_gemv<4, true, 4, true>(a, st);
-      default: return aq::launch_gemv<8, true, 4, true>(a, st);
+      default: return aq::launch_gemv<4, true, 4, true>(a, st);
     }
   }
   switch (mt) {
     case 1: return small ? aq::launch_gemv<1, true, 4>(a, st) : aq::launch_gemv<1, true, 16>(a, st);
     case 2: return small ? aq::launch_gemv<2, true, 4>(a, st) : aq::launch_gemv<2, true, 16>(a, st);
-    case 4: return small ? aq::launch_gemv<4, true, 4>(a, st) : aq::launch_gemv<4, true, 16>(a, st);
-    default: return small ? aq::launch_gemv<8, true, 4>(a, st) : aq::launch_gemv<8, true, 16>(a, st);
+    default: return small ? aq::launch_gemv<4, true, 4>(a, st) : aq::launch_gemv<4, true, 16>(a, st);
   }
 }
 
@@ -1316,7 +1008,7 @@ extern "C" int aq_gemv_w8a8_decode_residual(const void* x, int x_dtype, const in
   if (!x || !ws) return AQ_E_NULL;
   if (aq::check_ptr16(x) || aq::check_ptr16(ws)) return AQ_E_ALIGN;
   if (ws_bytes < aq_gemv_w8a8_workspace_bytes(M, K)) return AQ_E_WORKSPACE;
-  if (x_dtype == AQ_BF16 && mt > 0) {  // one launch: the GEMV kernel quantises the rows itself
+  {  // one launch where the GEMV kernel quantises the rows itself
     aq::GemvArgs a{};
     a.x = x;
     a.wq = wq;
@@ -1330,7 +1022,7 @@ extern "C" int aq_gemv_w8a8_decode_residual(const void* x, int x_dtype, const in
     a.K = (int)K;
     a.bias_dtype = bias_dtype;
     a.y_dtype = y_dtype;
-    const int frc = gemv_dispatch_fused(a, mt, static_cast<hipStream_t>(stream));
+    const int frc = gemv_dispatch_fused(a, x_dtype, mt, static_cast<hipStream_t>(stream));
     if (frc >= 0) return frc;
   }
   int8_t* xq = static_cast<int8_t*>(ws);
@@ -1403,10 +1095,10 @@ extern "C" int aq_gemv_fp8_decode_residual(const void* x, int x_dtype, const uin
   if (!x || !ws) return AQ_E_NULL;
   if (aq::check_ptr16(x) || aq::check_ptr16(ws)) return AQ_E_ALIGN;
   if (ws_bytes < aq_gemv_fp8_workspace_bytes(M, K)) return AQ_E_WORKSPACE;
-  if (x_dtype == AQ_BF16 && K <= 2048 && (K % 512) == 0) {  // one launch: the kernel casts the rows itself
+  if (x_dtype == AQ_BF16 && aq::gemv_rows_ok(aq::ROWS_FP8, M, K)) {  // one launch: the kernel casts the rows itself
     aq::GemvArgs a = gemv_fp8_args(wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K);
     a.x = x;
-    return aq::launch_gemv_mfma_fq(a, static_cast<hipStream_t>(stream), true);
+    return aq::launch_gemv_rows(a, aq::ROWS_FP8, static_cast<hipStream_t>(stream));
   }
   uint8_t* xq = static_cast<uint8_t*>(ws);
   float* sx = reinterpret_cast<float*>(static_cast<char*>(ws) + aq::align256((size_t)(M * K)));
@@ -1511,7 +1203,7 @@ extern "C" int aq_gemv_w8a8_decode_rmsnorm(const void* x, int x_dtype, const voi
   if (!x || !gamma || !ws) return AQ_E_NULL;
   if (aq::check_ptr16(x) || aq::check_ptr16(gamma) || aq::check_ptr16(ws)) return AQ_E_ALIGN;
   if (ws_bytes < aq_gemv_w8a8_workspace_bytes(M, K)) return AQ_E_WORKSPACE;
-  if (x_dtype == AQ_BF16 && mt > 0) {  // one launch: the GEMV kernel normalises and quantises the rows itself
+  {  // one launch where the GEMV kernel normalises and quantises the rows itself
     aq::GemvArgs a{};
     a.x = x;
     a.gamma = gamma;
@@ -1527,7 +1219,7 @@ extern "C" int aq_gemv_w8a8_decode_rmsnorm(const void* x, int x_dtype, const voi
     a.K = (int)K;
     a.bias_dtype = bias_dtype;
     a.y_dtype = y_dtype;
-    const int frc = gemv_dispatch_fused(a, mt, static_cast<hipStream_t>(stream));
+    const int frc = gemv_dispatch_fused(a, x_dtype, mt, static_cast<hipStream_t>(stream));
     if (frc >= 0) return frc;
   }
   int8_t* xq = static_cast<int8_t*>(ws);
@@ -1538,7 +1230,7 @@ extern "C" int aq_gemv_w8a8_decode_rmsnorm(const void* x, int x_dtype, const voi
 }
 
 extern "C" int aq_gemv_w8a8_decode_swiglu_ok(int x_dtype, int64_t M, int64_t F, int64_t K) {
-  return x_dtype == AQ_BF16 && aq::gemv_mfma_swiglu_ok(M, F, K) ? 1 : 0;
+  return x_dtype == AQ_BF16 && aq::gemv_swiglu_ok(M, F, K) ? 1 : 0;
 }
 
 extern "C" int aq_gemv_w8a8_decode_swiglu(const void* x, int x_dtype, const void* gamma, float eps, const int8_t* wq,
@@ -1565,7 +1257,7 @@ extern "C" int aq_gemv_w8a8_decode_swiglu(const void* x, int x_dtype, const void
   a.K = (int)K;
   a.bias_dtype = bias_dtype;
   a.y_dtype = h_dtype;
-  return aq::launch_gemv_mfma_swiglu(a, static_cast<hipStream_t>(stream));
+  return aq::launch_gemv_rows_swiglu(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int aq_gemv_w8a8_decode(const void* x, int x_dtype, const int8_t* wq, const float* sw,
@@ -1574,13 +1266,3 @@ extern "C" int aq_gemv_w8a8_decode(const void* x, int x_dtype, const int8_t* wq,
   return aq_gemv_w8a8_decode_residual(x, x_dtype, wq, sw, bias, bias_dtype, nullptr, y, y_dtype, M, N, K, ws, ws_bytes,
                                       stream);
 }
-
-#ifdef AQ_LAB
-// Lab build only (see aq_lab.h): the buffer the matrix-core GEMV's wavefronts leave their time stamps in.
-extern "C" int aq_lab_set_gemv_timeline(long long* buf) {
-  return (int)hipMemcpyToSymbol(HIP_SYMBOL(aq::gv_timeline), &buf, sizeof(buf));
-}
-extern "C" int aq_lab_set_gemv_skip_weights(int on) {
-  return (int)hipMemcpyToSymbol(HIP_SYMBOL(aq::gv_skip_weights), &on, sizeof(on));
-}
-#endif

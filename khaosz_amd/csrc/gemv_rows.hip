@@ -1,0 +1,444 @@
+// Decode path, one launch for rows of any length: a weight-streaming GEMV on the matrix core that quantises its own
+// token rows -- up to 16 of them, bf16 or fp32, K any multiple of 16 up to 8192 -- while its weights are in flight.
+// int8 (per-token scales, exact int32 sums: the bits of row quantiser + GEMV) and FP8 (e4m3, one scale per tensor,
+// fp32 sums in a fixed order), with the RMSNorm in front and the residual or the SwiGLU behind folded in.
+//
+// A workgroup of 8 wavefronts owns 8, 16, 32 or 64 weight rows: KS K parts x GR groups of R rows.  Every wavefront
+// requests its token rows, its share of the epilogue's operands and then ALL its weights (up to 16 loads of 16 bytes
+// per lane; longer parts rotate two register batches), rounds its token rows into LDS, and multiplies behind one
+// barrier; the K parts' sums meet in LDS and every thread finishes one output.
+//
+// What bounds it: at decode sizes the launch (1.8 us) and the latency of the token rows and weights, then how many
+// requests a compute unit has to take in.  The number of loads is therefore cut to the line: a kernel is built for
+// each row length class, so that no wavefront sends loads that fall outside its part.  An empty load (an offset past
+// the descriptor) returns zero without touching memory but still takes its turn in the address path: with a fixed 16
+// weight loads per lane and the epilogue's operands asked for by one wavefront in KS (20 small loads, most empty), the
+// same kernel took 1.5 to 2.5 us longer.  Measured (us, graph replay, weights from HBM, before -> now):
+//   bf16 16 x 2048 -> 8192 8.1 -> 6.5, 11 x 1536 -> 1536 5.9 -> 3.8, 8 x 2048 -> 3072 5.0 -> 3.95, 8 x 5632 -> 2048 7.3 -> 6.3;
+//   rows that took a quantiser launch of their own: 11 x 6912 -> 1536 13.6 -> 8.0, 16 x 1840 -> 9152 15.7 -> 8.9,
+//   11 x 5712 -> 4832 20.4 -> 13.8, fp32 8 x 6912 -> 1536 25 -> 8.3, 8 x 1536 -> 1536 6.7 -> 3.7;
+//   FP8 8 x 2048 -> 8192 7.4 -> 5.8, 4 x 688 -> 3520 8.7 -> 3.3, 8 x 6912 -> 1536 17.5 -> 8.4;
+//   up/gate + SwiGLU with the norm: 4 x 1536 -> 2 x 6912 7.3 -> 6.4, 8 x 2048 -> 2 x 5632 8.2 -> 7.6.
+#include <type_traits>
+
+#include "aq_common.h"
+#include "aq_gemv.h"
+#include "aq_rows.h"
+
+namespace aq {
+
+#ifdef AQ_LAB
+// Lab build only (csrc/aq_lab.h): where the wavefronts leave time stamps of the 100 MHz counter, 8 per wavefront, and a
+// switch that makes the kernel request no weight bytes (products of zeros).  The product library has neither.
+__device__ long long* gv_timeline = nullptr;
+__device__ int gv_skip_weights = 0;
+#define GV_STAMP(slot)                                                                                         \
+  do {                                                                                                         \
+    if (gv_timeline && lane == 0) gv_timeline[((size_t)blockIdx.x * 16 + wave) * 8 + (slot)] = wall_clock64(); \
+  } while (0)
+#else
+#define GV_STAMP(slot) \
+  do {                 \
+  } while (0)
+#endif
+
+constexpr int GX_WAVES = 8;  // wavefronts per workgroup
+constexpr int64_t GX_MAX_K = 8192;
+
+// KS K parts x GX_WAVES / KS groups of R weight rows.  RPW: token rows per wavefront (fp32 rows, twice as long in
+// registers, go one after the other instead), VPL: 16-byte vectors per lane and row -- together the row length class.
+// R = 8 fills half of a matrix-core operand (the other half repeats other pieces of the same rows and is not stored):
+// for short matrices, so that twice the compute units stream weights.
+// SWI: the weight is an MLP's up and gate projections stacked, rows [0, F) up and [F, 2F) gate; the first half of the
+// row groups takes rows of up, the second half the same rows of gate, and the output is up * silu(gate), the two as the
+// projections would have been stored (rounded to the output type first).
+template <int KS, int R, bool BF16, int RPW, int VPL, bool NORM, bool FP8, bool SWI = false>
+__global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
+  constexpr int GR = GX_WAVES / KS;
+  constexpr int HALVES = R / 8;                          // 8-row halves of a row group: loads per line
+  constexpr int MOST = VPL * (BF16 ? 4 : 2) / KS;        // lines of 128 bytes of a wavefront's K part, at most
+  constexpr int PART = MOST > 0 ? MOST * HALVES : HALVES;
+  constexpr int DEEP = RPW * VPL >= 32 ? 8 : 16;         // 16-byte weight loads in flight per lane, at most
+  constexpr bool LOOP = PART > DEEP;                     // longer parts rotate two register batches
+  constexpr int LOADS = LOOP ? DEEP / 2 : PART;          // loads per register batch
+  constexpr int LINES = LOADS / HALVES;                  // lines per register batch
+  static_assert(R == 8 || R == 16, "rows of one matrix-core operand, or half of them");
+  static_assert(!(FP8 && (NORM || !BF16)), "the FP8 cast takes bf16 rows as they are");
+  extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [M][pitch] token codes, [16] scales; later the partial sums
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave / KS, kh = wave % KS;
+  const int K = p.K, N = p.N, M = p.M;
+  const int nline_all = (K + 127) >> 7;
+  const int pitch = (nline_all << 7) + 16;  // 16 token rows then start 4 banks apart
+  const int per = (nline_all + KS - 1) / KS;
+  const int lbeg = kh * per, lend = lbeg + per < nline_all ? lbeg + per : nline_all;  // this wavefront's lines (none is possible)
+  const int FH = SWI ? N >> 1 : N;  // outputs per token
+  constexpr int GO = SWI ? GR / 2 : GR;
+  const int half = SWI && grp >= GO ? FH : 0;
+  const int n0 = __builtin_amdgcn_readfirstlane(half + (blockIdx.x * GO + (SWI ? grp % GO : grp)) * R);
+  const int nlim = half + FH;
+
+  // The outputs of the workgroup, GR * R weight rows of up to 16 tokens, are dealt out one to a thread (OPT of them):
+  // thread t takes row t % (GR R) of token t / (GR R).  Every wavefront then requests its share of the epilogue's
+  // operands; with four outputs per lane of one wavefront in KS, each wavefront sent out 20 small loads, most of them
+  // empty, ahead of its weights.
+  constexpr int OUT = GO * R, OPT = (OUT * 16 + GX_WAVES * 64 - 1) / (GX_WAVES * 64);
+  const int tok = lane & 15;  // of the products
+  const int b0 = blockIdx.x * OUT;
+  float swv[OPT], bv[OPT], swg[SWI ? OPT : 1], bg[SWI ? OPT : 1], sxv = 1.0f;
+  uint32_t rv[OPT];
+  const EpiOperands epi(p, true, false, !SWI);
+  auto load_epi = [&]() {
+#pragma unroll
+    for (int i = 0; i < OPT; ++i) {
+      const int t = tid + i * GX_WAVES * 64;
+      const int m = t / OUT, n = b0 + t % OUT;
+      const bool ok = m < M && n < FH;
+      swv[i] = epi.load_sw(FP8 ? 0 : n, FP8 || ok);
+      bv[i] = epi.load_bias(n, ok);
+      if constexpr (SWI) {
+        swg[i] = epi.load_sw(FH + n, ok);
+        bg[i] = epi.load_bias(FH + n, ok);
+      } else {
+        rv[i] = epi.load_res(m, n, ok, (int)p.ldr);
+      }
+    }
+  };
+
+  // weight stream: an instruction covers one line of 8 rows (lane l: row l % 8, 16-byte piece l / 8)
+  const int rows = n0 < nlim ? ((nlim - n0) < R ? (nlim - n0) : R) : 0;
+#ifdef AQ_LAB
+  const __amdgpu_buffer_rsrc_t Wr = make_rsrc(p.wq + (int64_t)(n0 < nlim ? n0 : 0) * K, gv_skip_weights ? 0u : (uint32_t)rows * (uint32_t)K);
+#else
+  const __amdgpu_buffer_rsrc_t Wr = make_rsrc(p.wq + (int64_t)(n0 < nlim ? n0 : 0) * K, (uint32_t)rows * (uint32_t)K);
+#endif
+  const uint32_t woff = (uint32_t)(lane & 7) * (uint32_t)K, woff8 = 8u * (uint32_t)K;
+  const int piece = (lane >> 3) * 16;
+  uint4 wa[LOADS], wb[LOOP ? LOADS : 1];
+  auto wload = [&](int line0, uint4* dst) {
+#pragma unroll
+    for (int t = 0; t < LINES; ++t) {
+      const int kb = (line0 + t) * 128 + piece;
+      const bool ok = (line0 + t) < lend && kb < K;  // past K the offset would alias the next row
+      const uint32_t o = woff + (uint32_t)kb;
+      dst[t * HALVES] = buffer_load_16_stream(Wr, ok ? o : OOB_OFFSET);
+      if constexpr (HALVES == 2) dst[t * HALVES + 1] = buffer_load_16_stream(Wr, ok ? o + woff8 : OOB_OFFSET);
+    }
+  };
+
+  float* const sx_lds = reinterpret_cast<float*>(xs + M * pitch);
+  GV_STAMP(0);
+  if constexpr (BF16) {
+    RowsToLds<true, RPW, VPL> xr;
+    xr.issue(p.x, M, K, K, wave, GX_WAVES, lane);
+    if constexpr (NORM) xr.issue_gamma(p.gamma, K, lane);
+    asm volatile("" ::: "memory");  // request order: token rows, epilogue operands, the weight stream
+    load_epi();
+    asm volatile("" ::: "memory");
+    wload(lbeg, wa);
+    if constexpr (LOOP) wload(lbeg + LINES, wb);
+    asm volatile("" ::: "memory");
+    if constexpr (!FP8) {
+      xr.template finish<NORM>(M, M, K, xs, pitch, sx_lds, wave, GX_WAVES, lane, p.eps);
+    } else {
+      float amax = 0.0f;
+#pragma unroll
+      for (int j = 0; j < RPW; ++j)
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+          float f[8];
+          RowIn<true>::unpack(xr.c[j][i], f);  // rows >= M and vectors past K were loaded as zeros
+          amax = fmaxf(amax, vec_amax<8>(f));
+        }
+      amax = wave_max(amax);
+      if (lane == 0) sx_lds[wave] = amax;
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();  // no memory fence: the weight loads stay in flight
+      asm volatile("" ::: "memory");
+      float all = 0.0f;
+#pragma unroll
+      for (int w = 0; w < GX_WAVES; ++w) all = fmaxf(all, sx_lds[w]);
+      float sc = __fdiv_rn(all, 448.0f);
+      if (all == 0.0f) sc = 1.0f;
+      sxv = sc;
+      const float rsc = __fdiv_rn(1.0f, sc);
+      const bool lean_ok = sc >= 5.421010862427522e-20f && sc <= 1.8446744073709552e19f;  // [2^-64, 2^64]
+      const int nvec = K / 8;
+#pragma unroll
+      for (int j = 0; j < RPW; ++j) {
+        const int m = wave + j * GX_WAVES;
+        if (m >= M) continue;  // uniform
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+          const int v = i * 64 + lane;
+          if (v < nvec) {
+            float f[8];
+            RowIn<true>::unpack(xr.c[j][i], f);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              // x / s as in the stand-alone cast: one correction with the correctly rounded reciprocal
+              float q;
+              if (__builtin_expect(lean_ok, 1)) {
+                q = f[e] * rsc;
+                q = __builtin_fmaf(__builtin_fmaf(-sc, q, f[e]), rsc, q);
+              } else {
+                q = __fdiv_rn(f[e], sc);
+              }
+              f[e] = fminf(fmaxf(q, -448.0f), 448.0f);
+            }
+            int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+            w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w0, true);
+            int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], 0, false);
+            w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], w1, true);
+            *reinterpret_cast<uint2*>(xs + m * pitch + v * 8) = make_uint2((uint32_t)w0, (uint32_t)w1);
+          }
+        }
+      }
+    }
+  } else {
+    // fp32 rows are twice as long in registers: one row of the wavefront at a time
+    {
+      RowsToLds<false, 1, VPL> xr;
+      xr.issue(p.x, M, K, K, wave, GX_WAVES, lane);
+      asm volatile("" ::: "memory");
+      load_epi();
+      asm volatile("" ::: "memory");
+      wload(lbeg, wa);
+      if constexpr (LOOP) wload(lbeg + LINES, wb);
+      asm volatile("" ::: "memory");
+      xr.template finish<false>(M, M, K, xs, pitch, sx_lds, wave, GX_WAVES, lane);
+    }
+    if (wave + GX_WAVES < M) {
+      RowsToLds<false, 1, VPL> xr;
+      xr.issue(p.x, M, K, K, wave + GX_WAVES, GX_WAVES, lane);
+      xr.template finish<false>(M, M, K, xs, pitch, sx_lds, wave + GX_WAVES, GX_WAVES, lane);
+    }
+  }
+  // the rest of a last, partly filled line: products with the zeros the weight loads answer there
+  for (int m = wave; m < M; m += GX_WAVES)
+    if (lane * 16 < pitch - 16 - K) *reinterpret_cast<uint4*>(xs + m * pitch + K + lane * 16) = make_uint4(0, 0, 0, 0);
+  GV_STAMP(3);
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();  // no memory fence: the weight loads stay in flight
+  asm volatile("" ::: "memory");
+  GV_STAMP(4);
+  float sxo[OPT];
+#pragma unroll
+  for (int i = 0; i < OPT; ++i) {
+    const int m = (tid + i * GX_WAVES * 64) / OUT;
+    sxo[i] = FP8 ? sxv : sx_lds[m < M ? m : 0];
+  }
+
+  using accv = std::conditional_t<FP8, v4f, v4i>;
+  accv accs[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) accs[i] = accv{0, 0, 0, 0};
+  const uint8_t* xl = xs + (tok < M ? tok : 0) * pitch + (lane >> 4) * 32;
+  constexpr int ROR8 = 0x128;  // DPP row_ror:8
+  constexpr int STEP = LINES < 4 ? LINES : 4;
+  auto consume = [&](int line0, const uint4* wc) {
+#pragma unroll
+    for (int t0 = 0; t0 < LINES; t0 += STEP) {
+      v4i x[2 * STEP];
+#pragma unroll
+      for (int t = 0; t < STEP; ++t) {
+        const int ln = (line0 + t0 + t) < lend ? (line0 + t0 + t) : 0;  // lines past the end multiply zero weights
+        x[2 * t] = *reinterpret_cast<const v4i*>(xl + ln * 128);
+        x[2 * t + 1] = *reinterpret_cast<const v4i*>(xl + ln * 128 + 16);
+      }
+#pragma unroll
+      for (int t = 0; t < STEP; ++t) {
+        const uint4 lo = wc[(t0 + t) * HALVES];
+        v4i w0, w1;
+        if constexpr (HALVES == 2) {
+          const uint4 hi = wc[(t0 + t) * HALVES + 1];
+          // lanes 8..15 of each row take hi from lane l - 8 (w0), lanes 0..7 take lo from lane l + 8 (w1)
+          w0 = v4i{__builtin_amdgcn_update_dpp((int)lo.x, (int)hi.x, ROR8, 0xf, 0xc, false),
+                   __builtin_amdgcn_update_dpp((int)lo.y, (int)hi.y, ROR8, 0xf, 0xc, false),
+                   __builtin_amdgcn_update_dpp((int)lo.z, (int)hi.z, ROR8, 0xf, 0xc, false),
+                   __builtin_amdgcn_update_dpp((int)lo.w, (int)hi.w, ROR8, 0xf, 0xc, false)};
+          w1 = v4i{__builtin_amdgcn_update_dpp((int)hi.x, (int)lo.x, ROR8, 0xf, 0x3, false),
+                   __builtin_amdgcn_update_dpp((int)hi.y, (int)lo.y, ROR8, 0xf, 0x3, false),
+                   __builtin_amdgcn_update_dpp((int)hi.z, (int)lo.z, ROR8, 0xf, 0x3, false),
+                   __builtin_amdgcn_update_dpp((int)hi.w, (int)lo.w, ROR8, 0xf, 0x3, false)};
+        } else {
+          // the operand's rows 8..15 repeat other pieces of rows 0..7: their products are never stored
+          w0 = v4i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w};
+          w1 = v4i{__builtin_amdgcn_update_dpp(0, (int)lo.x, ROR8, 0xf, 0xf, false),
+                   __builtin_amdgcn_update_dpp(0, (int)lo.y, ROR8, 0xf, 0xf, false),
+                   __builtin_amdgcn_update_dpp(0, (int)lo.z, ROR8, 0xf, 0xf, false),
+                   __builtin_amdgcn_update_dpp(0, (int)lo.w, ROR8, 0xf, 0xf, false)};
+        }
+        if constexpr (!FP8) {
+          accs[(2 * t) & 3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, x[2 * t], accs[(2 * t) & 3], 0, 0, 0);
+          accs[(2 * t + 1) & 3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, x[2 * t + 1], accs[(2 * t + 1) & 3], 0, 0, 0);
+        } else {
+          const v8i wl = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+          const v4i xa = x[2 * t], xb = x[2 * t + 1];
+          const v8i xl8 = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+          accs[t & 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wl, xl8, accs[t & 3], 0, 0, 0, 0, 0, 0);
+        }
+      }
+    }
+  };
+  if constexpr (!LOOP) {
+    consume(lbeg, wa);
+  } else {
+    for (int l0 = lbeg; l0 < lend; l0 += 2 * LINES) {
+      consume(l0, wa);
+      if (l0 + 2 * LINES < lend) wload(l0 + 2 * LINES, wa);
+      if (l0 + LINES < lend) consume(l0 + LINES, wb);
+      if (l0 + 3 * LINES < lend) wload(l0 + 3 * LINES, wb);
+    }
+  }
+  const accv acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
+  GV_STAMP(5);
+  // the K parts' sums meet in LDS: [K part][token][row of the workgroup]
+  __syncthreads();  // everyone is done reading the token codes: the buffer is reused
+  using acct = std::conditional_t<FP8, float, int>;
+  acct* const part = reinterpret_cast<acct*>(xs);
+  if (R == 16 || lane < 32)
+    *reinterpret_cast<accv*>(part + (kh * 16 + tok) * (GR * R) + grp * R + (lane >> 4) * 4) = acc;  // lane: 4 rows of a token
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < OPT; ++i) {
+    const int t = tid + i * GX_WAVES * 64;
+    const int m = t / OUT, n = b0 + t % OUT;
+    if (m >= M || n >= FH) continue;
+    const acct* const mine = part + m * (GR * R) + t % OUT;
+    acct sum = mine[0];
+#pragma unroll
+    for (int k = 1; k < KS; ++k) sum += mine[k * 16 * GR * R];  // fp32: a fixed order
+    float y = __fmul_rn(__fmul_rn((float)sum, sxo[i]), swv[i]);
+    if (p.bias) y = __fadd_rn(y, bv[i]);
+    if constexpr (SWI) {
+      acct gsum = mine[OUT];
+#pragma unroll
+      for (int k = 1; k < KS; ++k) gsum += mine[k * 16 * GR * R + OUT];
+      float g = __fmul_rn(__fmul_rn((float)gsum, sxo[i]), swg[i]);
+      if (p.bias) g = __fadd_rn(g, bg[i]);
+      if (p.y_dtype == AQ_BF16) {  // as the two projections would be stored
+        y = bf16_bits_to_f32(f32_to_bf16_bits(y));
+        g = bf16_bits_to_f32(f32_to_bf16_bits(g));
+      }
+      y = swiglu_repro(y, g);
+    } else if (p.res) y = p.y_dtype == AQ_BF16 ? add_residual_bf16(y, rv[i]) : __fadd_rn(y, __uint_as_float(rv[i]));
+    const int64_t o = (int64_t)m * FH + n;
+    if (p.y_dtype == AQ_BF16)
+      reinterpret_cast<uint16_t*>(p.y)[o] = (uint16_t)f32_to_bf16_bits(y);
+    else
+      reinterpret_cast<float*>(p.y)[o] = y;
+  }
+  GV_STAMP(6);
+}
+
+static size_t gemv_rows_lds(int64_t M, int64_t K, int ks, int rows_per_wg) {
+  const size_t codes = (size_t)M * (((K + 127) / 128) * 128 + 16) + 16 * sizeof(float);
+  const size_t sums = (size_t)ks * 16 * rows_per_wg * 4;  // come to lie over the codes
+  return codes < sums ? sums : codes;
+}
+
+// Weight rows per workgroup.  A workgroup's time grows with the token rows it rounds and with the weight rows it streams, a
+// token row costing as much as 7/4 weight rows of the same length (46 and 26 ps per element, fitted to 14 shapes x 5
+// batches x 4 row counts), and a round of workgroups over the compute units repeats the rounding: the fewest rounds x
+// (7 M + 4 rows).  Within 10 % of the best of the four at every point measured.
+static int rows_per_workgroup(int64_t M, int64_t N, int least, int most) {
+  const int64_t cus = device_cus();
+  int best = most;
+  int64_t cost = INT64_MAX;
+  for (int r = least; r <= most; r *= 2) {
+    const int64_t c = ((N + r - 1) / r + cus - 1) / cus * (7 * M + 4 * r);
+    if (c < cost) cost = c, best = r;
+  }
+  return best;
+}
+
+using rows_kernel_t = void (*)(GemvArgs);
+
+static int launch_rows(rows_kernel_t fn, LdsOptIn& opted, const GemvArgs& a, int ks, int rows_per_wg, int64_t outputs, int outputs_per_wg,
+                       hipStream_t st) {
+  const size_t lds = gemv_rows_lds(a.M, a.K, ks, rows_per_wg);
+  if (lds > 64 * 1024) {
+    const int e = opted.ensure(reinterpret_cast<const void*>(fn));
+    if (e) return e;
+  }
+  const unsigned grid = (unsigned)((outputs + outputs_per_wg - 1) / outputs_per_wg);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(GX_WAVES * 64), lds, st, a);
+  return (int)hipGetLastError();
+}
+
+// the row length class: vectors per lane of a row, rounded up to what kernels are built for
+static int length_class(int64_t vectors) { return vectors <= 128 ? 0 : vectors <= 256 ? 1 : vectors <= 512 ? 2 : 3; }
+
+template <int KS, int R>
+static int launch_shape(const GemvArgs& a, RowsKind kind, hipStream_t st) {
+#define AQ_GX(RPW, FP8)                                                                                   \
+  {gemv_rows_kernel<KS, R, true, RPW, 2, false, FP8>, gemv_rows_kernel<KS, R, true, RPW, 4, false, FP8>,  \
+   gemv_rows_kernel<KS, R, true, RPW, 8, false, FP8>, gemv_rows_kernel<KS, R, true, RPW, 16, false, FP8>}
+  static const rows_kernel_t i8[2][4] = {AQ_GX(1, false), AQ_GX(2, false)};
+#undef AQ_GX
+  // (16 rows of more than 4096 cannot stay in registers between the tensor's maximum and the cast: gemv_rows_ok)
+  static const rows_kernel_t f8[2][4] = {
+      {gemv_rows_kernel<KS, R, true, 1, 2, false, true>, gemv_rows_kernel<KS, R, true, 1, 4, false, true>,
+       gemv_rows_kernel<KS, R, true, 1, 8, false, true>, gemv_rows_kernel<KS, R, true, 1, 16, false, true>},
+      {gemv_rows_kernel<KS, R, true, 2, 2, false, true>, gemv_rows_kernel<KS, R, true, 2, 4, false, true>,
+       gemv_rows_kernel<KS, R, true, 2, 8, false, true>, nullptr}};
+  static const rows_kernel_t norm[2][2] = {
+      {gemv_rows_kernel<KS, R, true, 1, 2, true, false>, gemv_rows_kernel<KS, R, true, 1, 4, true, false>},
+      {gemv_rows_kernel<KS, R, true, 2, 2, true, false>, gemv_rows_kernel<KS, R, true, 2, 4, true, false>}};
+  static const rows_kernel_t f32[3] = {gemv_rows_kernel<KS, R, false, 1, 4, false, false>,
+                                       gemv_rows_kernel<KS, R, false, 1, 8, false, false>,
+                                       gemv_rows_kernel<KS, R, false, 1, 32, false, false>};
+  static LdsOptIn opted[2][4][4];
+  const int two = a.M > 8, len = length_class(a.K / (kind == ROWS_I8_F32 ? 4 : 8));
+  const int flen = a.K <= 1024 ? 0 : a.K <= 2048 ? 1 : 2;
+  const rows_kernel_t fn = kind == ROWS_I8_F32    ? f32[flen]
+                           : kind == ROWS_I8_NORM ? norm[two][len]
+                           : kind == ROWS_FP8     ? f8[two][len]
+                                                  : i8[two][len];
+  return launch_rows(fn, opted[two][kind][kind == ROWS_I8_F32 ? flen : len], a, KS, GX_WAVES / KS * R, a.N, GX_WAVES / KS * R, st);
+}
+
+bool gemv_rows_ok(RowsKind kind, int64_t M, int64_t K) {
+  if (M < 1 || M > 16 || K > GX_MAX_K) return false;
+  if (kind == ROWS_I8_NORM) return K <= 2048;      // the gain's vectors stay in registers next to the rows'
+  if (kind == ROWS_FP8) return M <= 8 || K <= 4096;
+  return true;
+}
+
+int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {
+  switch (rows_per_workgroup(a.M, a.N, 8, 64)) {
+    case 8: return launch_shape<8, 8>(a, kind, st);
+    case 16: return launch_shape<8, 16>(a, kind, st);
+    case 32: return launch_shape<4, 16>(a, kind, st);
+    default: return launch_shape<2, 16>(a, kind, st);
+  }
+}
+
+// a.N = 2 F; K <= 2048
+int launch_gemv_rows_swiglu(const GemvArgs& a, hipStream_t st) {
+#define AQ_GX(KS, RPW, NORM) \
+  {gemv_rows_kernel<KS, 16, true, RPW, 2, NORM, false, true>, gemv_rows_kernel<KS, 16, true, RPW, 4, NORM, false, true>}
+#define AQ_GX2(KS) {{AQ_GX(KS, 1, false), AQ_GX(KS, 1, true)}, {AQ_GX(KS, 2, false), AQ_GX(KS, 2, true)}}
+  static const rows_kernel_t table[2][2][2][2] = {AQ_GX2(4), AQ_GX2(2)};
+#undef AQ_GX2
+#undef AQ_GX
+  static LdsOptIn unused;  // rows of at most 2048: never more than 64 KiB
+  const int r = rows_per_workgroup(a.M, a.N, 32, 64);
+  return launch_rows(table[r == 64][a.M > 8][a.gamma != nullptr][a.K > 1024], unused, a, r == 64 ? 2 : 4, r, a.N / 2, r / 2, st);
+}
+
+}  // namespace aq
+
+#ifdef AQ_LAB
+// Lab build only (see aq_lab.h).
+extern "C" int aq_lab_set_gemv_timeline(long long* buf) {
+  return (int)hipMemcpyToSymbol(HIP_SYMBOL(aq::gv_timeline), &buf, sizeof(buf));
+}
+extern "C" int aq_lab_set_gemv_skip_weights(int on) {
+  return (int)hipMemcpyToSymbol(HIP_SYMBOL(aq::gv_skip_weights), &on, sizeof(on));
+}
+#endif

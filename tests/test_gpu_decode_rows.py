@@ -1,0 +1,83 @@
+"""The decode GEMV that quantises rows of any length (csrc/gemv_rows.hip), where its tiles can go wrong: rows that are not
+whole 128-byte lines, the ends of its row length classes, batches on both sides of 8, matrices that end inside a
+workgroup of each height, 16-bit and 32-bit rows, int8 and FP8 -- against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from khaosz_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+def _bits(t):
+    return t.detach().cpu().contiguous().view(torch.int16).numpy().view(np.uint16)
+
+
+def _rows(M, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(M, K, generator=g) * (0.2 + 3 * torch.rand(M, 1, generator=g))
+
+
+# N against workgroups of 8, 16, 32 and 64 rows on 256 compute units; K at line and class edges
+CASES = [(5, 1, 16), (8, 9, 112), (9, 33, 128), (16, 7, 144), (1, 2049, 1024), (4, 2047, 1040), (16, 2056, 2032), (11, 4097, 2048),
+         (7, 8201, 2064), (16, 8193, 528), (9, 1537, 4096), (16, 520, 4112), (3, 9000, 4128), (12, 100, 8176), (16, 16, 8192),
+         (2, 8208, 8192), (6, 16385, 272)]
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("M,N,K", CASES)
+def test_int8_rows_bit_exact(oracle, M, N, K, dtype):
+    x = _rows(M, K, M + K).to(dtype)
+    wq = torch.randint(-127, 128, (N, K), generator=torch.Generator().manual_seed(N), dtype=torch.int8)
+    sw = torch.rand(N, generator=torch.Generator().manual_seed(N + 1)) * 1e-3
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(2)) * 0.1
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(3)).to(dtype)
+    args = x.to(DEV), wq.to(DEV), sw.to(DEV), bias.to(DEV)
+    y = ops.gemv_w8a8_decode(*args)
+    bf = dtype == BF16
+    want = oracle.c_linear_w8a8(_bits(x) if bf else x.numpy(), wq.numpy(), sw.numpy(), bias.numpy(), x_bf16_bits=bf, bf16_out=bf)
+    got = _bits(y) if bf else y.cpu().numpy()
+    assert np.array_equal(got.view(np.uint16 if bf else np.uint32), want.view(np.uint16 if bf else np.uint32))
+    assert torch.equal(ops.gemv_w8a8_decode(*args, residual=res.to(DEV)), y + res.to(DEV))
+
+
+@pytest.mark.parametrize("M,N,K", [c for c in CASES if c[2] <= 2048])
+def test_norm_in_front_bit_exact(oracle, M, N, K):
+    x = _rows(M, K, M + K).to(BF16)
+    gam = (1 + 0.2 * torch.randn(K, generator=torch.Generator().manual_seed(4))).to(BF16)
+    wq = torch.randint(-127, 128, (N, K), generator=torch.Generator().manual_seed(N), dtype=torch.int8)
+    sw = torch.rand(N, generator=torch.Generator().manual_seed(N + 1)) * 1e-3
+    y = ops.gemv_w8a8_decode(x.to(DEV), wq.to(DEV), sw.to(DEV), norm=(gam.to(DEV), 1e-5))
+    qx, sx = oracle.c_rmsnorm_quant_i8(_bits(x), _bits(gam), 1e-5, bf16_bits=True)
+    want = oracle.c_dequant_epilogue(oracle.c_gemm_i8_i32(qx, wq.numpy()), sx, sw.numpy(), None, bf16_out=True)
+    assert np.array_equal(_bits(y), want)
+
+
+@pytest.mark.parametrize("M,N,K", CASES)
+def test_fp8_rows_within_tolerance(oracle, M, N, K):
+    """Codes that differ by one, a lost line, or NaN codes read behind a row's end would be far outside 1e-3 of the rms."""
+    x = _rows(M, K, M + K).to(BF16)
+    w = _rows(N, K, N) * 0.02
+    xq, sx = oracle.c_quant_tensor_fp8(_bits(x), bf16_bits=True)
+    wq, sw = oracle.c_quant_tensor_fp8(w.numpy())
+    y = ops.gemv_fp8_decode(x.to(DEV), torch.from_numpy(wq).to(DEV), torch.tensor([sw], device=DEV), out_dtype=F32).cpu().numpy()
+    exact = oracle.np_linear_fp8(xq, sx, wq, sw)
+    assert np.max(np.abs(y - exact)) <= 1e-3 * np.sqrt(np.mean(exact.astype(np.float64) ** 2))
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("M,F,K", [(1, 16, 512), (8, 48, 1024), (9, 4112, 512), (16, 6912, 1536), (5, 5632, 2048)])
+def test_up_gate_swiglu_is_the_separate_launches(M, F, K, norm):
+    g = torch.Generator(device=DEV).manual_seed(M + F)
+    x = torch.randn(M, K, generator=g, device=DEV).to(BF16)
+    wq = torch.randint(-127, 128, (2 * F, K), generator=g, device=DEV, dtype=torch.int8)
+    sw = torch.rand(2 * F, generator=g, device=DEV) * 1e-3
+    nm = ((1 + 0.2 * torch.randn(K, generator=g, device=DEV)).to(BF16), 1e-5) if norm else None
+    h = ops.gemv_w8a8_decode_swiglu(x, wq, sw, norm=nm)
+    ug = ops.gemv_w8a8_decode(x, wq, sw, norm=nm).float()
+    u, gate = ug[:, :F], ug[:, F:]
+    want = u * (gate / (1 + torch.exp(-gate)))
+    assert torch.allclose(h.float(), want, rtol=8e-3, atol=1e-6)
