@@ -1,13 +1,21 @@
-// Causal self-attention over a prompt (prefill from an empty cache): what the
+// Causal self-attention over a prompt or a chunk of one (prefill): what the
 // reference computes with repeat_kv + scaled_dot_product_attention
-// (astrai/model/components/attention.py:15-23, 93-100) when the query and key
-// positions coincide.  Grouped-query attention without repeating heads, bf16
-// tensors, fp32 softmax statistics and accumulation, head dimension 64 or 128.
+// (astrai/model/components/attention.py:15-23, 93-100).  Grouped-query attention
+// without repeating heads, bf16 tensors, fp32 softmax statistics and
+// accumulation, head dimension 64 or 128.  Keys and values come from the new
+// tokens' own rows, or from the paged cache (a chunk on top of cached tokens).
 //
-// Workgroup = (128 query positions, one query head, one sequence), 4 wavefronts
-// of 32 query rows; K/V are walked in blocks of 64 positions up to the causal
-// limit.  Everything is computed transposed so that no register ever has to
-// change lanes:
+// Workgroup = (32 QW query positions, one query head, one sequence), QW x KW
+// wavefronts.  A block of 64 keys against 32 queries is one serial chain of products,
+// softmax and products, about 0.85 us at head dimension 64 whatever else the device
+// does, and a query's blocks follow one another: a prompt of a few hundred tokens or a
+// short chunk on a long context leaves most of the chip idle while that chain runs.
+// KW > 1 shortens it: the KW wavefronts of a query row take KW blocks' scores and
+// probabilities side by side and leave them in LDS, then each adds all KW blocks, in
+// order, to its share of the head dimension.  Sums, running maxima and roundings are
+// those of KW = 1: same bits.
+//
+// Everything is computed transposed so that no register ever has to change lanes:
 //
 //   S^T[key, q] = K Q^T    v_mfma_f32_32x32x16_bf16 with A = K (rows of the LDS
 //                          tile, 16-byte reads), B = Q^T (the wavefront's query
@@ -20,12 +28,14 @@
 //   O^T[d, q] += V^T P^T   B = P^T: the probabilities a lane already holds are,
 //                          packed to bf16 in register order, exactly its operand
 //                          (the matrix core does not care which key sits in which
-//                          k slot as long as A agrees); A = V^T read from an LDS
-//                          tile that was written transposed ([d][key]) when the
-//                          block was staged, two 8-byte reads per operand.
+//                          k slot as long as A agrees); A = V^T through the
+//                          transposing LDS read (ds_read_b64_tr_b16: 4 keys of one
+//                          dimension per lane from 4 rows of 16 dimensions).
 //
-// The next block's K and V are fetched into registers while the current one is
-// being multiplied.
+// K and V rows go from memory straight into LDS (16 bytes per lane, no registers)
+// as they are, one block ahead of the products, into the other of two buffers: one
+// barrier per block.  A row's 16-byte pieces are permuted (row_key) so that both
+// the row reads of K and the transposing reads of V spread over all banks.
 #include "aq_common.h"
 
 namespace aq {
@@ -45,30 +55,56 @@ struct PrefillAttnArgs {
   const int64_t* table;  // [B, P] physical page ids, < 0: unmapped (zero keys and values)
   int64_t P, page, n_pages;
   int start, page_shift;
-  int paired;  // != 0: the second half of the workgroups takes the query blocks lightest first
+  int table_lds;  // entries of the page table that are copied into LDS first (all a launch needs, or 0: read from memory)
+  int paired;     // != 0: the second half of the workgroups takes the query blocks lightest first
 };
 
 typedef __bf16 pa_bf16x8 __attribute__((ext_vector_type(8)));
+typedef short pa_s16x4 __attribute__((ext_vector_type(4)));
 typedef float pa_f32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) void pa_lds_void;
+typedef __attribute__((address_space(3))) pa_s16x4 pa_lds_s16x4;
 
-constexpr int PA_QB = 128;  // query rows per workgroup
-constexpr int PA_KB = 64;   // keys per block
+__device__ const uint4 pa_zero_row[16] = {};  // what a row of an unmapped page reads as
 
-// Two workgroups per compute unit (2 wavefronts per SIMD, at most 256 registers each): the other workgroup's
-// matrix work is what overlaps this one's softmax and staging.
+// 16 bytes per lane from memory to LDS, 1 KiB in lane order from byte `at` (wavefront-uniform).  Written out because the compiler,
+// given the builtin, waits for every such load in flight before the next LDS read of any kind -- here the other buffer's,
+// requested a moment earlier.  The kernel waits itself, before the barrier that hands a buffer over.
+__device__ __forceinline__ void load_row_lds(const uint16_t* src, uint32_t at) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(at) : "memory");  // m0 needs a wait state
+}
+
+// The 16-byte piece of row r that sits in slot s of the row is s ^ row_key(r): the low bits of r, reversed.  16 rows
+// reading the same piece (K) fall on all slots of the bank lines; the 8 neighbouring rows x 64 bytes of a transposing
+// read (V) are told apart by their lowest bits, which reversed move a row's pieces by 64 bytes and more.
+template <int D>
+__device__ __forceinline__ int row_key(int row) {
+  if constexpr (D == 64)  // 128-byte rows: two to a bank line
+    return (int)(__builtin_bitreverse32((uint32_t)(row >> 1) & 7u) >> 29);
+  else
+    return (int)(__builtin_bitreverse32((uint32_t)row & 15u) >> 28);
+}
+
 // PAGED: a chunk of S new tokens on top of `start` cached ones -- K and V of all start + S positions come from the
 // paged cache (the new tokens' rows have been written there already), causality is by position.
-template <int D, bool PAGED = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(PrefillAttnArgs p) {
-  constexpr int KP = D + 8;       // K tile row pitch (elements): 16-byte reads of 32 rows hit distinct banks
-  constexpr int VP = PA_KB + 4;   // V^T tile row pitch
-  constexpr int DSTEPS = D / 16;  // matrix-core steps over the head dimension
-  constexpr int DT = D / 32;      // 32-row tiles of the transposed output
-  constexpr int CPT = PA_KB * (D / 8) / 256;  // 16-byte chunks of a K (or V) block per thread: 2 or 4
-  constexpr int KS_ELEMS = PA_KB * KP, VT_ELEMS = D * VP;
-  extern __shared__ __align__(16) uint16_t pa_lds[];  // [K tile | V^T tile]
+template <int D, int QW, int KW, bool PAGED>
+__global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(PrefillAttnArgs p) {
+  constexpr int QB = 32 * QW;                       // query rows of the workgroup
+  constexpr int KB = 64;                            // keys of a block
+  constexpr int NT = KB / 32;                       // 32-key tiles of a block
+  constexpr int DSTEPS = D / 16;                    // matrix-core steps over the head dimension
+  constexpr int DT = D / 32;                        // 32-row tiles of the transposed output
+  constexpr int ROWB = 2 * D;                       // bytes of a K or V row
+  constexpr int RPI = 1024 / ROWB, LPR = 64 / RPI;  // rows of a 1 KiB load, lanes of a row
+  constexpr int TILE = KB * ROWB;                   // bytes of a block's K (or V)
+  constexpr int LOADS = TILE / 1024 / QW;           // 1 KiB loads of K (and of V) per wavefront and block
+  constexpr int BUF = KW * 2 * TILE;
+  static_assert(LOADS >= 1 && TILE % (1024 * QW) == 0, "whole loads per wavefront");
+  __shared__ float maxima[KW][QW][32], psums[KW][QW][64];  // (KW > 1)
+  extern __shared__ __align__(1024) uint8_t pa_lds[];  // 2 buffers of KW [K block | V block]; page table (PAGED)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qw = wave % QW, kw = wave / QW;
   const int col = lane & 31, g = lane >> 5;
   const int S = p.S;
   // Workgroups are numbered heaviest first: a query block attends to every key block up to its own, so the
@@ -76,22 +112,95 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   // first, then the block before it, ... -- the long workgroups start at once and the short ones fill in
   // behind them (in launch order the light blocks of head 0 would start first and the heavy ones of the last
   // heads would run alone at the end: 34 -> 28 us at 8 x 512, 339 -> 219 us at 4 x 2048 x 32 heads).
-  // When the whole launch is resident at once (two workgroups per compute unit), the second half of the
-  // numbering runs lightest first instead: the workgroup that joins a heavy one on its compute unit is then a
-  // light one, and every compute unit gets the same sum (8 x 512 x 16 heads: 22.4 -> 21.6 us; with more
-  // workgroups than slots the descending order is the better one, 4 x 2048 x 32 heads 186 against 194 us).
-  const int nqb = (S + PA_QB - 1) / PA_QB, per = p.Hq * p.B;
+  // When the whole launch is resident at once, the second half of the numbering runs lightest first instead: the
+  // workgroup that joins a heavy one on its compute unit is then a light one.
+  const int nqb = (S + QB - 1) / QB, per = p.Hq * p.B;
   const int rank = (int)blockIdx.x / per, hrank = (nqb + 1) / 2;
   const int qblk = (p.paired && rank >= hrank) ? rank - hrank : nqb - 1 - rank;
-  const int q0 = qblk * PA_QB, h = ((int)blockIdx.x % per) % p.Hq,
-            b = ((int)blockIdx.x % per) / p.Hq;
+  const int q0 = qblk * QB, h = ((int)blockIdx.x % per) % p.Hq, b = ((int)blockIdx.x % per) / p.Hq;
   const int kvh = h / (p.Hq / p.Hkv);
-  const int qw0 = q0 + wave * 32;          // first query row of this wavefront
+  const int qw0 = q0 + qw * 32;            // first query row of this wavefront
   const int qpos = qw0 + col;              // this lane's query
   const int64_t tok0 = (int64_t)b * S;
   const int off = PAGED ? p.start : 0;     // position of query 0
   const int T = off + S;                   // key positions
   const int qw0p = qw0 + off, qposp = qpos + off;  // positions of the wavefront's first / this lane's query
+  const int last_q = (q0 + QB < S ? q0 + QB : S) - 1 + off;  // position of the workgroup's last query
+  const int last_w = last_q < qw0p + 31 ? last_q : qw0p + 31;  // ... and of the wavefront's
+  const int nblk = last_q / KB + 1;                          // blocks that hold a key some query of the workgroup may see
+  const int nit = (nblk + KW - 1) / KW;
+
+  // the page table of this sequence, ids checked, where blocks straddle pages: rows of unmapped pages read zeros
+  int* const table = reinterpret_cast<int*>(pa_lds + 2 * BUF);
+  auto phys_of = [&](int lp) -> int {
+    const int64_t t = p.table[(int64_t)b * p.P + lp];
+    return t >= 0 && t < p.n_pages ? (int)t : -1;
+  };
+  if constexpr (PAGED) {
+    if (p.table_lds) {
+      for (int i = tid; i < p.table_lds; i += QW * KW * 64) table[i] = phys_of(i);
+      __syncthreads();
+    }
+  }
+  // this lane's piece of the rows that the wavefront's loads bring: elements into the row
+  const int chunk0 = qw * LOADS;
+  int pc[LOADS];
+#pragma unroll
+  for (int c = 0; c < LOADS; ++c) pc[c] = ((lane % LPR) ^ row_key<D>((chunk0 + c) * RPI + lane / LPR)) * 8;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(pa_lds_void*)pa_lds;
+  const uint16_t* const kbase = p.k + tok0 * p.k_stride + (int64_t)kvh * D;
+  const uint16_t* const vbase = p.v + tok0 * p.v_stride + (int64_t)kvh * D;
+  auto issue = [&](int it, int buf) __attribute__((always_inline)) {
+    const int j = it * KW + kw;
+    if (j >= nblk) return;  // wavefront-uniform
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * BUF + kw * 2 * TILE + chunk0 * 1024);
+    const int rows = T - j * KB;  // rows past the last position: any row that is there, masked by causality
+    if (!PAGED || p.page % KB == 0) {
+      // the block's rows are equally spaced: contiguous tensors, or the whole block in one page (an unmapped one: a row
+      // of zeros again and again)
+      const uint16_t *ks, *vs;
+      int kstep, vstep;
+      if constexpr (PAGED) {
+        const int lp = __builtin_amdgcn_readfirstlane(p.page_shift >= 0 ? (j * KB) >> p.page_shift : j * KB / (int)p.page);
+        const int64_t phys = p.table[(int64_t)b * p.P + lp];
+        const int64_t first = ((phys * p.page + (j * KB - lp * (int)p.page)) * p.Hkv + kvh) * D;
+        const bool mapped = phys >= 0 && phys < p.n_pages;
+        ks = mapped ? p.kc + first : reinterpret_cast<const uint16_t*>(pa_zero_row);
+        vs = mapped ? p.vc + first : reinterpret_cast<const uint16_t*>(pa_zero_row);
+        kstep = vstep = mapped ? p.Hkv * D : 0;
+      } else {
+        kstep = (int)p.k_stride, vstep = (int)p.v_stride;
+        ks = kbase + (uint32_t)(j * KB * kstep);
+        vs = vbase + (uint32_t)(j * KB * vstep);
+      }
+#pragma unroll
+      for (int c = 0; c < LOADS; ++c) {
+        int r = (chunk0 + c) * RPI + lane / LPR;
+        r = r < rows ? r : rows - 1;
+        load_row_lds(ks + (uint32_t)(r * kstep + pc[c]), dst + c * 1024);
+        load_row_lds(vs + (uint32_t)(r * vstep + pc[c]), dst + TILE + c * 1024);
+      }
+      return;
+    }
+    // pages that blocks straddle.  Every address first, then the loads: a load is a fence to the compiler, and a page
+    // lookup behind each one would wait for LDS once per row
+    int64_t row[LOADS];
+#pragma unroll
+    for (int c = 0; c < LOADS; ++c) {
+      int key = (chunk0 + c) * RPI + lane / LPR;
+      key = j * KB + (key < rows ? key : rows - 1);
+      const int lp = key / (int)p.page, in_page = key - lp * (int)p.page;
+      const int phys = p.table_lds ? table[lp] : phys_of(lp);
+      row[c] = phys < 0 ? -1 : (((int64_t)phys * p.page + in_page) * p.Hkv + kvh) * D + pc[c];
+    }
+#pragma unroll
+    for (int c = 0; c < LOADS; ++c) {
+      const uint16_t* zero = reinterpret_cast<const uint16_t*>(pa_zero_row);
+      load_row_lds(row[c] < 0 ? zero : p.kc + row[c], dst + c * 1024);
+      load_row_lds(row[c] < 0 ? zero : p.vc + row[c], dst + TILE + c * 1024);
+    }
+  };
+  issue(0, 0);
 
   // Q^T operand: lane = (query col, dimensions 16 step + 8 g .. + 8); rows past S read row S - 1
   uint4 qf[DSTEPS];
@@ -101,271 +210,188 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
     for (int st = 0; st < DSTEPS; ++st) qf[st] = *reinterpret_cast<const uint4*>(src + st * 16);
   }
-  // staging, fetched one block ahead: 16-byte chunks (key, 8 dimensions).  K chunks go to threads in memory
-  // order (coalesced loads, row-major LDS tile).  V is written transposed; there a wavefront's lanes take
-  // consecutive KEYS of one chunk column, so that the stores of an instruction fall into consecutive LDS
-  // words instead of 4 banks.
-  // (scalars, not arrays: the compiler kept a 4-element array of these in scratch memory)
-  uint4 kreg0, kreg1, kreg2, kreg3, vreg0, vreg1, vreg2, vreg3;
-  kreg2 = kreg3 = vreg2 = vreg3 = make_uint4(0, 0, 0, 0);
-  // element offset of position t's row for this KV head in the paged caches, -1 when its page is unmapped
-  uint32_t kneg = 0, vneg = 0;  // bit c: the row of staging chunk c is not there
-  const int pshift = PAGED ? p.page_shift : 0;  // log2 of the page size, or -1 when it is not a power of two
-  auto paged_row = [&](int t) -> int64_t {
-    const int lp = pshift >= 0 ? t >> pshift : t / (int)p.page;
-    const int in_page = pshift >= 0 ? t & ((1 << pshift) - 1) : t - lp * (int)p.page;
-    const int64_t phys = p.table[(int64_t)b * p.P + lp];
-    return (phys >= 0 && phys < p.n_pages) ? ((phys * p.page + in_page) * p.Hkv + kvh) * D : -1;
-  };
-  int64_t kro0 = -1, kro1 = -1, kro2 = -1, kro3 = -1, vro = -1;  // row offsets of the block fetched next
-  auto lookup = [&](int j) __attribute__((always_inline)) {
-    if constexpr (PAGED) {
-      auto krow_of = [&](int c) -> int64_t {
-        int kr = j * PA_KB + (c * 256 + tid) / (D / 8);
-        return paged_row(kr < T ? kr : T - 1);
-      };
-      kro0 = krow_of(0);
-      kro1 = krow_of(1);
-      if constexpr (CPT > 2) {
-        kro2 = krow_of(2);
-        kro3 = krow_of(3);
-      }
-      const int vr = j * PA_KB + lane;
-      vro = paged_row(vr < T ? vr : T - 1);
-    }
-  };
-  // Direct kernel: K and V of this sequence and KV head behind buffer descriptors; a staging chunk's byte offset is
-  // a lane constant (computed once) plus the block's row distance -- one add per load where a 64-bit row product
-  // stood -- and rows past the sequence fall outside the descriptor and read as zero (they are masked anyway).
-  __amdgpu_buffer_rsrc_t Kd = make_rsrc(nullptr, 0), Vd = make_rsrc(nullptr, 0);
-  uint32_t koff[4] = {0, 0, 0, 0}, voff[4] = {0, 0, 0, 0};
-  uint32_t kblk = 0, vblk = 0;  // bytes between consecutive key blocks
-  if constexpr (!PAGED) {
-    Kd = make_rsrc(p.k + tok0 * p.k_stride + (int64_t)kvh * D, (uint32_t)(((int64_t)(S - 1) * p.k_stride + D) * 2));
-    Vd = make_rsrc(p.v + tok0 * p.v_stride + (int64_t)kvh * D, (uint32_t)(((int64_t)(S - 1) * p.v_stride + D) * 2));
-    kblk = (uint32_t)(PA_KB * p.k_stride * 2);
-    vblk = (uint32_t)(PA_KB * p.v_stride * 2);
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      const int idx = c * 256 + tid, key = idx / (D / 8), ch = idx % (D / 8);
-      koff[c] = (uint32_t)(key * (int)p.k_stride + ch * 8) * 2u;
-      voff[c] = (uint32_t)(lane * (int)p.v_stride + (wave + 4 * c) * 8) * 2u;
-    }
-  }
-  auto fetch1 = [&](int j, int c, uint4& kr_out, uint4& vr_out) __attribute__((always_inline)) {
-    const int idx = c * 256 + tid, key = idx / (D / 8), ch = idx % (D / 8);
-    if constexpr (!PAGED) {
-      kr_out = buffer_load_16(Kd, koff[c] + (uint32_t)j * kblk);
-      vr_out = buffer_load_16(Vd, voff[c] + (uint32_t)j * vblk);
-      return;
-    }
-    int kr = j * PA_KB + key;
-    kr = kr < T ? kr : T - 1;  // past the last position: any valid row, masked by causality
-    int vr = j * PA_KB + lane;
-    vr = vr < T ? vr : T - 1;
-    if constexpr (PAGED) {
-      // the rows' offsets were looked up one block earlier (lookup below): the page-table round trip is off
-      // the prefetch's path.  Rows of unmapped pages read row 0 and are zeroed when they are staged: a
-      // select on the loaded value here would make every load of the prefetch wait for the one before it.
-      const int64_t krow = c == 0 ? kro0 : c == 1 ? kro1 : c == 2 ? kro2 : kro3, vrow = vro;
-      kr_out = *reinterpret_cast<const uint4*>(p.kc + (krow >= 0 ? krow : 0) + ch * 8);
-      vr_out = *reinterpret_cast<const uint4*>(p.vc + (vrow >= 0 ? vrow : 0) + (wave + 4 * c) * 8);
-      kneg = (kneg & ~(1u << c)) | ((krow < 0 ? 1u : 0u) << c);
-      vneg = (vneg & ~(1u << c)) | ((vrow < 0 ? 1u : 0u) << c);
-    } else {
-      kr_out = *reinterpret_cast<const uint4*>(p.k + (tok0 + kr) * p.k_stride + (int64_t)kvh * D + ch * 8);
-      vr_out = *reinterpret_cast<const uint4*>(p.v + (tok0 + vr) * p.v_stride + (int64_t)kvh * D + (wave + 4 * c) * 8);
-    }
-  };
-  auto stage1 = [&](uint16_t* ks, uint16_t* vt, int c, const uint4& kr_in, const uint4& vr_in) __attribute__((always_inline)) {
-    const int idx = c * 256 + tid, key = idx / (D / 8), ch = idx % (D / 8);
-    uint4 kr_z = kr_in, vr_z = vr_in;
-    if constexpr (PAGED) {
-      if (kneg & (1u << c)) kr_z = make_uint4(0, 0, 0, 0);
-      if (vneg & (1u << c)) vr_z = make_uint4(0, 0, 0, 0);
-    }
-    *reinterpret_cast<uint4*>(&ks[key * KP + ch * 8]) = kr_z;
-    // V chunk (key = lane, dimensions 8 (wave + 4 c) .. + 8) into the transposed tile, two keys per 4-byte
-    // store: neighbouring lanes swap dwords (DPP) and byte-permute them into "one dimension, both keys" --
-    // even lanes then hold the even dimensions of the key pair, odd lanes the odd ones.
-    const bool odd = lane & 1;
-    const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
-    uint32_t* vdst = reinterpret_cast<uint32_t*>(&vt[((wave + 4 * c) * 8 + (odd ? 1 : 0)) * VP + (lane & ~1)]);
-    const uint32_t w[4] = {vr_z.x, vr_z.y, vr_z.z, vr_z.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[e], 0xB1 /* quad_perm [1,0,3,2] */, 0xf, 0xf, true);
-      // even lane: {mine.lo, other.lo} = dimension 2e of keys (lane, lane + 1); odd: {other.hi, mine.hi} = 2e + 1
-      vdst[e * VP] = __builtin_amdgcn_perm(other, w[e], sel);  // e * VP words = 2e rows of VP halfwords
-    }
-  };
-#define PA_FETCH(J)                        \
-  fetch1((J), 0, kreg0, vreg0);            \
-  fetch1((J), 1, kreg1, vreg1);            \
-  if constexpr (CPT > 2) {                 \
-    fetch1((J), 2, kreg2, vreg2);          \
-    fetch1((J), 3, kreg3, vreg3);          \
-  }
-#define PA_STAGE(BUF)                                                        \
-  {                                                                          \
-    uint16_t* ks_w = pa_lds + (BUF) * (KS_ELEMS + VT_ELEMS);                  \
-    uint16_t* vt_w = ks_w + KS_ELEMS;                                        \
-    stage1(ks_w, vt_w, 0, kreg0, vreg0);                                     \
-    stage1(ks_w, vt_w, 1, kreg1, vreg1);                                     \
-    if constexpr (CPT > 2) {                                                 \
-      stage1(ks_w, vt_w, 2, kreg2, vreg2);                                   \
-      stage1(ks_w, vt_w, 3, kreg3, vreg3);                                   \
-    }                                                                        \
-  }
+  // fragment addresses inside a block: K row `col`, piece 2 step + g; V rows 4 g + i / 4 (and 8 further), i = lane % 16,
+  // dimensions 16 (lane / 16 % 2) + 4 (i % 4) of a 32-dimension tile
+  const int kfr = col * ROWB + ((g ^ row_key<D>(col)) << 4);  // ^ (2 step) << 4
+  const int vrow = 4 * g + (lane & 15) / 4, vpiece = ((lane >> 4) & 1) * 2 + (lane & 3) / 2;
+  const int vfr0 = vrow * ROWB + ((vpiece ^ row_key<D>(vrow)) << 4) + (lane & 1) * 8;  // ^ dt << 6
+  const int vfr1 = (vrow + 8) * ROWB + ((vpiece ^ row_key<D>(vrow + 8)) << 4) + (lane & 1) * 8;
 
-  pa_f32x16 o[DT];
+  // dimension tiles whose sums this wavefront keeps: all, or with KW > 1 its share (with fewer tiles than wavefronts the
+  // last ones keep none)
+  constexpr int DTW = DT > KW ? DT / KW : 1;
+  const int dt0 = KW == 1 ? 0 : kw * DTW;
+  const bool sums = KW == 1 || dt0 < DT;
+  pa_f32x16 o[DTW];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < DTW; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
   float m = -INFINITY, l = 0.0f;  // running maximum of this lane's query; this lane's half of its denominator
 
-  const int last_q = (q0 + PA_QB < S ? q0 + PA_QB : S) - 1 + off;  // position of the workgroup's last query
-  const int nblk = last_q / PA_KB + 1;  // blocks that hold a key some query of the workgroup may see
-  // One LDS buffer, two barriers per block; the next block's global loads are in flight while this one is
-  // multiplied.  (Two buffers with one barrier per block measured 15 % slower.)
-  const uint16_t* ks = pa_lds;
-  const uint16_t* vt = pa_lds + KS_ELEMS;
-  lookup(0);
-  PA_FETCH(0)
-  if (nblk > 1) lookup(1);
-  for (int j = 0; j < nblk; ++j) {
-    __syncthreads();  // everyone is done reading the previous block's tiles
-    PA_STAGE(0)
+  for (int it = 0; it < nit; ++it) {
+    // block `it` has landed and everyone is done with the one before
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     __syncthreads();
-    if (j + 1 < nblk) {
-      PA_FETCH(j + 1)
-      if (j + 2 < nblk) lookup(j + 2);
-    }
-    const int kb0 = j * PA_KB;
-    if (kb0 > qw0p + 31) continue;  // wavefront-uniform: every key of the block is ahead of every query here
-    // ---- scores, transposed: two tiles of 32 keys
-    // The K fragments are read two dimension steps ahead of the products that take them, and the two tiles'
-    // accumulation chains alternate: left to itself the compiler put every LDS read right in front of its MFMA
-    // (one LDS round trip per product, sixteen in a row) and ran the second tile's chain after the first's.
-    // Each chain still adds its steps in ascending order: same bits.
-    pa_f32x16 s[2];
-    {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[0][r] = s[1][r] = 0.0f;
-      const uint16_t* k0 = &ks[col * KP + g * 8];
-      const uint16_t* k1 = k0 + 32 * KP;
-      constexpr int GRP = 2, NG = DSTEPS / GRP;
-      static_assert(DSTEPS % GRP == 0, "whole groups of dimension steps");
-      uint4 fa[2][GRP][2];
-      auto ldk = [&](int buf, int st0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < GRP; ++i) {
-          fa[buf][i][0] = *reinterpret_cast<const uint4*>(k0 + (st0 + i) * 16);
-          fa[buf][i][1] = *reinterpret_cast<const uint4*>(k1 + (st0 + i) * 16);
-        }
-      };
-      ldk(0, 0);
-      if (NG > 1) ldk(1, GRP);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int gi = 0; gi < NG; ++gi) {
-#pragma unroll
-        for (int i = 0; i < GRP; ++i) {
-          const pa_bf16x8 qv = __builtin_bit_cast(pa_bf16x8, qf[gi * GRP + i]);
-          s[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pa_bf16x8, fa[gi & 1][i][0]), qv, s[0], 0, 0, 0);
-          s[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pa_bf16x8, fa[gi & 1][i][1]), qv, s[1], 0, 0, 0);
-        }
-        if (gi + 2 < NG) ldk(gi & 1, (gi + 2) * GRP);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    // ---- online softmax for this lane's query; register r of tile kt is key kb0 + 32 kt + 8 (r / 4) + 4 g + r % 4.
-    // Scores stay unscaled; the scale (> 0) is applied to the maximum and inside the exponent's fma.
-    const bool diag = kb0 + PA_KB - 1 > qw0p;  // wavefront-uniform: some key of the block is ahead of some query
+    if (it + 1 < nit) issue(it + 1, (it + 1) & 1);
+    const int kb0 = (it * KW + kw) * KB;
+    const bool ahead = kb0 > last_w;  // wavefront-uniform: every key of the block is ahead of every query here
+    if (KW == 1 && ahead) continue;
+    uint8_t* const buf = pa_lds + (it & 1) * BUF;
+    const uint8_t* ks = buf + kw * 2 * TILE;
+    pa_f32x16 s[NT];
     float bm = -INFINITY;
-    if (diag) {  // a branch, not 32 compares and selects in every block: most blocks lie wholly behind the queries
+    if (!ahead) {
+      // ---- scores, transposed: NT tiles of 32 keys
+      // The K fragments are read two dimension steps ahead of the products that take them, and the tiles' accumulation
+      // chains alternate: left to itself the compiler put every LDS read right in front of its MFMA (one LDS round trip
+      // per product) and ran one tile's chain after the other's.
+      {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (kb0 + kt * 32 + 8 * (r / 4) + 4 * g + (r % 4) > qposp) s[kt][r] = -INFINITY;
+          for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+        constexpr int GRP = 4 / NT, NG = DSTEPS / GRP;
+        uint4 fa[2][GRP][NT];
+        auto ldk = [&](int buf, int st0) __attribute__((always_inline)) {
+#pragma unroll
+          for (int i = 0; i < GRP; ++i)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              fa[buf][i][t] = *reinterpret_cast<const uint4*>(ks + t * 32 * ROWB + (kfr ^ ((2 * (st0 + i)) << 4)));
+        };
+        ldk(0, 0);
+        if (NG > 1) ldk(1, GRP);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi) {
+#pragma unroll
+          for (int i = 0; i < GRP; ++i) {
+            const pa_bf16x8 qv = __builtin_bit_cast(pa_bf16x8, qf[gi * GRP + i]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pa_bf16x8, fa[gi & 1][i][t]), qv, s[t], 0, 0, 0);
+          }
+          if (gi + 2 < NG) ldk(gi & 1, (gi + 2) * GRP);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      // ---- online softmax for this lane's query; register r of tile kt is key kb0 + 32 kt + 8 (r / 4) + 4 g + r % 4.
+      // Scores stay unscaled; the scale (> 0) is applied to the maximum and inside the exponent's fma.
+      const bool diag = kb0 + KB - 1 > qw0p;  // wavefront-uniform: some key of the block is ahead of some query
+      if (diag) {  // a branch, not a compare and select per score in every block: most blocks lie wholly behind the queries
+#pragma unroll
+        for (int kt = 0; kt < NT; ++kt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (kb0 + kt * 32 + 8 * (r / 4) + 4 * g + (r % 4) > qposp) s[kt][r] = -INFINITY;
+      }
+#pragma unroll
+      for (int kt = 0; kt < NT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bm = fmaxf(bm, s[kt][r]);
+      bm = fmaxf(bm, __shfl_xor(bm, 32, 64)) * p.scale_log2e;
     }
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) bm = fmaxf(bm, s[kt][r]);
-    bm = fmaxf(bm, __shfl_xor(bm, 32, 64)) * p.scale_log2e;
     // The running maximum only has to bound the exponents, not equal the true maximum: it is raised (and the
     // accumulators rescaled) only when some query of the wavefront would otherwise see an exponent above 2^8;
     // with probabilities up to 256 nothing overflows and bf16 keeps its relative precision.  After the first
-    // blocks this is rare, and the 64-register rescale is skipped.
-    const bool raise = __builtin_amdgcn_ballot_w64(bm > m + 8.0f) != 0;  // m = -inf in block 0: raised there
-    float alpha = 1.0f;
-    if (raise) {
-      const float mn = fmaxf(m, bm);  // finite from block 0 on: key 0 is visible to every query
-      alpha = __builtin_amdgcn_exp2f(m - mn);
-      m = mn;
-      l *= alpha;
+    // block this is rare, and the rescale of the accumulators is skipped.
+    float alpha[KW], mk = m;  // factor of the sums in front of each block, the maximum this wavefront's block works with
+    bool raise[KW];           // wavefront-uniform
+    if constexpr (KW > 1) {
+      if (g == 0) maxima[kw][qw][col] = bm;
+      __syncthreads();
     }
-    float ps = 0.0f;
-    uint4 pf[2][2];  // P^T operands: tile kt, keys 16 s2 .. + 16
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      float pv[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][r], p.scale_log2e, -m));
-        ps += pv[r];
+    for (int k = 0; k < KW; ++k) {
+      const float b = KW == 1 ? bm : maxima[k][qw][col];
+      raise[k] = __builtin_amdgcn_ballot_w64(b > m + 8.0f) != 0;  // m = -inf in block 0: raised there
+      alpha[k] = 1.0f;
+      if (raise[k]) {
+        const float mn = fmaxf(m, b);  // finite from block 0 on: key 0 is visible to every query
+        alpha[k] = __builtin_amdgcn_exp2f(m - mn);
+        m = mn;
       }
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-        pf[kt][s2] = make_uint4(pack_bf16x2(pv[8 * s2 + 0], pv[8 * s2 + 1]), pack_bf16x2(pv[8 * s2 + 2], pv[8 * s2 + 3]),
-                                pack_bf16x2(pv[8 * s2 + 4], pv[8 * s2 + 5]), pack_bf16x2(pv[8 * s2 + 6], pv[8 * s2 + 7]));
+      if (k == kw || KW == 1) mk = m;
     }
-    l += ps;
-    // ---- output, transposed: O^T[d, q] = alpha O^T + V^T P^T
-    if (raise) {  // one branch for all tiles (a branch per tile kept the tiles' products apart)
+    uint4 pf[NT][2];  // P^T operands: tile kt, keys 16 s2 .. + 16
+    float ps = 0.0f;
+    if (!ahead) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
+      for (int kt = 0; kt < NT; ++kt) {
+        float pv[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
-    }
-    // V^T fragments of two dimension tiles at a time, all read before the pair's products, whose two chains
-    // alternate; each chain adds its four key groups in ascending order: same bits.
-    {
-      uint4 fv[DT][4];
-      auto ldv = [&](int dt) __attribute__((always_inline)) {
-        const uint16_t* vrow = &vt[(dt * 32 + col) * VP + 4 * g];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          // k slots of this lane group: keys 32 kt + 16 s2 + {4 g .. + 4, 8 + 4 g .. + 4}, kk = 2 kt + s2
-          const uint2 lo = *reinterpret_cast<const uint2*>(vrow + kk * 16);
-          const uint2 hi = *reinterpret_cast<const uint2*>(vrow + kk * 16 + 8);
-          fv[dt][kk] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        for (int r = 0; r < 16; ++r) {
+          pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][r], p.scale_log2e, -mk));
+          ps += pv[r];
         }
-      };
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) ldv(dt);
+        for (int s2 = 0; s2 < 2; ++s2)
+          pf[kt][s2] = make_uint4(pack_bf16x2(pv[8 * s2 + 0], pv[8 * s2 + 1]), pack_bf16x2(pv[8 * s2 + 2], pv[8 * s2 + 3]),
+                                  pack_bf16x2(pv[8 * s2 + 4], pv[8 * s2 + 5]), pack_bf16x2(pv[8 * s2 + 6], pv[8 * s2 + 7]));
+      }
+      if constexpr (KW > 1) {  // over the block's keys, which everyone has read
+        static_assert(QW * NT * 2048 <= TILE, "the probabilities fit the keys' place");
+        uint4* dst = reinterpret_cast<uint4*>(buf + kw * 2 * TILE + qw * NT * 2048) + lane;
+#pragma unroll
+        for (int kt = 0; kt < NT; ++kt)
+#pragma unroll
+          for (int s2 = 0; s2 < 2; ++s2) dst[(2 * kt + s2) * 64] = pf[kt][s2];
+        psums[kw][qw][lane] = ps;
+      }
+    }
+    if constexpr (KW > 1) __syncthreads();
+    // ---- output, transposed: O^T[d, q] = alpha O^T + V^T P^T, block by block
+#pragma unroll
+    for (int k = 0; k < KW; ++k) {
+      if (KW > 1 && ((it * KW + k) * KB > last_w || !sums)) break;  // wavefront-uniform
+      const uint8_t* vs = buf + k * 2 * TILE + TILE;
+      if (raise[k]) {  // one branch for all tiles (a branch per tile kept the tiles' products apart)
+        l *= alpha[k];
+#pragma unroll
+        for (int dt = 0; dt < DTW; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[dt][r] *= alpha[k];
+      }
+      if constexpr (KW > 1) {
+        const uint4* src = reinterpret_cast<const uint4*>(buf + k * 2 * TILE + qw * NT * 2048) + lane;
+#pragma unroll
+        for (int kt = 0; kt < NT; ++kt)
+#pragma unroll
+          for (int s2 = 0; s2 < 2; ++s2) pf[kt][s2] = src[(2 * kt + s2) * 64];
+        ps = psums[k][qw][lane];
+      }
+      l += ps;
+      // V^T fragments of all tiles, read before the products, whose chains alternate.  k slots of this lane group:
+      // keys 32 kt + 16 s2 + {4 g .. + 4, 8 + 4 g .. + 4}, kk = 2 kt + s2.
+      constexpr int KK = 2 * NT;
+      pa_bf16x8 fv[DTW][KK];
+#pragma unroll
+      for (int dt = 0; dt < DTW; ++dt)
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+          const uint8_t* at = vs + kk * 16 * ROWB;
+          const pa_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_s16x4*)(at + (vfr0 ^ ((dt0 + dt) << 6))));
+          const pa_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_s16x4*)(at + (vfr1 ^ ((dt0 + dt) << 6))));
+          fv[dt][kk] = __builtin_bit_cast(pa_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int d0 = 0; d0 < DT; d0 += 2) {
+      for (int d0 = 0; d0 < DTW; d0 += 2)
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const pa_bf16x8 pv8 = __builtin_bit_cast(pa_bf16x8, pf[kk >> 1][kk & 1]);
-          o[d0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pa_bf16x8, fv[d0][kk]), pv8, o[d0], 0, 0, 0);
-          o[d0 + 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pa_bf16x8, fv[d0 + 1][kk]), pv8, o[d0 + 1], 0, 0, 0);
-        }
-      }
+        for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+          for (int dt = d0; dt < (d0 + 2 < DTW ? d0 + 2 : DTW); ++dt)
+            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv[dt][kk], __builtin_bit_cast(pa_bf16x8, pf[kk >> 1][kk & 1]), o[dt], 0, 0, 0);
     }
   }
-  // ---- normalise and store: register r of tile dt is dimension 32 dt + 8 (r / 4) + 4 g + r % 4 of query col
   l += __shfl_xor(l, 32, 64);
-  if (qpos < S) {
+  // ---- normalise and store: register r of tile dt is dimension 32 dt + 8 (r / 4) + 4 g + r % 4 of query col
+  if (qpos < S && sums) {
     const float inv = 1.0f / l;
-    uint16_t* dst = p.out + ((tok0 + qpos) * p.Hq + h) * D + 4 * g;
+    uint16_t* dst = p.out + ((tok0 + qpos) * p.Hq + h) * D + dt0 * 32 + 4 * g;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DTW; ++dt)
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         uint2 w;
@@ -376,8 +402,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   }
 }
 
-#undef PA_FETCH
-#undef PA_STAGE
+constexpr int PA_TABLE_MAX = 2048;  // page-table entries kept in LDS
+
+template <int D, int QW, int KW, bool PAGED>
+static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
+  const int64_t wgs = ((int64_t)(a.S + 32 * QW - 1) / (32 * QW)) * a.Hq * a.B;
+  constexpr int KB = 64, BUFS = 2 * KW * 2 * KB * 2 * D;
+  a.paired = wgs <= (160 * 1024 / BUFS) * (int64_t)device_cus();
+  size_t lds = BUFS;
+  if constexpr (PAGED) {
+    const int64_t entries = ((int64_t)a.start + a.S + a.page - 1) / a.page;
+    a.table_lds = a.page % KB != 0 && entries <= PA_TABLE_MAX ? (int)entries : 0;
+    lds += (size_t)a.table_lds * sizeof(int);
+  }
+  hipLaunchKernelGGL((prefill_attn_kernel<D, QW, KW, PAGED>), dim3((unsigned)wgs), dim3(QW * KW * 64), lds, st, a);
+  return (int)hipGetLastError();
+}
+
+// How many wavefronts take a query row's blocks side by side.  One (128 queries per workgroup) moves the fewest K and V
+// bytes per query and is the faster form once the chip is full of such workgroups; with fewer, a launch lasts as long as
+// its longest chain of blocks, which two or four wavefronts shorten, 64 or 32 queries per workgroup.  The buffers of two
+// take 64 KiB at head dimension 64 (two workgroups per compute unit), 128 KiB at 128, those of four 128 KiB: they pay
+// while the launch is resident at once, and up to twice that where the chain is long.  us, head dimension 64, 24 heads
+// (1 | 2 | 4 wavefronts): 1 x 300 new tokens 7.3 | 6.8 | 6.0, 4 x 512 12.1 | 13.5 | 26, 1 x 2048 32 | 28 | 57, 64 on 1500
+// cached 29 | 22 | 16, 500 on 1500 36 | 27 | 32; head dimension 128, 16 heads (1 | 2): 1 x 1000 23 | 18, 4 x 300
+// 10.2 | 11.0, 64 on 1500 38 | 28.  Before, with keys staged through registers, one wavefront per query row and a page
+// lookup per row: 7.7, 12.4, 34, 48, 61; 27.5, 11.8, 76.
+template <int D, bool PAGED>
+static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
+  const int64_t heads = (int64_t)a.Hq * a.B, cus = device_cus(), T = (PAGED ? a.start : 0) + (int64_t)a.S;
+  const int64_t q32 = (a.S + 31) / 32 * heads, q64 = (a.S + 63) / 64 * heads;
+  if constexpr (D == 64) {
+    if (q32 <= cus) return launch_prefill_attn<D, 1, 4, PAGED>(a, st);
+  }
+  if (T > 128 && q64 <= (D == 128 ? 1 : T < 1024 ? 2 : 4) * cus) return launch_prefill_attn<D, 2, 2, PAGED>(a, st);
+  return launch_prefill_attn<D, 4, 1, PAGED>(a, st);
+}
 
 }  // namespace aq
 
@@ -392,10 +452,10 @@ extern "C" int aq_prefill_attn_causal(const void* q, int64_t q_stride, const voi
   if (aq::check_ptr16(q) || aq::check_ptr16(k) || aq::check_ptr16(v) || aq::check_ptr16(out) || (q_stride & 7) ||
       (k_stride & 7) || (v_stride & 7))
     return AQ_E_ALIGN;
-  if (S > (1 << 30) || Hq > 65535 || B > 65535 || ((S + aq::PA_QB - 1) / aq::PA_QB) * Hq * B > (int64_t)0x7fffffff)
+  if (S > (1 << 30) || Hq > 65535 || B > 65535 || ((S + 31) / 32) * Hq * B > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
   // 32-bit byte offsets inside one sequence's K and V (a key block past the end included)
-  if ((S + aq::PA_KB) * k_stride * 2 > (int64_t)0x7fffffff || (S + aq::PA_KB) * v_stride * 2 > (int64_t)0x7fffffff)
+  if ((S + 64) * k_stride * 2 > (int64_t)0x7fffffff || (S + 64) * v_stride * 2 > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
   aq::PrefillAttnArgs a{};
   a.q = static_cast<const uint16_t*>(q);
@@ -410,15 +470,8 @@ extern "C" int aq_prefill_attn_causal(const void* q, int64_t q_stride, const voi
   a.Hq = (int)Hq;
   a.Hkv = (int)Hkv;
   a.B = (int)B;
-  const dim3 grid((unsigned)(((S + aq::PA_QB - 1) / aq::PA_QB) * Hq * B));
-  a.paired = grid.x <= 2u * (unsigned)aq::device_cus();
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const size_t lds = (size_t)(aq::PA_KB * (D + 8) + D * (aq::PA_KB + 4)) * sizeof(uint16_t);  // 34 KiB at most
-  if (D == 128)
-    hipLaunchKernelGGL((aq::prefill_attn_kernel<128, false>), grid, dim3(256), lds, st, a);
-  else
-    hipLaunchKernelGGL((aq::prefill_attn_kernel<64, false>), grid, dim3(256), lds, st, a);
-  return (int)hipGetLastError();
+  return D == 128 ? aq::launch_prefill_attn<128, false>(a, st) : aq::launch_prefill_attn<64, false>(a, st);
 }
 
 extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
@@ -436,7 +489,7 @@ extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void
       (q_stride & 7))
     return AQ_E_ALIGN;
   if (start + S > (1 << 30) || Hq > 65535 || B > 65535 ||
-      ((S + aq::PA_QB - 1) / aq::PA_QB) * Hq * B > (int64_t)0x7fffffff)
+      ((S + 31) / 32) * Hq * B > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
   aq::PrefillAttnArgs a{};
   a.q = static_cast<const uint16_t*>(q);
@@ -457,13 +510,6 @@ extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void
   a.Hq = (int)Hq;
   a.Hkv = (int)Hkv;
   a.B = (int)B;
-  const dim3 grid((unsigned)(((S + aq::PA_QB - 1) / aq::PA_QB) * Hq * B));
-  a.paired = grid.x <= 2u * (unsigned)aq::device_cus();
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const size_t lds = (size_t)(aq::PA_KB * (D + 8) + D * (aq::PA_KB + 4)) * sizeof(uint16_t);
-  if (D == 128)
-    hipLaunchKernelGGL((aq::prefill_attn_kernel<128, true>), grid, dim3(256), lds, st, a);
-  else
-    hipLaunchKernelGGL((aq::prefill_attn_kernel<64, true>), grid, dim3(256), lds, st, a);
-  return (int)hipGetLastError();
+  return D == 128 ? aq::launch_prefill_attn<128, true>(a, st) : aq::launch_prefill_attn<64, true>(a, st);
 }

@@ -470,3 +470,27 @@ def test_qknorm_arguments_are_checked():
         ops.rope_kv_write(qkv, freqs, table, 0, kc, kc.clone(), Hq, Hkv, qk_norm=ops.QkNorm(g[:32], g, 1e-5))
     with pytest.raises(ValueError):
         ops.rope_paged_attn_decode(qkv, freqs, table, 1, kc, kc.clone(), Hq, Hkv, qk_norm=ops.QkNorm(g, g, -1.0))
+
+
+# (B, S, start, heads, page, D): two and four wavefronts to a query row, one where a launch fills the chip; blocks that
+# straddle pages, whole pages, a page table too long for LDS; ragged ends of query tiles and key blocks
+@pytest.mark.parametrize("B,S,start,Hq,Hkv,page,D", [(4, 290, 0, 8, 2, 16, 64), (4, 257, 77, 10, 2, 7, 64), (1, 33, 2090, 2, 1, 1, 64),
+                                                      (2, 65, 191, 3, 1, 64, 64), (16, 128, 1, 6, 2, 128, 64), (2, 129, 63, 4, 2, 64, 128),
+                                                      (8, 97, 130, 12, 3, 32, 128)])
+def test_prefill_attn_by_wavefronts_per_query_row(oracle, B, S, start, Hq, Hkv, page, D):
+    _say("prefill_attn wavefronts per row", B, S, start, Hq, Hkv, page, D)
+    T = start + S
+    P = -(-T // page)
+    g = torch.Generator().manual_seed(S + start + D)
+    q = (torch.randn(B, S, Hq, D, generator=g) * 1.5).to(torch.bfloat16)
+    kc = torch.randn(B * P, page, Hkv, D, generator=g).to(torch.bfloat16)
+    vc = torch.randn(B * P, page, Hkv, D, generator=g).to(torch.bfloat16)
+    table = torch.randperm(B * P, generator=g).view(B, P)
+    k, v = (c[table].reshape(B, P * page, Hkv, D)[:, :T].contiguous() for c in (kc, vc))
+    want = torch.from_numpy(oracle.c_prefill_attn_offset(_bits(q), _bits(k), _bits(v), start, D ** -0.5)
+                            .view(np.int16)).view(torch.bfloat16).float()
+    out = ops.prefill_attn_paged(q.to(DEV), kc.to(DEV), vc.to(DEV), table.to(DEV), start).cpu().float()
+    assert torch.allclose(out, want, rtol=1e-2, atol=1e-2)
+    assert ((out - want).norm() / want.norm()).item() < 5e-3
+    if start == 0:
+        assert torch.equal(out, ops.prefill_attn_causal(q.to(DEV), k.to(DEV), v.to(DEV)).cpu().float())
