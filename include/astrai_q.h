@@ -400,6 +400,24 @@ int aq_prefill_attn_paged(const void *q, int64_t q_stride, const void *k_cache, 
                           int64_t n_pages, void *out, float scale, int64_t B, int64_t S, int64_t Hq,
                           int64_t Hkv, int64_t D, void *stream);
 
+/* The two attention launches with ranges of memory to read ahead (at most three, 4-byte aligned, device
+ * memory): what the launches BEHIND attention will stream -- the weights of the output projection and of the
+ * MLP -- is brought into the last-level cache while attention leaves HBM idle.  A hint: results are those of
+ * the functions without it; ranges that are more than the library reads ahead (96 MiB in all), or a launch
+ * that fills the device by itself, are left alone. */
+typedef struct {
+  const void *ptr;
+  int64_t bytes;
+} aq_span;
+int aq_prefill_attn_causal_ahead(const void *q, int64_t q_stride, const void *k, int64_t k_stride,
+                                 const void *v, int64_t v_stride, void *out, float scale, int64_t B,
+                                 int64_t S, int64_t Hq, int64_t Hkv, int64_t D, const aq_span *ahead,
+                                 int n_ahead, void *stream);
+int aq_prefill_attn_paged_ahead(const void *q, int64_t q_stride, const void *k_cache, const void *v_cache,
+                                const int64_t *page_table, int64_t P, int64_t start, int64_t page_size,
+                                int64_t n_pages, void *out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                int64_t Hkv, int64_t D, const aq_span *ahead, int n_ahead, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -69,6 +69,10 @@ SYMBOLS = {
     "aq_gemv_w8a8_decode_attn": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "aq_prefill_attn_paged": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.c_float, _i64, _i64, _i64,
                                      _i64, _i64, _vp]),
+    "aq_prefill_attn_causal_ahead": (_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, ctypes.c_float, _i64, _i64, _i64, _i64, _i64,
+                                            _vp, _int, _vp]),
+    "aq_prefill_attn_paged_ahead": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.c_float, _i64, _i64,
+                                           _i64, _i64, _i64, _vp, _int, _vp]),
 }
 
 # csrc/aq_lab.h: the lab library's additions (measurement probes, the tile-forcing test hook)

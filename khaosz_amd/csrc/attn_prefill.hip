@@ -57,6 +57,9 @@ struct PrefillAttnArgs {
   int start, page_shift;
   int table_lds;  // entries of the page table that are copied into LDS first (all a launch needs, or 0: read from memory)
   int paired;     // != 0: the second half of the workgroups takes the query blocks lightest first
+  int wgs;        // workgroups that attend; the ones behind them read ahead
+  unsigned ahead_wgs;
+  Ahead ahead;
 };
 
 typedef __bf16 pa_bf16x8 __attribute__((ext_vector_type(8)));
@@ -89,6 +92,7 @@ __device__ __forceinline__ int row_key(int row) {
 // paged cache (the new tokens' rows have been written there already), causality is by position.
 template <int D, int QW, int KW, bool PAGED>
 __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(PrefillAttnArgs p) {
+  if ((int)blockIdx.x >= p.wgs) return read_ahead(p.ahead, (int)blockIdx.x - p.wgs, QW * KW * 64);
   constexpr int QB = 32 * QW;                       // query rows of the workgroup
   constexpr int KB = 64;                            // keys of a block
   constexpr int NT = KB / 32;                       // 32-key tiles of a block
@@ -407,6 +411,8 @@ constexpr int PA_TABLE_MAX = 2048;  // page-table entries kept in LDS
 template <int D, int QW, int KW, bool PAGED>
 static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
   const int64_t wgs = ((int64_t)(a.S + 32 * QW - 1) / (32 * QW)) * a.Hq * a.B;
+  a.wgs = (int)wgs;
+  if (wgs + AHEAD_WGS > 2 * device_cus()) a.ahead_wgs = 0;  // no room beside the workgroups that attend: they would run behind them
   constexpr int KB = 64, BUFS = 2 * KW * 2 * KB * 2 * D;
   a.paired = wgs <= (160 * 1024 / BUFS) * (int64_t)device_cus();
   size_t lds = BUFS;
@@ -415,7 +421,7 @@ static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
     a.table_lds = a.page % KB != 0 && entries <= PA_TABLE_MAX ? (int)entries : 0;
     lds += (size_t)a.table_lds * sizeof(int);
   }
-  hipLaunchKernelGGL((prefill_attn_kernel<D, QW, KW, PAGED>), dim3((unsigned)wgs), dim3(QW * KW * 64), lds, st, a);
+  hipLaunchKernelGGL((prefill_attn_kernel<D, QW, KW, PAGED>), dim3((unsigned)(wgs + a.ahead_wgs)), dim3(QW * KW * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 
@@ -441,9 +447,9 @@ static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
 
 }  // namespace aq
 
-extern "C" int aq_prefill_attn_causal(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+extern "C" int aq_prefill_attn_causal_ahead(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
                                       int64_t v_stride, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
-                                      int64_t Hkv, int64_t D, void* stream) {
+                                      int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
   if (D != 64 && D != 128) return AQ_E_SHAPE;
   if (B < 0 || S < 0 || Hq <= 0 || Hkv <= 0 || (Hq % Hkv) != 0 || !(scale > 0.0f)) return AQ_E_SHAPE;
   if (q_stride < Hq * D || k_stride < Hkv * D || v_stride < Hkv * D) return AQ_E_SHAPE;
@@ -457,7 +463,9 @@ extern "C" int aq_prefill_attn_causal(const void* q, int64_t q_stride, const voi
   // 32-bit byte offsets inside one sequence's K and V (a key block past the end included)
   if ((S + 64) * k_stride * 2 > (int64_t)0x7fffffff || (S + 64) * v_stride * 2 > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
+  if (n_ahead < 0 || (n_ahead > 0 && !ahead)) return AQ_E_NULL;
   aq::PrefillAttnArgs a{};
+  a.ahead_wgs = aq::set_ahead(a.ahead, ahead, n_ahead);
   a.q = static_cast<const uint16_t*>(q);
   a.k = static_cast<const uint16_t*>(k);
   a.v = static_cast<const uint16_t*>(v);
@@ -474,10 +482,16 @@ extern "C" int aq_prefill_attn_causal(const void* q, int64_t q_stride, const voi
   return D == 128 ? aq::launch_prefill_attn<128, false>(a, st) : aq::launch_prefill_attn<64, false>(a, st);
 }
 
-extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+extern "C" int aq_prefill_attn_causal(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                                      int64_t v_stride, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                      int64_t Hkv, int64_t D, void* stream) {
+  return aq_prefill_attn_causal_ahead(q, q_stride, k, k_stride, v, v_stride, out, scale, B, S, Hq, Hkv, D, nullptr, 0, stream);
+}
+
+extern "C" int aq_prefill_attn_paged_ahead(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
                                      const int64_t* page_table, int64_t P, int64_t start, int64_t page_size,
                                      int64_t n_pages, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
-                                     int64_t Hkv, int64_t D, void* stream) {
+                                     int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
   if (D != 64 && D != 128) return AQ_E_SHAPE;
   if (B < 0 || S < 0 || start < 0 || Hq <= 0 || Hkv <= 0 || (Hq % Hkv) != 0 || P <= 0 || page_size <= 0 ||
       n_pages <= 0 || !(scale > 0.0f) || q_stride < Hq * D)
@@ -491,7 +505,9 @@ extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void
   if (start + S > (1 << 30) || Hq > 65535 || B > 65535 ||
       ((S + 31) / 32) * Hq * B > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
+  if (n_ahead < 0 || (n_ahead > 0 && !ahead)) return AQ_E_NULL;
   aq::PrefillAttnArgs a{};
+  a.ahead_wgs = aq::set_ahead(a.ahead, ahead, n_ahead);
   a.q = static_cast<const uint16_t*>(q);
   a.out = static_cast<uint16_t*>(out);
   a.q_stride = q_stride;
@@ -512,4 +528,12 @@ extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void
   a.B = (int)B;
   hipStream_t st = static_cast<hipStream_t>(stream);
   return D == 128 ? aq::launch_prefill_attn<128, true>(a, st) : aq::launch_prefill_attn<64, true>(a, st);
+}
+
+extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+                                     const int64_t* page_table, int64_t P, int64_t start, int64_t page_size,
+                                     int64_t n_pages, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                     int64_t Hkv, int64_t D, void* stream) {
+  return aq_prefill_attn_paged_ahead(q, q_stride, k_cache, v_cache, page_table, P, start, page_size, n_pages, out, scale, B, S, Hq,
+                                     Hkv, D, nullptr, 0, stream);
 }

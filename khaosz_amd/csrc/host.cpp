@@ -53,8 +53,8 @@ namespace {
   X(aq_paged_attn_decode_slices)                                                                                 \
   X(aq_paged_attn_decode_partials_bytes)                                                                         \
   X(aq_paged_attn_decode_workspace_bytes)                                                                        \
-  X(aq_prefill_attn_causal)                                                                                      \
-  X(aq_prefill_attn_paged)
+  X(aq_prefill_attn_causal_ahead)                                                                                \
+  X(aq_prefill_attn_paged_ahead)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -785,12 +785,15 @@ int Block::queue(const void* in, void* out, const char** what) const {
                                                kn.p, qn.eps, c.stream)
                  : lib.aq_rope_kv_write(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, qr, kr, B, Hq, Hkv, D, c.stream);
     if (rc) return rc;
+    // what streams behind attention, which itself leaves HBM idle
+    const aq_span ahead[3] = {{o.w, o.N * o.K}, {ug.w, ug.N * ug.K}, {down.w, down.N * down.K}};
     if (direct) {
       *what = "aq_prefill_attn_causal";
-      rc = lib.aq_prefill_attn_causal(qr, A, kr, KV, q + 2 * (A + KV), W, att, scale, B, S, Hq, Hkv, D, c.stream);
+      rc = lib.aq_prefill_attn_causal_ahead(qr, A, kr, KV, q + 2 * (A + KV), W, att, scale, B, S, Hq, Hkv, D, ahead, 3, c.stream);
     } else {
       *what = "aq_prefill_attn_paged";
-      rc = lib.aq_prefill_attn_paged(qr, A, kc, vc, table, P, total - S, page, n_pages, att, scale, B, S, Hq, Hkv, D, c.stream);
+      rc = lib.aq_prefill_attn_paged_ahead(qr, A, kc, vc, table, P, total - S, page, n_pages, att, scale, B, S, Hq, Hkv, D, ahead, 3,
+                                           c.stream);
     }
     if (rc) return rc;
     rc = projected(o, att, in, x1, at_codes);

@@ -494,3 +494,24 @@ def test_prefill_attn_by_wavefronts_per_query_row(oracle, B, S, start, Hq, Hkv, 
     assert ((out - want).norm() / want.norm()).item() < 5e-3
     if start == 0:
         assert torch.equal(out, ops.prefill_attn_causal(q.to(DEV), k.to(DEV), v.to(DEV)).cpu().float())
+
+
+def test_prefill_attn_reading_ahead_changes_nothing():
+    """Spans that the attention launch reads ahead: none, ragged ends, more than it takes, a launch without room."""
+    import ctypes
+    lib = ops._abi.load()
+    g = torch.Generator().manual_seed(5)
+    weights = [torch.zeros(n, dtype=torch.int8, device=DEV) for n in (3, 128, 1000, 300000)]
+    over = torch.zeros(97 << 20, dtype=torch.int8, device=DEV)
+    for B, S, Hq, Hkv in ((2, 70, 4, 2), (4, 512, 40, 8)):
+        q, k, v = (torch.randn(B, S, h * 64, generator=g).to(torch.bfloat16).to(DEV) for h in (Hq, Hkv, Hkv))
+        want = ops.prefill_attn_causal(q.view(B, S, Hq, 64), k.view(B, S, Hkv, 64), v.view(B, S, Hkv, 64))
+        for chosen in ((), weights[:3], weights[1:], weights[3:], [over]):
+            spans = (ctypes.c_int64 * 6)(*[x for t in chosen for x in (t.data_ptr(), t.numel())])
+            out = torch.empty_like(want)
+            assert lib.aq_prefill_attn_causal_ahead(q.data_ptr(), Hq * 64, k.data_ptr(), Hkv * 64, v.data_ptr(), Hkv * 64,
+                                                    out.data_ptr(), 0.125, B, S, Hq, Hkv, 64, ctypes.addressof(spans),
+                                                    len(chosen), torch.cuda.current_stream().cuda_stream) == 0
+            assert torch.equal(out, want)
+    assert lib.aq_prefill_attn_causal_ahead(q.data_ptr(), Hq * 64, k.data_ptr(), Hkv * 64, v.data_ptr(), Hkv * 64, out.data_ptr(),
+                                            0.125, B, S, Hq, Hkv, 64, None, 2, 0) != 0
