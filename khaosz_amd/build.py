@@ -27,7 +27,7 @@ OBJ_DIR = os.path.join(HERE, "lib", "obj")
 LIB = os.path.join(HERE, "lib", "libastrai_q.so")
 LAB_LIB = os.path.join(HERE, "lib", "libastrai_q_lab.so")
 HOST_EXT = os.path.join(HERE, "_host.so")
-SOURCES = ["abi.hip", "quant.hip", "gemm_mfma.hip", "gemv.hip", "gemv_rows.hip", "attn_decode.hip", "attn_prefill.hip"]
+SOURCES = ["abi.hip", "quant.hip", "gemm_mfma.hip", "gemm_walk.hip", "gemv.hip", "gemv_rows.hip", "attn_decode.hip", "attn_prefill.hip"]
 # (source, object, extra flags) of the lab library's own objects; the other product objects are shared
 LAB_SOURCES = [("gemm_mfma.hip", "gemm_mfma_lab.o", ["-DAQ_LAB"]), ("gemv_rows.hip", "gemv_rows_lab.o", ["-DAQ_LAB"]),
                ("lab.hip", "lab.o", [])]
@@ -72,7 +72,8 @@ def build(force: bool = True, verbose: bool = False, stall_counters: bool = Fals
     os.makedirs(OBJ_DIR, exist_ok=True)
     lab_sources = [(src, obj, extra + (["-DAQ_LAB_STALL"] if stall_counters and src == "gemm_mfma.hip" else []))
                    for src, obj, extra in LAB_SOURCES]
-    headers = [os.path.join(CSRC, "aq_common.h"), os.path.join(CSRC, "aq_rows.h"), os.path.join(CSRC, "aq_gemv.h"), os.path.join(CSRC, "aq_lab.h"),
+    headers = [os.path.join(CSRC, "aq_common.h"), os.path.join(CSRC, "aq_rows.h"), os.path.join(CSRC, "aq_gemv.h"), os.path.join(CSRC, "aq_gemm.h"),
+               os.path.join(CSRC, "aq_lab.h"),
                os.path.join(HERE, "..", "include", "astrai_q.h")]
 
     def compile_one(job):

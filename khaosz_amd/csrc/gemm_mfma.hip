@@ -17,9 +17,7 @@
 // later sub-steps are issued between the MFMAs of the current one, with one
 // workgroup barrier per K step.  The epilogue is fused and runs straight from
 // the accumulator registers: int32 store, or dequantise (+bias) and cast.
-#include <type_traits>
-
-#include "aq_common.h"
+#include "aq_gemm.h"
 
 namespace aq {
 
@@ -98,24 +96,6 @@ using ShapeTall = Shape<2, 2, 4, 2, 1, 128, 3>;
 using ShapeHuge8 = Shape<4, 2, 2, 4, 1, 64, 4>;
 using ShapePair = Shape<2, 2, 2, 2, 2, 128, 3>;
 #endif
-constexpr int NUM_XCD = 8;
-constexpr int GROUP_M = 4;
-
-enum { OUT_I32 = 0, OUT_F32 = 1, OUT_BF16 = 2 };
-
-struct GemmArgs {
-  const uint8_t* A;
-  const uint8_t* B;
-  void* C;
-  int M, N, K;
-  int tiles_m, tiles_n;
-  const float* sx;   // int8: [M]; fp8: [1]
-  const float* sw;   // int8: [N]; fp8: [1]
-  const void* bias;  // [N] or null
-  int bias_dtype;
-  const void* res;   // [M, N] residual in the output's type, or null; may be C itself
-};
-
 // Workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2.
 // Re-number them so that one XCD owns a contiguous run of tile ids, and walk
 // tile ids in GROUP_M-tall column-major groups, so the tiles resident on an
@@ -133,56 +113,6 @@ __device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n,
   const int in_group = tile - group * group_sz;
   tm = first_m + in_group % gm;
   tn = in_group / gm;
-}
-
-template <bool FP8>
-struct Acc {
-  using type = v16i;
-};
-template <>
-struct Acc<true> {
-  using type = v16f;
-};
-
-// s_waitcnt with only the vector-memory counter constrained (gfx9 encoding:
-// vmcnt in bits 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima).
-#define AQ_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((n) & 15) | (((n) >> 4) << 14))
-// Workgroup barrier without the memory fence of __syncthreads(): the fence
-// would drain every outstanding global->LDS load, including the ones issued
-// two K steps ahead on purpose.  The empty asm statements stop the compiler
-// from moving LDS accesses across it.
-#define AQ_BARRIER()                   \
-  do {                                 \
-    asm volatile("" ::: "memory");     \
-    __builtin_amdgcn_s_barrier();      \
-    asm volatile("" ::: "memory");     \
-  } while (0)
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-
-template <bool FP8>
-struct Frag {
-  using type = v4i;  // 16 bytes of K per lane: v_mfma_i32_32x32x32_i8
-};
-template <>
-struct Frag<true> {
-  using type = v8i;  // 32 bytes of K per lane: v_mfma_scale_f32_32x32x64_f8f6f4
-};
-
-#ifndef AQ_FP8_SCALE
-#define AQ_FP8_SCALE 0
-#endif
-template <bool FP8>
-__device__ __forceinline__ typename Acc<FP8>::type mma(const typename Frag<FP8>::type& a,
-                                                       const typename Frag<FP8>::type& b,
-                                                       const typename Acc<FP8>::type& c) {
-  if constexpr (!FP8) {
-    return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-  } else {
-    // E8M0 scale 127 = 2^0 for both operands: plain e4m3 x e4m3.
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, AQ_FP8_SCALE, 0, AQ_FP8_SCALE);
-  }
 }
 
 // Issue order of one pipeline slot, as scheduling groups: GROUPS times
@@ -907,7 +837,11 @@ static int launch(GemmArgs& a, hipStream_t st) {
   if constexpr (FP8 && OUT != OUT_I32) {
     if (!forced && huge_fp8_ok(a)) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
   }
-  switch (choose_tile(a.M, a.N)) {
+  const int tile = choose_tile(a.M, a.N);
+  if constexpr (OUT == OUT_BF16) {  // more tiles than compute units: the kernel whose K loop goes on from tile to tile
+    if (!forced && tile == TILE_LARGE && gemm_walk_ok(a)) return gemm_walk_launch<FP8>(a, st);
+  }
+  switch (tile) {
     case TILE_SMALL: return launch_shape<FP8, OUT, ShapeSmall>(a, st);
     case TILE_N64: return launch_shape<FP8, OUT, ShapeN64>(a, st);
     case TILE_N32: return launch_shape<FP8, OUT, ShapeN32>(a, st);

@@ -1300,3 +1300,26 @@ def test_full_size_fp8_linearity_in_scales(oracle):
     assert np.max(np.abs(to_np(y[rows]) - exact)) <= 1e-3 * rms
     ref = torch.nn.functional.linear(x[rows].float(), w)
     assert ((y[rows] - ref).norm() / ref.norm()).item() < 0.06
+
+
+# more 256 x 128 tiles than compute units: whole rounds, a last round of whole and of halved tiles, ragged M (a half tile
+# that is all padding) and N, the shortest K that walks, K steps that fill the three buffers unevenly
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K", [(4096, 2176, 512), (2049, 4100, 640), (8192, 3200, 512), (4225, 6402, 768), (4000, 6400, 1024)])
+def test_gemm_walking_tiles(M, N, K, bias):
+    """The walk against the kernel of one tile shape after another (its own tests hold that against the oracle): same bits."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if -(-M // 256) * -(-N // 128) <= cus:
+        pytest.skip("one round on this device")
+    _say("gemm walk", M, N, K, bias)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    xq, wq = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
+    sx, sw = (torch.rand(n, generator=g, device=DEV) * 0.01 + 1e-4 for n in (M, N))
+    b = torch.randn(N, generator=g, device=DEV).to(torch.bfloat16) if bias else None
+    y = ops.linear_w8a8(xq, sx, wq, sw, b, out_dtype=torch.bfloat16)
+    x8, w8 = (torch.randn(n, K, generator=g, device=DEV).to(torch.float8_e4m3fn).view(torch.uint8) for n in (M, N))
+    y8 = ops.linear_fp8(x8, sx[:1], w8, sw[:1], b, out_dtype=torch.bfloat16)
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(256) == 0
+        assert torch.equal(y, ops.linear_w8a8(xq, sx, wq, sw, b, out_dtype=torch.bfloat16))
+        assert torch.equal(y8, ops.linear_fp8(x8, sx[:1], w8, sw[:1], b, out_dtype=torch.bfloat16))
