@@ -247,6 +247,47 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_kernel(const void* __restri
   }
 }
 
+// A row with some gate outside the range of the main path (an outlier beyond +-80, a denormal): rare, so it is simply done
+// again with the general divide, in two rolled loops that keep nothing in registers (maximum, then codes) and leave
+// the main path's register budget alone.
+template <bool BF16, int NC>
+__device__ __forceinline__ void swiglu_row_general(__amdgpu_buffer_rsrc_t Ur, __amdgpu_buffer_rsrc_t Gr, int nvec, int lane, int8_t* dst,
+                                                   float* scale) {
+  constexpr int EPV = RowIn<BF16>::EPV;
+  float am = 0.0f;
+  for (int i = 0; i < NC; ++i) {
+    const uint32_t off = (uint32_t)(i * 64 + lane) * 16u;
+    float u[EPV], g[EPV];
+    RowIn<BF16>::unpack(buffer_load_16(Ur, off), u);
+    RowIn<BF16>::unpack(buffer_load_16(Gr, off), g);
+#pragma unroll
+    for (int e = 0; e < EPV; ++e) am = fmaxf(am, fabsf(swiglu_repro(u[e], g[e])));
+  }
+  const RowScale rsc = row_scale(wave_max(am));
+  if (lane == 0) *scale = rsc.s;
+  for (int i = 0; i < NC; ++i) {
+    const int v = i * 64 + lane;
+    const uint32_t off = (uint32_t)v * 16u;
+    float u[EPV], g[EPV], hh[EPV];
+    uint32_t code[EPV / 4];
+    RowIn<BF16>::unpack(buffer_load_16(Ur, off), u);
+    RowIn<BF16>::unpack(buffer_load_16(Gr, off), g);
+#pragma unroll
+    for (int e = 0; e < EPV; ++e) hh[e] = swiglu_repro(u[e], g[e]);
+    quant_codes_packed<EPV>(hh, rsc.s, rsc.rs, rsc.fast_ok, code);
+    if (v < nvec) {
+      if constexpr (BF16) {
+        uint2 o;
+        o.x = code[0];
+        o.y = code[1];
+        store_wt(reinterpret_cast<uint2*>(dst + (int64_t)v * EPV), o);
+      } else {
+        store_wt(reinterpret_cast<uint32_t*>(dst + (int64_t)v * EPV), code[0]);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------ SwiGLU -> row quantise
 //
 // h = up * silu(gate) for one row of the fused up/gate projection's output
@@ -321,41 +362,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     int8_t* dst = q + row * (int64_t)F;
     if constexpr (BF16) ok = range.ok();
     if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
-      // Some gate of the row lies outside the range of the short divide (an outlier beyond +-80, a denormal):
-      // rare, so the row is simply done again with the general divide, in two rolled loops that keep nothing in
-      // registers (maximum, then codes) and leave the main path's register budget alone.
-      float am = 0.0f;
-      for (int i = 0; i < NC; ++i) {
-        const uint32_t off = (uint32_t)(i * 64 + lane) * 16u;
-        float u[EPV], g[EPV];
-        RowIn<BF16>::unpack(buffer_load_16(Ur, off), u);
-        RowIn<BF16>::unpack(buffer_load_16(Gr, off), g);
-#pragma unroll
-        for (int e = 0; e < EPV; ++e) am = fmaxf(am, fabsf(swiglu_repro(u[e], g[e])));
-      }
-      const RowScale rsc = row_scale(wave_max(am));
-      if (lane == 0) scale[row] = rsc.s;
-      for (int i = 0; i < NC; ++i) {
-        const int v = i * 64 + lane;
-        const uint32_t off = (uint32_t)v * 16u;
-        float u[EPV], g[EPV], hh[EPV];
-        uint32_t code[EPV / 4];
-        RowIn<BF16>::unpack(buffer_load_16(Ur, off), u);
-        RowIn<BF16>::unpack(buffer_load_16(Gr, off), g);
-#pragma unroll
-        for (int e = 0; e < EPV; ++e) hh[e] = swiglu_repro(u[e], g[e]);
-        quant_codes_packed<EPV>(hh, rsc.s, rsc.rs, rsc.fast_ok, code);
-        if (v < nvec) {
-          if constexpr (BF16) {
-            uint2 o;
-            o.x = code[0];
-            o.y = code[1];
-            store_wt(reinterpret_cast<uint2*>(dst + (int64_t)v * EPV), o);
-          } else {
-            store_wt(reinterpret_cast<uint32_t*>(dst + (int64_t)v * EPV), code[0]);
-          }
-        }
-      }
+      swiglu_row_general<BF16, NC>(Ur, Gr, nvec, lane, dst, scale + row);
       continue;
     }
     const RowScale rsc = row_scale(wave_max(amax));
@@ -378,6 +385,97 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
                                               i * 256, STORE_WT);
       }
     }
+  }
+}
+
+// The bf16 kernel for many rows: silu of a bf16 gate is a function of 16 bits, so a workgroup first tabulates it in LDS
+// (same operations, same bits) and a product costs an LDS read instead of an exponential and a divide: 15 operations
+// per element instead of 34 of what bounds these kernels.
+//
+// Entry i of either sign is silu of the bf16 pattern LUT_LOW + i: 2^-31 <= |g| < 128.  Smaller gates, zeros among them
+// (a prompt's rows hold a hundred), take the first entry: |h| <= max |u| 2^-31, which rounds to the code 0 and is no
+// maximum as long as the row's maximum is 2^10 times that.  Rows where it is not, or with a gate beyond, are done again.
+// The sign goes to bit 15 of the index, so that both halves of a pair of gates are a shift and an and away from their
+// byte offsets; the negative gates' entries then lie 128 KiB further up and the table spans a compute unit's LDS: one
+// workgroup each, a wavefront per row, rows dealt out over the compute units first.  Filling it takes 1.5 us of
+// arithmetic, most of it while the first rows are on their way.
+constexpr uint32_t LUT_LOW = 96u << 7, LUT_SIZE = 38u << 7;
+template <int NC>
+__global__ __launch_bounds__(NC <= 12 ? 1024 : 768) void swiglu_quant_lut_kernel(const void* __restrict__ ug, int64_t M, int F,
+                                                                                int64_t ld, int8_t* __restrict__ q,
+                                                                                float* __restrict__ scale) {
+  constexpr int NW = NC <= 12 ? 16 : 12;  // 128 or 168 registers a wavefront: a row's h is 8 NC of them
+  __shared__ __attribute__((aligned(16))) float table[0x8000 + LUT_SIZE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t row_bytes = (uint32_t)F * 2u;
+  uint4 cu[NC], cg[NC];
+  auto half_row = [&](int64_t row, int half) {
+    return make_rsrc(reinterpret_cast<const char*>(ug) + row * ld * 2 + half * (int64_t)row_bytes, row_bytes);
+  };
+  auto load = [&](int64_t row) {
+    const __amdgpu_buffer_rsrc_t Ur = half_row(row, 0), Gr = half_row(row, 1);  // vectors past the row read as zeros
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const uint32_t off = (uint32_t)(i * 64 + lane) * 16u;
+      cu[i] = buffer_load_16(Ur, off);
+      cg[i] = buffer_load_16(Gr, off);
+      __builtin_amdgcn_sched_barrier(0);  // pair by pair: they are waited for in this order
+    }
+    asm volatile("" ::: "memory");
+  };
+  int64_t row = blockIdx.x + (int64_t)wave * gridDim.x;
+  if (row < M) load(row);  // wavefront-uniform
+  for (uint32_t i = threadIdx.x; i < 2 * LUT_SIZE; i += NW * 64) {
+    const uint32_t neg = i >= LUT_SIZE ? 1u : 0u, at = i - neg * LUT_SIZE;
+    const float g = __uint_as_float((LUT_LOW + at + neg * 0x8000u) << 16);
+    table[at + neg * 0x8000u] = __fdiv_rn(g, __fadd_rn(1.0f, exp_repro(-g)));
+  }
+  __syncthreads();
+  const char* const lut = reinterpret_cast<const char*>(table);
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  for (; row < M; row += (int64_t)NW * gridDim.x) {
+    float h[NC][8];
+    float amax = 0.0f, umax = 0.0f;
+    u16x2 top = {0, 0};
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const uint32_t w[4] = {cg[i].x, cg[i].y, cg[i].z, cg[i].w};
+      float u[8];
+      RowIn<true>::unpack(cu[i], u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u16x2 at = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, w[e] & 0x7fff7fffu), (u16x2){LUT_LOW, LUT_LOW});
+        top = __builtin_elementwise_max(top, at);
+        const uint32_t x = __builtin_bit_cast(uint32_t, at) | (w[e] & 0x80008000u);
+        h[i][2 * e] = __fmul_rn(u[2 * e], *reinterpret_cast<const float*>(lut + ((x << 2) & 0x27ffcu)));
+        h[i][2 * e + 1] = __fmul_rn(u[2 * e + 1], *reinterpret_cast<const float*>(lut + ((x >> 14) & 0x27ffcu)));
+      }
+      amax = fmaxf(amax, vec_amax<8>(h[i]));
+      umax = fmaxf(umax, vec_amax<8>(u));
+      asm volatile("" ::"v"(h[i][0]), "v"(h[i][1]), "v"(h[i][2]), "v"(h[i][3]), "v"(h[i][4]), "v"(h[i][5]), "v"(h[i][6]), "v"(h[i][7]));
+      __builtin_amdgcn_sched_barrier(0);  // pairs in the order they arrive
+    }
+    int8_t* dst = q + row * (int64_t)F;
+    amax = wave_max(amax);
+    const bool ok = (top.x > top.y ? top.x : top.y) < LUT_SIZE && umax * 4.76837158203125e-7f <= amax && umax < INFINITY;  // 2^-21
+    if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
+      swiglu_row_general<true, NC>(half_row(row, 0), half_row(row, 1), F / 8, lane, dst, scale + row);
+    } else {
+      const RowScale rsc = row_scale(amax);
+      if (lane == 0) scale[row] = rsc.s;
+      const __amdgpu_buffer_rsrc_t Qr = make_rsrc(dst, (uint32_t)F);
+#pragma unroll
+      for (int i = 0; i < NC; ++i) {
+        uint32_t code[2];
+        quant_codes_packed<8>(h[i], rsc.s, rsc.rs, rsc.fast_ok, code);
+        typedef int v2i_t __attribute__((ext_vector_type(2)));
+        const v2i_t o = {(int)code[0], (int)code[1]};
+        __builtin_amdgcn_raw_buffer_store_b64(o, Qr, lane * 8, i * 512, STORE_WT);
+      }
+    }
+    const int64_t next = row + (int64_t)NW * gridDim.x;
+    if (next < M) load(next);
   }
 }
 
@@ -810,6 +908,26 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
                                hipStream_t st) {
   const int64_t vpl = (F / (BF16 ? 8 : 4) + 63) / 64;  // vector pairs per lane
   if (vpl > 16) return AQ_E_RANGE;
+  // many bf16 rows: the kernel that looks silu up.  Up to 1024 rows (1280 of more than 12 pairs per lane, twelve wavefronts
+  // to a compute unit) its table costs more than it saves: 1024 x 4096 6.8 us against 6.2 with a workgroup per row,
+  // 1100 x 6912 12.6 against 12.1; from there on us, before -> now: 1100 x 5632 14.7 -> 10.1, 2048 x 6912 20.0 -> 16.5,
+  // 4096 x 5632 28.5 -> 23.5, 4096 x 6912 38 -> 28, 8192 x 8192 89 -> 72, 2048 x 2048 6.5 -> 6.3 (shorter rows stay).
+  if constexpr (BF16) {
+    if (vpl >= 4 && vpl <= 16 && M > (vpl > 12 ? 1280 : 1024)) {
+      const dim3 g((unsigned)aq::device_cus());
+      switch (vpl) {
+#define AQ_SWIGLU_CASE(nc)                                                                                                      \
+  case nc:                                                                                                                      \
+    hipLaunchKernelGGL((aq::swiglu_quant_lut_kernel<nc>), g, dim3(nc <= 12 ? 1024 : 768), 0, st, ug, M, (int)F, ld, q, scale); \
+    break;
+        AQ_SWIGLU_CASE(4) AQ_SWIGLU_CASE(5) AQ_SWIGLU_CASE(6) AQ_SWIGLU_CASE(7) AQ_SWIGLU_CASE(8) AQ_SWIGLU_CASE(9)
+        AQ_SWIGLU_CASE(10) AQ_SWIGLU_CASE(11) AQ_SWIGLU_CASE(12) AQ_SWIGLU_CASE(13) AQ_SWIGLU_CASE(14) AQ_SWIGLU_CASE(15)
+        AQ_SWIGLU_CASE(16)
+#undef AQ_SWIGLU_CASE
+      }
+      return (int)hipGetLastError();
+    }
+  }
   // few rows, or rows too long for one wavefront's registers: a workgroup of vpl wavefronts per row
   if (vpl > 1 && (M <= AQ_SWIGLU_WG_MAX_M || vpl > 12)) {
     hipLaunchKernelGGL((aq::swiglu_quant_wg_kernel<BF16>), dim3((unsigned)M), dim3((unsigned)vpl * 64), 0, st, ug, (int)F,
@@ -827,11 +945,17 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
   switch (vpl) {
 #define AQ_SWIGLU_CASE(nc)                                                                                   \
   case nc: hipLaunchKernelGGL((aq::swiglu_quant_kernel<BF16, nc>), g, b, 0, st, ug, M, (int)F, ld, q, scale); break;
-    AQ_SWIGLU_CASE(1) AQ_SWIGLU_CASE(2) AQ_SWIGLU_CASE(3) AQ_SWIGLU_CASE(4) AQ_SWIGLU_CASE(5) AQ_SWIGLU_CASE(6)
-    AQ_SWIGLU_CASE(7) AQ_SWIGLU_CASE(8) AQ_SWIGLU_CASE(9) AQ_SWIGLU_CASE(10) AQ_SWIGLU_CASE(11) AQ_SWIGLU_CASE(12)
-#undef AQ_SWIGLU_CASE
-    default: return AQ_E_RANGE;
+    AQ_SWIGLU_CASE(1) AQ_SWIGLU_CASE(2) AQ_SWIGLU_CASE(3)
+    default: break;
   }
+  if constexpr (!BF16) {
+    switch (vpl) {
+      AQ_SWIGLU_CASE(4) AQ_SWIGLU_CASE(5) AQ_SWIGLU_CASE(6) AQ_SWIGLU_CASE(7) AQ_SWIGLU_CASE(8) AQ_SWIGLU_CASE(9)
+      AQ_SWIGLU_CASE(10) AQ_SWIGLU_CASE(11) AQ_SWIGLU_CASE(12)
+      default: break;
+    }
+  }
+#undef AQ_SWIGLU_CASE
   return (int)hipGetLastError();
 }
 

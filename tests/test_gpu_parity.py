@@ -1323,3 +1323,32 @@ def test_gemm_walking_tiles(M, N, K, bias):
         assert lab.aq_lab_set_gemm_tile(256) == 0
         assert torch.equal(y, ops.linear_w8a8(xq, sx, wq, sw, b, out_dtype=torch.bfloat16))
         assert torch.equal(y8, ops.linear_fp8(x8, sx[:1], w8, sw[:1], b, out_dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,F", [(1025, 2048), (1300, 6928), (1041, 2064), (2050, 4096)])
+def test_swiglu_quant_of_many_bf16_rows(oracle, M, F):
+    """Many rows take the kernel that looks silu up: every bf16 gate pattern, zeros, gates around both ends of its table,
+    rows whose maximum is small against their up half, and rows of ordinary values with a few zeros, against the oracle."""
+    _say("swiglu_quant many rows", M, F)
+    g = torch.Generator().manual_seed(M + F)
+    ug = torch.randn(M, 2 * F, generator=g).to(torch.bfloat16)
+    up, gate = ug[:, :F], ug[:, F:]
+    gate[torch.randint(0, M, (100,), generator=g), torch.randint(0, F, (100,), generator=g)] = 0.0
+    every = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    every = every[torch.isfinite(every.float())]
+    n = every.numel() // F
+    gate[:n] = every[:n * F].view(n, F)[:, torch.randperm(F, generator=g)]
+    up[:n] = 0.75  # no product overflows
+    inside = every[(every.float().abs() < 120) & ((every.float() == 0) | (every.float().abs() > 1e-12))]
+    at = torch.randint(0, inside.numel(), (20, F), generator=g)
+    gate[n:n + 20] = inside[at]                      # rows wholly inside the table, zeros among them
+    for i, v in enumerate((127.5, 128.0, -127.5, -128.0, 2.0 ** -31, 2.0 ** -32, -(2.0 ** -31), 1e-38)):
+        gate[n + 20 + i, i::97] = v
+    gate[n + 30], gate[n + 31] = 0.0, -0.0
+    up[n + 32], gate[n + 33] = 0.0, 1e-9             # an all-zero row, a row of small gates
+    up[n + 34, 5], gate[n + 34, 5] = 1e30, 0.0       # a large up value behind a zero gate
+    d = ug.to(DEV)
+    q, s = ops.swiglu_quant_rowwise_i8(d)
+    qo, so = oracle.c_swiglu_quant_i8(bf16_bits(d), bf16_bits=True)
+    assert np.array_equal(to_np(s), so)
+    assert np.array_equal(to_np(q), qo)
