@@ -106,6 +106,10 @@ int aq_linear_w8a8(const int8_t *xq, const float *sx, const int8_t *wq, const fl
  * astrai/inference/core/executor.py:59-94).
  * ws: device scratch of at least aq_gemv_w8a8_workspace_bytes(M, K). */
 size_t aq_gemv_w8a8_workspace_bytes(int64_t M, int64_t K);
+
+/* 1 where the decode entry points below (norm != 0: ..._rmsnorm) quantise the rows inside their one launch: ws is
+ * not touched then, and any 16-byte aligned pointer will do for it. */
+int aq_gemv_w8a8_decode_one_launch(int x_dtype, int norm, int64_t M, int64_t N, int64_t K);
 int aq_gemv_w8a8_decode(const void *x, int x_dtype, const int8_t *wq, const float *sw,
                         const void *bias, int bias_dtype, void *y, int y_dtype, int64_t M,
                         int64_t N, int64_t K, void *ws, size_t ws_bytes, void *stream);
@@ -206,6 +210,7 @@ int aq_linear_fp8_residual(const uint8_t *xq, const float *sx, const uint8_t *wq
  * aq_quant_tensor_fp8 + the codes entry.  K not a multiple of 256, or rows too long for a compute unit's
  * LDS: the tiled FP8 GEMM takes the call.  Replaces F.linear (linear.py:21) in the FP8 variant. */
 size_t aq_gemv_fp8_workspace_bytes(int64_t M, int64_t K);
+int aq_gemv_fp8_decode_one_launch(int x_dtype, int64_t M, int64_t K); /* as aq_gemv_w8a8_decode_one_launch */
 int aq_gemv_fp8_codes_residual(const uint8_t *xq, const float *sx, const uint8_t *wq, const float *sw,
                                const void *bias, int bias_dtype, const void *residual, void *y,
                                int y_dtype, int64_t M, int64_t N, int64_t K, void *stream);

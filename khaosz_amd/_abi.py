@@ -69,6 +69,8 @@ SYMBOLS = {
     "aq_gemv_w8a8_decode_attn": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "aq_prefill_attn_paged": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.c_float, _i64, _i64, _i64,
                                      _i64, _i64, _vp]),
+    "aq_gemv_w8a8_decode_one_launch": (_int, [_int, _int, _i64, _i64, _i64]),
+    "aq_gemv_fp8_decode_one_launch": (_int, [_int, _i64, _i64]),
     "aq_prefill_attn_causal_ahead": (_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, ctypes.c_float, _i64, _i64, _i64, _i64, _i64,
                                             _vp, _int, _vp]),
     "aq_prefill_attn_paged_ahead": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.c_float, _i64, _i64,

@@ -885,6 +885,11 @@ extern "C" size_t aq_gemv_w8a8_workspace_bytes(int64_t M, int64_t K) {
 // *mt_out: the token-count bucket of the GEMV kernels, or -1 when the activation codes of that bucket do
 // not fit the LDS of a compute unit (rows longer than 10 096 bytes at 9..16 tokens, 20 208 at 5..8, ...):
 // such a call is served by the tiled MFMA GEMM, which takes any M (same integer sums, same epilogue: same bits).
+static int gemv_bucket(int64_t M, int64_t K) {
+  const int mt = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
+  return (int64_t)mt * K + 64 + 2048 > aq::GV_MAX_LDS ? -1 : mt;  // codes, scales, K-part sums
+}
+
 static int gemv_check(const int8_t* wq, const float* sw, const void* bias, int bias_dtype, const void* residual,
                       const void* y, int y_dtype, int64_t M, int64_t N, int64_t K, int* mt_out) {
   if (y_dtype != AQ_F32 && y_dtype != AQ_BF16) return AQ_E_DTYPE;
@@ -896,8 +901,7 @@ static int gemv_check(const int8_t* wq, const float* sw, const void* bias, int b
   if (aq::check_ptr16(wq) || aq::check_ptr16(y) || aq::check_ptr16(residual)) return AQ_E_ALIGN;
   if (aq::check_ptr(sw, 4) || aq::check_ptr(bias, bias_dtype == AQ_BF16 ? 2 : 4)) return AQ_E_ALIGN;
   if (N > (1 << 25) || K > (1 << 22)) return AQ_E_RANGE;  // 16 rows of N outputs are indexed in 32 bits
-  const int mt = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
-  *mt_out = (int64_t)mt * K + 64 + 2048 > aq::GV_MAX_LDS ? -1 : mt;  // codes, scales, K-part sums
+  *mt_out = gemv_bucket(M, K);
   return AQ_OK;
 }
 
@@ -931,14 +935,22 @@ static bool dot_kernel_better(int64_t M, int64_t N, int64_t K, bool norm) {
   return M < 3 || N > 2048;
 }
 
+enum FusedRoute { FUSED_NONE, FUSED_DOT, FUSED_ROWS };
+static aq::RowsKind fused_kind(bool norm, bool bf16) { return norm ? aq::ROWS_I8_NORM : bf16 ? aq::ROWS_I8 : aq::ROWS_I8_F32; }
+static FusedRoute fused_route(int x_dtype, bool norm, int mt, int64_t M, int64_t N, int64_t K) {
+  const bool bf16 = x_dtype == AQ_BF16;
+  const int64_t vpl = (K / 8 + 63) / 64;  // 16-byte vectors per lane per bf16 row
+  const bool dot = bf16 && M <= 4 && mt > 0 && vpl <= (norm ? 4 : 16);
+  if ((bf16 || !norm) && aq::gemv_rows_ok(fused_kind(norm, bf16), M, K) && !(dot && dot_kernel_better(M, N, K, norm))) return FUSED_ROWS;
+  return dot ? FUSED_DOT : FUSED_NONE;
+}
+
 static int gemv_dispatch_fused(const aq::GemvArgs& a, int x_dtype, int mt, hipStream_t st) {
-  const bool norm = a.gamma != nullptr, bf16 = x_dtype == AQ_BF16;
-  const int64_t vpl = (a.K / 8 + 63) / 64;  // 16-byte vectors per lane per bf16 row
-  const bool dot = bf16 && a.M <= 4 && mt > 0 && vpl <= (norm ? 4 : 16);
-  const aq::RowsKind kind = norm ? aq::ROWS_I8_NORM : bf16 ? aq::ROWS_I8 : aq::ROWS_I8_F32;
-  if ((bf16 || !norm) && aq::gemv_rows_ok(kind, a.M, a.K) && !(dot && dot_kernel_better(a.M, a.N, a.K, norm)))
-    return aq::launch_gemv_rows(a, kind, st);
-  if (!dot) return -1;
+  const bool norm = a.gamma != nullptr;
+  const int64_t vpl = (a.K / 8 + 63) / 64;
+  const FusedRoute route = fused_route(x_dtype, norm, mt, a.M, a.N, a.K);
+  if (route == FUSED_ROWS) return aq::launch_gemv_rows(a, fused_kind(norm, x_dtype == AQ_BF16), st);
+  if (route == FUSED_NONE) return -1;
   // A short matrix with long rows (an MLP's down projection): with whole rows per wavefront its N / 32 workgroups
   // would leave most compute units without loads in flight.  4 K parts -- 8 weight rows per workgroup, every wavefront
   // rounding one token row first: 7.0 -> 4.8 us for one row of 5632 against 2048 weight rows (2 parts: 8.0, 8 parts:
@@ -963,6 +975,11 @@ static int gemv_dispatch_fused(const aq::GemvArgs& a, int x_dtype, int mt, hipSt
     case 2: return small ? aq::launch_gemv<2, true, 4>(a, st) : aq::launch_gemv<2, true, 16>(a, st);
     default: return small ? aq::launch_gemv<4, true, 4>(a, st) : aq::launch_gemv<4, true, 16>(a, st);
   }
+}
+
+extern "C" int aq_gemv_w8a8_decode_one_launch(int x_dtype, int norm, int64_t M, int64_t N, int64_t K) {
+  if ((x_dtype != AQ_F32 && x_dtype != AQ_BF16) || M < 1 || M > 16 || N < 1 || K < 1 || K % 16 || K > (1 << 22)) return 0;
+  return fused_route(x_dtype, norm != 0, gemv_bucket(M, K), M, N, K) != FUSED_NONE ? 1 : 0;
 }
 
 extern "C" int aq_gemv_w8a8_codes_residual(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
@@ -1040,6 +1057,10 @@ extern "C" size_t aq_gemv_fp8_workspace_bytes(int64_t M, int64_t K) {
   return aq::align256((size_t)(M * K)) + 256 + AQ_FP8_AMAX_WS_BYTES;  // codes, the scale, the quantiser's partial maxima
 }
 
+extern "C" int aq_gemv_fp8_decode_one_launch(int x_dtype, int64_t M, int64_t K) {
+  return x_dtype == AQ_BF16 && M >= 1 && M <= 16 && aq::gemv_rows_ok(aq::ROWS_FP8, M, K) ? 1 : 0;
+}
+
 static int gemv_fp8_check(const uint8_t* wq, const float* sw, const void* bias, int bias_dtype, const void* residual,
                           const void* y, int y_dtype, int64_t M, int64_t N, int64_t K) {
   if (y_dtype != AQ_F32 && y_dtype != AQ_BF16) return AQ_E_DTYPE;
@@ -1095,7 +1116,7 @@ extern "C" int aq_gemv_fp8_decode_residual(const void* x, int x_dtype, const uin
   if (!x || !ws) return AQ_E_NULL;
   if (aq::check_ptr16(x) || aq::check_ptr16(ws)) return AQ_E_ALIGN;
   if (ws_bytes < aq_gemv_fp8_workspace_bytes(M, K)) return AQ_E_WORKSPACE;
-  if (x_dtype == AQ_BF16 && aq::gemv_rows_ok(aq::ROWS_FP8, M, K)) {  // one launch: the kernel casts the rows itself
+  if (aq_gemv_fp8_decode_one_launch(x_dtype, M, K)) {  // one launch: the kernel casts the rows itself
     aq::GemvArgs a = gemv_fp8_args(wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K);
     a.x = x;
     return aq::launch_gemv_rows(a, aq::ROWS_FP8, static_cast<hipStream_t>(stream));

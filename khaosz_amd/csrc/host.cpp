@@ -36,6 +36,8 @@ namespace {
   X(aq_linear_w8a8_residual)                                                                                     \
   X(aq_linear_fp8_residual)                                                                                      \
   X(aq_gemv_w8a8_workspace_bytes)                                                                                \
+  X(aq_gemv_w8a8_decode_one_launch)                                                                              \
+  X(aq_gemv_fp8_decode_one_launch)                                                                               \
   X(aq_gemv_w8a8_decode_residual)                                                                                \
   X(aq_gemv_w8a8_decode_rmsnorm)                                                                                 \
   X(aq_gemv_w8a8_codes_residual)                                                                                 \
@@ -537,10 +539,14 @@ PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                         : fp8             ? static_cast<int64_t>(lib.aq_gemv_fp8_workspace_bytes(r.M, r.K))
                                           : static_cast<int64_t>(lib.aq_gemv_w8a8_workspace_bytes(r.M, r.K));
   const int64_t room = codes + (r.M > DECODE_ROWS ? (fp8 ? 256 + AQ_FP8_AMAX_WS_BYTES : 4 * r.M) : 0);
-  Tensor ws = c.empty({room}, ScalarType::Byte);
-  char* base = static_cast<char*>(ws.mutable_data_ptr());
-  auto* sx = reinterpret_cast<float*>(base + codes);
   void* yp = y.mutable_data_ptr();
+  // a launch that quantises its rows itself touches no workspace: an allocation is 0.4 us of a 5 us call
+  const bool alone = r.M <= DECODE_ROWS && (fp8 ? lib.aq_gemv_fp8_decode_one_launch(r.code, r.M, r.K)
+                                                : lib.aq_gemv_w8a8_decode_one_launch(r.code, gain != nullptr, r.M, N, r.K));
+  Tensor ws;
+  if (!alone) ws = c.empty({room}, ScalarType::Byte);
+  char* base = static_cast<char*>(alone ? yp : ws.mutable_data_ptr());
+  auto* sx = reinterpret_cast<float*>(base + codes);
   const void* wp = w->const_data_ptr();
   const auto* sp = static_cast<const float*>(s->const_data_ptr());
   const char* what = "";
