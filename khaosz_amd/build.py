@@ -27,7 +27,7 @@ OBJ_DIR = os.path.join(HERE, "lib", "obj")
 LIB = os.path.join(HERE, "lib", "libastrai_q.so")
 LAB_LIB = os.path.join(HERE, "lib", "libastrai_q_lab.so")
 HOST_EXT = os.path.join(HERE, "_host.so")
-SOURCES = ["abi.hip", "quant.hip", "gemm_mfma.hip", "gemm_walk.hip", "gemv.hip", "gemv_rows.hip", "attn_decode.hip", "attn_prefill.hip"]
+SOURCES = ["abi.hip", "quant.hip", "gemm_mfma.hip", "gemm_walk.hip", "gemm_slices.hip", "gemv.hip", "gemv_rows.hip", "attn_decode.hip", "attn_prefill.hip"]
 # (source, object, extra flags) of the lab library's own objects; the other product objects are shared
 LAB_SOURCES = [("gemm_mfma.hip", "gemm_mfma_lab.o", ["-DAQ_LAB"]), ("gemv_rows.hip", "gemv_rows_lab.o", ["-DAQ_LAB"]),
                ("lab.hip", "lab.o", [])]

@@ -26,6 +26,25 @@ struct GemmArgs {
   const void* res;   // [M, N] residual in the output's type, or null; may be C itself
 };
 
+// Workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2.
+// Re-number them so that one XCD owns a contiguous run of tile ids, and walk
+// tile ids in GROUP_M-tall column-major groups, so the tiles resident on an
+// XCD at one time share A rows and B rows (4 x 8 tiles = 2 MB + 2 MB of
+// operands for the 4096 x 2048 x 2048 case).
+__device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int nt = tiles_m * tiles_n;
+  const int per = nt / NUM_XCD, rem = nt % NUM_XCD;
+  const int xcd = pid % NUM_XCD, idx = pid / NUM_XCD;
+  const int tile = xcd * per + (xcd < rem ? xcd : rem) + idx;
+  const int group_sz = GROUP_M * tiles_n;
+  const int group = tile / group_sz;
+  const int first_m = group * GROUP_M;
+  const int gm = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
+  const int in_group = tile - group * group_sz;
+  tm = first_m + in_group % gm;
+  tn = in_group / gm;
+}
+
 template <bool FP8>
 struct Acc {
   using type = v16i;
@@ -74,6 +93,11 @@ __device__ __forceinline__ typename Acc<FP8>::type mma(const typename Frag<FP8>:
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, AQ_FP8_SCALE, 0, AQ_FP8_SCALE);
   }
 }
+
+// gemm_slices.hip: tiles of 32 tm x 32, K cut among a workgroup's wavefronts
+int gemm_slices_rows(int64_t M, int64_t N);
+template <bool FP8, int OUT>
+int gemm_slices_launch(GemmArgs& a, int tm, hipStream_t st);
 
 // gemm_walk.hip
 bool gemm_walk_ok(const GemmArgs& a);

@@ -96,25 +96,6 @@ using ShapeTall = Shape<2, 2, 4, 2, 1, 128, 3>;
 using ShapeHuge8 = Shape<4, 2, 2, 4, 1, 64, 4>;
 using ShapePair = Shape<2, 2, 2, 2, 2, 128, 3>;
 #endif
-// Workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2.
-// Re-number them so that one XCD owns a contiguous run of tile ids, and walk
-// tile ids in GROUP_M-tall column-major groups, so the tiles resident on an
-// XCD at one time share A rows and B rows (4 x 8 tiles = 2 MB + 2 MB of
-// operands for the 4096 x 2048 x 2048 case).
-__device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int nt = tiles_m * tiles_n;
-  const int per = nt / NUM_XCD, rem = nt % NUM_XCD;
-  const int xcd = pid % NUM_XCD, idx = pid / NUM_XCD;
-  const int tile = xcd * per + (xcd < rem ? xcd : rem) + idx;
-  const int group_sz = GROUP_M * tiles_n;
-  const int group = tile / group_sz;
-  const int first_m = group * GROUP_M;
-  const int gm = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
-  const int in_group = tile - group * group_sz;
-  tm = first_m + in_group % gm;
-  tn = in_group / gm;
-}
-
 // Issue order of one pipeline slot, as scheduling groups: GROUPS times
 // [1 MFMA, NDS LDS reads, this group's share of the NLD global loads].
 // (0x008 = MFMA, 0x100 = LDS read, 0x020 = vector-memory read.)
@@ -765,7 +746,7 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
 // 6 % of it.  The small tiles are for launches of a few rounds only.
 enum TileKind {
   TILE_AUTO = 0, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129,
-  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513
+  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_SLICES32 = 34, TILE_SLICES64 = 35
 };
 #ifdef AQ_LAB
 static int g_forced_tile = 0;  // lab build only: TILE_AUTO = by shape, otherwise forced (tuning and tests)
@@ -841,6 +822,10 @@ static int launch(GemmArgs& a, hipStream_t st) {
   if constexpr (OUT == OUT_BF16) {  // more tiles than compute units: the kernel whose K loop goes on from tile to tile
     if (!forced && tile == TILE_LARGE && gemm_walk_ok(a)) return gemm_walk_launch<FP8>(a, st);
   }
+  if constexpr (OUT != OUT_I32) {
+    const int tm = forced ? (tile == TILE_SLICES32 ? 1 : tile == TILE_SLICES64 ? 2 : 0) : gemm_slices_rows(a.M, a.N);
+    if (tm) return gemm_slices_launch<FP8, OUT>(a, tm, st);
+  }
   switch (tile) {
     case TILE_SMALL: return launch_shape<FP8, OUT, ShapeSmall>(a, st);
     case TILE_N64: return launch_shape<FP8, OUT, ShapeN64>(a, st);
@@ -890,7 +875,7 @@ extern "C" int aq_lab_read_clock(long long* host2) {
   return (int)hipMemcpyFromSymbol(host2, HIP_SYMBOL(aq::aq_lab_clock), 64);
 }
 extern "C" int aq_lab_set_gemm_tile(int rows) {
-  if (rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
+  if (rows != 34 && rows != 35 && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
   aq::g_forced_tile = rows;
   return AQ_OK;
 }
@@ -934,14 +919,14 @@ extern "C" int aq_linear_w8a8_residual(const int8_t* xq, const float* sx, const 
       aq::check_ptr(residual, 4))
     return AQ_E_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // 17..32 rows (and decode batches of rows too long for the GEMV kernels): the weight-streaming kernel takes
-  // them (not when a test has forced a tile shape)
+  // 17..32 rows of more than 8192 outputs (and decode batches of rows too long for the GEMV kernels): the weight-streaming
+  // kernel takes them (not when a test has forced a tile shape)
 #ifdef AQ_LAB
   const bool tile_forced = aq::g_forced_tile != 0;
 #else
   const bool tile_forced = false;
 #endif
-  if (!tile_forced && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
+  if (!tile_forced && !aq::gemm_slices_rows(M, N) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
     return aq::gemv_tokens_launch(xq, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, st, false);
   aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);
   a.sx = sx;
@@ -969,13 +954,13 @@ extern "C" int aq_linear_fp8_residual(const uint8_t* xq, const float* sx, const 
       aq::check_ptr(residual, 4))
     return AQ_E_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // 17..32 rows: the weight-streaming kernel, as for int8 (fp32 sums in its own fixed order)
+  // 17..32 rows of many outputs: the weight-streaming kernel, as for int8 (fp32 sums in its own fixed order)
 #ifdef AQ_LAB
   const bool tile_forced = aq::g_forced_tile != 0;
 #else
   const bool tile_forced = false;
 #endif
-  if (!tile_forced && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
+  if (!tile_forced && !aq::gemm_slices_rows(M, N) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
     return aq::gemv_tokens_launch(reinterpret_cast<const int8_t*>(xq), sx, reinterpret_cast<const int8_t*>(wq), sw, bias,
                                   bias_dtype, residual, y, y_dtype, M, N, K, st, true);
   aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);

@@ -1352,3 +1352,29 @@ def test_swiglu_quant_of_many_bf16_rows(oracle, M, F):
     qo, so = oracle.c_swiglu_quant_i8(bf16_bits(d), bf16_bits=True)
     assert np.array_equal(to_np(s), so)
     assert np.array_equal(to_np(q), qo)
+
+
+# K cut among the wavefronts: fewer K steps than wavefronts, a ragged last step, ragged rows and columns, odd N, one tile
+@pytest.mark.parametrize("kind", [34, 35])
+@pytest.mark.parametrize("M,N,K", [(17, 33, 16), (33, 96, 400), (70, 75, 1040), (64, 64, 512), (65, 1001, 2064), (200, 512, 1936)])
+def test_gemm_with_k_cut_among_wavefronts(oracle, M, N, K, kind):
+    _say("gemm slices", M, N, K, kind)
+    rng = np.random.default_rng(M + N + K)
+    xq, wq = (rng.integers(-128, 128, (n, K), dtype=np.int8) for n in (M, N))
+    sx, sw = (rng.random(n, dtype=np.float32) * 0.01 + 1e-4 for n in (M, N))
+    b = rng.standard_normal(N).astype(np.float32)
+    acc = oracle.c_gemm_i8_i32(xq, wq)
+    d = [torch.from_numpy(t).to(DEV) for t in (xq, sx, wq, sw, b)]
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(kind) == 0
+        for out in (torch.bfloat16, torch.float32):
+            bias = d[4].to(torch.bfloat16) if out is torch.bfloat16 else d[4]
+            y = ops.linear_w8a8(d[0], d[1], d[2], d[3], bias, out_dtype=out)
+            want = oracle.c_dequant_epilogue(acc, sx, sw, bias.float().cpu().numpy(), bf16_out=out is torch.bfloat16)
+            assert np.array_equal(bf16_bits(y) if out is torch.bfloat16 else to_np(y), want)
+            res = torch.randn(M, N, device=DEV, dtype=out)
+            assert torch.equal(ops.linear_w8a8(d[0], d[1], d[2], d[3], bias, out_dtype=out, residual=res), y + res)
+        x8, w8 = (torch.from_numpy(rng.standard_normal((n, K)).astype(np.float32)).to(DEV).to(torch.float8_e4m3fn) for n in (M, N))
+        y = ops.linear_fp8(x8.view(torch.uint8), d[1][:1], w8.view(torch.uint8), d[3][:1], d[4], out_dtype=torch.float32)
+        want = (x8.float().cpu().double() @ w8.float().cpu().double().T) * float(sx[0]) * float(sw[0]) + torch.from_numpy(b).double()
+        assert torch.allclose(y.cpu().double(), want, rtol=1e-3, atol=1e-4 * want.abs().max().item())
