@@ -626,7 +626,7 @@ static int rope_kv_write(const void* qkv, const float* freqs, int64_t freqs_stri
   a.q_gain = static_cast<const uint16_t*>(q_gain);
   a.k_gain = static_cast<const uint16_t*>(k_gain);
   a.eps = eps;
-  hipLaunchKernelGGL(aq::rope_kv_write_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0,
+  aq::queue_kernel(aq::rope_kv_write_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), a);
   return (int)hipGetLastError();
 }
@@ -658,11 +658,11 @@ extern "C" int64_t aq_paged_attn_decode_workspace_bytes(int64_t B, int64_t Hq, i
 template <int G, int D>
 static void attn_launch(bool rope, dim3 grid, dim3 block, hipStream_t st, const aq::AttnArgs& a) {
   if (rope && a.q_gain)
-    hipLaunchKernelGGL((aq::paged_attn_decode_kernel<G, D, true, true>), grid, block, 0, st, a);
+    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, true, true>), grid, block, 0, st, a);
   else if (rope)
-    hipLaunchKernelGGL((aq::paged_attn_decode_kernel<G, D, true>), grid, block, 0, st, a);
+    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, true>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((aq::paged_attn_decode_kernel<G, D, false>), grid, block, 0, st, a);
+    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, false>), grid, block, 0, st, a);
 }
 
 // q == nullptr: the fused form, queries and the new token come from qkv / freqs.
@@ -742,7 +742,7 @@ static int attn_decode(const void* q, const void* qkv, const float* freqs, int64
 #undef AQ_ATTN_CASE
   int rc = (int)hipGetLastError();
   if (rc != 0 || ns == 1 || partials) return rc;
-  hipLaunchKernelGGL(aq::attn_merge_kernel, dim3((unsigned)(B * Hq)), dim3((unsigned)(D / 2)), 0, st, a.ws, a.out, a.NS,
+  aq::queue_kernel(aq::attn_merge_kernel, dim3((unsigned)(B * Hq)), dim3((unsigned)(D / 2)), 0, st, a.ws, a.out, a.NS,
                      (int)D);
   return (int)hipGetLastError();
 }

@@ -421,7 +421,7 @@ static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
     a.table_lds = a.page % KB != 0 && entries <= PA_TABLE_MAX ? (int)entries : 0;
     lds += (size_t)a.table_lds * sizeof(int);
   }
-  hipLaunchKernelGGL((prefill_attn_kernel<D, QW, KW, PAGED>), dim3((unsigned)(wgs + a.ahead_wgs)), dim3(QW * KW * 64), lds, st, a);
+  aq::queue_kernel((prefill_attn_kernel<D, QW, KW, PAGED>), dim3((unsigned)(wgs + a.ahead_wgs)), dim3(QW * KW * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 

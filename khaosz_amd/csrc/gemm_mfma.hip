@@ -795,7 +795,7 @@ static int launch_shape(GemmArgs& a, hipStream_t st) {
   // 3-5 % faster than queueing a workgroup per tile once there are more tiles than compute units
   const int64_t ntiles = (int64_t)a.tiles_m * a.tiles_n, cus = device_cus();
   const unsigned grid = (unsigned)(ntiles < cus ? ntiles : cus);
-  hipLaunchKernelGGL((gemm_kernel<FP8, OUT, S>), dim3(grid), dim3(S::NTHREADS), 0, st, a);
+  aq::queue_kernel((gemm_kernel<FP8, OUT, S>), dim3(grid), dim3(S::NTHREADS), 0, st, a);
   return (int)hipGetLastError();
 }
 

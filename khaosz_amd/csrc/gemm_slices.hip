@@ -214,7 +214,7 @@ template <bool FP8, int OUT, int W, int TM, int TN, int BK, int NST>
 static int launch_slices(GemmArgs& a, hipStream_t st) {
   a.tiles_m = (a.M + 32 * TM - 1) / (32 * TM);
   a.tiles_n = (a.N + 32 * TN - 1) / (32 * TN);
-  hipLaunchKernelGGL((gemm_slices_kernel<FP8, OUT, W, TM, TN, BK, NST>), dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(W * 64), 0,
+  aq::queue_kernel((gemm_slices_kernel<FP8, OUT, W, TM, TN, BK, NST>), dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(W * 64), 0,
                      st, a);
   return (int)hipGetLastError();
 }

@@ -295,7 +295,7 @@ int gemm_walk_launch(const GemmArgs& a, hipStream_t st) {
   const int cus = device_cus(), nt = w.g.tiles_m * w.g.tiles_n, rest = nt % cus;
   w.halves = rest <= cus / 2 && nt >= 3 * cus ? 2 * rest : 0;
   w.full = nt - w.halves / 2;
-  hipLaunchKernelGGL((gemm_walk_kernel<FP8>), dim3((unsigned)cus), dim3(512), 0, st, w);
+  aq::queue_kernel((gemm_walk_kernel<FP8>), dim3((unsigned)cus), dim3(512), 0, st, w);
   return (int)hipGetLastError();
 }
 template int gemm_walk_launch<false>(const GemmArgs&, hipStream_t);

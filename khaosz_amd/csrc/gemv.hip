@@ -300,7 +300,7 @@ static int launch_gemv_fw(GemvArgs a, hipStream_t st) {
     const int e = opted.ensure(reinterpret_cast<const void*>(&gemv_w8a8_kernel<MT, FUSED, VPL, NORM, MERGE, FW, FK>));
     if (e) return e;
   }
-  hipLaunchKernelGGL((gemv_w8a8_kernel<MT, FUSED, VPL, NORM, MERGE, FW, FK>), dim3(grid), dim3(sh.waves * 64), lds, st, a);
+  aq::queue_kernel((gemv_w8a8_kernel<MT, FUSED, VPL, NORM, MERGE, FW, FK>), dim3(grid), dim3(sh.waves * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 
@@ -597,7 +597,7 @@ static int launch_gemv_mfma(GemvArgs a, hipStream_t st, bool fp8 = false) {
     const int e = opted[fp8 * 8 + fixed * 4 + res * 2 + long_rows].ensure(reinterpret_cast<const void*>(fn));
     if (e) return e;
   }
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(a.ksplit * a.groups * 64), lds, st, a);
+  aq::queue_kernel(fn, dim3(grid), dim3(a.ksplit * a.groups * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 
@@ -832,7 +832,7 @@ static int launch_gemv_tokens_shape(const GemvArgs& a, hipStream_t st, bool fp8)
   static LdsOptIn opted[4];
   const int e = opted[(fp8 ? 2 : 0) + (a.res ? 1 : 0)].ensure(reinterpret_cast<const void*>(fn));
   if (e) return e;
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(KS * GRP * 64), lds, st, a);
+  aq::queue_kernel(fn, dim3(grid), dim3(KS * GRP * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 

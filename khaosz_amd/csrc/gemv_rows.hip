@@ -366,7 +366,7 @@ static int launch_rows(rows_kernel_t fn, LdsOptIn& opted, const GemvArgs& a, int
     if (e) return e;
   }
   const unsigned grid = (unsigned)((outputs + outputs_per_wg - 1) / outputs_per_wg);
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(GX_WAVES * 64), lds, st, a);
+  aq::queue_kernel(fn, dim3(grid), dim3(GX_WAVES * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 

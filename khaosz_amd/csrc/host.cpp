@@ -19,6 +19,7 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "../../include/astrai_q.h"
@@ -391,7 +392,7 @@ PyObject *k_modules, *k_buffers, *k_parameters, *k_qweight, *k_w_scale, *k_bias,
     *k_fwd_pre_hooks, *k_compiled, *k_attention, *k_mlp, *k_input_norm, *k_post_norm, *k_qkv, *k_upgate, *k_o_proj, *k_down, *k_q_norm,
     *k_k_norm, *k_decode_attention, *k_use_qk_norm, *k_use_gate, *k_n_heads, *k_n_kv_heads, *k_head_dim, *k_layer_id, *k_swiglu_quant,
     *k_norm_quant, *k_residual_adds, *k_k_layers, *k_v_layers, *k_page_table, *k_total_len, *k_seq_lens, *k_invalid, *k_page_size,
-    *k_shared, *k_residual, *k_norm;
+    *k_shared, *k_residual, *k_norm, *k_call;
 
 PyObject* dict_of(PyObject* o) {  // borrowed; null if it has none
   PyObject** d = _PyObject_GetDictPtr(o);
@@ -415,6 +416,8 @@ struct Types {
   PyObject* global_hooks = nullptr;  // tuple of the dicts of hooks that run for every module
   PyObject* ops_dict = nullptr;      // the operators' module and, by name, the operators as they were defined
   PyObject *linear_ops = nullptr, *block_ops = nullptr;
+  uint64_t linear_ops_version = 0, block_ops_version = 0;  // of ops_dict when it last held them all
+  PyObject* module = nullptr;  // torch.nn.Module
   PyObject *rms_norm = nullptr, *gqa = nullptr, *mlp = nullptr, *paged_kv = nullptr;
 } types;
 
@@ -432,13 +435,22 @@ bool ordinary(PyObject* m, PyObject* type, bool called) {
 
 // Nothing watches module calls globally, and the operators are the package's own: a program that replaces one (to
 // count or trace calls) has every call go through its replacement, on the step-by-step path.
+// The operators' dictionary is looked through again only once it has changed (its version tag is never used twice).
 bool unobserved(PyObject* operators) {
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(types.global_hooks); ++i)
     if (PyDict_GET_SIZE(PyTuple_GET_ITEM(types.global_hooks, i))) return false;
+#if PY_VERSION_HEX < 0x030c0000
+  uint64_t& seen = operators == types.block_ops ? types.block_ops_version : types.linear_ops_version;
+  const uint64_t version = reinterpret_cast<PyDictObject*>(types.ops_dict)->ma_version_tag;
+  if (seen == version) return true;
+#endif
   PyObject *name, *own;
   Py_ssize_t at = 0;
   while (PyDict_Next(operators, &at, &name, &own))
     if (PyDict_GetItem(types.ops_dict, name) != own) return false;
+#if PY_VERSION_HEX < 0x030c0000
+  seen = version;
+#endif
   return true;
 }
 
@@ -489,25 +501,27 @@ bool gain_of(PyObject* m, int64_t K, int dev, Gain* g) {
 constexpr int64_t DECODE_ROWS = 16;                  // QuantLinear.DECODE_MAX_ROWS, Fp8Linear.DECODE_MAX_ROWS
 constexpr int64_t FP8_ONEPASS_MIN_BYTES = 16 << 20;  // ops.FP8_ONEPASS_MIN_BYTES
 
-// linear_call(layer, args, kwargs) -> what calling the QuantLinear or Fp8Linear gives, or None where nn.Module's own call has
-// to serve: hooks, a shared input, FP8 inputs that are quantised in one launch with a state the module keeps.
-PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(3);
-  PyObject *layer = args[0], *given = args[1], *named = args[2];
+// What calling the QuantLinear or Fp8Linear gives, or None where nn.Module's own call has to serve: hooks, a shared input, FP8
+// inputs that are quantised in one launch with a state the module keeps.
+PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs, PyObject* names) {
+  AQ_TRY
   const bool fp8 = reinterpret_cast<PyObject*>(Py_TYPE(layer)) == types.fp8_linear;
-  if (!types.linear_ops || PyTuple_GET_SIZE(given) != 1 || !ordinary(layer, fp8 ? types.fp8_linear : types.quant_linear, true) ||
+  if (!lib.aq_error_string || !types.linear_ops || nargs != 1 || !ordinary(layer, fp8 ? types.fp8_linear : types.quant_linear, true) ||
       !unobserved(types.linear_ops))
     return none();
   PyObject *residual = nullptr, *norm = nullptr;
-  if (const Py_ssize_t n = PyDict_GET_SIZE(named)) {
-    residual = PyDict_GetItem(named, k_residual);
-    norm = fp8 ? nullptr : PyDict_GetItem(named, k_norm);
-    if (n != (residual != nullptr) + (norm != nullptr)) return none();
-    if (norm == Py_None) norm = nullptr;
+  for (Py_ssize_t i = 0; names && i < PyTuple_GET_SIZE(names); ++i) {
+    PyObject* name = PyTuple_GET_ITEM(names, i);  // interned, as keyword names are; another text of the same value takes the general path
+    if (name == k_residual)
+      residual = args[1 + i];
+    else if (name == k_norm && !fp8)
+      norm = args[1 + i] == Py_None ? nullptr : args[1 + i];
+    else
+      return none();
   }
   PyObject* d = dict_of(layer);
   if (!fp8 && get(d, k_shared) != Py_None) return none();
-  const Tensor *x = unpack(PyTuple_GET_ITEM(given, 0)), *w, *s;
+  const Tensor *x = unpack(args[0]), *w, *s;
   Call c;
   Rows r;
   Bias b;
@@ -583,12 +597,43 @@ PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   AQ_CATCH
 }
 
-// set_linear_types(QuantLinear, Fp8Linear, hook dicts, ops.__dict__, {name: operator as defined})
+// __call__ of the quantized layers
+PyObject* linear_call(PyObject* layer, PyObject* const* args, Py_ssize_t nargs, PyObject* names) {
+  PyObject* y = linear_native(layer, args, nargs, names);
+  if (y != Py_None) return y;
+  Py_DECREF(y);
+  PyObject* call = PyObject_GetAttr(types.module, k_call);  // looked up each time: tracers replace it
+  if (!call) return nullptr;
+  PyObject* few[8];
+  const Py_ssize_t n = nargs + (names ? PyTuple_GET_SIZE(names) : 0);
+  PyObject** all = n < 8 ? few : static_cast<PyObject**>(PyMem_Malloc((n + 1) * sizeof(PyObject*)));
+  if (all) {
+    all[0] = layer;
+    std::copy(args, args + n, all + 1);
+    y = PyObject_Vectorcall(call, all, nargs + 1, names);
+  } else {
+    y = PyErr_NoMemory();
+  }
+  if (all != few) PyMem_Free(all);
+  Py_DECREF(call);
+  return y;
+}
+PyMethodDef linear_call_def = {"__call__", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(linear_call)),
+                               METH_FASTCALL | METH_KEYWORDS, nullptr};
+
+// linear_call_method(cls) -> linear_call as a method of that class
+PyObject* linear_call_method(PyObject*, PyObject* cls) {
+  if (!PyType_Check(cls)) return PyErr_Format(PyExc_TypeError, "linear_call_method");
+  return PyDescr_NewMethod(reinterpret_cast<PyTypeObject*>(cls), &linear_call_def);
+}
+
+// set_linear_types(QuantLinear, Fp8Linear, hook dicts, ops.__dict__, {name: operator as defined}, torch.nn.Module)
 PyObject* set_linear_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_ARGS(5);
+  AQ_ARGS(6);
   if (!PyTuple_Check(args[2]) || !PyDict_Check(args[3]) || !PyDict_Check(args[4])) return PyErr_Format(PyExc_TypeError, "set_linear_types");
-  for (Py_ssize_t i = 0; i < 5; ++i) Py_INCREF(args[i]);  // for the life of the process
+  for (Py_ssize_t i = 0; i < 6; ++i) Py_INCREF(args[i]);  // for the life of the process
   types.quant_linear = args[0], types.fp8_linear = args[1], types.global_hooks = args[2], types.ops_dict = args[3], types.linear_ops = args[4];
+  types.module = args[5];
   Py_RETURN_NONE;
 }
 
@@ -865,7 +910,7 @@ PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
     AQ_METHOD(set_linear_types),
     AQ_METHOD(set_block_types),
-    AQ_METHOD(linear_call),
+    {"linear_call_method", linear_call_method, METH_O, nullptr},
     AQ_METHOD(quant_rowwise_i8),
     AQ_METHOD(rmsnorm_quant_rowwise_i8),
     AQ_METHOD(swiglu_quant_rowwise_i8),
@@ -899,7 +944,8 @@ PyMODINIT_FUNC PyInit__host() {
               {&k_norm_quant, "_norm_quant"}, {&k_residual_adds, "_residual_adds"}, {&k_k_layers, "k_layers"},
               {&k_v_layers, "v_layers"},      {&k_page_table, "page_table"},    {&k_total_len, "total_len"},
               {&k_seq_lens, "seq_lens"},      {&k_invalid, "_invalid"},         {&k_page_size, "page_size"},
-              {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"}};
+              {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"},
+              {&k_call, "__call__"}};
   for (const auto& k : keys)
     if (!(*k.key = PyUnicode_InternFromString(k.name))) return nullptr;
   return PyModule_Create(&module);

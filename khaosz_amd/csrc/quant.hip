@@ -822,18 +822,18 @@ extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_
     const unsigned g = (unsigned)M;
     if (x_dtype == AQ_BF16) {
       if (nvec <= 256)
-        hipLaunchKernelGGL((aq::quant_row_wg_kernel<true, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
       else if (nvec <= 512)
-        hipLaunchKernelGGL((aq::quant_row_wg_kernel<true, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
       else
-        hipLaunchKernelGGL((aq::quant_row_wg_kernel<true, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
     } else {
       if (nvec <= 256)
-        hipLaunchKernelGGL((aq::quant_row_wg_kernel<false, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
       else if (nvec <= 512)
-        hipLaunchKernelGGL((aq::quant_row_wg_kernel<false, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
       else
-        hipLaunchKernelGGL((aq::quant_row_wg_kernel<false, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
     }
     return (int)hipGetLastError();
   }
@@ -844,23 +844,23 @@ extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_
   const unsigned grid = (unsigned)wgs;
   if (x_dtype == AQ_BF16) {
     if (full_row)
-      hipLaunchKernelGGL((aq::quant_rowwise_i8_kernel<true, 4, true, true>), dim3(grid), dim3(256), 0, st, x, M,
+      aq::queue_kernel((aq::quant_rowwise_i8_kernel<true, 4, true, true>), dim3(grid), dim3(256), 0, st, x, M,
                          (int)K, ldx, q, scale);
     else if (small_row)
-      hipLaunchKernelGGL((aq::quant_rowwise_i8_kernel<true, 4, true, false>), dim3(grid), dim3(256), 0, st, x, M,
+      aq::queue_kernel((aq::quant_rowwise_i8_kernel<true, 4, true, false>), dim3(grid), dim3(256), 0, st, x, M,
                          (int)K, ldx, q, scale);
     else
-      hipLaunchKernelGGL((aq::quant_rowwise_i8_kernel<true, 16, false, false>), dim3(grid), dim3(256), 0, st, x,
+      aq::queue_kernel((aq::quant_rowwise_i8_kernel<true, 16, false, false>), dim3(grid), dim3(256), 0, st, x,
                          M, (int)K, ldx, q, scale);
   } else {
     if (full_row)
-      hipLaunchKernelGGL((aq::quant_rowwise_i8_kernel<false, 4, true, true>), dim3(grid), dim3(256), 0, st, x, M,
+      aq::queue_kernel((aq::quant_rowwise_i8_kernel<false, 4, true, true>), dim3(grid), dim3(256), 0, st, x, M,
                          (int)K, ldx, q, scale);
     else if (small_row)
-      hipLaunchKernelGGL((aq::quant_rowwise_i8_kernel<false, 4, true, false>), dim3(grid), dim3(256), 0, st, x, M,
+      aq::queue_kernel((aq::quant_rowwise_i8_kernel<false, 4, true, false>), dim3(grid), dim3(256), 0, st, x, M,
                          (int)K, ldx, q, scale);
     else
-      hipLaunchKernelGGL((aq::quant_rowwise_i8_kernel<false, 16, false, false>), dim3(grid), dim3(256), 0, st, x,
+      aq::queue_kernel((aq::quant_rowwise_i8_kernel<false, 16, false, false>), dim3(grid), dim3(256), 0, st, x,
                          M, (int)K, ldx, q, scale);
   }
   return (int)hipGetLastError();
@@ -874,11 +874,11 @@ static int launch_rmsnorm_quant(const void* x, const void* gamma, float eps, int
   if (wgs > 1024) wgs = 1024;  // four workgroups per CU; wavefronts walk the remaining rows
   const dim3 g((unsigned)wgs), b(256);
   if (vpl <= 4)
-    hipLaunchKernelGGL((aq::rmsnorm_quant_kernel<BF16, 4, true>), g, b, 0, st, x, gamma, eps, M, (int)K, ldx, q, scale);
+    aq::queue_kernel((aq::rmsnorm_quant_kernel<BF16, 4, true>), g, b, 0, st, x, gamma, eps, M, (int)K, ldx, q, scale);
   else if (vpl <= 12)
-    hipLaunchKernelGGL((aq::rmsnorm_quant_kernel<BF16, 12, false>), g, b, 0, st, x, gamma, eps, M, (int)K, ldx, q, scale);
+    aq::queue_kernel((aq::rmsnorm_quant_kernel<BF16, 12, false>), g, b, 0, st, x, gamma, eps, M, (int)K, ldx, q, scale);
   else if (vpl <= 24)  // 24 vectors per lane is what fits the register file without spilling for bf16 rows
-    hipLaunchKernelGGL((aq::rmsnorm_quant_kernel<BF16, 24, false>), g, b, 0, st, x, gamma, eps, M, (int)K, ldx, q, scale);
+    aq::queue_kernel((aq::rmsnorm_quant_kernel<BF16, 24, false>), g, b, 0, st, x, gamma, eps, M, (int)K, ldx, q, scale);
   else
     return AQ_E_RANGE;
   return (int)hipGetLastError();
@@ -918,7 +918,7 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
       switch (vpl) {
 #define AQ_SWIGLU_CASE(nc)                                                                                                      \
   case nc:                                                                                                                      \
-    hipLaunchKernelGGL((aq::swiglu_quant_lut_kernel<nc>), g, dim3(nc <= 12 ? 1024 : 768), 0, st, ug, M, (int)F, ld, q, scale); \
+    aq::queue_kernel((aq::swiglu_quant_lut_kernel<nc>), g, dim3(nc <= 12 ? 1024 : 768), 0, st, ug, M, (int)F, ld, q, scale); \
     break;
         AQ_SWIGLU_CASE(4) AQ_SWIGLU_CASE(5) AQ_SWIGLU_CASE(6) AQ_SWIGLU_CASE(7) AQ_SWIGLU_CASE(8) AQ_SWIGLU_CASE(9)
         AQ_SWIGLU_CASE(10) AQ_SWIGLU_CASE(11) AQ_SWIGLU_CASE(12) AQ_SWIGLU_CASE(13) AQ_SWIGLU_CASE(14) AQ_SWIGLU_CASE(15)
@@ -930,7 +930,7 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
   }
   // few rows, or rows too long for one wavefront's registers: a workgroup of vpl wavefronts per row
   if (vpl > 1 && (M <= AQ_SWIGLU_WG_MAX_M || vpl > 12)) {
-    hipLaunchKernelGGL((aq::swiglu_quant_wg_kernel<BF16>), dim3((unsigned)M), dim3((unsigned)vpl * 64), 0, st, ug, (int)F,
+    aq::queue_kernel((aq::swiglu_quant_wg_kernel<BF16>), dim3((unsigned)M), dim3((unsigned)vpl * 64), 0, st, ug, (int)F,
                        ld, q, scale);
     return (int)hipGetLastError();
   }
@@ -944,7 +944,7 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
   // is 11 pairs per lane, and a 12th would be 8 % more work)
   switch (vpl) {
 #define AQ_SWIGLU_CASE(nc)                                                                                   \
-  case nc: hipLaunchKernelGGL((aq::swiglu_quant_kernel<BF16, nc>), g, b, 0, st, ug, M, (int)F, ld, q, scale); break;
+  case nc: aq::queue_kernel((aq::swiglu_quant_kernel<BF16, nc>), g, b, 0, st, ug, M, (int)F, ld, q, scale); break;
     AQ_SWIGLU_CASE(1) AQ_SWIGLU_CASE(2) AQ_SWIGLU_CASE(3)
     default: break;
   }
@@ -989,10 +989,10 @@ int quant_tensor_fp8_onepass(const void* x, int x_dtype, int64_t numel, uint8_t*
   int g = aq::device_cus();
   if (g > AQ_FP8_ONEPASS_WS_BYTES / 8) g = AQ_FP8_ONEPASS_WS_BYTES / 8;
   if (x_dtype == AQ_BF16)
-    hipLaunchKernelGGL((aq::quant_fp8_onepass_kernel<true>), dim3((unsigned)g), dim3(aq::ONEPASS_THREADS), 0, st, x, nvec,
+    aq::queue_kernel((aq::quant_fp8_onepass_kernel<true>), dim3((unsigned)g), dim3(aq::ONEPASS_THREADS), 0, st, x, nvec,
                        static_cast<unsigned long long*>(ws), q, scale, spin_limit);
   else
-    hipLaunchKernelGGL((aq::quant_fp8_onepass_kernel<false>), dim3((unsigned)g), dim3(aq::ONEPASS_THREADS), 0, st, x, nvec,
+    aq::queue_kernel((aq::quant_fp8_onepass_kernel<false>), dim3((unsigned)g), dim3(aq::ONEPASS_THREADS), 0, st, x, nvec,
                        static_cast<unsigned long long*>(ws), q, scale, spin_limit);
   return (int)hipGetLastError();
 }
@@ -1024,12 +1024,12 @@ extern "C" int aq_quant_tensor_fp8(const void* x, int x_dtype, int64_t numel, ui
   (void)ablocks;
   ablocks = aq::AMAX_SLOTS;
   if (x_dtype == AQ_BF16) {
-    hipLaunchKernelGGL((aq::amax_kernel<true>), dim3((unsigned)ablocks), dim3(aq::AMAX_THREADS), 0, st, x, nvec, amax_ws);
-    hipLaunchKernelGGL((aq::cast_fp8_kernel<true>), dim3((unsigned)blocks), dim3(256), 0, st, x, nvec,
+    aq::queue_kernel((aq::amax_kernel<true>), dim3((unsigned)ablocks), dim3(aq::AMAX_THREADS), 0, st, x, nvec, amax_ws);
+    aq::queue_kernel((aq::cast_fp8_kernel<true>), dim3((unsigned)blocks), dim3(256), 0, st, x, nvec,
                        amax_ws, q, scale);
   } else {
-    hipLaunchKernelGGL((aq::amax_kernel<false>), dim3((unsigned)ablocks), dim3(aq::AMAX_THREADS), 0, st, x, nvec, amax_ws);
-    hipLaunchKernelGGL((aq::cast_fp8_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, st, x, nvec,
+    aq::queue_kernel((aq::amax_kernel<false>), dim3((unsigned)ablocks), dim3(aq::AMAX_THREADS), 0, st, x, nvec, amax_ws);
+    aq::queue_kernel((aq::cast_fp8_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, st, x, nvec,
                        amax_ws, q, scale);
   }
   return (int)hipGetLastError();

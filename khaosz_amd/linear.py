@@ -126,19 +126,20 @@ class _SharedInput:
         return y
 
 
-_linear_call = None  # the native call of a quantized layer once it is loaded
+_told = False  # whether the native host path knows the layers
 
 
 def linear_native():
     """The native host path, told about the layers' classes, the hooks that run for every module, and the operators as
     defined: while a program has one of those replaced (to count or trace calls), calls go through its replacement."""
-    global _linear_call
+    global _told
     h = ops._native()
-    if _linear_call is None:
+    if not _told:
         m = torch.nn.modules.module
         h.set_linear_types(QuantLinear, Fp8Linear, (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
-                                                    m._global_backward_pre_hooks), ops.__dict__, _OPERATORS)
-        _linear_call = h.linear_call
+                                                    m._global_backward_pre_hooks), ops.__dict__, _OPERATORS, nn.Module)
+        _NativeCall.__call__ = h.linear_call_method(_NativeCall)
+        _told = True
     return h
 
 
@@ -151,11 +152,9 @@ class _NativeCall(Linear):
     """A quantized Linear's call: natively in one step where nothing observes it (no hooks, plain tensors), through
     ``nn.Module.__call__`` and ``forward`` otherwise -- the same launches and bits."""
 
-    def __call__(self, *args, **kwargs):
-        if _linear_call is None:
-            linear_native()
-        y = _linear_call(self, args, kwargs)
-        return super().__call__(*args, **kwargs) if y is None else y
+    def __call__(self, *args, **kwargs):  # the first call of a process; then the native method is in its place
+        linear_native()
+        return _NativeCall.__call__(self, *args, **kwargs)
 
 
 class QuantLinear(_NativeCall):

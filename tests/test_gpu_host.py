@@ -96,3 +96,34 @@ def test_what_the_native_functions_do_not_take_goes_the_general_way(rows):
             q(wide[:, :256].double())
         with pytest.raises(RuntimeError, match="GPU only"):
             q(wide[:, :256].cpu())
+
+
+class _Sub(QuantLinear):
+    pass
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17])
+def test_forms_of_a_layer_call(rows):
+    """The native method answers or hands over to nn.Module's call, whatever way the arguments come."""
+    torch.manual_seed(5)
+    base = torch.nn.Linear(256, 128).to(DEV).to(DT)
+    layer, sub = QuantLinear.from_linear(base), _Sub.from_linear(base)
+    x, r = torch.randn(2, rows, 256, device=DEV).to(DT)[0], torch.randn(rows, 128, device=DEV).to(DT)
+    norm = torch.rand(256, device=DEV).to(DT), 1e-5
+    with torch.inference_mode():
+        for args, kw in (((), {}), ((), {"residual": None}), ((), {"residual": r}), ((r,), {}), ((), {"norm": norm}),
+                         ((), {"residual": r, "norm": norm}), ((), {"norm": None})):
+            want = layer.forward(x, *args, **kw)
+            assert torch.equal(layer(x, *args, **kw), want) and torch.equal(sub(x, *args, **kw), want)
+        assert torch.equal(layer(x=x), layer.forward(x))
+        with pytest.raises(TypeError):
+            layer(x, other=r)
+        with pytest.raises(TypeError):
+            layer()
+        with pytest.raises(ValueError):
+            layer(x[:, :128])
+        seen = []
+        handle = layer.register_forward_hook(lambda m, a, y: seen.append(y))
+        y = layer(x)
+        handle.remove()
+        assert len(seen) == 1 and torch.equal(seen[0], y) and torch.equal(y, layer(x)) and len(seen) == 1
