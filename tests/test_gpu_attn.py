@@ -138,6 +138,12 @@ def test_paged_attn_decode_sequences_at_different_positions(oracle, B, Hq, Hkv, 
     assert torch.equal(a, b) and torch.equal(k1, k2) and torch.equal(v1, v2)
 
 
+@pytest.mark.parametrize("T,lens", [(2500, [2500, 70]), (1100, [1024, 1023]), (257, [256, 1])])
+def test_paged_attn_decode_leaves_out_what_is_masked(oracle, T, lens):
+    """Wavefronts and whole slices past a sequence's length read nothing; the new token's is stored all the same."""
+    test_paged_attn_decode_sequences_at_different_positions(oracle, 2, 6, 1, 64, T, 64, lens)
+
+
 def test_paged_attn_workspace_reuse_and_checks(oracle):
     """A caller-owned workspace gives the same bits as a per-call one; a short one is refused."""
     _say("paged_attn_workspace")
