@@ -819,7 +819,7 @@ static int launch(GemmArgs& a, hipStream_t st) {
     if (!forced && huge_fp8_ok(a)) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
   }
   const int tile = choose_tile(a.M, a.N);
-  if constexpr (OUT == OUT_BF16) {  // more tiles than compute units: the kernel whose K loop goes on from tile to tile
+  if constexpr (OUT == OUT_BF16) {  // many tiles, or a residual: the kernel whose K loop goes on from tile to tile
     if (!forced && tile == TILE_LARGE && gemm_walk_ok(a)) return gemm_walk_launch<FP8>(a, st);
   }
   if constexpr (OUT != OUT_I32) {

@@ -1325,6 +1325,31 @@ def test_gemm_walking_tiles(M, N, K, bias):
         assert torch.equal(y8, ops.linear_fp8(x8, sx[:1], w8, sw[:1], b, out_dtype=torch.bfloat16))
 
 
+# one round (whole, ragged), several with whole and with halved tiles at their end; the residual apart from and in the output
+@pytest.mark.parametrize("residual", [False, True])
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 512), (3001, 2046, 640), (2049, 4100, 768), (4225, 6402, 512)])
+def test_gemm_walk_of_one_round_and_residuals(M, N, K, residual):
+    """256 x 128 tiles with and without a residual: the bits of the kernel of one tile after another."""
+    _say("gemm walk residual", M, N, K, residual)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    xq, wq = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
+    sx, sw = (torch.rand(n, generator=g, device=DEV) * 0.01 + 1e-4 for n in (M, N))
+    x8, w8 = (torch.randn(n, K, generator=g, device=DEV).to(torch.float8_e4m3fn).view(torch.uint8) for n in (M, N))
+    r = torch.randn(M, N, generator=g, device=DEV).to(torch.bfloat16) if residual else None
+    run = lambda: (ops.linear_w8a8(xq, sx, wq, sw, None, out_dtype=torch.bfloat16, residual=r),
+                   ops.linear_fp8(x8, sx[:1], w8, sw[:1], None, out_dtype=torch.bfloat16, residual=r))
+    got = run()
+    if residual:  # the sum takes the residual's place
+        y = r.clone()
+        assert _abi.load().aq_linear_w8a8_residual(xq.data_ptr(), sx.data_ptr(), wq.data_ptr(), sw.data_ptr(), None, 0, y.data_ptr(),
+                                                   y.data_ptr(), _abi.AQ_BF16, M, N, K, torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(y, got[0])
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(256) == 0
+        for a, b in zip(got, run()):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("M,F", [(1025, 2048), (1300, 6928), (1041, 2064), (2050, 4096)])
 def test_swiglu_quant_of_many_bf16_rows(oracle, M, F):
     """Many rows take the kernel that looks silu up: every bf16 gate pattern, zeros, gates around both ends of its table,
