@@ -179,12 +179,19 @@ PyObject* pair(const Tensor& a, const Tensor& b) {
 }
 
 // The library calls queue work and may wait while the device's queue is full: other Python threads run meanwhile.
+// The lock is taken back on every way out: an exception is turned into a Python error, which needs it.  (Not in a
+// destructor: Python ends a thread that waits for the lock at exit by unwinding it from there.)
 template <class F>
 int queued(F&& launch) {
+  PyThreadState* const thread = PyEval_SaveThread();
   int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = launch();
-  Py_END_ALLOW_THREADS;
+  try {
+    rc = launch();
+  } catch (...) {
+    PyEval_RestoreThread(thread);
+    throw;
+  }
+  PyEval_RestoreThread(thread);
   return rc;
 }
 
@@ -675,8 +682,16 @@ struct Block {
   Proj qkv, o, ug, down;
   Gain n1, n2, qn, kn;
 
+  // the intermediate results' places in the scratch memory, `most` bytes
+  size_t x1, sx, qkv_rows, att, codes, q, k, parts, up_gate, h_codes, most;
+  int64_t parts_bytes;
+
   bool read(PyObject* block, PyObject* x, PyObject* rotary, PyObject* cache);
-  int queue(const void* in, void* out, const char** what) const;
+  void lay_out();
+  bool few() const { return M <= DECODE_ROWS; }
+  bool step() const { return S == 1; }
+  bool merge() const { return step() && merge_in_projection(B, Hq * D, total); }
+  int queue(const void* in, void* out, char* base, const char** what) const;  // allocates nothing: runs without the interpreter lock
 };
 
 bool Block::read(PyObject* block, PyObject* px, PyObject* protary, PyObject* cache) {
@@ -751,30 +766,32 @@ bool Block::read(PyObject* block, PyObject* px, PyObject* protary, PyObject* cac
   return true;
 }
 
-// Queues the block's launches: the ones, in the order and with the operands, of the step-by-step path in block.py.
-int Block::queue(const void* in, void* out, const char** what) const {
-  const bool few = M <= DECODE_ROWS, step = S == 1;
-  const int64_t W = qkv.N, A = Hq * D, KV = Hkv * D;
-  const bool merge = step && merge_in_projection(B, A, total);
+void Block::lay_out() {
+  const int64_t A = Hq * D, KV = Hkv * D, longest = dim > A ? dim : A, widest = F > dim ? F : dim;
   Scratch m;
-  const size_t at_x1 = m.take(2 * M * dim), at_sx = m.take(4 * M), shared = m.used;
+  x1 = m.take(2 * M * dim), sx = m.take(4 * M);
+  const size_t shared = m.used;
   // attention
-  const size_t at_qkv = m.take(2 * M * W), at_att = m.take(2 * M * A);
-  const int64_t longest = dim > A ? dim : A;
-  const size_t at_codes = m.take(few ? lib.aq_gemv_w8a8_workspace_bytes(M, longest) : static_cast<size_t>(M * longest));
-  const size_t at_q = step ? 0 : m.take(2 * M * A), at_k = step || !direct ? 0 : m.take(2 * M * KV);
-  const int64_t parts_bytes = !step   ? 0
-                              : merge ? lib.aq_paged_attn_decode_partials_bytes(B, Hq, total)
-                                      : lib.aq_paged_attn_decode_workspace_bytes(B, Hq, Hkv, total);
-  const size_t at_parts = m.take(static_cast<size_t>(parts_bytes));
+  qkv_rows = m.take(2 * M * qkv.N), att = m.take(2 * M * A);
+  codes = m.take(few() ? lib.aq_gemv_w8a8_workspace_bytes(M, longest) : static_cast<size_t>(M * longest));
+  q = step() ? 0 : m.take(2 * M * A), k = step() || !direct ? 0 : m.take(2 * M * KV);
+  parts_bytes = !step()   ? 0
+                : merge() ? lib.aq_paged_attn_decode_partials_bytes(B, Hq, total)
+                          : lib.aq_paged_attn_decode_workspace_bytes(B, Hq, Hkv, total);
+  parts = m.take(static_cast<size_t>(parts_bytes));
   // the MLP, over the attention's results
   m.used = shared;
-  const size_t at_ug = m.take(2 * M * (swiglu_gemv ? F : 2 * F));
-  const size_t at_hq = m.take(few ? lib.aq_gemv_w8a8_workspace_bytes(M, F > dim ? F : dim) : static_cast<size_t>(M * (F > dim ? F : dim)));
-  Tensor mem = c.empty({static_cast<int64_t>(m.most)}, ScalarType::Byte);
-  char* base = static_cast<char*>(mem.mutable_data_ptr());
-  void* x1 = base + at_x1;
-  float* sx = reinterpret_cast<float*>(base + at_sx);
+  up_gate = m.take(2 * M * (swiglu_gemv ? F : 2 * F));
+  h_codes = m.take(few() ? lib.aq_gemv_w8a8_workspace_bytes(M, widest) : static_cast<size_t>(M * widest));
+  most = m.most;
+}
+
+// Queues the block's launches: the ones, in the order and with the operands, of the step-by-step path in block.py.
+int Block::queue(const void* in, void* out, char* base, const char** what) const {
+  const bool few = this->few();
+  const int64_t W = qkv.N, A = Hq * D, KV = Hkv * D;
+  void* x1 = base + this->x1;
+  float* sx = reinterpret_cast<float*>(base + this->sx);
 
   // y = projection of normalised tokens / of tokens as they are (+ residual); codes: room for M rows of the projection's K
   auto normed = [&](const Proj& p, const Gain& g, const void* x, void* y, size_t at) {
@@ -806,12 +823,12 @@ int Block::queue(const void* in, void* out, const char** what) const {
                                        c.stream);
   };
 
-  char *q = base + at_qkv, *att = base + at_att, *parts = base + at_parts;
-  int rc = normed(qkv, n1, in, q, at_codes);
+  char *q = base + qkv_rows, *att = base + this->att, *parts = base + this->parts;
+  int rc = normed(qkv, n1, in, q, codes);
   if (rc) return rc;
-  if (step) {
+  if (step()) {
     *what = "aq_rope_paged_attn_decode";
-    if (merge) {
+    if (merge()) {
       rc = qk_norm ? lib.aq_rope_paged_attn_decode_partials_qknorm(q, fr, fr_stride, table, P, total, lens, page, kc, vc, n_pages, scale, B,
                                                                    Hq, Hkv, D, qn.p, kn.p, qn.eps, parts, parts_bytes, c.stream)
                    : lib.aq_rope_paged_attn_decode_partials(q, fr, fr_stride, table, P, total, lens, page, kc, vc, n_pages, scale, B, Hq,
@@ -827,10 +844,10 @@ int Block::queue(const void* in, void* out, const char** what) const {
                    : lib.aq_rope_paged_attn_decode(q, fr, fr_stride, table, P, total, lens, page, kc, vc, n_pages, scale, att, B, Hq, Hkv,
                                                    D, ws, parts_bytes, c.stream);
       if (rc) return rc;
-      rc = projected(o, att, in, x1, at_codes);
+      rc = projected(o, att, in, x1, codes);
     }
   } else {
-    char *qr = base + at_q, *kr = direct ? base + at_k : nullptr;
+    char *qr = base + this->q, *kr = direct ? base + k : nullptr;
     *what = "aq_rope_kv_write";
     rc = qk_norm ? lib.aq_rope_kv_write_qknorm(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, qr, kr, B, Hq, Hkv, D, qn.p,
                                                kn.p, qn.eps, c.stream)
@@ -847,17 +864,17 @@ int Block::queue(const void* in, void* out, const char** what) const {
                                            c.stream);
     }
     if (rc) return rc;
-    rc = projected(o, att, in, x1, at_codes);
+    rc = projected(o, att, in, x1, codes);
   }
   if (rc) return rc;
 
-  char *h = base + at_ug, *hq = base + at_hq;
+  char *h = base + up_gate, *hq = base + h_codes;
   if (swiglu_gemv) {
     *what = "aq_gemv_w8a8_decode_swiglu";
     rc = lib.aq_gemv_w8a8_decode_swiglu(x1, AQ_BF16, n2.p, n2.eps, ug.w, ug.s, ug.b.p, ug.b.code, h, AQ_BF16, M, F, dim, c.stream);
-    return rc ? rc : projected(down, h, x1, out, at_hq);
+    return rc ? rc : projected(down, h, x1, out, h_codes);
   }
-  rc = normed(ug, n2, x1, h, at_hq);
+  rc = normed(ug, n2, x1, h, h_codes);
   if (rc) return rc;
   *what = "aq_swiglu_quant_rowwise_i8";
   rc = lib.aq_swiglu_quant_rowwise_i8(h, AQ_BF16, M, F, 2 * F, reinterpret_cast<int8_t*>(hq), sx, c.stream);
@@ -875,9 +892,11 @@ PyObject* block_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!types.block_ops || !unobserved(types.block_ops)) return none();
   Block b;
   if (!b.read(args[0], args[1], args[2], args[3])) return none();
-  Tensor y = b.c.empty({b.B, b.S, b.dim}, ScalarType::BFloat16);
+  b.lay_out();
+  Tensor y = b.c.empty({b.B, b.S, b.dim}, ScalarType::BFloat16), mem = b.c.empty({static_cast<int64_t>(b.most)}, ScalarType::Byte);
   const char* what = "";
-  const int rc = queued([&] { return b.queue(b.hold_x.const_data_ptr(), y.mutable_data_ptr(), &what); });
+  const int rc = queued(
+      [&] { return b.queue(b.hold_x.const_data_ptr(), y.mutable_data_ptr(), static_cast<char*>(mem.mutable_data_ptr()), &what); });
   return rc ? fail(rc, what) : THPVariable_Wrap(y);
   AQ_CATCH
 }

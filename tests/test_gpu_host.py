@@ -127,3 +127,45 @@ def test_forms_of_a_layer_call(rows):
         y = layer(x)
         handle.remove()
         assert len(seen) == 1 and torch.equal(seen[0], y) and torch.equal(y, layer(x)) and len(seen) == 1
+
+
+class _Room:
+    """Inside it torch's allocator may take ``room`` bytes more from the device than it already holds."""
+
+    def __init__(self, room):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        self.fraction = (torch.cuda.memory_reserved() + room) / torch.cuda.mem_get_info()[1]
+
+    def __enter__(self):
+        torch.cuda.set_per_process_memory_fraction(self.fraction)
+
+    def __exit__(self, *exc):
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def test_out_of_memory_in_a_block_is_an_error_and_the_program_goes_on():
+    """The block's scratch memory, 31.5 MiB for these tokens, does not fit; its output, 4 MiB, does."""
+    b = _block()
+    x, fr, cache, table = _case(b, 1, 4096, 0)
+    cache.bind(table, 4096)
+    with torch.inference_mode():
+        want = b(x, fr, None, cache)
+        with _Room(24 << 20):
+            y = torch.empty_like(x)
+            with pytest.raises(RuntimeError):  # what the block will ask for
+                torch.empty(31 << 20, dtype=torch.uint8, device=DEV)
+            del y
+            with pytest.raises(RuntimeError, match="out of memory"):
+                b(x, fr, None, cache)
+        assert torch.equal(b(x, fr, None, cache), want)
+
+
+def test_out_of_memory_in_a_layer_is_an_error_and_the_program_goes_on():
+    q = QuantLinear(256, 8192, device=DEV)
+    x = torch.randn(4096, 256, device=DEV).to(DT)
+    with torch.inference_mode():
+        want = q(x)
+        with _Room(24 << 20), pytest.raises(RuntimeError, match="out of memory"):
+            q(x)
+        assert torch.equal(q(x), want)
