@@ -9,7 +9,8 @@
 // Every function here serves the plain case only: tensors of exactly torch.Tensor or nn.Parameter, contiguous, on the
 // current device, of the types the kernels take.  For anything else it returns None (nothing has been queued then) and
 // the Python code that calls it goes on with its general path, which copies what is not contiguous and raises the
-// errors.  So there is no second set of error messages here; what the C ABI itself refuses is raised as _abi.check does.
+// errors.  So there is no second set of error messages here; what the C ABI itself refuses is raised as _abi.check does,
+// and what torch throws (out of memory) as torch's own functions raise it.
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <Python.h>
@@ -17,6 +18,7 @@
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
@@ -195,13 +197,6 @@ int queued(F&& launch) {
   return rc;
 }
 
-#define AQ_TRY try {
-#define AQ_CATCH                                       \
-  }                                                    \
-  catch (const std::exception& e) {                    \
-    PyErr_SetString(PyExc_RuntimeError, e.what());     \
-    return nullptr;                                    \
-  }
 #define AQ_ARGS(n)                                                                       \
   if (nargs != (n)) return PyErr_Format(PyExc_TypeError, "expected %d arguments", n);    \
   if (!lib.aq_error_string) return PyErr_Format(PyExc_RuntimeError, "no library is bound")
@@ -210,7 +205,7 @@ int queued(F&& launch) {
 
 // quant_rowwise_i8(x) -> (codes, scales)
 PyObject* quant_rowwise_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(1);
+  HANDLE_TH_ERRORS AQ_ARGS(1);
   const Tensor* x = unpack(args[0]);
   Call c;
   Rows r;
@@ -222,12 +217,12 @@ PyObject* quant_rowwise_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                    static_cast<float*>(s.mutable_data_ptr()), c.stream);
   });
   return rc ? fail(rc, "aq_quant_rowwise_i8") : pair(q, s);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // rmsnorm_quant_rowwise_i8(x, gamma, eps) -> (codes, scales)
 PyObject* rmsnorm_quant_rowwise_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(3);
+  HANDLE_TH_ERRORS AQ_ARGS(3);
   const Tensor *x = unpack(args[0]), *g = unpack(args[1]);
   Call c;
   Rows r;
@@ -242,12 +237,12 @@ PyObject* rmsnorm_quant_rowwise_i8(PyObject*, PyObject* const* args, Py_ssize_t 
                                            c.stream);
   });
   return rc ? fail(rc, "aq_rmsnorm_quant_rowwise_i8") : pair(q, s);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // swiglu_quant_rowwise_i8(ug) -> (codes, scales)
 PyObject* swiglu_quant_rowwise_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(1);
+  HANDLE_TH_ERRORS AQ_ARGS(1);
   const Tensor* x = unpack(args[0]);
   Call c;
   Rows r;
@@ -260,12 +255,12 @@ PyObject* swiglu_quant_rowwise_i8(PyObject*, PyObject* const* args, Py_ssize_t n
                                           static_cast<float*>(s.mutable_data_ptr()), c.stream);
   });
   return rc ? fail(rc, "aq_swiglu_quant_rowwise_i8") : pair(q, s);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // gemv_w8a8_decode(x, wq, sw, bias, out_dtype, residual, gamma, eps) -> y [M, N]: at most 16 rows
 PyObject* gemv_w8a8_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(8);
+  HANDLE_TH_ERRORS AQ_ARGS(8);
   const Tensor *x = unpack(args[0]), *w, *s;
   Call c;
   Rows r;
@@ -298,7 +293,7 @@ PyObject* gemv_w8a8_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                                 N, r.K, ws.mutable_data_ptr(), need, c.stream);
   });
   return rc ? fail(rc, "aq_gemv_w8a8_decode") : THPVariable_Wrap(y);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // (xq, sx, wq, sw, bias, out_dtype, residual) -> y [M, N] through one of the entry points that take codes
@@ -327,14 +322,14 @@ PyObject* on_codes(PyObject* const* args, bool fp8, int64_t max_rows, const char
 
 #define AQ_ON_CODES(NAME, ENTRY, CODE, FP8, MAX_ROWS)                                                                       \
   PyObject* NAME(PyObject*, PyObject* const* args, Py_ssize_t nargs) {                                                      \
-    AQ_TRY AQ_ARGS(7);                                                                                                      \
+    HANDLE_TH_ERRORS AQ_ARGS(7);                                                                                            \
     return on_codes(args, FP8, MAX_ROWS, #ENTRY,                                                                            \
                     [](const void* xq, const float* sx, const void* w, const float* sw, const Bias& b, const void* res,     \
                        void* y, int y_code, int64_t M, int64_t N, int64_t K, void* stream) {                                \
                       return lib.ENTRY(static_cast<const CODE*>(xq), sx, static_cast<const CODE*>(w), sw, b.p, b.code, res, \
                                        y, y_code, M, N, K, stream);                                                         \
                     });                                                                                                     \
-    AQ_CATCH                                                                                                                \
+    END_HANDLE_TH_ERRORS                                                                                                    \
   }
 AQ_ON_CODES(linear_w8a8, aq_linear_w8a8_residual, int8_t, false, INT64_MAX)
 AQ_ON_CODES(gemv_w8a8_codes, aq_gemv_w8a8_codes_residual, int8_t, false, 16)
@@ -342,7 +337,7 @@ AQ_ON_CODES(linear_fp8, aq_linear_fp8_residual, uint8_t, true, INT64_MAX)
 
 // gemv_fp8_decode(x, wq, sw, bias, out_dtype, residual) -> y [M, N]: at most 16 rows
 PyObject* gemv_fp8_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(6);
+  HANDLE_TH_ERRORS AQ_ARGS(6);
   const Tensor *x = unpack(args[0]), *w, *s;
   Call c;
   Rows r;
@@ -363,12 +358,12 @@ PyObject* gemv_fp8_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                            act_code(type), r.M, N, r.K, ws.mutable_data_ptr(), need, c.stream);
   });
   return rc ? fail(rc, "aq_gemv_fp8_decode") : THPVariable_Wrap(y);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // quant_tensor_fp8(x, state or None) -> (codes with x's shape, scale [1]); with the state: the one-launch form
 PyObject* quant_tensor_fp8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(2);
+  HANDLE_TH_ERRORS AQ_ARGS(2);
   const Tensor* x = unpack(args[0]);
   Call c;
   if (!x || !c.at(*x) || act_code(x->scalar_type()) < 0 || !x->is_contiguous() || x->numel() % 16 || x->numel() == 0) return none();
@@ -389,7 +384,7 @@ PyObject* quant_tensor_fp8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                            static_cast<uint32_t*>(ws.mutable_data_ptr()), AQ_FP8_AMAX_WS_BYTES, c.stream);
   });
   return rc ? fail(rc, state ? "aq_quant_tensor_fp8_onepass" : "aq_quant_tensor_fp8") : pair(q, s);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // ---- module attributes, read where nn.Module keeps them ----------------------------------------------------------
@@ -511,7 +506,7 @@ constexpr int64_t FP8_ONEPASS_MIN_BYTES = 16 << 20;  // ops.FP8_ONEPASS_MIN_BYTE
 // What calling the QuantLinear or Fp8Linear gives, or None where nn.Module's own call has to serve: hooks, a shared input, FP8
 // inputs that are quantised in one launch with a state the module keeps.
 PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs, PyObject* names) {
-  AQ_TRY
+  HANDLE_TH_ERRORS
   const bool fp8 = reinterpret_cast<PyObject*>(Py_TYPE(layer)) == types.fp8_linear;
   if (!lib.aq_error_string || !types.linear_ops || nargs != 1 || !ordinary(layer, fp8 ? types.fp8_linear : types.quant_linear, true) ||
       !unobserved(types.linear_ops))
@@ -601,7 +596,7 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
     return lib.aq_linear_w8a8_residual(q, sx, static_cast<const int8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
   });
   return rc ? fail(rc, what) : THPVariable_Wrap(y);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // __call__ of the quantized layers
@@ -888,7 +883,7 @@ int Block::queue(const void* in, void* out, char* base, const char** what) const
 
 // block_forward(block, x, rotary, cache) -> the block's output, or None where the step-by-step path has to serve
 PyObject* block_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_TRY AQ_ARGS(4);
+  HANDLE_TH_ERRORS AQ_ARGS(4);
   if (!types.block_ops || !unobserved(types.block_ops)) return none();
   Block b;
   if (!b.read(args[0], args[1], args[2], args[3])) return none();
@@ -898,7 +893,7 @@ PyObject* block_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int rc = queued(
       [&] { return b.queue(b.hold_x.const_data_ptr(), y.mutable_data_ptr(), static_cast<char*>(mem.mutable_data_ptr()), &what); });
   return rc ? fail(rc, what) : THPVariable_Wrap(y);
-  AQ_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // set_block_types(RMSNorm, GQA, MLP, PagedKV, {name: operator as defined})

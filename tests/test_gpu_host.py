@@ -129,18 +129,22 @@ def test_forms_of_a_layer_call(rows):
         assert len(seen) == 1 and torch.equal(seen[0], y) and torch.equal(y, layer(x)) and len(seen) == 1
 
 
-class _Room:
-    """Inside it torch's allocator may take ``room`` bytes more from the device than it already holds."""
-
-    def __init__(self, room):
-        torch.cuda.synchronize()
-        torch.cuda.empty_cache()
-        self.fraction = (torch.cuda.memory_reserved() + room) / torch.cuda.mem_get_info()[1]
+class _Full:
+    """Inside it torch's allocator has 24 MiB left, and no piece of 28 MiB or more."""
 
     def __enter__(self):
-        torch.cuda.set_per_process_memory_fraction(self.fraction)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (24 << 20)) / torch.cuda.mem_get_info()[1])
+        self.held = []
+        try:
+            while True:  # what is free between the blocks in use
+                self.held.append(torch.empty(28 << 20, dtype=torch.uint8, device=DEV))
+        except torch.OutOfMemoryError:
+            pass
 
     def __exit__(self, *exc):
+        self.held = None
         torch.cuda.set_per_process_memory_fraction(1.0)
 
 
@@ -151,12 +155,9 @@ def test_out_of_memory_in_a_block_is_an_error_and_the_program_goes_on():
     cache.bind(table, 4096)
     with torch.inference_mode():
         want = b(x, fr, None, cache)
-        with _Room(24 << 20):
-            y = torch.empty_like(x)
-            with pytest.raises(RuntimeError):  # what the block will ask for
-                torch.empty(31 << 20, dtype=torch.uint8, device=DEV)
-            del y
-            with pytest.raises(RuntimeError, match="out of memory"):
+        with _Full():
+            torch.empty_like(x)
+            with pytest.raises(torch.OutOfMemoryError):
                 b(x, fr, None, cache)
         assert torch.equal(b(x, fr, None, cache), want)
 
@@ -166,6 +167,18 @@ def test_out_of_memory_in_a_layer_is_an_error_and_the_program_goes_on():
     x = torch.randn(4096, 256, device=DEV).to(DT)
     with torch.inference_mode():
         want = q(x)
-        with _Room(24 << 20), pytest.raises(RuntimeError, match="out of memory"):
+        with _Full(), pytest.raises(torch.OutOfMemoryError):
             q(x)
         assert torch.equal(q(x), want)
+
+
+def test_out_of_memory_in_an_operator_has_torchs_type():
+    x = torch.randn(8192, 4096, device=DEV, dtype=DT)
+    wq, sw = torch.zeros(8192, 4096, dtype=torch.int8, device=DEV), torch.ones(8192, device=DEV)
+    xq, sx = ops.quant_rowwise_i8(x)
+    with _Full():
+        for call in (lambda: ops.quant_rowwise_i8(x), lambda: ops.rmsnorm_quant_rowwise_i8(x, x[0], 1e-5),
+                     lambda: ops.quant_tensor_fp8(x), lambda: ops.linear_w8a8(xq, sx, wq, sw)):
+            with pytest.raises(torch.OutOfMemoryError):
+                call()
+    assert torch.equal(ops.quant_rowwise_i8(x)[0], xq)
