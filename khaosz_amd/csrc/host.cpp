@@ -84,6 +84,13 @@ using at::Tensor;
 // The tensor behind a Python object, or null: a subclass (fake, functional, quantised by someone else) is not plain.
 const Tensor* unpack(PyObject* o) { return o && THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
 
+struct Held {  // a reference to a Python object (two copies of a Tensor cost 0.08 us, of its Python object nothing)
+  PyObject* const o;
+  explicit Held(PyObject* p) : o(p) { Py_INCREF(o); }
+  ~Held() { Py_DECREF(o); }
+  Held(const Held&) = delete;
+};
+
 // aq dtype code of an activation type, -1 for one the kernels do not take
 int act_code(ScalarType t) { return t == ScalarType::BFloat16 ? AQ_BF16 : t == ScalarType::Float ? AQ_F32 : -1; }
 
@@ -528,9 +535,9 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   Rows r;
   Bias b;
   const void* res;
-  if (!x || x->requires_grad() || !c.at(*x) || !rows_of(*x, &r) ||
-      !weight_of(nested(d, k_buffers, k_qweight), nested(d, k_buffers, k_w_scale), r.K, c.dev, fp8, &w, &s))
-    return none();
+  PyObject *wq = nested(d, k_buffers, k_qweight), *sw = nested(d, k_buffers, k_w_scale);
+  if (!x || x->requires_grad() || !c.at(*x) || !rows_of(*x, &r) || !weight_of(wq, sw, r.K, c.dev, fp8, &w, &s)) return none();
+  const Held hold_w(wq), hold_s(sw);  // the module may be given others while the interpreter lock is released
   const int64_t N = w->size(0);
   const ScalarType type = x->scalar_type();
   PyObject* bias = nested(d, k_parameters, k_bias);

@@ -1,9 +1,13 @@
 """The native host path (csrc/host.cpp): a fused block queued in one call gives the bits of the step-by-step path, keeps out of
 the way of hooks and replaced operators, and operators fed with what the native functions do not take still answer."""
+import ctypes
+import pathlib
+import subprocess
+
 import pytest
 import torch
 
-from khaosz_amd import QuantLinear, fuse_shared_inputs, ops, quantize_model
+from khaosz_amd import QuantLinear, _abi, fuse_shared_inputs, ops, quantize_model
 from khaosz_amd.block import DecoderBlock, PagedKV, rotary_table
 
 pytestmark = pytest.mark.gpu
@@ -182,3 +186,59 @@ def test_out_of_memory_in_an_operator_has_torchs_type():
             with pytest.raises(torch.OutOfMemoryError):
                 call()
     assert torch.equal(ops.quant_rowwise_i8(x)[0], xq)
+
+
+_INTERRUPTED = """
+#include <dlfcn.h>
+#include "astrai_q.h"
+void (*aq_test_between)(void);
+int aq_linear_w8a8_residual(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw, const void* b, int bt,
+                            const void* r, void* y, int yt, int64_t M, int64_t N, int64_t K, void* st) {
+  static int (*real)(const int8_t*, const float*, const int8_t*, const float*, const void*, int, const void*, void*, int,
+                     int64_t, int64_t, int64_t, void*);
+  if (!real) *(void**)&real = dlsym(RTLD_NEXT, "aq_linear_w8a8_residual");
+  aq_test_between();
+  return real(xq, sx, wq, sw, b, bt, r, y, yt, M, N, K, st);
+}
+"""
+
+
+@pytest.fixture
+def between(tmp_path):
+    """Binds the native path to a library whose GEMM entry calls a Python function before it queues its launch -- what
+    another thread may do while the interpreter lock is released."""
+    src, so = tmp_path / "between.c", tmp_path / "between.so"
+    src.write_text(_INTERRUPTED)
+    product = _abi.LIB_PATH
+    subprocess.run(["gcc", "-D_GNU_SOURCE", "-shared", "-fPIC", "-I", str(pathlib.Path(__file__).parent.parent / "include"), str(src),
+                    "-o", str(so), "-Wl,--no-as-needed", product, f"-Wl,-rpath,{pathlib.Path(product).parent}"], check=True)
+    lib, done = ctypes.CDLL(str(so)), []
+
+    def bind(f):
+        done.append(ctypes.CFUNCTYPE(None)(f))
+        ctypes.c_void_p.in_dll(lib, "aq_test_between").value = ctypes.cast(done[-1], ctypes.c_void_p).value
+        _abi.host().bind(lib._handle)
+
+    yield bind
+    _abi.host().bind(_abi.load()._handle)
+
+
+def test_a_layer_holds_its_weight_for_the_length_of_a_call(between):
+    """Another thread gives the module new buffers after the call has let go of the interpreter lock and before its GEMM
+    is queued: the old ones stay until it is."""
+    torch.manual_seed(2)
+    base = torch.nn.Linear(512, 8192).to(DEV).to(DT)
+    q, x = QuantLinear.from_linear(base), torch.randn(64, 512, device=DEV).to(DT)
+    with torch.inference_mode():
+        want = q(x)
+        old = []
+
+        def swap():
+            old.append(torch.cuda.memory_allocated())
+            q._buffers["qweight"], q._buffers["w_scale"] = torch.ones_like(q.qweight), torch.ones_like(q.w_scale)
+            old.append(torch.cuda.memory_allocated())
+
+        between(swap)
+        y = q(x)
+    assert torch.equal(y, want)
+    assert old[1] - old[0] >= 8192 * 512 + 4 * 8192  # the new ones beside the old ones
