@@ -21,7 +21,6 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
-#include <algorithm>
 #include <cmath>
 
 #include "../../include/astrai_q.h"
@@ -401,7 +400,7 @@ PyObject *k_modules, *k_buffers, *k_parameters, *k_qweight, *k_w_scale, *k_bias,
     *k_fwd_pre_hooks, *k_compiled, *k_attention, *k_mlp, *k_input_norm, *k_post_norm, *k_qkv, *k_upgate, *k_o_proj, *k_down, *k_q_norm,
     *k_k_norm, *k_decode_attention, *k_use_qk_norm, *k_use_gate, *k_n_heads, *k_n_kv_heads, *k_head_dim, *k_layer_id, *k_swiglu_quant,
     *k_norm_quant, *k_residual_adds, *k_k_layers, *k_v_layers, *k_page_table, *k_total_len, *k_seq_lens, *k_invalid, *k_page_size,
-    *k_shared, *k_residual, *k_norm, *k_call;
+    *k_shared, *k_residual, *k_norm;
 
 PyObject* dict_of(PyObject* o) {  // borrowed; null if it has none
   PyObject** d = _PyObject_GetDictPtr(o);
@@ -426,7 +425,6 @@ struct Types {
   PyObject* ops_dict = nullptr;      // the operators' module and, by name, the operators as they were defined
   PyObject *linear_ops = nullptr, *block_ops = nullptr;
   uint64_t linear_ops_version = 0, block_ops_version = 0;  // of ops_dict when it last held them all
-  PyObject* module = nullptr;  // torch.nn.Module
   PyObject *rms_norm = nullptr, *gqa = nullptr, *mlp = nullptr, *paged_kv = nullptr;
 } types;
 
@@ -606,43 +604,35 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   END_HANDLE_TH_ERRORS
 }
 
-// __call__ of the quantized layers
-PyObject* linear_call(PyObject* layer, PyObject* const* args, Py_ssize_t nargs, PyObject* names) {
-  PyObject* y = linear_native(layer, args, nargs, names);
-  if (y != Py_None) return y;
-  Py_DECREF(y);
-  PyObject* call = PyObject_GetAttr(types.module, k_call);  // looked up each time: tracers replace it
-  if (!call) return nullptr;
-  PyObject* few[8];
-  const Py_ssize_t n = nargs + (names ? PyTuple_GET_SIZE(names) : 0);
-  PyObject** all = n < 8 ? few : static_cast<PyObject**>(PyMem_Malloc((n + 1) * sizeof(PyObject*)));
-  if (all) {
-    all[0] = layer;
-    std::copy(args, args + n, all + 1);
-    y = PyObject_Vectorcall(call, all, nargs + 1, names);
-  } else {
-    y = PyErr_NoMemory();
+// The call of the quantized layers' __call__, a Python function: its own code serves what linear_native does not take, and
+// is what a compiler that traces the call reads (a method written in C it could not).
+PyObject* linear_call(PyObject* function, PyObject* const* args, size_t nargsf, PyObject* names) {
+  const Py_ssize_t nargs = PyVectorcall_NARGS(nargsf);
+  if (nargs > 0) {
+    PyObject* y = linear_native(args[0], args + 1, nargs - 1, names);
+    if (y != Py_None) return y;
+    Py_DECREF(y);
   }
-  if (all != few) PyMem_Free(all);
-  Py_DECREF(call);
-  return y;
-}
-PyMethodDef linear_call_def = {"__call__", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(linear_call)),
-                               METH_FASTCALL | METH_KEYWORDS, nullptr};
-
-// linear_call_method(cls) -> linear_call as a method of that class
-PyObject* linear_call_method(PyObject*, PyObject* cls) {
-  if (!PyType_Check(cls)) return PyErr_Format(PyExc_TypeError, "linear_call_method");
-  return PyDescr_NewMethod(reinterpret_cast<PyTypeObject*>(cls), &linear_call_def);
+  return _PyFunction_Vectorcall(function, args, nargsf, names);
 }
 
-// set_linear_types(QuantLinear, Fp8Linear, hook dicts, ops.__dict__, {name: operator as defined}, torch.nn.Module)
+// serve_calls(function): has calls of _NativeCall.__call__ come to linear_call
+PyObject* serve_calls(PyObject*, PyObject* function) {
+  if (!PyFunction_Check(function)) return PyErr_Format(PyExc_TypeError, "serve_calls");
+#if PY_VERSION_HEX >= 0x030c0000
+  PyFunction_SetVectorcall(reinterpret_cast<PyFunctionObject*>(function), linear_call);
+#else
+  reinterpret_cast<PyFunctionObject*>(function)->vectorcall = linear_call;
+#endif
+  Py_RETURN_NONE;
+}
+
+// set_linear_types(QuantLinear, Fp8Linear, hook dicts, ops.__dict__, {name: operator as defined})
 PyObject* set_linear_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_ARGS(6);
+  AQ_ARGS(5);
   if (!PyTuple_Check(args[2]) || !PyDict_Check(args[3]) || !PyDict_Check(args[4])) return PyErr_Format(PyExc_TypeError, "set_linear_types");
-  for (Py_ssize_t i = 0; i < 6; ++i) Py_INCREF(args[i]);  // for the life of the process
+  for (Py_ssize_t i = 0; i < 5; ++i) Py_INCREF(args[i]);  // for the life of the process
   types.quant_linear = args[0], types.fp8_linear = args[1], types.global_hooks = args[2], types.ops_dict = args[3], types.linear_ops = args[4];
-  types.module = args[5];
   Py_RETURN_NONE;
 }
 
@@ -931,7 +921,7 @@ PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
     AQ_METHOD(set_linear_types),
     AQ_METHOD(set_block_types),
-    {"linear_call_method", linear_call_method, METH_O, nullptr},
+    {"serve_calls", serve_calls, METH_O, nullptr},
     AQ_METHOD(quant_rowwise_i8),
     AQ_METHOD(rmsnorm_quant_rowwise_i8),
     AQ_METHOD(swiglu_quant_rowwise_i8),
@@ -965,8 +955,7 @@ PyMODINIT_FUNC PyInit__host() {
               {&k_norm_quant, "_norm_quant"}, {&k_residual_adds, "_residual_adds"}, {&k_k_layers, "k_layers"},
               {&k_v_layers, "v_layers"},      {&k_page_table, "page_table"},    {&k_total_len, "total_len"},
               {&k_seq_lens, "seq_lens"},      {&k_invalid, "_invalid"},         {&k_page_size, "page_size"},
-              {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"},
-              {&k_call, "__call__"}};
+              {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"}};
   for (const auto& k : keys)
     if (!(*k.key = PyUnicode_InternFromString(k.name))) return nullptr;
   return PyModule_Create(&module);

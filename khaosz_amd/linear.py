@@ -137,8 +137,8 @@ def linear_native():
     if not _told:
         m = torch.nn.modules.module
         h.set_linear_types(QuantLinear, Fp8Linear, (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
-                                                    m._global_backward_pre_hooks), ops.__dict__, _OPERATORS, nn.Module)
-        _NativeCall.__call__ = h.linear_call_method(_NativeCall)
+                                                    m._global_backward_pre_hooks), ops.__dict__, _OPERATORS)
+        h.serve_calls(_NativeCall.__call__)
         _told = True
     return h
 
@@ -152,9 +152,13 @@ class _NativeCall(Linear):
     """A quantized Linear's call: natively in one step where nothing observes it (no hooks, plain tensors), through
     ``nn.Module.__call__`` and ``forward`` otherwise -- the same launches and bits."""
 
-    def __call__(self, *args, **kwargs):  # the first call of a process; then the native method is in its place
-        linear_native()
-        return _NativeCall.__call__(self, *args, **kwargs)
+    def __call__(self, *args, **kwargs):
+        # Calls come to native code first (``serve_calls``), once a layer has been called; what it leaves comes here, and
+        # torch.compile, which traces this function, sees nn.Module's call.
+        if not _told and not torch.compiler.is_compiling() and type(self) in (QuantLinear, Fp8Linear):
+            linear_native()
+            return self(*args, **kwargs)
+        return super().__call__(*args, **kwargs)
 
 
 class QuantLinear(_NativeCall):

@@ -242,3 +242,16 @@ def test_a_layer_holds_its_weight_for_the_length_of_a_call(between):
         y = q(x)
     assert torch.equal(y, want)
     assert old[1] - old[0] >= 8192 * 512 + 4 * 8192  # the new ones beside the old ones
+
+
+def test_a_compiled_layer_and_block_give_the_same_bits():
+    b = _block()
+    x, fr, cache, table = _case(b, 2, 1, 30)
+    cache.bind(table, 31)
+    q = b.mlp.down
+    h = torch.randn(5, 1408, device=DEV).to(DT)
+    with torch.inference_mode():
+        want, block_want = q(h), b(x, fr, None, cache)
+        torch._dynamo.reset()
+        assert torch.equal(torch.compile(lambda h: q(h) * 2, backend="eager")(h), want * 2)
+        assert torch.equal(torch.compile(b, backend="eager")(x, fr, None, cache), block_want)

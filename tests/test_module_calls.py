@@ -1,0 +1,50 @@
+"""What a program may do to the quantized layers' calls from Python, whatever the native path does: trace and replace them."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from khaosz_amd import QuantLinear
+
+
+def _float_forward(self, x, residual=None, norm=None):
+    y = F.linear(x, self.qweight.to(x.dtype)) * self.w_scale
+    return y if residual is None else y + residual
+
+
+class _Float(QuantLinear):
+    """The layer in torch's own operators, for a machine without the GPU."""
+    forward = _float_forward
+
+
+def _layer(cls):
+    q = cls(32, 16)
+    q.qweight.random_(-100, 100, generator=torch.Generator().manual_seed(1))
+    return q, torch.randn(4, 32, generator=torch.Generator().manual_seed(2))
+
+
+@pytest.fixture(params=[False, True], ids=["before", "after"])
+def told(request):
+    """Before and after the process's first call of a layer that goes to native code."""
+    from khaosz_amd import linear
+    if request.param:
+        linear.linear_native()
+    return request.param
+
+
+@pytest.mark.parametrize("inside", [False, True])
+def test_a_subclass_with_a_forward_of_its_own_compiles_without_a_graph_break(told, inside):
+    q, x = _layer(_Float)
+    want = q(x)
+    torch._dynamo.reset()
+    f = torch.compile((lambda x: q(x) * 2) if inside else q, fullgraph=True, backend="eager")
+    assert torch.equal(f(x), want * 2 if inside else want)
+    h = q.register_forward_hook(lambda m, a, y: y * 2)
+    assert torch.equal(torch.compile(lambda x: q(x), fullgraph=True, backend="eager")(x), want * 2)
+    h.remove()
+
+
+def test_a_subclass_is_traced_by_fx_and_export(told):
+    q, x = _layer(_Float)
+    model = torch.nn.Sequential(q, torch.nn.ReLU())
+    assert torch.equal(torch.fx.symbolic_trace(model)(x), model(x))
+    assert torch.equal(torch.export.export(model, (x,)).module()(x), model(x))
