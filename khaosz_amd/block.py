@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from . import ops
-from .linear import Linear, QuantLinear, linear_native
+from .linear import Linear, QuantLinear, as_defined, linear_native
 
 
 class RMSNorm(nn.Module):
@@ -458,6 +458,7 @@ _OPERATORS = {name: getattr(ops, name) for name in (
     "quant_rowwise_i8", "rmsnorm_quant_rowwise_i8", "swiglu_quant_rowwise_i8", "linear_w8a8", "gemv_w8a8_decode", "gemv_swiglu_ok",
     "gemv_w8a8_decode_swiglu", "gemv_w8a8_codes", "rope_kv_write", "attn_gemv_fusable", "rope_paged_attn_decode", "gemv_w8a8_attn",
     "prefill_attn_causal", "prefill_attn_paged")}
+_CLASSES = as_defined(GQA, MLP, PagedKV)
 _host = None  # the native block step once it is loaded
 
 
@@ -465,7 +466,7 @@ def _native():
     global _host
     if _host is None:
         h = linear_native()
-        h.set_block_types(RMSNorm, GQA, MLP, PagedKV, _OPERATORS)
+        h.set_block_types(RMSNorm, GQA, MLP, PagedKV, _CLASSES, _OPERATORS)
         _host = h.block_forward
     return _host
 

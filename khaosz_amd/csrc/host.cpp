@@ -400,7 +400,7 @@ PyObject *k_modules, *k_buffers, *k_parameters, *k_qweight, *k_w_scale, *k_bias,
     *k_fwd_pre_hooks, *k_compiled, *k_attention, *k_mlp, *k_input_norm, *k_post_norm, *k_qkv, *k_upgate, *k_o_proj, *k_down, *k_q_norm,
     *k_k_norm, *k_decode_attention, *k_use_qk_norm, *k_use_gate, *k_n_heads, *k_n_kv_heads, *k_head_dim, *k_layer_id, *k_swiglu_quant,
     *k_norm_quant, *k_residual_adds, *k_k_layers, *k_v_layers, *k_page_table, *k_total_len, *k_seq_lens, *k_invalid, *k_page_size,
-    *k_shared, *k_residual, *k_norm;
+    *k_shared, *k_residual, *k_norm, *k_forward_codes, *k_forward_attn;
 
 PyObject* dict_of(PyObject* o) {  // borrowed; null if it has none
   PyObject** d = _PyObject_GetDictPtr(o);
@@ -418,21 +418,61 @@ bool integer(PyObject* d, PyObject* key, int64_t* v) {
   return true;
 }
 
+// A class, and what its instances' calls go through as the package defined it: (class, name, value) for each method.
+struct Class {
+  PyObject *type = nullptr, *defined = nullptr;
+  unsigned version = 0;  // the class's tag when it last was as defined
+};
+
+// No method has been replaced, on the class, one of its bases or nn.Module.  A class that changes, or one of whose bases
+// does, loses its version tag, which is never used twice: usually one compare.
+bool as_defined(Class& c) {
+#if PY_VERSION_HEX < 0x030c0000
+  const auto* t = reinterpret_cast<PyTypeObject*>(c.type);
+  const bool tagged = PyType_HasFeature(const_cast<PyTypeObject*>(t), Py_TPFLAGS_VALID_VERSION_TAG);
+  if (tagged && c.version && c.version == t->tp_version_tag) return true;
+#endif
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(c.defined); ++i) {
+    PyObject* d = PyTuple_GET_ITEM(c.defined, i);
+    if (_PyType_Lookup(reinterpret_cast<PyTypeObject*>(PyTuple_GET_ITEM(d, 0)), PyTuple_GET_ITEM(d, 1)) != PyTuple_GET_ITEM(d, 2)) return false;
+  }
+#if PY_VERSION_HEX < 0x030c0000
+  c.version = PyType_HasFeature(const_cast<PyTypeObject*>(t), Py_TPFLAGS_VALID_VERSION_TAG) ? t->tp_version_tag : 0;
+#endif
+  return true;
+}
+
+// {class: ((class, name, value), ...)} as linear.as_defined() makes it; held for the life of the process
+bool take_class(PyObject* classes, PyObject* type, Class* c) {
+  PyObject* defined = PyDict_GetItem(classes, type);
+  if (!PyType_Check(type) || !defined || !PyTuple_CheckExact(defined)) return false;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(defined); ++i) {
+    PyObject* d = PyTuple_GET_ITEM(defined, i);
+    if (!PyTuple_CheckExact(d) || PyTuple_GET_SIZE(d) != 3 || !PyType_Check(PyTuple_GET_ITEM(d, 0)) || !PyUnicode_CheckExact(PyTuple_GET_ITEM(d, 1)))
+      return false;
+  }
+  Py_INCREF(type);
+  Py_INCREF(defined);
+  *c = {type, defined, 0};
+  return true;
+}
+
 // What the functions that stand for a module's call are told about the Python side, once (set_linear_types, set_block_types).
 struct Types {
-  PyObject *quant_linear = nullptr, *fp8_linear = nullptr;
+  Class quant_linear, fp8_linear, gqa, mlp, paged_kv;
   PyObject* global_hooks = nullptr;  // tuple of the dicts of hooks that run for every module
   PyObject* ops_dict = nullptr;      // the operators' module and, by name, the operators as they were defined
   PyObject *linear_ops = nullptr, *block_ops = nullptr;
   uint64_t linear_ops_version = 0, block_ops_version = 0;  // of ops_dict when it last held them all
-  PyObject *rms_norm = nullptr, *gqa = nullptr, *mlp = nullptr, *paged_kv = nullptr;
+  PyObject* rms_norm = nullptr;
 } types;
 
-// A module whose forward may be replaced by what it is known to do: exactly the class, nothing hooked, nothing wrapped.
-// `called`: the step-by-step path would call it as a module (hooks would run); otherwise only its tensors are read.
-bool ordinary(PyObject* m, PyObject* type, bool called) {
-  if (!m || reinterpret_cast<PyObject*>(Py_TYPE(m)) != type) return false;
-  if (!called) return true;
+bool exactly(PyObject* o, PyObject* type) { return o && reinterpret_cast<PyObject*>(Py_TYPE(o)) == type; }
+
+// A module whose forward may be replaced by what it is known to do: exactly the class, as it was defined, nothing hooked,
+// nothing wrapped.
+bool ordinary(PyObject* m, Class& c) {
+  if (!exactly(m, c.type) || !as_defined(c)) return false;
   PyObject* d = dict_of(m);
   if (!d || PyDict_GetItem(d, k_forward)) return false;
   PyObject *h = get(d, k_fwd_hooks), *p = get(d, k_fwd_pre_hooks), *comp = get(d, k_compiled);
@@ -468,10 +508,10 @@ struct Proj {  // a QuantLinear's tensors, held for the length of the call
   Bias b;
   int64_t N = 0, K = 0;
 };
-bool proj_of(PyObject* m, int dev, bool called, Proj* p) {
-  if (!ordinary(m, types.quant_linear, called)) return false;
+bool proj_of(PyObject* m, int dev, Proj* p) {
+  if (!ordinary(m, types.quant_linear)) return false;
   PyObject* d = dict_of(m);
-  if (called && get(d, k_shared) != Py_None) return false;
+  if (get(d, k_shared) != Py_None) return false;
   const Tensor *w = unpack(nested(d, k_buffers, k_qweight)), *s = unpack(nested(d, k_buffers, k_w_scale));
   if (!w || !s || w->dim() != 2 || !plain(*w, ScalarType::Char, dev) || !plain(*s, ScalarType::Float, dev)) return false;
   p->N = w->size(0);
@@ -492,7 +532,7 @@ struct Gain {
   float eps = 0.f;
 };
 bool gain_of(PyObject* m, int64_t K, int dev, Gain* g) {
-  if (!ordinary(m, types.rms_norm, false)) return false;
+  if (!exactly(m, types.rms_norm)) return false;  // not called: its tensors are read
   PyObject* d = dict_of(m);
   const Tensor* w = unpack(nested(d, k_parameters, k_weight));
   PyObject* eps = get(d, k_norm_eps);
@@ -512,8 +552,8 @@ constexpr int64_t FP8_ONEPASS_MIN_BYTES = 16 << 20;  // ops.FP8_ONEPASS_MIN_BYTE
 // inputs that are quantised in one launch with a state the module keeps.
 PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs, PyObject* names) {
   HANDLE_TH_ERRORS
-  const bool fp8 = reinterpret_cast<PyObject*>(Py_TYPE(layer)) == types.fp8_linear;
-  if (!lib.aq_error_string || !types.linear_ops || nargs != 1 || !ordinary(layer, fp8 ? types.fp8_linear : types.quant_linear, true) ||
+  const bool fp8 = exactly(layer, types.fp8_linear.type);
+  if (!lib.aq_error_string || !types.linear_ops || nargs != 1 || !ordinary(layer, fp8 ? types.fp8_linear : types.quant_linear) ||
       !unobserved(types.linear_ops))
     return none();
   PyObject *residual = nullptr, *norm = nullptr;
@@ -627,12 +667,14 @@ PyObject* serve_calls(PyObject*, PyObject* function) {
   Py_RETURN_NONE;
 }
 
-// set_linear_types(QuantLinear, Fp8Linear, hook dicts, ops.__dict__, {name: operator as defined})
+// set_linear_types(QuantLinear, Fp8Linear, {class: what it defines}, hook dicts, ops.__dict__, {name: operator as defined})
 PyObject* set_linear_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_ARGS(5);
-  if (!PyTuple_Check(args[2]) || !PyDict_Check(args[3]) || !PyDict_Check(args[4])) return PyErr_Format(PyExc_TypeError, "set_linear_types");
-  for (Py_ssize_t i = 0; i < 5; ++i) Py_INCREF(args[i]);  // for the life of the process
-  types.quant_linear = args[0], types.fp8_linear = args[1], types.global_hooks = args[2], types.ops_dict = args[3], types.linear_ops = args[4];
+  AQ_ARGS(6);
+  if (!PyDict_Check(args[2]) || !take_class(args[2], args[0], &types.quant_linear) || !take_class(args[2], args[1], &types.fp8_linear) ||
+      !PyTuple_Check(args[3]) || !PyDict_Check(args[4]) || !PyDict_Check(args[5]))
+    return PyErr_Format(PyExc_TypeError, "set_linear_types");
+  for (Py_ssize_t i = 3; i < 6; ++i) Py_INCREF(args[i]);  // for the life of the process
+  types.global_hooks = args[3], types.ops_dict = args[4], types.linear_ops = args[5];
   Py_RETURN_NONE;
 }
 
@@ -697,15 +739,16 @@ bool Block::read(PyObject* block, PyObject* px, PyObject* protary, PyObject* cac
   PyObject* d = dict_of(block);
   if (!d || !truth(d, k_norm_quant) || !truth(d, k_residual_adds)) return false;
   PyObject *att = nested(d, k_modules, k_attention), *mlp = nested(d, k_modules, k_mlp);
-  if (!ordinary(att, types.gqa, true) || !ordinary(mlp, types.mlp, true)) return false;
+  if (!ordinary(att, types.gqa) || !ordinary(mlp, types.mlp)) return false;
   PyObject *ad = dict_of(att), *md = dict_of(mlp);
   int64_t layer;
   if (!truth(ad, k_decode_attention) || !truth(md, k_swiglu_quant) || get(ad, k_use_gate) != Py_False || !integer(ad, k_n_heads, &Hq) ||
       !integer(ad, k_n_kv_heads, &Hkv) || !integer(ad, k_head_dim, &D) || !integer(ad, k_layer_id, &layer))
     return false;
   qk_norm = truth(ad, k_use_qk_norm);
-  if (!proj_of(get(ad, k_qkv), c.dev, true, &qkv) || !proj_of(nested(ad, k_modules, k_o_proj), c.dev, true, &o) ||
-      !proj_of(get(md, k_upgate), c.dev, true, &ug) || !proj_of(nested(md, k_modules, k_down), c.dev, true, &down) ||
+  PyObject *po = nested(ad, k_modules, k_o_proj), *pdown = nested(md, k_modules, k_down);
+  if (!proj_of(get(ad, k_qkv), c.dev, &qkv) || !proj_of(po, c.dev, &o) || get(dict_of(po), k_forward_attn) ||
+      !proj_of(get(md, k_upgate), c.dev, &ug) || !proj_of(pdown, c.dev, &down) || get(dict_of(pdown), k_forward_codes) ||
       !gain_of(nested(d, k_modules, k_input_norm), dim, c.dev, &n1) || !gain_of(nested(d, k_modules, k_post_norm), dim, c.dev, &n2))
     return false;
   if (qk_norm && (!gain_of(nested(ad, k_modules, k_q_norm), D, c.dev, &qn) || !gain_of(nested(ad, k_modules, k_k_norm), D, c.dev, &kn)))
@@ -715,7 +758,7 @@ bool Block::read(PyObject* block, PyObject* px, PyObject* protary, PyObject* cac
       F > SWIGLU_MAX_F || down.K != F || down.N != dim)
     return false;
   // the cache
-  if (!cache || reinterpret_cast<PyObject*>(Py_TYPE(cache)) != types.paged_kv) return false;
+  if (!exactly(cache, types.paged_kv.type) || !as_defined(types.paged_kv)) return false;
   PyObject* cd = dict_of(cache);
   const Tensor *k = unpack(get(cd, k_k_layers)), *v = unpack(get(cd, k_v_layers)), *t = unpack(get(cd, k_page_table));
   if (!k || !v || !t || !integer(cd, k_total_len, &total) || !integer(cd, k_page_size, &page)) return false;
@@ -893,12 +936,15 @@ PyObject* block_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// set_block_types(RMSNorm, GQA, MLP, PagedKV, {name: operator as defined})
+// set_block_types(RMSNorm, GQA, MLP, PagedKV, {class: what it defines}, {name: operator as defined})
 PyObject* set_block_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_ARGS(5);
-  if (!PyDict_Check(args[4])) return PyErr_Format(PyExc_TypeError, "set_block_types");
-  for (Py_ssize_t i = 0; i < 5; ++i) Py_INCREF(args[i]);  // for the life of the process
-  types.rms_norm = args[0], types.gqa = args[1], types.mlp = args[2], types.paged_kv = args[3], types.block_ops = args[4];
+  AQ_ARGS(6);
+  if (!PyDict_Check(args[4]) || !take_class(args[4], args[1], &types.gqa) || !take_class(args[4], args[2], &types.mlp) ||
+      !take_class(args[4], args[3], &types.paged_kv) || !PyDict_Check(args[5]))
+    return PyErr_Format(PyExc_TypeError, "set_block_types");
+  Py_INCREF(args[0]);  // for the life of the process
+  Py_INCREF(args[5]);
+  types.rms_norm = args[0], types.block_ops = args[5];
   Py_RETURN_NONE;
 }
 
@@ -955,7 +1001,8 @@ PyMODINIT_FUNC PyInit__host() {
               {&k_norm_quant, "_norm_quant"}, {&k_residual_adds, "_residual_adds"}, {&k_k_layers, "k_layers"},
               {&k_v_layers, "v_layers"},      {&k_page_table, "page_table"},    {&k_total_len, "total_len"},
               {&k_seq_lens, "seq_lens"},      {&k_invalid, "_invalid"},         {&k_page_size, "page_size"},
-              {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"}};
+              {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"},
+              {&k_forward_codes, "forward_codes"}, {&k_forward_attn, "forward_attn"}};
   for (const auto& k : keys)
     if (!(*k.key = PyUnicode_InternFromString(k.name))) return nullptr;
   return PyModule_Create(&module);

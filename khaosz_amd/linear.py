@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import logging
 import math
+from types import FunctionType
 from typing import Iterable, Optional, Sequence, Set, Tuple
 
 import torch
@@ -129,6 +130,16 @@ class _SharedInput:
 _told = False  # whether the native host path knows the layers
 
 
+def as_defined(*classes):
+    """What calls of these classes' instances go through, by name, as it is now.  Taken when the module is imported: while a
+    program has a method replaced on a class (to count calls, or to do something else), the native path stands aside."""
+    def of(cls):
+        names = [n for n, v in vars(cls).items() if isinstance(v, (FunctionType, property))] + ["__call__", "_call_impl", "_wrapped_call_impl"]
+        found = {n: vars(c)[n] for c in reversed(cls.__mro__) for n in names if n in vars(c)}  # the nearest class's last
+        return tuple((cls, n, v) for n, v in found.items()) + ((nn.Module, "__call__", vars(nn.Module)["__call__"]),)
+    return {cls: of(cls) for cls in classes}
+
+
 def linear_native():
     """The native host path, told about the layers' classes, the hooks that run for every module, and the operators as
     defined: while a program has one of those replaced (to count or trace calls), calls go through its replacement."""
@@ -136,7 +147,7 @@ def linear_native():
     h = ops._native()
     if not _told:
         m = torch.nn.modules.module
-        h.set_linear_types(QuantLinear, Fp8Linear, (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
+        h.set_linear_types(QuantLinear, Fp8Linear, _CLASSES, (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
                                                     m._global_backward_pre_hooks), ops.__dict__, _OPERATORS)
         h.serve_calls(_NativeCall.__call__)
         _told = True
@@ -374,6 +385,8 @@ class Fp8Linear(_NativeCall):
             y = ops.linear_fp8(xq, sx, wq, sw, bias, out_dtype=x.dtype, residual=residual)
         return y if x2 is x else y.view(x.shape[:-1] + (n,))
 
+
+_CLASSES = as_defined(QuantLinear, Fp8Linear)
 
 # Child names quantized by default: the projections of GQA (attention.py:57-67, `gate` is its optional output
 # gate), of MLA (attention.py:140-156: q_proj, kv_a_proj, kv_b_proj, o_proj, gate) and of every MLP, the experts of

@@ -7,8 +7,8 @@ import subprocess
 import pytest
 import torch
 
-from khaosz_amd import QuantLinear, _abi, fuse_shared_inputs, ops, quantize_model
-from khaosz_amd.block import DecoderBlock, PagedKV, rotary_table
+from khaosz_amd import Fp8Linear, QuantLinear, _abi, fuse_shared_inputs, ops, quantize_model
+from khaosz_amd.block import GQA, MLP, DecoderBlock, PagedKV, rotary_table
 
 pytestmark = pytest.mark.gpu
 DEV, DT = "cuda:0", torch.bfloat16
@@ -75,6 +75,48 @@ def test_hooks_on_a_fused_blocks_children_still_run():
         assert torch.equal(b(x, fr, None, cache), want) and len(seen) == 1
         h.remove()
         assert torch.equal(b(x, fr, None, cache), want) and len(seen) == 1
+
+
+def _counted(monkeypatch, owner, name):
+    """Replaces owner.name by a function that does the same; the list it returns grows by one a call."""
+    calls, real = [], getattr(owner, name)
+    monkeypatch.setattr(owner, name, lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    return calls
+
+
+@pytest.mark.parametrize("owner,name", [(QuantLinear, "forward"), (Fp8Linear, "forward"), (QuantLinear, "__call__"),
+                                        (torch.nn.Module, "__call__"), (torch.nn.Module, "_call_impl"), (QuantLinear, "_call_impl")])
+def test_a_method_replaced_on_a_layers_class_is_called(monkeypatch, owner, name):
+    base = torch.nn.Linear(256, 128).to(DEV).to(DT)
+    layer = (Fp8Linear if owner is Fp8Linear else QuantLinear).from_linear(base)
+    x = torch.randn(5, 256, device=DEV).to(DT)
+    with torch.inference_mode():
+        want = layer(x)
+        with monkeypatch.context() as m:
+            calls = _counted(m, owner, name)
+            assert torch.equal(layer(x), want) and len(calls) == 1
+        assert torch.equal(layer(x), want) and len(calls) == 1
+
+
+@pytest.mark.parametrize("S,owner,name", [(S, o, n) for S in (1, 40) for o, n in (
+    (GQA, "forward"), (MLP, "forward"), (QuantLinear, "forward"), (torch.nn.Module, "__call__"), (GQA, "_project_qkv"))] + [
+    (40, QuantLinear, "forward_codes"), (1, QuantLinear, "forward_attn"), (1, PagedKV, "attn_workspace"), (40, "down", "forward_codes"),
+    (1, "o_proj", "forward_attn"), (1, "attention", "forward")])
+def test_a_method_replaced_inside_a_fused_block_is_called(monkeypatch, S, owner, name):
+    """On a class, or (a text) on one of the block's own modules."""
+    b = _block()
+    x, fr, cache, table = _case(b, 2, S, 0 if S > 1 else 299)
+    cache.bind(table, S if S > 1 else 300)
+    if isinstance(owner, str):
+        owner = {"down": b.mlp.down, "o_proj": b.attention.o_proj, "attention": b.attention}[owner]
+    with torch.inference_mode():
+        want = b(x, fr, None, cache)
+        with monkeypatch.context() as m:
+            calls = _counted(m, owner, name)
+            assert torch.equal(b(x, fr, None, cache), want) and calls
+        n = len(calls)
+        assert torch.equal(b(x, fr, None, cache), want)
+        assert len(calls) == n
 
 
 @pytest.mark.parametrize("rows", [3, 40])

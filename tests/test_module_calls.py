@@ -48,3 +48,11 @@ def test_a_subclass_is_traced_by_fx_and_export(told):
     model = torch.nn.Sequential(q, torch.nn.ReLU())
     assert torch.equal(torch.fx.symbolic_trace(model)(x), model(x))
     assert torch.equal(torch.export.export(model, (x,)).module()(x), model(x))
+
+
+def test_a_forward_replaced_on_the_class_is_compiled_without_a_graph_break(monkeypatch, told):
+    q, x = _layer(QuantLinear)
+    monkeypatch.setattr(QuantLinear, "forward", _float_forward)
+    want = _float_forward(q, x)
+    torch._dynamo.reset()
+    assert torch.equal(q(x), want) and torch.equal(torch.compile(q, fullgraph=True, backend="eager")(x), want)
