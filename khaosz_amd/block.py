@@ -452,13 +452,15 @@ class DecoderBlock(nn.Module):
         return add(self.mlp(self.post_attention_norm(x), **kw(x)), x)
 
 
-# The operators a fused block's step consists of, as defined.  While a program has one of them replaced (to count or
+# The operators a fused block's step consists of, and the limits that choose among them, as defined.  While a program has one of them replaced (to count or
 # trace calls), blocks go operator by operator, through its replacement.
 _OPERATORS = {name: getattr(ops, name) for name in (
     "quant_rowwise_i8", "rmsnorm_quant_rowwise_i8", "swiglu_quant_rowwise_i8", "linear_w8a8", "gemv_w8a8_decode", "gemv_swiglu_ok",
     "gemv_w8a8_decode_swiglu", "gemv_w8a8_codes", "rope_kv_write", "attn_gemv_fusable", "rope_paged_attn_decode", "gemv_w8a8_attn",
-    "prefill_attn_causal", "prefill_attn_paged")}
+    "prefill_attn_causal", "prefill_attn_paged", "RMSNORM_QUANT_MAX_K", "SWIGLU_QUANT_MAX_F", "GEMV_ATTN_MAX_ROWS", "GEMV_ATTN_MAX_K",
+    "GEMV_ATTN_MAX_SLICES", "GEMV_ATTN_SLICE", "GEMV_ATTN_MAX_WORK")}
 _CLASSES = as_defined(GQA, MLP, PagedKV)
+_MERGE = (ops.GEMV_ATTN_MAX_ROWS, ops.GEMV_ATTN_MAX_K, ops.GEMV_ATTN_MAX_SLICES, ops.GEMV_ATTN_SLICE, ops.GEMV_ATTN_MAX_WORK)
 _host = None  # the native block step once it is loaded
 
 
@@ -466,7 +468,8 @@ def _native():
     global _host
     if _host is None:
         h = linear_native()
-        h.set_block_types(RMSNorm, GQA, MLP, PagedKV, _CLASSES, _OPERATORS)
+        h.set_block_types(RMSNorm, GQA, MLP, PagedKV, _CLASSES, _OPERATORS, _MERGE, _OPERATORS["RMSNORM_QUANT_MAX_K"],
+                          _OPERATORS["SWIGLU_QUANT_MAX_F"])
         _host = h.block_forward
     return _host
 

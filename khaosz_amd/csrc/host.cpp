@@ -18,10 +18,12 @@
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
+#include <initializer_list>
 
 #include "../../include/astrai_q.h"
 
@@ -400,7 +402,7 @@ PyObject *k_modules, *k_buffers, *k_parameters, *k_qweight, *k_w_scale, *k_bias,
     *k_fwd_pre_hooks, *k_compiled, *k_attention, *k_mlp, *k_input_norm, *k_post_norm, *k_qkv, *k_upgate, *k_o_proj, *k_down, *k_q_norm,
     *k_k_norm, *k_decode_attention, *k_use_qk_norm, *k_use_gate, *k_n_heads, *k_n_kv_heads, *k_head_dim, *k_layer_id, *k_swiglu_quant,
     *k_norm_quant, *k_residual_adds, *k_k_layers, *k_v_layers, *k_page_table, *k_total_len, *k_seq_lens, *k_invalid, *k_page_size,
-    *k_shared, *k_residual, *k_norm, *k_forward_codes, *k_forward_attn;
+    *k_shared, *k_residual, *k_norm, *k_decode_rows, *k_forward_codes, *k_forward_attn;
 
 PyObject* dict_of(PyObject* o) {  // borrowed; null if it has none
   PyObject** d = _PyObject_GetDictPtr(o);
@@ -465,16 +467,33 @@ struct Types {
   PyObject *linear_ops = nullptr, *block_ops = nullptr;
   uint64_t linear_ops_version = 0, block_ops_version = 0;  // of ops_dict when it last held them all
   PyObject* rms_norm = nullptr;
+  // Limits, as the Python side had them when it was imported.  A call goes the general way while one of them is another.
+  int64_t decode_rows = 0, fp8_decode_rows = 0, fp8_onepass_min_bytes = 0;
+  struct Merge {
+    int64_t rows, width, slices, slice, work;
+  } merge = {};
+  PyObject *norm_max_k = nullptr, *swiglu_max_f = nullptr;  // {dtype: limit}, read at each call
 } types;
+
+// whole numbers, all positive, from a tuple
+bool limits_of(PyObject* t, std::initializer_list<int64_t*> to) {
+  if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != static_cast<Py_ssize_t>(to.size())) return false;
+  Py_ssize_t i = 0;
+  for (int64_t* v : to) {
+    PyObject* o = PyTuple_GET_ITEM(t, i++);
+    if (!PyLong_CheckExact(o) || (*v = PyLong_AsLongLong(o)) < 1) return false;
+  }
+  return true;
+}
 
 bool exactly(PyObject* o, PyObject* type) { return o && reinterpret_cast<PyObject*>(Py_TYPE(o)) == type; }
 
 // A module whose forward may be replaced by what it is known to do: exactly the class, as it was defined, nothing hooked,
-// nothing wrapped.
+// nothing wrapped, no row limit of its own.
 bool ordinary(PyObject* m, Class& c) {
   if (!exactly(m, c.type) || !as_defined(c)) return false;
   PyObject* d = dict_of(m);
-  if (!d || PyDict_GetItem(d, k_forward)) return false;
+  if (!d || PyDict_GetItem(d, k_forward) || PyDict_GetItem(d, k_decode_rows)) return false;
   PyObject *h = get(d, k_fwd_hooks), *p = get(d, k_fwd_pre_hooks), *comp = get(d, k_compiled);
   return (!h || (PyDict_Check(h) && PyDict_GET_SIZE(h) == 0)) && (!p || (PyDict_Check(p) && PyDict_GET_SIZE(p) == 0)) &&
          (!comp || comp == Py_None);
@@ -545,9 +564,6 @@ bool gain_of(PyObject* m, int64_t K, int dev, Gain* g) {
   return true;
 }
 
-constexpr int64_t DECODE_ROWS = 16;                  // QuantLinear.DECODE_MAX_ROWS, Fp8Linear.DECODE_MAX_ROWS
-constexpr int64_t FP8_ONEPASS_MIN_BYTES = 16 << 20;  // ops.FP8_ONEPASS_MIN_BYTES
-
 // What calling the QuantLinear or Fp8Linear gives, or None where nn.Module's own call has to serve: hooks, a shared input, FP8
 // inputs that are quantised in one launch with a state the module keeps.
 PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs, PyObject* names) {
@@ -590,20 +606,21 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
     eps = static_cast<float>(PyFloat_AS_DOUBLE(PyTuple_GET_ITEM(norm, 1)));
   }
   const int64_t x_bytes = x->numel() * x->element_size();
-  if (fp8 && r.M > DECODE_ROWS && x_bytes >= FP8_ONEPASS_MIN_BYTES) return none();
+  const bool few = r.M <= (fp8 ? types.fp8_decode_rows : types.decode_rows);
+  if (fp8 && !few && x_bytes >= types.fp8_onepass_min_bytes) return none();
   c.current_stream();
   c10::DimVector shape(x->sizes());
   shape.back() = N;
   Tensor y = c.empty(shape, type);
   // codes and scales of the tokens (and, for FP8, the partial maxima)
-  const int64_t codes = r.M > DECODE_ROWS ? (r.M * r.K + 255) & ~int64_t(255)
-                        : fp8             ? static_cast<int64_t>(lib.aq_gemv_fp8_workspace_bytes(r.M, r.K))
-                                          : static_cast<int64_t>(lib.aq_gemv_w8a8_workspace_bytes(r.M, r.K));
-  const int64_t room = codes + (r.M > DECODE_ROWS ? (fp8 ? 256 + AQ_FP8_AMAX_WS_BYTES : 4 * r.M) : 0);
+  const int64_t codes = !few  ? (r.M * r.K + 255) & ~int64_t(255)
+                        : fp8 ? static_cast<int64_t>(lib.aq_gemv_fp8_workspace_bytes(r.M, r.K))
+                              : static_cast<int64_t>(lib.aq_gemv_w8a8_workspace_bytes(r.M, r.K));
+  const int64_t room = codes + (!few ? (fp8 ? 256 + AQ_FP8_AMAX_WS_BYTES : 4 * r.M) : 0);
   void* yp = y.mutable_data_ptr();
   // a launch that quantises its rows itself touches no workspace: an allocation is 0.4 us of a 5 us call
-  const bool alone = r.M <= DECODE_ROWS && (fp8 ? lib.aq_gemv_fp8_decode_one_launch(r.code, r.M, r.K)
-                                                : lib.aq_gemv_w8a8_decode_one_launch(r.code, gain != nullptr, r.M, N, r.K));
+  const bool alone = few && (fp8 ? lib.aq_gemv_fp8_decode_one_launch(r.code, r.M, r.K)
+                                 : lib.aq_gemv_w8a8_decode_one_launch(r.code, gain != nullptr, r.M, N, r.K));
   Tensor ws;
   if (!alone) ws = c.empty({room}, ScalarType::Byte);
   char* base = static_cast<char*>(alone ? yp : ws.mutable_data_ptr());
@@ -612,7 +629,7 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   const auto* sp = static_cast<const float*>(s->const_data_ptr());
   const char* what = "";
   const int rc = queued([&]() -> int {
-    if (r.M <= DECODE_ROWS) {
+    if (few) {
       what = fp8 ? "aq_gemv_fp8_decode" : "aq_gemv_w8a8_decode";
       if (fp8)
         return lib.aq_gemv_fp8_decode_residual(r.p, r.code, static_cast<const uint8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K,
@@ -667,11 +684,13 @@ PyObject* serve_calls(PyObject*, PyObject* function) {
   Py_RETURN_NONE;
 }
 
-// set_linear_types(QuantLinear, Fp8Linear, {class: what it defines}, hook dicts, ops.__dict__, {name: operator as defined})
+// set_linear_types(QuantLinear, Fp8Linear, {class: what it defines}, hook dicts, ops.__dict__, {name: operator or limit as defined},
+//                  (row limit, row limit, bytes from which FP8 inputs are quantised in one launch))
 PyObject* set_linear_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_ARGS(6);
+  AQ_ARGS(7);
   if (!PyDict_Check(args[2]) || !take_class(args[2], args[0], &types.quant_linear) || !take_class(args[2], args[1], &types.fp8_linear) ||
-      !PyTuple_Check(args[3]) || !PyDict_Check(args[4]) || !PyDict_Check(args[5]))
+      !PyTuple_Check(args[3]) || !PyDict_Check(args[4]) || !PyDict_Check(args[5]) ||
+      !limits_of(args[6], {&types.decode_rows, &types.fp8_decode_rows, &types.fp8_onepass_min_bytes}))
     return PyErr_Format(PyExc_TypeError, "set_linear_types");
   for (Py_ssize_t i = 3; i < 6; ++i) Py_INCREF(args[i]);  // for the life of the process
   types.global_hooks = args[3], types.ops_dict = args[4], types.linear_ops = args[5];
@@ -690,16 +709,27 @@ struct Scratch {
   }
 };
 
-// Limits of the output projection that merges attention slices itself, and the rule when that pays (ops.py,
-// attn_gemv_fusable: every workgroup repeats the merge of all rows).
-constexpr int64_t ATTN_MAX_ROWS = 8, SLICE = 256;
+// ops.attn_gemv_fusable: whether the output projection merges the attention's slices itself
 bool merge_in_projection(int64_t B, int64_t width, int64_t total) {
-  if (B > ATTN_MAX_ROWS || width > AQ_GEMV_ATTN_MAX_K || total <= SLICE || total > AQ_GEMV_ATTN_MAX_SLICES * SLICE) return false;
-  return B * width * ((total + SLICE - 1) / SLICE) <= 32768;
+  const Types::Merge& m = types.merge;
+  if (B < 1 || B > m.rows || width > m.width || total <= m.slice || total > m.slices * m.slice) return false;
+  return B * width * ((total + m.slice - 1) / m.slice) <= m.work;
 }
 
-constexpr int64_t NORM_MAX_K = 12288;   // ops.RMSNORM_QUANT_MAX_K, bf16
-constexpr int64_t SWIGLU_MAX_F = 8192;  // ops.SWIGLU_QUANT_MAX_F, bf16
+// attn_gemv_fusable(B, width, total) -> bool, for comparison with the operator's rule
+PyObject* attn_gemv_fusable(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  AQ_ARGS(3);
+  int64_t v[3];
+  for (int i = 0; i < 3; ++i)
+    if ((v[i] = PyLong_AsLongLong(args[i])) == -1 && PyErr_Occurred()) return nullptr;
+  return PyBool_FromLong(types.block_ops && merge_in_projection(v[0], v[1], v[2]));
+}
+
+// an operator's limit for bf16 rows: its entry in {dtype: limit}
+int64_t limit_of(PyObject* by_type) {
+  PyObject* v = get(by_type, reinterpret_cast<PyObject*>(torch::getTHPDtype(ScalarType::BFloat16)));
+  return v && PyLong_CheckExact(v) ? PyLong_AsLongLong(v) : 0;
+}
 
 // A DecoderBlock with every fusion on (fuse_shared_inputs(norms, decode_attention, residuals)), applied to bf16 tokens over
 // a paged cache: what it works on, read and checked under the interpreter lock.
@@ -722,7 +752,7 @@ struct Block {
 
   bool read(PyObject* block, PyObject* x, PyObject* rotary, PyObject* cache);
   void lay_out();
-  bool few() const { return M <= DECODE_ROWS; }
+  bool few() const { return M <= types.decode_rows; }
   bool step() const { return S == 1; }
   bool merge() const { return step() && merge_in_projection(B, Hq * D, total); }
   int queue(const void* in, void* out, char* base, const char** what) const;  // allocates nothing: runs without the interpreter lock
@@ -733,7 +763,7 @@ bool Block::read(PyObject* block, PyObject* px, PyObject* protary, PyObject* cac
   const Tensor *x = unpack(px), *rot = unpack(protary);
   if (!x || !rot || !c.at(*x) || !plain(*x, ScalarType::BFloat16, c.dev) || x->dim() != 3) return false;
   B = x->size(0), S = x->size(1), dim = x->size(2), M = B * S;
-  if (M < 1 || dim > NORM_MAX_K || !aligned16(x->const_data_ptr()) || x->requires_grad()) return false;
+  if (M < 1 || dim > limit_of(types.norm_max_k) || !aligned16(x->const_data_ptr()) || x->requires_grad()) return false;
   hold_x = *x;
   // the modules
   PyObject* d = dict_of(block);
@@ -755,7 +785,7 @@ bool Block::read(PyObject* block, PyObject* px, PyObject* protary, PyObject* cac
     return false;
   F = ug.N / 2;
   if (qkv.K != dim || qkv.N != (Hq + 2 * Hkv) * D || o.K != Hq * D || o.N != dim || ug.K != dim || ug.N % 2 || F % 16 ||
-      F > SWIGLU_MAX_F || down.K != F || down.N != dim)
+      F > limit_of(types.swiglu_max_f) || down.K != F || down.N != dim)
     return false;
   // the cache
   if (!exactly(cache, types.paged_kv.type) || !as_defined(types.paged_kv)) return false;
@@ -936,15 +966,16 @@ PyObject* block_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// set_block_types(RMSNorm, GQA, MLP, PagedKV, {class: what it defines}, {name: operator as defined})
+// set_block_types(RMSNorm, GQA, MLP, PagedKV, {class: what it defines}, {name: operator or limit as defined}, (limits of
+//                 attn_gemv_fusable), {dtype: longest row the norm takes}, {dtype: longest row the activation takes})
 PyObject* set_block_types(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  AQ_ARGS(6);
+  AQ_ARGS(9);
   if (!PyDict_Check(args[4]) || !take_class(args[4], args[1], &types.gqa) || !take_class(args[4], args[2], &types.mlp) ||
-      !take_class(args[4], args[3], &types.paged_kv) || !PyDict_Check(args[5]))
+      !take_class(args[4], args[3], &types.paged_kv) || !PyDict_Check(args[5]) || !PyDict_Check(args[7]) || !PyDict_Check(args[8]) ||
+      !limits_of(args[6], {&types.merge.rows, &types.merge.width, &types.merge.slices, &types.merge.slice, &types.merge.work}))
     return PyErr_Format(PyExc_TypeError, "set_block_types");
-  Py_INCREF(args[0]);  // for the life of the process
-  Py_INCREF(args[5]);
-  types.rms_norm = args[0], types.block_ops = args[5];
+  for (int i : {0, 5, 7, 8}) Py_INCREF(args[i]);  // for the life of the process
+  types.rms_norm = args[0], types.block_ops = args[5], types.norm_max_k = args[7], types.swiglu_max_f = args[8];
   Py_RETURN_NONE;
 }
 
@@ -967,6 +998,7 @@ PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
     AQ_METHOD(set_linear_types),
     AQ_METHOD(set_block_types),
+    AQ_METHOD(attn_gemv_fusable),
     {"serve_calls", serve_calls, METH_O, nullptr},
     AQ_METHOD(quant_rowwise_i8),
     AQ_METHOD(rmsnorm_quant_rowwise_i8),
@@ -1002,6 +1034,7 @@ PyMODINIT_FUNC PyInit__host() {
               {&k_v_layers, "v_layers"},      {&k_page_table, "page_table"},    {&k_total_len, "total_len"},
               {&k_seq_lens, "seq_lens"},      {&k_invalid, "_invalid"},         {&k_page_size, "page_size"},
               {&k_shared, "_shared"},         {&k_residual, "residual"},        {&k_norm, "norm"},
+              {&k_decode_rows, "DECODE_MAX_ROWS"},
               {&k_forward_codes, "forward_codes"}, {&k_forward_attn, "forward_attn"}};
   for (const auto& k : keys)
     if (!(*k.key = PyUnicode_InternFromString(k.name))) return nullptr;

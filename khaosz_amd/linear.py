@@ -14,7 +14,6 @@ from __future__ import annotations
 
 import logging
 import math
-from types import FunctionType
 from typing import Iterable, Optional, Sequence, Set, Tuple
 
 import torch
@@ -131,10 +130,10 @@ _told = False  # whether the native host path knows the layers
 
 
 def as_defined(*classes):
-    """What calls of these classes' instances go through, by name, as it is now.  Taken when the module is imported: while a
-    program has a method replaced on a class (to count calls, or to do something else), the native path stands aside."""
+    """What calls of these classes' instances go through, by name, as it is now: methods and limits.  Taken when the module is
+    imported: while a program has one of them replaced on a class, the native path stands aside."""
     def of(cls):
-        names = [n for n, v in vars(cls).items() if isinstance(v, (FunctionType, property))] + ["__call__", "_call_impl", "_wrapped_call_impl"]
+        names = [n for n in vars(cls) if not n.startswith("__")] + ["__call__", "_call_impl", "_wrapped_call_impl"]
         found = {n: vars(c)[n] for c in reversed(cls.__mro__) for n in names if n in vars(c)}  # the nearest class's last
         return tuple((cls, n, v) for n, v in found.items()) + ((nn.Module, "__call__", vars(nn.Module)["__call__"]),)
     return {cls: of(cls) for cls in classes}
@@ -148,7 +147,7 @@ def linear_native():
     if not _told:
         m = torch.nn.modules.module
         h.set_linear_types(QuantLinear, Fp8Linear, _CLASSES, (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
-                                                    m._global_backward_pre_hooks), ops.__dict__, _OPERATORS)
+                                                    m._global_backward_pre_hooks), ops.__dict__, _OPERATORS, _LIMITS)
         h.serve_calls(_NativeCall.__call__)
         _told = True
     return h
@@ -156,7 +155,7 @@ def linear_native():
 
 _OPERATORS = {name: getattr(ops, name) for name in (
     "quant_rowwise_i8", "rmsnorm_quant_rowwise_i8", "linear_w8a8", "gemv_w8a8_decode", "quant_tensor_fp8", "linear_fp8",
-    "gemv_fp8_decode")}
+    "gemv_fp8_decode", "FP8_ONEPASS_MIN_BYTES")}
 
 
 class _NativeCall(Linear):
@@ -387,6 +386,7 @@ class Fp8Linear(_NativeCall):
 
 
 _CLASSES = as_defined(QuantLinear, Fp8Linear)
+_LIMITS = QuantLinear.DECODE_MAX_ROWS, Fp8Linear.DECODE_MAX_ROWS, ops.FP8_ONEPASS_MIN_BYTES
 
 # Child names quantized by default: the projections of GQA (attention.py:57-67, `gate` is its optional output
 # gate), of MLA (attention.py:140-156: q_proj, kv_a_proj, kv_b_proj, o_proj, gate) and of every MLP, the experts of

@@ -3,6 +3,7 @@ the way of hooks and replaced operators, and operators fed with what the native 
 import ctypes
 import pathlib
 import subprocess
+import sys
 
 import pytest
 import torch
@@ -117,6 +118,65 @@ def test_a_method_replaced_inside_a_fused_block_is_called(monkeypatch, S, owner,
         n = len(calls)
         assert torch.equal(b(x, fr, None, cache), want)
         assert len(calls) == n
+
+
+def _frames(f):
+    """f() and the names of the Python functions that it ran (the native path runs none)."""
+    seen = []
+    sys.setprofile(lambda frame, event, arg: seen.append(frame.f_code.co_name) if event == "call" else None)
+    try:
+        y = f()
+    finally:
+        sys.setprofile(None)
+    return y, seen
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("own", [False, True], ids=["of the class", "of the layer"])
+def test_a_changed_row_limit_decides(monkeypatch, fp8, own):
+    cls, gemm = (Fp8Linear, "linear_fp8") if fp8 else (QuantLinear, "linear_w8a8")
+    layer = cls.from_linear(torch.nn.Linear(256, 128).to(DEV).to(DT))
+    x = torch.randn(5, 256, device=DEV).to(DT)
+    with torch.inference_mode():
+        layer(x)
+        assert gemm not in _frames(lambda: layer(x))[1]
+        monkeypatch.setattr(layer if own else cls, "DECODE_MAX_ROWS", 4)
+        y, seen = _frames(lambda: layer(x))
+        assert gemm in seen and torch.equal(y, layer.forward(x))
+
+
+def test_a_changed_size_for_the_one_launch_quantiser_decides(monkeypatch):
+    layer = Fp8Linear.from_linear(torch.nn.Linear(256, 128).to(DEV).to(DT))
+    x = torch.randn(40, 256, device=DEV).to(DT)
+    with torch.inference_mode():
+        want = layer(x)
+        assert len(layer._quant_states) == 0
+        monkeypatch.setattr(ops, "FP8_ONEPASS_MIN_BYTES", 0)
+        assert torch.equal(layer(x), want) and len(layer._quant_states) == 1
+
+
+@pytest.mark.parametrize("S,limit,value,function", [
+    (40, "RMSNORM_QUANT_MAX_K", 256, "rmsnorm_quant_rowwise_i8"), (40, "SWIGLU_QUANT_MAX_F", 1024, "swiglu_quant_rowwise_i8"),
+    (1, "GEMV_ATTN_MAX_ROWS", 1, "forward_attn"), (1, "GEMV_ATTN_MAX_K", 256, "forward_attn"),
+    (1, "GEMV_ATTN_MAX_SLICES", 1, "forward_attn"), (1, "GEMV_ATTN_MAX_WORK", 100, "forward_attn")])
+def test_a_changed_limit_of_an_operator_decides_in_a_fused_block(monkeypatch, S, limit, value, function):
+    b = _block()
+    x, fr, cache, table = _case(b, 2, S, 0 if S > 1 else 299)
+    cache.bind(table, S if S > 1 else 300)
+    step = lambda: b(x, fr, None, cache)
+    monkeypatch.setattr(ops, "quant_tensor_fp8", None)  # no block uses it; layers by themselves go through their forward now
+    with torch.inference_mode():
+        step()
+        assert "_project_qkv" not in _frames(step)[1]
+        with monkeypatch.context() as m:
+            m.setattr(ops, "gemv_swiglu_ok", lambda x, f: False)  # a replaced operator: the step-by-step path
+            assert function in _frames(step)[1]
+        if isinstance(getattr(ops, limit), dict):
+            monkeypatch.setitem(getattr(ops, limit), DT, value)
+        else:
+            monkeypatch.setattr(ops, limit, value)
+        seen = _frames(step)[1]
+        assert "_project_qkv" in seen and function not in seen
 
 
 @pytest.mark.parametrize("rows", [3, 40])

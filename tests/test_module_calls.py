@@ -56,3 +56,13 @@ def test_a_forward_replaced_on_the_class_is_compiled_without_a_graph_break(monke
     want = _float_forward(q, x)
     torch._dynamo.reset()
     assert torch.equal(q(x), want) and torch.equal(torch.compile(q, fullgraph=True, backend="eager")(x), want)
+
+
+def test_the_native_rule_for_the_merge_inside_the_projection_is_the_operators():
+    from khaosz_amd import block, ops
+    block._native()
+    host = ops._native()
+    for B in range(0, 12):
+        for heads, d in ((1, 64), (8, 64), (24, 64), (31, 64), (32, 64), (16, 128), (17, 128), (33, 64)):
+            for total in (1, 255, 256, 257, 512, 513, 768, 769, 1024, 1025, 5000):
+                assert host.attn_gemv_fusable(B, heads * d, total) == ops.attn_gemv_fusable(B, heads, d, total)
