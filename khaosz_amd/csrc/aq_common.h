@@ -393,19 +393,25 @@ inline void queue_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds
   }(args...);
 }
 
-// Compute units of the current device, asked of the runtime once per device (launch shapes are
-// sized by it: a partition mode that exposes fewer compute units per device gets fewer workgroups).
+// A count that depends on the current device alone, asked of the runtime once per device.
 // The cache is written with the same value by whichever thread comes first: a benign race.
-inline int device_cus() {
-  static int cached[64] = {};
+template <class F>
+inline int per_device(int (&cached)[64], int otherwise, F&& ask) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return otherwise;
   int v = cached[dev];
   if (v <= 0) {
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
+    if (ask(&v, dev) != hipSuccess || v <= 0) v = otherwise;
     cached[dev] = v;
   }
   return v;
+}
+
+// Compute units of the current device (launch shapes are sized by it: a partition mode that exposes fewer compute units
+// per device gets fewer workgroups).
+inline int device_cus() {
+  static int cached[64] = {};
+  return per_device(cached, 256, [](int* v, int dev) { return hipDeviceGetAttribute(v, hipDeviceAttributeMultiprocessorCount, dev); });
 }
 
 }  // namespace aq

@@ -406,22 +406,33 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
   }
 }
 
-constexpr int PA_TABLE_MAX = 2048;  // page-table entries kept in LDS
+constexpr int PA_TABLE_MAX = 2048;                         // page-table entries kept in LDS
+constexpr int LDS_BYTES = 160 * 1024, STATIC_LDS = 1536;  // of a compute unit; of a workgroup beside its buffers, at most
 
 template <int D, int QW, int KW, bool PAGED>
 static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
   const int64_t wgs = ((int64_t)(a.S + 32 * QW - 1) / (32 * QW)) * a.Hq * a.B;
   a.wgs = (int)wgs;
-  if (wgs + AHEAD_WGS > 2 * device_cus()) a.ahead_wgs = 0;  // no room beside the workgroups that attend: they would run behind them
   constexpr int KB = 64, BUFS = 2 * KW * 2 * KB * 2 * D;
-  a.paired = wgs <= (160 * 1024 / BUFS) * (int64_t)device_cus();
   size_t lds = BUFS;
   if constexpr (PAGED) {
     const int64_t entries = ((int64_t)a.start + a.S + a.page - 1) / a.page;
     a.table_lds = a.page % KB != 0 && entries <= PA_TABLE_MAX ? (int)entries : 0;
     lds += (size_t)a.table_lds * sizeof(int);
   }
-  aq::queue_kernel((prefill_attn_kernel<D, QW, KW, PAGED>), dim3((unsigned)(wgs + a.ahead_wgs)), dim3(QW * KW * 64), lds, st, a);
+  constexpr auto kernel = prefill_attn_kernel<D, QW, KW, PAGED>;
+  // Workgroups that the device holds at once.  Registers decide at head dimension 64 with one wavefront per query row (124
+  // and 128 of them: four, where the buffers would allow five), the buffers elsewhere; a page table in LDS may cost another.
+  // Launches of four to five workgroups per compute unit, numbered as if resident -> heaviest first, us: 4 x 1408 x 24 heads
+  // 42.8 -> 41.2, 4 x 1536 46.0 -> 44.3, 1 x 6400 186 -> 164, 10 x 600 27.8 -> 26.3, 10 x 512 x 32 26.8 -> 25.9; 12 x 512 x 24
+  // the other way, 23.7 -> 24.8.
+  static int cached[64] = {};
+  int per_cu = per_device(cached, 1, [&](int* v, int) { return hipOccupancyMaxActiveBlocksPerMultiprocessor(v, kernel, QW * KW * 64, BUFS); });
+  if (lds > BUFS && per_cu > LDS_BYTES / (int)(lds + STATIC_LDS)) per_cu = LDS_BYTES / (int)(lds + STATIC_LDS);
+  const int64_t room = (int64_t)per_cu * device_cus();
+  a.paired = wgs <= room;
+  if (wgs + AHEAD_WGS > 2 * device_cus()) a.ahead_wgs = 0;  // no room beside the workgroups that attend: they would run behind them
+  aq::queue_kernel(kernel, dim3((unsigned)(wgs + a.ahead_wgs)), dim3(QW * KW * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 

@@ -502,6 +502,18 @@ def test_prefill_attn_by_wavefronts_per_query_row(oracle, B, S, start, Hq, Hkv, 
         assert torch.equal(out, ops.prefill_attn_causal(q.to(DEV), k.to(DEV), v.to(DEV)).cpu().float())
 
 
+@pytest.mark.parametrize("B,S,Hq,D", [(7, 384, 48, 64), (9, 512, 32, 64), (10, 500, 32, 64), (11, 512, 32, 64), (5, 640, 24, 128)])
+def test_prefill_attn_numbering_of_workgroups(B, S, Hq, D):
+    """Launches around what the device holds at once (1024 workgroups of head dimension 64, 512 of 128): 1008, 1152, 1280, 1408
+    and 600 of them give what each sequence gives by itself, whichever order they run in."""
+    _say("prefill_attn numbering", B, S, Hq, D)
+    g = torch.Generator(device=DEV).manual_seed(B)
+    q, k, v = (torch.randn(B, S, h, D, generator=g, device=DEV, dtype=torch.bfloat16) for h in (Hq, Hq // 4, Hq // 4))
+    out = ops.prefill_attn_causal(q, k, v)
+    for b in range(B):
+        assert torch.equal(out[b], ops.prefill_attn_causal(q[b:b + 1], k[b:b + 1], v[b:b + 1])[0])
+
+
 def test_prefill_attn_reading_ahead_changes_nothing():
     """Spans that the attention launch reads ahead: none, ragged ends, more than it takes, a launch without room."""
     import ctypes
