@@ -425,13 +425,17 @@ static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
   // and 128 of them: four, where the buffers would allow five), the buffers elsewhere; a page table in LDS may cost another.
   // Launches of four to five workgroups per compute unit, numbered as if resident -> heaviest first, us: 4 x 1408 x 24 heads
   // 42.8 -> 41.2, 4 x 1536 46.0 -> 44.3, 1 x 6400 186 -> 164, 10 x 600 27.8 -> 26.3, 10 x 512 x 32 26.8 -> 25.9; 12 x 512 x 24
-  // the other way, 23.7 -> 24.8.
+  // and 9 x 512 x 32 the other way, 23.7 -> 24.8 and 23.4 -> 24.6.
   static int cached[64] = {};
   int per_cu = per_device(cached, 1, [&](int* v, int) { return hipOccupancyMaxActiveBlocksPerMultiprocessor(v, kernel, QW * KW * 64, BUFS); });
   if (lds > BUFS && per_cu > LDS_BYTES / (int)(lds + STATIC_LDS)) per_cu = LDS_BYTES / (int)(lds + STATIC_LDS);
   const int64_t room = (int64_t)per_cu * device_cus();
   a.paired = wgs <= room;
-  if (wgs + AHEAD_WGS > 2 * device_cus()) a.ahead_wgs = 0;  // no room beside the workgroups that attend: they would run behind them
+  // No reading ahead without room beside the workgroups that attend: it would run behind them.  24-layer model, 1536 wide, ms,
+  // room for two workgroups per compute unit in all kernels -> for as many as fit: 8 x 512 tokens 6.37 -> 6.10, 6 x 512
+  // 5.23 -> 4.97, 5 x 512 4.64 -> 4.30, 9 x 384 5.49 -> 5.31; and no longer beside one that fills its compute unit: 1 x 300
+  // 1.70 -> 1.67, 300 on 700 cached 1.83 -> 1.81, 2 x 128 1.53 -> 1.55.
+  if (wgs + AHEAD_WGS > room) a.ahead_wgs = 0;
   aq::queue_kernel(kernel, dim3((unsigned)(wgs + a.ahead_wgs)), dim3(QW * KW * 64), lds, st, a);
   return (int)hipGetLastError();
 }

@@ -521,7 +521,7 @@ def test_prefill_attn_reading_ahead_changes_nothing():
     g = torch.Generator().manual_seed(5)
     weights = [torch.zeros(n, dtype=torch.int8, device=DEV) for n in (3, 128, 1000, 300000)]
     over = torch.zeros(97 << 20, dtype=torch.int8, device=DEV)
-    for B, S, Hq, Hkv in ((2, 70, 4, 2), (4, 512, 40, 8)):
+    for B, S, Hq, Hkv in ((2, 70, 4, 2), (4, 512, 40, 8), (7, 512, 32, 8), (9, 512, 32, 8)):  # the last: no room
         q, k, v = (torch.randn(B, S, h * 64, generator=g).to(torch.bfloat16).to(DEV) for h in (Hq, Hkv, Hkv))
         want = ops.prefill_attn_causal(q.view(B, S, Hq, 64), k.view(B, S, Hkv, 64), v.view(B, S, Hkv, 64))
         for chosen in ((), weights[:3], weights[1:], weights[3:], [over]):
