@@ -366,6 +366,15 @@ __device__ __forceinline__ void read_ahead(const Ahead& a, int wg, int nthreads)
   }
   asm volatile("" ::"v"(seen));  // the loads are wanted, their values are not
 }
+inline int check_spans(const aq_span* spans, int n) {
+  if (n < 0 || (n > 0 && !spans)) return AQ_E_NULL;
+  for (int i = 0; i < n; ++i) {
+    if (spans[i].bytes < 0) return AQ_E_SHAPE;
+    if (spans[i].bytes > 0 && !spans[i].ptr) return AQ_E_NULL;
+    if (check_ptr(spans[i].ptr, 4)) return AQ_E_ALIGN;
+  }
+  return AQ_OK;
+}
 // Up to AHEAD_SPANS ranges; whole lines inside each (the last dword read lies in the range).  Over AHEAD_MOST bytes in all
 // nothing is read: too much to wait in the cache until its launch comes.  Returns the workgroups to add.
 constexpr int64_t AHEAD_MOST = 96 << 20;

@@ -478,7 +478,7 @@ extern "C" int aq_prefill_attn_causal_ahead(const void* q, int64_t q_stride, con
   // 32-bit byte offsets inside one sequence's K and V (a key block past the end included)
   if ((S + 64) * k_stride * 2 > (int64_t)0x7fffffff || (S + 64) * v_stride * 2 > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
-  if (n_ahead < 0 || (n_ahead > 0 && !ahead)) return AQ_E_NULL;
+  if (const int rc = aq::check_spans(ahead, n_ahead)) return rc;
   aq::PrefillAttnArgs a{};
   a.ahead_wgs = aq::set_ahead(a.ahead, ahead, n_ahead);
   a.q = static_cast<const uint16_t*>(q);
@@ -520,7 +520,7 @@ extern "C" int aq_prefill_attn_paged_ahead(const void* q, int64_t q_stride, cons
   if (start + S > (1 << 30) || Hq > 65535 || B > 65535 ||
       ((S + 31) / 32) * Hq * B > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
-  if (n_ahead < 0 || (n_ahead > 0 && !ahead)) return AQ_E_NULL;
+  if (const int rc = aq::check_spans(ahead, n_ahead)) return rc;
   aq::PrefillAttnArgs a{};
   a.ahead_wgs = aq::set_ahead(a.ahead, ahead, n_ahead);
   a.q = static_cast<const uint16_t*>(q);

@@ -2,6 +2,7 @@
 declares, rejects bad arguments before touching a GPU, and the host module keeps
 the reference's Linear surface (astrai/model/components/linear.py:7-21) and swap
 invariants (tests/module/test_lora.py in the reference)."""
+import ctypes
 import os
 import re
 
@@ -39,6 +40,15 @@ def test_lab_library_holds_the_product_and_the_lab_symbols():
     for name in _abi.SYMBOLS:
         assert hasattr(lab, name), name
     assert lab.aq_lab_set_gemm_tile(3) == -2 and lab.aq_lab_set_gemm_tile(0) == 0
+
+
+@pytest.mark.parametrize("ptr,nbytes,code", [(1 << 20, -128, -2), (0, 128, -1), ((1 << 20) + 2, 128, -4)])
+def test_ranges_to_read_ahead_are_checked(ptr, nbytes, code):
+    lib, P = _abi.load(), 1 << 20  # a fake pointer; refused before any launch
+    good = [1 << 20, 1 << 10]
+    spans = (ctypes.c_int64 * 4)(*good, ptr, nbytes)
+    assert lib.aq_prefill_attn_causal_ahead(P, 64, P, 64, P, 64, P, 0.1, 1, 1, 1, 1, 64, ctypes.addressof(spans), 2, None) == code
+    assert lib.aq_prefill_attn_paged_ahead(P, 64, P, P, P, 1, 0, 16, 1, P, 0.1, 1, 1, 1, 1, 64, ctypes.addressof(spans), 2, None) == code
 
 
 def test_argument_validation_happens_before_any_launch():
