@@ -399,12 +399,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
 // byte offsets; the negative gates' entries then lie 128 KiB further up and the table spans a compute unit's LDS: one
 // workgroup each, a wavefront per row, rows dealt out over the compute units first.  Filling it takes 1.5 us of
 // arithmetic, most of it while the first rows are on their way.
+//
+// A lane holds 8 NC values of h and 8 NC of the row in flight.  Up to 11 pairs fit the 128 registers that sixteen wavefronts
+// leave each, longer rows get twelve wavefronts of 168.  (Twelve pairs on sixteen wavefronts spill 5 registers: 4096 x 6144
+// 24.6 us against 23.5, 4096 x 5648 23.5 against 22.7, 1100 x 6144 9.3 against 9.1.)
 constexpr uint32_t LUT_LOW = 96u << 7, LUT_SIZE = 38u << 7;
+constexpr int lut_waves(int nc) { return nc <= 11 ? 16 : 12; }
 template <int NC>
-__global__ __launch_bounds__(NC <= 12 ? 1024 : 768) void swiglu_quant_lut_kernel(const void* __restrict__ ug, int64_t M, int F,
+__global__ __launch_bounds__(lut_waves(NC) * 64) void swiglu_quant_lut_kernel(const void* __restrict__ ug, int64_t M, int F,
                                                                                 int64_t ld, int8_t* __restrict__ q,
                                                                                 float* __restrict__ scale) {
-  constexpr int NW = NC <= 12 ? 16 : 12;  // 128 or 168 registers a wavefront: a row's h is 8 NC of them
+  constexpr int NW = lut_waves(NC);
   __shared__ __attribute__((aligned(16))) float table[0x8000 + LUT_SIZE];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -908,17 +913,17 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
                                hipStream_t st) {
   const int64_t vpl = (F / (BF16 ? 8 : 4) + 63) / 64;  // vector pairs per lane
   if (vpl > 16) return AQ_E_RANGE;
-  // many bf16 rows: the kernel that looks silu up.  Up to 1024 rows (1280 of more than 12 pairs per lane, twelve wavefronts
-  // to a compute unit) its table costs more than it saves: 1024 x 4096 6.8 us against 6.2 with a workgroup per row,
-  // 1100 x 6912 12.6 against 12.1; from there on us, before -> now: 1100 x 5632 14.7 -> 10.1, 2048 x 6912 20.0 -> 16.5,
-  // 4096 x 5632 28.5 -> 23.5, 4096 x 6912 38 -> 28, 8192 x 8192 89 -> 72, 2048 x 2048 6.5 -> 6.3 (shorter rows stay).
+  // many bf16 rows: the kernel that looks silu up.  Up to 1024 rows (1280 of more than 12 pairs per lane) its table costs
+  // more than it saves: 1024 x 4096 6.8 us against 6.2 with a workgroup per row, 1100 x 6912 12.6 against 12.1; from there on
+  // us, before -> now: 1100 x 5632 14.7 -> 10.1, 2048 x 6912 20.0 -> 16.5, 4096 x 5632 28.5 -> 23.5, 4096 x 6912 38 -> 28,
+  // 8192 x 8192 89 -> 72, 2048 x 2048 6.5 -> 6.3 (shorter rows stay).
   if constexpr (BF16) {
     if (vpl >= 4 && vpl <= 16 && M > (vpl > 12 ? 1280 : 1024)) {
       const dim3 g((unsigned)aq::device_cus());
       switch (vpl) {
 #define AQ_SWIGLU_CASE(nc)                                                                                                      \
   case nc:                                                                                                                      \
-    aq::queue_kernel((aq::swiglu_quant_lut_kernel<nc>), g, dim3(nc <= 12 ? 1024 : 768), 0, st, ug, M, (int)F, ld, q, scale); \
+    aq::queue_kernel((aq::swiglu_quant_lut_kernel<nc>), g, dim3(aq::lut_waves(nc) * 64), 0, st, ug, M, (int)F, ld, q, scale); \
     break;
         AQ_SWIGLU_CASE(4) AQ_SWIGLU_CASE(5) AQ_SWIGLU_CASE(6) AQ_SWIGLU_CASE(7) AQ_SWIGLU_CASE(8) AQ_SWIGLU_CASE(9)
         AQ_SWIGLU_CASE(10) AQ_SWIGLU_CASE(11) AQ_SWIGLU_CASE(12) AQ_SWIGLU_CASE(13) AQ_SWIGLU_CASE(14) AQ_SWIGLU_CASE(15)

@@ -1350,7 +1350,7 @@ def test_gemm_walk_of_one_round_and_residuals(M, N, K, residual):
             assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("M,F", [(1025, 2048), (1300, 6928), (1041, 2064), (2050, 4096)])
+@pytest.mark.parametrize("M,F", [(1025, 2048), (1300, 6928), (1041, 2064), (2050, 4096), (1100, 5648), (1030, 6144)])
 def test_swiglu_quant_of_many_bf16_rows(oracle, M, F):
     """Many rows take the kernel that looks silu up: every bf16 gate pattern, zeros, gates around both ends of its table,
     rows whose maximum is small against their up half, and rows of ordinary values with a few zeros, against the oracle."""
