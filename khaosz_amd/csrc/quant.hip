@@ -410,7 +410,10 @@ __global__ __launch_bounds__(lut_waves(NC) * 64) void swiglu_quant_lut_kernel(co
                                                                                 int64_t ld, int8_t* __restrict__ q,
                                                                                 float* __restrict__ scale) {
   constexpr int NW = lut_waves(NC);
-  __shared__ __attribute__((aligned(16))) float table[0x8000 + LUT_SIZE];
+  // All of a compute unit's LDS, so that every index a gate can give lies inside: 13 bits of it and the sign.  A gate beyond
+  // the table reads an entry that nobody wrote; its row is done again.
+  __shared__ __attribute__((aligned(16))) float table[0xa000];
+  static_assert(LUT_SIZE <= 0x2000 && sizeof(table) == 160 * 1024, "13 bits of index");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t row_bytes = (uint32_t)F * 2u;
