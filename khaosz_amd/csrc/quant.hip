@@ -908,9 +908,7 @@ extern "C" int aq_rmsnorm_quant_rowwise_i8(const void* x, int x_dtype, const voi
                             : launch_rmsnorm_quant<false>(x, gamma, eps, M, K, ldx, q, scale, st);
 }
 
-#ifndef AQ_SWIGLU_WG_MAX_M
-#define AQ_SWIGLU_WG_MAX_M 1024
-#endif
+constexpr int64_t SWIGLU_WG_MAX_M = 1024;  // rows up to which each gets a workgroup
 template <bool BF16>
 static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld, int8_t* q, float* scale,
                                hipStream_t st) {
@@ -921,7 +919,7 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
   // us, before -> now: 1100 x 5632 14.7 -> 10.1, 2048 x 6912 20.0 -> 16.5, 4096 x 5632 28.5 -> 23.5, 4096 x 6912 38 -> 28,
   // 8192 x 8192 89 -> 72, 2048 x 2048 6.5 -> 6.3 (shorter rows stay).
   if constexpr (BF16) {
-    if (vpl >= 4 && vpl <= 16 && M > (vpl > 12 ? 1280 : 1024)) {
+    if (vpl >= 4 && vpl <= 16 && M > (vpl > 12 ? 1280 : SWIGLU_WG_MAX_M)) {
       const dim3 g((unsigned)aq::device_cus());
       switch (vpl) {
 #define AQ_SWIGLU_CASE(nc)                                                                                                      \
@@ -937,7 +935,7 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
     }
   }
   // few rows, or rows too long for one wavefront's registers: a workgroup of vpl wavefronts per row
-  if (vpl > 1 && (M <= AQ_SWIGLU_WG_MAX_M || vpl > 12)) {
+  if (vpl > 1 && (M <= SWIGLU_WG_MAX_M || vpl > 12)) {
     aq::queue_kernel((aq::swiglu_quant_wg_kernel<BF16>), dim3((unsigned)M), dim3((unsigned)vpl * 64), 0, st, ug, (int)F,
                        ld, q, scale);
     return (int)hipGetLastError();
@@ -951,17 +949,14 @@ static int launch_swiglu_quant(const void* ug, int64_t M, int64_t F, int64_t ld,
   // as many vector pairs per lane as the row has (a slot past the row costs its full arithmetic: a 5632-wide row
   // is 11 pairs per lane, and a 12th would be 8 % more work)
   switch (vpl) {
-#define AQ_SWIGLU_CASE(nc)                                                                                   \
-  case nc: aq::queue_kernel((aq::swiglu_quant_kernel<BF16, nc>), g, b, 0, st, ug, M, (int)F, ld, q, scale); break;
-    AQ_SWIGLU_CASE(1) AQ_SWIGLU_CASE(2) AQ_SWIGLU_CASE(3)
-    default: break;
-  }
-  if constexpr (!BF16) {
-    switch (vpl) {
-      AQ_SWIGLU_CASE(4) AQ_SWIGLU_CASE(5) AQ_SWIGLU_CASE(6) AQ_SWIGLU_CASE(7) AQ_SWIGLU_CASE(8) AQ_SWIGLU_CASE(9)
-      AQ_SWIGLU_CASE(10) AQ_SWIGLU_CASE(11) AQ_SWIGLU_CASE(12)
-      default: break;
-    }
+#define AQ_SWIGLU_CASE(nc)                                                                                            \
+  case nc:                                                                                                            \
+    if constexpr (BF16 && nc >= 4) return AQ_E_RANGE; /* bf16 rows of this length have gone one of the ways above */  \
+    else aq::queue_kernel((aq::swiglu_quant_kernel<BF16, nc>), g, b, 0, st, ug, M, (int)F, ld, q, scale);             \
+    break;
+    AQ_SWIGLU_CASE(1) AQ_SWIGLU_CASE(2) AQ_SWIGLU_CASE(3) AQ_SWIGLU_CASE(4) AQ_SWIGLU_CASE(5) AQ_SWIGLU_CASE(6)
+    AQ_SWIGLU_CASE(7) AQ_SWIGLU_CASE(8) AQ_SWIGLU_CASE(9) AQ_SWIGLU_CASE(10) AQ_SWIGLU_CASE(11) AQ_SWIGLU_CASE(12)
+    default: return AQ_E_RANGE;
   }
 #undef AQ_SWIGLU_CASE
   return (int)hipGetLastError();
