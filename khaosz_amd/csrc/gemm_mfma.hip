@@ -823,7 +823,7 @@ static int launch(GemmArgs& a, hipStream_t st) {
     if (!forced && tile == TILE_LARGE && gemm_walk_ok(a)) return gemm_walk_launch<FP8>(a, st);
   }
   if constexpr (OUT != OUT_I32) {
-    const int tm = forced ? (tile == TILE_SLICES32 ? 1 : tile == TILE_SLICES64 ? 2 : 0) : gemm_slices_rows(a.M, a.N);
+    const int tm = forced ? (tile == TILE_SLICES32 ? 1 : tile == TILE_SLICES64 ? 2 : 0) : gemm_slices_rows(a.M, a.N, a.K);
     if (tm) return gemm_slices_launch<FP8, OUT>(a, tm, st);
   }
   switch (tile) {
@@ -926,7 +926,7 @@ extern "C" int aq_linear_w8a8_residual(const int8_t* xq, const float* sx, const 
 #else
   const bool tile_forced = false;
 #endif
-  if (!tile_forced && !aq::gemm_slices_rows(M, N) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
+  if (!tile_forced && !aq::gemm_slices_rows(M, N, K) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
     return aq::gemv_tokens_launch(xq, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, st, false);
   aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);
   a.sx = sx;
@@ -960,7 +960,7 @@ extern "C" int aq_linear_fp8_residual(const uint8_t* xq, const float* sx, const 
 #else
   const bool tile_forced = false;
 #endif
-  if (!tile_forced && !aq::gemm_slices_rows(M, N) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
+  if (!tile_forced && !aq::gemm_slices_rows(M, N, K) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
     return aq::gemv_tokens_launch(reinterpret_cast<const int8_t*>(xq), sx, reinterpret_cast<const int8_t*>(wq), sw, bias,
                                   bias_dtype, residual, y, y_dtype, M, N, K, st, true);
   aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);

@@ -221,10 +221,26 @@ static int launch_slices(GemmArgs& a, hipStream_t st) {
 
 // 1: 32 x 32 tiles, 2: 64 x 32, 0: neither.  One tile per compute unit: a second round costs as much as the first, and the
 // kernels with larger tiles move fewer bytes.  Up to 16 rows have kernels of their own.
-int gemm_slices_rows(int64_t M, int64_t N) {
-  const int64_t cus = device_cus(), n32 = (N + 31) / 32;
+//
+// Measured, us, the path before (gemm_kernel's tiles; up to 32 rows the weight-streaming GEMV) -> here, weights in the
+// last-level cache | streamed from HBM:
+//   32 x 32, more than 32 rows: faster at every size tried (N 512 to 4096, K 512 to 8192), 64 x 2048 x 512 3.5 -> 3.1 | 3.9 -> 3.4,
+//     64 x 4096 x 8192 12.2 -> 8.9 | 17.4 -> 12.7, 333 x 512 x 6912 10.5 -> 6.1 | 10.6 -> 7.7.
+//   32 x 32, 17..32 rows: 32 x 256 x 2048 4.6 -> 3.7 | 4.7 -> 4.7, 32 x 2048 x 2048 5.1 -> 3.7 | 5.2 -> 5.4, 24 x 512 x 8192
+//     9.9 -> 6.2 | 9.6 -> 10.8, 32 x 2048 x 8192 10.3 -> 6.7 | 10.4 -> 12.1, 32 x 8192 x 4096 8.2 -> 6.2 | 9.3 -> 9.5: a fifth to two
+//     thirds faster from the cache, level to 16 % slower from HBM, where the GEMV has more loads in flight.
+//   64 x 32: every tile reads all 64 rows of A.  K below 1536 is over before that is hidden (64 x 6144 x 512 3.5 -> 3.8 |
+//     4.0 -> 4.3, x 1024 4.1 -> 4.3 | 5.5 -> 5.7, x 1536 4.6 -> 4.6 | 6.4 -> 6.3; 1000 x 512 x 1024 4.1 -> 4.4 | 4.5 -> 4.6), and so
+//     is not a wide matrix whose weights alone keep the memory busy (64 x 8192 x 6912 11.5 -> 12.9 | 16.8 -> 17.4, 64 x 5632 x 6912
+//     11.1 -> 11.5 | 15.8 -> 16.3, 40 x 8192 x 5120 9.5 -> 10.1 | 12.8 -> 13.0): those stay with the larger tiles.  Between them
+//     64 x 5120 x 5120 8.9 -> 7.8 | 13.7 -> 13.0, 40 x 6912 x 6912 11.0 -> 10.7 | 14.3 -> 14.6, 200 x 2048 x 6912 10.8 -> 9.4 |
+//     11.9 -> 11.8, 128 x 4096 x 8192 12.4 -> 11.9 | 17.3 -> 16.5.
+int gemm_slices_rows(int64_t M, int64_t N, int64_t K) {
+  const int64_t cus = device_cus(), n32 = (N + 31) / 32, tiles = (M + 63) / 64 * n32;
   if (M <= 16) return 0;
-  return (M + 31) / 32 * n32 <= cus ? 1 : (M + 63) / 64 * n32 <= cus ? 2 : 0;
+  if ((M + 31) / 32 * n32 <= cus) return 1;
+  const bool streams = M <= 64 && N * K > (32 << 20) && M * tiles > 9600;  // much weight, and many tiles that each read A
+  return tiles <= cus && K >= 1536 && !streams ? 2 : 0;
 }
 
 template <bool FP8, int OUT>

@@ -1379,6 +1379,30 @@ def test_swiglu_quant_of_many_bf16_rows(oracle, M, F):
     assert np.array_equal(to_np(q), qo)
 
 
+# Both sides of the rule for 64 x 32 tiles with K cut among wavefronts: K around 1536, weights around 32 MiB, tiles around one
+# per compute unit
+@pytest.mark.parametrize("M,N,K", [(64, 5120, 1520), (64, 5120, 1536), (33, 8193, 1536), (64, 8192, 4096), (64, 8192, 4112),
+                                   (48, 6400, 5248), (48, 6432, 5248), (65, 4096, 1536), (65, 4097, 1536)])
+def test_gemm_rule_for_k_cut_among_wavefronts(M, N, K):
+    """Whichever kernel the rule takes, int8 sums are the same bits as the tiles cut among wavefronts; FP8 sums differ by their
+    order alone: fp32 sums of K products by at most 2 K 2^-24 of the sum of their magnitudes (0.64 sqrt(K) times the result's
+    rms), bf16 results by a rounding more."""
+    _say("gemm slices rule", M, N, K)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    xq, wq = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
+    sx, sw = (torch.rand(n, generator=g, device=DEV) * 0.01 + 1e-4 for n in (M, N))
+    x8, w8 = (torch.randn(n, K, generator=g, device=DEV).to(torch.float8_e4m3fn).view(torch.uint8) for n in (M, N))
+    run = lambda: (ops.linear_w8a8(xq, sx, wq, sw, None, out_dtype=torch.bfloat16),
+                   ops.linear_fp8(x8, sx[:1], w8, sw[:1], None, out_dtype=torch.bfloat16))
+    got = run()
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(35) == 0
+        want = run()
+    assert torch.equal(got[0], want[0])
+    rms = want[1].float().square().mean().sqrt()
+    assert torch.allclose(got[1].float(), want[1].float(), rtol=2 ** -7, atol=2 * 2 ** -24 * K * 0.64 * K ** 0.5 * rms.item())
+
+
 # K cut among the wavefronts: fewer K steps than wavefronts, a ragged last step, ragged rows and columns, odd N, one tile
 @pytest.mark.parametrize("kind", [34, 35])
 @pytest.mark.parametrize("M,N,K", [(17, 33, 16), (33, 96, 400), (70, 75, 1040), (64, 64, 512), (65, 1001, 2064), (200, 512, 1936)])
