@@ -608,12 +608,12 @@ static bool gemv_swiglu_ok(int64_t M, int64_t F, int64_t K) {
 
 // ---------------------------------------------------------------------------
 // 17..32 tokens on codes: the same weight stream (every weight byte HBM -> registers once, operands assembled by
-// one DPP rotation per dword) with TG = 2 groups of 16 tokens multiplied against each weight fragment.  Between the
-// decode batch sizes above and the tiled GEMM (whose smallest tile, 64 x 32, spends the matrix-core time of 64
-// rows whatever M is: 32 x 8192 x 2048 in 6.9 us with the weights streamed from HBM) this kernel stays a
-// bandwidth-bound launch (6.0 us); from 33 tokens on, with a third and fourth token group, it was the slower one
-// (48 rows: 6.1 us, 64 rows: 7.6 us with the weights in the last-level cache, where a 128 x 32 tile took 5.8 us),
-// so those go to the tiles.  Same integer sums, same epilogue: the bits of the tiled GEMM.
+// one DPP rotation per dword) with TG = 2 groups of 16 tokens multiplied against each weight fragment: a bandwidth-bound
+// launch for matrices of more 32-row blocks than compute units, where the GEMM whose wavefronts share K would take a second
+// round of tiles (its comment has both sides; at one tile per compute unit it is the faster one from the last-level cache
+// and level to 16 % slower from HBM).  Also the decode batch sizes whose rows are too long for the kernels above.  From 33
+// tokens on, with a third and fourth token group, it was the slower one (48 rows: 6.1 us, 64 rows: 7.6 us with the weights
+// in the last-level cache, where a 128 x 32 tile took 5.8 us).  Same integer sums, same epilogue: the bits of the tiled GEMM.
 // K is walked in chunks of 1024 bytes per wavefront (KS wavefronts per row group: 1024-, 2048- or 4096-byte chunks
 // per workgroup), the token codes of one chunk at a time in LDS, so that rows of any length are taken (an MLP's
 // down projection) and the LDS of a compute unit holds several workgroups.  A chunk's codes are requested into
@@ -836,21 +836,16 @@ static int launch_gemv_tokens_shape(const GemvArgs& a, hipStream_t st, bool fp8)
   return (int)hipGetLastError();
 }
 
-// Chunk and workgroup shapes, from timings of 17..32 rows over N = 256..16384, K = 512..4096:
-//   * chunks no longer than the rows, or wavefronts idle: 1024 bytes up to K = 1024, else 2048; 4096 over 8
-//     wavefronts for K >= 4096 while every compute unit gets at most one workgroup (32 x 6144 x 4096: 7.5 us
-//     against 8.5 us), on 16 rows per workgroup while that still gives no compute unit a second one (32 x 2048 x
-//     5632: 9.5 us against 11.1 us; x 11008: 13.4 us against 16.6 us);
-//   * 32 rows per workgroup while there are no more 32-row blocks than compute units (32 x 8192 x 2048: 5.2 us, 64
-//     rows 6.8 us), 64 rows beyond (32 x 16384 x 2048: 7.0 us against 7.4 us: half the copies of the token codes).
+// Chunk and workgroup shapes.  Two kinds of call come here: 17..32 rows of more 32-row blocks than compute units (fewer take
+// the GEMM whose wavefronts share K), and 16 rows or fewer whose rows are too long for the GEMV kernels, 9.9 KB and more.
+//   * more 32-row blocks than compute units: 64 rows per workgroup, half the copies of the token codes (32 x 16384 x 2048:
+//     7.0 us against 7.4 us with 32), in chunks no longer than the rows, 1024 or 2048 bytes;
+//   * else 4096-byte chunks over 4 or 8 wavefronts, 16 rows per workgroup while that gives no compute unit a second one.
 // (gemv_tokens_ok and gemv_tokens_launch are not static: the tiled GEMM's entry points in gemm_mfma.hip hand these
 // shapes over)
 int launch_gemv_tokens(const GemvArgs& a, hipStream_t st, bool fp8) {
-  const bool wide = (a.N + 31) / 32 > device_cus();
-  if (a.K <= 1024) return wide ? launch_gemv_tokens_shape<1, 4>(a, st, fp8) : launch_gemv_tokens_shape<1, 2>(a, st, fp8);
-  if (wide) return launch_gemv_tokens_shape<2, 4>(a, st, fp8);
-  if (a.K >= 4096) return (a.N + 15) / 16 <= device_cus() ? launch_gemv_tokens_shape<4, 1>(a, st, fp8) : launch_gemv_tokens_shape<4, 2>(a, st, fp8);
-  return launch_gemv_tokens_shape<2, 2>(a, st, fp8);
+  if ((a.N + 31) / 32 > device_cus()) return a.K <= 1024 ? launch_gemv_tokens_shape<1, 4>(a, st, fp8) : launch_gemv_tokens_shape<2, 4>(a, st, fp8);
+  return (a.N + 15) / 16 <= device_cus() ? launch_gemv_tokens_shape<4, 1>(a, st, fp8) : launch_gemv_tokens_shape<4, 2>(a, st, fp8);
 }
 
 int gemv_tokens_launch(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw, const void* bias,
