@@ -1,5 +1,5 @@
-// The tiled GEMM of gemm_mfma.hip for more 256 x 128 tiles than compute units, or with a residual: at most one resident workgroup per compute unit walks tiles, and its K
-// loop does not stop between them.
+// The tiled GEMM of gemm_mfma.hip for more 256 x 128 tiles than compute units, or with a residual: at most one resident
+// workgroup per compute unit walks tiles, and its K loop does not stop between them.
 //
 // What bounds it: a tile of K = 1536 or 2048 is 12 to 16 K steps of 1024 matrix-core cycles, and the separate tiles of
 // gemm_kernel put a drain of the stores, the latency of the first stages, a step without loads and the epilogue around

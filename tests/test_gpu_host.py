@@ -4,6 +4,7 @@ import ctypes
 import pathlib
 import subprocess
 import sys
+import threading
 
 import pytest
 import torch
@@ -340,7 +341,12 @@ def test_a_layer_holds_its_weight_for_the_length_of_a_call(between):
             q._buffers["qweight"], q._buffers["w_scale"] = torch.ones_like(q.qweight), torch.ones_like(q.w_scale)
             old.append(torch.cuda.memory_allocated())
 
-        between(swap)
+        def another_thread():
+            t = threading.Thread(target=swap)
+            t.start()
+            t.join()
+
+        between(another_thread)
         y = q(x)
     assert torch.equal(y, want)
     assert old[1] - old[0] >= 8192 * 512 + 4 * 8192  # the new ones beside the old ones
@@ -357,3 +363,28 @@ def test_a_compiled_layer_and_block_give_the_same_bits():
         torch._dynamo.reset()
         assert torch.equal(torch.compile(lambda h: q(h) * 2, backend="eager")(h), want * 2)
         assert torch.equal(torch.compile(b, backend="eager")(x, fr, None, cache), block_want)
+
+
+def test_threads_on_streams_of_their_own_share_a_layer_and_a_block():
+    b = _block()
+    x, fr, cache, table = _case(b, 3, 40, 0)
+    cache.bind(table, 40)
+    h = torch.randn(9, 1408, device=DEV).to(DT)
+    with torch.inference_mode():
+        want = b(x, fr, None, cache), b.mlp.down(h)
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work():
+        with torch.cuda.stream(torch.cuda.Stream()), torch.inference_mode():
+            for _ in range(50):
+                got = b(x, fr, None, cache), b.mlp.down(h)  # every thread writes the same keys and values
+                if not (torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])):
+                    wrong.append(1)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

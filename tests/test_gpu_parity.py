@@ -707,12 +707,11 @@ def test_up_gate_gemv_with_the_activation_refuses_what_it_does_not_serve():
                                  (2048, 5632), (8200, 6912), (77, 11008), (40, 128), (12000, 4224), (8400, 1024),
                                  (4200, 4224)])
 def test_a_few_dozen_rows_same_bits_as_the_oracle(oracle, M, N, K):
-    """17..32 rows: the Linear on codes hands them to the weight-streaming matrix-core kernel with 2 groups of
-    16 tokens, which walks rows of any length (whole 128-byte lines) in chunks: 1024-byte chunks for short rows,
-    2048 otherwise, 4096 for K >= 4096; 16, 32 or 64 rows per workgroup by the number of row blocks against the
-    compute units; ragged last chunks, rows shorter than a chunk.  33..64 rows: the tiled GEMM, whose tile
-    narrows to 128 x 64 or 128 x 32 for so few rows.  int32 sums and the frozen epilogue: bit for bit against the
-    oracle, bf16 and fp32 outputs, with bias and residual, odd N."""
+    """17..64 rows: the GEMM whose wavefronts share K while there is at most one of its 32-column tiles per compute unit; with
+    more, 17..32 rows of whole 128-byte lines go to the weight-streaming matrix-core kernel with 2 groups of 16 tokens,
+    which walks rows of any length in chunks of 1024 or 2048 bytes (ragged last chunks, rows shorter than a chunk), and
+    33..64 rows to the narrow tiles.  int32 sums and the frozen epilogue: bit for bit against the oracle, bf16 and fp32
+    outputs, with bias and residual, odd N."""
     _say("linear, few dozen rows", M, N, K)
     x = make_x(M, K, 50 + M).to(torch.bfloat16)
     w = make_x(N, K, 51) * 0.02
@@ -986,9 +985,9 @@ def test_linear_fp8_within_tolerance(oracle, tile, M, N, K):
 @pytest.mark.parametrize("N,K", [(8192, 2048), (77, 512), (3072, 1536), (200, 256), (8400, 2304), (130, 4096),
                                  (8400, 1024), (300, 5632), (4200, 4224)])
 def test_linear_fp8_a_few_dozen_rows(oracle, M, N, K):
-    """17..32 rows of FP8 codes (whole 128-byte lines) go to the weight-streaming kernel (one 16x16x128 product
-    per 128-byte line and token group, fp32 sums, chunks and K parts added in a fixed order), in every chunk and
-    workgroup shape of its dispatch; 33..64 rows to the narrow tiles.  Against the float64 sum of the oracle's codes inside the stated
+    """17..64 rows of FP8 codes: the GEMM whose wavefronts share K, or, with more 32-column tiles than compute units, the
+    weight-streaming kernel for 17..32 rows (one 16x16x128 product per 128-byte line and token group, fp32 sums, chunks and
+    K parts added in a fixed order) and the narrow tiles.  Against the float64 sum of the oracle's codes inside the stated
     tolerance, against the tiled GEMM on the same codes (a forced tile shape keeps it on the tiles) within the
     change of summation order, with bias and residual, and the same bits on a second call."""
     _say("linear_fp8, few dozen rows", M, N, K)
