@@ -10,9 +10,9 @@ already resident in HBM:
           int8 GEMV against W int8 [8192, 2048] -> dequant -> y bf16.  HBM-bound; value = GB/s of
           algorithmic bytes N*K + 4N + 2MK + 2MN.  The weight rotates over 40 distinct buffers
           (671 MB) so that no step finds its weight in the 256 MB last-level cache.
-  prefill  x bf16 [4096, 2048] -> per-token int8 quantise -> int8 MFMA GEMM against
+  prefill x bf16 [4096, 2048] -> per-token int8 quantise -> int8 MFMA GEMM against
           W [2048, 2048] -> fused scale + bias -> y bf16.  value = TOPS of 2*M*N*K.
-  fp8     (configs[3])  x bf16 [2048, 8192], W [2048, 8192] e4m3, per-tensor scales.
+  fp8     x bf16 [2048, 8192], W [2048, 8192] e4m3, per-tensor scales.
 
 The K timed steps are captured once into a HIP graph and replayed, so the figure is the GPU's,
 not the Python launch loop's; the eager (un-captured) figure is reported beside it.  The
@@ -256,7 +256,7 @@ def bench_decode(torch, ops, args, dev):
         "workload": f"decode_gemv_w8a8 M={M} K={K} N={N} bf16->int8 per-token, W int8 per-channel, bf16 out",
         "value": gbs, "unit": "GB/s", "ms_per_step": ms, "eager_ms_per_step": ms_eager,
         "ms_per_step_p10_p50_p90": d_step, "bytes_per_step": bytes_alg, "dtype": "int8",
-        "roofline": {"bound": "hbm", "kernel": ("gemv_mfma_kernel<.., FQ>" if M > 4 else "gemv_w8a8_kernel<.., FUSED>")
+        "roofline": {"bound": "hbm", "kernel": ("gemv_rows_kernel" if M > 4 else "gemv_w8a8_kernel<.., FUSED>")
                      + " (quantises its rows itself: the whole step)",
                      "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": gbs / PEAK_HBM_GBS,
                      "traffic": traffic, "traffic_source": traffic_src,

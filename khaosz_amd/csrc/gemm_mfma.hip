@@ -17,6 +17,9 @@
 // later sub-steps are issued between the MFMAs of the current one, with one
 // workgroup barrier per K step.  The epilogue is fused and runs straight from
 // the accumulator registers: int32 store, or dequantise (+bias) and cast.
+// Two other kernels take calls from here: gemm_walk.hip the 256 x 128 tiles of
+// several rounds or with a residual (bf16 outputs), gemm_slices.hip a few dozen
+// to a few hundred rows.
 #include "aq_gemm.h"
 
 namespace aq {

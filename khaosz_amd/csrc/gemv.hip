@@ -1,8 +1,10 @@
 // Decode path (M <= 16 tokens): a weight-streaming int8 GEMV.  The weight
 // matrix is read exactly once with 16-byte loads, one wavefront reading 1 KiB
-// contiguous of a row per instruction; the few activation rows are quantised
-// by the row-wise kernel into the caller's workspace, pulled into LDS once per
-// workgroup by direct global->LDS loads and reused by every row of W.
+// contiguous of a row per instruction; the few activation rows come as codes
+// (the caller's, or the row-wise kernel's in the caller's workspace), pulled into
+// LDS once per workgroup by direct global->LDS loads and reused by every row of W,
+// or are quantised by the workgroup itself (FUSED: up to 4 bf16 rows; more rows,
+// fp32 and FP8 ones take gemv_rows.hip, see gemv_dispatch_fused).
 // Products are v_dot4_i32_i8 (no MFMA tiles, no LDS staging of W); a wavefront
 // reduces its 4 x MT partial sums with a transposed butterfly so that each
 // lane ends up owning one output, then applies the same dequantising epilogue

@@ -295,7 +295,9 @@ __device__ __forceinline__ void swiglu_row_general(__amdgpu_buffer_rsrc_t Ur, __
 // scales the down projection consumes.  Replaces the activation, the product and
 // the quantiser launches (three passes over [M, F]) by one.  A lane first turns
 // its NC vector pairs into h (fp32, kept in registers; the inputs die as it goes),
-// then reduces the absmax and rounds.
+// then reduces the absmax and rounds.  For fp32 rows, and for bf16 rows of up to
+// three vector pairs per lane; longer bf16 rows look silu up when there are many
+// of them (swiglu_quant_lut_kernel), and few rows get a workgroup each.
 //
 // The kernel is bound by its vector arithmetic (about 34 operations per element at first: the exponential's
 // polynomial, a correctly rounded divide, the two-correction rounding; 4096 x 5632 was 20 us of it at 2.4 GHz),
@@ -311,7 +313,8 @@ __device__ __forceinline__ void swiglu_row_general(__amdgpu_buffer_rsrc_t Ur, __
 //    for such rows, and the rounding add packs its own byte (quant_codes_packed).
 //  * NC is the row's own number of vector pairs per lane (a pair past the row would cost its full arithmetic).
 // Four wavefronts fit a SIMD (128 registers: a row's h is 88 of them at F = 5632); the SIMD serves the oldest
-// first, so a compute unit's 16 rows finish one after the other, 4096 x 5632 bf16 in 26.2 us (at first: 31.5).
+// first, so a compute unit's 16 rows finish one after the other, 4096 x 5632 bf16 in 26.2 us (at first: 31.5; those
+// rows look silu up now, 22.7).
 template <bool BF16, int NC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void swiglu_quant_kernel(
     const void* __restrict__ ug, int64_t M, int F, int64_t ld, int8_t* __restrict__ q, float* __restrict__ scale) {
