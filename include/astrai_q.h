@@ -92,9 +92,9 @@ int aq_gemm_i8_i32(const int8_t *xq, const int8_t *wq, int32_t *acc, int64_t M, 
  * fp32, then one round-to-nearest-even cast to y_dtype.  Replaces the whole
  * F.linear(x, weight, bias) of linear.py:21 for M > 16.
  * bias may be NULL (the reference never constructs a Linear with bias=True).
- * Any M: a tiled matrix-core GEMM whose tile is chosen by shape (128 x 32 up to 256 x 128), except
- * that 17..32 rows (K a multiple of 128) run on the weight-streaming kernel of the decode path
- * instead, with the same bits. */
+ * Any M: a matrix-core GEMM whose tile is chosen by shape (32 x 32 up to 256 x 256), except that 17..32 rows
+ * of many outputs (K a multiple of 128) run on the weight-streaming kernel of the decode path instead, with
+ * the same bits. */
 int aq_linear_w8a8(const int8_t *xq, const float *sx, const int8_t *wq, const float *sw,
                    const void *bias, int bias_dtype, void *y, int y_dtype, int64_t M,
                    int64_t N, int64_t K, void *stream);
@@ -107,8 +107,9 @@ int aq_linear_w8a8(const int8_t *xq, const float *sx, const int8_t *wq, const fl
  * ws: device scratch of at least aq_gemv_w8a8_workspace_bytes(M, K). */
 size_t aq_gemv_w8a8_workspace_bytes(int64_t M, int64_t K);
 
-/* 1 where the decode entry points below (norm != 0: ..._rmsnorm) quantise the rows inside their one launch: ws is
- * not touched then, and any 16-byte aligned pointer will do for it. */
+/* 1 where the decode entry points below (norm != 0: ..._rmsnorm) quantise the rows inside their one launch (rows of at
+ * most 8192 elements, with the norm bf16 rows of at most 2048): ws is not touched then, and any 16-byte aligned pointer
+ * will do for it. */
 int aq_gemv_w8a8_decode_one_launch(int x_dtype, int norm, int64_t M, int64_t N, int64_t K);
 int aq_gemv_w8a8_decode(const void *x, int x_dtype, const int8_t *wq, const float *sw,
                         const void *bias, int bias_dtype, void *y, int y_dtype, int64_t M,
@@ -159,7 +160,7 @@ int aq_gemv_w8a8_codes_residual(const int8_t *xq, const float *sx, const int8_t 
  * y = linear(quantise(rmsnorm(x) * gamma)) (+ bias) (+ residual), the codes and
  * scales being those aq_rmsnorm_quant_rowwise_i8 gives (same fixed arithmetic),
  * so the result equals that call followed by aq_gemv_w8a8_codes_residual bit
- * for bit.  One launch for up to 8 bf16 rows of at most 2048 elements, those two
+ * for bit.  One launch for bf16 rows of at most 2048 elements, those two
  * calls through ws otherwise.  gamma: [K] in x's dtype; residual may be NULL.
  * Replaces the norm + Linear pairs of a decode step (decoder_block.py:50-51,57
  * feeding attention.py:83-85 and mlp.py:25). */
@@ -205,8 +206,8 @@ int aq_linear_fp8_residual(const uint8_t *xq, const float *sx, const uint8_t *wq
  * on e4m3 codes (one 16x16x128 matrix-core product per 128-byte line), per-tensor scales, fp32 accumulation,
  * y = ((acc * sx) * sw + bias) cast, + residual.  aq_gemv_fp8_codes_residual takes codes and scale as
  * aq_quant_tensor_fp8 writes them; aq_gemv_fp8_decode_residual takes the rows themselves and, for bf16 rows
- * of K <= 2048 (K a multiple of 512), casts them inside the GEMV kernel (one launch: the tensor's maximum goes
- * round the workgroup first), otherwise through ws (aq_gemv_fp8_workspace_bytes(M, K) bytes) by
+ * of K <= 8192 (K <= 4096 for 9..16 of them), casts them inside the GEMV kernel (one launch: the tensor's maximum
+ * goes round the workgroup first), otherwise through ws (aq_gemv_fp8_workspace_bytes(M, K) bytes) by
  * aq_quant_tensor_fp8 + the codes entry.  K not a multiple of 256, or rows too long for a compute unit's
  * LDS: the tiled FP8 GEMM takes the call.  Replaces F.linear (linear.py:21) in the FP8 variant. */
 size_t aq_gemv_fp8_workspace_bytes(int64_t M, int64_t K);

@@ -298,7 +298,7 @@ def gemv_w8a8_decode(x, wq, sw, bias=None, out_dtype=None, workspace: Optional[t
                      residual=None, norm=None) -> torch.Tensor:
     """Decode path for at most 16 rows of ``x [M, K]``: fused per-token quantise + int8 GEMV + epilogue.
     ``norm = (gamma [K], eps)``: RMS-normalise the rows first (the codes ``rmsnorm_quant_rowwise_i8``
-    gives), in the same launch for up to 8 bfloat16 rows of at most 2048 elements."""
+    gives), in the same launch for bfloat16 rows of at most 2048 elements."""
     if workspace is None:
         gamma, eps = norm if norm is not None else (None, 0.0)
         y = (_host or _native()).gemv_w8a8_decode(x, wq, sw, bias, out_dtype, residual, gamma, eps)
@@ -832,7 +832,7 @@ def gemv_fp8_codes(xq, sx, wq, sw, bias=None, out_dtype=torch.bfloat16, residual
 def gemv_fp8_decode(x, wq, sw, bias=None, out_dtype=None, workspace: Optional[torch.Tensor] = None,
                     residual=None) -> torch.Tensor:
     """FP8 decode path for at most 16 rows of ``x [M, K]``: per-tensor e4m3 cast + GEMV + epilogue, one launch for
-    bfloat16 rows of at most 2048 elements."""
+    bfloat16 rows of at most 8192 elements (4096 for more than 8 rows)."""
     if workspace is None:
         y = (_host or _native()).gemv_fp8_decode(x, wq, sw, bias, out_dtype, residual)
         if y is not None:
