@@ -148,7 +148,7 @@ def linear_native():
         m = torch.nn.modules.module
         h.set_linear_types(QuantLinear, Fp8Linear, _CLASSES, (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks,
                                                     m._global_backward_pre_hooks), ops.__dict__, _OPERATORS, _LIMITS)
-        h.serve_calls(_NativeCall.__call__)
+        h.serve_calls(_NativeCall)
         _told = True
     return h
 

@@ -66,3 +66,32 @@ def test_the_native_rule_for_the_merge_inside_the_projection_is_the_operators():
         for heads, d in ((1, 64), (8, 64), (24, 64), (31, 64), (32, 64), (16, 128), (17, 128), (33, 64)):
             for total in (1, 255, 256, 257, 512, 513, 768, 769, 1024, 1025, 5000):
                 assert host.attn_gemv_fusable(B, heads * d, total) == ops.attn_gemv_fusable(B, heads, d, total)
+
+
+def test_what_native_code_leaves_goes_to_the_next_call_behind_the_layers(monkeypatch, told):
+    """As the Python code of their ``__call__`` would have it: a base class's call, or nn.Module's as it is now."""
+    seen = []
+
+    class Watched(torch.nn.Module):
+        def __call__(self, *args, **kwargs):
+            seen.append(kwargs)
+            return super().__call__(*args, **kwargs)
+
+    class Both(_Float, Watched):
+        pass
+
+    for cls, count in ((_Float, 0), (Both, 1)):
+        q, x = _layer(cls)
+        r = torch.ones(4, 16)
+        assert torch.equal(q(x, residual=r), _float_forward(q, x, r)) and len(seen) == count
+        with monkeypatch.context() as m:
+            calls, real = [], torch.nn.Module.__call__
+            m.setattr(torch.nn.Module, "__call__", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+            assert torch.equal(q(x, r), _float_forward(q, x, r)) and len(calls) == 1
+        with pytest.raises(TypeError):
+            q()
+        seen.clear()
+    with pytest.raises((TypeError, AttributeError)):
+        QuantLinear.__call__(3)
+    with pytest.raises(TypeError):
+        QuantLinear.__call__()
