@@ -424,6 +424,25 @@ int aq_prefill_attn_paged_ahead(const void *q, int64_t q_stride, const void *k_c
                                 int64_t n_pages, void *out, float scale, int64_t B, int64_t S, int64_t Hq,
                                 int64_t Hkv, int64_t D, const aq_span *ahead, int n_ahead, void *stream);
 
+/* A prompt's attention on query heads as the fused projection left them, the rotation of aq_rope_kv_write (and, with q_gain, the
+ * RMSNorm of aq_rope_kv_write_qknorm) applied as they are read: the same bits without writing the rotated queries and reading
+ * them back.  aq_rope_kv_cache_write is aq_rope_kv_write without q_out.  freqs, freqs_stride and the layouts are as there, k_gain
+ * and q_gain NULL without qk-norm, the rest as in the functions above. */
+int aq_rope_kv_cache_write(const void *qkv, const float *freqs, int64_t freqs_stride,
+                           const int64_t *page_table, int64_t P, int64_t pos, int64_t S, int64_t page_size,
+                           void *k_cache, void *v_cache, int64_t n_pages, void *k_out, int64_t B, int64_t Hq,
+                           int64_t Hkv, int64_t D, const void *k_gain, float eps, void *stream);
+int aq_rope_prefill_attn_causal_ahead(const void *q, int64_t q_stride, const float *freqs,
+                                      int64_t freqs_stride, const void *q_gain, float eps, const void *k,
+                                      int64_t k_stride, const void *v, int64_t v_stride, void *out,
+                                      float scale, int64_t B, int64_t S, int64_t Hq, int64_t Hkv, int64_t D,
+                                      const aq_span *ahead, int n_ahead, void *stream);
+int aq_rope_prefill_attn_paged_ahead(const void *q, int64_t q_stride, const float *freqs, int64_t freqs_stride,
+                                     const void *q_gain, float eps, const void *k_cache, const void *v_cache,
+                                     const int64_t *page_table, int64_t P, int64_t start, int64_t page_size,
+                                     int64_t n_pages, void *out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                     int64_t Hkv, int64_t D, const aq_span *ahead, int n_ahead, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -75,6 +75,12 @@ SYMBOLS = {
                                             _vp, _int, _vp]),
     "aq_prefill_attn_paged_ahead": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.c_float, _i64, _i64,
                                            _i64, _i64, _i64, _vp, _int, _vp]),
+    "aq_rope_kv_cache_write": (_int, [_vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64,
+                                      _vp, ctypes.c_float, _vp]),
+    "aq_rope_prefill_attn_causal_ahead": (_int, [_vp, _i64, _vp, _i64, _vp, ctypes.c_float, _vp, _i64, _vp, _i64, _vp, ctypes.c_float,
+                                                 _i64, _i64, _i64, _i64, _i64, _vp, _int, _vp]),
+    "aq_rope_prefill_attn_paged_ahead": (_int, [_vp, _i64, _vp, _i64, _vp, ctypes.c_float, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp,
+                                                ctypes.c_float, _i64, _i64, _i64, _i64, _i64, _vp, _int, _vp]),
 }
 
 # csrc/aq_lab.h: the lab library's additions (measurement probes, the tile-forcing test hook)

@@ -73,7 +73,7 @@ def build(force: bool = True, verbose: bool = False, stall_counters: bool = Fals
     lab_sources = [(src, obj, extra + (["-DAQ_LAB_STALL"] if stall_counters and src == "gemm_mfma.hip" else []))
                    for src, obj, extra in LAB_SOURCES]
     headers = [os.path.join(CSRC, "aq_common.h"), os.path.join(CSRC, "aq_rows.h"), os.path.join(CSRC, "aq_gemv.h"), os.path.join(CSRC, "aq_gemm.h"),
-               os.path.join(CSRC, "aq_lab.h"),
+               os.path.join(CSRC, "aq_lab.h"), os.path.join(CSRC, "aq_rope.h"),
                os.path.join(HERE, "..", "include", "astrai_q.h")]
 
     def compile_one(job):

@@ -19,70 +19,10 @@
 // (table entry < 0 or out of range) are skipped on write and read as zero keys
 // and values, as the reference's gather does.
 #include "aq_common.h"
+#include "aq_rope.h"
 #include "aq_rows.h"
 
 namespace aq {
-
-// Rotates 8 consecutive elements (4 interleaved pairs): (x0 + i x1)(c + i s) with four rounded
-// products, one rounded difference and one rounded sum per pair.
-__device__ __forceinline__ uint4 rope8(uint4 x, const float* cs /* 4 (cos, sin) pairs */) {
-  const float4 a = *reinterpret_cast<const float4*>(cs), b = *reinterpret_cast<const float4*>(cs + 4);
-  const float c[4] = {a.x, a.z, b.x, b.z}, sn[4] = {a.y, a.w, b.y, b.w};
-  const uint32_t in[4] = {x.x, x.y, x.z, x.w};
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = __uint_as_float(in[i] << 16), x1 = __uint_as_float(in[i] & 0xffff0000u);
-    const float r0 = __fsub_rn(__fmul_rn(x0, c[i]), __fmul_rn(x1, sn[i]));
-    const float r1 = __fadd_rn(__fmul_rn(x0, sn[i]), __fmul_rn(x1, c[i]));
-    o[i] = pack_bf16x2(r0, r1);
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-// the same on table values already in registers
-__device__ __forceinline__ uint4 rope8(uint4 x, float4 a, float4 b) {
-  const float c[4] = {a.x, a.z, b.x, b.z}, sn[4] = {a.y, a.w, b.y, b.w};
-  const uint32_t in[4] = {x.x, x.y, x.z, x.w};
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = __uint_as_float(in[i] << 16), x1 = __uint_as_float(in[i] & 0xffff0000u);
-    const float r0 = __fsub_rn(__fmul_rn(x0, c[i]), __fmul_rn(x1, sn[i]));
-    const float r1 = __fadd_rn(__fmul_rn(x0, sn[i]), __fmul_rn(x1, c[i]));
-    o[i] = pack_bf16x2(r0, r1);
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-// RMSNorm over the head dimension of a rotated query or key (attention.py:62-64, 86-89: after the rotation, before
-// the key goes into the cache).  The rotated values are taken as they are stored, rounded to bf16.  Sum of squares
-// in a fixed order that does not depend on which kernel holds the vector how: per 8-element chunk the rounded
-// squares are added in memory order, then the D / 8 chunk sums are combined by a butterfly over the chunk index
-// (chunk c with c ^ 1, then ^ 2, ^ 4, ^ 8; fl(a + b) is the same whichever partner computes it).  Then
-// r = 1 / sqrt(ss / D + eps) (every operation correctly rounded) and y = bf16((x * r) * gain).
-__device__ __forceinline__ float chunk_sumsq(uint4 x) {
-  const uint32_t in[4] = {x.x, x.y, x.z, x.w};
-  float s = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = __uint_as_float(in[i] << 16), x1 = __uint_as_float(in[i] & 0xffff0000u);
-    s = __fadd_rn(s, __fmul_rn(x0, x0));
-    s = __fadd_rn(s, __fmul_rn(x1, x1));
-  }
-  return s;
-}
-__device__ __forceinline__ uint4 chunk_normed(uint4 x, float r, uint4 gain) {
-  const uint32_t in[4] = {x.x, x.y, x.z, x.w}, gn[4] = {gain.x, gain.y, gain.z, gain.w};
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = __uint_as_float(in[i] << 16), x1 = __uint_as_float(in[i] & 0xffff0000u);
-    const float g0 = __uint_as_float(gn[i] << 16), g1 = __uint_as_float(gn[i] & 0xffff0000u);
-    o[i] = pack_bf16x2(__fmul_rn(__fmul_rn(x0, r), g0), __fmul_rn(__fmul_rn(x1, r), g1));
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
 
 struct RopeArgs {
   const uint16_t* qkv;   // [B, S, (Hq + 2 Hkv) * D]
@@ -91,7 +31,7 @@ struct RopeArgs {
   const int64_t* table;  // [B, P]
   uint16_t* kc;          // [n_pages, page, Hkv, D]
   uint16_t* vc;
-  uint16_t* q_out;       // [B, S, Hq, D]
+  uint16_t* q_out;       // [B, S, Hq, D], or null: the query heads are left alone
   uint16_t* k_out;       // [B, S, Hkv, D] rotated keys, or null
   int64_t P, pos, page, n_pages, S;
   int B, Hq, Hkv, D;
@@ -100,25 +40,24 @@ struct RopeArgs {
   float eps;
 };
 
-// one thread per 16-byte chunk (8 elements) of a head vector of a token
+// One thread per 16-byte chunk (8 elements) of a head vector of a token.  Without q_out the query heads are left to whoever reads
+// them (the prefill attention rotates its own): 4096 tokens of 16 + 2 x 4 heads of 128 move 21 MB instead of 50, and the launch, at
+// the rate of a copy either way, takes 6.2 us instead of 11.3 (attention 0.2 to 0.8 more; 2048 tokens of 24 + 2 x 4 heads of 64:
+// 4.6 -> 2.8, attention 0.8 more).
 __global__ __launch_bounds__(256) void rope_kv_write_kernel(RopeArgs p) {
-  const int64_t heads = p.Hq + 2 * p.Hkv;
+  const int h0 = p.q_out ? 0 : p.Hq;
+  const int64_t heads = p.Hq + 2 * p.Hkv - h0;
   const int cph = p.D / 8;  // chunks per head vector
   const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (c >= (int64_t)p.B * p.S * heads * cph) return;
   const int ch = (int)(c % cph);
   const int64_t hv = c / cph, tokn = hv / heads;
-  const int h = (int)(hv % heads);
+  const int h = (int)(hv % heads) + h0;
   const int64_t b = tokn / p.S, s = tokn % p.S;
-  uint4 x = *reinterpret_cast<const uint4*>(p.qkv + hv * p.D + ch * 8);
+  uint4 x = *reinterpret_cast<const uint4*>(p.qkv + (tokn * (p.Hq + 2 * p.Hkv) + h) * p.D + ch * 8);
   if (h < p.Hq + p.Hkv) x = rope8(x, p.freqs + b * p.freqs_stride + s * p.D + ch * 8);  // v heads do not rotate
-  if (p.q_gain) {  // uniform: qk-norm.  A head vector's D / 8 chunks sit in neighbouring lanes of one DPP row.
-    float ss = chunk_sumsq(x);
-    ss = __fadd_rn(ss, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0xB1, 0xf, 0xf, false)));   // c ^ 1
-    ss = __fadd_rn(ss, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0x4E, 0xf, 0xf, false)));   // c ^ 2
-    ss = __fadd_rn(ss, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0x141, 0xf, 0xf, false)));  // the other quad of the half row: c ^ 4
-    if (p.D == 128)
-      ss = __fadd_rn(ss, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0x140, 0xf, 0xf, false)));  // the other half row: c ^ 8
+  if (p.q_gain) {  // uniform: qk-norm
+    const float ss = p.D == 128 ? head_sumsq<128>(x) : head_sumsq<64>(x);
     if (h < p.Hq + p.Hkv) {
       const uint16_t* gain = h < p.Hq ? p.q_gain : p.k_gain;
       x = chunk_normed(x, rms_scale(ss, (float)p.D, p.eps), *reinterpret_cast<const uint4*>(gain + ch * 8));
@@ -590,22 +529,22 @@ inline int64_t attn_workspace_bytes(int64_t B, int64_t Hq, int64_t ns) {
 
 }  // namespace aq
 
-// q_gain == nullptr: no qk-norm (then k_gain and eps are not looked at)
+// q_gain == nullptr: no qk-norm (then k_gain and eps are not looked at).  keys_only: q_out is not written.
 static int rope_kv_write(const void* qkv, const float* freqs, int64_t freqs_stride, const int64_t* page_table,
                          int64_t P, int64_t pos, int64_t S, int64_t page_size, void* k_cache, void* v_cache,
                          int64_t n_pages, void* q_out, void* k_out, int64_t B, int64_t Hq, int64_t Hkv, int64_t D,
-                         const void* q_gain, const void* k_gain, float eps, void* stream) {
+                         const void* q_gain, const void* k_gain, float eps, void* stream, bool keys_only = false) {
   if (D != 64 && D != 128) return AQ_E_SHAPE;
   if (q_gain && (!k_gain || !(eps >= 0.0f))) return k_gain ? AQ_E_SHAPE : AQ_E_NULL;
   if (aq::check_ptr16(q_gain) || (q_gain && aq::check_ptr16(k_gain))) return AQ_E_ALIGN;
   if (B < 0 || S < 0 || Hq <= 0 || Hkv <= 0 || P <= 0 || pos < 0 || page_size <= 0 || n_pages <= 0) return AQ_E_SHAPE;
   if (freqs_stride != 0 && freqs_stride < S * D) return AQ_E_SHAPE;
   if (B == 0 || S == 0) return AQ_OK;
-  if (!qkv || !freqs || !page_table || !k_cache || !v_cache || !q_out) return AQ_E_NULL;
+  if (!qkv || !freqs || !page_table || !k_cache || !v_cache || (!q_out && !keys_only)) return AQ_E_NULL;
   if (aq::check_ptr16(qkv) || aq::check_ptr16(k_cache) || aq::check_ptr16(v_cache) || aq::check_ptr16(q_out) ||
       aq::check_ptr16(freqs) || (freqs_stride & 3) || (k_out && aq::check_ptr16(k_out)))
     return AQ_E_ALIGN;
-  const int64_t chunks = B * S * (Hq + 2 * Hkv) * (D / 8);
+  const int64_t chunks = B * S * ((keys_only ? 0 : Hq) + 2 * Hkv) * (D / 8);
   if (chunks > (int64_t)0x7fffffff * 256) return AQ_E_RANGE;
   aq::RopeArgs a{};
   a.qkv = static_cast<const uint16_t*>(qkv);
@@ -649,6 +588,14 @@ extern "C" int aq_rope_kv_write_qknorm(const void* qkv, const float* freqs, int6
   if (!q_gain || !k_gain) return AQ_E_NULL;
   return rope_kv_write(qkv, freqs, freqs_stride, page_table, P, pos, S, page_size, k_cache, v_cache, n_pages, q_out, k_out,
                        B, Hq, Hkv, D, q_gain, k_gain, eps, stream);
+}
+
+extern "C" int aq_rope_kv_cache_write(const void* qkv, const float* freqs, int64_t freqs_stride, const int64_t* page_table,
+                                      int64_t P, int64_t pos, int64_t S, int64_t page_size, void* k_cache, void* v_cache,
+                                      int64_t n_pages, void* k_out, int64_t B, int64_t Hq, int64_t Hkv, int64_t D,
+                                      const void* k_gain, float eps, void* stream) {
+  return rope_kv_write(qkv, freqs, freqs_stride, page_table, P, pos, S, page_size, k_cache, v_cache, n_pages, nullptr, k_out, B,
+                       Hq, Hkv, D, k_gain, k_gain, eps, stream, true);
 }
 
 extern "C" int64_t aq_paged_attn_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t total_len) {

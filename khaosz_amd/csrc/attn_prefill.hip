@@ -37,6 +37,7 @@
 // barrier per block.  A row's 16-byte pieces are permuted (row_key) so that both
 // the row reads of K and the transposing reads of V spread over all banks.
 #include "aq_common.h"
+#include "aq_rope.h"
 
 namespace aq {
 
@@ -55,6 +56,11 @@ struct PrefillAttnArgs {
   const int64_t* table;  // [B, P] physical page ids, < 0: unmapped (zero keys and values)
   int64_t P, page, n_pages;
   int start, page_shift;
+  // freqs != null: q holds heads as the projection left them, which are rotated (and, with q_gain, RMS-normalised) as they are read
+  const float* freqs;    // [S, D/2, 2] (cos, sin) per sequence; sequences freqs_stride floats apart (0: shared)
+  int64_t freqs_stride;
+  const uint16_t* q_gain;
+  float eps;
   int table_lds;  // entries of the page table that are copied into LDS first (all a launch needs, or 0: read from memory)
   int paired;     // != 0: the second half of the workgroups takes the query blocks lightest first
   int wgs;        // workgroups that attend; the ones behind them read ahead
@@ -206,13 +212,41 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
   };
   issue(0, 0);
 
-  // Q^T operand: lane = (query col, dimensions 16 step + 8 g .. + 8); rows past S read row S - 1
+  // The wavefront's 32 query rows, whole rows at a time, through the second buffer (nothing is requested into it before the first
+  // barrier) to the lanes that take them: Q^T operand, lane = (query col, dimensions 16 step + 8 g .. + 8); rows past S read
+  // row S - 1.  (A lane reading its own query's pieces touches a line with every piece, of the rotary table
+  // too: 3.5 us of 25 at 8 x 512 x 16 heads of 128.)
   uint4 qf[DSTEPS];
   {
-    const int qr = qpos < S ? qpos : S - 1;
-    const uint16_t* src = p.q + (tok0 + qr) * p.q_stride + (int64_t)h * D + g * 8;
+    constexpr int NQ = 32 / RPI;
+    static_assert(QW * KW * 32 * ROWB <= BUF, "the queries fit a buffer");
+    const int piece = lane % LPR;
+    uint4 x[NQ];
+    float4 fa[NQ], fb[NQ];
 #pragma unroll
-    for (int st = 0; st < DSTEPS; ++st) qf[st] = *reinterpret_cast<const uint4*>(src + st * 16);
+    for (int i = 0; i < NQ; ++i) {
+      const int r = qw0 + i * RPI + lane / LPR, qr = r < S ? r : S - 1;
+      x[i] = *reinterpret_cast<const uint4*>(p.q + (tok0 + qr) * p.q_stride + (int64_t)h * D + piece * 8);
+      if (p.freqs) {  // uniform
+        const float* cs = p.freqs + (int64_t)b * p.freqs_stride + (int64_t)qr * D + piece * 8;
+        fa[i] = *reinterpret_cast<const float4*>(cs);
+        fb[i] = *reinterpret_cast<const float4*>(cs + 4);
+      }
+    }
+    uint8_t* const mine = pa_lds + BUF + wave * 32 * ROWB;
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int row = i * RPI + lane / LPR;
+      if (p.freqs) {  // what rope_kv_write_kernel does to the query heads: same bits
+        x[i] = rope8(x[i], fa[i], fb[i]);
+        if (p.q_gain)
+          x[i] = chunk_normed(x[i], rms_scale(head_sumsq<D>(x[i]), (float)D, p.eps), *reinterpret_cast<const uint4*>(p.q_gain + piece * 8));
+      }
+      *reinterpret_cast<uint4*>(mine + row * ROWB + ((piece ^ row_key<D>(row)) << 4)) = x[i];
+    }
+#pragma unroll
+    for (int st = 0; st < DSTEPS; ++st)
+      qf[st] = *reinterpret_cast<const uint4*>(mine + col * ROWB + (((2 * st + g) ^ row_key<D>(col)) << 4));
   }
   // fragment addresses inside a block: K row `col`, piece 2 step + g; V rows 4 g + i / 4 (and 8 further), i = lane % 16,
   // dimensions 16 (lane / 16 % 2) + 4 (i % 4) of a 32-dimension tile
@@ -462,9 +496,28 @@ static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
 
 }  // namespace aq
 
-extern "C" int aq_prefill_attn_causal_ahead(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
-                                      int64_t v_stride, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
-                                      int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
+namespace {
+struct Rotation {  // of the query heads as they are read; freqs null: they are rotated already
+  const float* freqs = nullptr;
+  int64_t freqs_stride = 0;
+  const void* q_gain = nullptr;
+  float eps = 0.0f;
+};
+int check_rotation(const Rotation& r, int64_t S, int64_t D) {
+  if ((r.freqs_stride != 0 && r.freqs_stride < S * D) || (r.q_gain && !(r.eps >= 0.0f))) return AQ_E_SHAPE;
+  return aq::check_ptr16(r.freqs) || (r.freqs_stride & 3) || aq::check_ptr16(r.q_gain) ? AQ_E_ALIGN : AQ_OK;
+}
+void set_rotation(aq::PrefillAttnArgs& a, const Rotation& r) {
+  a.freqs = r.freqs;
+  a.freqs_stride = r.freqs_stride;
+  a.q_gain = static_cast<const uint16_t*>(r.q_gain);
+  a.eps = r.eps;
+}
+}  // namespace
+
+static int prefill_attn_causal(const void* q, int64_t q_stride, const Rotation& rot, const void* k, int64_t k_stride, const void* v,
+                               int64_t v_stride, void* out, float scale, int64_t B, int64_t S, int64_t Hq, int64_t Hkv, int64_t D,
+                               const aq_span* ahead, int n_ahead, void* stream) {
   if (D != 64 && D != 128) return AQ_E_SHAPE;
   if (B < 0 || S < 0 || Hq <= 0 || Hkv <= 0 || (Hq % Hkv) != 0 || !(scale > 0.0f)) return AQ_E_SHAPE;
   if (q_stride < Hq * D || k_stride < Hkv * D || v_stride < Hkv * D) return AQ_E_SHAPE;
@@ -479,7 +532,9 @@ extern "C" int aq_prefill_attn_causal_ahead(const void* q, int64_t q_stride, con
   if ((S + 64) * k_stride * 2 > (int64_t)0x7fffffff || (S + 64) * v_stride * 2 > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
   if (const int rc = aq::check_spans(ahead, n_ahead)) return rc;
+  if (const int rc = check_rotation(rot, S, D)) return rc;
   aq::PrefillAttnArgs a{};
+  set_rotation(a, rot);
   a.ahead_wgs = aq::set_ahead(a.ahead, ahead, n_ahead);
   a.q = static_cast<const uint16_t*>(q);
   a.k = static_cast<const uint16_t*>(k);
@@ -497,13 +552,28 @@ extern "C" int aq_prefill_attn_causal_ahead(const void* q, int64_t q_stride, con
   return D == 128 ? aq::launch_prefill_attn<128, false>(a, st) : aq::launch_prefill_attn<64, false>(a, st);
 }
 
+extern "C" int aq_prefill_attn_causal_ahead(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                                            int64_t v_stride, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                            int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
+  return prefill_attn_causal(q, q_stride, Rotation{}, k, k_stride, v, v_stride, out, scale, B, S, Hq, Hkv, D, ahead, n_ahead, stream);
+}
+
+extern "C" int aq_rope_prefill_attn_causal_ahead(const void* q, int64_t q_stride, const float* freqs, int64_t freqs_stride,
+                                                 const void* q_gain, float eps, const void* k, int64_t k_stride, const void* v,
+                                                 int64_t v_stride, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                                 int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
+  if (!freqs && B > 0 && S > 0) return AQ_E_NULL;
+  return prefill_attn_causal(q, q_stride, Rotation{freqs, freqs_stride, q_gain, eps}, k, k_stride, v, v_stride, out, scale, B, S, Hq,
+                             Hkv, D, ahead, n_ahead, stream);
+}
+
 extern "C" int aq_prefill_attn_causal(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
                                       int64_t v_stride, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
                                       int64_t Hkv, int64_t D, void* stream) {
   return aq_prefill_attn_causal_ahead(q, q_stride, k, k_stride, v, v_stride, out, scale, B, S, Hq, Hkv, D, nullptr, 0, stream);
 }
 
-extern "C" int aq_prefill_attn_paged_ahead(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+static int prefill_attn_paged(const void* q, int64_t q_stride, const Rotation& rot, const void* k_cache, const void* v_cache,
                                      const int64_t* page_table, int64_t P, int64_t start, int64_t page_size,
                                      int64_t n_pages, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
                                      int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
@@ -521,7 +591,9 @@ extern "C" int aq_prefill_attn_paged_ahead(const void* q, int64_t q_stride, cons
       ((S + 31) / 32) * Hq * B > (int64_t)0x7fffffff)
     return AQ_E_RANGE;
   if (const int rc = aq::check_spans(ahead, n_ahead)) return rc;
+  if (const int rc = check_rotation(rot, S, D)) return rc;
   aq::PrefillAttnArgs a{};
+  set_rotation(a, rot);
   a.ahead_wgs = aq::set_ahead(a.ahead, ahead, n_ahead);
   a.q = static_cast<const uint16_t*>(q);
   a.out = static_cast<uint16_t*>(out);
@@ -543,6 +615,24 @@ extern "C" int aq_prefill_attn_paged_ahead(const void* q, int64_t q_stride, cons
   a.B = (int)B;
   hipStream_t st = static_cast<hipStream_t>(stream);
   return D == 128 ? aq::launch_prefill_attn<128, true>(a, st) : aq::launch_prefill_attn<64, true>(a, st);
+}
+
+extern "C" int aq_prefill_attn_paged_ahead(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+                                           const int64_t* page_table, int64_t P, int64_t start, int64_t page_size,
+                                           int64_t n_pages, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                           int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
+  return prefill_attn_paged(q, q_stride, Rotation{}, k_cache, v_cache, page_table, P, start, page_size, n_pages, out, scale, B, S, Hq,
+                            Hkv, D, ahead, n_ahead, stream);
+}
+
+extern "C" int aq_rope_prefill_attn_paged_ahead(const void* q, int64_t q_stride, const float* freqs, int64_t freqs_stride,
+                                                const void* q_gain, float eps, const void* k_cache, const void* v_cache,
+                                                const int64_t* page_table, int64_t P, int64_t start, int64_t page_size,
+                                                int64_t n_pages, void* out, float scale, int64_t B, int64_t S, int64_t Hq,
+                                                int64_t Hkv, int64_t D, const aq_span* ahead, int n_ahead, void* stream) {
+  if (!freqs && B > 0 && S > 0) return AQ_E_NULL;
+  return prefill_attn_paged(q, q_stride, Rotation{freqs, freqs_stride, q_gain, eps}, k_cache, v_cache, page_table, P, start, page_size,
+                            n_pages, out, scale, B, S, Hq, Hkv, D, ahead, n_ahead, stream);
 }
 
 extern "C" int aq_prefill_attn_paged(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,

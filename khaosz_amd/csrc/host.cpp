@@ -50,8 +50,7 @@ namespace {
   X(aq_gemv_w8a8_decode_attn)                                                                                    \
   X(aq_gemv_fp8_workspace_bytes)                                                                                 \
   X(aq_gemv_fp8_decode_residual)                                                                                 \
-  X(aq_rope_kv_write)                                                                                            \
-  X(aq_rope_kv_write_qknorm)                                                                                     \
+  X(aq_rope_kv_cache_write)                                                                                      \
   X(aq_rope_paged_attn_decode)                                                                                   \
   X(aq_rope_paged_attn_decode_qknorm)                                                                            \
   X(aq_rope_paged_attn_decode_partials)                                                                          \
@@ -59,8 +58,8 @@ namespace {
   X(aq_paged_attn_decode_slices)                                                                                 \
   X(aq_paged_attn_decode_partials_bytes)                                                                         \
   X(aq_paged_attn_decode_workspace_bytes)                                                                        \
-  X(aq_prefill_attn_causal_ahead)                                                                                \
-  X(aq_prefill_attn_paged_ahead)
+  X(aq_rope_prefill_attn_causal_ahead)                                                                           \
+  X(aq_rope_prefill_attn_paged_ahead)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -763,7 +762,7 @@ struct Block {
   Gain n1, n2, qn, kn;
 
   // the intermediate results' places in the scratch memory, `most` bytes
-  size_t x1, sx, qkv_rows, att, codes, q, k, parts, up_gate, h_codes, most;
+  size_t x1, sx, qkv_rows, att, codes, k, parts, up_gate, h_codes, most;
   int64_t parts_bytes;
 
   bool read(PyObject* block, PyObject* x, PyObject* rotary, PyObject* cache);
@@ -855,7 +854,7 @@ void Block::lay_out() {
   // attention
   qkv_rows = m.take(2 * M * qkv.N), att = m.take(2 * M * A);
   codes = m.take(few() ? lib.aq_gemv_w8a8_workspace_bytes(M, longest) : static_cast<size_t>(M * longest));
-  q = step() ? 0 : m.take(2 * M * A), k = step() || !direct ? 0 : m.take(2 * M * KV);
+  k = step() || !direct ? 0 : m.take(2 * M * KV);
   parts_bytes = !step()   ? 0
                 : merge() ? lib.aq_paged_attn_decode_partials_bytes(B, Hq, total)
                           : lib.aq_paged_attn_decode_workspace_bytes(B, Hq, Hkv, total);
@@ -928,21 +927,23 @@ int Block::queue(const void* in, void* out, char* base, const char** what) const
       rc = projected(o, att, in, x1, codes);
     }
   } else {
-    char *qr = base + this->q, *kr = direct ? base + k : nullptr;
-    *what = "aq_rope_kv_write";
-    rc = qk_norm ? lib.aq_rope_kv_write_qknorm(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, qr, kr, B, Hq, Hkv, D, qn.p,
-                                               kn.p, qn.eps, c.stream)
-                 : lib.aq_rope_kv_write(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, qr, kr, B, Hq, Hkv, D, c.stream);
+    // attention rotates its queries as it reads them from the projection's rows
+    char* kr = direct ? base + k : nullptr;
+    const void *qg = qk_norm ? qn.p : nullptr, *kg = qk_norm ? kn.p : nullptr;
+    *what = "aq_rope_kv_cache_write";
+    rc = lib.aq_rope_kv_cache_write(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, kr, B, Hq, Hkv, D, kg, qn.eps,
+                                    c.stream);
     if (rc) return rc;
     // what streams behind attention, which itself leaves HBM idle
     const aq_span ahead[3] = {{o.w, o.N * o.K}, {ug.w, ug.N * ug.K}, {down.w, down.N * down.K}};
     if (direct) {
-      *what = "aq_prefill_attn_causal";
-      rc = lib.aq_prefill_attn_causal_ahead(qr, A, kr, KV, q + 2 * (A + KV), W, att, scale, B, S, Hq, Hkv, D, ahead, 3, c.stream);
+      *what = "aq_rope_prefill_attn_causal";
+      rc = lib.aq_rope_prefill_attn_causal_ahead(q, W, fr, fr_stride, qg, qn.eps, kr, KV, q + 2 * (A + KV), W, att, scale, B, S, Hq, Hkv, D,
+                                                 ahead, 3, c.stream);
     } else {
-      *what = "aq_prefill_attn_paged";
-      rc = lib.aq_prefill_attn_paged_ahead(qr, A, kc, vc, table, P, total - S, page, n_pages, att, scale, B, S, Hq, Hkv, D, ahead, 3,
-                                           c.stream);
+      *what = "aq_rope_prefill_attn_paged";
+      rc = lib.aq_rope_prefill_attn_paged_ahead(q, W, fr, fr_stride, qg, qn.eps, kc, vc, table, P, total - S, page, n_pages, att, scale, B,
+                                                S, Hq, Hkv, D, ahead, 3, c.stream);
     }
     if (rc) return rc;
     rc = projected(o, att, in, x1, codes);

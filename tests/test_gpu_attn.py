@@ -533,3 +533,45 @@ def test_prefill_attn_reading_ahead_changes_nothing():
             assert torch.equal(out, want)
     assert lib.aq_prefill_attn_causal_ahead(q.data_ptr(), Hq * 64, k.data_ptr(), Hkv * 64, v.data_ptr(), Hkv * 64, out.data_ptr(),
                                             0.125, B, S, Hq, Hkv, 64, None, 2, 0) != 0
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,start,Hq,Hkv,page,shared", [(1, 1, 0, 1, 1, 64, True), (3, 21, 0, 4, 2, 8, False), (2, 130, 0, 6, 2, 64, True),
+                                                          (1, 33, 31, 4, 4, 32, True), (2, 300, 100, 24, 4, 128, False), (4, 512, 0, 16, 4, 64, True)])
+def test_prefill_attn_that_rotates_its_queries_gives_the_bits_of_two_launches(B, S, start, Hq, Hkv, page, shared, D, norm):
+    """aq_rope_kv_cache_write + the attention that reads queries from the projection's rows, against rope_kv_write + the
+    attention on rotated queries: caches and outputs, on every number of wavefronts per query row."""
+    from khaosz_amd import _abi
+
+    _say("prefill_attn rotates q", B, S, start, Hq, Hkv, page, shared, D, norm)
+    g = torch.Generator().manual_seed(S + D)
+    P = (start + S + page - 1) // page
+    n_pages, W = B * P + 2, (Hq + 2 * Hkv) * D
+    qkv = torch.randn(B, S, W, generator=g).to(torch.bfloat16).to(DEV)
+    ang = torch.rand(1 if shared else B, S, D // 2, generator=g) * 6.28
+    freqs = torch.polar(torch.ones_like(ang), ang).to(DEV)
+    table = torch.randperm(n_pages, generator=g)[:B * P].view(B, P).to(DEV)
+    if B > 2:
+        table[1, -1] = -1
+    kc, vc = (torch.randn(n_pages, page, Hkv, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    qk = ops.QkNorm(*(torch.rand(D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2)), 1e-5) if norm else None
+    k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+    q, k = ops.rope_kv_write(qkv, freqs.expand(B, -1, -1), table, start, k1, v1, Hq, Hkv, return_k=True, qk_norm=qk)
+    v = qkv[..., (Hq + Hkv) * D:].view(B, S, Hkv, D)
+    want = [ops.prefill_attn_paged(q, k1, v1, table, start)] + ([ops.prefill_attn_causal(q, k, v)] if start == 0 else [])
+    lib, st = _abi.load(), torch.cuda.current_stream().cuda_stream
+    fr, stride = torch.view_as_real(freqs).contiguous(), 0 if shared else S * D
+    qg, kg, eps = (qk[0].data_ptr(), qk[1].data_ptr(), qk[2]) if norm else (None, None, 0.0)
+    kd = torch.empty_like(k)
+    assert lib.aq_rope_kv_cache_write(qkv.data_ptr(), fr.data_ptr(), stride, table.data_ptr(), P, start, S, page, k2.data_ptr(), v2.data_ptr(),
+                                      n_pages, kd.data_ptr(), B, Hq, Hkv, D, kg, eps, st) == 0
+    assert torch.equal(kd, k) and torch.equal(k2, k1) and torch.equal(v2, v1)
+    out = torch.empty_like(q)
+    assert lib.aq_rope_prefill_attn_paged_ahead(qkv.data_ptr(), W, fr.data_ptr(), stride, qg, eps, k2.data_ptr(), v2.data_ptr(), table.data_ptr(),
+                                                P, start, page, n_pages, out.data_ptr(), D ** -0.5, B, S, Hq, Hkv, D, None, 0, st) == 0
+    assert torch.equal(out, want[0])
+    if start == 0:
+        assert lib.aq_rope_prefill_attn_causal_ahead(qkv.data_ptr(), W, fr.data_ptr(), stride, qg, eps, k.data_ptr(), Hkv * D, v.data_ptr(), W,
+                                                     out.data_ptr(), D ** -0.5, B, S, Hq, Hkv, D, None, 0, st) == 0
+        assert torch.equal(out, want[1])
