@@ -56,7 +56,7 @@ struct PrefillAttnArgs {
   const int64_t* table;  // [B, P] physical page ids, < 0: unmapped (zero keys and values)
   int64_t P, page, n_pages;
   int start, page_shift;
-  // freqs != null: q holds heads as the projection left them, which are rotated (and, with q_gain, RMS-normalised) as they are read
+  // ROT kernels:
   const float* freqs;    // [S, D/2, 2] (cos, sin) per sequence; sequences freqs_stride floats apart (0: shared)
   int64_t freqs_stride;
   const uint16_t* q_gain;
@@ -96,7 +96,8 @@ __device__ __forceinline__ int row_key(int row) {
 
 // PAGED: a chunk of S new tokens on top of `start` cached ones -- K and V of all start + S positions come from the
 // paged cache (the new tokens' rows have been written there already), causality is by position.
-template <int D, int QW, int KW, bool PAGED>
+// ROT: q holds heads as the projection left them; they are rotated (and, with q_gain, RMS-normalised) as they are read.
+template <int D, int QW, int KW, bool PAGED, bool ROT>
 __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(PrefillAttnArgs p) {
   if ((int)blockIdx.x >= p.wgs) return read_ahead(p.ahead, (int)blockIdx.x - p.wgs, QW * KW * 64);
   constexpr int QB = 32 * QW;                       // query rows of the workgroup
@@ -212,12 +213,17 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
   };
   issue(0, 0);
 
-  // The wavefront's 32 query rows, whole rows at a time, through the second buffer (nothing is requested into it before the first
-  // barrier) to the lanes that take them: Q^T operand, lane = (query col, dimensions 16 step + 8 g .. + 8); rows past S read
-  // row S - 1.  (A lane reading its own query's pieces touches a line with every piece, of the rotary table
-  // too: 3.5 us of 25 at 8 x 512 x 16 heads of 128.)
+  // Q^T operand: lane = (query col, dimensions 16 step + 8 g .. + 8); rows past S read row S - 1
   uint4 qf[DSTEPS];
-  {
+  if constexpr (!ROT) {
+    const int qr = qpos < S ? qpos : S - 1;
+    const uint16_t* src = p.q + (tok0 + qr) * p.q_stride + (int64_t)h * D + g * 8;
+#pragma unroll
+    for (int st = 0; st < DSTEPS; ++st) qf[st] = *reinterpret_cast<const uint4*>(src + st * 16);
+  } else {
+    // whole rows at a time, through the second buffer (nothing is requested into it before the first barrier) to the lanes that
+    // take them.  (A lane reading its own query's pieces touches a line with every piece, of the rotary table too: 3.5 us of 25
+    // at 8 x 512 x 16 heads of 128.)  Same bits as rope_kv_write_kernel's.
     constexpr int NQ = 32 / RPI;
     static_assert(QW * KW * 32 * ROWB <= BUF, "the queries fit a buffer");
     const int piece = lane % LPR;
@@ -226,22 +232,18 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
       const int r = qw0 + i * RPI + lane / LPR, qr = r < S ? r : S - 1;
+      const float* cs = p.freqs + (int64_t)b * p.freqs_stride + (int64_t)qr * D + piece * 8;
       x[i] = *reinterpret_cast<const uint4*>(p.q + (tok0 + qr) * p.q_stride + (int64_t)h * D + piece * 8);
-      if (p.freqs) {  // uniform
-        const float* cs = p.freqs + (int64_t)b * p.freqs_stride + (int64_t)qr * D + piece * 8;
-        fa[i] = *reinterpret_cast<const float4*>(cs);
-        fb[i] = *reinterpret_cast<const float4*>(cs + 4);
-      }
+      fa[i] = *reinterpret_cast<const float4*>(cs);
+      fb[i] = *reinterpret_cast<const float4*>(cs + 4);
     }
     uint8_t* const mine = pa_lds + BUF + wave * 32 * ROWB;
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
       const int row = i * RPI + lane / LPR;
-      if (p.freqs) {  // what rope_kv_write_kernel does to the query heads: same bits
-        x[i] = rope8(x[i], fa[i], fb[i]);
-        if (p.q_gain)
-          x[i] = chunk_normed(x[i], rms_scale(head_sumsq<D>(x[i]), (float)D, p.eps), *reinterpret_cast<const uint4*>(p.q_gain + piece * 8));
-      }
+      x[i] = rope8(x[i], fa[i], fb[i]);
+      if (p.q_gain)  // uniform
+        x[i] = chunk_normed(x[i], rms_scale(head_sumsq<D>(x[i]), (float)D, p.eps), *reinterpret_cast<const uint4*>(p.q_gain + piece * 8));
       *reinterpret_cast<uint4*>(mine + row * ROWB + ((piece ^ row_key<D>(row)) << 4)) = x[i];
     }
 #pragma unroll
@@ -443,7 +445,7 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
 constexpr int PA_TABLE_MAX = 2048;                         // page-table entries kept in LDS
 constexpr int LDS_BYTES = 160 * 1024, STATIC_LDS = 1536;  // of a compute unit; of a workgroup beside its buffers, at most
 
-template <int D, int QW, int KW, bool PAGED>
+template <int D, int QW, int KW, bool PAGED, bool ROT>
 static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
   const int64_t wgs = ((int64_t)(a.S + 32 * QW - 1) / (32 * QW)) * a.Hq * a.B;
   a.wgs = (int)wgs;
@@ -454,7 +456,7 @@ static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
     a.table_lds = a.page % KB != 0 && entries <= PA_TABLE_MAX ? (int)entries : 0;
     lds += (size_t)a.table_lds * sizeof(int);
   }
-  constexpr auto kernel = prefill_attn_kernel<D, QW, KW, PAGED>;
+  constexpr auto kernel = prefill_attn_kernel<D, QW, KW, PAGED, ROT>;
   // Workgroups that the device holds at once.  Registers decide at head dimension 64 with one wavefront per query row (124
   // and 128 of them: four, where the buffers would allow five), the buffers elsewhere; a page table in LDS may cost another.
   // Launches of four to five workgroups per compute unit, numbered as if resident -> heaviest first, us: 4 x 1408 x 24 heads
@@ -483,15 +485,21 @@ static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
 // cached 29 | 22 | 16, 500 on 1500 36 | 27 | 32; head dimension 128, 16 heads (1 | 2): 1 x 1000 23 | 18, 4 x 300
 // 10.2 | 11.0, 64 on 1500 38 | 28.  Before, with keys staged through registers, one wavefront per query row and a page
 // lookup per row: 7.7, 12.4, 34, 48, 61; 27.5, 11.8, 76.
-template <int D, bool PAGED>
+template <int D, bool PAGED, bool ROT>
 static int launch_prefill_attn(PrefillAttnArgs& a, hipStream_t st) {
   const int64_t heads = (int64_t)a.Hq * a.B, cus = device_cus(), T = (PAGED ? a.start : 0) + (int64_t)a.S;
   const int64_t q32 = (a.S + 31) / 32 * heads, q64 = (a.S + 63) / 64 * heads;
   if constexpr (D == 64) {
-    if (q32 <= cus) return launch_prefill_attn<D, 1, 4, PAGED>(a, st);
+    if (q32 <= cus) return launch_prefill_attn<D, 1, 4, PAGED, ROT>(a, st);
   }
-  if (T > 128 && q64 <= (D == 128 ? 1 : T < 1024 ? 2 : 4) * cus) return launch_prefill_attn<D, 2, 2, PAGED>(a, st);
-  return launch_prefill_attn<D, 4, 1, PAGED>(a, st);
+  if (T > 128 && q64 <= (D == 128 ? 1 : T < 1024 ? 2 : 4) * cus) return launch_prefill_attn<D, 2, 2, PAGED, ROT>(a, st);
+  return launch_prefill_attn<D, 4, 1, PAGED, ROT>(a, st);
+}
+
+template <bool PAGED>
+static int launch_prefill_attn(PrefillAttnArgs& a, int64_t D, hipStream_t st) {
+  if (a.freqs) return D == 128 ? launch_prefill_attn<128, PAGED, true>(a, st) : launch_prefill_attn<64, PAGED, true>(a, st);
+  return D == 128 ? launch_prefill_attn<128, PAGED, false>(a, st) : launch_prefill_attn<64, PAGED, false>(a, st);
 }
 
 }  // namespace aq
@@ -549,7 +557,7 @@ static int prefill_attn_causal(const void* q, int64_t q_stride, const Rotation& 
   a.Hkv = (int)Hkv;
   a.B = (int)B;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return D == 128 ? aq::launch_prefill_attn<128, false>(a, st) : aq::launch_prefill_attn<64, false>(a, st);
+  return aq::launch_prefill_attn<false>(a, D, st);
 }
 
 extern "C" int aq_prefill_attn_causal_ahead(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
@@ -614,7 +622,7 @@ static int prefill_attn_paged(const void* q, int64_t q_stride, const Rotation& r
   a.Hkv = (int)Hkv;
   a.B = (int)B;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return D == 128 ? aq::launch_prefill_attn<128, true>(a, st) : aq::launch_prefill_attn<64, true>(a, st);
+  return aq::launch_prefill_attn<true>(a, D, st);
 }
 
 extern "C" int aq_prefill_attn_paged_ahead(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,

@@ -50,6 +50,8 @@ namespace {
   X(aq_gemv_w8a8_decode_attn)                                                                                    \
   X(aq_gemv_fp8_workspace_bytes)                                                                                 \
   X(aq_gemv_fp8_decode_residual)                                                                                 \
+  X(aq_rope_kv_write)                                                                                            \
+  X(aq_rope_kv_write_qknorm)                                                                                     \
   X(aq_rope_kv_cache_write)                                                                                      \
   X(aq_rope_paged_attn_decode)                                                                                   \
   X(aq_rope_paged_attn_decode_qknorm)                                                                            \
@@ -58,6 +60,8 @@ namespace {
   X(aq_paged_attn_decode_slices)                                                                                 \
   X(aq_paged_attn_decode_partials_bytes)                                                                         \
   X(aq_paged_attn_decode_workspace_bytes)                                                                        \
+  X(aq_prefill_attn_causal_ahead)                                                                                \
+  X(aq_prefill_attn_paged_ahead)                                                                                 \
   X(aq_rope_prefill_attn_causal_ahead)                                                                           \
   X(aq_rope_prefill_attn_paged_ahead)
 
@@ -762,13 +766,18 @@ struct Block {
   Gain n1, n2, qn, kn;
 
   // the intermediate results' places in the scratch memory, `most` bytes
-  size_t x1, sx, qkv_rows, att, codes, k, parts, up_gate, h_codes, most;
+  size_t x1, sx, qkv_rows, att, codes, q, k, parts, up_gate, h_codes, most;
   int64_t parts_bytes;
 
   bool read(PyObject* block, PyObject* x, PyObject* rotary, PyObject* cache);
   void lay_out();
   bool few() const { return M <= types.decode_rows; }
   bool step() const { return S == 1; }
+  // Whether a prompt's attention rotates its queries itself: from 8 MB of them on, which then are not written and read back.  With
+  // less, the launch that rotates takes the same few microseconds whatever it moves, and rotating is one more link in the attention
+  // launch's chain: us a block, rotated before -> in attention: 8 x 512 tokens of 16 heads of 128 (16.8 MB) 274.4 -> 270.7; 24 layers:
+  // 4 x 512 of 24 heads of 64 (6.3 MB) 3703 -> 3687, 2 x 150 (0.9 MB) 1680 -> 1706; 2 x 82 on 21 cached, qk-norm (0.7 MB) 58.9 -> 61.9.
+  bool rotates() const { return !step() && M * Hq * D >= (int64_t(4) << 20); }
   bool merge() const { return step() && merge_in_projection(B, Hq * D, total); }
   int queue(const void* in, void* out, char* base, const char** what) const;  // allocates nothing: runs without the interpreter lock
 };
@@ -854,7 +863,7 @@ void Block::lay_out() {
   // attention
   qkv_rows = m.take(2 * M * qkv.N), att = m.take(2 * M * A);
   codes = m.take(few() ? lib.aq_gemv_w8a8_workspace_bytes(M, longest) : static_cast<size_t>(M * longest));
-  k = step() || !direct ? 0 : m.take(2 * M * KV);
+  q = step() || rotates() ? 0 : m.take(2 * M * A), k = step() || !direct ? 0 : m.take(2 * M * KV);
   parts_bytes = !step()   ? 0
                 : merge() ? lib.aq_paged_attn_decode_partials_bytes(B, Hq, total)
                           : lib.aq_paged_attn_decode_workspace_bytes(B, Hq, Hkv, total);
@@ -927,23 +936,30 @@ int Block::queue(const void* in, void* out, char* base, const char** what) const
       rc = projected(o, att, in, x1, codes);
     }
   } else {
-    // attention rotates its queries as it reads them from the projection's rows
-    char* kr = direct ? base + k : nullptr;
+    char *qr = base + this->q, *kr = direct ? base + k : nullptr;
     const void *qg = qk_norm ? qn.p : nullptr, *kg = qk_norm ? kn.p : nullptr;
-    *what = "aq_rope_kv_cache_write";
-    rc = lib.aq_rope_kv_cache_write(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, kr, B, Hq, Hkv, D, kg, qn.eps,
-                                    c.stream);
+    const bool late = rotates();
+    *what = "aq_rope_kv_write";
+    rc = late ? lib.aq_rope_kv_cache_write(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, kr, B, Hq, Hkv, D, kg, qn.eps,
+                                           c.stream)
+         : qk_norm ? lib.aq_rope_kv_write_qknorm(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, qr, kr, B, Hq, Hkv, D, qg,
+                                                 kg, qn.eps, c.stream)
+                   : lib.aq_rope_kv_write(q, fr, fr_stride, table, P, total - S, S, page, kc, vc, n_pages, qr, kr, B, Hq, Hkv, D, c.stream);
     if (rc) return rc;
     // what streams behind attention, which itself leaves HBM idle
     const aq_span ahead[3] = {{o.w, o.N * o.K}, {ug.w, ug.N * ug.K}, {down.w, down.N * down.K}};
     if (direct) {
-      *what = "aq_rope_prefill_attn_causal";
-      rc = lib.aq_rope_prefill_attn_causal_ahead(q, W, fr, fr_stride, qg, qn.eps, kr, KV, q + 2 * (A + KV), W, att, scale, B, S, Hq, Hkv, D,
-                                                 ahead, 3, c.stream);
+      *what = "aq_prefill_attn_causal";
+      const char* v = q + 2 * (A + KV);
+      rc = late ? lib.aq_rope_prefill_attn_causal_ahead(q, W, fr, fr_stride, qg, qn.eps, kr, KV, v, W, att, scale, B, S, Hq, Hkv, D, ahead,
+                                                        3, c.stream)
+                : lib.aq_prefill_attn_causal_ahead(qr, A, kr, KV, v, W, att, scale, B, S, Hq, Hkv, D, ahead, 3, c.stream);
     } else {
-      *what = "aq_rope_prefill_attn_paged";
-      rc = lib.aq_rope_prefill_attn_paged_ahead(q, W, fr, fr_stride, qg, qn.eps, kc, vc, table, P, total - S, page, n_pages, att, scale, B,
-                                                S, Hq, Hkv, D, ahead, 3, c.stream);
+      *what = "aq_prefill_attn_paged";
+      rc = late ? lib.aq_rope_prefill_attn_paged_ahead(q, W, fr, fr_stride, qg, qn.eps, kc, vc, table, P, total - S, page, n_pages, att,
+                                                       scale, B, S, Hq, Hkv, D, ahead, 3, c.stream)
+                : lib.aq_prefill_attn_paged_ahead(qr, A, kc, vc, table, P, total - S, page, n_pages, att, scale, B, S, Hq, Hkv, D, ahead, 3,
+                                                  c.stream);
     }
     if (rc) return rc;
     rc = projected(o, att, in, x1, codes);
