@@ -100,9 +100,11 @@ template <bool FP8, int OUT>
 int gemm_slices_launch(GemmArgs& a, int tm, hipStream_t st);
 
 // gemm_walk.hip
-bool gemm_walk_ok(const GemmArgs& a);
-template <bool FP8>
-int gemm_walk_launch(const GemmArgs& a, hipStream_t st);
+// The last round of 256 x 128 tiles is cut in two behind three rounds or more, when at most half the compute units have a tile in it.
+inline bool gemm_walk_halves(int64_t tiles, int64_t cus) { return tiles % cus != 0 && tiles % cus <= cus / 2 && tiles >= 3 * cus; }
+bool gemm_walk_ok(const GemmArgs& a, int out);
+template <bool FP8, int OUT>
+int gemm_walk_launch(const GemmArgs& a, hipStream_t st, int width);
 
 }  // namespace aq
 

@@ -17,9 +17,9 @@
 // later sub-steps are issued between the MFMAs of the current one, with one
 // workgroup barrier per K step.  The epilogue is fused and runs straight from
 // the accumulator registers: int32 store, or dequantise (+bias) and cast.
-// Two other kernels take calls from here: gemm_walk.hip the 256 x 128 tiles of
-// several rounds or with a residual (bf16 outputs), gemm_slices.hip a few dozen
-// to a few hundred rows.
+// Two other kernels take calls from here: gemm_walk.hip the 256 x 128 and
+// 256 x 192 tiles of K from 512 (even N), gemm_slices.hip a few dozen to a few
+// hundred rows.
 #include "aq_gemm.h"
 
 namespace aq {
@@ -748,33 +748,49 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
 // 33..2048 rows against N = 1024..16384 and K = 1024..5632, where the rule picks the fastest shape or one within
 // 6 % of it.  The small tiles are for launches of a few rounds only.
 enum TileKind {
-  TILE_AUTO = 0, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129,
-  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_SLICES32 = 34, TILE_SLICES64 = 35
+  TILE_AUTO = 0, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129, TILE_WIDE = 192,
+  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258, TILE_SLICES32 = 34, TILE_SLICES64 = 35
 };
 #ifdef AQ_LAB
 static int g_forced_tile = 0;  // lab build only: TILE_AUTO = by shape, otherwise forced (tuning and tests)
 #endif
 
-static int choose_tile_for(int64_t M, int64_t N, int64_t cus) {
-  auto rounds = [cus](int64_t tiles) {
+// Where gemm_walk_kernel can take the call, its tiles stand for the 256 x 128 one: that at the same cost of a round but less of a
+// last one (0.7 + 0.1 of its fill; 0.55 where its tiles are cut in two), and 256 x 192 at 1.45 of a round (last 0.7 + 0.2): with
+// five fragments read and 56 KiB brought in for three columns of products, where 256 x 128 has four and 48 for two, it is the
+// faster one, by up to a third, where it saves a round or most of one.  Measured over 470 random sizes of 300..8192 rows, N
+// 512..11264, K 512..8192, int8 and FP8, on several cards: what this picks is 0.2 % from the faster of the two in the mean, 7 % at
+// most but for one size in a hundred (256 x 128 alone: 5 %, 43 %).  us, gemm_kernel's tiles -> 256 x 192 (256 x 128 of the walk):
+// 4096 x 3072 x 2048 31.5 -> 25.2 (30.2), FP8 27.6 -> 22.8 (27.5), 1476 x 6480 x 4448 72.5 -> 49.2 (69), 6263 x 1456 x 3696 63 -> 42.8
+// (59), 6952 x 1232 x 992 with a residual 30.2 -> 17.7 (26), FP8 2954 x 11104 x 4000 172 -> 142 (172); not 4096 x 11264 x 2048 (95, 109).
+static int choose_tile_for(int64_t M, int64_t N, int64_t cus, bool walk = false) {
+  auto rounds = [cus](int64_t tiles, double last, double fill) {
     const int64_t full = tiles / cus, rest = tiles % cus;
     if (full == 0) return 1.0;
-    return (double)full + (rest ? 0.5 + 0.5 * (double)rest / cus : 0.0);
+    return (double)full + (rest ? last + fill * (double)rest / cus : 0.0);
   };
   struct Cand {
     int kind, bm, bn;
     double round_us;
     bool small;
+    double last, fill;  // of a round, for a last one behind others
   };
-  static const Cand cands[] = {{TILE_LARGE, 256, 128, 15.0, false}, {TILE_SMALL, 128, 128, 10.8, false},
-                               {TILE_N64, 128, 64, 7.0, true},      {TILE_N32, 128, 32, 5.0, true},
-                               {TILE_M64N64, 64, 64, 4.6, true},    {TILE_M64N32, 64, 32, 3.5, true}};
+  static const Cand cands[] = {{TILE_LARGE, 256, 128, 15.0, false, 0.5, 0.5}, {TILE_SMALL, 128, 128, 10.8, false, 0.5, 0.5},
+                               {TILE_N64, 128, 64, 7.0, true, 0, 0},          {TILE_N32, 128, 32, 5.0, true, 0, 0},
+                               {TILE_M64N64, 64, 64, 4.6, true, 0, 0},        {TILE_M64N32, 64, 32, 3.5, true, 0, 0},
+                               {TILE_WIDE, 256, 192, 21.75, false, 0.7, 0.2}};
   int best = TILE_LARGE;
   double cost = 0.0;
   for (const Cand& c : cands) {
+    if (c.kind == TILE_WIDE && !walk) continue;
     const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
     if (c.small && tiles > 4 * cus) continue;
-    const double us = c.round_us * (c.small ? (double)((tiles + cus - 1) / cus) : rounds(tiles));
+    double last = c.last, fill = c.fill;
+    if (c.kind == TILE_LARGE && walk) {
+      const bool halves = gemm_walk_halves(tiles, cus);
+      last = halves ? 0.55 : 0.7, fill = halves ? 0.0 : 0.1;
+    }
+    const double us = c.round_us * (c.small ? (double)((tiles + cus - 1) / cus) : rounds(tiles, last, fill));
     if (c.kind == TILE_LARGE || us < cost) {
       cost = us;
       best = c.kind;
@@ -783,11 +799,11 @@ static int choose_tile_for(int64_t M, int64_t N, int64_t cus) {
   return best;
 }
 
-static int choose_tile(int64_t M, int64_t N) {
+static int choose_tile(int64_t M, int64_t N, bool walk) {
 #ifdef AQ_LAB
   if (g_forced_tile) return g_forced_tile;
 #endif
-  return choose_tile_for(M, N, device_cus());
+  return choose_tile_for(M, N, device_cus(), walk);
 }
 
 template <bool FP8, int OUT, class S>
@@ -804,9 +820,11 @@ static int launch_shape(GemmArgs& a, hipStream_t st) {
 
 // FP8 launches the 256 x 256 tile serves and gains on: whole 256-row multiples, even N, whole 64-byte K steps, no
 // residual (the tile's one K-loop and epilogue variant), and at least two rounds of such tiles over the compute
-// units (one round -- 4096^3 -- measured level with the 256 x 128 tile, 57.0 against 57.7 us).
+// units (one round -- 4096^3 -- measured level with the 256 x 128 tile, 57.0 against 57.7 us) of more than 2048 in K: its loop
+// stops between tiles, gemm_walk_kernel's does not.  us, this | that: 8192^3 432 | 461, 4096 x 8192 x 4096 117 | 122,
+// 4096 x 11264 x 2048 90.7 | 91.5, 8192 x 4096 x 2048 63.8 | 60.8, 8192 x 6912 x 1536 93.6 | 82.1, 4096 x 8192 x 1024 39.8 | 36.2.
 static bool huge_fp8_ok(const GemmArgs& a) {
-  if ((a.K % ShapeHuge::BK) != 0 || (a.N % 2) != 0 || (a.M % ShapeHuge::BM) != 0 || a.res != nullptr) return false;
+  if (a.K <= 2048 || (a.K % ShapeHuge::BK) != 0 || (a.N % 2) != 0 || (a.M % ShapeHuge::BM) != 0 || a.res != nullptr) return false;
   const int64_t tiles = (int64_t)(a.M / ShapeHuge::BM) * ((a.N + ShapeHuge::BN - 1) / ShapeHuge::BN);
   return tiles >= 2 * (int64_t)device_cus();
 }
@@ -821,9 +839,14 @@ static int launch(GemmArgs& a, hipStream_t st) {
   if constexpr (FP8 && OUT != OUT_I32) {
     if (!forced && huge_fp8_ok(a)) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
   }
-  const int tile = choose_tile(a.M, a.N);
-  if constexpr (OUT == OUT_BF16) {  // many tiles, or a residual: the kernel whose K loop goes on from tile to tile
-    if (!forced && tile == TILE_LARGE && gemm_walk_ok(a)) return gemm_walk_launch<FP8>(a, st);
+  const bool walk = OUT != OUT_I32 && gemm_walk_ok(a, OUT);
+  const int tile = choose_tile(a.M, a.N, walk);
+  if constexpr (OUT != OUT_I32) {
+    if (walk && tile == TILE_LARGE && !forced) return gemm_walk_launch<FP8, OUT>(a, st, 128);
+    if (walk && tile == TILE_WIDE) return gemm_walk_launch<FP8, OUT>(a, st, 192);
+#ifdef AQ_LAB
+    if (walk && tile == TILE_WALK) return gemm_walk_launch<FP8, OUT>(a, st, 128);
+#endif
   }
   if constexpr (OUT != OUT_I32) {
     const int tm = forced ? (tile == TILE_SLICES32 ? 1 : tile == TILE_SLICES64 ? 2 : 0) : gemm_slices_rows(a.M, a.N, a.K);
@@ -878,7 +901,7 @@ extern "C" int aq_lab_read_clock(long long* host2) {
   return (int)hipMemcpyFromSymbol(host2, HIP_SYMBOL(aq::aq_lab_clock), 64);
 }
 extern "C" int aq_lab_set_gemm_tile(int rows) {
-  if (rows != 34 && rows != 35 && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
+  if (rows != 192 && rows != 258 && rows != 34 && rows != 35 && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
   aq::g_forced_tile = rows;
   return AQ_OK;
 }

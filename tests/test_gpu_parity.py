@@ -1426,3 +1426,29 @@ def test_gemm_with_k_cut_among_wavefronts(oracle, M, N, K, kind):
         y = ops.linear_fp8(x8.view(torch.uint8), d[1][:1], w8.view(torch.uint8), d[3][:1], d[4], out_dtype=torch.float32)
         want = (x8.float().cpu().double() @ w8.float().cpu().double().T) * float(sx[0]) * float(sw[0]) + torch.from_numpy(b).double()
         assert torch.allclose(y.cpu().double(), want, rtol=1e-3, atol=1e-4 * want.abs().max().item())
+
+
+# Both tiles of the walk: less than a tile, edges of a tile and of a K step, one round and several (whole and halved at their end)
+@pytest.mark.parametrize("kind", [192, 258])
+@pytest.mark.parametrize("M,N,K", [(1, 2, 512), (255, 190, 528), (257, 194, 640), (256, 192, 1008), (4100, 3300, 528), (4097, 13826, 512)])
+def test_gemm_walk_tiles_give_the_bits_of_separate_tiles(M, N, K, kind):
+    """K of any multiple of 16, bf16 and fp32 outputs, a bias, the residual: against the 256 x 128 tile of gemm_kernel (which the
+    oracle's tests cover); FP8 too, whose sums run in the same order."""
+    _say("gemm walk tiles", M, N, K, kind)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    xq, wq = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
+    sx, sw = (torch.rand(n, generator=g, device=DEV) * 0.01 + 1e-4 for n in (M, N))
+    x8, w8 = (torch.randn(n, K, generator=g, device=DEV).to(torch.float8_e4m3fn).view(torch.uint8) for n in (M, N))
+    b, r = torch.randn(N, generator=g, device=DEV), torch.randn(M, N, generator=g, device=DEV).to(torch.bfloat16)
+
+    def run():
+        for out, bias, res in ((torch.bfloat16, None, None), (torch.float32, b, None), (torch.bfloat16, b.to(torch.bfloat16), r)):
+            yield ops.linear_w8a8(xq, sx, wq, sw, bias, out_dtype=out, residual=res)
+            yield ops.linear_fp8(x8, sx[:1], w8, sw[:1], bias, out_dtype=out, residual=res)
+
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(kind) == 0
+        got = list(run())
+        assert lab.aq_lab_set_gemm_tile(256) == 0
+        for y, want in zip(got, run()):
+            assert torch.equal(y, want)
