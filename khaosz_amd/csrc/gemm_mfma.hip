@@ -174,9 +174,23 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   const uint32_t row32 = (uint32_t)(RPG * NWAVES) * (uint32_t)K;  // byte distance between a wavefront's row groups
   constexpr int NLOADS = A_LOADS + B_LOADS;
   const int nk = (K + BK - 1) / BK;
+  // Two accumulator columns per wavefront, bf16 outputs and an even N: a lane's two are neighbours of the output, which the order of
+  // B's rows in a stage makes them (column 2 c + j behind accumulator j of lane c), so that a row's 32 lanes store a whole
+  // 128-byte line (fp32 and int32 outputs fill one with a column each).
+  constexpr bool ADJ = TN == 2 && OUT == OUT_BF16;
+  const bool pair_ok = (N & 1) == 0;  // uniform: bf16 rows start dword-aligned, pairs never straddle N
   uint32_t ld_vo[A_LOADS > B_LOADS ? A_LOADS : B_LOADS];  // EXACT: lane offset of row group i, A and B alike
+  uint32_t ld_vb[ADJ ? B_LOADS : 1];                       // ... of B, where its rows have an order of their own
 #pragma unroll
   for (int i = 0; i < (A_LOADS > B_LOADS ? A_LOADS : B_LOADS); ++i) ld_vo[i] = ld_off + (uint32_t)i * row32;
+  if constexpr (ADJ) {
+#pragma unroll
+    for (int i = 0; i < B_LOADS; ++i) {
+      const int r = ld_row + i * RPG * NWAVES, own = (r & ~63) + 2 * (r & 31) + ((r >> 5) & 1);
+      ld_vb[i] = (uint32_t)(pair_ok ? own : r) * (uint32_t)K + ld_piece;
+    }
+  }
+  auto b_off = [&](int i) { return ADJ ? ld_vb[ADJ ? i : 0] : ld_vo[i]; };
   // load number `idx` (0..NLOADS-1) of K step kt into stage buffer `buf`
   auto issue_load = [&](int kt, int buf, int idx) {
     if constexpr (EXACT) {
@@ -187,21 +201,20 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
         __builtin_amdgcn_raw_ptr_buffer_load_lds(Ar, (lds_void*)(st + idx * (1024 * NWAVES)), 16, ld_vo[idx], k0s, 0, 0);
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(Br, (lds_void*)(st + BM * BK + (idx - A_LOADS) * (1024 * NWAVES)), 16,
-                                                 ld_vo[idx - A_LOADS], k0s, 0, 0);
+                                                 b_off(idx - A_LOADS), k0s, 0, 0);
       return;
     }
     const int k0 = kt * BK;
     // K is a multiple of 16: a piece is all in or all out.  Pieces past K would
     // alias the next row, so they are pushed outside the descriptor (-> zeros).
-    const uint32_t off = (k0 + ld_piece) < K ? ld_off + (uint32_t)k0 : OOB_OFFSET;
+    const bool in = k0 + ld_piece < K;
     uint8_t* st = smem + buf * STAGE + wave * 1024;
     if (idx < A_LOADS)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(Ar, (lds_void*)(st + idx * (1024 * NWAVES)), 16,
-                                               off == OOB_OFFSET ? OOB_OFFSET : off + idx * row32, 0, 0, 0);
+                                               in ? ld_vo[idx] + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(Br, (lds_void*)(st + BM * BK + (idx - A_LOADS) * (1024 * NWAVES)), 16,
-                                               off == OOB_OFFSET ? OOB_OFFSET : off + (idx - A_LOADS) * row32,
-                                               0, 0, 0);
+                                               in ? b_off(idx - A_LOADS) + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
   };
 
 #ifdef AQ_LAB_STALL
@@ -354,6 +367,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   uint32_t bias_raw[TN];
   const bool has_bias = OUT != OUT_I32 && p.bias != nullptr;
   const bool bias_bf16 = p.bias_dtype == AQ_BF16;
+  auto column = [&](int j) { return ADJ && pair_ok ? 2 * col + j : j * 32 + col; };  // inside the wavefront's
   auto load_epilogue_operands = [&]() {
     if constexpr (FP8) {
       sx1 = *p.sx;
@@ -362,7 +376,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
           make_rsrc(has_bias ? p.bias : (const void*)p.sw, has_bias ? (uint32_t)N * (bias_bf16 ? 2u : 4u) : 0u);
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const uint32_t n = (uint32_t)(n0 + wave_n * WAVE_N + j * 32 + col);  // past N, or no bias: outside -> 0
+        const uint32_t n = (uint32_t)(n0 + wave_n * WAVE_N + column(j));  // past N, or no bias: outside -> 0
         bias_raw[j] = bias_bf16 ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(Bsr, n * 2u, 0, 0)
                                 : (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(Bsr, n * 4u, 0, 0);
       }
@@ -404,7 +418,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
           make_rsrc(has_bias ? p.bias : p.sw, has_bias ? (uint32_t)N * (bias_bf16 ? 2u : 4u) : 0u);
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const uint32_t n = (uint32_t)(n0 + wave_n * WAVE_N + j * 32 + col);  // past N: outside -> 0
+        const uint32_t n = (uint32_t)(n0 + wave_n * WAVE_N + column(j));  // past N: outside -> 0
         swn[j] = __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(Wsr, n * 4u, 0, 0));
         bias_raw[j] = bias_bf16 ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(Bsr, n * 2u, 0, 0)
                                 : (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(Bsr, n * 4u, 0, 0);
@@ -563,7 +577,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   const bool has_res = !BIG && OUT != OUT_I32 && p.res != nullptr;  // uniform (big sub-tiles are not launched with a residual)
   const __amdgpu_buffer_rsrc_t Rr = make_rsrc(
       reinterpret_cast<const uint8_t*>(has_res ? p.res : p.C) + ((int64_t)mw * N + nw) * ESZ, has_res ? 0x40000000u : 0u);
-  const bool pair_ok = (N & 1) == 0;  // uniform: bf16 rows start dword-aligned, pairs never straddle N
   const bool odd = lane & 1;
   const uint32_t perm_sel = odd ? 0x03020706u : 0x05040100u;
   const uint32_t rowb = (uint32_t)N * ESZ;
@@ -688,7 +701,54 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
       }
     }
   };
-  if constexpr (BIG) {
+  // Neighbouring columns in a lane: a dword of output per row, 32 lanes a line.  us, half a line by pairs of lanes -> so:
+  // 2048 x 1536 x 1536 + residual 10.8 -> 10.4, 512 x 8192 x 1024 8.3 -> 7.8, 500 x 10992 x 1024 10.4 -> 9.1, 2000 x 5040 x 256
+  // 13.1 -> 11.9 (on other cards the halves cost up to half of such a launch, see gemm_walk.hip).
+  auto store_lines = [&](auto check_c) {
+    constexpr bool CHECK_M = decltype(check_c)::value;
+    const uint32_t at0 = nw + 2 * col < N ? (uint32_t)rq * rowb + (uint32_t)(2 * col) * ESZ : OOB_OFFSET;
+    auto at = [&](int r) { return CHECK_M && mw + r + rq >= M ? OOB_OFFSET : at0; };
+    uint32_t rr[TME][16];  // all of the residual, requested before any of it is used
+    if (has_res) {
+#pragma unroll
+      for (int i = 0; i < TME; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int r = i * 32 + e / 4 * 8 + e % 4;
+          rr[i][e] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(Rr, at(r), r * rowb, 0);
+        }
+    }
+    float bn[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) bn[j] = !has_bias ? 0.0f : bias_bf16 ? bf16_bits_to_f32(bias_raw[j]) : __uint_as_float(bias_raw[j]);
+#pragma unroll
+    for (int i = 0; i < TME; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int r = i * 32 + e / 4 * 8 + e % 4;
+        float y[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          if constexpr (FP8)
+            y[j] = __fadd_rn(__fmul_rn(__fmul_rn(acc[i][j][e], sx1), sw1), bn[j]);
+          else
+            y[j] = __fadd_rn(__fmul_rn(__fmul_rn((float)acc[i][j][e], sxr[i][e / 4][e % 4]), swn[j]), bn[j]);
+        }
+        uint32_t pk = pack_bf16x2(y[0], y[1]);
+        if (has_res)  // rounded output + residual, rounded again: what a separate add gives
+          pk = pack_bf16x2(__fadd_rn(__uint_as_float(pk << 16), __uint_as_float(rr[i][e] << 16)),
+                           __fadd_rn(__uint_as_float(pk & 0xffff0000u), __uint_as_float(rr[i][e] & 0xffff0000u)));
+        __builtin_amdgcn_raw_buffer_store_b32(pk, Cr, at(r), r * rowb, STORE_WT);
+      }
+  };
+  if constexpr (ADJ) {
+    if (pair_ok && rows_inside)
+      store_lines(no{});
+    else if (pair_ok)
+      store_lines(yes{});
+    else
+      store_all(yes{}, no{});
+  } else if constexpr (BIG) {
     store_all(no{}, yes{});  // one variant (256 outputs per lane): the launcher sends ragged M and odd N to another shape
   } else {
     if (rows_inside && pair_ok)
