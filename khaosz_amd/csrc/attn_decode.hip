@@ -96,6 +96,7 @@ struct AttnArgs {
   const uint16_t* q_gain;  // QKN kernels: [D] RMSNorm gains of the rotated q / k heads
   const uint16_t* k_gain;
   float eps;
+  int page_shift;  // log2 of the page, or -1
 };
 
 constexpr int ATT_WAVES = 4;
@@ -104,20 +105,16 @@ constexpr int ATT_KPG = ATT_WAVES * ATT_KPW; // positions per workgroup
 constexpr int ATT_MAX_D = 128;
 constexpr float ATT_MASKED = -1.0e30f;  // score (exp2 domain) of a cached position the sequence may not attend to
 
-// maximum / sum over each row of 16 consecutive lanes, result in all of them
-__device__ __forceinline__ float row16_max(float v) {
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false)));   // quad_perm [1,0,3,2]
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false)));   // quad_perm [2,3,0,1]
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false)));  // row_half_mirror
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false)));  // row_mirror
-  return v;
+// the value 16 / 32 lanes away (lane ^ 16, lane ^ 32)
+__device__ __forceinline__ float lanes16_other(float v) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float((threadIdx.x & 16) ? r.x : r.y);
 }
-__device__ __forceinline__ float row16_sum(float v) {
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false));
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false));
-  return v;
+__device__ __forceinline__ float lanes32_other(float v) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float((threadIdx.x & 32) ? r.x : r.y);
 }
 
 typedef __bf16 attn_bf16x8 __attribute__((ext_vector_type(8)));
@@ -129,18 +126,22 @@ typedef float attn_f32x4 __attribute__((ext_vector_type(4)));
 // separate workgroups so that a decode batch of a few sequences still spreads
 // over the device.  Every K and V load of a wavefront, 16 bytes per lane, is
 // requested before anything is computed.
-//   scores   on the matrix core: S[head, key] = Q K^T as v_mfma_f32_16x16x32_bf16
-//            tiles, the G <= 8 query heads padded to 16 rows, four tiles of 16
+//   scores   on the matrix core: S[key, head] = K Q^T as v_mfma_f32_16x16x32_bf16
+//            tiles, the G <= 8 query heads padded to 16 columns, four tiles of 16
 //            keys, D / 32 steps each.  K rows are loaded straight in operand
 //            order (lane l: key l % 16 of the tile, dimensions 8 (l / 16) .. + 8
 //            of the step), queries likewise; a lane ends up with the scores of
-//            one key per tile for 4 heads;
-//   softmax  maximum and denominator over a row of 16 lanes by DPP and over the
-//            four tiles in registers; probabilities to LDS;
+//            one head for 4 keys per tile;
+//   softmax  maximum and denominator over a lane's 16 keys in registers and over
+//            the 4 lanes of a head by row swaps (with heads in registers and keys
+//            in lanes every head took four DPP steps, twice); probabilities to LDS;
 //   values   V rows are loaded CPR = D / 8 lanes to a row (a load covers 4 or 8
 //            whole rows); a lane accumulates p * V over the keys it loaded (8
-//            dimensions x G heads, fma), the key groups are summed with xor
-//            shuffles.
+//            dimensions x G heads), the key groups are summed by swaps.
+// A launch of few sequences is one wavefront's chain of latencies, most of it
+// between the lookup of its pages and its sums (8 x 544 positions, 16/4 heads of
+// 128: 9.6 us, 4 x 576, 24/4 heads of 64: 7.0; 10.1 and 7.7 with a row lookup
+// per load, heads in registers and all sums by fused multiply-add).
 // The wavefronts' (maximum, denominator, numerator) are merged through LDS and
 // either normalised into the output (NS == 1) or left in the workspace for
 // attn_merge_kernel.
@@ -163,7 +164,9 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
   constexpr int ATT_THREADS = ATT_WAVES * 64;
   constexpr int PART = D + 4;    // numerator[D], maximum, denominator, 2 floats of padding
   static_assert(D == 64 || D == 128, "head dimension");
-  __shared__ __align__(16) float p_s[ATT_WAVES][KPW][G];
+  constexpr int NM = (G + 1) / 4, GV = G > 4 * NM ? G - 4 * NM : 0;  // groups of 4 heads on the matrix core; heads past them (1, 2)
+  constexpr int GP = 4 * NM + GV, PS = KPW + 16;                    // (rows of 80: 4 heads x 16 keys in 64 banks, both ways)
+  __shared__ __align__(16) float p_s[ATT_WAVES][GP][PS];
   __shared__ float m_s[ATT_WAVES][G], l_s[ATT_WAVES][G];
   __shared__ __align__(16) float acc_s[ATT_WAVES][G][D];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -186,12 +189,6 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
 
   constexpr int KS = D / 32;                  // matrix-core steps over the head dimension
   const int col = lane & 15, kq = lane >> 4;  // operand row / column, group of 8 dimensions inside a step
-  float acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[g][e] = 0.0f;
-  }
   // The queries (and their rotary table values) do not depend on the page table: requested first, used after
   // the K and V loads have been issued, so that the wavefront waits for one memory round trip less.
   uint4 qraw[KS];
@@ -236,9 +233,19 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
       }
     }
   }
-  // lane L looks up the row of position t0 + L (element offset, -1: unmapped or past T)
-  int64_t row = -1;
-  if (t0 + lane < T) {
+  // Where the rows are (element offsets, -1: unmapped or past T).  Pages of whole wavefronts (a multiple of 64 positions): all of this
+  // one's rows lie in one page, one lookup, and every load's address is that plus the lane's own offset.  Otherwise lane L looks
+  // up the row of position t0 + L.
+  const bool whole = p.page % KPW == 0;  // uniform
+  const int rstep = p.Hkv * D;           // elements between consecutive positions of a page
+  int64_t first = -1, row = -1;
+  if (whole) {
+    if (t0 < T) {
+      const int64_t lp = p.page_shift >= 0 ? t0 >> p.page_shift : t0 / p.page;
+      const int64_t phys = lp < p.P ? p.table[(int64_t)b * p.P + lp] : -1;
+      if (phys >= 0 && phys < p.n_pages) first = ((phys * p.page + (t0 - lp * p.page)) * p.Hkv + kvh) * D;
+    }
+  } else if (t0 + lane < T) {
     const int64_t t = t0 + lane;
     const int64_t lp = t / p.page;
     const int64_t phys = lp < p.P ? p.table[(int64_t)b * p.P + lp] : -1;
@@ -261,37 +268,51 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
     // (the fix-ups below are selects on data, kept out of the issue loops: with them inside, the compiler
     // waited for each load before issuing the next).
     uint4 kb[4][KS], vv[NL];
-    uint32_t kneg = 0, vneg = 0;  // bit t / i: that row is not there
+    uint64_t there;  // bit per position: its row is there
+    if (whole) {
+      // (20 lookups by shuffle, with 64-bit arithmetic each, took 0.3 us of the launch at head dimension 64, and 0.1 to 0.2 at 128, where
+      // 32 loads of 1 KiB wait for each other to be taken)
+      const uint16_t *ks0 = p.kc + (first >= 0 ? first : 0) + (uint32_t)(col * rstep + kq * 8);
+      const uint16_t *vs0 = p.vc + (first >= 0 ? first : 0) + (uint32_t)(sub * rstep + ch * 8);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int64_t r = row_of(t * 16 + col);
-      kneg |= (r < 0 ? 1u : 0u) << t;
-      const uint16_t* src = p.kc + (r >= 0 ? r : 0) + kq * 8;
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) kb[t][ks] = *reinterpret_cast<const uint4*>(src + ks * 32);
-    }
+        for (int ks = 0; ks < KS; ++ks) kb[t][ks] = *reinterpret_cast<const uint4*>(ks0 + t * 16 * rstep + ks * 32);
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int64_t r = row_of(i * RPL + sub);
-      vneg |= (r < 0 ? 1u : 0u) << i;
-      vv[i] = *reinterpret_cast<const uint4*>(p.vc + (r >= 0 ? r : 0) + ch * 8);
+      for (int i = 0; i < NL; ++i) vv[i] = *reinterpret_cast<const uint4*>(vs0 + i * RPL * rstep);
+      there = first < 0 ? 0 : ~0ull >> (t0 + KPW > T ? (int)(t0 + KPW - T) : 0);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int64_t r = row_of(t * 16 + col);
+        const uint16_t* src = p.kc + (r >= 0 ? r : 0) + kq * 8;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) kb[t][ks] = *reinterpret_cast<const uint4*>(src + ks * 32);
+      }
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const int64_t r = row_of(i * RPL + sub);
+        vv[i] = *reinterpret_cast<const uint4*>(p.vc + (r >= 0 ? r : 0) + ch * 8);
+      }
+      there = __builtin_amdgcn_ballot_w64(row >= 0);
     }
     __builtin_amdgcn_sched_barrier(0);  // nothing that waits for a load may move above the last load's issue
-    if (__builtin_amdgcn_ballot_w64(row < 0) != 0) {  // wavefront-uniform; rare: a hole, or the wavefront that holds T - 1
+    if (there != ~0ull) {  // wavefront-uniform; rare: a hole, or the wavefront that holds T - 1
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-          if (kneg & (1u << t)) kb[t][ks] = make_uint4(0, 0, 0, 0);
+          if (!(there >> (t * 16 + col) & 1)) kb[t][ks] = make_uint4(0, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < NL; ++i)
-        if (vneg & (1u << i)) vv[i] = make_uint4(0, 0, 0, 0);
+        if (!(there >> (i * RPL + sub) & 1)) vv[i] = make_uint4(0, 0, 0, 0);
     }
     if (ROPE && has_new) {  // wavefront-uniform: this wavefront owns position T - 1
       // the new key and value: rotated here, stored into their page slot, and used from registers in place
       // of what was just read from that slot
       const uint16_t* tok = p.qkv + (int64_t)b * (p.Hq + 2 * p.Hkv) * D;
-      const int64_t rn = row_of((int)(T - 1 - t0));  // the same in every lane; -1: its page is unmapped
+      // the same in every lane; -1: its page is unmapped
+      const int64_t rn = !whole ? row_of((int)(T - 1 - t0)) : first < 0 ? -1 : first + (T - 1 - t0) * rstep;
       if (rn >= 0) {
         const int tn = (int)(T - 1 - t0) >> 4, cn = (int)(T - 1 - t0) & 15;  // tile and column of the new key
         uint4 kn[KS];
@@ -329,61 +350,120 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
     for (int ks = 0; ks < KS; ++ks) {
       if (col >= G) qa[ks] = make_uint4(0, 0, 0, 0);
     }
-    // ---- scores: S[head][key] per tile; this lane gets key col of the tile, heads 4 kq .. + 4
+    // ---- scores: S[key][head] per tile; this lane gets head col, keys 4 kq .. + 4 of the tile
     attn_f32x4 sc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       attn_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(attn_bf16x8, qa[ks]),
-                                                   __builtin_bit_cast(attn_bf16x8, kb[t][ks]), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(attn_bf16x8, kb[t][ks]),
+                                                   __builtin_bit_cast(attn_bf16x8, qa[ks]), c, 0, 0, 0);
       sc[t] = c;
     }
-    // ---- softmax over the wavefront's 64 positions, per head
+    // ---- softmax over the wavefront's 64 positions of head col: 16 in this lane, the others 16 and 32 lanes away
+    const int n_all = T - t0 < KPW ? (int)(T - t0) : KPW, n_vis = vis - t0 < n_all ? (vis > t0 ? (int)(vis - t0) : 0) : n_all;
+    float pv[4][4], mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pv[t][r] = sc[t][r] * p.scale_log2e;
+    if (n_vis < KPW) {  // wavefront-uniform
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = t * 16 + 4 * kq + r;
+          pv[t][r] = key < n_vis ? pv[t][r] : key < n_all ? ATT_MASKED : -INFINITY;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, pv[t][r]);
+    mx = fmaxf(mx, lanes16_other(mx));
+    mx = fmaxf(mx, lanes32_other(mx));  // finite: position t0 is valid
+    float part[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int head = 4 * kq + r;
-      float sv[4], mx = -INFINITY;
+      part[r] = 0.0f;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const int64_t pos = t0 + t * 16 + col;
-        sv[t] = pos < T ? (pos < vis ? sc[t][r] * p.scale_log2e : ATT_MASKED) : -INFINITY;
-        mx = fmaxf(mx, sv[t]);
+        pv[t][r] = __builtin_amdgcn_exp2f(pv[t][r] - mx);  // 0 for positions past T
+        part[r] += pv[t][r];
       }
-      mx = row16_max(mx);  // finite: position t0 is valid
-      float sum = 0.0f;
+    }
+    float sum = (part[0] + part[1]) + (part[2] + part[3]);
+    sum += lanes16_other(sum);
+    sum += lanes32_other(sum);
+    if (col < GP) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float pv = __builtin_amdgcn_exp2f(sv[t] - mx);  // 0 for positions past T
-        sum += pv;
-        if (head < G) p_s[wave][t * 16 + col][head] = pv;
-      }
-      sum = row16_sum(sum);
-      if (col == 0 && head < G) {
-        m_s[wave][head] = mx;
-        l_s[wave][head] = sum;
+      for (int t = 0; t < 4; ++t)
+        *reinterpret_cast<float4*>(&p_s[wave][col][t * 16 + 4 * kq]) = make_float4(pv[t][0], pv[t][1], pv[t][2], pv[t][3]);
+      if (kq == 0 && col < G) {
+        m_s[wave][col] = mx;
+        l_s[wave][col] = sum;
       }
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);  // this wavefront's LDS writes are done (wavefront-private region)
     asm volatile("" ::: "memory");
     // ---- numerator (unmapped rows and positions past T contribute zeros)
+    // Four heads at a time as outer products on the matrix core, 16 of 4 heads x 4 lanes: a lane's element of V times its key's
+    // probability of each head, added to the lane's own four sums with one rounding: the bits of the fused multiply-add that the
+    // heads past them take (also for infinities and denormals), in the same order.  A product took 10 clocks where four
+    // fused multiply-adds take 16 (launch of 8 x 544 positions at head dimension 128, 4 heads: 9.97 -> 9.55 us; 4 x 576, 64, 6 heads:
+    // 7.13 -> 6.97), and one register holds the probabilities of PER loads, each broadcast to the lanes of its keys.
+    constexpr int PER = CPR / 4, CB = PER == 4 ? 2 : 1;               // blocks of 4 lanes that share a key
+    attn_f32x4 accm[NM > 0 ? NM : 1][8];
+    float acc[GV > 0 ? GV : 1][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+      for (int m = 0; m < NM; ++m) accm[m][e] = attn_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int g = 0; g < GV; ++g) acc[g][e] = 0.0f;
+    }
+    float pm[NM > 0 ? NM : 1][NL / PER];
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+      for (int i = 0; i < NL / PER; ++i)
+        pm[m][i] = p_s[wave][4 * m + (lane & 3)][(i * PER + ((lane >> 2) & (PER - 1))) * RPL + sub];
+    auto outer = [&](float pj, float v, attn_f32x4 c, int step) {  // the block is an immediate
+      switch (step) {
+        case 0: return __builtin_amdgcn_mfma_f32_4x4x1f32(pj, v, c, CB, 0, 0);
+        case 1: return __builtin_amdgcn_mfma_f32_4x4x1f32(pj, v, c, CB, 1, 0);
+        case 2: return __builtin_amdgcn_mfma_f32_4x4x1f32(pj, v, c, CB, 2, 0);
+        default: return __builtin_amdgcn_mfma_f32_4x4x1f32(pj, v, c, CB, 3, 0);
+      }
+    };
+    auto widened = [&](int i, int e) {  // element e of load i
+      const uint32_t w = e < 2 ? vv[i].x : e < 4 ? vv[i].y : e < 6 ? vv[i].z : vv[i].w;
+      return __uint_as_float(e & 1 ? w & 0xffff0000u : w << 16);
+    };
+    // The next load's values are widened before this one's products, which stay together: a product waits two slots for a
+    // register written just before it, and 11 clocks after any other vector instruction (products and widening in turn: 9.84 us).
+    float v8[2][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v8[0][e] = widened(0, e);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      float v8[8];
-      v8[0] = __uint_as_float(vv[i].x << 16);
-      v8[1] = __uint_as_float(vv[i].x & 0xffff0000u);
-      v8[2] = __uint_as_float(vv[i].y << 16);
-      v8[3] = __uint_as_float(vv[i].y & 0xffff0000u);
-      v8[4] = __uint_as_float(vv[i].z << 16);
-      v8[5] = __uint_as_float(vv[i].z & 0xffff0000u);
-      v8[6] = __uint_as_float(vv[i].w << 16);
-      v8[7] = __uint_as_float(vv[i].w & 0xffff0000u);
+      float pg[GV > 0 ? GV : 1];
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float pj = p_s[wave][i * RPL + sub][g];
+      for (int g = 0; g < GV; ++g) pg[g] = p_s[wave][4 * NM + g][i * RPL + sub];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[g][e] = __builtin_fmaf(pj, v8[e], acc[g][e]);
+      for (int e = 0; e < 8; ++e) {
+        if (i + 1 < NL) v8[(i + 1) & 1][e] = widened(i + 1, e);
+#pragma unroll
+        for (int g = 0; g < GV; ++g) acc[g][e] = __builtin_fmaf(pg[g], v8[i & 1][e], acc[g][e]);
+      }
+      if constexpr (NM > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) accm[m][e] = outer(pm[m][i / PER], v8[i & 1][e], accm[m][e], i % PER);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
     // Sum over the RPL key groups (lanes CPR apart) with a transposed butterfly: at each stage a lane keeps
@@ -393,7 +473,7 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
       constexpr int NV = 8 * G;
       float a[NV];
 #pragma unroll
-      for (int j = 0; j < NV; ++j) a[j] = acc[j / 8][j % 8];
+      for (int j = 0; j < NV; ++j) a[j] = j / 8 < 4 * NM ? accm[j / 32][j % 8][j / 8 % 4] : acc[j / 8 - 4 * NM][j % 8];
       int base = 0;  // first original index of the values this lane still holds
 #pragma unroll
       for (int st = 0; (CPR << st) < 64; ++st) {
@@ -409,10 +489,10 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
                                        : __builtin_amdgcn_permlane16_swap(__float_as_uint(a[i]), __float_as_uint(a[i + h]), false, false);
             a[i] = __uint_as_float(r.x) + __uint_as_float(r.y);
           } else {
-            // select by mask rather than by ?: -- the compiler turned the latter into per-exchange branches
-            const uint32_t lo = __float_as_uint(a[i]), hi = __float_as_uint(a[i + h]);
-            const uint32_t t = (lo ^ hi) & (up ? 0xffffffffu : 0u);
-            a[i] = __uint_as_float(t ^ lo) + __shfl_xor(__uint_as_float(t ^ hi), off, 64);  // keep + partner's send
+            // 8 lanes away inside rows of 16 (head dimension 64): both halves' sums, then this lane's one
+            const float lo = a[i] + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a[i]), 0x128, 0xf, 0xf, false));
+            const float hi = a[i + h] + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a[i + h]), 0x128, 0xf, 0xf, false));
+            a[i] = up ? hi : lo;
           }
         }
         base += up ? h : 0;
@@ -673,6 +753,9 @@ static int attn_decode(const void* q, const void* qkv, const float* freqs, int64
   a.q_gain = static_cast<const uint16_t*>(q_gain);
   a.k_gain = static_cast<const uint16_t*>(k_gain);
   a.eps = eps;
+  a.page_shift = -1;
+  for (int sh = 0; sh < 62; ++sh)
+    if (page_size == ((int64_t)1 << sh)) a.page_shift = sh;
   const dim3 grid((unsigned)(B * Hkv * ns)), block(aq::ATT_WAVES * 64);
   hipStream_t st = static_cast<hipStream_t>(stream);
 #define AQ_ATTN_CASE(G_)                                            \

@@ -575,3 +575,55 @@ def test_prefill_attn_that_rotates_its_queries_gives_the_bits_of_two_launches(B,
         assert lib.aq_rope_prefill_attn_causal_ahead(qkv.data_ptr(), W, fr.data_ptr(), stride, qg, eps, k.data_ptr(), Hkv * D, v.data_ptr(), W,
                                                      out.data_ptr(), D ** -0.5, B, S, Hq, Hkv, D, None, 0, st) == 0
         assert torch.equal(out, want[1])
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(1, 1, 64), (4, 2, 128), (6, 2, 64), (8, 2, 128), (12, 2, 64), (12, 2, 128), (16, 2, 64)])
+@pytest.mark.parametrize("T", [1, 64, 191, 193, 640, 1000])
+def test_paged_attn_decode_page_sizes_give_the_same_bits(Hq, Hkv, D, T):
+    """The same cached positions under pages of whole wavefronts (64 positions, 128, 192: one lookup each) and under pages that a
+    wavefront's positions straddle (16, 96): outputs and the new token's rows bit for bit, with a hole, with masked sequences."""
+    B, span, heads = 3, 192, Hq + 2 * Hkv
+    n = (T + span - 1) // span                          # 192 is a multiple of every page but 128: stretches of 384
+    n += n & 1
+    _say("page sizes", Hq, Hkv, D, T)
+    g = torch.Generator().manual_seed(T * Hq + D)
+    k, v = (torch.randn(B, n * span, Hkv, D, generator=g).to(torch.bfloat16) for _ in range(2))
+    qkv = torch.randn(B, heads * D, generator=g).to(torch.bfloat16).to(DEV)
+    ang = torch.rand(B, D // 2, generator=g) * 6.28
+    freqs = torch.polar(torch.ones_like(ang), ang).to(DEV)
+    lens = torch.tensor([T, max(1, T - 100), (T + 1) // 2]).to(DEV)
+    got = []
+    for page in (64, 128, 192, 16, 96):
+        P = n * span // page
+        order = torch.randperm(B * P, generator=g)
+        kc, vc = (torch.empty(B * P, page, Hkv, D, dtype=torch.bfloat16) for _ in range(2))
+        kc[order], vc[order] = k.view(B * P, page, Hkv, D), v.view(B * P, page, Hkv, D)
+        table = order.view(B, P).clone()
+        if n > 2:
+            table[B - 1, 384 // page: 768 // page] = -1  # (T = 640, 1000: the last sequence's positions 384 .. 768)
+        kc, vc, table = kc.to(DEV), vc.to(DEV), table.to(DEV)
+        outs = [ops.rope_paged_attn_decode(qkv, freqs, table, T, kc, vc, Hq, Hkv, seq_lens=sl) for sl in (None, lens)]
+        q = qkv.view(B, heads, D)[:, :Hq].contiguous()
+        outs.append(ops.paged_attn_decode(q, kc, vc, table, T))
+        back = order.to(DEV)
+        got.append([o.view(torch.int16) for o in outs + [kc[back].view(B, -1), vc[back].view(B, -1)]])
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(2, 1, 64), (3, 1, 128), (4, 1, 64), (6, 1, 64), (6, 1, 128), (8, 1, 128)])
+def test_paged_attn_decode_infinite_values_stay_in_their_dimension(Hq, Hkv, D):
+    """An infinite value at a position that every head weighs makes that dimension of every head infinite and changes no other bit."""
+    T, page = 200, 64
+    g = torch.Generator().manual_seed(D + Hq)
+    q = (torch.randn(1, Hq, D, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+    kc, vc = (torch.randn(4, page, Hkv, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    table = torch.arange(4).view(1, 4).to(DEV)
+    clean = ops.paged_attn_decode(q, kc, vc, table, T)
+    for pos, dim, val in [(0, 0, float("inf")), (77, D - 1, float("-inf")), (T - 1, 13, float("inf"))]:
+        w = vc.clone()
+        w[pos // page, pos % page, 0, dim] = val
+        out = ops.paged_attn_decode(q, kc, w, table, T)
+        assert bool((out[..., dim].float() == val).all())
+        keep = torch.arange(D) != dim
+        assert torch.equal(out[..., keep].view(torch.int16), clean[..., keep].view(torch.int16))
