@@ -77,6 +77,18 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(RopeArgs p) {
   *reinterpret_cast<uint4*>(dst) = x;
 }
 
+// n / d for 0 <= n < 2^31 as a product: mul = ceil(2^(31 + s) / d) with s = ceil(log2 d), so mul d - 2^(31 + s) < d <= 2^s and
+// the quotient is exact.
+struct UDiv {
+  uint32_t mul, shift;
+  static UDiv of(uint32_t d) {
+    uint32_t s = 0;
+    while (((uint64_t)1 << s) < d) ++s;
+    return {(uint32_t)((((uint64_t)1 << (31 + s)) + d - 1) / d), s};
+  }
+  __device__ __forceinline__ uint32_t operator()(uint32_t n) const { return __umulhi(2 * n, mul) >> shift; }
+};
+
 struct AttnArgs {
   const uint16_t* q;     // [B, Hq, D]
   const uint16_t* kc;    // [n_pages, page, Hkv, D]
@@ -96,7 +108,9 @@ struct AttnArgs {
   const uint16_t* q_gain;  // QKN kernels: [D] RMSNorm gains of the rotated q / k heads
   const uint16_t* k_gain;
   float eps;
-  int page_shift;  // log2 of the page, or -1
+  int page_shift;  // log2 of a page of 64, 128, 256 .. positions, otherwise 62
+  const int64_t* lens_at;  // lens, or without them anything of B numbers (the table): read without asking, beside the table
+  UDiv by_hkv, by_ns;
 };
 
 constexpr int ATT_WAVES = 4;
@@ -174,38 +188,39 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
   const int sub = lane / CPR, ch = lane % CPR;  // key within a load, 16-byte chunk of the row
   // the KV heads of one slice are neighbours in the launch order: together they read whole
   // [position][Hkv][D] stretches of the pages at about the same time
-  const int kvh = blockIdx.x % p.Hkv, bs = blockIdx.x / p.Hkv;
-  const int split = bs % p.NS, b = bs / p.NS;
+  const int bs = p.by_hkv(blockIdx.x), kvh = blockIdx.x - bs * p.Hkv;
+  const int b = p.by_ns(bs), split = bs - b * p.NS;
   const int64_t T = p.T;
   const int64_t t0 = (int64_t)split * KPG + wave * KPW;  // first position of this wavefront
-  // A sequence shorter than T (a decode batch of sequences at different positions): positions from its own
-  // length on are masked, as the additive mask of the reference's forward does.  The mask value is finite, so
-  // a wavefront or slice whose positions are all masked leaves a partial result that later merges weigh with 0.
-  int64_t vis = T;
-  if (p.lens) {
-    const int64_t l = p.lens[b];
-    vis = l < T ? (l > 0 ? l : 0) : T;
-  }
+  // Where the rows are.  Pages of 64, 128, 256 .. positions: all of this wavefront's rows lie in one page, one lookup, and every
+  // load's address is that plus the lane's own offset.  The table's entry (otherwise its first, not used) and the sequence's
+  // length are requested before anything else and first used behind the queries' requests (8 x 544 positions, 16/4 heads of 128:
+  // 9.46 us; 9.60 with divisions by the numbers of heads and slices, a wait for the length and the lookup behind them).
+  const bool whole = p.page_shift < 62;  // uniform
+  const int64_t lp0 = t0 >> p.page_shift;
+  int64_t entry = p.table[(int64_t)b * p.P + (lp0 < p.P ? lp0 : p.P - 1)];
+  int64_t len = p.lens_at[b];
+  asm volatile("" ::"s"(p.T), "s"(p.page), "s"(p.n_pages), "s"(p.lens), "s"(p.kc), "s"(p.vc));  // arguments: one request for all
+  __builtin_amdgcn_sched_barrier(0);
 
   constexpr int KS = D / 32;                  // matrix-core steps over the head dimension
   const int col = lane & 15, kq = lane >> 4;  // operand row / column, group of 8 dimensions inside a step
   // The queries (and their rotary table values) do not depend on the page table: requested first, used after
-  // the K and V loads have been issued, so that the wavefront waits for one memory round trip less.
+  // the K and V loads have been issued, so that the wavefront waits for one memory round trip less.  (Wavefronts past T request
+  // them too: a branch here would end the stretch in which the scalar requests go out together.)
   uint4 qraw[KS];
   float4 fa[KS], fb[KS];
-  if (t0 < T) {
-    const int hq = col < G ? col : 0;  // heads past G: zero rows of the operand (their loads read head 0)
+  const int hq = col < G ? col : 0;  // heads past G: zero rows of the operand (their loads read head 0)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int d0 = ks * 32 + kq * 8;
-      if constexpr (ROPE) {
-        qraw[ks] = *reinterpret_cast<const uint4*>(p.qkv + ((int64_t)b * (p.Hq + 2 * p.Hkv) + kvh * G + hq) * D + d0);
-        const float* cs = p.freqs + (int64_t)b * p.freqs_stride + d0;
-        fa[ks] = *reinterpret_cast<const float4*>(cs);
-        fb[ks] = *reinterpret_cast<const float4*>(cs + 4);
-      } else {
-        qraw[ks] = *reinterpret_cast<const uint4*>(p.q + ((int64_t)b * p.Hq + kvh * G + hq) * D + d0);
-      }
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d0 = ks * 32 + kq * 8;
+    if constexpr (ROPE) {
+      qraw[ks] = *reinterpret_cast<const uint4*>(p.qkv + ((int64_t)b * (p.Hq + 2 * p.Hkv) + kvh * G + hq) * D + d0);
+      const float* cs = p.freqs + (int64_t)b * p.freqs_stride + d0;
+      fa[ks] = *reinterpret_cast<const float4*>(cs);
+      fb[ks] = *reinterpret_cast<const float4*>(cs + 4);
+    } else {
+      qraw[ks] = *reinterpret_cast<const uint4*>(p.q + ((int64_t)b * p.Hq + kvh * G + hq) * D + d0);
     }
   }
   // RMSNorm of a rotated head vector held as KS chunks per lane (chunk 4 ks + kq), gains requested by the caller
@@ -225,32 +240,30 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
   };
   uint4 qgain[KS], kgain[KS];
   if constexpr (QKN) {
-    if (t0 < T) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        qgain[ks] = *reinterpret_cast<const uint4*>(p.q_gain + ks * 32 + kq * 8);
-        kgain[ks] = *reinterpret_cast<const uint4*>(p.k_gain + ks * 32 + kq * 8);
-      }
+    for (int ks = 0; ks < KS; ++ks) {
+      qgain[ks] = *reinterpret_cast<const uint4*>(p.q_gain + ks * 32 + kq * 8);
+      kgain[ks] = *reinterpret_cast<const uint4*>(p.k_gain + ks * 32 + kq * 8);
     }
   }
-  // Where the rows are (element offsets, -1: unmapped or past T).  Pages of whole wavefronts (a multiple of 64 positions): all of this
-  // one's rows lie in one page, one lookup, and every load's address is that plus the lane's own offset.  Otherwise lane L looks
-  // up the row of position t0 + L.
-  const bool whole = p.page % KPW == 0;  // uniform
-  const int rstep = p.Hkv * D;           // elements between consecutive positions of a page
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" : "+s"(entry), "+s"(len));  // not requested later than above
+  // (element offsets, -1: unmapped or past T; pages that wavefronts straddle: lane L looks up the row of position t0 + L)
+  const int rstep = p.Hkv * D;  // elements between consecutive positions of a page
   int64_t first = -1, row = -1;
   if (whole) {
-    if (t0 < T) {
-      const int64_t lp = p.page_shift >= 0 ? t0 >> p.page_shift : t0 / p.page;
-      const int64_t phys = lp < p.P ? p.table[(int64_t)b * p.P + lp] : -1;
-      if (phys >= 0 && phys < p.n_pages) first = ((phys * p.page + (t0 - lp * p.page)) * p.Hkv + kvh) * D;
-    }
+    if (t0 < T && lp0 < p.P && entry >= 0 && entry < p.n_pages)
+      first = (((entry << p.page_shift) + (t0 - (lp0 << p.page_shift))) * p.Hkv + kvh) * D;
   } else if (t0 + lane < T) {
     const int64_t t = t0 + lane;
     const int64_t lp = t / p.page;
     const int64_t phys = lp < p.P ? p.table[(int64_t)b * p.P + lp] : -1;
     if (phys >= 0 && phys < p.n_pages) row = ((phys * p.page + t % p.page) * p.Hkv + kvh) * D;
   }
+  // A sequence shorter than T (a decode batch of sequences at different positions): positions from its own
+  // length on are masked, as the additive mask of the reference's forward does.  The mask value is finite, so
+  // a wavefront or slice whose positions are all masked leaves a partial result that later merges weigh with 0.
+  const int64_t vis = p.lens && len < T ? (len > 0 ? len : 0) : T;
   // Positions that are all masked weigh nothing in the merges: their keys and values are not read (model step of 11 sequences
   // spread over 1400 positions: 941 -> 922 us).  Not so where every position is masked, and the new token's wavefront
   // has it to store.  Asked only here, so that nothing above waits for the length.
@@ -753,8 +766,11 @@ static int attn_decode(const void* q, const void* qkv, const float* freqs, int64
   a.q_gain = static_cast<const uint16_t*>(q_gain);
   a.k_gain = static_cast<const uint16_t*>(k_gain);
   a.eps = eps;
-  a.page_shift = -1;
-  for (int sh = 0; sh < 62; ++sh)
+  a.lens_at = seq_lens ? seq_lens : page_table;
+  a.by_hkv = aq::UDiv::of((uint32_t)Hkv);
+  a.by_ns = aq::UDiv::of((uint32_t)ns);
+  a.page_shift = 62;
+  for (int sh = 6; sh < 62; ++sh)
     if (page_size == ((int64_t)1 << sh)) a.page_shift = sh;
   const dim3 grid((unsigned)(B * Hkv * ns)), block(aq::ATT_WAVES * 64);
   hipStream_t st = static_cast<hipStream_t>(stream);

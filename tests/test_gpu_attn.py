@@ -580,8 +580,8 @@ def test_prefill_attn_that_rotates_its_queries_gives_the_bits_of_two_launches(B,
 @pytest.mark.parametrize("Hq,Hkv,D", [(1, 1, 64), (4, 2, 128), (6, 2, 64), (8, 2, 128), (12, 2, 64), (12, 2, 128), (16, 2, 64)])
 @pytest.mark.parametrize("T", [1, 64, 191, 193, 640, 1000])
 def test_paged_attn_decode_page_sizes_give_the_same_bits(Hq, Hkv, D, T):
-    """The same cached positions under pages of whole wavefronts (64 positions, 128, 192: one lookup each) and under pages that a
-    wavefront's positions straddle (16, 96): outputs and the new token's rows bit for bit, with a hole, with masked sequences."""
+    """The same cached positions under pages of whole wavefronts (64 positions, 128: one lookup each) and under other pages (192;
+    16 and 96, which a wavefront's positions straddle): outputs and the new token's rows bit for bit, with a hole, with masked sequences."""
     B, span, heads = 3, 192, Hq + 2 * Hkv
     n = (T + span - 1) // span                          # 192 is a multiple of every page but 128: stretches of 384
     n += n & 1
