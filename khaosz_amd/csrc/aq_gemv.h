@@ -19,7 +19,7 @@ struct GemvArgs {
   int ksplit, groups;  // matrix-core variant: wavefronts sharing a row group, row groups per workgroup
   const void* gamma;   // NORM kernels: RMSNorm gain [K] in x's dtype
   float eps;
-  const float* parts;  // MERGE kernels: attention partial results in place of x
+  const float* parts;  // attention partial results in place of x (gemv_rows_kernel<.., WPR>)
   int parts_ns, parts_d;
 };
 
@@ -100,5 +100,6 @@ enum RowsKind { ROWS_I8, ROWS_I8_NORM, ROWS_I8_F32, ROWS_FP8 };
 bool gemv_rows_ok(RowsKind kind, int64_t M, int64_t K);
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st);
 int launch_gemv_rows_swiglu(const GemvArgs& a, hipStream_t st);
+int launch_gemv_rows_attn(const GemvArgs& a, hipStream_t st);  // rows from a.parts; M <= 8, K <= 2048
 
 }  // namespace aq

@@ -83,13 +83,11 @@ constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v / 2); }
 // workgroup covers GV_ROWS * wavefronts weight rows; the launcher shrinks it
 // when N is too small for 8-wavefront workgroups to reach every compute unit.
 // NORM (with FUSED): the rows are RMS-normalised with the gain p.gamma before they are quantised.
-// MERGE > 0 (with FUSED): the rows are a decode step's attention output, combined here from the attention
-// kernel's partial results of up to MERGE slices (p.parts) -- the separate merge launch disappears.
 // FW: wavefronts per workgroup of a FUSED kernel (8, or 4 for short matrices).
 // FK: K parts of a FUSED kernel (1; 4 for a short matrix with long rows, an MLP's down projection: every wavefront
 // still rounds a row, then FK wavefronts share a group of weight rows, so that the launch has a workgroup for
 // every compute unit where whole rows per wavefront would leave most of them without loads in flight).
-template <int MT, bool FUSED, int VPL, bool NORM = false, int MERGE = 0, int FW = GV_WAVES, int FK = 1>
+template <int MT, bool FUSED, int VPL, bool NORM = false, int FW = GV_WAVES, int FK = 1>
 __global__ __launch_bounds__(GV_THREADS) void gemv_w8a8_kernel(GemvArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [MT][K] activation codes, then [MT] scales
   const int tid = threadIdx.x, lane = tid & 63;
@@ -136,10 +134,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_w8a8_kernel(GemvArgs p) {
   // and quantises them while the weight loads queued behind are in flight.
   constexpr int RPW = FUSED ? (MT + WAVES - 1) / WAVES : 1;
   RowsToLds<true, RPW, VPL> xrows;
-  AttnRows<RPW, VPL, MERGE> arows;
-  if constexpr (MERGE > 0) {
-    arows.issue(p.parts, M, K, p.parts_d, p.parts_ns, wave, WAVES, lane);
-  } else if constexpr (FUSED) {
+  if constexpr (FUSED) {
     xrows.issue(p.x, M, K, K, wave, WAVES, lane);
     if constexpr (NORM) xrows.issue_gamma(p.gamma, K, lane);
   } else {
@@ -183,7 +178,6 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_w8a8_kernel(GemvArgs p) {
   // compiler place that wait), then make every wavefront's part visible through
   // a barrier that does not drain the weight loads.
   if constexpr (FUSED) {
-    if constexpr (MERGE > 0) arows.merge(xrows.c, M, K, p.parts_ns, wave, WAVES, lane);
     xrows.template finish<NORM>(M, MT, K, xs, K, sx_lds, wave, WAVES, lane, p.eps);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wavefront's LDS writes are done
   } else {
@@ -286,7 +280,7 @@ static GemvShape gemv_shape(int N, int K, bool fused, int mt) {
   return sh;
 }
 
-template <int MT, bool FUSED, int VPL, bool NORM, int MERGE, int FW, int FK = 1>
+template <int MT, bool FUSED, int VPL, bool NORM, int FW, int FK = 1>
 static int launch_gemv_fw(GemvArgs a, hipStream_t st) {
   GemvShape sh = gemv_shape(a.N, a.K, FUSED, MT);
   if (FUSED) {
@@ -299,23 +293,23 @@ static int launch_gemv_fw(GemvArgs a, hipStream_t st) {
   const size_t lds = (size_t)MT * a.K + MT * sizeof(float) + (sh.ksplit > 1 ? (size_t)sh.waves * 64 * sizeof(int) : 0);
   if (lds > 64 * 1024) {  // beyond the default dynamic-LDS limit: opt this kernel in, once per device
     static LdsOptIn opted;
-    const int e = opted.ensure(reinterpret_cast<const void*>(&gemv_w8a8_kernel<MT, FUSED, VPL, NORM, MERGE, FW, FK>));
+    const int e = opted.ensure(reinterpret_cast<const void*>(&gemv_w8a8_kernel<MT, FUSED, VPL, NORM, FW, FK>));
     if (e) return e;
   }
-  aq::queue_kernel((gemv_w8a8_kernel<MT, FUSED, VPL, NORM, MERGE, FW, FK>), dim3(grid), dim3(sh.waves * 64), lds, st, a);
+  aq::queue_kernel((gemv_w8a8_kernel<MT, FUSED, VPL, NORM, FW, FK>), dim3(grid), dim3(sh.waves * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 
 // Fused kernels on a short matrix (N / 32 workgroups would leave most compute units without one) run with 4
 // wavefronts per workgroup instead of 8: twice the workgroups, each quantising the rows again but reaching a
 // compute unit of its own (q/k/v 3072 x 2048 at M = 8: 5.6 -> 5.2 us; 1536 x 1536 at M = 4: 3.8 -> 3.5 us).
-// Only where a wavefront still holds at most one row of the in-kernel merge and the rows are short.
-template <int MT, bool FUSED, int VPL, bool NORM = false, int MERGE = 0>
+// Only where the rows are short.
+template <int MT, bool FUSED, int VPL, bool NORM = false>
 static int launch_gemv(GemvArgs a, hipStream_t st) {
-  if constexpr (FUSED && VPL <= 4 && (MERGE == 0 || MT <= 4)) {
-    if (a.N <= 4096) return launch_gemv_fw<MT, FUSED, VPL, NORM, MERGE, 4>(a, st);
+  if constexpr (FUSED && VPL <= 4) {
+    if (a.N <= 4096) return launch_gemv_fw<MT, FUSED, VPL, NORM, 4>(a, st);
   }
-  return launch_gemv_fw<MT, FUSED, VPL, NORM, MERGE, GV_WAVES>(a, st);
+  return launch_gemv_fw<MT, FUSED, VPL, NORM, GV_WAVES>(a, st);
 }
 
 #ifndef AQ_GV_MFMA_MIN_M
@@ -954,9 +948,9 @@ static int gemv_dispatch_fused(const aq::GemvArgs& a, int x_dtype, int mt, hipSt
   // 12.1 us for 8 rows).
   if (!norm && (a.N + 31) / 32 * 4 <= aq::device_cus() && a.K > 4096) {
     switch (mt) {
-      case 1: return aq::launch_gemv_fw<1, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
-      case 2: return aq::launch_gemv_fw<2, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
-      default: return aq::launch_gemv_fw<4, true, 16, false, 0, aq::GV_WAVES, 4>(a, st);
+      case 1: return aq::launch_gemv_fw<1, true, 16, false, aq::GV_WAVES, 4>(a, st);
+      case 2: return aq::launch_gemv_fw<2, true, 16, false, aq::GV_WAVES, 4>(a, st);
+      default: return aq::launch_gemv_fw<4, true, 16, false, aq::GV_WAVES, 4>(a, st);
     }
   }
   const bool small = vpl <= 4;
@@ -1201,13 +1195,7 @@ extern "C" int aq_gemv_w8a8_decode_attn(const float* partials, int64_t n_slices,
   a.bias_dtype = bias_dtype;
   a.y_dtype = y_dtype;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  constexpr int NS = AQ_GEMV_ATTN_MAX_SLICES;
-  switch (mt) {
-    case 1: return aq::launch_gemv<1, true, 4, false, NS>(a, st);
-    case 2: return aq::launch_gemv<2, true, 4, false, NS>(a, st);
-    case 4: return aq::launch_gemv<4, true, 4, false, NS>(a, st);
-    default: return aq::launch_gemv<8, true, 4, false, NS>(a, st);
-  }
+  return aq::launch_gemv_rows_attn(a, st);
 }
 
 extern "C" int aq_gemv_w8a8_decode_rmsnorm(const void* x, int x_dtype, const void* gamma, float eps, const int8_t* wq,

@@ -52,7 +52,10 @@ constexpr int64_t GX_MAX_K = 8192;
 // SWI: the weight is an MLP's up and gate projections stacked, rows [0, F) up and [F, 2F) gate; the first half of the
 // row groups takes rows of up, the second half the same rows of gate, and the output is up * silu(gate), the two as the
 // projections would have been stored (rounded to the output type first).
-template <int KS, int R, bool BF16, int RPW, int VPL, bool NORM, bool FP8, bool SWI = false>
+// WPR > 0: the rows (up to 8, of up to 2048) are a decode step's attention output, combined here from the attention kernel's partial
+// results of up to 4 slices (p.parts), WPR wavefronts to a row: 4 rows of 1536 in 3 slices are 78 KB to request, and all
+// eight wavefronts ask for them at once (whole rows in 4 of 4 wavefronts, vector ALU products, N = 1536: 5.8 us; 5.3).
+template <int KS, int R, bool BF16, int RPW, int VPL, bool NORM, bool FP8, bool SWI = false, int WPR = 0>
 __global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
   constexpr int GR = GX_WAVES / KS;
   constexpr int HALVES = R / 8;                          // 8-row halves of a row group: loads per line
@@ -129,7 +132,52 @@ __global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
 
   float* const sx_lds = reinterpret_cast<float*>(xs + M * pitch);
   GV_STAMP(0);
-  if constexpr (BF16) {
+  if constexpr (WPR > 0) {
+    static_assert(BF16 && RPW == 1 && VPL == 4 && !NORM && !FP8 && !SWI, "attention rows");
+    constexpr int VR = WPR < 4 ? 4 / WPR : 1;  // vectors of a row per lane
+    const int m = wave / WPR, q = wave % WPR;
+    AttnRows<VR, AQ_GEMV_ATTN_MAX_SLICES> ar;
+    ar.issue(p.parts, m < M, m, K, p.parts_d, p.parts_ns, q * 64, WPR * 64, lane);
+    asm volatile("" ::: "memory");  // request order: token rows, epilogue operands, the weight stream
+    load_epi();
+    asm volatile("" ::: "memory");
+    wload(lbeg, wa);
+    static_assert(!LOOP, "all weights are in flight");
+    asm volatile("" ::: "memory");
+    uint4 c[VR];
+    ar.merge(c, m < M, K, p.parts_ns, q * 64, WPR * 64, lane);
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < VR; ++i) {
+      float f[8];
+      RowIn<true>::unpack(c[i], f);
+      amax = fmaxf(amax, vec_amax<8>(f));
+    }
+    amax = wave_max(amax);
+    if constexpr (WPR > 1) {  // the row's wavefronts
+      if (lane == 0) sx_lds[8 + wave] = amax;
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();  // no memory fence: the weight loads stay in flight
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int w = 0; w < WPR; ++w) amax = fmaxf(amax, sx_lds[8 + m * WPR + w]);
+    }
+    constexpr int STEPS = quant_steps<true, false>();
+    const RowScale rsc = row_scale<STEPS>(amax);
+    if (lane == 0 && q == 0 && m < M) sx_lds[m] = rsc.s;
+#pragma unroll
+    for (int i = 0; i < VR; ++i) {
+      const int v = (i * WPR + q) * 64 + lane;
+      if (m < M && v < K / 8) {
+        float f[8];
+        uint32_t code[2];
+        RowIn<true>::unpack(c[i], f);
+        quant_codes_packed<8, STEPS>(f, rsc.s, rsc.rs, rsc.fast_ok, code);
+        *reinterpret_cast<uint2*>(xs + m * pitch + v * 8) = make_uint2(code[0], code[1]);
+      }
+    }
+  } else if constexpr (BF16) {
     RowsToLds<true, RPW, VPL> xr;
     xr.issue(p.x, M, K, K, wave, GX_WAVES, lane);
     if constexpr (NORM) xr.issue_gamma(p.gamma, K, lane);
@@ -429,6 +477,20 @@ int launch_gemv_rows_swiglu(const GemvArgs& a, hipStream_t st) {
   static LdsOptIn unused;  // rows of at most 2048: never more than 64 KiB
   const int r = rows_per_workgroup(a.M, a.N, 32, 64);
   return launch_rows(table[r == 64][a.M > 8][a.gamma != nullptr][a.K > 1024], unused, a, r == 64 ? 2 : 4, r, a.N / 2, r / 2, st);
+}
+
+// Rows from a.parts: M <= 8, K <= 2048.
+int launch_gemv_rows_attn(const GemvArgs& a, hipStream_t st) {
+#define AQ_GX(KS, R)                                                                                                             \
+  {gemv_rows_kernel<KS, R, true, 1, 4, false, false, false, 8>, gemv_rows_kernel<KS, R, true, 1, 4, false, false, false, 4>,     \
+   gemv_rows_kernel<KS, R, true, 1, 4, false, false, false, 2>, gemv_rows_kernel<KS, R, true, 1, 4, false, false, false, 1>}
+  static const rows_kernel_t table[4][4] = {AQ_GX(8, 8), AQ_GX(8, 16), AQ_GX(4, 16), AQ_GX(2, 16)};
+#undef AQ_GX
+  static LdsOptIn unused;  // 8 rows of at most 2048: never more than 64 KiB
+  const int rows = rows_per_workgroup(a.M, a.N, 8, 64);
+  const int shape = rows == 8 ? 0 : rows == 16 ? 1 : rows == 32 ? 2 : 3;
+  const int wpr = a.M <= 1 ? 0 : a.M <= 2 ? 1 : a.M <= 4 ? 2 : 3;
+  return launch_rows(table[shape][wpr], unused, a, shape < 2 ? 8 : shape == 2 ? 4 : 2, rows, a.N, rows, st);
 }
 
 }  // namespace aq

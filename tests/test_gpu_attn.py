@@ -627,3 +627,27 @@ def test_paged_attn_decode_infinite_values_stay_in_their_dimension(Hq, Hkv, D):
         assert bool((out[..., dim].float() == val).all())
         keep = torch.arange(D) != dim
         assert torch.equal(out[..., keep].view(torch.int16), clean[..., keep].view(torch.int16))
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("N", [40, 3000, 5000, 9001])
+@pytest.mark.parametrize("heads,D,T", [(3, 64, 300), (9, 128, 1024), (16, 128, 700), (25, 64, 257)])
+def test_output_projection_on_partials_by_shape_of_workgroup(M, N, heads, D, T):
+    """One to eight rows, 8 to 64 weight rows per workgroup, rows whose last vectors leave wavefronts without work: the bits of
+    the merged attention followed by the decode GEMV.  One sequence is empty-handed in its later slices."""
+    _say("partials by shape", M, N, heads, D, T)
+    K, P, page = heads * D, 5, 256
+    g = torch.Generator().manual_seed(M * N + K)
+    qkv = torch.randn(M, 3 * K, generator=g).to(torch.bfloat16).to(DEV)
+    ang = torch.rand(M, D // 2, generator=g) * 6.28
+    freqs = torch.polar(torch.ones_like(ang), ang).to(DEV)
+    kc, vc = (torch.randn(P * M, page, heads, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    table = torch.randperm(P * M, generator=g).view(M, P).to(DEV)
+    lens = torch.tensor([T] * (M - 1) + [17]).to(DEV)
+    wq = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).to(DEV)
+    sw = (torch.rand(N, generator=g) * 0.01 + 1e-3).to(DEV)
+    bias, res = torch.randn(N, generator=g).to(DEV), torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV)
+    attn = ops.rope_paged_attn_decode(qkv, freqs, table, T, kc, vc, heads, heads, seq_lens=lens)
+    parts = ops.rope_paged_attn_decode(qkv, freqs, table, T, kc, vc, heads, heads, seq_lens=lens, partials=True)
+    want = ops.gemv_w8a8_decode(attn.view(M, K), wq, sw, bias, residual=res)
+    assert torch.equal(ops.gemv_w8a8_attn(parts, wq, sw, bias, residual=res), want)
