@@ -40,6 +40,22 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return *reinterpret_cast<const uint32_t*>(&b);
 }
 
+// The values of lanes l and l ^ 16 (l ^ 32), in one order for both: for sums and maxima, which take them in any.  A row (half) swap is
+// one instruction; the same exchange through LDS (ds_bpermute) is a round trip.
+struct LanePair {
+  float x, y;
+};
+__device__ __forceinline__ LanePair lanes16_pair(float v) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r.x), __uint_as_float(r.y)};
+}
+__device__ __forceinline__ LanePair lanes32_pair(float v) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r.x), __uint_as_float(r.y)};
+}
+
 // Maximum of a non-negative value over the 64 lanes, returned in every lane
 // (as a wavefront-uniform scalar).  Four DPP steps (quad swaps, then the
 // half-row and row mirrors) leave each row of 16 lanes holding its maximum;

@@ -79,9 +79,9 @@ __device__ __forceinline__ float wave_sum_butterfly(float v) {
   v = __fadd_rn(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false)));
   v = __fadd_rn(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false)));
   v = __fadd_rn(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false)));
-  v = __fadd_rn(v, __shfl_xor(v, 16, 64));
-  v = __fadd_rn(v, __shfl_xor(v, 32, 64));
-  return v;
+  const LanePair r16 = lanes16_pair(v);
+  const LanePair r32 = lanes32_pair(__fadd_rn(r16.x, r16.y));
+  return __fadd_rn(r32.x, r32.y);
 }
 
 // 1 / sqrt(mean(x^2) + eps) of a row from its sum of squares: correctly rounded divide, add,

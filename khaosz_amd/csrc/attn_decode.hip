@@ -119,18 +119,6 @@ constexpr int ATT_KPG = ATT_WAVES * ATT_KPW; // positions per workgroup
 constexpr int ATT_MAX_D = 128;
 constexpr float ATT_MASKED = -1.0e30f;  // score (exp2 domain) of a cached position the sequence may not attend to
 
-// the value 16 / 32 lanes away (lane ^ 16, lane ^ 32)
-__device__ __forceinline__ float lanes16_other(float v) {
-  typedef unsigned u2 __attribute__((ext_vector_type(2)));
-  const u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float((threadIdx.x & 16) ? r.x : r.y);
-}
-__device__ __forceinline__ float lanes32_other(float v) {
-  typedef unsigned u2 __attribute__((ext_vector_type(2)));
-  const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float((threadIdx.x & 32) ? r.x : r.y);
-}
-
 typedef __bf16 attn_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float attn_f32x4 __attribute__((ext_vector_type(4)));
 
@@ -229,8 +217,9 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       ss[ks] = chunk_sumsq(v[ks]);
-      ss[ks] = __fadd_rn(ss[ks], __shfl_xor(ss[ks], 16, 64));  // c ^ 1
-      ss[ks] = __fadd_rn(ss[ks], __shfl_xor(ss[ks], 32, 64));  // c ^ 2
+      const LanePair c1 = lanes16_pair(ss[ks]);                  // c ^ 1
+      const LanePair c2 = lanes32_pair(__fadd_rn(c1.x, c1.y));  // c ^ 2
+      ss[ks] = __fadd_rn(c2.x, c2.y);
     }
     float tot = __fadd_rn(ss[0], ss[1]);                            // c ^ 4
     if constexpr (KS == 4) tot = __fadd_rn(tot, __fadd_rn(ss[2], ss[3]));  // c ^ 8
@@ -394,8 +383,9 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, pv[t][r]);
-    mx = fmaxf(mx, lanes16_other(mx));
-    mx = fmaxf(mx, lanes32_other(mx));  // finite: position t0 is valid
+    const LanePair m16 = lanes16_pair(mx);
+    const LanePair m32 = lanes32_pair(fmaxf(m16.x, m16.y));
+    mx = fmaxf(m32.x, m32.y);  // finite: position t0 is valid
     float part[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -406,9 +396,9 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
         part[r] += pv[t][r];
       }
     }
-    float sum = (part[0] + part[1]) + (part[2] + part[3]);
-    sum += lanes16_other(sum);
-    sum += lanes32_other(sum);
+    const LanePair s16 = lanes16_pair((part[0] + part[1]) + (part[2] + part[3]));
+    const LanePair s32 = lanes32_pair(s16.x + s16.y);
+    const float sum = s32.x + s32.y;
     if (col < GP) {
 #pragma unroll
       for (int t = 0; t < 4; ++t)

@@ -330,7 +330,8 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
       for (int kt = 0; kt < NT; ++kt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) bm = fmaxf(bm, s[kt][r]);
-      bm = fmaxf(bm, __shfl_xor(bm, 32, 64)) * p.scale_log2e;
+      const LanePair b2 = lanes32_pair(bm);
+      bm = fmaxf(b2.x, b2.y) * p.scale_log2e;
     }
     // The running maximum only has to bound the exponents, not equal the true maximum: it is raised (and the
     // accumulators rescaled) only when some query of the wavefront would otherwise see an exponent above 2^8;
@@ -425,7 +426,8 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
             o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv[dt][kk], __builtin_bit_cast(pa_bf16x8, pf[kk >> 1][kk & 1]), o[dt], 0, 0, 0);
     }
   }
-  l += __shfl_xor(l, 32, 64);
+  const LanePair l2 = lanes32_pair(l);
+  l = l2.x + l2.y;
   // ---- normalise and store: register r of tile dt is dimension 32 dt + 8 (r / 4) + 4 g + r % 4 of query col
   if (qpos < S && sums) {
     const float inv = 1.0f / l;
