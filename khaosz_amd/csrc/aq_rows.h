@@ -101,7 +101,12 @@ __device__ __forceinline__ float rms_scale(float ss, float k, float eps) {
 // squares of its vectors lane, lane + 64, ... in ascending order, elements in
 // memory order, then the butterfly): the arithmetic of the stand-alone
 // norm-and-quantise kernel, bit for bit.  gamma is requested by issue_gamma().
-template <bool BF16, int RPW, int VPL>
+// WHOLE: a row's vectors are rounded without a branch around each, only the stores are masked.  Zeros past the row can cost less
+// than a branch, which ends the stretch that is scheduled together: gemv_rows_kernel takes 5.0 us for 4 x 6912 -> 1536, 5.4 with a
+// branch around each vector, 6.1 for 8 x 5632 -> 2048, 6.4, and 4.5 for 8 x 2048 -> 3072 with the norm, 4.6.  Wavefronts of two rows,
+// whose time goes into the zeros too, lose (11 x 1536 -> 2048 with the norm 4.9 us, 4.7), and so do the vector ALU's short
+// kernels (0.03).
+template <bool BF16, int RPW, int VPL, bool WHOLE = false>
 struct RowsToLds {
   static constexpr int EPV = RowIn<BF16>::EPV;
   uint4 c[RPW][VPL];
@@ -175,21 +180,41 @@ struct RowsToLds {
       constexpr int STEPS = quant_steps<BF16, NORM>();
       const RowScale rsc = row_scale<STEPS>(wave_max(amax));
       if (lane == 0 && m < M) sx[m] = rsc.s;
-#pragma unroll
-      for (int i = 0; i < VPL; ++i) {
+      auto store = [&](int i, const uint32_t* code) {
         const int v = i * 64 + lane;
-        if (v < nvec) {
-          float f[EPV];
-          uint32_t code[EPV / 4];
-          values<NORM>(j, i, r, f);
-          quant_codes_packed<EPV, STEPS>(f, rsc.s, rsc.rs, rsc.fast_ok, code);  // zero rows give zero codes
-          uint8_t* dst = xs + m * pitch + v * EPV;
-          if constexpr (BF16) {
-            *reinterpret_cast<uint2*>(dst) = make_uint2(code[0], code[1]);
-          } else {
-            *reinterpret_cast<uint32_t*>(dst) = code[0];
+        uint8_t* dst = xs + m * pitch + v * EPV;
+        if (v >= nvec) return;
+        if constexpr (BF16) {
+          *reinterpret_cast<uint2*>(dst) = make_uint2(code[0], code[1]);
+        } else {
+          *reinterpret_cast<uint32_t*>(dst) = code[0];
+        }
+      };
+      if constexpr (!WHOLE) {
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+          if (i * 64 + lane < nvec) {
+            float f[EPV];
+            uint32_t code[EPV / 4];
+            values<NORM>(j, i, r, f);
+            quant_codes_packed<EPV, STEPS>(f, rsc.s, rsc.rs, rsc.fast_ok, code);  // zero rows give zero codes
+            store(i, code);
           }
         }
+      } else {
+        uint32_t code[VPL][EPV / 4];
+        auto round = [&](bool fast) {
+#pragma unroll
+          for (int i = 0; i < VPL; ++i) {
+            float f[EPV];
+            values<NORM>(j, i, r, f);
+            quant_codes_packed<EPV, STEPS>(f, rsc.s, rsc.rs, fast, code[i]);
+          }
+        };
+        if (__builtin_expect(rsc.fast_ok, 1)) round(true);
+        else round(false);
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) store(i, code[i]);
       }
     }
   }

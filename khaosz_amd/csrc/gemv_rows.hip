@@ -178,7 +178,7 @@ __global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
       }
     }
   } else if constexpr (BF16) {
-    RowsToLds<true, RPW, VPL> xr;
+    RowsToLds<true, RPW, VPL, RPW == 1> xr;
     xr.issue(p.x, M, K, K, wave, GX_WAVES, lane);
     if constexpr (NORM) xr.issue_gamma(p.gamma, K, lane);
     asm volatile("" ::: "memory");  // request order: token rows, epilogue operands, the weight stream
