@@ -77,6 +77,24 @@ __device__ __forceinline__ float wave_max(float v) {
   return __uint_as_float(ab > cd ? ab : cd);
 }
 
+// The same for unsigned numbers.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+#define AQ_DPP_MAX(ctrl)                                                                                 \
+  {                                                                                                      \
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, ctrl, 0xf, 0xf, false);     \
+    x = x > o ? x : o;                                                                                   \
+  }
+  AQ_DPP_MAX(0xB1)
+  AQ_DPP_MAX(0x4E)
+  AQ_DPP_MAX(0x141)
+  AQ_DPP_MAX(0x140)
+#undef AQ_DPP_MAX
+  const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)x, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)x, 16);
+  const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)x, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)x, 48);
+  const uint32_t ab = a > b ? a : b, cd = c > d ? c : d;
+  return ab > cd ? ab : cd;
+}
+
 // Exact definition: q = clamp(rint(a / s), -127, 127), correctly rounded divide,
 // round-half-to-even.  Returned as a 32-bit pattern whose low byte is the code.
 __device__ __forceinline__ uint32_t quant_code_exact(float a, float s) {

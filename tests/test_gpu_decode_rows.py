@@ -81,3 +81,26 @@ def test_up_gate_swiglu_is_the_separate_launches(M, F, K, norm):
     u, gate = ug[:, :F], ug[:, F:]
     want = u * (gate / (1 + torch.exp(-gate)))
     assert torch.allclose(h.float(), want, rtol=8e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("M,K", [(8, 6912), (9, 4112), (11, 6912), (16, 8192), (16, 2048)])
+def test_rows_with_nan_and_infinities_equal_single_rows(M, K):
+    """The row maximum by bits (more rows than keep their floats in registers) and by floats: NaN is left out of both, infinities and
+    denormals count.  A batch gives each row what the row gives alone."""
+    x = _rows(M, K, M * K).to(BF16)
+    x[0, K - 1] = float("nan")
+    x[1, 5], x[1, K // 2] = float("nan"), 1e4
+    x[2, 77] = float("-inf")
+    x[3] = float("nan")
+    x[4], x[5] = 0.0, -0.0
+    x[6] *= 1e-38
+    x[7, 0], x[7, 1] = float("-nan"), float("inf")
+    x[M - 1, 3] = -3e38
+    wq = torch.randint(-127, 128, (300, K), generator=torch.Generator().manual_seed(K), dtype=torch.int8).to(DEV)
+    sw = (torch.rand(300, generator=torch.Generator().manual_seed(5)) * 1e-3).to(DEV)
+    x = x.to(DEV)
+    got = ops.gemv_w8a8_decode(x, wq, sw).float()
+    want = torch.cat([ops.gemv_w8a8_decode(x[m:m + 1], wq, sw) for m in range(M)]).float()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+    assert bool(got[:2].isfinite().all()) and bool((got[4:6] == 0).all())
