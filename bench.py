@@ -332,7 +332,7 @@ def bench_prefill(torch, ops, args, dev):
         "workload": f"prefill_linear_w8a8 M={M} K={K} N={N} quantise + int8 MFMA GEMM + scale/bias epilogue, bf16 out",
         "value": tops, "unit": "TOPS", "ms_per_step": ms, "ms_per_step_p10_p50_p90": d_step, "ops_per_step": ops_alg,
         "dtype": "int8",
-        "roofline": {"bound": "mfma", "kernel": "gemm_kernel<int8,bf16>", "achieved": tops_k, "peak": PEAK_INT8_TOPS,
+        "roofline": {"bound": "mfma", "kernel": "gemm_walk_kernel<int8,bf16>", "achieved": tops_k, "peak": PEAK_INT8_TOPS,
                      "unit": "TOP/s", "frac": tops_k / PEAK_INT8_TOPS, "traffic": traffic, "traffic_source": traffic_src,
                      "kernel_us": ms_k * 1e3, "kernel_us_p10_p50_p90": [v * 1e3 for v in d_k],
                      "algorithmic_ops": ops_alg, **cond, **mfma_ceiling_fields(tops_k, False, clock_mhz),

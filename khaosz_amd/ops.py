@@ -546,8 +546,8 @@ class AttnPartials(NamedTuple):
 GEMV_ATTN_MAX_ROWS, GEMV_ATTN_MAX_K, GEMV_ATTN_MAX_SLICES = 8, 2048, 4
 GEMV_ATTN_SLICE = 256  # positions of a slice
 # Every workgroup of the projection repeats the merge of all rows, so it pays only while that is little work
-# (rows x row length x slices): 4 x 1536 x 3 saves 1.2 us per step over the separate merge launch, 8 x 2048 x 3
-# loses 0.8 us.
+# (rows x row length x slices): 4 x 1536 x 3 saves 0.3 us per step over the separate merge launch, 1 x 1536 x 3 1.2,
+# 8 x 2048 x 3 loses 1.2 us.
 GEMV_ATTN_MAX_WORK = 32768
 
 
