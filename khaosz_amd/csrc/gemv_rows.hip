@@ -14,10 +14,10 @@
 // the descriptor) returns zero without touching memory but still takes its turn in the address path: with a fixed 16
 // weight loads per lane and the epilogue's operands asked for by one wavefront in KS (20 small loads, most empty), the
 // same kernel took 1.5 to 2.5 us longer.  Measured (us, graph replay, weights from HBM, before -> now):
-//   bf16 16 x 2048 -> 8192 8.1 -> 6.5, 11 x 1536 -> 1536 5.9 -> 3.8, 8 x 2048 -> 3072 5.0 -> 3.95, 8 x 5632 -> 2048 7.3 -> 6.3;
-//   rows that took a quantiser launch of their own: 11 x 6912 -> 1536 13.6 -> 8.0, 16 x 1840 -> 9152 15.7 -> 8.9,
+//   bf16 16 x 2048 -> 8192 8.1 -> 6.5, 11 x 1536 -> 1536 5.9 -> 3.8, 8 x 2048 -> 3072 5.0 -> 3.9, 8 x 5632 -> 2048 7.3 -> 6.1;
+//   rows that took a quantiser launch of their own: 11 x 6912 -> 1536 13.6 -> 7.7, 16 x 1840 -> 9152 15.7 -> 8.9,
 //   11 x 5712 -> 4832 20.4 -> 13.8, fp32 8 x 6912 -> 1536 25 -> 8.3, 8 x 1536 -> 1536 6.7 -> 3.7;
-//   FP8 8 x 2048 -> 8192 7.4 -> 5.8, 4 x 688 -> 3520 8.7 -> 3.3, 8 x 6912 -> 1536 17.5 -> 8.4;
+//   FP8 8 x 2048 -> 8192 7.4 -> 5.6, 4 x 688 -> 3520 8.7 -> 3.0, 8 x 6912 -> 1536 17.5 -> 8.2;
 //   up/gate + SwiGLU with the norm: 4 x 1536 -> 2 x 6912 7.3 -> 6.4, 8 x 2048 -> 2 x 5632 8.2 -> 7.6.
 #include <type_traits>
 
