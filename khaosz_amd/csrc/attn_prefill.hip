@@ -246,6 +246,8 @@ __global__ __launch_bounds__(QW* KW * 64) __attribute__((amdgpu_waves_per_eu(2))
         x[i] = chunk_normed(x[i], rms_scale(head_sumsq<D>(x[i]), (float)D, p.eps), *reinterpret_cast<const uint4*>(p.q_gain + piece * 8));
       *reinterpret_cast<uint4*>(mine + row * ROWB + ((piece ^ row_key<D>(row)) << 4)) = x[i];
     }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): other lanes' pieces are read next (the rows are this wavefront's own: no barrier)
+    asm volatile("" ::: "memory");
 #pragma unroll
     for (int st = 0; st < DSTEPS; ++st)
       qf[st] = *reinterpret_cast<const uint4*>(mine + col * ROWB + (((2 * st + g) ^ row_key<D>(col)) << 4));
