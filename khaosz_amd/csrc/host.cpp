@@ -773,11 +773,16 @@ struct Block {
   void lay_out();
   bool few() const { return M <= types.decode_rows; }
   bool step() const { return S == 1; }
-  // Whether a prompt's attention rotates its queries itself: from 8 MB of them on, which then are not written and read back.  With
-  // less, the launch that rotates takes the same few microseconds whatever it moves, and rotating is one more link in the attention
-  // launch's chain: us a block, rotated before -> in attention: 8 x 512 tokens of 16 heads of 128 (16.8 MB) 274.4 -> 270.7; 24 layers:
-  // 4 x 512 of 24 heads of 64 (6.3 MB) 3703 -> 3687, 2 x 150 (0.9 MB) 1680 -> 1706; 2 x 82 on 21 cached, qk-norm (0.7 MB) 58.9 -> 61.9.
-  bool rotates() const { return !step() && M * Hq * D >= (int64_t(4) << 20); }
+  // Whether a prompt's attention rotates its queries itself, which then are not written and read back: from 4 MB of them on, 8 MB with
+  // qk-norm.  With less, the launch that rotates takes the same few microseconds whatever it moves, and rotating (qk-norm: and a sum
+  // over the head) is one more link in the attention launch's chain.  us a block, rotated before -> in attention:
+  //   16 heads of 128, MB of queries: 1.0 64.1 -> 64.6, 2.8 96.7 -> 97.3, 3.1 104.4 -> 104.1, 4.2 108.5 -> 108.4, 4.6 124.2 -> 123.6,
+  //     5.9 137.0 -> 136.2, 8.4 156.9 -> 154.6, 16.4 268.1 -> 264.6; with qk-norm 3.9 104.8 -> 106.6, 5.6 139.7 -> 141.3, 7.9 160.1 ->
+  //     161.1, 8.4 157.1 -> 156.5, 10.5 189.7 -> 189.0, 16.8 271.8 -> 268.2;
+  //   24 heads of 64: 0.8 58.4 -> 59.1, 2.1 83.8 -> 83.6, 2.9 108.6 -> 109.1, 3.9 116.2 -> 115.6, 4.7 125.3 -> 124.7, 6.3 143.5 -> 142.3, 8.4 186.4
+  //     -> 184.3; with qk-norm 3.1 99.8 -> 101.1, 6.3 146.3 -> 146.6, 7.9 168.5 -> 167.6, 11.8 222.0 -> 219.4.
+  // (48 + 52 sizes, on an empty cache and on top of tokens; on this side of the line 0.2 to 1.5 % faster, one in ten level or 0.4 % slower.)
+  bool rotates() const { return !step() && M * Hq * D >= (int64_t(qk_norm ? 4 : 2) << 20); }
   bool merge() const { return step() && merge_in_projection(B, Hq * D, total); }
   int queue(const void* in, void* out, char* base, const char** what) const;  // allocates nothing: runs without the interpreter lock
 };

@@ -66,6 +66,31 @@ def test_block_in_one_call_is_the_step_by_step_path(monkeypatch, qk_norm, B, S, 
         assert torch.equal(a, c)
 
 
+@pytest.mark.parametrize("hidden,qk_norm,B,S,cached", [
+    (512, False, 4, 1023, 0), (512, False, 4, 1025, 0), (512, False, 5, 900, 37), (512, True, 8, 1023, 0), (512, True, 8, 1025, 0),
+    (512, True, 9, 950, 70), (1024, False, 3, 683, 0), (1024, False, 4, 600, 51), (1024, True, 5, 820, 0), (1024, True, 6, 700, 100)])
+def test_block_that_rotates_queries_in_attention_is_the_step_by_step_path(monkeypatch, hidden, qk_norm, B, S, cached):
+    """Prompts on both sides of the sizes from which the block has the attention rotate (and normalise) its queries."""
+    d = hidden // 8
+    b = _block(hidden=hidden, use_qk_norm=qk_norm)
+    if qk_norm:
+        with torch.no_grad():
+            for norm in (b.attention.q_norm, b.attention.k_norm):
+                norm.weight.copy_(torch.rand(d, device=DEV) + 0.5)
+    x, fr, cache, table = _case(b, B, S, cached, d=d, page=64)
+    cache.bind(table, cached + S)
+    k0, v0 = cache.k_layers.clone(), cache.v_layers.clone()
+    with torch.inference_mode():
+        got = b(x, fr, None, cache), cache.k_layers.clone(), cache.v_layers.clone()
+        cache.k_layers.copy_(k0)
+        cache.v_layers.copy_(v0)
+        calls = _counted(monkeypatch, ops, "rope_kv_write")  # a replaced operator: the step-by-step path serves
+        want = b(x, fr, None, cache), cache.k_layers, cache.v_layers
+    assert len(calls) == 1
+    for a, c in zip(got, want):
+        assert torch.equal(a, c)
+
+
 def test_hooks_on_a_fused_blocks_children_still_run():
     b = _block()
     x, fr, cache, table = _case(b, 2, 1, 30)
