@@ -407,16 +407,20 @@ static size_t gemv_rows_lds(int64_t M, int64_t K, int ks, int rows_per_wg) {
   return codes < sums ? sums : codes;
 }
 
-// Weight rows per workgroup.  A workgroup's time grows with the token rows it rounds and with the weight rows it streams, a
-// token row costing as much as 7/4 weight rows of the same length (46 and 26 ps per element, fitted to 14 shapes x 5
-// batches x 4 row counts), and a round of workgroups over the compute units repeats the rounding: the fewest rounds x
-// (7 M + 4 rows).  Within 10 % of the best of the four at every point measured.
-static int rows_per_workgroup(int64_t M, int64_t N, int least, int most) {
-  const int64_t cus = device_cus();
+// Weight rows per workgroup: the fewest rounds of workgroups over the compute units x what a workgroup takes.  Rows of more
+// than 2048 take 130 to 240 registers: one workgroup to a unit, every round begins with the latency of its rows and rounds them
+// again, 8 M + 4 r + 64 quarters of a weight row (`alone`: rows with the norm or SwiGLU, too).  Shorter rows as they are take 50
+// to 90: two or three workgroups share a unit, a round starts under the one before, 5 M + 4 r + 12.  Fitted to 10 600 random sizes
+// of all kinds (N 512..11264, K 512..8192, 1 to 16 rows, attention rows too): 0.2 % from the best of the four in the mean, 1 in 50
+// more than 4 %, 15 % at most.  us, with 7 M + 4 r for all -> so: fp32 2 x 2592 -> 8352 23.2 -> 11.0, 1 x 6864 -> 4352 18.7 -> 14.1; FP8
+// 1 x 4576 -> 9696 27.0 -> 16.7, 2 x 4816 -> 4560 17.1 -> 11.6, 1 x 512 -> 4848 4.08 -> 3.62; int8 3 x 3328 -> 10720 11.4 -> 9.8; norm 3 x 1408 ->
+// 9408 6.7 -> 6.0; SwiGLU 14 x 2048 -> 2 x 8416 18.5 -> 17.0.  With the larger cost for short rows 3 x 864 -> 10832 4.55 -> 5.08.
+static int rows_per_workgroup(int64_t M, int64_t N, bool alone, int least, int most) {
+  const int64_t cus = device_cus(), fixed = alone ? 8 * M + 64 : 5 * M + 12;
   int best = most;
   int64_t cost = INT64_MAX;
   for (int r = least; r <= most; r *= 2) {
-    const int64_t c = ((N + r - 1) / r + cus - 1) / cus * (7 * M + 4 * r);
+    const int64_t c = ((N + r - 1) / r + cus - 1) / cus * (fixed + 4 * r);
     if (c < cost) cost = c, best = r;
   }
   return best;
@@ -476,7 +480,7 @@ bool gemv_rows_ok(RowsKind kind, int64_t M, int64_t K) {
 }
 
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {
-  switch (rows_per_workgroup(a.M, a.N, 8, 64)) {
+  switch (rows_per_workgroup(a.M, a.N, kind == ROWS_I8_NORM || a.K > 2048, 8, 64)) {
     case 8: return launch_shape<8, 8>(a, kind, st);
     case 16: return launch_shape<8, 16>(a, kind, st);
     case 32: return launch_shape<4, 16>(a, kind, st);
@@ -493,7 +497,7 @@ int launch_gemv_rows_swiglu(const GemvArgs& a, hipStream_t st) {
 #undef AQ_GX2
 #undef AQ_GX
   static LdsOptIn unused;  // rows of at most 2048: never more than 64 KiB
-  const int r = rows_per_workgroup(a.M, a.N, 32, 64);
+  const int r = rows_per_workgroup(a.M, a.N, true, 32, 64);
   return launch_rows(table[r == 64][a.M > 8][a.gamma != nullptr][a.K > 1024], unused, a, r == 64 ? 2 : 4, r, a.N / 2, r / 2, st);
 }
 
@@ -505,7 +509,10 @@ int launch_gemv_rows_attn(const GemvArgs& a, hipStream_t st) {
   static const rows_kernel_t table[4][4] = {AQ_GX(8, 8), AQ_GX(8, 16), AQ_GX(4, 16), AQ_GX(2, 16)};
 #undef AQ_GX
   static LdsOptIn unused;  // 8 rows of at most 2048: never more than 64 KiB
-  const int rows = rows_per_workgroup(a.M, a.N, 8, 64);
+  // 3 or 4 rows of up to 1024 in 2 or 3 slices: 16 weight rows at least, us with 8 -> 16: 3 x 704 -> 704 4.10 -> 3.65, 4 x 256 -> 1056
+  // 4.05 -> 3.64, 3 x 960 -> 544 4.10 -> 4.23 (level at 4 slices; 2 and 5 to 8 rows 2 % slower with 16)
+  const bool few_bytes = (a.M == 3 || a.M == 4) && a.K <= 1024 && a.parts_ns < 4;
+  const int rows = rows_per_workgroup(a.M, a.N, false, few_bytes ? 16 : 8, 64);
   const int shape = rows == 8 ? 0 : rows == 16 ? 1 : rows == 32 ? 2 : 3;
   const int wpr = a.M <= 1 ? 0 : a.M <= 2 ? 1 : a.M <= 4 ? 2 : 3;
   return launch_rows(table[shape][wpr], unused, a, shape < 2 ? 8 : shape == 2 ? 4 : 2, rows, a.N, rows, st);
