@@ -823,7 +823,11 @@ static int g_forced_tile = 0;  // lab build only: TILE_AUTO = by shape, otherwis
 // most but for one size in a hundred (256 x 128 alone: 5 %, 43 %).  us, gemm_kernel's tiles -> 256 x 192 (256 x 128 of the walk):
 // 4096 x 3072 x 2048 31.5 -> 25.2 (30.2), FP8 27.6 -> 22.8 (27.5), 1476 x 6480 x 4448 72.5 -> 49.2 (69), 6263 x 1456 x 3696 63 -> 42.8
 // (59), 6952 x 1232 x 992 with a residual 30.2 -> 17.7 (26), FP8 2954 x 11104 x 4000 172 -> 142 (172); not 4096 x 11264 x 2048 (95, 109).
-static int choose_tile_for(int64_t M, int64_t N, int64_t cus, bool walk = false) {
+// With a residual, 256 x 192 takes 1.6 of a round: both types hold 48 bytes of it per lane beside 96 accumulators, and ask for a third
+// (int8) or all of it (FP8) only when the products are done.  At 1.45, of 600 random sizes with a residual it was 6 % slower than the
+// faster of the two for one in twenty, up to 19 %; now 0.25 % in the mean, 3 % for one in twenty (us, 256 x 192 | 256 x 128: FP8 3668 x 4864 x 512
+// 24.8 | 21.2, int8 4780 x 9200 x 3840 192 | 169, FP8 6678 x 10632 x 6032 472 | 509).
+static int choose_tile_for(int64_t M, int64_t N, int64_t cus, bool walk = false, bool res = false) {
   auto rounds = [cus](int64_t tiles, double last, double fill) {
     const int64_t full = tiles / cus, rest = tiles % cus;
     if (full == 0) return 1.0;
@@ -835,10 +839,10 @@ static int choose_tile_for(int64_t M, int64_t N, int64_t cus, bool walk = false)
     bool small;
     double last, fill;  // of a round, for a last one behind others
   };
-  static const Cand cands[] = {{TILE_LARGE, 256, 128, 15.0, false, 0.5, 0.5}, {TILE_SMALL, 128, 128, 10.8, false, 0.5, 0.5},
-                               {TILE_N64, 128, 64, 7.0, true, 0, 0},          {TILE_N32, 128, 32, 5.0, true, 0, 0},
-                               {TILE_M64N64, 64, 64, 4.6, true, 0, 0},        {TILE_M64N32, 64, 32, 3.5, true, 0, 0},
-                               {TILE_WIDE, 256, 192, 21.75, false, 0.7, 0.2}};
+  const Cand cands[] = {{TILE_LARGE, 256, 128, 15.0, false, 0.5, 0.5}, {TILE_SMALL, 128, 128, 10.8, false, 0.5, 0.5},
+                        {TILE_N64, 128, 64, 7.0, true, 0, 0},          {TILE_N32, 128, 32, 5.0, true, 0, 0},
+                        {TILE_M64N64, 64, 64, 4.6, true, 0, 0},        {TILE_M64N32, 64, 32, 3.5, true, 0, 0},
+                        {TILE_WIDE, 256, 192, res ? 24.0 : 21.75, false, 0.7, 0.2}};
   int best = TILE_LARGE;
   double cost = 0.0;
   for (const Cand& c : cands) {
@@ -859,11 +863,11 @@ static int choose_tile_for(int64_t M, int64_t N, int64_t cus, bool walk = false)
   return best;
 }
 
-static int choose_tile(int64_t M, int64_t N, bool walk) {
+static int choose_tile(int64_t M, int64_t N, bool walk, bool res) {
 #ifdef AQ_LAB
   if (g_forced_tile) return g_forced_tile;
 #endif
-  return choose_tile_for(M, N, device_cus(), walk);
+  return choose_tile_for(M, N, device_cus(), walk, res);
 }
 
 template <bool FP8, int OUT, class S>
@@ -900,7 +904,7 @@ static int launch(GemmArgs& a, hipStream_t st) {
     if (!forced && huge_fp8_ok(a)) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
   }
   const bool walk = OUT != OUT_I32 && gemm_walk_ok(a, OUT);
-  const int tile = choose_tile(a.M, a.N, walk);
+  const int tile = choose_tile(a.M, a.N, walk, a.res != nullptr);
   if constexpr (OUT != OUT_I32) {
     if (walk && tile == TILE_LARGE && !forced) return gemm_walk_launch<FP8, OUT>(a, st, 128);
     if (walk && tile == TILE_WIDE) return gemm_walk_launch<FP8, OUT>(a, st, 192);

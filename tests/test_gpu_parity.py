@@ -1452,3 +1452,25 @@ def test_gemm_walk_tiles_give_the_bits_of_separate_tiles(M, N, K, kind):
         assert lab.aq_lab_set_gemm_tile(256) == 0
         for y, want in zip(got, run()):
             assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("kind", [192, 258])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_gemm_walk_tiles_add_to_a_residual_in_place(kind, fp8):
+    """The sum takes the residual's place, in tiles that ask for parts of it behind stores of others: ragged rows, several rounds."""
+    M, N, K = 4100, 5002, 528
+    _say("gemm walk in place", kind, fp8)
+    g = torch.Generator(device=DEV).manual_seed(kind + fp8)
+    if fp8:
+        x, w = (torch.randn(n, K, generator=g, device=DEV).to(torch.float8_e4m3fn).view(torch.uint8) for n in (M, N))
+    else:
+        x, w = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
+    sx, sw = (torch.rand(1 if fp8 else n, generator=g, device=DEV) * 0.01 + 1e-4 for n in (M, N))
+    res = torch.randn(M, N, generator=g, device=DEV).to(torch.bfloat16)
+    op, entry = (ops.linear_fp8, "aq_linear_fp8_residual") if fp8 else (ops.linear_w8a8, "aq_linear_w8a8_residual")
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(kind) == 0
+        want = op(x, sx, w, sw, None, out_dtype=torch.bfloat16, residual=res)
+        assert getattr(lab, entry)(x.data_ptr(), sx.data_ptr(), w.data_ptr(), sw.data_ptr(), None, 0, res.data_ptr(), res.data_ptr(),
+                                   _abi.AQ_BF16, M, N, K, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(res, want)
