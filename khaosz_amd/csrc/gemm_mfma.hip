@@ -93,7 +93,7 @@ using ShapeN64 = Shape<2, 2, 2, 1, 1, 128, 4>;
 using ShapeN32 = Shape<4, 1, 1, 1, 1, 128, 4>;
 using ShapeM64N64 = Shape<2, 2, 1, 1, 1, 128, 4>;
 using ShapeM64N32 = Shape<2, 1, 1, 1, 1, 128, 6>;
-using ShapeHuge = Shape<2, 2, 4, 4, 1, 64, 4>;  // product: FP8 launches of two rounds or more (see huge_fp8_ok)
+using ShapeHuge = Shape<2, 2, 4, 4, 1, 64, 4>;  // product: large FP8 launches of odd 64-byte K steps (see huge_fp8_ok)
 #ifdef AQ_LAB
 using ShapeTall = Shape<2, 2, 4, 2, 1, 128, 3>;
 using ShapeHuge8 = Shape<4, 2, 2, 4, 1, 64, 4>;
@@ -882,15 +882,20 @@ static int launch_shape(GemmArgs& a, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// FP8 launches the 256 x 256 tile serves and gains on: whole 256-row multiples, even N, whole 64-byte K steps, no
-// residual (the tile's one K-loop and epilogue variant), and at least two rounds of such tiles over the compute
-// units (one round -- 4096^3 -- measured level with the 256 x 128 tile, 57.0 against 57.7 us) of more than 2048 in K: its loop
-// stops between tiles, gemm_walk_kernel's does not.  us, this | that: 8192^3 432 | 461, 4096 x 8192 x 4096 117 | 122,
-// 4096 x 11264 x 2048 90.7 | 91.5, 8192 x 4096 x 2048 63.8 | 60.8, 8192 x 6912 x 1536 93.6 | 82.1, 4096 x 8192 x 1024 39.8 | 36.2.
+// FP8 launches the 256 x 256 tile serves and gains on: whole 256-row multiples, even N, no residual (the tile's one K-loop and
+// epilogue variant), and, against the walked tiles at 3491 random sizes:
+// * K of an odd number of 64-byte steps: rows then begin in the middle of a line, which 128-byte steps bring in as two halves of
+//   lines and 64-byte steps do not.  K of whole lines never gains: 256 x 256 / the walked tiles, K 2049..2560 1.18, up to 4096 1.10, up
+//   to 8192 1.06, up to 16384 1.02 (us 5376 x 7278 x 2816 121 | 93, 4096 x 10688 x 3584 140 | 127, 8192^3 432 | 429, 4096 x 8192 x 4096 112 | 110).
+// * K above 3072: its loop stops between tiles, gemm_walk_kernel's does not: K 1024..2048 1.10, up to 2560 1.00, up to 3072 0.99,
+//   up to 4096 0.96, up to 5120 0.94, up to 8192 0.90 (us 4864 x 8640 x 3264 126 | 131, 7424 x 6440 x 5312 212 | 244, 7424 x 5760 x 8000 294 | 327).
+// * two rounds at least, and the last one more than half full: with less 1.04 to 1.14 at any K.
+// In all 6 % faster than the walk where it is taken, and the choice 2 % from the best tile in the mean (taken for any K above 2048
+// and any last round, 11 %).
 static bool huge_fp8_ok(const GemmArgs& a) {
-  if (a.K <= 2048 || (a.K % ShapeHuge::BK) != 0 || (a.N % 2) != 0 || (a.M % ShapeHuge::BM) != 0 || a.res != nullptr) return false;
-  const int64_t tiles = (int64_t)(a.M / ShapeHuge::BM) * ((a.N + ShapeHuge::BN - 1) / ShapeHuge::BN);
-  return tiles >= 2 * (int64_t)device_cus();
+  if (a.K <= 3072 || a.K % (2 * ShapeHuge::BK) != ShapeHuge::BK || (a.N % 2) != 0 || (a.M % ShapeHuge::BM) != 0 || a.res != nullptr) return false;
+  const int64_t tiles = (int64_t)(a.M / ShapeHuge::BM) * ((a.N + ShapeHuge::BN - 1) / ShapeHuge::BN), cus = device_cus();
+  return tiles >= 2 * cus && (tiles % cus == 0 || 2 * (tiles % cus) > cus);
 }
 
 template <bool FP8, int OUT>

@@ -469,15 +469,15 @@ def test_every_product_tile_on_the_shipped_library(oracle, kind):
         assert torch.equal(y8.cpu(), ref)
 
 
-def test_product_fp8_256x256_tile(oracle):
-    """FP8 launches of two rounds or more of 256 x 256 tiles take that tile in the shipped library (whole 256-row
-    multiples, even N, whole 64-byte K steps, no residual).  Exact-in-fp32 operands against a float product, a
-    random-data slab against the oracle within the FP8 tolerance, and the neighbouring shapes that must NOT take it
-    (ragged M, a residual) against the same references."""
+@pytest.mark.parametrize("K", [3136, 3200, 192])
+def test_product_fp8_256x256_tile(oracle, K):
+    """FP8 launches of two rounds or more of 256 x 256 tiles take that tile in the shipped library where it is the faster one
+    (whole 256-row multiples, even N, an odd number of 64-byte K steps above 3072, a last round more than half full, no residual):
+    K = 3136.  Exact-in-fp32 operands against a float product, a random-data slab against the oracle within the FP8
+    tolerance, and the neighbouring shapes that must NOT take it (other K, ragged M) against the same references."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    N, K = 2048 + 130, 192                      # ragged N (even), three K steps
-    M = 256 * ((2 * cus + (N + 255) // 256 - 1) // ((N + 255) // 256))
-    assert (M // 256) * ((N + 255) // 256) >= 2 * cus
+    N = 2048 + 130                              # ragged N (even)
+    M = 256 * next(m for m in range(1, 4 * cus) if 9 * m >= 2 * cus and (9 * m % cus == 0 or 2 * (9 * m % cus) > cus))
     _say("product fp8 256x256", M, N, K)
     gt = torch.Generator().manual_seed(305)
     b8 = torch.randint(0x30, 0x40, (N, K), generator=gt, dtype=torch.uint8)
