@@ -9,23 +9,7 @@
 namespace aq {
 
 // Rotates 8 consecutive elements (4 interleaved pairs): (x0 + i x1)(c + i s) with four rounded
-// products, one rounded difference and one rounded sum per pair.
-__device__ __forceinline__ uint4 rope8(uint4 x, const float* cs /* 4 (cos, sin) pairs */) {
-  const float4 a = *reinterpret_cast<const float4*>(cs), b = *reinterpret_cast<const float4*>(cs + 4);
-  const float c[4] = {a.x, a.z, b.x, b.z}, sn[4] = {a.y, a.w, b.y, b.w};
-  const uint32_t in[4] = {x.x, x.y, x.z, x.w};
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = __uint_as_float(in[i] << 16), x1 = __uint_as_float(in[i] & 0xffff0000u);
-    const float r0 = __fsub_rn(__fmul_rn(x0, c[i]), __fmul_rn(x1, sn[i]));
-    const float r1 = __fadd_rn(__fmul_rn(x0, sn[i]), __fmul_rn(x1, c[i]));
-    o[i] = pack_bf16x2(r0, r1);
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-// the same on table values already in registers
+// products, one rounded difference and one rounded sum per pair.  a, b: 4 (cos, sin) pairs.
 __device__ __forceinline__ uint4 rope8(uint4 x, float4 a, float4 b) {
   const float c[4] = {a.x, a.z, b.x, b.z}, sn[4] = {a.y, a.w, b.y, b.w};
   const uint32_t in[4] = {x.x, x.y, x.z, x.w};
@@ -38,6 +22,9 @@ __device__ __forceinline__ uint4 rope8(uint4 x, float4 a, float4 b) {
     o[i] = pack_bf16x2(r0, r1);
   }
   return make_uint4(o[0], o[1], o[2], o[3]);
+}
+__device__ __forceinline__ uint4 rope8(uint4 x, const float* cs) {
+  return rope8(x, *reinterpret_cast<const float4*>(cs), *reinterpret_cast<const float4*>(cs + 4));
 }
 
 // RMSNorm over the head dimension of a rotated query or key (attention.py:62-64, 86-89: after the rotation, before
