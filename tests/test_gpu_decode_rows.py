@@ -70,6 +70,26 @@ def test_fp8_rows_within_tolerance(oracle, M, N, K):
     assert np.max(np.abs(y - exact)) <= 1e-3 * np.sqrt(np.mean(exact.astype(np.float64) ** 2))
 
 
+# rows that are cast without a branch per vector and rows that are not, one and two to a wavefront, every length class
+@pytest.mark.parametrize("scale", [3e-26, 1e-22, 1.0, 7e21, 2e28])
+@pytest.mark.parametrize("M,K", [(1, 512), (8, 2048), (5, 4080), (8, 8192), (9, 1040), (16, 2048), (11, 4096)])
+def test_fp8_rows_are_cast_like_the_oracle(oracle, M, K, scale):
+    """The codes that the GEMV's own cast makes, read back through a weight of ones on the diagonal: scales on both sides of
+    [2^-64, 2^64], outside of which the cast takes the full divide, values on and next to the midpoints of e4m3."""
+    tab = oracle.np_e4m3fn_table().astype(np.float32)
+    steps = np.sort(np.unique(np.concatenate([tab[:127], (tab[:126] + tab[1:127]) / 2])))
+    g = torch.Generator().manual_seed(M * K)
+    x = torch.from_numpy(steps)[torch.randint(0, len(steps), (M, K), generator=g)] * (1 - 2 * torch.randint(0, 2, (M, K), generator=g))
+    x[:, ::3] = (torch.rand(M, (K + 2) // 3, generator=g) * 2 - 1) * 448
+    x[M - 1, K - 1] = -448.0  # the largest: the scale is the one asked for, but for its rounding to bf16
+    x = (x.double() * scale).to(BF16)
+    xq, sx = oracle.c_quant_tensor_fp8(_bits(x), bf16_bits=True)
+    w = torch.zeros(K, K, dtype=torch.uint8, device=DEV)
+    w.diagonal().fill_(0x38)
+    y = ops.gemv_fp8_decode(x.to(DEV), w, torch.ones(1, device=DEV), out_dtype=F32).cpu().numpy()
+    assert np.array_equal(y, tab[xq] * np.float32(sx))
+
+
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("M,F,K", [(1, 16, 512), (8, 48, 1024), (9, 4112, 512), (16, 6912, 1536), (5, 5632, 2048)])
 def test_up_gate_swiglu_is_the_separate_launches(M, F, K, norm):
