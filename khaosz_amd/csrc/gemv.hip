@@ -923,17 +923,24 @@ static int gemv_dispatch(const aq::GemvArgs& a, int mt, hipStream_t st) {
 }
 
 // One launch where a kernel quantises (and normalises) the rows itself; -1 when the shape takes two.
-// Up to 4 bf16 rows, the dot-product kernel: one wavefront rounds a row, the others start on their weights, and the few
-// products per weight dword are no load on the vector ALU (1 x 2048 -> 8192: 5.1 us against 5.8, 4 x 5712 -> 4832 9.6
-// against 10.7).  gemv_rows.hip for everything else: more rows; fp32 rows; 3 or 4 rows of a matrix of at most 2048 rows
-// (4 x 1536 -> 1536 3.44 -> 3.28) or of more than 8192, which the dot-product kernel walks in two and more rounds of
-// workgroups that repeat the rounding (4 x 1840 -> 9152 6.9 -> 6.6), any number of long ones there (1 x 8192 -> 11264
-// 23.8 -> 19.3), and the norm in front of a matrix of at most 4096 rows (4 x 1536 -> 2048 4.07 -> 3.70).
+// Up to 4 bf16 rows have two kernels.  The dot-product kernel: one wavefront rounds a row, the others start on their weights, and
+// the few products per weight dword are no load on the vector ALU; it keeps its place with many weights per row.  gemv_rows.hip
+// for everything else: more rows; fp32 rows; rows of up to 1024 (3 and 4 of them, or of many weight rows); rows of 2049 to 4096,
+// which the dot-product kernel holds in registers for 8192 and, on short matrices, does not cut into K parts; longer ones of
+// 2049 to 4096 weight rows, too many for those parts.
+// Timed on both at 7433 random sizes, 1 to 4 rows, N 512..11264, K 512..8192, with the norm up to 2048: what this picks is 0.4 % from
+// the faster one in the mean, 3.4 % for one in twenty.  us, this | the other: 1 x 3168 -> 1472 4.0 | 5.6, 4 x 3008 -> 1488 4.0 | 5.7, 1 x 6016
+// -> 3440 6.7 | 7.8, 1 x 896 -> 9536 4.5 | 5.0, 4 x 1616 -> 1504 3.4 | 3.6; dot products 1 x 1968 -> 5648 4.5 | 5.5, 1 x 6880 -> 1585 4.8 | 5.9, 1 x
+// 7088 -> 9312 18.0 | 21.6, 4 x 5024 -> 9600 15.0 | 15.9; with the norm 4 x 800 -> 10032 4.9 | 5.9, dot products 1 x 1744 -> 5839 4.4 | 5.1.
+// (Where the two are within 4 % alone, the norm in front of a short matrix and 3 or 4 long rows to one, rows follow what wrote them:
+// the 24-layer step of 4 with 6912 -> 1536 here 648 us, by dot products 657.)
 static bool dot_kernel_better(int64_t M, int64_t N, int64_t K, bool norm) {
   if (M > 4) return false;
-  if (norm) return N > 4096 && (M < 3 || N <= 8192);
-  if (N > 8192) return M < 3 && K <= 4096;
-  return M < 3 || N > 2048;
+  if (norm) return K > 1024 && N > 4096 && (M < 3 || N <= 8192);
+  if (K <= 1024) return M < 3 && N <= 8192;
+  if (K <= 2048) return M < 3 || N > 2048;
+  if (K <= 4096) return N > 4096 && N <= 8192;
+  return N > 4096 || (M < 3 && N <= 2048);
 }
 
 enum FusedRoute { FUSED_NONE, FUSED_DOT, FUSED_ROWS };

@@ -26,7 +26,9 @@ CASES = [(5, 1, 16), (8, 9, 112), (9, 33, 128), (16, 7, 144), (1, 2049, 1024), (
          (7, 8201, 2064), (16, 8193, 528), (9, 1537, 4096), (16, 520, 4112), (3, 9000, 4128), (12, 100, 8176), (16, 16, 8192),
          (2, 8208, 8192), (6, 16385, 272),
          # few rows of a matrix of two rounds and more, short rows and long ones (which count their rounds differently)
-         (3, 500, 8192), (5, 2500, 4608), (2, 4600, 2400), (3, 9001, 1040), (4, 8300, 2064), (1, 4353, 6864)]
+         (3, 500, 8192), (5, 2500, 4608), (2, 4600, 2400), (3, 9001, 1040), (4, 8300, 2064), (1, 4353, 6864),
+         # up to 4 rows, where the dot-product kernel takes over and where it does not
+         (2, 3000, 6000), (1, 1500, 3168), (4, 6000, 3200), (2, 4097, 1040)]
 
 
 @pytest.mark.parametrize("dtype", [BF16, F32])

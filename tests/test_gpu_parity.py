@@ -161,7 +161,7 @@ def test_bf16_rows_one_product_rounding_for_every_mantissa_of_the_maximum(oracle
 
 def test_bf16_rows_one_product_rounding_inside_the_decode_kernels(oracle):
     """The same rows (every mantissa of the maximum, every value up to it) through the kernels that quantise
-    their rows themselves: 16 rows a call through the matrix-core GEMV, 8 and 3 through the dot-product one.
+    their rows themselves: 16 and 8 rows a call through the matrix-core GEMV, 2 through the dot-product one.
     The weight is the identity, so the output is the codes times the row's scale, exactly."""
     K = 2048
     wq = torch.eye(K, dtype=torch.int8, device=DEV)
@@ -171,7 +171,7 @@ def test_bf16_rows_one_product_rounding_inside_the_decode_kernels(oracle):
         qo, so = oracle.c_quant_rowwise_i8(bits, bf16_bits=True)
         want = qo.astype(np.float32) * so[:, None]
         xd = torch.from_numpy(bits.view(np.int16)).to(DEV).view(torch.bfloat16)
-        for rows in (16, 8, 3):
+        for rows in (16, 8, 2):
             for r0 in range(0, xd.shape[0], rows):
                 y = ops.gemv_w8a8_decode(xd[r0:r0 + rows].contiguous(), wq, sw, None, out_dtype=torch.float32)
                 assert np.array_equal(to_np(y), want[r0:r0 + rows]), f"mantissa {m}, rows {r0}.. ({rows} a call)"
