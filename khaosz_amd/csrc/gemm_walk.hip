@@ -6,9 +6,9 @@
 // them: 22 k cycles a tile for 13 k of K loop.  Here the last two steps of a tile already request the next tile's first
 // two stages, so its first fragments are in registers when the epilogue ends, and the epilogue's stores drain under the
 // next tile's first step.  (gemm_kernel also requests three stages past the last one for the sake of an even count, a
-// quarter of all fills at K = 1536.)  Row scales wait in LDS and the output's end is the descriptors' (one epilogue, no row checks):
-// 156 to 212 registers instead of 229, and one round of tiles is faster too, 4096 x 2048 x 2048 19.1 us in gemm_kernel, 18.2 here,
-// 1234 x 4576 x 2528 22.7 -> 21.2.
+// quarter of all fills at K = 1536.)  Row scales wait in LDS and the output's end is the descriptors' (one epilogue, no row checks): an
+// int8 tile takes 160 registers, with a residual 206, where gemm_kernel takes 227 (FP8 194 and 231, where it takes 164; 256 x 192
+// tiles 192 to 256).  One round of tiles is faster too, 4096 x 2048 x 2048 19.1 us in gemm_kernel, 18.2 here, 1234 x 4576 x 2528 22.7 -> 21.2.
 //
 // 256 x 192: 4096 x 3072 is 16 x 24 tiles of 256 x 128, one and a half rounds in the time of two, and 16 x 16 of these.  Three stages of 56 KiB do not fit LDS: two, and a stage is requested whole as soon as its place is free.  (Half
 // steps through five 28 KiB stages, four times the barriers: 10 to 15 % slower.  256 x 256 on the same two buffers: level with

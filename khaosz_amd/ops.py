@@ -545,9 +545,11 @@ class AttnPartials(NamedTuple):
 
 GEMV_ATTN_MAX_ROWS, GEMV_ATTN_MAX_K, GEMV_ATTN_MAX_SLICES = 8, 2048, 4
 GEMV_ATTN_SLICE = 256  # positions of a slice
-# Every workgroup of the projection repeats the merge of all rows, so it pays only while that is little work
-# (rows x row length x slices): 4 x 1536 x 3 saves 0.3 us per step over the separate merge launch, 1 x 1536 x 3 1.2,
-# 8 x 2048 x 3 loses 1.2 us.
+# Every workgroup of the projection repeats the merge of all rows, so it pays only while that is little work (rows x row
+# length x slices).  A decode step with the merge in o_proj | in a launch of its own, us: 24 layers 1536 wide, 4 rows x 3
+# slices (18432) 644.6 | 652.1, 5 x 3 (23040) 737.1 | 735.2, 5 x 4 (30720) 759.7 | 747.1; 8 blocks 2048 wide, 3 x 3 237.2 | 243.6,
+# 4 x 3 (24576) 241.8 | 242.7, 8 x 2 (32768) 276.0 | 273.2.  Attention and o_proj alone, separate minus merged: 1 x 1536 x 3 1.3,
+# 4 x 1536 x 3 0.3, 8 x 2048 x 3 -1.4.  (Level around 22000; the limit is what callers ask attn_gemv_fusable about.)
 GEMV_ATTN_MAX_WORK = 32768
 
 
