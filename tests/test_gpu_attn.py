@@ -536,12 +536,20 @@ def test_prefill_attn_reading_ahead_changes_nothing():
 
 
 @pytest.mark.parametrize("norm", [False, True])
-@pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("B,S,start,Hq,Hkv,page,shared", [(1, 1, 0, 1, 1, 64, True), (3, 21, 0, 4, 2, 8, False), (2, 130, 0, 6, 2, 64, True),
-                                                          (1, 33, 31, 4, 4, 32, True), (2, 300, 100, 24, 4, 128, False), (4, 512, 0, 16, 4, 64, True)])
-def test_prefill_attn_that_rotates_its_queries_gives_the_bits_of_two_launches(B, S, start, Hq, Hkv, page, shared, D, norm):
+@pytest.mark.parametrize("B,S,start,Hq,Hkv,page,shared,D,queries", [
+    (1, 1, 0, 1, 1, 64, True, 64, 32), (3, 21, 0, 4, 2, 8, False, 64, 32), (2, 130, 0, 6, 2, 64, True, 64, 32), (1, 33, 31, 4, 4, 32, True, 64, 32),
+    (2, 300, 100, 24, 4, 128, False, 64, 64), (4, 512, 0, 16, 4, 64, True, 64, 64),
+    (5, 500, 0, 24, 4, 64, False, 64, 128), (5, 487, 77, 24, 4, 48, True, 64, 128), (9, 97, 0, 30, 6, 64, True, 64, 128),
+    (1, 1, 0, 1, 1, 64, True, 128, 128), (3, 21, 0, 4, 2, 8, False, 128, 128), (2, 130, 0, 6, 2, 64, True, 128, 64), (1, 33, 31, 4, 4, 32, True, 128, 128),
+    (2, 300, 100, 24, 4, 128, False, 128, 64), (4, 512, 0, 16, 4, 64, True, 128, 128), (3, 475, 77, 16, 4, 48, True, 128, 128)])
+def test_prefill_attn_that_rotates_its_queries_gives_the_bits_of_two_launches(B, S, start, Hq, Hkv, page, shared, D, queries, norm):
     """aq_rope_kv_cache_write + the attention that reads queries from the projection's rows, against rope_kv_write + the
-    attention on rotated queries: caches and outputs, on every number of wavefronts per query row."""
+    attention on rotated queries: caches and outputs.  queries: of a workgroup, by which the three forms (four, two and one
+    wavefront side by side on a query row) are told apart."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    q32, q64 = (-(-S // n) * Hq * B for n in (32, 64))
+    two = start + S > 128 and q64 <= (1 if D == 128 else 2 if start + S < 1024 else 4) * cus
+    assert queries == (32 if D == 64 and q32 <= cus else 64 if two else 128)
     from khaosz_amd import _abi
 
     _say("prefill_attn rotates q", B, S, start, Hq, Hkv, page, shared, D, norm)
