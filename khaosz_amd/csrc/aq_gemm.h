@@ -95,7 +95,7 @@ __device__ __forceinline__ typename Acc<FP8>::type mma(const typename Frag<FP8>:
 }
 
 // gemm_slices.hip: tiles of 32 tm x 32, K cut among a workgroup's wavefronts
-int gemm_slices_rows(int64_t M, int64_t N, int64_t K);
+int gemm_slices_rows(int64_t M, int64_t N, int64_t K, int64_t cus);
 template <bool FP8, int OUT>
 int gemm_slices_launch(GemmArgs& a, int tm, hipStream_t st);
 

@@ -20,9 +20,11 @@ extern "C" {
  * unsynchronised -- which is why it does not exist in the product library. */
 int aq_lab_set_gemm_tile(int rows);
 
-/* The tile the library would pick for an M x N output on a device of `compute_units` compute units, in the
- * numbering above (a pure function of its arguments: no device is touched). */
-int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int compute_units);
+/* The tile with which the library multiplies M x K by N x K codes (y_dtype AQ_F32, AQ_BF16, or -1 for int32 sums; residual: whether
+ * there is one) on a device of `compute_units` compute units, in the numbering above, with 34 and 35 (32 x 32 and 64 x 32, K cut
+ * among the wavefronts) and 512 (256 x 256).  A pure function of its arguments: no device is touched.  (Calls of few rows that
+ * a weight-streaming kernel takes do not get here.) */
+int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8, int y_dtype, int residual, int compute_units);
 
 /* Clock counters the lab build's tiled GEMM leaves behind (wavefront 0 of workgroup 0 of the LAST GEMM launch that
  * completed): host int64[8].  [0] shader-clock cycles and [1] 100 MHz reference ticks between the kernel's first and

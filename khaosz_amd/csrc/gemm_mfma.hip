@@ -863,13 +863,6 @@ static int choose_tile_for(int64_t M, int64_t N, int64_t cus, bool walk = false,
   return best;
 }
 
-static int choose_tile(int64_t M, int64_t N, bool walk, bool res) {
-#ifdef AQ_LAB
-  if (g_forced_tile) return g_forced_tile;
-#endif
-  return choose_tile_for(M, N, device_cus(), walk, res);
-}
-
 template <bool FP8, int OUT, class S>
 static int launch_shape(GemmArgs& a, hipStream_t st) {
   a.tiles_m = (a.M + S::BM - 1) / S::BM;
@@ -892,34 +885,43 @@ static int launch_shape(GemmArgs& a, hipStream_t st) {
 // * two rounds at least, and the last one more than half full: with less 1.04 to 1.14 at any K.
 // In all 6 % faster than the walk where it is taken, and the choice 2 % from the best tile in the mean (taken for any K above 2048
 // and any last round, 11 %).
-static bool huge_fp8_ok(const GemmArgs& a) {
+static bool huge_fp8_ok(const GemmArgs& a, int64_t cus) {
   if (a.K <= 3072 || a.K % (2 * ShapeHuge::BK) != ShapeHuge::BK || (a.N % 2) != 0 || (a.M % ShapeHuge::BM) != 0 || a.res != nullptr) return false;
-  const int64_t tiles = (int64_t)(a.M / ShapeHuge::BM) * ((a.N + ShapeHuge::BN - 1) / ShapeHuge::BN), cus = device_cus();
+  const int64_t tiles = (int64_t)(a.M / ShapeHuge::BM) * ((a.N + ShapeHuge::BN - 1) / ShapeHuge::BN);
   return tiles >= 2 * cus && (tiles % cus == 0 || 2 * (tiles % cus) > cus);
+}
+
+// The tile that takes a call on a device of `cus` compute units.  TILE_WALK and TILE_WIDE: of gemm_walk_kernel, TILE_SLICES32 and
+// TILE_SLICES64: of gemm_slices_kernel.
+static int choose_tile(const GemmArgs& a, bool fp8, int out, int64_t cus) {
+  if (fp8 && out != OUT_I32 && huge_fp8_ok(a, cus)) return TILE_HUGE;
+  const bool walk = out != OUT_I32 && gemm_walk_ok(a, out);
+  const int tile = choose_tile_for(a.M, a.N, cus, walk, a.res != nullptr);
+  if (walk && tile == TILE_LARGE) return TILE_WALK;
+  if (tile == TILE_WIDE || out == OUT_I32) return tile;
+  const int tm = gemm_slices_rows(a.M, a.N, a.K, cus);
+  return tm == 1 ? TILE_SLICES32 : tm == 2 ? TILE_SLICES64 : tile;
 }
 
 template <bool FP8, int OUT>
 static int launch(GemmArgs& a, hipStream_t st) {
+  int tile = choose_tile(a, FP8, OUT, device_cus());
 #ifdef AQ_LAB
-  const bool forced = g_forced_tile != 0;
-#else
-  const bool forced = false;
-#endif
-  if constexpr (FP8 && OUT != OUT_I32) {
-    if (!forced && huge_fp8_ok(a)) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
+  if (g_forced_tile) {
+    tile = g_forced_tile;
+    if ((tile == TILE_WALK || tile == TILE_WIDE) && (OUT == OUT_I32 || !gemm_walk_ok(a, OUT))) tile = TILE_LARGE;
+    if (tile == TILE_HUGE && (a.K % ShapeHuge::BK != 0 || a.N % 2 != 0 || a.M % ShapeHuge::BM != 0 || a.res != nullptr)) tile = TILE_LARGE;
   }
-  const bool walk = OUT != OUT_I32 && gemm_walk_ok(a, OUT);
-  const int tile = choose_tile(a.M, a.N, walk, a.res != nullptr);
-  if constexpr (OUT != OUT_I32) {
-    if (walk && tile == TILE_LARGE && !forced) return gemm_walk_launch<FP8, OUT>(a, st, 128);
-    if (walk && tile == TILE_WIDE) return gemm_walk_launch<FP8, OUT>(a, st, 192);
-#ifdef AQ_LAB
-    if (walk && tile == TILE_WALK) return gemm_walk_launch<FP8, OUT>(a, st, 128);
 #endif
-  }
   if constexpr (OUT != OUT_I32) {
-    const int tm = forced ? (tile == TILE_SLICES32 ? 1 : tile == TILE_SLICES64 ? 2 : 0) : gemm_slices_rows(a.M, a.N, a.K);
-    if (tm) return gemm_slices_launch<FP8, OUT>(a, tm, st);
+    switch (tile) {
+      case TILE_WALK: return gemm_walk_launch<FP8, OUT>(a, st, 128);
+      case TILE_WIDE: return gemm_walk_launch<FP8, OUT>(a, st, 192);
+      case TILE_SLICES32: return gemm_slices_launch<FP8, OUT>(a, 1, st);
+      case TILE_SLICES64: return gemm_slices_launch<FP8, OUT>(a, 2, st);
+    }
+    if constexpr (FP8)
+      if (tile == TILE_HUGE) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
   }
   switch (tile) {
     case TILE_SMALL: return launch_shape<FP8, OUT, ShapeSmall>(a, st);
@@ -929,10 +931,7 @@ static int launch(GemmArgs& a, hipStream_t st) {
     case TILE_M64N32: return launch_shape<FP8, OUT, ShapeM64N32>(a, st);
 #ifdef AQ_LAB
     case TILE_TALL: return launch_shape<FP8, OUT, ShapeTall>(a, st);
-    case TILE_HUGE:
-      if ((a.K % ShapeHuge::BK) == 0 && (a.N % 2) == 0 && (a.M % ShapeHuge::BM) == 0 && a.res == nullptr)
-        return launch_shape<FP8, OUT, ShapeHuge>(a, st);
-      return launch_shape<FP8, OUT, ShapeLarge>(a, st);
+    case TILE_HUGE: return launch_shape<FP8, OUT, ShapeHuge>(a, st);
     case TILE_HUGE8: return launch_shape<FP8, OUT, ShapeHuge8>(a, st);
     case TILE_PAIR: return launch_shape<FP8, OUT, ShapePair>(a, st);
 #endif
@@ -974,9 +973,13 @@ extern "C" int aq_lab_set_gemm_tile(int rows) {
   aq::g_forced_tile = rows;
   return AQ_OK;
 }
-extern "C" int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int compute_units) {
-  if (M <= 0 || N <= 0 || compute_units <= 0) return AQ_E_SHAPE;
-  return aq::choose_tile_for(M, N, compute_units);
+extern "C" int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8, int y_dtype, int residual, int compute_units) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 16 || M > (1 << 30) || N > (1 << 20) || K > (1 << 22) || compute_units <= 0) return AQ_E_SHAPE;
+  if ((fp8 && y_dtype < 0) || (y_dtype >= 0 && y_dtype != AQ_F32 && y_dtype != AQ_BF16) || (y_dtype < 0 && residual)) return AQ_E_DTYPE;
+  static const char some = 0;
+  aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
+  a.res = residual ? &some : nullptr;  // only whether there is one
+  return aq::choose_tile(a, fp8 != 0, y_dtype < 0 ? aq::OUT_I32 : y_dtype == AQ_BF16 ? aq::OUT_BF16 : aq::OUT_F32, compute_units);
 }
 #endif
 
@@ -1021,7 +1024,7 @@ extern "C" int aq_linear_w8a8_residual(const int8_t* xq, const float* sx, const 
 #else
   const bool tile_forced = false;
 #endif
-  if (!tile_forced && !aq::gemm_slices_rows(M, N, K) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
+  if (!tile_forced && !aq::gemm_slices_rows(M, N, K, aq::device_cus()) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
     return aq::gemv_tokens_launch(xq, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, st, false);
   aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);
   a.sx = sx;
@@ -1055,7 +1058,7 @@ extern "C" int aq_linear_fp8_residual(const uint8_t* xq, const float* sx, const 
 #else
   const bool tile_forced = false;
 #endif
-  if (!tile_forced && !aq::gemm_slices_rows(M, N, K) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
+  if (!tile_forced && !aq::gemm_slices_rows(M, N, K, aq::device_cus()) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
     return aq::gemv_tokens_launch(reinterpret_cast<const int8_t*>(xq), sx, reinterpret_cast<const int8_t*>(wq), sw, bias,
                                   bias_dtype, residual, y, y_dtype, M, N, K, st, true);
   aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);

@@ -235,8 +235,8 @@ static int launch_slices(GemmArgs& a, hipStream_t st) {
 //     11.1 -> 11.5 | 15.8 -> 16.3, 40 x 8192 x 5120 9.5 -> 10.1 | 12.8 -> 13.0): those stay with the larger tiles.  Between them
 //     64 x 5120 x 5120 8.9 -> 7.8 | 13.7 -> 13.0, 40 x 6912 x 6912 11.0 -> 10.7 | 14.3 -> 14.6, 200 x 2048 x 6912 10.8 -> 9.4 |
 //     11.9 -> 11.8, 128 x 4096 x 8192 12.4 -> 11.9 | 17.3 -> 16.5.
-int gemm_slices_rows(int64_t M, int64_t N, int64_t K) {
-  const int64_t cus = device_cus(), n32 = (N + 31) / 32, tiles = (M + 63) / 64 * n32;
+int gemm_slices_rows(int64_t M, int64_t N, int64_t K, int64_t cus) {
+  const int64_t n32 = (N + 31) / 32, tiles = (M + 63) / 64 * n32;
   if (M <= 16) return 0;
   if ((M + 31) / 32 * n32 <= cus) return 1;
   const bool streams = M <= 64 && N * K > (32 << 20) && M * tiles > 9600;  // much weight, and many tiles that each read A

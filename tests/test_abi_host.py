@@ -264,13 +264,12 @@ def test_package_exports():
 
 
 def test_gemm_tile_choice_for_the_benchmark_shapes_and_a_few_hundred_rows():
-    """The tile shape is picked on the host from M, N and the number of compute units alone.  Pinned here for
-    256 compute units: the benchmark configurations keep the wide tiles (one round of 256 tiles of 256 x 128
-    for the prefill configuration, 256 tiles of 128 x 128 for the FP8 one), a few hundred rows get the small
-    tiles that still give every compute unit at most one tile, and a launch of many rounds never takes a small
-    tile."""
+    """The tile of a launch by tiles alone (int32 sums: no kernel that walks tiles or cuts K) is picked on the host from M, N and the
+    number of compute units.  Pinned here for 256 compute units: the benchmark configurations keep the wide tiles (one round of
+    256 tiles of 256 x 128 for the prefill configuration, 256 tiles of 128 x 128 for the FP8 one), a few hundred rows get the small
+    tiles that still give every compute unit at most one tile, and a launch of many rounds never takes a small tile."""
     lab = _abi.load_lab()
-    pick = lambda M, N: lab.aq_lab_choose_gemm_tile(M, N, 256)
+    pick = lambda M, N: lab.aq_lab_choose_gemm_tile(M, N, 2048, 0, -1, 0, 256)
     assert pick(4096, 2048) == 256          # configuration 3: 256 tiles of 256 x 128, one round
     assert pick(2048, 2048) == 128          # configuration 4: 256 tiles of 128 x 128
     assert pick(8192, 8192) == 256
@@ -285,7 +284,35 @@ def test_gemm_tile_choice_for_the_benchmark_shapes_and_a_few_hundred_rows():
     assert pick(512, 2048) == 65 and pick(1024, 2048) == 64 and pick(256, 2048) == 33
     for M, N in ((8192, 8192), (100000, 4096), (1 << 20, 1 << 20)):
         assert pick(M, N) in (128, 256)
-    assert lab.aq_lab_choose_gemm_tile(0, 8, 256) == -2 and lab.aq_lab_choose_gemm_tile(8, 8, 0) == -2
+    for bad in ((0, 8, 64, 0, -1, 0, 256), (8, 8, 64, 0, -1, 0, 0), (8, 8, 24, 0, 1, 0, 256)):
+        assert lab.aq_lab_choose_gemm_tile(*bad) == -2
+    for bad in ((8, 8, 64, 1, -1, 0, 256), (8, 8, 64, 0, -1, 1, 256), (8, 8, 64, 0, 2, 0, 256)):  # FP8 sums, a residual on sums, no type
+        assert lab.aq_lab_choose_gemm_tile(*bad) == -3
+
+
+def test_gemm_tile_choice_where_tiles_are_walked_or_k_is_cut():
+    """What a Linear's launch takes on 256 compute units: walked tiles of 256 x 128 (258) or 256 x 192 (192) with K from 512 and an even
+    N, tiles with K cut among the wavefronts (34, 35) for few rows, 256 x 256 (512) for some FP8 launches, else the tile above."""
+    lab = _abi.load_lab()
+    f32, bf16 = _abi.AQ_F32, _abi.AQ_BF16
+    pick = lambda M, N, K, fp8=0, out=bf16, res=0: lab.aq_lab_choose_gemm_tile(M, N, K, fp8, out, res, 256)
+    # block of 2048, 8 x 512 tokens: q/k/v, o, down; up/gate, whose last round is halved (5.55 rounds of 15 against 3.84 of 21.75; whole
+    # it would be 5.75); the 24-layer model's up/gate on 4 x 512, halved too
+    assert pick(4096, 3072, 2048) == 192 and pick(4096, 2048, 2048, res=1) == 258 and pick(4096, 2048, 5632, res=1) == 258
+    assert pick(4096, 11264, 2048) == 258 and pick(2048, 13824, 1536) == 258
+    # the residual's cost
+    assert pick(3668, 4864, 512, fp8=1) == 192 and pick(3668, 4864, 512, fp8=1, res=1) == 258
+    # what is not walked: short K, an odd N, a residual under fp32 outputs
+    assert pick(4096, 3072, 496) == 256 and pick(4096, 3071, 2048) == 256
+    assert pick(4096, 3072, 2048, out=f32) == 192 and pick(4096, 3072, 2048, out=f32, res=1) == 256
+    # FP8: an odd number of 64-byte steps above 3072, a last round more than half full, whole rows of tiles, no residual
+    assert pick(4864, 8640, 3264, fp8=1) == 512 and pick(4864, 8640, 3264) != 512
+    for M, N, K, res in ((4864, 8640, 3328, 0), (4864, 8640, 3008, 0), (4863, 8640, 3264, 0), (4864, 8640, 3264, 1), (4096, 9216, 3264, 0),
+                         (8192, 8192, 8192, 0)):
+        assert pick(M, N, K, fp8=1, res=res) in (192, 258)
+    # K cut among the wavefronts; a tile too many for that
+    assert pick(64, 2048, 2048, out=f32) == 34 and pick(200, 2048, 6912) == 35 and pick(200, 2048, 1520) == 33
+    assert pick(333, 1536, 6912, res=1) == 65
 
 
 def test_quant_tensor_fp8_refuses_a_workspace_smaller_than_its_slots():

@@ -421,12 +421,14 @@ PRODUCT_TILES = {256: "256 x 128", 128: "128 x 128", 64: "128 x 64", 32: "128 x 
 
 def _smallest_shape_for_tile(kind, cus):
     """The (M, N) of fewest outputs for which the library's own rule (a pure function, asked of the lab library;
-    no GEMM runs there) picks tile `kind` on a device of `cus` compute units."""
+    no GEMM runs there) picks tile `kind` on a device of `cus` compute units for every product of the test below."""
     lab = _abi.load_lab()
     best = None
     for M in range(33, 2100, 7):
         for N in list(range(32, 2100, 32)) + [3072, 4096, 8192]:
-            if lab.aq_lab_choose_gemm_tile(M, N, cus) == kind and (best is None or M * N < best[0] * best[1]):
+            if (best is None or M * N < best[0] * best[1]) and all(
+                    lab.aq_lab_choose_gemm_tile(M, N, K, fp8, out, 0, cus) == kind
+                    for K in (144, 256) for fp8, out in ((0, -1), (0, _abi.AQ_BF16), (0, _abi.AQ_F32), (1, _abi.AQ_F32))):
                 best = (M, N)
     return best
 
@@ -1301,15 +1303,21 @@ def test_full_size_fp8_linearity_in_scales(oracle):
     assert ((y[rows] - ref).norm() / ref.norm()).item() < 0.06
 
 
-# more 256 x 128 tiles than compute units: whole rounds, a last round of whole and of halved tiles, ragged M (a half tile
-# that is all padding) and N, the shortest K that walks, K steps that fill the three buffers unevenly
-@pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("M,N,K", [(4096, 2176, 512), (2049, 4100, 640), (8192, 3200, 512), (4225, 6402, 768), (4000, 6400, 1024)])
-def test_gemm_walking_tiles(M, N, K, bias):
-    """The walk against the kernel of one tile shape after another (its own tests hold that against the oracle): same bits."""
+def _assert_walked(M, N, K, tile, residual=False):
+    """int8 and FP8 Linears of these sizes take walked tiles: 258 (256 x 128) or 192 (256 x 192)."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    if -(-M // 256) * -(-N // 128) <= cus:
-        pytest.skip("one round on this device")
+    lab = _abi.load_lab()
+    assert [lab.aq_lab_choose_gemm_tile(M, N, K, fp8, _abi.AQ_BF16, int(residual), cus) for fp8 in (0, 1)] == [tile, tile]
+
+
+# more tiles than compute units: whole rounds, a last round of whole and of halved tiles, ragged M (a half tile that is all
+# padding) and N, the shortest K that walks, K steps that fill the buffers unevenly; of 256 x 128 (258) and 256 x 192
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K,tile", [(4096, 2176, 512, 192), (2049, 4100, 640, 192), (8192, 3200, 512, 258), (4225, 6402, 768, 258),
+                                        (4000, 6400, 1024, 258)])
+def test_gemm_walking_tiles(M, N, K, bias, tile):
+    """The walk against the kernel of one tile shape after another (its own tests hold that against the oracle): same bits."""
+    _assert_walked(M, N, K, tile)
     _say("gemm walk", M, N, K, bias)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     xq, wq = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
@@ -1326,9 +1334,10 @@ def test_gemm_walking_tiles(M, N, K, bias):
 
 # one round (whole, ragged), several with whole and with halved tiles at their end; the residual apart from and in the output
 @pytest.mark.parametrize("residual", [False, True])
-@pytest.mark.parametrize("M,N,K", [(4096, 2048, 512), (3001, 2046, 640), (2049, 4100, 768), (4225, 6402, 512)])
-def test_gemm_walk_of_one_round_and_residuals(M, N, K, residual):
-    """256 x 128 tiles with and without a residual: the bits of the kernel of one tile after another."""
+@pytest.mark.parametrize("M,N,K,tile", [(4096, 2048, 512, 258), (3001, 2046, 640, 258), (2049, 4100, 768, 192), (4225, 6402, 512, 258)])
+def test_gemm_walk_of_one_round_and_residuals(M, N, K, residual, tile):
+    """Walked tiles with and without a residual: the bits of the kernel of one tile after another."""
+    _assert_walked(M, N, K, tile, residual)
     _say("gemm walk residual", M, N, K, residual)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     xq, wq = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
