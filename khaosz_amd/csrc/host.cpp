@@ -880,7 +880,8 @@ void Block::lay_out() {
   most = m.most;
 }
 
-// Queues the block's launches: the ones, in the order and with the operands, of the step-by-step path in block.py.
+// Queues the block's launches: the ones, in the order and with the operands, of the step-by-step path in block.py, but that a prompt's
+// queries may be rotated in its attention instead of before it (rotates(); the same bits).
 int Block::queue(const void* in, void* out, char* base, const char** what) const {
   const bool few = this->few();
   const int64_t W = qkv.N, A = Hq * D, KV = Hkv * D;
