@@ -882,6 +882,7 @@ static int launch_shape(GemmArgs& a, hipStream_t st) {
 //   to 8192 1.06, up to 16384 1.02 (us 5376 x 7278 x 2816 121 | 93, 4096 x 10688 x 3584 140 | 127, 8192^3 432 | 429, 4096 x 8192 x 4096 112 | 110).
 // * K above 3072: its loop stops between tiles, gemm_walk_kernel's does not: K 1024..2048 1.10, up to 2560 1.00, up to 3072 0.99,
 //   up to 4096 0.96, up to 5120 0.94, up to 8192 0.90 (us 4864 x 8640 x 3264 126 | 131, 7424 x 6440 x 5312 212 | 244, 7424 x 5760 x 8000 294 | 327).
+//   K below 512, which is not walked: 1.25 of gemm_kernel's other tiles with bf16 outputs, 1.04 with fp32 ones (120 sizes).
 // * two rounds at least, and the last one more than half full: with less 1.04 to 1.14 at any K.
 // In all 6 % faster than the walk where it is taken, and the choice 2 % from the best tile in the mean (taken for any K above 2048
 // and any last round, 11 %).
