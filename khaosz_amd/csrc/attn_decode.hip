@@ -110,7 +110,7 @@ struct AttnArgs {
   float eps;
   int page_shift;  // log2 of a page of 64, 128, 256 .. positions, otherwise 62
   const int64_t* lens_at;  // lens, or without them anything of B numbers (the table): read without asking, beside the table
-  UDiv by_hkv, by_ns;
+  UDiv by_hkv, by_ns, by_page;  // by_page: pages of other sizes, of launches whose positions it takes (mul 0: a division)
 };
 
 constexpr int ATT_WAVES = 4;
@@ -190,6 +190,18 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
   int64_t len = p.lens_at[b];
   asm volatile("" ::"s"(p.T), "s"(p.page), "s"(p.n_pages), "s"(p.lens), "s"(p.kc), "s"(p.vc));  // arguments: one request for all
   __builtin_amdgcn_sched_barrier(0);
+  // Pages that a wavefront's positions straddle: lane L looks up the page of position t0 + L, also before the queries are requested.
+  // (Behind them, the wait for the length and a division: 10 x 786 positions, 16/4 heads of 128, pages of 16 9.66 us, 9.37 so;
+  // 11 x 117, 24/4 heads of 64 6.48, 6.34.)
+  int64_t phys = -1;
+  int64_t in_page = 0;
+  if (!whole && t0 + lane < T) {
+    const int64_t t = t0 + lane;
+    const int64_t lp = p.by_page.mul ? (int64_t)p.by_page((uint32_t)t) : t / p.page;
+    in_page = t - lp * p.page;
+    if (lp < p.P) phys = p.table[(int64_t)b * p.P + lp];
+  }
+  __builtin_amdgcn_sched_barrier(0);
 
   constexpr int KS = D / 32;                  // matrix-core steps over the head dimension
   const int col = lane & 15, kq = lane >> 4;  // operand row / column, group of 8 dimensions inside a step
@@ -237,17 +249,14 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
   }
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("" : "+s"(entry), "+s"(len));  // not requested later than above
-  // (element offsets, -1: unmapped or past T; pages that wavefronts straddle: lane L looks up the row of position t0 + L)
+  // (element offsets, -1: unmapped or past T; row: of lane L, of position t0 + L)
   const int rstep = p.Hkv * D;  // elements between consecutive positions of a page
   int64_t first = -1, row = -1;
   if (whole) {
     if (t0 < T && lp0 < p.P && entry >= 0 && entry < p.n_pages)
       first = (((entry << p.page_shift) + (t0 - (lp0 << p.page_shift))) * p.Hkv + kvh) * D;
-  } else if (t0 + lane < T) {
-    const int64_t t = t0 + lane;
-    const int64_t lp = t / p.page;
-    const int64_t phys = lp < p.P ? p.table[(int64_t)b * p.P + lp] : -1;
-    if (phys >= 0 && phys < p.n_pages) row = ((phys * p.page + t % p.page) * p.Hkv + kvh) * D;
+  } else if (phys >= 0 && phys < p.n_pages) {
+    row = ((phys * p.page + in_page) * p.Hkv + kvh) * D;
   }
   // A sequence shorter than T (a decode batch of sequences at different positions): positions from its own
   // length on are masked, as the additive mask of the reference's forward does.  The mask value is finite, so
@@ -759,6 +768,7 @@ static int attn_decode(const void* q, const void* qkv, const float* freqs, int64
   a.lens_at = seq_lens ? seq_lens : page_table;
   a.by_hkv = aq::UDiv::of((uint32_t)Hkv);
   a.by_ns = aq::UDiv::of((uint32_t)ns);
+  if (total_len <= ((int64_t)1 << 31) && page_size <= ((int64_t)1 << 31)) a.by_page = aq::UDiv::of((uint32_t)page_size);
   a.page_shift = 62;
   for (int sh = 6; sh < 62; ++sh)
     if (page_size == ((int64_t)1 << sh)) a.page_shift = sh;

@@ -619,6 +619,28 @@ def test_paged_attn_decode_page_sizes_give_the_same_bits(Hq, Hkv, D, T):
         assert all(torch.equal(a, b) for a, b in zip(got[0], other))
 
 
+@pytest.mark.parametrize("page", [192, (1 << 31) - 1, (1 << 31) + 1, (1 << 33) + 3])
+def test_paged_attn_decode_of_large_pages(page):
+    """One page, of which a few positions are in use: its size fits the multiplication that finds a position's page, or does not."""
+    from khaosz_amd import _abi
+
+    B, Hq, Hkv, D, T = 1, 4, 2, 64, 130
+    g = torch.Generator().manual_seed(7)
+    qkv = torch.randn(B, (Hq + 2 * Hkv) * D, generator=g).to(torch.bfloat16).to(DEV)
+    ang = torch.rand(B, D // 2, generator=g) * 6.28
+    freqs = torch.polar(torch.ones_like(ang), ang).to(DEV)
+    fr = torch.view_as_real(freqs).contiguous()
+    kc, vc = (torch.randn(1, 256, Hkv, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    table = torch.zeros(B, 1, dtype=torch.int64, device=DEV)
+    k2, v2 = kc.clone(), vc.clone()
+    want = ops.rope_paged_attn_decode(qkv, freqs, table, T, kc, vc, Hq, Hkv)
+    out = torch.empty_like(want)
+    assert _abi.load().aq_rope_paged_attn_decode(qkv.data_ptr(), fr.data_ptr(), D, table.data_ptr(), 1, T, None, page, k2.data_ptr(),
+                                                 v2.data_ptr(), 1, D ** -0.5, out.data_ptr(), B, Hq, Hkv, D, None, 0,
+                                                 torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out, want) and torch.equal(k2, kc) and torch.equal(v2, vc)
+
+
 @pytest.mark.parametrize("Hq,Hkv,D", [(2, 1, 64), (3, 1, 128), (4, 1, 64), (6, 1, 64), (6, 1, 128), (8, 1, 128)])
 def test_paged_attn_decode_infinite_values_stay_in_their_dimension(Hq, Hkv, D):
     """An infinite value at a position that every head weighs makes that dimension of every head infinite and changes no other bit."""
