@@ -156,7 +156,8 @@ typedef float attn_f32x4 __attribute__((ext_vector_type(4)));
 // QKN (with ROPE): the rotated queries and the rotated new key are RMS-normalised over the head dimension (see
 // chunk_sumsq) before they are used and stored: what rope_kv_write_kernel does with gains, same bits.  A head
 // vector's chunk c = 4 ks + kq sits in register ks of the lane with that kq.
-template <int G, int D, bool ROPE, bool QKN = false>
+// WHOLE: pages of 64, 128, 256 .. positions: a wavefront's rows lie in one page.
+template <int G, int D, bool WHOLE, bool ROPE, bool QKN = false>
 __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnArgs p) {
   static_assert(!QKN || ROPE, "qk-norm belongs to the kernels that rotate");
   constexpr int CPR = D / 8;     // 16-byte chunks per row: 16 or 8
@@ -180,24 +181,19 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
   const int b = p.by_ns(bs), split = bs - b * p.NS;
   const int64_t T = p.T;
   const int64_t t0 = (int64_t)split * KPG + wave * KPW;  // first position of this wavefront
-  // Where the rows are.  Pages of 64, 128, 256 .. positions: all of this wavefront's rows lie in one page, one lookup, and every
-  // load's address is that plus the lane's own offset.  The table's entry (otherwise its first, not used) and the sequence's
-  // length are requested before anything else and first used behind the queries' requests (8 x 544 positions, 16/4 heads of 128:
-  // 9.46 us; 9.60 with divisions by the numbers of heads and slices, a wait for the length and the lookup behind them).
-  const bool whole = p.page_shift < 62;  // uniform
-  const int64_t lp0 = t0 >> p.page_shift;
-  int64_t entry = p.table[(int64_t)b * p.P + (lp0 < p.P ? lp0 : p.P - 1)];
-  int64_t len = p.lens_at[b];
-  asm volatile("" ::"s"(p.T), "s"(p.page), "s"(p.n_pages), "s"(p.lens), "s"(p.kc), "s"(p.vc));  // arguments: one request for all
-  __builtin_amdgcn_sched_barrier(0);
-  // Pages that a wavefront's positions straddle: lane L looks up the page of position t0 + L, also before the queries are requested.
-  // (Behind them, the wait for the length and a division: 10 x 786 positions, 16/4 heads of 128, pages of 16 9.66 us, 9.37 so;
-  // 11 x 117, 24/4 heads of 64 6.48, 6.34.)
-  int64_t phys = -1;
-  int64_t in_page = 0;
-  if (!whole && t0 + lane < T) {
-    const int64_t t = t0 + lane;
-    const int64_t lp = p.by_page.mul ? (int64_t)p.by_page((uint32_t)t) : t / p.page;
+  // Where the rows are.  WHOLE: one lookup, and every load's address is that plus the lane's own offset.  The table's entry
+  // (otherwise its first, not used) and the sequence's length are requested before anything else and first used behind the
+  // queries' requests (8 x 544 positions, 16/4 heads of 128: 9.46 us; 9.60 with divisions by the numbers of heads and slices, a
+  // wait for the length and the lookup behind them).  Other pages: lane L looks up the page of position t0 + L, as early.  Kernels
+  // of their own: with both ways in one, their loads became one stretch behind the addresses of all of them (pages of 64 and more,
+  // 16/4 heads of 128 and 24/4 of 64: 4 % longer; pages of 16: 10 x 786 positions of 16/4 9.37 us, 8.91 so, 14 x 647 of 24/4 8.48, 7.93).
+  const int64_t lp0 = WHOLE ? t0 >> p.page_shift : 0;
+  int64_t entry = 0, phys = -1, in_page = 0, len = p.lens_at[b];
+  if constexpr (WHOLE) {
+    entry = p.table[(int64_t)b * p.P + (lp0 < p.P ? lp0 : p.P - 1)];
+    asm volatile("" ::"s"(p.T), "s"(p.page), "s"(p.n_pages), "s"(p.lens), "s"(p.kc), "s"(p.vc));  // arguments: one request for all
+  } else if (t0 + lane < T) {
+    const int64_t t = t0 + lane, lp = p.by_page.mul ? (int64_t)p.by_page((uint32_t)t) : t / p.page;
     in_page = t - lp * p.page;
     if (lp < p.P) phys = p.table[(int64_t)b * p.P + lp];
   }
@@ -248,11 +244,11 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" : "+s"(entry), "+s"(len));  // not requested later than above
+  if constexpr (WHOLE) asm volatile("" : "+s"(entry), "+s"(len));  // not requested later than above
   // (element offsets, -1: unmapped or past T; row: of lane L, of position t0 + L)
   const int rstep = p.Hkv * D;  // elements between consecutive positions of a page
   int64_t first = -1, row = -1;
-  if (whole) {
+  if constexpr (WHOLE) {
     if (t0 < T && lp0 < p.P && entry >= 0 && entry < p.n_pages)
       first = (((entry << p.page_shift) + (t0 - (lp0 << p.page_shift))) * p.Hkv + kvh) * D;
   } else if (phys >= 0 && phys < p.n_pages) {
@@ -280,7 +276,7 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
     // waited for each load before issuing the next).
     uint4 kb[4][KS], vv[NL];
     uint64_t there;  // bit per position: its row is there
-    if (whole) {
+    if constexpr (WHOLE) {
       // (20 lookups by shuffle, with 64-bit arithmetic each, took 0.3 us of the launch at head dimension 64, and 0.1 to 0.2 at 128, where
       // 32 loads of 1 KiB wait for each other to be taken)
       const uint16_t *ks0 = p.kc + (first >= 0 ? first : 0) + (uint32_t)(col * rstep + kq * 8);
@@ -323,7 +319,7 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
       // of what was just read from that slot
       const uint16_t* tok = p.qkv + (int64_t)b * (p.Hq + 2 * p.Hkv) * D;
       // the same in every lane; -1: its page is unmapped
-      const int64_t rn = !whole ? row_of((int)(T - 1 - t0)) : first < 0 ? -1 : first + (T - 1 - t0) * rstep;
+      const int64_t rn = !WHOLE ? row_of((int)(T - 1 - t0)) : first < 0 ? -1 : first + (T - 1 - t0) * rstep;
       if (rn >= 0) {
         const int tn = (int)(T - 1 - t0) >> 4, cn = (int)(T - 1 - t0) & 15;  // tile and column of the new key
         uint4 kn[KS];
@@ -696,14 +692,14 @@ extern "C" int64_t aq_paged_attn_decode_workspace_bytes(int64_t B, int64_t Hq, i
   return ns == 1 ? 0 : aq::attn_workspace_bytes(B, Hq, ns);
 }
 
-template <int G, int D>
+template <int G, int D, bool WHOLE>
 static void attn_launch(bool rope, dim3 grid, dim3 block, hipStream_t st, const aq::AttnArgs& a) {
   if (rope && a.q_gain)
-    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, true, true>), grid, block, 0, st, a);
+    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, WHOLE, true, true>), grid, block, 0, st, a);
   else if (rope)
-    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, true>), grid, block, 0, st, a);
+    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, WHOLE, true>), grid, block, 0, st, a);
   else
-    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, false>), grid, block, 0, st, a);
+    aq::queue_kernel((aq::paged_attn_decode_kernel<G, D, WHOLE, false>), grid, block, 0, st, a);
 }
 
 // q == nullptr: the fused form, queries and the new token come from qkv / freqs.
@@ -774,10 +770,11 @@ static int attn_decode(const void* q, const void* qkv, const float* freqs, int64
     if (page_size == ((int64_t)1 << sh)) a.page_shift = sh;
   const dim3 grid((unsigned)(B * Hkv * ns)), block(aq::ATT_WAVES * 64);
   hipStream_t st = static_cast<hipStream_t>(stream);
-#define AQ_ATTN_CASE(G_)                                            \
-  case G_:                                                          \
-    if (D == 128) attn_launch<G_, 128>(rope, grid, block, st, a);   \
-    else attn_launch<G_, 64>(rope, grid, block, st, a);             \
+  const bool whole = a.page_shift < 62;
+#define AQ_ATTN_CASE(G_)                                                                                                          \
+  case G_:                                                                                                                        \
+    if (D == 128) (whole ? attn_launch<G_, 128, true> : attn_launch<G_, 128, false>)(rope, grid, block, st, a);                   \
+    else (whole ? attn_launch<G_, 64, true> : attn_launch<G_, 64, false>)(rope, grid, block, st, a);                              \
     break;
   switch (G) {
     AQ_ATTN_CASE(1)
