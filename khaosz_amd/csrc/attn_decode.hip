@@ -119,6 +119,22 @@ constexpr int ATT_KPG = ATT_WAVES * ATT_KPW; // positions per workgroup
 constexpr int ATT_MAX_D = 128;
 constexpr float ATT_MASKED = -1.0e30f;  // score (exp2 domain) of a cached position the sequence may not attend to
 
+// maximum / sum over each row of 16 consecutive lanes, result in all of them
+__device__ __forceinline__ float row16_max(float v) {
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false)));   // quad_perm [1,0,3,2]
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false)));   // quad_perm [2,3,0,1]
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false)));  // row_half_mirror
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false)));  // row_mirror
+  return v;
+}
+__device__ __forceinline__ float row16_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false));
+  return v;
+}
+
 typedef __bf16 attn_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float attn_f32x4 __attribute__((ext_vector_type(4)));
 
@@ -136,7 +152,8 @@ typedef float attn_f32x4 __attribute__((ext_vector_type(4)));
 //            one head for 4 keys per tile;
 //   softmax  maximum and denominator over a lane's 16 keys in registers and over
 //            the 4 lanes of a head by row swaps (with heads in registers and keys
-//            in lanes every head took four DPP steps, twice); probabilities to LDS;
+//            in lanes, as one or two heads are, every head takes four DPP steps,
+//            twice); probabilities to LDS;
 //   values   V rows are loaded CPR = D / 8 lanes to a row (a load covers 4 or 8
 //            whole rows); a lane accumulates p * V over the keys it loaded (8
 //            dimensions x G heads), the key groups are summed by swaps.
@@ -168,6 +185,7 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
   constexpr int PART = D + 4;    // numerator[D], maximum, denominator, 2 floats of padding
   static_assert(D == 64 || D == 128, "head dimension");
   constexpr int NM = (G + 1) / 4, GV = G > 4 * NM ? G - 4 * NM : 0;  // groups of 4 heads on the matrix core; heads past them (1, 2)
+  constexpr bool FEW = G <= 2;
   constexpr int GP = 4 * NM + GV, PS = KPW + 16;                    // (rows of 80: 4 heads x 16 keys in 64 banks, both ways)
   __shared__ __align__(16) float p_s[ATT_WAVES][GP][PS];
   __shared__ float m_s[ATT_WAVES][G], l_s[ATT_WAVES][G];
@@ -357,60 +375,88 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void paged_attn_decode_kernel(AttnA
     for (int ks = 0; ks < KS; ++ks) {
       if (col >= G) qa[ks] = make_uint4(0, 0, 0, 0);
     }
-    // ---- scores: S[key][head] per tile; this lane gets head col, keys 4 kq .. + 4 of the tile
+    // ---- scores and softmax over the wavefront's 64 positions.  One or two heads: S[head][key] per tile, this lane gets key col,
+    // heads 4 kq .. + 4 (kq = 0 holds the heads there are): 4 exponentials per head, where a lane with a head of its own takes 16
+    // (11 x 479 positions, 8/8 heads of 64: 7.26 us, 6.90 so; 1 x 356, 4/2 of 128: 7.85, 7.58; with three heads level).
     attn_f32x4 sc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       attn_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(attn_bf16x8, kb[t][ks]),
-                                                   __builtin_bit_cast(attn_bf16x8, qa[ks]), c, 0, 0, 0);
+      for (int ks = 0; ks < KS; ++ks) {
+        const attn_bf16x8 k8 = __builtin_bit_cast(attn_bf16x8, kb[t][ks]), q8 = __builtin_bit_cast(attn_bf16x8, qa[ks]);
+        c = FEW ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(q8, k8, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, q8, c, 0, 0, 0);
+      }
       sc[t] = c;
     }
-    // ---- softmax over the wavefront's 64 positions of head col: 16 in this lane, the others 16 and 32 lanes away
     const int n_all = T - t0 < KPW ? (int)(T - t0) : KPW, n_vis = vis - t0 < n_all ? (vis > t0 ? (int)(vis - t0) : 0) : n_all;
-    float pv[4][4], mx = -INFINITY;
+    if constexpr (FEW) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+      for (int r = 0; r < G; ++r) {
+        float pv[4], mx = -INFINITY, sum = 0.0f;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) pv[t][r] = sc[t][r] * p.scale_log2e;
-    if (n_vis < KPW) {  // wavefront-uniform
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = t * 16 + 4 * kq + r;
-          pv[t][r] = key < n_vis ? pv[t][r] : key < n_all ? ATT_MASKED : -INFINITY;
+        for (int t = 0; t < 4; ++t) {
+          const int key = t * 16 + col;
+          pv[t] = key < n_vis ? sc[t][r] * p.scale_log2e : key < n_all ? ATT_MASKED : -INFINITY;
+          mx = fmaxf(mx, pv[t]);
         }
-    }
+        mx = row16_max(mx);  // finite: position t0 is valid
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, pv[t][r]);
-    const LanePair m16 = lanes16_pair(mx);
-    const LanePair m32 = lanes32_pair(fmaxf(m16.x, m16.y));
-    mx = fmaxf(m32.x, m32.y);  // finite: position t0 is valid
-    float part[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      part[r] = 0.0f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        pv[t][r] = __builtin_amdgcn_exp2f(pv[t][r] - mx);  // 0 for positions past T
-        part[r] += pv[t][r];
+        for (int t = 0; t < 4; ++t) {
+          pv[t] = __builtin_amdgcn_exp2f(pv[t] - mx);  // 0 for positions past T
+          sum += pv[t];
+          if (kq == 0) p_s[wave][r][t * 16 + col] = pv[t];
+        }
+        sum = row16_sum(sum);
+        if (lane == 0) {
+          m_s[wave][r] = mx;
+          l_s[wave][r] = sum;
+        }
       }
-    }
-    const LanePair s16 = lanes16_pair((part[0] + part[1]) + (part[2] + part[3]));
-    const LanePair s32 = lanes32_pair(s16.x + s16.y);
-    const float sum = s32.x + s32.y;
-    if (col < GP) {
+    } else {
+      // S[key][head]: this lane gets head col, keys 4 kq .. + 4 of the tile: 16 positions of it, the others 16 and 32 lanes away
+      float pv[4][4], mx = -INFINITY;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        *reinterpret_cast<float4*>(&p_s[wave][col][t * 16 + 4 * kq]) = make_float4(pv[t][0], pv[t][1], pv[t][2], pv[t][3]);
-      if (kq == 0 && col < G) {
-        m_s[wave][col] = mx;
-        l_s[wave][col] = sum;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pv[t][r] = sc[t][r] * p.scale_log2e;
+      if (n_vis < KPW) {  // wavefront-uniform
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int key = t * 16 + 4 * kq + r;
+            pv[t][r] = key < n_vis ? pv[t][r] : key < n_all ? ATT_MASKED : -INFINITY;
+          }
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, pv[t][r]);
+      const LanePair m16 = lanes16_pair(mx);
+      const LanePair m32 = lanes32_pair(fmaxf(m16.x, m16.y));
+      mx = fmaxf(m32.x, m32.y);  // finite: position t0 is valid
+      float part[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        part[r] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          pv[t][r] = __builtin_amdgcn_exp2f(pv[t][r] - mx);  // 0 for positions past T
+          part[r] += pv[t][r];
+        }
+      }
+      const LanePair s16 = lanes16_pair((part[0] + part[1]) + (part[2] + part[3]));
+      const LanePair s32 = lanes32_pair(s16.x + s16.y);
+      const float sum = s32.x + s32.y;
+      if (col < GP) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          *reinterpret_cast<float4*>(&p_s[wave][col][t * 16 + 4 * kq]) = make_float4(pv[t][0], pv[t][1], pv[t][2], pv[t][3]);
+        if (kq == 0 && col < G) {
+          m_s[wave][col] = mx;
+          l_s[wave][col] = sum;
+        }
       }
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);  // this wavefront's LDS writes are done (wavefront-private region)
