@@ -409,12 +409,13 @@ static size_t gemv_rows_lds(int64_t M, int64_t K, int ks, int rows_per_wg) {
 
 // Weight rows per workgroup: the fewest rounds of workgroups over the compute units x what a workgroup takes.  Rows of more
 // than 2048 take 130 to 240 registers: one workgroup to a unit, every round begins with the latency of its rows and rounds them
-// again, 8 M + 4 r + 64 quarters of a weight row (`alone`: rows with the norm or SwiGLU, too).  Shorter rows as they are take 50
-// to 90: two or three workgroups share a unit, a round starts under the one before, 5 M + 4 r + 12.  Fitted to 10 600 random sizes
-// of all kinds (N 512..11264, K 512..8192, 1 to 16 rows, attention rows too): 0.2 % from the best of the four in the mean, 1 in 50
-// more than 4 %, 15 % at most.  us, with 7 M + 4 r for all -> so: fp32 2 x 2592 -> 8352 23.2 -> 11.0, 1 x 6864 -> 4352 18.7 -> 14.1; FP8
-// 1 x 4576 -> 9696 27.0 -> 16.7, 2 x 4816 -> 4560 17.1 -> 11.6, 1 x 512 -> 4848 4.08 -> 3.62; int8 3 x 3328 -> 10720 11.4 -> 9.8; norm 3 x 1408 ->
-// 9408 6.7 -> 6.0; SwiGLU 14 x 2048 -> 2 x 8416 18.5 -> 17.0.  With the larger cost for short rows 3 x 864 -> 10832 4.55 -> 5.08.
+// again, 8 M + 4 r + 64 quarters of a weight row (`alone`: rows with the norm, too).  Shorter rows as they are, of SwiGLU as well, take
+// 50 to 90: two or three workgroups share a unit, a round starts under the one before, 5 M + 4 r + 12.  Fitted to 10 600 random sizes
+// (N 512..11264, K 512..8192, 1 to 16 rows, attention rows too).  us, with 7 M + 4 r for all -> so: fp32 2 x 2592 -> 8352 23.2 -> 11.0,
+// 1 x 6864 -> 4352 18.7 -> 14.1; FP8 1 x 4576 -> 9696 27.0 -> 16.7, 2 x 4816 -> 4560 17.1 -> 11.6, 1 x 512 -> 4848 4.08 -> 3.62; int8 3 x 3328 ->
+// 10720 11.4 -> 9.8; norm 3 x 1408 -> 9408 6.7 -> 6.0; norm and SwiGLU 14 x 2048 -> 2 x 8416 18.5 -> 17.0.  With the larger cost for short
+// rows 3 x 864 -> 10832 4.55 -> 5.08, SwiGLU without the norm 13 x 1536 -> 2 x 8272 9.7 -> 13.2 (959 sizes of it: up to 33 % from the
+// better of its two, so 3 %).
 static int rows_per_workgroup(int64_t M, int64_t N, bool alone, int least, int most) {
   const int64_t cus = device_cus(), fixed = alone ? 8 * M + 64 : 5 * M + 12;
   int best = most;
@@ -497,7 +498,7 @@ int launch_gemv_rows_swiglu(const GemvArgs& a, hipStream_t st) {
 #undef AQ_GX2
 #undef AQ_GX
   static LdsOptIn unused;  // rows of at most 2048: never more than 64 KiB
-  const int r = rows_per_workgroup(a.M, a.N, true, 32, 64);
+  const int r = rows_per_workgroup(a.M, a.N, a.gamma != nullptr, 32, 64);
   return launch_rows(table[r == 64][a.M > 8][a.gamma != nullptr][a.K > 1024], unused, a, r == 64 ? 2 : 4, r, a.N / 2, r / 2, st);
 }
 

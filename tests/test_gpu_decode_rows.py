@@ -93,7 +93,7 @@ def test_fp8_rows_are_cast_like_the_oracle(oracle, M, K, scale):
 
 
 @pytest.mark.parametrize("norm", [False, True])
-@pytest.mark.parametrize("M,F,K", [(1, 16, 512), (8, 48, 1024), (9, 4112, 512), (16, 6912, 1536), (5, 5632, 2048)])
+@pytest.mark.parametrize("M,F,K", [(1, 16, 512), (8, 48, 1024), (9, 4112, 512), (16, 6912, 1536), (5, 5632, 2048), (13, 8272, 1536)])
 def test_up_gate_swiglu_is_the_separate_launches(M, F, K, norm):
     g = torch.Generator(device=DEV).manual_seed(M + F)
     x = torch.randn(M, K, generator=g, device=DEV).to(BF16)
