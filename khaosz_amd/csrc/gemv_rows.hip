@@ -480,8 +480,27 @@ bool gemv_rows_ok(RowsKind kind, int64_t M, int64_t K) {
   return true;
 }
 
+// Rows of up to 2048 and so many outputs that the rounds run into each other: 32 weight rows, 0 to 0.5 % from the best of the four
+// (2900 sizes up to 64 K outputs; by cost the last round decides, up to 38 % wrong).  Not 9 and more rows with the norm, whose
+// workgroups are alone.  us, by cost -> so: 15 x 1472 -> 38250 21.8 -> 16.7, norm 3 x 1392 -> 35618 17.4 -> 13.9.
+static bool rounds_merge(const GemvArgs& a, bool norm) {
+  return a.K <= 2048 && a.N > (a.K > 1024 ? 64 : 128) * device_cus() && !(a.M > 8 && (norm || a.K <= 1024));
+}
+
+// Two exceptions, 2200 sizes with weights from HBM:
+// * 1 to 4 bf16 rows of 3073 to 4096, where 64-row workgroups would be a round of which at most 5/8 of the units have one: five rounds
+//   of 8-row workgroups overlap enough.  us, 64 -> 8: FP8 2 x 3824 -> 8896 14.6 -> 12.7, 1 x 3440 -> 8864 13.4 -> 12.0, int8 1 x 3440 -> 10128 12.9
+//   -> 11.4; not 1 x 2864 -> 10160 (11.2 | 11.5), nor with six rounds (FP8 3 x 3504 -> 11000 13.1 | 14.0).
+// * 1 to 4 fp32 rows of 1025 to 2048, whose rounds overlap the less the larger they are: 16 at most, 1 x 1424 -> 4128 4.7 -> 4.2 (in the
+//   mean 1.6 % from the best of the four, so 0.8 %).
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {
-  switch (rows_per_workgroup(a.M, a.N, kind == ROWS_I8_NORM || a.K > 2048, 8, 64)) {
+  const bool few = a.M <= 4, f32 = kind == ROWS_I8_F32, norm = kind == ROWS_I8_NORM;
+  int rows = 32;
+  if (!rounds_merge(a, norm) || (f32 && a.K <= 1024)) {
+    rows = rows_per_workgroup(a.M, a.N, norm || a.K > 2048, 8, few && f32 && a.K > 1024 && a.K <= 2048 ? 16 : 64);
+    if (rows == 64 && few && !f32 && a.K > 3072 && a.K <= 4096 && a.N <= 5 * 8 * device_cus()) rows = 8;
+  }
+  switch (rows) {
     case 8: return launch_shape<8, 8>(a, kind, st);
     case 16: return launch_shape<8, 16>(a, kind, st);
     case 32: return launch_shape<4, 16>(a, kind, st);
@@ -498,7 +517,8 @@ int launch_gemv_rows_swiglu(const GemvArgs& a, hipStream_t st) {
 #undef AQ_GX2
 #undef AQ_GX
   static LdsOptIn unused;  // rows of at most 2048: never more than 64 KiB
-  const int r = rows_per_workgroup(a.M, a.N, a.gamma != nullptr, 32, 64);
+  const bool norm = a.gamma != nullptr;
+  const int r = a.K > 1024 && rounds_merge(a, norm) ? 32 : rows_per_workgroup(a.M, a.N, norm, 32, 64);
   return launch_rows(table[r == 64][a.M > 8][a.gamma != nullptr][a.K > 1024], unused, a, r == 64 ? 2 : 4, r, a.N / 2, r / 2, st);
 }
 
