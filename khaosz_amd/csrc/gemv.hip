@@ -926,8 +926,9 @@ static int gemv_dispatch(const aq::GemvArgs& a, int mt, hipStream_t st) {
 // Up to 4 bf16 rows have two kernels.  The dot-product kernel: one wavefront rounds a row, the others start on their weights, and
 // the few products per weight dword are no load on the vector ALU; it keeps its place with many weights per row.  gemv_rows.hip
 // for everything else: more rows; fp32 rows; rows of up to 1024 (3 and 4 of them, or of many weight rows); rows of 2049 to 4096,
-// which the dot-product kernel holds in registers for 8192 and, on short matrices, does not cut into K parts; longer ones of
-// 2049 to 4096 weight rows, too many for those parts.
+// which the dot-product kernel holds in registers for 8192 and, on short matrices, does not cut into K parts (but 1 and 2 of
+// them where 64-row workgroups are left a last round that is nearly empty: 1 x 3632 -> 10517 13.3 us, 12.0 by dot products, 1 x 3728 ->
+// 38113 39.9, 31.8); longer ones of 2049 to 4096 weight rows, too many for those parts.
 // Timed on both at 7433 random sizes, 1 to 4 rows, N 512..11264, K 512..8192, with the norm up to 2048: what this picks is 0.4 % from
 // the faster one in the mean, 3.4 % for one in twenty.  us, this | the other: 1 x 3168 -> 1472 4.0 | 5.6, 4 x 3008 -> 1488 4.0 | 5.7, 1 x 6016
 // -> 3440 6.7 | 7.8, 1 x 896 -> 9536 4.5 | 5.0, 4 x 1616 -> 1504 3.4 | 3.6; dot products 1 x 1968 -> 5648 4.5 | 5.5, 1 x 6880 -> 1585 4.8 | 5.9, 1 x
@@ -939,7 +940,7 @@ static bool dot_kernel_better(int64_t M, int64_t N, int64_t K, bool norm) {
   if (norm) return K > 1024 && N > 4096 && (M < 3 || N <= 8192);
   if (K <= 1024) return M < 3 && N <= 8192;
   if (K <= 2048) return M < 3 || N > 2048;
-  if (K <= 4096) return N > 4096 && N <= 8192;
+  if (K <= 4096) return N > 4096 && (N <= 8192 || (M < 3 && N > (K > 3072 ? 10240 : 16384)));
   return N > 4096 || (M < 3 && N <= 2048);
 }
 
