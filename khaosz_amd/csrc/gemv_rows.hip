@@ -482,7 +482,8 @@ bool gemv_rows_ok(RowsKind kind, int64_t M, int64_t K) {
 
 // Rows of up to 2048 and so many outputs that the rounds run into each other: 32 weight rows, 0 to 0.5 % from the best of the four
 // (2900 sizes up to 64 K outputs; by cost the last round decides, up to 38 % wrong).  Not 9 and more rows with the norm, whose
-// workgroups are alone.  us, by cost -> so: 15 x 1472 -> 38250 21.8 -> 16.7, norm 3 x 1392 -> 35618 17.4 -> 13.9.
+// workgroups are alone, nor 1 to 4 fp32 rows (4 x 1536 -> 20184 8.9 with 16, 10.3 with 32).  us, by cost -> so: 15 x 1472 -> 38250 21.8
+// -> 16.7, norm 3 x 1392 -> 35618 17.4 -> 13.9.
 static bool rounds_merge(const GemvArgs& a, bool norm) {
   return a.K <= 2048 && a.N > (a.K > 1024 ? 64 : 128) * device_cus() && !(a.M > 8 && (norm || a.K <= 1024));
 }
@@ -496,7 +497,7 @@ static bool rounds_merge(const GemvArgs& a, bool norm) {
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {
   const bool few = a.M <= 4, f32 = kind == ROWS_I8_F32, norm = kind == ROWS_I8_NORM;
   int rows = 32;
-  if (!rounds_merge(a, norm) || (f32 && a.K <= 1024)) {
+  if (!rounds_merge(a, norm) || (f32 && (few || a.K <= 1024))) {
     rows = rows_per_workgroup(a.M, a.N, norm || a.K > 2048, 8, few && f32 && a.K > 1024 && a.K <= 2048 ? 16 : 64);
     if (rows == 64 && few && !f32 && a.K > 3072 && a.K <= 4096 && a.N <= 5 * 8 * device_cus()) rows = 8;
   }
