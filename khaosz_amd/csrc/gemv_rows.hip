@@ -247,15 +247,24 @@ __global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
         };
         if constexpr (WHOLE) {
           uint2 code[VPL];
-          if (__builtin_expect(lean_ok, 1)) {
+          auto stretch = [&](auto from, auto to) {
+            constexpr int I0 = decltype(from)::value, I1 = decltype(to)::value;
+            if (__builtin_expect(lean_ok, 1)) {
 #pragma unroll
-            for (int i = 0; i < VPL; ++i) code[i] = cast(xr.c[j][i], true);
-          } else {
+              for (int i = I0; i < I1; ++i) code[i] = cast(xr.c[j][i], true);
+            } else {
 #pragma unroll
-            for (int i = 0; i < VPL; ++i) code[i] = cast(xr.c[j][i], false);
-          }
+              for (int i = I0; i < I1; ++i) code[i] = cast(xr.c[j][i], false);
+            }
 #pragma unroll
-          for (int i = 0; i < VPL; ++i) store(i, code[i]);
+            for (int i = I0; i < I1; ++i) store(i, code[i]);
+          };
+          // Long rows in two stretches, of which rows that fill up to 5/8 of the kernel's vectors skip the second: with one, 5 to 8 rows
+          // took longer than with a branch around each vector (K up to 2560 4 %, 4097..5120 6 %; so 3 % and 5 % less than that).
+          constexpr int HEAD = VPL < 8 ? VPL : VPL * 5 / 8;
+          stretch(std::integral_constant<int, 0>{}, std::integral_constant<int, HEAD>{});
+          if constexpr (HEAD < VPL)
+            if (nvec > HEAD * 64) stretch(std::integral_constant<int, HEAD>{}, std::integral_constant<int, VPL>{});
         } else {
 #pragma unroll
           for (int i = 0; i < VPL; ++i)

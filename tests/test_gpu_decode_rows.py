@@ -75,7 +75,8 @@ def test_fp8_rows_within_tolerance(oracle, M, N, K):
 
 # rows that are cast without a branch per vector and rows that are not, one and two to a wavefront, every length class
 @pytest.mark.parametrize("scale", [3e-26, 1e-22, 1.0, 7e21, 2e28])
-@pytest.mark.parametrize("M,K", [(1, 512), (8, 2048), (5, 4080), (8, 8192), (9, 1040), (16, 2048), (11, 4096)])
+@pytest.mark.parametrize("M,K", [(1, 512), (8, 2048), (5, 4080), (8, 8192), (9, 1040), (16, 2048), (11, 4096), (7, 2560), (6, 2576), (8, 5120),
+                                 (3, 5136)])
 def test_fp8_rows_are_cast_like_the_oracle(oracle, M, K, scale):
     """The codes that the GEMV's own cast makes, read back through a weight of ones on the diagonal: scales on both sides of
     [2^-64, 2^64], outside of which the cast takes the full divide, values on and next to the midpoints of e4m3."""
