@@ -159,8 +159,8 @@ typedef float attn_f32x4 __attribute__((ext_vector_type(4)));
 //            dimensions x G heads), the key groups are summed by swaps.
 // A launch of few sequences is one wavefront's chain of latencies, most of it
 // between the lookup of its pages and its sums (8 x 544 positions, 16/4 heads of
-// 128: 9.6 us, 4 x 576, 24/4 heads of 64: 7.0; 10.1 and 7.7 with a row lookup
-// per load, heads in registers and all sums by fused multiply-add).
+// 128: 6.9 us from a graph, 4 x 576, 24/4 heads of 64: 5.3; 8.1 and 6.3 with a
+// row lookup per load, heads in registers and all sums by fused multiply-add).
 // The wavefronts' (maximum, denominator, numerator) are merged through LDS and
 // either normalised into the output (NS == 1) or left in the workspace for
 // attn_merge_kernel.
