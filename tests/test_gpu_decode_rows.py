@@ -29,7 +29,7 @@ CASES = [(5, 1, 16), (8, 9, 112), (9, 33, 128), (16, 7, 144), (1, 2049, 1024), (
          (3, 500, 8192), (5, 2500, 4608), (2, 4600, 2400), (3, 9001, 1040), (4, 8300, 2064), (1, 4353, 6864),
          (2, 9000, 4016), (1, 10248, 3200), (3, 16400, 1040), (12, 16400, 2048), (2, 32784, 528), (1, 6200, 1488),
          # up to 4 rows, where the dot-product kernel takes over and where it does not
-         (2, 3000, 6000), (1, 1500, 3168), (4, 6000, 3200), (2, 4097, 1040)]
+         (2, 3000, 6000), (1, 1500, 3168), (4, 6000, 3200), (2, 4097, 1040), (1, 16392, 2112), (2, 16380, 3072)]
 
 
 @pytest.mark.parametrize("dtype", [BF16, F32])
