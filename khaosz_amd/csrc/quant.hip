@@ -828,23 +828,29 @@ extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_
   // bf16 rows of <= 2048 do as well one wavefront per row once there are enough rows to fill the
   // device; a handful of rows (decode) always gains from the shorter per-lane chain of a workgroup per row
   const int64_t wg_min_vec = (x_dtype == AQ_BF16 && M >= 64) ? 257 : 128;
-  if (nvec >= wg_min_vec && nvec <= 1024) {
-    // enough rows to fill the device and rows of 128..1024 vectors: one workgroup per row
+  if (nvec >= wg_min_vec && nvec <= 2048) {
+    // Rows of up to 2048 vectors (fp32 8192, bf16 16384): one workgroup per row, in registers between maximum and rounding.  With a
+    // wavefront per row, of which 1024 vectors stay in registers and the rest are read twice, the longer half took two to three times as
+    // long, us: fp32 64 x 6912 15.6 -> 5.0, 1000 x 6912 21.5 -> 9.1, 4096 x 8192 62 -> 33, 333 x 4112 10.8 -> 4.5; bf16 64 x 16384 13.1 -> 3.6.
     const unsigned g = (unsigned)M;
     if (x_dtype == AQ_BF16) {
       if (nvec <= 256)
         aq::queue_kernel((aq::quant_row_wg_kernel<true, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
       else if (nvec <= 512)
         aq::queue_kernel((aq::quant_row_wg_kernel<true, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
-      else
+      else if (nvec <= 1024)
         aq::queue_kernel((aq::quant_row_wg_kernel<true, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+      else
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 8>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
     } else {
       if (nvec <= 256)
         aq::queue_kernel((aq::quant_row_wg_kernel<false, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
       else if (nvec <= 512)
         aq::queue_kernel((aq::quant_row_wg_kernel<false, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
-      else
+      else if (nvec <= 1024)
         aq::queue_kernel((aq::quant_row_wg_kernel<false, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+      else
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 8>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
     }
     return (int)hipGetLastError();
   }
