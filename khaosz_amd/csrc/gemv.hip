@@ -1290,3 +1290,41 @@ extern "C" int aq_gemv_w8a8_decode(const void* x, int x_dtype, const int8_t* wq,
   return aq_gemv_w8a8_decode_residual(x, x_dtype, wq, sw, bias, bias_dtype, nullptr, y, y_dtype, M, N, K, ws, ws_bytes,
                                       stream);
 }
+
+// ---------------------------------------------------------------------------
+// 17 rows and more, quantised in the launch that multiplies them: the decode kernel on tiles of up to 16 rows (gemv_rows.hip).
+extern "C" int aq_linear_few_rows_ok(int x_dtype, int norm, int fp8, int64_t M, int64_t N, int64_t K) {
+  if ((x_dtype != AQ_F32 && x_dtype != AQ_BF16) || M <= 16 || N < 1 || K < 1 || K % 16) return 0;
+  if ((fp8 || norm) && (x_dtype != AQ_BF16 || (fp8 && norm))) return 0;
+  return aq::gemv_rows_tiled_ok(fp8 ? aq::ROWS_FP8 : fused_kind(norm != 0, x_dtype == AQ_BF16), M, N, K) ? 1 : 0;
+}
+
+extern "C" int aq_linear_few_rows(const void* x, int x_dtype, const void* gamma, float eps, const void* wq, int fp8, const float* sw,
+                                  const void* bias, int bias_dtype, const void* residual, void* y, int y_dtype, int64_t M, int64_t N,
+                                  int64_t K, void* stream) {
+  if ((x_dtype != AQ_F32 && x_dtype != AQ_BF16) || (y_dtype != AQ_F32 && y_dtype != AQ_BF16)) return AQ_E_DTYPE;
+  if (bias && bias_dtype != AQ_F32 && bias_dtype != AQ_BF16) return AQ_E_DTYPE;
+  if (M < 0 || N < 0 || K <= 0 || K % 16 || (gamma && !(eps >= 0.0f))) return AQ_E_SHAPE;
+  if (M == 0 || N == 0) return AQ_OK;
+  if (!x || !wq || !sw || !y) return AQ_E_NULL;
+  if (aq::check_ptr16(x) || aq::check_ptr16(gamma) || aq::check_ptr16(wq) || aq::check_ptr16(y) || aq::check_ptr(residual, 4) ||
+      aq::check_ptr(sw, 4) || aq::check_ptr(bias, bias_dtype == AQ_BF16 ? 2 : 4))
+    return AQ_E_ALIGN;
+  if (!aq_linear_few_rows_ok(x_dtype, gamma != nullptr, fp8, M, N, K)) return AQ_E_RANGE;
+  aq::GemvArgs a{};
+  a.x = x;
+  a.gamma = gamma;
+  a.eps = eps;
+  a.wq = static_cast<const int8_t*>(wq);
+  a.sw = sw;
+  a.bias = bias;
+  a.res = residual;
+  a.ldr = N;
+  a.y = y;
+  a.M = (int)M;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.bias_dtype = bias_dtype;
+  a.y_dtype = y_dtype;
+  return aq::launch_gemv_rows(a, fp8 ? aq::ROWS_FP8 : fused_kind(gamma != nullptr, x_dtype == AQ_BF16), static_cast<hipStream_t>(stream));
+}

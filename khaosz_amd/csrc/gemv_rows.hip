@@ -55,7 +55,9 @@ constexpr int64_t GX_MAX_K = 8192;
 // WPR > 0: the rows (up to 8, of up to 2048) are a decode step's attention output, combined here from the attention kernel's partial
 // results of up to 4 slices (p.parts), WPR wavefronts to a row: 4 rows of 1536 in 3 slices are 78 KB to request, and all
 // eight wavefronts ask for them at once (whole rows in 4 of 4 wavefronts, vector ALU products, N = 1536: 5.8 us; 5.3).
-template <int KS, int R, bool BF16, int RPW, int VPL, bool NORM, bool FP8, bool SWI = false, int WPR = 0>
+// TILED: more than 16 rows, a tile of p.tile_rows of them per blockIdx.y.  FP8: the scale is the maximum of all rows', the other tiles'
+// read besides.  (Kernels of their own: 25 registers more (FP8), and 0.03 to 0.05 us a launch for the tile's place.)
+template <int KS, int R, bool BF16, int RPW, int VPL, bool NORM, bool FP8, bool SWI = false, int WPR = 0, bool TILED = false>
 __global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
   constexpr int GR = GX_WAVES / KS;
   // rows rounded without a branch around each vector (see RowsToLds), where the registers allow it: with 16 vectors beside
@@ -74,7 +76,18 @@ __global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave / KS, kh = wave % KS;
-  const int K = p.K, N = p.N, M = p.M;
+  const int K = p.K, N = p.N;
+  [[maybe_unused]] const void* const all_x = p.x;  // FP8: the tensor whose maximum sets the scale
+  [[maybe_unused]] const int all_rows = p.M;
+  if constexpr (TILED) {
+    const int first = blockIdx.y * p.tile_rows;
+    p.M = all_rows - first < p.tile_rows ? all_rows - first : p.tile_rows;
+    p.x = static_cast<const uint8_t*>(p.x) + (int64_t)first * K * (BF16 ? 2 : 4);
+    const int64_t out = (int64_t)first * (SWI ? N >> 1 : N) * (p.y_dtype == AQ_BF16 ? 2 : 4);
+    p.y = static_cast<uint8_t*>(p.y) + out;
+    if (p.res) p.res = static_cast<const uint8_t*>(p.res) + out;
+  }
+  const int M = p.M;
   const int nline_all = (K + 127) >> 7;
   const int pitch = (nline_all << 7) + 16;  // 16 token rows then start 4 banks apart
   const int per = (nline_all + KS - 1) / KS;
@@ -202,6 +215,21 @@ __global__ __launch_bounds__(GX_WAVES * 64) void gemv_rows_kernel(GemvArgs p) {
           RowIn<true>::unpack(xr.c[j][i], f);  // rows >= M and vectors past K were loaded as zeros
           amax = fmaxf(amax, vec_amax<8>(f));
         }
+      if constexpr (TILED) {  // and of the other tiles
+        const uint4* const src = static_cast<const uint4*>(all_x);
+        const int nv = all_rows * (K / 8);
+        for (int v = tid; v < nv; v += 8 * GX_WAVES * 64) {
+          uint4 t[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) t[u] = src[v + u * GX_WAVES * 64 < nv ? v + u * GX_WAVES * 64 : v];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            float f[8];
+            RowIn<true>::unpack(t[u], f);
+            amax = fmaxf(amax, vec_amax<8>(f));
+          }
+        }
+      }
       amax = wave_max(amax);
       if (lane == 0) sx_lds[wave] = amax;
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
@@ -440,40 +468,37 @@ using rows_kernel_t = void (*)(GemvArgs);
 
 static int launch_rows(rows_kernel_t fn, LdsOptIn& opted, const GemvArgs& a, int ks, int rows_per_wg, int64_t outputs, int outputs_per_wg,
                        hipStream_t st) {
-  const size_t lds = gemv_rows_lds(a.M, a.K, ks, rows_per_wg);
+  const size_t lds = gemv_rows_lds(a.tile_rows ? a.tile_rows : a.M, a.K, ks, rows_per_wg);
   if (lds > 64 * 1024) {
     const int e = opted.ensure(reinterpret_cast<const void*>(fn));
     if (e) return e;
   }
   const unsigned grid = (unsigned)((outputs + outputs_per_wg - 1) / outputs_per_wg);
-  aq::queue_kernel(fn, dim3(grid), dim3(GX_WAVES * 64), lds, st, a);
+  const unsigned tiles = a.tile_rows ? (unsigned)((a.M + a.tile_rows - 1) / a.tile_rows) : 1u;
+  aq::queue_kernel(fn, dim3(grid, tiles), dim3(GX_WAVES * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 
 // the row length class: vectors per lane of a row, rounded up to what kernels are built for
 static int length_class(int64_t vectors) { return vectors <= 128 ? 0 : vectors <= 256 ? 1 : vectors <= 512 ? 2 : 3; }
 
-template <int KS, int R>
+template <int KS, int R, bool TILED>
 static int launch_shape(const GemvArgs& a, RowsKind kind, hipStream_t st) {
-#define AQ_GX(RPW, FP8)                                                                                   \
-  {gemv_rows_kernel<KS, R, true, RPW, 2, false, FP8>, gemv_rows_kernel<KS, R, true, RPW, 4, false, FP8>,  \
-   gemv_rows_kernel<KS, R, true, RPW, 8, false, FP8>, gemv_rows_kernel<KS, R, true, RPW, 16, false, FP8>}
-  static const rows_kernel_t i8[2][4] = {AQ_GX(1, false), AQ_GX(2, false)};
-#undef AQ_GX
+#define AQ_GX(BF16, RPW, VPL, NORM, FP8) gemv_rows_kernel<KS, R, BF16, RPW, VPL, NORM, FP8, false, 0, TILED>
+  static const rows_kernel_t i8[2][4] = {
+      {AQ_GX(true, 1, 2, false, false), AQ_GX(true, 1, 4, false, false), AQ_GX(true, 1, 8, false, false), AQ_GX(true, 1, 16, false, false)},
+      {AQ_GX(true, 2, 2, false, false), AQ_GX(true, 2, 4, false, false), AQ_GX(true, 2, 8, false, false), AQ_GX(true, 2, 16, false, false)}};
   // (16 rows of more than 4096 cannot stay in registers between the tensor's maximum and the cast: gemv_rows_ok)
   static const rows_kernel_t f8[2][4] = {
-      {gemv_rows_kernel<KS, R, true, 1, 2, false, true>, gemv_rows_kernel<KS, R, true, 1, 4, false, true>,
-       gemv_rows_kernel<KS, R, true, 1, 8, false, true>, gemv_rows_kernel<KS, R, true, 1, 16, false, true>},
-      {gemv_rows_kernel<KS, R, true, 2, 2, false, true>, gemv_rows_kernel<KS, R, true, 2, 4, false, true>,
-       gemv_rows_kernel<KS, R, true, 2, 8, false, true>, nullptr}};
-  static const rows_kernel_t norm[2][2] = {
-      {gemv_rows_kernel<KS, R, true, 1, 2, true, false>, gemv_rows_kernel<KS, R, true, 1, 4, true, false>},
-      {gemv_rows_kernel<KS, R, true, 2, 2, true, false>, gemv_rows_kernel<KS, R, true, 2, 4, true, false>}};
-  static const rows_kernel_t f32[3] = {gemv_rows_kernel<KS, R, false, 1, 4, false, false>,
-                                       gemv_rows_kernel<KS, R, false, 1, 8, false, false>,
-                                       gemv_rows_kernel<KS, R, false, 1, 32, false, false>};
+      {AQ_GX(true, 1, 2, false, true), AQ_GX(true, 1, 4, false, true), AQ_GX(true, 1, 8, false, true),
+       TILED ? nullptr : gemv_rows_kernel<KS, R, true, 1, 16, false, true>},
+      {AQ_GX(true, 2, 2, false, true), AQ_GX(true, 2, 4, false, true), AQ_GX(true, 2, 8, false, true), nullptr}};
+  static const rows_kernel_t norm[2][2] = {{AQ_GX(true, 1, 2, true, false), AQ_GX(true, 1, 4, true, false)},
+                                           {AQ_GX(true, 2, 2, true, false), AQ_GX(true, 2, 4, true, false)}};
+  static const rows_kernel_t f32[3] = {AQ_GX(false, 1, 4, false, false), AQ_GX(false, 1, 8, false, false), AQ_GX(false, 1, 32, false, false)};
+#undef AQ_GX
   static LdsOptIn opted[2][4][4];
-  const int two = a.M > 8, len = length_class(a.K / (kind == ROWS_I8_F32 ? 4 : 8));
+  const int two = (TILED ? a.tile_rows : a.M) > 8, len = length_class(a.K / (kind == ROWS_I8_F32 ? 4 : 8));
   const int flen = a.K <= 1024 ? 0 : a.K <= 2048 ? 1 : 2;
   const rows_kernel_t fn = kind == ROWS_I8_F32    ? f32[flen]
                            : kind == ROWS_I8_NORM ? norm[two][len]
@@ -503,18 +528,74 @@ static bool rounds_merge(const GemvArgs& a, bool norm) {
 //   -> 11.4; not 1 x 2864 -> 10160 (11.2 | 11.5), nor with six rounds (FP8 3 x 3504 -> 11000 13.1 | 14.0).
 // * 1 to 4 fp32 rows of 1025 to 2048, whose rounds overlap the less the larger they are: 16 at most, 1 x 1424 -> 4128 4.7 -> 4.2 (in the
 //   mean 1.6 % from the best of the four, so 0.8 %).
+// More than 16 rows: tiles of 9..16 or of up to 8 rows, each with its own workgroups over the weight rows.  Every tile reads the
+// weights and every workgroup rounds its tile's rows again, so it is the faster form while tiles x outputs x row length is small:
+// one launch then stands for the quantiser's and the GEMM's (FP8: the maximum's, the cast's and the GEMM's), 3.3 to 5 us of which are
+// launches and first requests.  Both ways as fitted to 4265 random sizes of 17 to 200 rows, us (K in units of 1024; `length`: the row
+// length class, whose vectors are requested whether the row has them or not):
+//   tiles      start + rounds over the compute units x (row x tile rows x length + weight x weight rows x K + all x M x K)
+//   launches   two[0] + two[1] K + two[2] M N K / 10^6 + (more than one tile of 32 x 32 per unit: two[3]) + two[4] N K / 10^4
+// Taken where the tiles are 10 % ahead by that: two sizes in five, at 0.77 of the time in the mean, one in 60 of them slower (by 1 to 8 %, three
+// by more); the choice is 1 % from the faster way in the mean.  us, launches -> tiles: bf16 32 x 2048 -> 2048 6.8 -> 4.7, 64 x 1024 -> 3072 6.4 ->
+// 5.1, 32 x 512 -> 8192 5.9 -> 4.8, fp32 64 x 512 -> 2048 5.7 -> 4.2, norm 48 x 1024 -> 2048 6.6 -> 4.3, FP8 35 x 1456 -> 944 8.5 -> 6.3; not 64 x 2048 ->
+// 3072 (6.9, tiles 8.1) nor fp32 64 x 2048 -> 2048 (7.2, 7.6).
+struct TiledCost {
+  double start, row, weight, all, two[5];
+};
+static const TiledCost& tiled_cost(RowsKind kind) {
+  static const TiledCost i8 = {3.07, 0.038, 0.038, 0, {5.5, 0.77, 2.32, 0.91, 0.47}}, norm = {3.24, 0.083, 0.033, 0, {5.79, 0.95, 1.8, 0.86, 0.98}},
+                         f32 = {3.26, 0.041, 0.042, 0, {5.0, 1.3, 2.06, 0.82, 0.58}}, f8 = {3.81, 0.054, 0.047, 0.018, {7.53, 0.82, 3.34, 0.67, 0.38}};
+  return kind == ROWS_I8 ? i8 : kind == ROWS_I8_NORM ? norm : kind == ROWS_I8_F32 ? f32 : f8;
+}
+struct Tiled {
+  int tile_rows, weight_rows;
+  double us;
+};
+static Tiled tiled_best(RowsKind kind, int64_t M, int64_t N, int64_t K) {
+  const TiledCost& c = tiled_cost(kind);
+  const double k = (double)K / 1024, length = K <= 1024 ? 1 : K <= 2048 ? 2 : kind == ROWS_I8_F32 ? 11.2 : K <= 4096 ? 4 : 8;
+  const int64_t cus = device_cus();
+  Tiled best = {0, 0, 1e30};
+  for (int most = 8; most <= 16; most += 8) {
+    const int64_t tiles = (M + most - 1) / most, rows = (M + tiles - 1) / tiles;
+    for (int r = 16; r <= 64; r *= 2) {
+      const double us = c.start + (double)(((N + r - 1) / r * tiles + cus - 1) / cus) * (c.row * rows * length + c.weight * r * k + c.all * M * k);
+      if (us < best.us) best = {(int)rows, r, us};
+    }
+  }
+  return best;
+}
+bool gemv_rows_tiled_ok(RowsKind kind, int64_t M, int64_t N, int64_t K) {
+  // Tiles of more outputs than 80 to a compute unit never gained (64 x 512 -> 8192: 6.3 | 6.6).
+  if (M <= 16 || (M + 15) / 16 * N > 80 * device_cus() || K > (kind == ROWS_I8_NORM ? 2048 : kind == ROWS_FP8 ? 4096 : GX_MAX_K)) return false;
+  const double* two = tiled_cost(kind).two;
+  const double k = (double)K / 1024, nk = (double)N * k;
+  const bool rounds = (M + 31) / 32 * ((N + 31) / 32) > device_cus();
+  return tiled_best(kind, M, N, K).us < 0.9 * (two[0] + two[1] * k + two[2] * M * nk / 1e6 + (rounds ? two[3] : 0) + two[4] * nk / 1e4);
+}
+
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {
   const bool few = a.M <= 4, f32 = kind == ROWS_I8_F32, norm = kind == ROWS_I8_NORM;
+  if (a.M > 16) {
+    const Tiled best = tiled_best(kind, a.M, a.N, a.K);
+    GemvArgs t = a;
+    t.tile_rows = best.tile_rows;
+    switch (best.weight_rows) {
+      case 16: return launch_shape<8, 16, true>(t, kind, st);
+      case 32: return launch_shape<4, 16, true>(t, kind, st);
+      default: return launch_shape<2, 16, true>(t, kind, st);
+    }
+  }
   int rows = 32;
   if (!rounds_merge(a, norm) || (f32 && (few || a.K <= 1024))) {
     rows = rows_per_workgroup(a.M, a.N, norm || a.K > 2048, 8, few && f32 && a.K > 1024 && a.K <= 2048 ? 16 : 64);
     if (rows == 64 && few && !f32 && a.K > 3072 && a.K <= 4096 && a.N <= 5 * 8 * device_cus()) rows = 8;
   }
   switch (rows) {
-    case 8: return launch_shape<8, 8>(a, kind, st);
-    case 16: return launch_shape<8, 16>(a, kind, st);
-    case 32: return launch_shape<4, 16>(a, kind, st);
-    default: return launch_shape<2, 16>(a, kind, st);
+    case 8: return launch_shape<8, 8, false>(a, kind, st);
+    case 16: return launch_shape<8, 16, false>(a, kind, st);
+    case 32: return launch_shape<4, 16, false>(a, kind, st);
+    default: return launch_shape<2, 16, false>(a, kind, st);
   }
 }
 

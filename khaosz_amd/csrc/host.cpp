@@ -42,6 +42,8 @@ namespace {
   X(aq_gemv_w8a8_workspace_bytes)                                                                                \
   X(aq_gemv_w8a8_decode_one_launch)                                                                              \
   X(aq_gemv_fp8_decode_one_launch)                                                                               \
+  X(aq_linear_few_rows_ok)                                                                                       \
+  X(aq_linear_few_rows)                                                                                          \
   X(aq_gemv_w8a8_decode_residual)                                                                                \
   X(aq_gemv_w8a8_decode_rmsnorm)                                                                                 \
   X(aq_gemv_w8a8_codes_residual)                                                                                 \
@@ -622,8 +624,9 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   const int64_t room = codes + (!few ? (fp8 ? 256 + AQ_FP8_AMAX_WS_BYTES : 4 * r.M) : 0);
   void* yp = y.mutable_data_ptr();
   // a launch that quantises its rows itself touches no workspace: an allocation is 0.4 us of a 5 us call
-  const bool alone = few && (fp8 ? lib.aq_gemv_fp8_decode_one_launch(r.code, r.M, r.K)
-                                 : lib.aq_gemv_w8a8_decode_one_launch(r.code, gain != nullptr, r.M, N, r.K));
+  const bool tiles = !few && lib.aq_linear_few_rows_ok(r.code, gain != nullptr, fp8, r.M, N, r.K);
+  const bool alone = tiles || (few && (fp8 ? lib.aq_gemv_fp8_decode_one_launch(r.code, r.M, r.K)
+                                 : lib.aq_gemv_w8a8_decode_one_launch(r.code, gain != nullptr, r.M, N, r.K)));
   Tensor ws;
   if (!alone) ws = c.empty({room}, ScalarType::Byte);
   char* base = static_cast<char*>(alone ? yp : ws.mutable_data_ptr());
@@ -632,6 +635,10 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   const auto* sp = static_cast<const float*>(s->const_data_ptr());
   const char* what = "";
   const int rc = queued([&]() -> int {
+    if (tiles) {
+      what = "aq_linear_few_rows";
+      return lib.aq_linear_few_rows(r.p, r.code, gain, eps, wp, fp8, sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
+    }
     if (few) {
       what = fp8 ? "aq_gemv_fp8_decode" : "aq_gemv_w8a8_decode";
       if (fp8)
@@ -881,7 +888,8 @@ void Block::lay_out() {
 }
 
 // Queues the block's launches: the ones, in the order and with the operands, of the step-by-step path in block.py, but that a prompt's
-// queries may be rotated in its attention instead of before it (rotates(); the same bits).
+// queries may be rotated in its attention instead of before it (rotates()), and a small prompt's rows quantised in the launch that
+// multiplies them (aq_linear_few_rows); the same bits.
 int Block::queue(const void* in, void* out, char* base, const char** what) const {
   const bool few = this->few();
   const int64_t W = qkv.N, A = Hq * D, KV = Hkv * D;
@@ -896,6 +904,10 @@ int Block::queue(const void* in, void* out, char* base, const char** what) const
       return lib.aq_gemv_w8a8_decode_rmsnorm(x, AQ_BF16, g.p, g.eps, p.w, p.s, p.b.p, p.b.code, nullptr, y, AQ_BF16, M, p.N, p.K, room,
                                              lib.aq_gemv_w8a8_workspace_bytes(M, p.K), c.stream);
     }
+    if (lib.aq_linear_few_rows_ok(AQ_BF16, 1, 0, M, p.N, p.K)) {
+      *what = "aq_linear_few_rows";
+      return lib.aq_linear_few_rows(x, AQ_BF16, g.p, g.eps, p.w, 0, p.s, p.b.p, p.b.code, nullptr, y, AQ_BF16, M, p.N, p.K, c.stream);
+    }
     *what = "aq_rmsnorm_quant_rowwise_i8";
     int rc = lib.aq_rmsnorm_quant_rowwise_i8(x, AQ_BF16, g.p, AQ_BF16, g.eps, M, p.K, p.K, static_cast<int8_t*>(room), sx, c.stream);
     if (rc) return rc;
@@ -909,6 +921,10 @@ int Block::queue(const void* in, void* out, char* base, const char** what) const
       *what = "aq_gemv_w8a8_decode";
       return lib.aq_gemv_w8a8_decode_residual(x, AQ_BF16, p.w, p.s, p.b.p, p.b.code, res, y, AQ_BF16, M, p.N, p.K, room,
                                               lib.aq_gemv_w8a8_workspace_bytes(M, p.K), c.stream);
+    }
+    if (lib.aq_linear_few_rows_ok(AQ_BF16, 0, 0, M, p.N, p.K)) {
+      *what = "aq_linear_few_rows";
+      return lib.aq_linear_few_rows(x, AQ_BF16, nullptr, 0.f, p.w, 0, p.s, p.b.p, p.b.code, res, y, AQ_BF16, M, p.N, p.K, c.stream);
     }
     *what = "aq_quant_rowwise_i8";
     int rc = lib.aq_quant_rowwise_i8(x, AQ_BF16, M, p.K, p.K, static_cast<int8_t*>(room), sx, c.stream);
