@@ -220,6 +220,25 @@ int aq_gemv_fp8_decode_residual(const void *x, int x_dtype, const uint8_t *wq, c
                                 int y_dtype, int64_t M, int64_t N, int64_t K, void *ws, size_t ws_bytes,
                                 void *stream);
 
+/* Codes in rows that begin ldx (ldq) bytes apart, at least K and a multiple of 16: the quantisers that write them and
+ * the Linears that take them (otherwise aq_quant_rowwise_i8, aq_quant_tensor_fp8(_onepass) of M * K elements,
+ * aq_linear_w8a8_residual and aq_linear_fp8_residual).  With rows that begin on 128-byte lines the tiled kernels bring in
+ * half as many lines of them: aq_linear_codes_pitch is the distance to take for a Linear of M > 16 rows, K or the next
+ * multiple of 128. */
+int64_t aq_linear_codes_pitch(int fp8, int64_t M, int64_t N, int64_t K);
+int aq_quant_rowwise_i8_strided(const void *x, int x_dtype, int64_t M, int64_t K, int64_t ldx, int8_t *q, int64_t ldq,
+                                float *scale, void *stream);
+int aq_quant_tensor_fp8_strided(const void *x, int x_dtype, int64_t M, int64_t K, uint8_t *q, int64_t ldq,
+                                float *scale, uint32_t *amax_ws, size_t ws_bytes, void *stream);
+int aq_quant_tensor_fp8_onepass_strided(const void *x, int x_dtype, int64_t M, int64_t K, uint8_t *q, int64_t ldq,
+                                        float *scale, void *ws, size_t ws_bytes, void *stream);
+int aq_linear_w8a8_strided(const int8_t *xq, int64_t ldx, const float *sx, const int8_t *wq, const float *sw,
+                           const void *bias, int bias_dtype, const void *residual, void *y, int y_dtype, int64_t M,
+                           int64_t N, int64_t K, void *stream);
+int aq_linear_fp8_strided(const uint8_t *xq, int64_t ldx, const float *sx, const uint8_t *wq, const float *sw,
+                          const void *bias, int bias_dtype, const void *residual, void *y, int y_dtype, int64_t M,
+                          int64_t N, int64_t K, void *stream);
+
 /* A Linear of 17 rows and more in one launch that quantises them itself (normalises them first, with gamma), for small
  * ones: aq_linear_few_rows_ok tells whether that is the faster form of a shape, for rows of x_dtype (norm and fp8: bf16, and not
  * both), and aq_linear_few_rows takes no other (AQ_E_RANGE).  The bits of aq_quant_rowwise_i8 (aq_rmsnorm_quant_rowwise_i8) +

@@ -371,6 +371,18 @@ __device__ __forceinline__ void store_wt(uint2* p, uint2 v) {
 #endif
 }
 
+// n / d for 0 <= n < 2^31 as a product: mul = ceil(2^(31 + s) / d) with s = ceil(log2 d), so mul d - 2^(31 + s) < d <= 2^s and
+// the quotient is exact.
+struct UDiv {
+  uint32_t mul, shift;
+  static UDiv of(uint32_t d) {
+    uint32_t s = 0;
+    while (((uint64_t)1 << s) < d) ++s;
+    return {(uint32_t)((((uint64_t)1 << (31 + s)) + d - 1) / d), s};
+  }
+  __device__ __forceinline__ uint32_t operator()(uint32_t n) const { return __umulhi(2 * n, mul) >> shift; }
+};
+
 inline int check_ptr16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ? AQ_E_ALIGN : AQ_OK; }
 inline int check_ptr(const void* p, unsigned align) { return (reinterpret_cast<uintptr_t>(p) & (align - 1u)) ? AQ_E_ALIGN : AQ_OK; }
 

@@ -18,6 +18,7 @@ struct GemmArgs {
   const uint8_t* B;
   void* C;
   int M, N, K;
+  int lda;           // bytes between rows of A: K, or more (rows that begin on lines)
   int tiles_m, tiles_n;
   const float* sx;   // int8: [M]; fp8: [1]
   const float* sw;   // int8: [N]; fp8: [1]

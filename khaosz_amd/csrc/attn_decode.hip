@@ -77,18 +77,6 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(RopeArgs p) {
   *reinterpret_cast<uint4*>(dst) = x;
 }
 
-// n / d for 0 <= n < 2^31 as a product: mul = ceil(2^(31 + s) / d) with s = ceil(log2 d), so mul d - 2^(31 + s) < d <= 2^s and
-// the quotient is exact.
-struct UDiv {
-  uint32_t mul, shift;
-  static UDiv of(uint32_t d) {
-    uint32_t s = 0;
-    while (((uint64_t)1 << s) < d) ++s;
-    return {(uint32_t)((((uint64_t)1 << (31 + s)) + d - 1) / d), s};
-  }
-  __device__ __forceinline__ uint32_t operator()(uint32_t n) const { return __umulhi(2 * n, mul) >> shift; }
-};
-
 struct AttnArgs {
   const uint16_t* q;     // [B, Hq, D]
   const uint16_t* kc;    // [n_pages, page, Hkv, D]

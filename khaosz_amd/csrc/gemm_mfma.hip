@@ -155,7 +155,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   // Tile-local buffer descriptors: rows past the M / N edge fall outside and read as zero.
   const int rows_a = (M - m0) < BM ? (M - m0) : BM;
   const int rows_b = (N - n0) < BN ? (N - n0) : BN;
-  const __amdgpu_buffer_rsrc_t Ar = make_rsrc(p.A + (int64_t)m0 * K, (uint32_t)rows_a * (uint32_t)K);
+  const __amdgpu_buffer_rsrc_t Ar = make_rsrc(p.A + (int64_t)m0 * p.lda, (uint32_t)rows_a * (uint32_t)p.lda);
   const __amdgpu_buffer_rsrc_t Br = make_rsrc(p.B + (int64_t)n0 * K, (uint32_t)rows_b * (uint32_t)K);
 
   const int col = lane & 31;
@@ -179,10 +179,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   // 128-byte line (fp32 and int32 outputs fill one with a column each).
   constexpr bool ADJ = TN == 2 && OUT == OUT_BF16;
   const bool pair_ok = (N & 1) == 0;  // uniform: bf16 rows start dword-aligned, pairs never straddle N
-  uint32_t ld_vo[A_LOADS > B_LOADS ? A_LOADS : B_LOADS];  // EXACT: lane offset of row group i, A and B alike
+  uint32_t ld_vo[A_LOADS > B_LOADS ? A_LOADS : B_LOADS];  // lane offset of row group i; EXACT: A and B alike
+  uint32_t ld_va[EXACT ? 1 : A_LOADS];                     // not EXACT: of A, whose rows may be further apart
   uint32_t ld_vb[ADJ ? B_LOADS : 1];                       // ... of B, where its rows have an order of their own
 #pragma unroll
   for (int i = 0; i < (A_LOADS > B_LOADS ? A_LOADS : B_LOADS); ++i) ld_vo[i] = ld_off + (uint32_t)i * row32;
+  if constexpr (!EXACT) {
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i) ld_va[i] = (uint32_t)(ld_row + i * RPG * NWAVES) * (uint32_t)p.lda + ld_piece;
+  }
   if constexpr (ADJ) {
 #pragma unroll
     for (int i = 0; i < B_LOADS; ++i) {
@@ -211,7 +216,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
     uint8_t* st = smem + buf * STAGE + wave * 1024;
     if (idx < A_LOADS)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(Ar, (lds_void*)(st + idx * (1024 * NWAVES)), 16,
-                                               in ? ld_vo[idx] + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
+                                               in ? ld_va[EXACT ? 0 : idx] + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(Br, (lds_void*)(st + BM * BK + (idx - A_LOADS) * (1024 * NWAVES)), 16,
                                                in ? b_off(idx - A_LOADS) + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
@@ -784,7 +789,7 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
     }
   } clk;
 #endif
-  const bool exact = (p.K % S::BK) == 0;  // uniform
+  const bool exact = (p.K % S::BK) == 0 && p.lda == p.K;  // uniform
   for (int pid = blockIdx.x; pid < nt; pid += gridDim.x) {
     if constexpr (S::BIG)
       gemm_tile<FP8, OUT, S, true>(p, smem, pid);  // launched for whole K steps and even N only
@@ -887,7 +892,7 @@ static int launch_shape(GemmArgs& a, hipStream_t st) {
 // In all 6 % faster than the walk where it is taken, and the choice 2 % from the best tile in the mean (taken for any K above 2048
 // and any last round, 11 %).
 static bool huge_fp8_ok(const GemmArgs& a, int64_t cus) {
-  if (a.K <= 3072 || a.K % (2 * ShapeHuge::BK) != ShapeHuge::BK || (a.N % 2) != 0 || (a.M % ShapeHuge::BM) != 0 || a.res != nullptr) return false;
+  if (a.lda != a.K || a.K <= 3072 || a.K % (2 * ShapeHuge::BK) != ShapeHuge::BK || (a.N % 2) != 0 || (a.M % ShapeHuge::BM) != 0 || a.res != nullptr) return false;
   const int64_t tiles = (int64_t)(a.M / ShapeHuge::BM) * ((a.N + ShapeHuge::BN - 1) / ShapeHuge::BN);
   return tiles >= 2 * cus && (tiles % cus == 0 || 2 * (tiles % cus) > cus);
 }
@@ -959,7 +964,7 @@ static GemmArgs make_args(const void* A, const void* B, void* C, int64_t M, int6
   a.C = C;
   a.M = (int)M;
   a.N = (int)N;
-  a.K = (int)K;
+  a.K = a.lda = (int)K;
   return a;
 }
 
@@ -1004,36 +1009,48 @@ bool gemv_tokens_ok(int64_t M, int64_t N, int64_t K);
 int gemv_tokens_launch(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw, const void* bias,
                        int bias_dtype, const void* residual, void* y, int y_dtype, int64_t M, int64_t N, int64_t K,
                        hipStream_t st, bool fp8);
+
+// 17..32 rows of more than 8192 outputs (and decode batches of rows too long for the GEMV kernels): the weight-streaming kernel takes
+// them (not when a test has forced a tile shape)
+static bool streams_weights(int64_t M, int64_t N, int64_t K) {
+#ifdef AQ_LAB
+  if (g_forced_tile) return false;
+#endif
+  return !gemm_slices_rows(M, N, K, device_cus()) && gemv_tokens_ok(M, N, K);
+}
 }  // namespace aq
 
-extern "C" int aq_linear_w8a8_residual(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
-                                       const void* bias, int bias_dtype, const void* residual, void* y, int y_dtype,
-                                       int64_t M, int64_t N, int64_t K, void* stream) {
+namespace aq {
+// y = codes [M, K], rows ldx bytes apart, times weights [N, K], scaled
+static int linear_codes(bool fp8, const void* xq, int64_t ldx, const float* sx, const void* wq, const float* sw, const void* bias, int bias_dtype,
+                        const void* residual, void* y, int y_dtype, int64_t M, int64_t N, int64_t K, void* stream) {
   if (y_dtype != AQ_F32 && y_dtype != AQ_BF16) return AQ_E_DTYPE;
   if (bias && bias_dtype != AQ_F32 && bias_dtype != AQ_BF16) return AQ_E_DTYPE;
-  int rc = aq::check_gemm(xq, wq, y, M, N, K);
+  int rc = check_gemm(xq, wq, y, M, N, K);
+  if (!rc && (ldx < K || ldx % 16 || ldx > (1 << 22))) return ldx < K ? AQ_E_SHAPE : ldx % 16 ? AQ_E_ALIGN : AQ_E_RANGE;
   if (rc || M == 0 || N == 0) return rc;
   if (!sx || !sw) return AQ_E_NULL;
-  if (aq::check_ptr(sx, 4) || aq::check_ptr(sw, 4) || aq::check_ptr(bias, bias_dtype == AQ_BF16 ? 2 : 4) ||
-      aq::check_ptr(residual, 4))
-    return AQ_E_ALIGN;
+  if (check_ptr(sx, 4) || check_ptr(sw, 4) || check_ptr(bias, bias_dtype == AQ_BF16 ? 2 : 4) || check_ptr(residual, 4)) return AQ_E_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // 17..32 rows of more than 8192 outputs (and decode batches of rows too long for the GEMV kernels): the weight-streaming
-  // kernel takes them (not when a test has forced a tile shape)
-#ifdef AQ_LAB
-  const bool tile_forced = aq::g_forced_tile != 0;
-#else
-  const bool tile_forced = false;
-#endif
-  if (!tile_forced && !aq::gemm_slices_rows(M, N, K, aq::device_cus()) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
-    return aq::gemv_tokens_launch(xq, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, st, false);
-  aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);
+  if (ldx == K && streams_weights(M, N, K) && check_ptr16(residual) == 0)
+    return gemv_tokens_launch(static_cast<const int8_t*>(xq), sx, static_cast<const int8_t*>(wq), sw, bias, bias_dtype, residual, y, y_dtype, M, N, K,
+                              st, fp8);
+  GemmArgs a = make_args(xq, wq, y, M, N, K);
+  a.lda = (int)ldx;
   a.sx = sx;
   a.sw = sw;
   a.bias = bias;
   a.bias_dtype = bias_dtype;
   a.res = residual;
-  return y_dtype == AQ_BF16 ? aq::launch<false, aq::OUT_BF16>(a, st) : aq::launch<false, aq::OUT_F32>(a, st);
+  if (fp8) return y_dtype == AQ_BF16 ? launch<true, OUT_BF16>(a, st) : launch<true, OUT_F32>(a, st);
+  return y_dtype == AQ_BF16 ? launch<false, OUT_BF16>(a, st) : launch<false, OUT_F32>(a, st);
+}
+}  // namespace aq
+
+extern "C" int aq_linear_w8a8_residual(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
+                                       const void* bias, int bias_dtype, const void* residual, void* y, int y_dtype,
+                                       int64_t M, int64_t N, int64_t K, void* stream) {
+  return aq::linear_codes(false, xq, K, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, stream);
 }
 
 extern "C" int aq_linear_fp8(const uint8_t* xq, const float* sx, const uint8_t* wq, const float* sw,
@@ -1044,29 +1061,30 @@ extern "C" int aq_linear_fp8(const uint8_t* xq, const float* sx, const uint8_t* 
 extern "C" int aq_linear_fp8_residual(const uint8_t* xq, const float* sx, const uint8_t* wq, const float* sw,
                                       const void* bias, int bias_dtype, const void* residual, void* y, int y_dtype,
                                       int64_t M, int64_t N, int64_t K, void* stream) {
-  if (y_dtype != AQ_F32 && y_dtype != AQ_BF16) return AQ_E_DTYPE;
-  if (bias && bias_dtype != AQ_F32 && bias_dtype != AQ_BF16) return AQ_E_DTYPE;
-  int rc = aq::check_gemm(xq, wq, y, M, N, K);
-  if (rc || M == 0 || N == 0) return rc;
-  if (!sx || !sw) return AQ_E_NULL;
-  if (aq::check_ptr(sx, 4) || aq::check_ptr(sw, 4) || aq::check_ptr(bias, bias_dtype == AQ_BF16 ? 2 : 4) ||
-      aq::check_ptr(residual, 4))
-    return AQ_E_ALIGN;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  // 17..32 rows of many outputs: the weight-streaming kernel, as for int8 (fp32 sums in its own fixed order)
-#ifdef AQ_LAB
-  const bool tile_forced = aq::g_forced_tile != 0;
-#else
-  const bool tile_forced = false;
-#endif
-  if (!tile_forced && !aq::gemm_slices_rows(M, N, K, aq::device_cus()) && aq::gemv_tokens_ok(M, N, K) && aq::check_ptr16(residual) == 0)
-    return aq::gemv_tokens_launch(reinterpret_cast<const int8_t*>(xq), sx, reinterpret_cast<const int8_t*>(wq), sw, bias,
-                                  bias_dtype, residual, y, y_dtype, M, N, K, st, true);
-  aq::GemmArgs a = aq::make_args(xq, wq, y, M, N, K);
-  a.sx = sx;
-  a.sw = sw;
-  a.bias = bias;
-  a.bias_dtype = bias_dtype;
-  a.res = residual;
-  return y_dtype == AQ_BF16 ? aq::launch<true, aq::OUT_BF16>(a, st) : aq::launch<true, aq::OUT_F32>(a, st);
+  return aq::linear_codes(true, xq, K, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, stream);
+}
+
+extern "C" int aq_linear_w8a8_strided(const int8_t* xq, int64_t ldx, const float* sx, const int8_t* wq, const float* sw,
+                                      const void* bias, int bias_dtype, const void* residual, void* y, int y_dtype,
+                                      int64_t M, int64_t N, int64_t K, void* stream) {
+  return aq::linear_codes(false, xq, ldx, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, stream);
+}
+
+extern "C" int aq_linear_fp8_strided(const uint8_t* xq, int64_t ldx, const float* sx, const uint8_t* wq, const float* sw,
+                                     const void* bias, int bias_dtype, const void* residual, void* y, int y_dtype,
+                                     int64_t M, int64_t N, int64_t K, void* stream) {
+  return aq::linear_codes(true, xq, ldx, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, stream);
+}
+
+// Rows of K bytes that are no whole number of 128-byte lines begin in the middle of one, all but every eighth, and each 128-byte step of such
+// a row is two halves of lines: twice the requests, of which a compute unit has so many in flight.  The weights are the caller's; the codes
+// of the activations are written here, to rows that begin on lines.  us, K apart -> whole lines (all rows on lines, weights too): 798 x 4704 -> 1648 19.4 -> 16.2
+// (13.9), 333 x 6896 -> 1536 18.5 -> 14.9 (12.6), 2048 x 6896 -> 1536 35.3 -> 30.0 (25.0), 4096 x 2032 -> 11264 108 -> 92.5 (89.4), 7601 x 4272 -> 1096 47.7 ->
+// 44.9 (40.5), FP8 4958 x 1264 -> 6288 51.2 -> 43.2, 952 x 3392 -> 1392 13.2 -> 11.8 (10.8); level with few rows (64 x 2032 -> 2048 4.2).  Not where the
+// 256 x 256 FP8 tile serves, whose 64-byte steps halve no line, nor the weight-streaming kernel, which takes rows as they are.
+extern "C" int64_t aq_linear_codes_pitch(int fp8, int64_t M, int64_t N, int64_t K) {
+  if (M <= 16 || N < 1 || K < 1 || K % 16 || K % 128 == 0 || K > (1 << 22) - 128 || M > (1 << 30) || M * K / 8 > (int64_t)0x7fffffff) return K;
+  if (aq::streams_weights(M, N, K)) return K;
+  aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
+  return fp8 && aq::huge_fp8_ok(a, aq::device_cus()) ? K : (K + 127) / 128 * 128;
 }

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(W * 64) void gemm_slices_kernel(GemmArgs p) {
     asm volatile("" ::: "memory");
   }
 
-  const __amdgpu_buffer_rsrc_t Ar = make_rsrc(p.A + (int64_t)m0 * K, (uint32_t)(M - m0 < BM ? M - m0 : BM) * (uint32_t)K);
+  const __amdgpu_buffer_rsrc_t Ar = make_rsrc(p.A + (int64_t)m0 * p.lda, (uint32_t)(M - m0 < BM ? M - m0 : BM) * (uint32_t)p.lda);
   const __amdgpu_buffer_rsrc_t Br = make_rsrc(p.B + (int64_t)n0 * K, (uint32_t)(N - n0 < BN ? N - n0 : BN) * (uint32_t)K);
   const int steps = (K + BK - 1) / BK;
   uint8_t* const mine = smem + wave * S::WAVE_LDS;
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(W * 64) void gemm_slices_kernel(GemmArgs p) {
       const int ia = i < A_LOADS ? i : i - A_LOADS;
       const int row = ia * RPG + lane / PPR;
       const int k = k0 + ((lane % PPR) ^ (row / RPL % PPR)) * 16;
-      const uint32_t off = k < K ? (uint32_t)row * (uint32_t)K + (uint32_t)k : OOB_OFFSET;  // past K (or the last step): zeros
+      const uint32_t off = k < K ? (uint32_t)row * (uint32_t)(i < A_LOADS ? p.lda : K) + (uint32_t)k : OOB_OFFSET;  // past K (or the last step): zeros
       __builtin_amdgcn_raw_ptr_buffer_load_lds(i < A_LOADS ? Ar : Br, (lds_void*)(mine + buf * S::STAGE + i * 1024), 16, off, 0, 0, 0);
     }
   };

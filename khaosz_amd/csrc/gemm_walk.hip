@@ -58,7 +58,7 @@ __device__ __forceinline__ void walk(const WalkArgs& w, uint8_t* smem, int pid, 
   const int wave_m = wave / 2, wave_n = wave % 2;
   const int M = p.M, N = p.N, K = p.K, nk = (K + BK - 1) / BK;
   const int col = lane & 31, rq = (lane >> 5) * 4;
-  const __amdgpu_buffer_rsrc_t Ar = make_rsrc(p.A, (uint32_t)M * (uint32_t)K), Br = make_rsrc(p.B, (uint32_t)N * (uint32_t)K);
+  const __amdgpu_buffer_rsrc_t Ar = make_rsrc(p.A, (uint32_t)M * (uint32_t)p.lda), Br = make_rsrc(p.B, (uint32_t)N * (uint32_t)K);
 
   // A load instruction of a wavefront fills 1 KiB = 8 tile rows; wavefront w owns the row groups w, w + 8, ... of A and B.
   // The 16-byte pieces of a row are permuted as in gemm_kernel: piece c of row r at slot c ^ (r / 2 % 8).
@@ -89,7 +89,7 @@ __device__ __forceinline__ void walk(const WalkArgs& w, uint8_t* smem, int pid, 
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i) {
       const int r = at.m0 + ld_row + 64 * i;
-      vo[i] = (uint32_t)(r < M ? r : M - 1) * (uint32_t)K + (uint32_t)ld_piece;
+      vo[i] = (uint32_t)(r < M ? r : M - 1) * (uint32_t)p.lda + (uint32_t)ld_piece;
     }
 #pragma unroll
     for (int i = 0; i < B_LOADS; ++i) {
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(WalkArgs w) {
 // Four K steps at least (one to begin a tile's loop, two that request the next tile's stages), pairs of columns, operands within
 // a 32-bit offset.  (Which tile, and whether this kernel at all: choose_tile_for.)
 bool gemm_walk_ok(const GemmArgs& a, int out) {
-  if (a.K < 512 || a.N % 2 || (int64_t)a.M * a.K > (int64_t)OOB_OFFSET || (int64_t)a.N * a.K > (int64_t)OOB_OFFSET) return false;
+  if (a.K < 512 || a.N % 2 || (int64_t)a.M * a.lda > (int64_t)OOB_OFFSET || (int64_t)a.N * a.K > (int64_t)OOB_OFFSET) return false;
   return out == OUT_BF16 || !a.res;
 }
 

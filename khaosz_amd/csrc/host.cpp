@@ -42,6 +42,11 @@ namespace {
   X(aq_gemv_w8a8_workspace_bytes)                                                                                \
   X(aq_gemv_w8a8_decode_one_launch)                                                                              \
   X(aq_gemv_fp8_decode_one_launch)                                                                               \
+  X(aq_linear_codes_pitch)                                                                                       \
+  X(aq_quant_rowwise_i8_strided)                                                                                 \
+  X(aq_quant_tensor_fp8_strided)                                                                                 \
+  X(aq_linear_w8a8_strided)                                                                                      \
+  X(aq_linear_fp8_strided)                                                                                       \
   X(aq_linear_few_rows_ok)                                                                                       \
   X(aq_linear_few_rows)                                                                                          \
   X(aq_gemv_w8a8_decode_residual)                                                                                \
@@ -617,8 +622,9 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   c10::DimVector shape(x->sizes());
   shape.back() = N;
   Tensor y = c.empty(shape, type);
-  // codes and scales of the tokens (and, for FP8, the partial maxima)
-  const int64_t codes = !few  ? (r.M * r.K + 255) & ~int64_t(255)
+  // codes and scales of the tokens (and, for FP8, the partial maxima); the codes of a tile's rows begin on lines
+  const int64_t pitch = few || gain ? r.K : lib.aq_linear_codes_pitch(fp8, r.M, N, r.K);
+  const int64_t codes = !few  ? (r.M * pitch + 255) & ~int64_t(255)
                         : fp8 ? static_cast<int64_t>(lib.aq_gemv_fp8_workspace_bytes(r.M, r.K))
                               : static_cast<int64_t>(lib.aq_gemv_w8a8_workspace_bytes(r.M, r.K));
   const int64_t room = codes + (!few ? (fp8 ? 256 + AQ_FP8_AMAX_WS_BYTES : 4 * r.M) : 0);
@@ -653,18 +659,24 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
     if (fp8) {
       auto* q = reinterpret_cast<uint8_t*>(base);
       what = "aq_quant_tensor_fp8";
-      if (int e = lib.aq_quant_tensor_fp8(r.p, r.code, x->numel(), q, sx, reinterpret_cast<uint32_t*>(base + codes + 256),
-                                          AQ_FP8_AMAX_WS_BYTES, c.stream))
+      auto* maxima = reinterpret_cast<uint32_t*>(base + codes + 256);
+      if (int e = pitch != r.K ? lib.aq_quant_tensor_fp8_strided(r.p, r.code, r.M, r.K, q, pitch, sx, maxima, AQ_FP8_AMAX_WS_BYTES, c.stream)
+                               : lib.aq_quant_tensor_fp8(r.p, r.code, x->numel(), q, sx, maxima, AQ_FP8_AMAX_WS_BYTES, c.stream))
         return e;
       what = "aq_linear_fp8";
+      if (pitch != r.K)
+        return lib.aq_linear_fp8_strided(q, pitch, sx, static_cast<const uint8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
       return lib.aq_linear_fp8_residual(q, sx, static_cast<const uint8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
     }
     auto* q = reinterpret_cast<int8_t*>(base);
     what = gain ? "aq_rmsnorm_quant_rowwise_i8" : "aq_quant_rowwise_i8";
-    if (int e = gain ? lib.aq_rmsnorm_quant_rowwise_i8(r.p, r.code, gain, r.code, eps, r.M, r.K, r.K, q, sx, c.stream)
-                     : lib.aq_quant_rowwise_i8(r.p, r.code, r.M, r.K, r.K, q, sx, c.stream))
+    if (int e = gain           ? lib.aq_rmsnorm_quant_rowwise_i8(r.p, r.code, gain, r.code, eps, r.M, r.K, r.K, q, sx, c.stream)
+                : pitch != r.K ? lib.aq_quant_rowwise_i8_strided(r.p, r.code, r.M, r.K, r.K, q, pitch, sx, c.stream)
+                               : lib.aq_quant_rowwise_i8(r.p, r.code, r.M, r.K, r.K, q, sx, c.stream))
       return e;
     what = "aq_linear_w8a8";
+    if (pitch != r.K)
+      return lib.aq_linear_w8a8_strided(q, pitch, sx, static_cast<const int8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
     return lib.aq_linear_w8a8_residual(q, sx, static_cast<const int8_t*>(wp), sp, b.p, b.code, res, yp, r.code, r.M, N, r.K, c.stream);
   });
   return rc ? fail(rc, what) : THPVariable_Wrap(y);

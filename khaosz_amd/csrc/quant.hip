@@ -36,7 +36,7 @@ __device__ __forceinline__ void quant_store(const uint4& v, float s, float rs, b
 template <bool BF16, int NC, bool PREFETCH, bool FULL>
 __global__ __launch_bounds__(256) void quant_rowwise_i8_kernel(const void* __restrict__ x, int64_t M,
                                                                  int K, int64_t ldx,
-                                                                 int8_t* __restrict__ q,
+                                                                 int8_t* __restrict__ q, int64_t ldq,
                                                                  float* __restrict__ scale) {
   constexpr int EPV = RowIn<BF16>::EPV;
   const int lane = threadIdx.x & 63;
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void quant_rowwise_i8_kernel(const void* __res
   };
   auto process = [&](int64_t r, const uint4 (&c)[NC]) {
     const uint4* src = row_src(r);
-    int8_t* dst = q + r * (int64_t)K;
+    int8_t* dst = q + r * ldq;
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) void quant_rowwise_i8_kernel(const void* __res
 // bounds a launch whose rows are all requested at once.
 template <bool BF16, int NV>
 __global__ __launch_bounds__(256) void quant_row_wg_kernel(const void* __restrict__ x, int K, int64_t ldx,
-                                                            int8_t* __restrict__ q, float* __restrict__ scale) {
+                                                            int8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale) {
   constexpr int EPV = RowIn<BF16>::EPV;
   __shared__ float wmax[4];
   const int tid = threadIdx.x;
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void quant_row_wg_kernel(const void* __restric
   const int nvec = K / EPV;
   const uint4* src =
       reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(x) + row * ldx * (BF16 ? 2 : 4));
-  int8_t* dst = q + row * (int64_t)K;
+  int8_t* dst = q + row * ldq;
   uint4 c[NV];
   float amax = 0.0f;
 #pragma unroll
@@ -616,10 +616,20 @@ __device__ __forceinline__ void fp8_prescale(float* f, float s, float rs, bool l
   }
 }
 
+// Where the codes of vector v go: one after another, or to rows `gap` bytes apart behind their ends (fewer than 2^31 vectors then).
+struct CodeRows {
+  UDiv by_row;  // vectors of a row
+  int64_t gap;
+  template <int EPV>
+  __device__ __forceinline__ int64_t at(int64_t v) const {
+    return v * EPV + (gap ? (int64_t)by_row((uint32_t)v) * gap : 0);  // uniform
+  }
+};
+
 template <bool BF16>
 __global__ __launch_bounds__(256) void cast_fp8_kernel(const void* __restrict__ x, int64_t nvec,
                                                         const uint32_t* __restrict__ amax_slots,
-                                                        uint8_t* __restrict__ q,
+                                                        uint8_t* __restrict__ q, CodeRows rows,
                                                         float* __restrict__ scale) {
   constexpr int EPV = RowIn<BF16>::EPV;
   // Pass 2 starts by combining the partial maxima: one slot per thread (1 KiB, served by the L2), a
@@ -664,9 +674,9 @@ __global__ __launch_bounds__(256) void cast_fp8_kernel(const void* __restrict__ 
         uint2 o;
         o.x = (uint32_t)w0;
         o.y = (uint32_t)w1;
-        store_wt(reinterpret_cast<uint2*>(q + v * EPV), o);
+        store_wt(reinterpret_cast<uint2*>(q + rows.at<EPV>(v)), o);
       } else {
-        store_wt(reinterpret_cast<uint32_t*>(q + v * EPV), (uint32_t)w0);
+        store_wt(reinterpret_cast<uint32_t*>(q + rows.at<EPV>(v)), (uint32_t)w0);
       }
     }
   }
@@ -692,7 +702,7 @@ constexpr int ONEPASS_R = 8;
 template <bool BF16>
 __global__ __launch_bounds__(ONEPASS_THREADS) void quant_fp8_onepass_kernel(const void* __restrict__ x, int64_t nvec,
                                                                             unsigned long long* __restrict__ slots,
-                                                                            uint8_t* __restrict__ q,
+                                                                            uint8_t* __restrict__ q, CodeRows rows,
                                                                             float* __restrict__ scale, int spin_limit) {
   constexpr int EPV = RowIn<BF16>::EPV;
   constexpr int NW = ONEPASS_THREADS / 64;
@@ -789,9 +799,9 @@ __global__ __launch_bounds__(ONEPASS_THREADS) void quant_fp8_onepass_kernel(cons
       uint2 o;
       o.x = (uint32_t)w0;
       o.y = (uint32_t)w1;
-      store_wt(reinterpret_cast<uint2*>(q + i * EPV), o);
+      store_wt(reinterpret_cast<uint2*>(q + rows.at<EPV>(i)), o);
     } else {
-      store_wt(reinterpret_cast<uint32_t*>(q + i * EPV), (uint32_t)w0);
+      store_wt(reinterpret_cast<uint32_t*>(q + rows.at<EPV>(i)), (uint32_t)w0);
     }
   };
 #pragma unroll
@@ -806,10 +816,11 @@ __global__ __launch_bounds__(ONEPASS_THREADS) void quant_fp8_onepass_kernel(cons
 
 // ------------------------------------------------------------------- C ABI
 
-extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
-                                   int8_t* q, float* scale, void* stream) {
+// Codes go to rows ldq apart.
+extern "C" int aq_quant_rowwise_i8_strided(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, int8_t* q, int64_t ldq,
+                                           float* scale, void* stream) {
   if (x_dtype != AQ_F32 && x_dtype != AQ_BF16) return AQ_E_DTYPE;
-  if (M < 0 || K < 0 || (K % 16) != 0 || ldx < K) return AQ_E_SHAPE;
+  if (M < 0 || K < 0 || (K % 16) != 0 || ldx < K || ldq < K) return AQ_E_SHAPE;
   if (M == 0 || K == 0) {
     // K == 0: amax of an empty row is 0, so every scale is 1; nothing to do for codes.
     if (K == 0 && M > 0) return AQ_E_SHAPE;
@@ -818,7 +829,7 @@ extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_
   if (!x || !q || !scale) return AQ_E_NULL;
   if (K > (int64_t)1 << 30 || M > (int64_t)1 << 31) return AQ_E_RANGE;
   const int esz = x_dtype == AQ_BF16 ? 2 : 4;
-  if (aq::check_ptr16(x) || aq::check_ptr16(q) || ((ldx * esz) & 15)) return AQ_E_ALIGN;
+  if (aq::check_ptr16(x) || aq::check_ptr16(q) || ((ldx * esz) & 15) || (ldq & 15)) return AQ_E_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Rows that fit 4 cached vectors per lane (2048 bf16 / 1024 fp32) take the
   // double-buffered kernel; with enough rows each wavefront gets two of them so
@@ -835,22 +846,22 @@ extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_
     const unsigned g = (unsigned)M;
     if (x_dtype == AQ_BF16) {
       if (nvec <= 256)
-        aq::queue_kernel((aq::quant_row_wg_kernel<true, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
       else if (nvec <= 512)
-        aq::queue_kernel((aq::quant_row_wg_kernel<true, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
       else if (nvec <= 1024)
-        aq::queue_kernel((aq::quant_row_wg_kernel<true, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
       else
-        aq::queue_kernel((aq::quant_row_wg_kernel<true, 8>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<true, 8>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
     } else {
       if (nvec <= 256)
-        aq::queue_kernel((aq::quant_row_wg_kernel<false, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 1>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
       else if (nvec <= 512)
-        aq::queue_kernel((aq::quant_row_wg_kernel<false, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 2>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
       else if (nvec <= 1024)
-        aq::queue_kernel((aq::quant_row_wg_kernel<false, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 4>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
       else
-        aq::queue_kernel((aq::quant_row_wg_kernel<false, 8>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, scale);
+        aq::queue_kernel((aq::quant_row_wg_kernel<false, 8>), dim3(g), dim3(256), 0, st, x, (int)K, ldx, q, ldq, scale);
     }
     return (int)hipGetLastError();
   }
@@ -862,25 +873,29 @@ extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_
   if (x_dtype == AQ_BF16) {
     if (full_row)
       aq::queue_kernel((aq::quant_rowwise_i8_kernel<true, 4, true, true>), dim3(grid), dim3(256), 0, st, x, M,
-                         (int)K, ldx, q, scale);
+                         (int)K, ldx, q, ldq, scale);
     else if (small_row)
       aq::queue_kernel((aq::quant_rowwise_i8_kernel<true, 4, true, false>), dim3(grid), dim3(256), 0, st, x, M,
-                         (int)K, ldx, q, scale);
+                         (int)K, ldx, q, ldq, scale);
     else
       aq::queue_kernel((aq::quant_rowwise_i8_kernel<true, 16, false, false>), dim3(grid), dim3(256), 0, st, x,
-                         M, (int)K, ldx, q, scale);
+                         M, (int)K, ldx, q, ldq, scale);
   } else {
     if (full_row)
       aq::queue_kernel((aq::quant_rowwise_i8_kernel<false, 4, true, true>), dim3(grid), dim3(256), 0, st, x, M,
-                         (int)K, ldx, q, scale);
+                         (int)K, ldx, q, ldq, scale);
     else if (small_row)
       aq::queue_kernel((aq::quant_rowwise_i8_kernel<false, 4, true, false>), dim3(grid), dim3(256), 0, st, x, M,
-                         (int)K, ldx, q, scale);
+                         (int)K, ldx, q, ldq, scale);
     else
       aq::queue_kernel((aq::quant_rowwise_i8_kernel<false, 16, false, false>), dim3(grid), dim3(256), 0, st, x,
-                         M, (int)K, ldx, q, scale);
+                         M, (int)K, ldx, q, ldq, scale);
   }
   return (int)hipGetLastError();
+}
+
+extern "C" int aq_quant_rowwise_i8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, int8_t* q, float* scale, void* stream) {
+  return aq_quant_rowwise_i8_strided(x, x_dtype, M, K, ldx, q, K, scale, stream);
 }
 
 template <bool BF16>
@@ -987,8 +1002,20 @@ extern "C" int aq_swiglu_quant_rowwise_i8(const void* ug, int dtype, int64_t M, 
 
 // (not static: the lab library's hook in lab.hip calls it with its own bound on the wait)
 namespace aq {
+// codes one after another (K = 0), or in rows of K, ldq apart
+static int code_rows(int64_t numel, int64_t K, int64_t ldq, int epv, CodeRows* rows) {
+  *rows = CodeRows{};
+  if (K == 0 || ldq == K) return AQ_OK;
+  if (K < 0 || K % 16 || ldq < K || numel % K) return AQ_E_SHAPE;
+  if (ldq % 16) return AQ_E_ALIGN;
+  if (numel / epv > (int64_t)0x7fffffff || K > (1 << 30)) return AQ_E_RANGE;
+  rows->by_row = UDiv::of((uint32_t)(K / epv));
+  rows->gap = ldq - K;
+  return AQ_OK;
+}
+
 int quant_tensor_fp8_onepass(const void* x, int x_dtype, int64_t numel, uint8_t* q, float* scale, void* ws,
-                             size_t ws_bytes, int spin_limit, hipStream_t st) {
+                             size_t ws_bytes, int spin_limit, hipStream_t st, int64_t K, int64_t ldq) {
   if (x_dtype != AQ_F32 && x_dtype != AQ_BF16) return AQ_E_DTYPE;
   if (numel < 0 || (numel % 16) != 0) return AQ_E_SHAPE;
   if (!scale || !ws) return AQ_E_NULL;
@@ -997,15 +1024,17 @@ int quant_tensor_fp8_onepass(const void* x, int x_dtype, int64_t numel, uint8_t*
   if (aq::check_ptr16(x) || aq::check_ptr16(q) || aq::check_ptr(ws, 8) || aq::check_ptr(scale, 4)) return AQ_E_ALIGN;
   const int epv = x_dtype == AQ_BF16 ? 8 : 4;
   const int64_t nvec = numel / epv;
+  CodeRows rows;
+  if (const int rc = code_rows(numel, K, ldq, epv, &rows)) return rc;
   // one workgroup per compute unit, at most one per slot; always the same count on a device, whatever the size
   int g = aq::device_cus();
   if (g > AQ_FP8_ONEPASS_WS_BYTES / 8) g = AQ_FP8_ONEPASS_WS_BYTES / 8;
   if (x_dtype == AQ_BF16)
     aq::queue_kernel((aq::quant_fp8_onepass_kernel<true>), dim3((unsigned)g), dim3(aq::ONEPASS_THREADS), 0, st, x, nvec,
-                       static_cast<unsigned long long*>(ws), q, scale, spin_limit);
+                       static_cast<unsigned long long*>(ws), q, rows, scale, spin_limit);
   else
     aq::queue_kernel((aq::quant_fp8_onepass_kernel<false>), dim3((unsigned)g), dim3(aq::ONEPASS_THREADS), 0, st, x, nvec,
-                       static_cast<unsigned long long*>(ws), q, scale, spin_limit);
+                       static_cast<unsigned long long*>(ws), q, rows, scale, spin_limit);
   return (int)hipGetLastError();
 }
 }  // namespace aq
@@ -1013,11 +1042,17 @@ int quant_tensor_fp8_onepass(const void* x, int x_dtype, int64_t numel, uint8_t*
 extern "C" int aq_quant_tensor_fp8_onepass(const void* x, int x_dtype, int64_t numel, uint8_t* q, float* scale,
                                            void* ws, size_t ws_bytes, void* stream) {
   // 4096 polls of a few hundred nanoseconds each: a millisecond or two before a workgroup stops waiting
-  return aq::quant_tensor_fp8_onepass(x, x_dtype, numel, q, scale, ws, ws_bytes, 4096, static_cast<hipStream_t>(stream));
+  return aq::quant_tensor_fp8_onepass(x, x_dtype, numel, q, scale, ws, ws_bytes, 4096, static_cast<hipStream_t>(stream), 0, 0);
 }
 
-extern "C" int aq_quant_tensor_fp8(const void* x, int x_dtype, int64_t numel, uint8_t* q,
-                                   float* scale, uint32_t* amax_ws, size_t ws_bytes, void* stream) {
+extern "C" int aq_quant_tensor_fp8_onepass_strided(const void* x, int x_dtype, int64_t M, int64_t K, uint8_t* q, int64_t ldq, float* scale,
+                                                   void* ws, size_t ws_bytes, void* stream) {
+  if (M < 0 || K <= 0 || M > (1 << 30) || K > (1 << 30)) return AQ_E_SHAPE;
+  return aq::quant_tensor_fp8_onepass(x, x_dtype, M * K, q, scale, ws, ws_bytes, 4096, static_cast<hipStream_t>(stream), K, ldq);
+}
+
+static int quant_tensor_fp8(const void* x, int x_dtype, int64_t numel, uint8_t* q, float* scale, uint32_t* amax_ws, size_t ws_bytes,
+                            void* stream, int64_t K, int64_t ldq) {
   if (x_dtype != AQ_F32 && x_dtype != AQ_BF16) return AQ_E_DTYPE;
   if (numel < 0 || (numel % 16) != 0) return AQ_E_SHAPE;
   if (!scale || !amax_ws) return AQ_E_NULL;
@@ -1027,6 +1062,8 @@ extern "C" int aq_quant_tensor_fp8(const void* x, int x_dtype, int64_t numel, ui
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int epv = x_dtype == AQ_BF16 ? 8 : 4;
   const int64_t nvec = numel / epv;
+  aq::CodeRows rows;
+  if (const int rc = aq::code_rows(numel, K, ldq, epv, &rows)) return rc;
   int64_t blocks = (nvec + 255) / 256;
   if (blocks > 2048) blocks = 2048;  // 8 workgroups per CU, grid-stride beyond
   if (blocks < 1) blocks = 1;
@@ -1038,12 +1075,22 @@ extern "C" int aq_quant_tensor_fp8(const void* x, int x_dtype, int64_t numel, ui
   if (x_dtype == AQ_BF16) {
     aq::queue_kernel((aq::amax_kernel<true>), dim3((unsigned)ablocks), dim3(aq::AMAX_THREADS), 0, st, x, nvec, amax_ws);
     aq::queue_kernel((aq::cast_fp8_kernel<true>), dim3((unsigned)blocks), dim3(256), 0, st, x, nvec,
-                       amax_ws, q, scale);
+                       amax_ws, q, rows, scale);
   } else {
     aq::queue_kernel((aq::amax_kernel<false>), dim3((unsigned)ablocks), dim3(aq::AMAX_THREADS), 0, st, x, nvec, amax_ws);
     aq::queue_kernel((aq::cast_fp8_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, st, x, nvec,
-                       amax_ws, q, scale);
+                       amax_ws, q, rows, scale);
   }
   return (int)hipGetLastError();
 }
 
+extern "C" int aq_quant_tensor_fp8(const void* x, int x_dtype, int64_t numel, uint8_t* q, float* scale, uint32_t* amax_ws, size_t ws_bytes,
+                                   void* stream) {
+  return quant_tensor_fp8(x, x_dtype, numel, q, scale, amax_ws, ws_bytes, stream, 0, 0);
+}
+
+extern "C" int aq_quant_tensor_fp8_strided(const void* x, int x_dtype, int64_t M, int64_t K, uint8_t* q, int64_t ldq, float* scale,
+                                           uint32_t* amax_ws, size_t ws_bytes, void* stream) {
+  if (M < 0 || K <= 0 || M > (1 << 30) || K > (1 << 30)) return AQ_E_SHAPE;
+  return quant_tensor_fp8(x, x_dtype, M * K, q, scale, amax_ws, ws_bytes, stream, K, ldq);
+}

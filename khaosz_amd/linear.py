@@ -376,11 +376,14 @@ class Fp8Linear(_NativeCall):
         if x2.size(0) <= self.DECODE_MAX_ROWS:  # decode step: the weight-streaming GEMV
             y = ops.gemv_fp8_decode(x2, wq, sw, bias, out_dtype=x.dtype, residual=residual)
         else:
-            state = None
+            state, rows = None, {}
             if x2.numel() * x2.element_size() >= ops.FP8_ONEPASS_MIN_BYTES:  # quantised in one launch
                 ops._need_gpu(x, wq)
                 state = self._quant_states.get(x.device, lambda: ops.fp8_onepass_state(x.device))
-            xq, sx = ops.quant_tensor_fp8(x2, state=state)
+                pitch = ops.codes_pitch(x2.size(0), n, k, True)
+                if pitch != k:
+                    rows = {"pitch": pitch}
+            xq, sx = ops.quant_tensor_fp8(x2, state=state, **rows)
             y = ops.linear_fp8(xq, sx, wq, sw, bias, out_dtype=x.dtype, residual=residual)
         return y if x2 is x else y.view(x.shape[:-1] + (n,))
 

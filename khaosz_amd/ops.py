@@ -182,14 +182,22 @@ def fp8_onepass_state(device) -> torch.Tensor:
     return torch.zeros((_abi.AQ_FP8_ONEPASS_WS_BYTES // 8,), dtype=torch.int64, device=device)
 
 
+def codes_pitch(M: int, N: int, K: int, fp8: bool) -> int:
+    """Bytes between the rows of the codes that a Linear ``[M, K] -> [M, N]`` reads fastest: K, or the next multiple of 128."""
+    return _abi.load().aq_linear_codes_pitch(int(fp8), M, N, K)
+
+
 def quant_tensor_fp8(x: torch.Tensor, state: Optional[torch.Tensor] = None,
-                     onepass: Optional[bool] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+                     onepass: Optional[bool] = None, pitch: Optional[int] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """Per-tensor OCP e4m3fn -> (codes uint8 with x's shape, scale f32 [1]).
     ``state`` (from ``fp8_onepass_state``): allows the one-launch form, which reads x from HBM once instead of
-    twice -- same codes and scale; taken for tensors of ``FP8_ONEPASS_MIN_BYTES`` and more, or as ``onepass`` says."""
+    twice -- same codes and scale; taken for tensors of ``FP8_ONEPASS_MIN_BYTES`` and more, or as ``onepass`` says.
+    ``pitch`` (of a 2-D x, at least its row length and a multiple of 16): the codes' rows begin that many bytes apart."""
     if onepass is None:
         onepass = state is not None and x.numel() * x.element_size() >= FP8_ONEPASS_MIN_BYTES
-    if state is not None or not onepass:
+    if pitch is not None and x.dim() != 2:
+        raise ValueError("a pitch needs rows")
+    if (state is not None or not onepass) and pitch is None:
         r = (_host or _native()).quant_tensor_fp8(x, state if onepass else None)
         if r is not None:
             return r
@@ -198,8 +206,10 @@ def quant_tensor_fp8(x: torch.Tensor, state: Optional[torch.Tensor] = None,
     n = xc.numel()
     if n % 16:
         raise ValueError(f"numel must be a multiple of 16, got {n}")
-    q = torch.empty(xc.shape, dtype=torch.uint8, device=x.device)
+    q = torch.empty(xc.shape if pitch is None else (xc.shape[0], pitch), dtype=torch.uint8, device=x.device)
     s = torch.empty((1,), dtype=torch.float32, device=x.device)
+    lib, size = _abi.load(), (n,) if pitch is None else tuple(xc.shape)
+    to = (q.data_ptr(),) if pitch is None else (q.data_ptr(), pitch)
     if onepass:
         if state is None:
             raise ValueError("the one-launch form needs the state tensor of fp8_onepass_state()")
@@ -208,16 +218,16 @@ def quant_tensor_fp8(x: torch.Tensor, state: Optional[torch.Tensor] = None,
                 or state.device != x.device:
             raise ValueError("state must come from fp8_onepass_state() for x's device")
         with _OnDevice(x.device):
-            rc = _abi.load().aq_quant_tensor_fp8_onepass(xc.data_ptr(), _dt(xc, "x"), n, q.data_ptr(), s.data_ptr(),
-                                                         state.data_ptr(), state.numel() * 8, _stream(x))
+            f = lib.aq_quant_tensor_fp8_onepass if pitch is None else lib.aq_quant_tensor_fp8_onepass_strided
+            rc = f(xc.data_ptr(), _dt(xc, "x"), *size, *to, s.data_ptr(), state.data_ptr(), state.numel() * 8, _stream(x))
         _abi.check(rc, "aq_quant_tensor_fp8_onepass")
-        return q, s
+        return q if pitch is None else q[:, :xc.shape[1]], s
     ws = torch.empty((_abi.AQ_FP8_AMAX_WS_BYTES // 4,), dtype=torch.int32, device=x.device)  # partial maxima, stateless
     with _OnDevice(x.device):
-        rc = _abi.load().aq_quant_tensor_fp8(xc.data_ptr(), _dt(xc, "x"), n, q.data_ptr(), s.data_ptr(),
-                                             ws.data_ptr(), ws.numel() * 4, _stream(x))
+        f = lib.aq_quant_tensor_fp8 if pitch is None else lib.aq_quant_tensor_fp8_strided
+        rc = f(xc.data_ptr(), _dt(xc, "x"), *size, *to, s.data_ptr(), ws.data_ptr(), ws.numel() * 4, _stream(x))
     _abi.check(rc, "aq_quant_tensor_fp8")
-    return q, s
+    return q if pitch is None else q[:, :xc.shape[1]], s
 
 
 def gemm_i8_i32(xq: torch.Tensor, wq: torch.Tensor) -> torch.Tensor:
@@ -785,16 +795,18 @@ def linear_fp8(xq, sx, wq, sw, bias=None, out_dtype=torch.bfloat16, residual=Non
         raise ValueError("sx and sw must be float32 device scalars")
     if out_dtype not in _DT:
         raise ValueError(f"out_dtype {out_dtype} is not supported")
-    xq, wq = xq.contiguous(), wq.contiguous()
+    wq, ld = wq.contiguous(), xq.stride(0)
+    if xq.stride(1) != 1 or ld < K or ld % 16 or M < 2 or xq.data_ptr() % 16:
+        xq, ld = xq.contiguous(), K
     b, bdt = _bias_args(bias, N)
     r = _residual_arg(residual, M, N, out_dtype, xq.device)
     y = torch.empty((M, N), dtype=out_dtype, device=xq.device)
     if M and N:
         with _OnDevice(xq.device):
-            rc = _abi.load().aq_linear_fp8_residual(xq.data_ptr(), sx.data_ptr(), wq.data_ptr(), sw.data_ptr(),
-                                                    b.data_ptr() if b is not None else None, bdt,
-                                                    r.data_ptr() if r is not None else None, y.data_ptr(),
-                                                    _DT[out_dtype], M, N, K, _stream(xq))
+            rc = _abi.load().aq_linear_fp8_strided(xq.data_ptr(), ld, sx.data_ptr(), wq.data_ptr(), sw.data_ptr(),
+                                                   b.data_ptr() if b is not None else None, bdt,
+                                                   r.data_ptr() if r is not None else None, y.data_ptr(),
+                                                   _DT[out_dtype], M, N, K, _stream(xq))
         _abi.check(rc, "aq_linear_fp8")
     elif r is not None:
         y.copy_(r.view(M, N))
