@@ -81,6 +81,7 @@ struct Shape {
   static constexpr bool BIG = TM * TN >= 16;
   static constexpr int SX_BYTES = BIG ? BM * 4 : 0;
   static constexpr int LDS_BYTES = NSTAGE * STAGE + SX_BYTES;
+  static constexpr int LDS_LINES = NSTAGE * STAGE + BN * BK;  // with a stage more of B (see gemm_tile)
   static_assert(BK == 64 || BK == 128, "K bytes per stage");
   static_assert(NWAVES % 2 == 0, "the piece permutation assumes a wavefront's row groups share parity");
   static_assert((BM * BK / 1024) % NWAVES == 0 && (BN * BK / 1024) % NWAVES == 0, "whole 1 KiB loads per wavefront");
@@ -116,11 +117,16 @@ __device__ __forceinline__ void sched_pattern() {
 #ifdef AQ_LAB
 __device__ long long aq_lab_clock[16];
 #endif
-// EXACT: K is a whole number of BK-byte steps, so every 16-byte piece of every step lies inside its row and the
-// global->LDS loads need no per-lane range logic: a loop-invariant lane offset per row group and the K step as a
-// scalar offset, no vector ALU work per load.
-template <bool FP8, int OUT, class S, bool EXACT>
+// How the rows of A and B lie in 128-byte lines, K and the distance between A's rows being given:
+//   EXACT  K is a whole number of BK-byte steps and rows are K apart: every 16-byte piece of every step lies inside its row and the
+//          global->LDS loads need no per-lane range logic: a loop-invariant lane offset per row group and the K step as a scalar offset, no
+//          vector ALU work per load.
+//   ANY    K may end inside a step, and each load checks it.
+//   LINES  the same, and the loads of B are whole lines, wherever its rows begin (see `phase`); for long K.
+enum Rows { EXACT_ROWS, ANY_ROWS, LINE_ROWS };
+template <bool FP8, int OUT, class S, Rows ROWS>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int pid) {
+  constexpr bool EXACT = ROWS == EXACT_ROWS, LINES = ROWS == LINE_ROWS;
   constexpr int WM = S::WM, WN = S::WN, TM = S::TM, TN = S::TN, WK = S::WK, BK = S::BK, NSTAGE = S::NSTAGE;
   constexpr int NWAVES = S::NWAVES, NTHREADS = S::NTHREADS, WAVE_M = S::WAVE_M, WAVE_N = S::WAVE_N;
   constexpr int BM = S::BM, BN = S::BN, STAGE = S::STAGE;
@@ -180,24 +186,46 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   constexpr bool ADJ = TN == 2 && OUT == OUT_BF16;
   const bool pair_ok = (N & 1) == 0;  // uniform: bf16 rows start dword-aligned, pairs never straddle N
   uint32_t ld_vo[A_LOADS > B_LOADS ? A_LOADS : B_LOADS];  // lane offset of row group i; EXACT: A and B alike
-  uint32_t ld_va[EXACT ? 1 : A_LOADS];                     // not EXACT: of A, whose rows may be further apart
-  uint32_t ld_vb[ADJ ? B_LOADS : 1];                       // ... of B, where its rows have an order of their own
+  uint32_t ld_vb[ADJ || !EXACT ? B_LOADS : 1];             // ... of B, where its rows have an order or a distance of their own
+  // row of the tile of B that row r of a stage holds
+  auto b_row = [&](int r) { return ADJ && pair_ok ? (r & ~63) + 2 * (r & 31) + ((r >> 5) & 1) : r; };
+  // LINES: rows of B begin anywhere in a line, `phase` bytes behind its beginning (A's rows the caller lays out: lda).  A stage of B holds a
+  // line of every row: line t has bytes BK t - phase .. + BK of the row, piece q of a step (of the row's own bytes) in piece q's place of line
+  // s, or of line s + 1 where 16 q + phase is past the line's end.  Step s takes pieces of both, so one stage more of B is kept, and a load
+  // brings one line of each row where a step of the row's own bytes would touch two.
+  auto phase = [&](int row) { return (int)((reinterpret_cast<uintptr_t>(p.B) + (uint64_t)(uint32_t)(n0 + row) * (uint32_t)K) & (BK - 1)); };
+  // Byte of the row that this lane's piece of line 0 begins at.  Rows 8 apart have one phase, so it is the same for every row group (ADJ: for
+  // every other one).
+  constexpr int NKB = ADJ ? 2 : 1;
+  int ld_kb[LINES ? NKB : 1];
+  if constexpr (EXACT) {
 #pragma unroll
-  for (int i = 0; i < (A_LOADS > B_LOADS ? A_LOADS : B_LOADS); ++i) ld_vo[i] = ld_off + (uint32_t)i * row32;
-  if constexpr (!EXACT) {
+    for (int i = 0; i < (A_LOADS > B_LOADS ? A_LOADS : B_LOADS); ++i) ld_vo[i] = ld_off + (uint32_t)i * row32;
+    if constexpr (ADJ) {
 #pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) ld_va[i] = (uint32_t)(ld_row + i * RPG * NWAVES) * (uint32_t)p.lda + ld_piece;
-  }
-  if constexpr (ADJ) {
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i) {
-      const int r = ld_row + i * RPG * NWAVES, own = (r & ~63) + 2 * (r & 31) + ((r >> 5) & 1);
-      ld_vb[i] = (uint32_t)(pair_ok ? own : r) * (uint32_t)K + ld_piece;
+      for (int i = 0; i < B_LOADS; ++i) ld_vb[i] = (uint32_t)b_row(ld_row + i * RPG * NWAVES) * (uint32_t)K + ld_piece;
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i) ld_vo[i] = (uint32_t)(ld_row + i * RPG * NWAVES) * (uint32_t)p.lda + ld_piece;
+    if constexpr (LINES) {
+#pragma unroll
+      for (int i = 0; i < NKB; ++i) {
+        const int ph = phase(b_row(ld_row + i * RPG * NWAVES));
+        ld_kb[i] = ld_piece + ph < BK ? ld_piece : ld_piece - BK;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < B_LOADS; ++i)
+      ld_vb[i] = (uint32_t)b_row(ld_row + i * RPG * NWAVES) * (uint32_t)K + (uint32_t)(LINES ? ld_kb[LINES ? i % NKB : 0] + BK : ld_piece);
   }
-  auto b_off = [&](int i) { return ADJ ? ld_vb[ADJ ? i : 0] : ld_vo[i]; };
-  // load number `idx` (0..NLOADS-1) of K step kt into stage buffer `buf`
-  auto issue_load = [&](int kt, int buf, int idx) {
+  auto b_off = [&](int i) { return ADJ || !EXACT ? ld_vb[ADJ || !EXACT ? i : 0] : ld_vo[i]; };
+  constexpr int A_STAGE = LINES ? BM * BK : STAGE;                                  // bytes between stages of A
+  constexpr int B_FIRST = NSTAGE * A_STAGE, B_LAST = B_FIRST + NSTAGE * (BN * BK);  // LINES: B's have a ring of their own, of NSTAGE + 1
+  auto behind = [](int at) { return at == B_LAST ? B_FIRST : at + BN * BK; };
+  int b_ld = B_FIRST;  // LINES: where the line of B goes that issue_load requests
+  // load number `idx` (0..NLOADS-1) of K step kt into stage buffer `buf`; LINES: of A, and of line kt + 1 of B
+  auto issue_load = [&](int kt, int buf, int idx, auto kind) {
     if constexpr (EXACT) {
       // steps past the last one request the last step again (into a stage nobody reads): in range by construction
       const int k0s = (kt < nk ? kt : nk - 1) * BK;  // wavefront-uniform: a scalar offset
@@ -209,17 +237,30 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
                                                  b_off(idx - A_LOADS), k0s, 0, 0);
       return;
     }
-    const int k0 = kt * BK;
-    // K is a multiple of 16: a piece is all in or all out.  Pieces past K would
-    // alias the next row, so they are pushed outside the descriptor (-> zeros).
-    const bool in = k0 + ld_piece < K;
-    uint8_t* st = smem + buf * STAGE + wave * 1024;
-    if (idx < A_LOADS)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(Ar, (lds_void*)(st + idx * (1024 * NWAVES)), 16,
-                                               in ? ld_va[EXACT ? 0 : idx] + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
-    else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(Br, (lds_void*)(st + BM * BK + (idx - A_LOADS) * (1024 * NWAVES)), 16,
-                                               in ? b_off(idx - A_LOADS) + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
+    // K is a multiple of 16: a piece is all in or all out.  Pieces past K would alias the next row, so they are pushed outside the
+    // descriptor (-> zeros); so are all of the steps past the last one.
+    uint8_t* sta = smem + buf * A_STAGE + wave * 1024;
+    uint8_t* stb = (LINES ? smem + b_ld : smem + buf * STAGE + BM * BK) + wave * 1024;
+    if constexpr (!LINES) {
+      const int k0 = kt * BK;
+      const bool in = k0 + ld_piece < K;
+      if (idx < A_LOADS)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(Ar, (lds_void*)(sta + idx * (1024 * NWAVES)), 16, in ? ld_vo[idx] + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(Br, (lds_void*)(stb + (idx - A_LOADS) * (1024 * NWAVES)), 16,
+                                                 in ? b_off(idx - A_LOADS) + (uint32_t)k0 : OOB_OFFSET, 0, 0, 0);
+    } else {
+      // most steps need no check (a compare and a select in each load are 10 % of an int8 launch of 64 x 64 tiles)
+      constexpr bool WHOLE = decltype(kind)::value == 2;      // nothing of the step or of the line is past K
+      const int k0s = (WHOLE || kt < nk ? kt : nk - 1) * BK;  // less than the bytes behind the descriptor
+      const int i = idx - A_LOADS;
+      if (idx < A_LOADS)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(Ar, (lds_void*)(sta + idx * (1024 * NWAVES)), 16,
+                                                 WHOLE || kt * BK + ld_piece < K ? ld_vo[idx] : OOB_OFFSET, k0s, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(Br, (lds_void*)(stb + i * (1024 * NWAVES)), 16,
+                                                 WHOLE || kt * BK + BK + ld_kb[LINES ? i % NKB : 0] < K ? b_off(i) : OOB_OFFSET, k0s, 0, 0);
+    }
   };
 
 #ifdef AQ_LAB_STALL
@@ -247,13 +288,41 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   // of two, so adding the sub-step number to that base is an XOR and folds into the permutation
   const int swz = (FP8 ? ((((lane >> 5) * 2) ^ fsw) << 4) : (((lane >> 5) ^ fsw) << 4)) ^ (wave_k * NKS * KSUB);
   using frag_t = typename Frag<FP8>::type;
+  // LINES: pieces of a step from this byte on lie in the line behind, by accumulator column where those are rows of two phases (ADJ)
+  constexpr int PP = FP8 ? 2 : 1, NJ = ADJ ? TN : 1;  // 16-byte pieces of a lane's fragment
+  int fb_end[LINES ? NJ : 1];
+  if constexpr (LINES) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      fb_end[j] = BK - phase(b_row(wave_n * WAVE_N + j * 32 + (lane & 31))) - wave_k * NKS * KSUB - (lane >> 5) * PP * 16;
+  }
+  int line_cur = 0;  // LINES: offset of the line of B that belongs to the stage whose fragments are read, and of the one behind
+  int line_next = 0;
+  auto read_b = [&](int ks, int j) -> frag_t {
+    auto piece = [&](int pp) {
+      const int o = ((ks * 2 * PP) << 4 ^ swz ^ pp << 4) + fr_b - BM * BK + j * 32 * BK;
+      return *reinterpret_cast<const v4i*>(smem + o + (ks * KSUB + pp * 16 >= fb_end[ADJ && LINES ? j : 0] ? line_next : line_cur));
+    };
+    if constexpr (!FP8) {
+      return piece(0);
+    } else {
+      const v4i lo = piece(0), hi = piece(1);
+      return v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    }
+  };
   auto load_frags = [&](const uint8_t* st, int ks, frag_t (&a)[TM], frag_t (&b)[TN]) {
+    if constexpr (LINES) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[j] = read_b(ks, j);
+    }
     if constexpr (!FP8) {
       const int o = ((ks * 2) << 4) ^ swz;
 #pragma unroll
       for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const v4i*>(st + fr_a + i * 32 * BK + o);
+      if constexpr (!LINES) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) b[j] = *reinterpret_cast<const v4i*>(st + fr_b + j * 32 * BK + o);
+        for (int j = 0; j < TN; ++j) b[j] = *reinterpret_cast<const v4i*>(st + fr_b + j * 32 * BK + o);
+      }
     } else {
       const int o0 = ((ks * 4) << 4) ^ swz, o1 = o0 ^ 16;
 #pragma unroll
@@ -262,11 +331,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
         const v4i hi = *reinterpret_cast<const v4i*>(st + fr_a + i * 32 * BK + o1);
         a[i] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       }
+      if constexpr (!LINES) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const v4i lo = *reinterpret_cast<const v4i*>(st + fr_b + j * 32 * BK + o0);
-        const v4i hi = *reinterpret_cast<const v4i*>(st + fr_b + j * 32 * BK + o1);
-        b[j] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        for (int j = 0; j < TN; ++j) {
+          const v4i lo = *reinterpret_cast<const v4i*>(st + fr_b + j * 32 * BK + o0);
+          const v4i hi = *reinterpret_cast<const v4i*>(st + fr_b + j * 32 * BK + o1);
+          b[j] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        }
       }
     }
   };
@@ -281,6 +352,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   auto load_frag = [&](const uint8_t* st, int ks, int f, frag_t (&a)[TM], frag_t (&b)[TN]) {
     const bool is_a = f == 0 || f > TN;
     const int idx = f == 0 ? 0 : f <= TN ? f - 1 : f - TN;
+    if (LINES && !is_a) {
+      b[idx] = read_b(ks, idx);
+      return;
+    }
     const uint8_t* base = st + (is_a ? fr_a : fr_b) + idx * 32 * BK;
     if constexpr (!FP8) {
       const v4i v = *reinterpret_cast<const v4i*>(base + (((ks * 2) << 4) ^ swz));
@@ -301,7 +376,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   auto slot = [&](auto cur_c, const uint8_t* st_next, int ks_next, auto loads_c, int kt_ld, int buf_ld,
                   auto q_c) {
     constexpr int CUR = decltype(cur_c)::value;
-    constexpr bool LOADS = decltype(loads_c)::value;
+    constexpr bool LOADS = decltype(loads_c)::value != 0;
     constexpr int Q = decltype(q_c)::value;
     constexpr int LD0 = (Q * NLOADS) / NKS, LPS = LOADS ? ((Q + 1) * NLOADS) / NKS - LD0 : 0;
     constexpr int NMMA = TM * TN, NFR = TM + TN;
@@ -320,7 +395,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
           if (2 * (m / STRIDE) + 1 < NFR) load_frag(st_next, ks_next, 2 * (m / STRIDE) + 1, af[CUR ^ 1], bf[CUR ^ 1]);
         } else if (m % STRIDE == 1 && m / STRIDE < NPAIR) {
 #pragma unroll
-          for (int q = ((m / STRIDE) * LPS) / NPAIR; q < ((m / STRIDE + 1) * LPS) / NPAIR; ++q) issue_load(kt_ld, buf_ld, LD0 + q);
+          for (int q = ((m / STRIDE) * LPS) / NPAIR; q < ((m / STRIDE + 1) * LPS) / NPAIR; ++q) issue_load(kt_ld, buf_ld, LD0 + q, loads_c);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -333,7 +408,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
 #pragma unroll
         for (int f = (m * NFR) / GROUPS; f < ((m + 1) * NFR) / GROUPS; ++f) load_frag(st_next, ks_next, f, af[CUR ^ 1], bf[CUR ^ 1]);
 #pragma unroll
-        for (int q = (m * LPS) / GROUPS; q < ((m + 1) * LPS) / GROUPS; ++q) issue_load(kt_ld, buf_ld, LD0 + q);
+        for (int q = (m * LPS) / GROUPS; q < ((m + 1) * LPS) / GROUPS; ++q) issue_load(kt_ld, buf_ld, LD0 + q, loads_c);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -345,8 +420,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   using q1 = integral_constant<int, 1>;
   using q2 = integral_constant<int, 2>;
   using q3 = integral_constant<int, 3>;
-  using yes = integral_constant<bool, true>;
-  using no = integral_constant<bool, false>;
+  using no = integral_constant<int, 0>;
+  using yes = integral_constant<int, 1>;
+  using whole = integral_constant<int, 2>;
 
   // Rotated software pipeline over K steps ("stages" s = 0 .. nk-1):
   //   iteration s:  slots    MFMAs of (s, 0 .. NKS-2)       | read fragments (s, 1 .. NKS-1)
@@ -430,15 +506,24 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
       }
     }
   };
+  if constexpr (LINES) {
 #pragma unroll
-  for (int q = 0; q < NLOADS; ++q) issue_load(0, 0, q);
+    for (int i = 0; i < B_LOADS; ++i)  // line 0: bytes before the row are never read
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(Br, (lds_void*)(smem + b_ld + wave * 1024 + i * (1024 * NWAVES)), 16,
+                                               (uint32_t)ld_kb[LINES ? i % NKB : 0] < (uint32_t)K ? b_off(i) - BK : OOB_OFFSET, 0, 0, 0);
+    b_ld = behind(b_ld);
+  }
+#pragma unroll
+  for (int q = 0; q < NLOADS; ++q) issue_load(0, 0, q, yes{});
   asm volatile("" ::: "memory");  // keep the request order: stage 0, epilogue operands, the other stages
   load_epilogue_operands();
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int st = 1; st < NSTAGE; ++st)
+  for (int st = 1; st < NSTAGE; ++st) {
+    b_ld = behind(b_ld);
 #pragma unroll
-    for (int q = 0; q < NLOADS; ++q) issue_load(st, st, q);
+    for (int q = 0; q < NLOADS; ++q) issue_load(st, st, q, yes{});
+  }
 
   // sub-steps 0 .. NKS-2 of a stage whose first fragments sit in af[C0]
   auto middle_slots = [&](auto c0_c, const uint8_t* stc, auto loads_c, int kt_ld, int buf_ld) {
@@ -461,23 +546,29 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
 #ifdef AQ_LAB_STALL
   const long long tl_stage0 = clock64();
 #endif
+  b_ld = line_cur = B_FIRST;  // the loop's loads of B go where the line was that the step before took first
+  line_next = behind(line_cur);
+  auto next_lines = [&] {
+    if constexpr (LINES) b_ld = line_cur, line_cur = line_next, line_next = behind(line_next);
+  };
   load_frags(smem, 0, af[0], bf[0]);
   middle_slots(k0{}, smem, no{}, 0, 0);  // no loads to issue yet: every stage buffer is in flight
   __builtin_amdgcn_s_waitcnt(0xc07f);        // lgkmcnt(0): the last fragments of stage 0 are in registers
   AQ_WAIT_VMCNT((NSTAGE - 2) * NLOADS);  // stage 1 has landed
   AQ_BARRIER();
   // slot A of stage 0: its buffer (0) is free now and takes stage NSTAGE
-  slot(last_of(k0{}), smem + STAGE, 0, yes{}, NSTAGE, 0, q0{});
+  next_lines();
+  slot(last_of(k0{}), smem + A_STAGE, 0, yes{}, NSTAGE, 0, q0{});
   int b_prev = 0;  // buffer of stage s-1
 #ifdef AQ_LAB_STALL
   long long st_t0 = 0, st_t1 = 0, st_sum = 0;
   const long long st_begin = clock64();
 #endif
-  auto stage = [&](int s, auto c0_c) {
+  auto stage = [&](int s, auto c0_c, auto loads_c) {
     const int b_cur = b_prev == NSTAGE - 1 ? 0 : b_prev + 1;
     const int b_next = b_cur == NSTAGE - 1 ? 0 : b_cur + 1;
     // sub-steps 0 .. NKS-2 of stage s; the rest of stage s-1+NSTAGE's loads go into stage s-1's buffer
-    middle_slots(c0_c, smem + b_cur * STAGE, yes{}, s - 1 + NSTAGE, b_prev);
+    middle_slots(c0_c, smem + b_cur * A_STAGE, loads_c, s - 1 + NSTAGE, b_prev);
 #ifdef AQ_LAB_STALL
     const long long st_now = clock64();
 #endif
@@ -490,18 +581,25 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
     st_t1 = clock64();
 #endif
     // slot A: last sub-step of stage s | first fragments of stage s+1 | first loads of stage s+NSTAGE
-    slot(last_of(c0_c), smem + b_next * STAGE, 0, yes{}, s + NSTAGE, b_cur, q0{});
+    next_lines();
+    slot(last_of(c0_c), smem + b_next * A_STAGE, 0, loads_c, s + NSTAGE, b_cur, q0{});
     b_prev = b_cur;
   };
+  int s = 1;
   if constexpr (NKS % 2 == 0) {
-    for (int s = 1; s < nk; ++s) stage(s, k0{});
+    if constexpr (LINES)
+      for (const int end = K / BK - 1 - NSTAGE; s < end; ++s) stage(s, k0{}, whole{});  // line s + NSTAGE + 1 ends before K
+    for (; s < nk; ++s) stage(s, k0{}, yes{});
   } else {  // one sub-step per stage: the fragment buffers alternate per stage
-    int s = 1;
-    for (; s + 1 < nk; s += 2) {
-      stage(s, k1{});
-      stage(s + 1, k0{});
-    }
-    if (s < nk) stage(s, k1{});
+    auto pairs = [&](int end, auto loads_c) {
+      for (; s + 1 < end; s += 2) {
+        stage(s, k1{}, loads_c);
+        stage(s + 1, k0{}, loads_c);
+      }
+    };
+    if constexpr (LINES) pairs(K / BK - 1 - NSTAGE, whole{});
+    pairs(nk, yes{});
+    if (s < nk) stage(s, k1{}, yes{});
   }
   AQ_WAIT_VMCNT(0);  // drain the padding loads before the workgroup's LDS can be released or reused
 #ifdef AQ_LAB_STALL
@@ -773,9 +871,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
 
 // A workgroup walks tiles pid, pid + gridDim.x, ...: with more tiles than compute units the launch is one
 // resident workgroup per compute unit instead of a queue of short-lived ones (the LDS stages allow one at a time).
-template <bool FP8, int OUT, class S>
+template <bool FP8, int OUT, class S, Rows ROWS>
 __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[S::LDS_BYTES];
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[ROWS == LINE_ROWS ? S::LDS_LINES : S::LDS_BYTES];
   const int nt = p.tiles_m * p.tiles_n;
 #ifdef AQ_LAB
   struct Clk {
@@ -789,14 +887,8 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
     }
   } clk;
 #endif
-  const bool exact = (p.K % S::BK) == 0 && p.lda == p.K;  // uniform
   for (int pid = blockIdx.x; pid < nt; pid += gridDim.x) {
-    if constexpr (S::BIG)
-      gemm_tile<FP8, OUT, S, true>(p, smem, pid);  // launched for whole K steps and even N only
-    else if (exact)
-      gemm_tile<FP8, OUT, S, true>(p, smem, pid);
-    else
-      gemm_tile<FP8, OUT, S, false>(p, smem, pid);
+    gemm_tile<FP8, OUT, S, ROWS>(p, smem, pid);
     if (pid + (int)gridDim.x < nt) __syncthreads();  // every wavefront is done with the stages before they are refilled
   }
 }
@@ -876,7 +968,23 @@ static int launch_shape(GemmArgs& a, hipStream_t st) {
   // 3-5 % faster than queueing a workgroup per tile once there are more tiles than compute units
   const int64_t ntiles = (int64_t)a.tiles_m * a.tiles_n, cus = device_cus();
   const unsigned grid = (unsigned)(ntiles < cus ? ntiles : cus);
-  aq::queue_kernel((gemm_kernel<FP8, OUT, S>), dim3(grid), dim3(S::NTHREADS), 0, st, a);
+  if constexpr (!S::BIG) {  // (big sub-tiles are launched for whole K steps only)
+    if (a.K % S::BK != 0 || a.lda != a.K) {
+      // Lines from 11 of them on: the extra line and the longer prologue cost 0.2..0.3 us.  us, ANY -> LINES at K 1008, 1520, 3056, 4592 (rows of A on
+      // lines): 64 x 64 tiles, 333 x 1536 5.08 -> 5.47, 6.17 -> 6.15, 8.81 -> 8.25, 11.01 -> 10.14; 128 x 64, 798 x 1648 7.26 -> 7.27, 8.61 -> 8.45, 12.2 ->
+      // 11.5, 15.9 -> 14.7; 128 x 128, 2048 x 1536 8.89 -> 8.73, 10.9 -> 10.7, 16.8 -> 15.6, 22.7 -> 21.0, FP8 8.34 -> 8.17, 10.3 -> 9.8, 15.9 -> 14.2, 21.4 ->
+      // 18.5.  Not with 32 outputs in a tile, where a wavefront's select serves one product: 64 x 32 tiles 6.57 -> 7.02 at K 2032, 10.3 -> 10.6 at 4592.
+      if constexpr (S::BN > 32) {
+        if (a.K >= 11 * S::BK) {
+          aq::queue_kernel((gemm_kernel<FP8, OUT, S, LINE_ROWS>), dim3(grid), dim3(S::NTHREADS), 0, st, a);
+          return (int)hipGetLastError();
+        }
+      }
+      aq::queue_kernel((gemm_kernel<FP8, OUT, S, ANY_ROWS>), dim3(grid), dim3(S::NTHREADS), 0, st, a);
+      return (int)hipGetLastError();
+    }
+  }
+  aq::queue_kernel((gemm_kernel<FP8, OUT, S, EXACT_ROWS>), dim3(grid), dim3(S::NTHREADS), 0, st, a);
   return (int)hipGetLastError();
 }
 

@@ -49,6 +49,35 @@ def test_a_gap_between_rows_changes_no_bit(tile, M, N, K, out, fp8):
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("K", [1392, 1424, 1520, 1648, 2032])
+@pytest.mark.parametrize("tile,M,N", [(65, 330, 1536), (65, 321, 1535), (64, 700, 1600), (64, 700, 1603), (128, 1500, 2050), (256, 6700, 1345)])
+def test_weights_that_begin_anywhere_in_a_line(tile, M, N, K, fp8):
+    """Around the length from which the tiles load the weights by lines: the same steps as on rows filled with zeros to whole lines, hence the
+    same bits; a row of large values (e4m3: NaN) shows in its own column only."""
+    lib = _abi.load()
+    assert _abi.load_lab().aq_lab_choose_gemm_tile(M, N, K, int(fp8), _abi.AQ_BF16, 0, 256) == tile
+    ld = (K + 127) // 128 * 128
+    a, w = _codes(M, K, fp8, 3), _codes(N, K, fp8, 4)
+    w[N // 2] = 0x7F
+    rows, full = torch.zeros(M, ld, dtype=a.dtype, device=DEV), torch.zeros(N, ld, dtype=a.dtype, device=DEV)
+    rows[:, :K], full[:, :K] = a, w
+    sx, sw = torch.rand(1 if fp8 else M, device=DEV) * 1e-2, torch.rand(1 if fp8 else N, device=DEV) * 1e-2
+    fn = lib.aq_linear_fp8_strided if fp8 else lib.aq_linear_w8a8_strided
+    for out in (BF16, F32):
+        code = _abi.AQ_BF16 if out == BF16 else _abi.AQ_F32
+        want = torch.empty(M, N, device=DEV, dtype=out)
+        assert fn(rows.data_ptr(), ld, sx.data_ptr(), full.data_ptr(), sw.data_ptr(), None, 0, None, want.data_ptr(), code, M, N, ld, _stream()) == 0
+        assert torch.isfinite(want).sum().item() == M * (N - 1 if fp8 else N)
+        for start in (0, 16, 80):
+            base = torch.empty(N * K + 128, dtype=w.dtype, device=DEV)
+            b = base[start:start + N * K].view(N, K)
+            b.copy_(w)
+            y = torch.zeros(M, N, device=DEV, dtype=out)
+            assert fn(rows.data_ptr(), ld, sx.data_ptr(), b.data_ptr(), sw.data_ptr(), None, 0, None, y.data_ptr(), code, M, N, K, _stream()) == 0
+            assert torch.equal(torch.nan_to_num(y, 7.0), torch.nan_to_num(want, 7.0))
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("M,K", [(1, 48), (70, 1040), (70, 2064), (300, 4112), (5000, 272), (300, 9008), (20, 16400)])
 def test_quantisers_write_rows_with_a_gap(M, K, dtype):
