@@ -95,10 +95,11 @@ __device__ __forceinline__ typename Acc<FP8>::type mma(const typename Frag<FP8>:
   }
 }
 
-// gemm_slices.hip: tiles of 32 tm x 32, K cut among a workgroup's wavefronts
-int gemm_slices_rows(int64_t M, int64_t N, int64_t K, int64_t cus);
+// gemm_slices.hip: small tiles, K cut among a workgroup's wavefronts
+enum SlicesTile { SLICES_32X32 = 1, SLICES_48X32, SLICES_32X48, SLICES_64X32, SLICES_32X64, SLICES_48X48 };
+int gemm_slices_tile(int64_t M, int64_t N, int64_t K, int64_t cus);
 template <bool FP8, int OUT>
-int gemm_slices_launch(GemmArgs& a, int tm, hipStream_t st);
+int gemm_slices_launch(GemmArgs& a, int tile, hipStream_t st);
 
 // gemm_walk.hip
 // The last round of 256 x 128 tiles is cut in two behind three rounds or more, when at most half the compute units have a tile in it.

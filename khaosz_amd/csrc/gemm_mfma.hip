@@ -906,7 +906,8 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
 // 6 % of it.  The small tiles are for launches of a few rounds only.
 enum TileKind {
   TILE_AUTO = 0, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129, TILE_WIDE = 192,
-  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258, TILE_SLICES32 = 34, TILE_SLICES64 = 35
+  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258,
+  TILE_SLICES32 = 34, TILE_SLICES64 = 35, TILE_SLICES48X32 = 36, TILE_SLICES32X48 = 37, TILE_SLICES32X64 = 38, TILE_SLICES48 = 39
 };
 #ifdef AQ_LAB
 static int g_forced_tile = 0;  // lab build only: TILE_AUTO = by shape, otherwise forced (tuning and tests)
@@ -1005,16 +1006,23 @@ static bool huge_fp8_ok(const GemmArgs& a, int64_t cus) {
   return tiles >= 2 * cus && (tiles % cus == 0 || 2 * (tiles % cus) > cus);
 }
 
-// The tile that takes a call on a device of `cus` compute units.  TILE_WALK and TILE_WIDE: of gemm_walk_kernel, TILE_SLICES32 and
-// TILE_SLICES64: of gemm_slices_kernel.
+// The tile that takes a call on a device of `cus` compute units.  TILE_WALK and TILE_WIDE: of gemm_walk_kernel, TILE_SLICES..: of
+// gemm_slices_kernel.
 static int choose_tile(const GemmArgs& a, bool fp8, int out, int64_t cus) {
   if (fp8 && out != OUT_I32 && huge_fp8_ok(a, cus)) return TILE_HUGE;
   const bool walk = out != OUT_I32 && gemm_walk_ok(a, out);
   const int tile = choose_tile_for(a.M, a.N, cus, walk, a.res != nullptr);
   if (walk && tile == TILE_LARGE) return TILE_WALK;
   if (tile == TILE_WIDE || out == OUT_I32) return tile;
-  const int tm = gemm_slices_rows(a.M, a.N, a.K, cus);
-  return tm == 1 ? TILE_SLICES32 : tm == 2 ? TILE_SLICES64 : tile;
+  switch (gemm_slices_tile(a.M, a.N, a.K, cus)) {
+    case SLICES_32X32: return TILE_SLICES32;
+    case SLICES_48X32: return TILE_SLICES48X32;
+    case SLICES_32X48: return TILE_SLICES32X48;
+    case SLICES_64X32: return TILE_SLICES64;
+    case SLICES_32X64: return TILE_SLICES32X64;
+    case SLICES_48X48: return TILE_SLICES48;
+  }
+  return tile;
 }
 
 template <bool FP8, int OUT>
@@ -1031,8 +1039,12 @@ static int launch(GemmArgs& a, hipStream_t st) {
     switch (tile) {
       case TILE_WALK: return gemm_walk_launch<FP8, OUT>(a, st, 128);
       case TILE_WIDE: return gemm_walk_launch<FP8, OUT>(a, st, 192);
-      case TILE_SLICES32: return gemm_slices_launch<FP8, OUT>(a, 1, st);
-      case TILE_SLICES64: return gemm_slices_launch<FP8, OUT>(a, 2, st);
+      case TILE_SLICES32: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X32, st);
+      case TILE_SLICES48X32: return gemm_slices_launch<FP8, OUT>(a, SLICES_48X32, st);
+      case TILE_SLICES32X48: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X48, st);
+      case TILE_SLICES64: return gemm_slices_launch<FP8, OUT>(a, SLICES_64X32, st);
+      case TILE_SLICES32X64: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X64, st);
+      case TILE_SLICES48: return gemm_slices_launch<FP8, OUT>(a, SLICES_48X48, st);
     }
     if constexpr (FP8)
       if (tile == TILE_HUGE) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
@@ -1083,7 +1095,7 @@ extern "C" int aq_lab_read_clock(long long* host2) {
   return (int)hipMemcpyFromSymbol(host2, HIP_SYMBOL(aq::aq_lab_clock), 64);
 }
 extern "C" int aq_lab_set_gemm_tile(int rows) {
-  if (rows != 192 && rows != 258 && rows != 34 && rows != 35 && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
+  if (rows != 192 && rows != 258 && (rows < 34 || rows > 39) && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
   aq::g_forced_tile = rows;
   return AQ_OK;
 }
@@ -1093,7 +1105,9 @@ extern "C" int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8,
   static const char some = 0;
   aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
   a.res = residual ? &some : nullptr;  // only whether there is one
-  return aq::choose_tile(a, fp8 != 0, y_dtype < 0 ? aq::OUT_I32 : y_dtype == AQ_BF16 ? aq::OUT_BF16 : aq::OUT_F32, compute_units);
+  const int tile = aq::choose_tile(a, fp8 != 0, y_dtype < 0 ? aq::OUT_I32 : y_dtype == AQ_BF16 ? aq::OUT_BF16 : aq::OUT_F32, compute_units);
+  // 48 x 48 tiles with K cut serve in the place of larger ones, whose number stands for both here
+  return tile == aq::TILE_SLICES48 ? aq::choose_tile_for(M, N, compute_units) : tile;
 }
 #endif
 
@@ -1124,7 +1138,7 @@ static bool streams_weights(int64_t M, int64_t N, int64_t K) {
 #ifdef AQ_LAB
   if (g_forced_tile) return false;
 #endif
-  return !gemm_slices_rows(M, N, K, device_cus()) && gemv_tokens_ok(M, N, K);
+  return !gemm_slices_tile(M, N, K, device_cus()) && gemv_tokens_ok(M, N, K);
 }
 }  // namespace aq
 
