@@ -228,7 +228,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   auto issue_load = [&](int kt, int buf, int idx, auto kind) {
     if constexpr (EXACT) {
       // steps past the last one request the last step again (into a stage nobody reads): in range by construction
-      const int k0s = (kt < nk ? kt : nk - 1) * BK;  // wavefront-uniform: a scalar offset
+      const int k0s = (decltype(kind)::value == 2 || kt < nk ? kt : nk - 1) * BK;  // wavefront-uniform: a scalar offset
       uint8_t* st = smem + buf * STAGE + wave * 1024;
       if (idx < A_LOADS)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(Ar, (lds_void*)(st + idx * (1024 * NWAVES)), 16, ld_vo[idx], k0s, 0, 0);
@@ -564,9 +564,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   long long st_t0 = 0, st_t1 = 0, st_sum = 0;
   const long long st_begin = clock64();
 #endif
-  auto stage = [&](int s, auto c0_c, auto loads_c) {
-    const int b_cur = b_prev == NSTAGE - 1 ? 0 : b_prev + 1;
-    const int b_next = b_cur == NSTAGE - 1 ? 0 : b_cur + 1;
+  auto stage_in = [&](int s, auto c0_c, auto loads_c, int b_prev, int b_cur, int b_next) {
     // sub-steps 0 .. NKS-2 of stage s; the rest of stage s-1+NSTAGE's loads go into stage s-1's buffer
     middle_slots(c0_c, smem + b_cur * A_STAGE, loads_c, s - 1 + NSTAGE, b_prev);
 #ifdef AQ_LAB_STALL
@@ -583,9 +581,27 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
     // slot A: last sub-step of stage s | first fragments of stage s+1 | first loads of stage s+NSTAGE
     next_lines();
     slot(last_of(c0_c), smem + b_next * A_STAGE, 0, loads_c, s + NSTAGE, b_cur, q0{});
+  };
+  auto stage = [&](int s, auto c0_c, auto loads_c) {
+    const int b_cur = b_prev == NSTAGE - 1 ? 0 : b_prev + 1;
+    const int b_next = b_cur == NSTAGE - 1 ? 0 : b_cur + 1;
+    stage_in(s, c0_c, loads_c, b_prev, b_cur, b_next);
     b_prev = b_cur;
   };
   int s = 1;
+  // Long K: a turn of the loop is NSTAGE steps, whose buffers are then constants -- LDS addresses become offsets of the reads, and what is
+  // left beside products, reads and loads is the load's m0 (27 instructions a step instead of 56 with 64 x 64 tiles, 62 instead of 92 with
+  // 128 x 128).  us, step by step -> so: 128 x 128, 2048 x 2048 x 8192 34.6 -> 33.7, FP8 31.0 -> 29.9, 2048 x 1536 x 6912 27.0 -> 26.0, x 8192 29.5 -> 28.0;
+  // 64 x 64, 512 x 2048 x 6912 13.3 -> 13.2, FP8 13.2 -> 12.9; 64 x 32, 200 x 2048 x 6912 11.1 -> 10.6, FP8 11.3 -> 10.3.  Shorter K: level in the mean,
+  // between 1000 x 4096 x 2048 13.8 -> 14.8 and 2048 x 1536 x 4096 17.3 -> 16.7; two wavefronts per SIMD (256 x 128): 4096 x 3071 x 6912 104 -> 106.
+  if constexpr (EXACT && NKS % 2 == 0 && NWAVES <= 4 && !BIG) {
+    if (nk >= 48) {  // uniform
+      for (; s + 2 * NSTAGE <= nk; s += NSTAGE) {
+#pragma unroll
+        for (int u = 0; u < NSTAGE; ++u) stage_in(s + u, k0{}, whole{}, u, (u + 1) % NSTAGE, (u + 2) % NSTAGE);
+      }
+    }
+  }
   if constexpr (NKS % 2 == 0) {
     if constexpr (LINES)
       for (const int end = K / BK - 1 - NSTAGE; s < end; ++s) stage(s, k0{}, whole{});  // line s + NSTAGE + 1 ends before K

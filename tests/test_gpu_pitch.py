@@ -78,6 +78,24 @@ def test_weights_that_begin_anywhere_in_a_line(tile, M, N, K, fp8):
             assert torch.equal(torch.nan_to_num(y, 7.0), torch.nan_to_num(want, 7.0))
 
 
+@pytest.mark.parametrize("K", [6016, 6144, 6272, 6400, 6528, 6656, 6784])
+@pytest.mark.parametrize("tile", [128, 64, 65, 33])
+def test_long_rows_in_whole_turns_of_the_stages(tile, K):
+    """Around the length from which a turn of the loop is as many steps as there are stages, with every remainder of 3, 4 and 6: the bits of
+    the tile that goes step by step (sums run in the same order)."""
+    M, N = 150, 200
+    a, w, a8, w8 = _codes(M, K, False, 5), _codes(N, K, False, 6), _codes(M, K, True, 7), _codes(N, K, True, 8)
+    sx, sw, r = torch.rand(M, device=DEV) * 1e-2, torch.rand(N, device=DEV) * 1e-2, torch.randn(M, N, device=DEV).to(BF16)
+    run = lambda: (ops.linear_w8a8(a, sx, w, sw, None, out_dtype=F32), ops.linear_w8a8(a, sx, w, sw, None, out_dtype=BF16, residual=r),
+                   ops.linear_fp8(a8, sx[:1], w8, sw[:1], None, out_dtype=F32))
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(tile) == 0
+        got = run()
+        assert lab.aq_lab_set_gemm_tile(256) == 0
+        for y, want in zip(got, run()):
+            assert torch.isfinite(y).all() and torch.equal(y, want)
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("M,K", [(1, 48), (70, 1040), (70, 2064), (300, 4112), (5000, 272), (300, 9008), (20, 16400)])
 def test_quantisers_write_rows_with_a_gap(M, K, dtype):
