@@ -923,7 +923,8 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
 enum TileKind {
   TILE_AUTO = 0, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129, TILE_WIDE = 192,
   TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258,
-  TILE_SLICES32 = 34, TILE_SLICES64 = 35, TILE_SLICES48X32 = 36, TILE_SLICES32X48 = 37, TILE_SLICES32X64 = 38, TILE_SLICES48 = 39
+  TILE_SLICES32 = 34, TILE_SLICES64 = 35, TILE_SLICES48X32 = 36, TILE_SLICES32X48 = 37, TILE_SLICES32X64 = 38, TILE_SLICES48 = 39,
+  TILE_SLICES16 = 40, TILE_SLICES16X32 = 41, TILE_SLICES32X16 = 42, TILE_SLICES16X64 = 43
 };
 #ifdef AQ_LAB
 static int g_forced_tile = 0;  // lab build only: TILE_AUTO = by shape, otherwise forced (tuning and tests)
@@ -1031,6 +1032,10 @@ static int choose_tile(const GemmArgs& a, bool fp8, int out, int64_t cus) {
   if (walk && tile == TILE_LARGE) return TILE_WALK;
   if (tile == TILE_WIDE || out == OUT_I32) return tile;
   switch (gemm_slices_tile(a.M, a.N, a.K, cus)) {
+    case SLICES_16X16: return TILE_SLICES16;
+    case SLICES_16X32: return TILE_SLICES16X32;
+    case SLICES_16X64: return TILE_SLICES16X64;
+    case SLICES_32X16: return TILE_SLICES32X16;
     case SLICES_32X32: return TILE_SLICES32;
     case SLICES_48X32: return TILE_SLICES48X32;
     case SLICES_32X48: return TILE_SLICES32X48;
@@ -1055,6 +1060,10 @@ static int launch(GemmArgs& a, hipStream_t st) {
     switch (tile) {
       case TILE_WALK: return gemm_walk_launch<FP8, OUT>(a, st, 128);
       case TILE_WIDE: return gemm_walk_launch<FP8, OUT>(a, st, 192);
+      case TILE_SLICES16: return gemm_slices_launch<FP8, OUT>(a, SLICES_16X16, st);
+      case TILE_SLICES16X32: return gemm_slices_launch<FP8, OUT>(a, SLICES_16X32, st);
+      case TILE_SLICES16X64: return gemm_slices_launch<FP8, OUT>(a, SLICES_16X64, st);
+      case TILE_SLICES32X16: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X16, st);
       case TILE_SLICES32: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X32, st);
       case TILE_SLICES48X32: return gemm_slices_launch<FP8, OUT>(a, SLICES_48X32, st);
       case TILE_SLICES32X48: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X48, st);
@@ -1111,7 +1120,7 @@ extern "C" int aq_lab_read_clock(long long* host2) {
   return (int)hipMemcpyFromSymbol(host2, HIP_SYMBOL(aq::aq_lab_clock), 64);
 }
 extern "C" int aq_lab_set_gemm_tile(int rows) {
-  if (rows != 192 && rows != 258 && (rows < 34 || rows > 39) && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
+  if (rows != 192 && rows != 258 && (rows < 34 || rows > 43) && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
   aq::g_forced_tile = rows;
   return AQ_OK;
 }
@@ -1122,7 +1131,8 @@ extern "C" int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8,
   aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
   a.res = residual ? &some : nullptr;  // only whether there is one
   const int tile = aq::choose_tile(a, fp8 != 0, y_dtype < 0 ? aq::OUT_I32 : y_dtype == AQ_BF16 ? aq::OUT_BF16 : aq::OUT_F32, compute_units);
-  // 48 x 48 tiles with K cut serve in the place of larger ones, whose number stands for both here
+  // tiles with K cut: 32 x 32 stands for the smaller ones too, the larger tile whose place 48 x 48 take for both
+  if (tile == aq::TILE_SLICES16 || tile == aq::TILE_SLICES16X32 || tile == aq::TILE_SLICES32X16) return aq::TILE_SLICES32;
   return tile == aq::TILE_SLICES48 ? aq::choose_tile_for(M, N, compute_units) : tile;
 }
 #endif
@@ -1148,13 +1158,14 @@ int gemv_tokens_launch(const int8_t* xq, const float* sx, const int8_t* wq, cons
                        int bias_dtype, const void* residual, void* y, int y_dtype, int64_t M, int64_t N, int64_t K,
                        hipStream_t st, bool fp8);
 
-// 17..32 rows of more than 8192 outputs (and decode batches of rows too long for the GEMV kernels): the weight-streaming kernel takes
-// them (not when a test has forced a tile shape)
+// 17..32 rows of more outputs than tiles cut among wavefronts serve (and decode batches of as many whose rows are too long for the GEMV
+// kernels): the weight-streaming kernel takes them (not when a test has forced a tile shape)
 static bool streams_weights(int64_t M, int64_t N, int64_t K) {
 #ifdef AQ_LAB
   if (g_forced_tile) return false;
 #endif
-  return !gemm_slices_tile(M, N, K, device_cus()) && gemv_tokens_ok(M, N, K);
+  const int64_t cus = device_cus();
+  return (M <= 16 ? (N + 31) / 32 > cus : !gemm_slices_tile(M, N, K, cus)) && gemv_tokens_ok(M, N, K);
 }
 }  // namespace aq
 

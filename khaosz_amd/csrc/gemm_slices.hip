@@ -1,4 +1,4 @@
-// The GEMM of a few dozen to a few hundred rows: tiles of 32 x 32 to 48 x 48, K cut among the wavefronts of a workgroup.
+// The GEMM of up to a few hundred rows: tiles of 16 x 16 to 48 x 48, K cut among the wavefronts of a workgroup.
 //
 // What bounds it: with few rows a compute unit has at most one small tile, and in a K loop shared by a workgroup's
 // wavefronts every K step costs the latency of its barrier, its LDS reads and its waits, 430 to 450 cycles for 128 to 256
@@ -9,8 +9,8 @@
 // unit, 75 to 90 GB/s, and so the tile is the smallest of which every compute unit has at most one: hence products of 16 x 16, of
 // which tiles come in steps of 16.
 //
-// us, 64 x 32 tile of gemm_kernel (or the weight-streaming GEMV up to 32 rows) -> here: 32 x 2048 x 2048 4.8 -> 3.7,
-// 64 x 2048 x 2048 5.4 -> 3.74, 64 x 1536 x 6912 10.4 -> 5.9, 128 x 2048 x 8192 11.8 -> 8.1, weights from HBM 13.9 -> 9.8;
+// us, 64 x 32 tile of gemm_kernel (or the weight-streaming GEMV up to 32 rows) -> here: 32 x 2048 x 2048 4.8 -> 2.9,
+// 64 x 2048 x 2048 5.4 -> 3.2, 64 x 1536 x 6912 10.4 -> 5.2, 128 x 2048 x 8192 11.8 -> 8.1, weights from HBM 13.9 -> 9.8;
 // 200 x 1536 x 6912 10.5 -> 9.2 (48 x 32).  Wider tiles (64 x 48, 64 x 64), 64-byte steps, three and four stages, eight wavefronts on
 // the 32 x 32 tile measured 0 to 40 % slower.  Products of 32 x 32, and a compare and a select in every load, which only a step in
 // which K ends needs: 32 x 32 tiles 3 to 4 % slower (64 x 2048 x 2048 3.83, K 2032 3.84 | 3.79), 64 x 32 1 to 2 % (200 x 1536 x 6912 10.26 | 10.12).
@@ -257,15 +257,20 @@ static int launch_slices(GemmArgs& a, hipStream_t st) {
 }
 
 // The tile of a launch, 0: none of them.  One tile per compute unit: a second round costs as much as the first, and the
-// kernels with larger tiles move fewer bytes.  Up to 16 rows have kernels of their own.
+// kernels with larger tiles move fewer bytes.
 //
 // Measured, us, the path before (gemm_kernel's tiles; up to 32 rows the weight-streaming GEMV) -> here, weights in the
 // last-level cache | streamed from HBM:
+//   16 x 16, 16 x 32 and 32 x 16 against 32 x 32 (520 sizes drawn from 17..130 rows, N 100 to 9000, K 256 to 9000): 0.84 | 0.86 in the mean, by
+//     K 0.89 to 0.70, none slower.  Four wavefronts; eight on 16 x 16 0.93 of these from HBM with K from 4096, 1.06 from the cache.
+//   Up to 16 rows (codes whose quantiser is a launch of its own, of rows too long or too wide for the kernels that round them): FP8 and tiles of
+//     gemm_kernel 0.57 | 0.63 (181 sizes of 9..16 rows, the GEMV on codes or 64 x 32 tiles before), none slower: 12 x 816 x 6416 11.4 -> 4.3 | 11.6 -> 5.2, 9 x
+//     5820 x 5120 18.4 -> 7.1 | 18.1 -> 8.5; 1..8 rows 0.56 | 0.68.  Beyond 8192 outputs 16 x 64 (0.71 | 0.78 for 59 sizes up to 16384, two of them
+//     slower, by 4 and 5 %), then rounds of 16 x 32 (0.74 | 0.81).  12 x 4096 x 11008 16.1 -> 10.1 | 16.5 -> 13.1 (the weight-streaming kernel).
 //   32 x 32, more than 32 rows: faster at every size tried (N 512 to 4096, K 512 to 8192), 64 x 2048 x 512 3.5 -> 3.1 | 3.9 -> 3.4,
 //     64 x 4096 x 8192 12.2 -> 8.8 | 17.4 -> 12.6, 333 x 512 x 6912 10.5 -> 6.0 | 10.6 -> 7.6.
-//   32 x 32, 17..32 rows: 32 x 256 x 2048 4.6 -> 3.6 | 4.7 -> 4.6, 32 x 2048 x 2048 5.1 -> 3.6 | 5.2 -> 5.2, 24 x 512 x 8192
-//     9.9 -> 6.2 | 9.6 -> 10.8, 32 x 2048 x 8192 10.3 -> 6.7 | 10.4 -> 12.1, 32 x 8192 x 4096 8.2 -> 6.2 | 9.3 -> 9.5: a fifth to two
-//     thirds faster from the cache, level to 16 % slower from HBM, where the GEMV has more loads in flight.
+//   17..32 rows, the GEMV -> the smallest tile that fits (32 x 2048 is 16 x 16): 32 x 256 x 2048 4.6 -> 2.9 | 4.7 -> 3.3, 32 x 2048 x 2048 5.1 -> 2.9 |
+//     5.2 -> 4.0, 24 x 512 x 8192 9.9 -> 4.3 | 9.6 -> 6.4, 32 x 8192 x 4096 8.2 -> 6.1 | 9.3 -> 9.3 (32 x 32).
 //   48 x 32 and 32 x 48, where 32 x 32 are too many (120 sizes drawn from 17..800 rows, N 256 to 16384, K 256 to 9000): 0.90 | 0.92 in the
 //     mean, 200 x 1536 x 6912 10.3 -> 9.2 | 11.7 -> 10.2 (64 x 32 tiles before), 22 x 9456 x 1280 FP8 0.66 | 0.77 (the GEMV before); the slowest 0.95 | 1.06
 //     (24 x 10912 x 768).
@@ -279,8 +284,11 @@ static int launch_slices(GemmArgs& a, hipStream_t st) {
 //     11.1 | 17.1 -> 13.2, FP8 12.6 -> 11.1 | 15.3 -> 12.4; with K 1536 to 3072 1.07 | 1.05 in the mean, and up to 64 rows 39 x 11824 x 3840 9.9 -> 10.9 | 13.7 ->
 //     12.9.
 int gemm_slices_tile(int64_t M, int64_t N, int64_t K, int64_t cus) {
-  if (M <= 16) return 0;
   auto fits = [&](int64_t bm, int64_t bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn) <= cus; };
+  if (fits(16, 16)) return SLICES_16X16;
+  if (fits(16, 32)) return SLICES_16X32;
+  if (M <= 16) return fits(16, 64) ? SLICES_16X64 : SLICES_16X32;
+  if (fits(32, 16)) return SLICES_32X16;
   if (fits(32, 32)) return SLICES_32X32;
   if (fits(48, 32)) return SLICES_48X32;
   if (fits(32, 48)) return SLICES_32X48;
@@ -293,6 +301,10 @@ int gemm_slices_tile(int64_t M, int64_t N, int64_t K, int64_t cus) {
 template <bool FP8, int OUT>
 int gemm_slices_launch(GemmArgs& a, int tile, hipStream_t st) {
   switch (tile) {
+    case SLICES_16X16: return launch_slices<FP8, OUT, 4, 1, 1, 128, 2>(a, st);
+    case SLICES_16X32: return launch_slices<FP8, OUT, 4, 1, 2, 128, 2>(a, st);
+    case SLICES_16X64: return launch_slices<FP8, OUT, 8, 1, 4, 128, 1>(a, st);
+    case SLICES_32X16: return launch_slices<FP8, OUT, 4, 2, 1, 128, 2>(a, st);
     case SLICES_32X32: return launch_slices<FP8, OUT, 4, 2, 2, 128, 2>(a, st);
     case SLICES_48X32: return launch_slices<FP8, OUT, 4, 3, 2, 128, 2>(a, st);
     case SLICES_32X48: return launch_slices<FP8, OUT, 4, 2, 3, 128, 2>(a, st);

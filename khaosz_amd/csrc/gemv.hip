@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "aq_common.h"
+#include "aq_gemm.h"
 #include "aq_gemv.h"
 #include "aq_rows.h"
 
@@ -352,10 +353,7 @@ constexpr int GM_BATCH = 8;    // MFMA steps (64 K bytes each) per register batc
 // compiler drain the weight loads at the join, 0.4 us of a 6.5 us launch).
 // XR: rounds of token-code vectors (8 per thread each) requested ahead of the weight stream; rows too long for
 // XR rounds copy the rest afterwards, which waits for the weight loads in flight.
-// FP8: weights and tokens are OCP e4m3fn codes with one scale per tensor (p.sx, p.sw point to scalars) and the
-// products run on v_mfma_f32_16x16x128_f8f6f4 -- one instruction per 128-byte line instead of two -- with fp32
-// accumulation.
-template <int KS, int GR, bool RES, int XR, bool FP8 = false>
+template <int KS, int GR, bool RES, int XR>
 __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [16][K + 16] token codes, [16] scales, 16 spare bytes; later the partial sums
   const int tid = threadIdx.x, lane = tid & 63;
@@ -384,11 +382,11 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
   const EpiOperands epi(p, kh == 0, true, RES);
   float sxv = 0.0f;
   auto load_epi = [&]() {
-    sxv = epi.load_sx(FP8 ? 0 : tok, FP8 || tok < M);
+    sxv = epi.load_sx(tok, tok < M);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int n = rbase + r;
-      swv[r] = epi.load_sw(FP8 ? 0 : n, FP8 || n < N);
+      swv[r] = epi.load_sw(n, n < N);
       bv[r] = epi.load_bias(n, n < N);
       rv[r] = RES ? epi.load_res(tok, n, tok < M && n < N, (int)p.ldr) : 0u;
     }
@@ -468,10 +466,9 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
   // Four independent accumulators (summed at the end: int32, exact in any order) and a batch's token
   // fragments read from LDS up front: one chain of 16 dependent read -> MFMA steps took 0.6 us after the
   // token codes had landed, which is all on the kernel's critical path.
-  using accv = std::conditional_t<FP8, v4f, v4i>;
-  accv accs[4];
+  v4i accs[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) accs[i] = accv{0, 0, 0, 0};
+  for (int i = 0; i < 4; ++i) accs[i] = v4i{0, 0, 0, 0};
   // MFMA step (t, e) of line t takes, for weight row r = lane % 16 and token lane % 16, the line's piece
   // 2 (lane / 16) + e: K bytes t 128 + (2 q + e) 16 of the wavefront's part.  (Any assignment of K bytes to the
   // steps' k slots is a valid product as long as both operands use the same one.)  Lane l holds piece l / 8 of
@@ -501,16 +498,8 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
                       __builtin_amdgcn_update_dpp((int)hi.y, (int)lo.y, ROR8, 0xf, 0x3, false),
                       __builtin_amdgcn_update_dpp((int)hi.z, (int)lo.z, ROR8, 0xf, 0x3, false),
                       __builtin_amdgcn_update_dpp((int)hi.w, (int)lo.w, ROR8, 0xf, 0x3, false)};
-      if constexpr (!FP8) {
-        accs[(2 * t) & 3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, x[2 * t], accs[(2 * t) & 3], 0, 0, 0);
-        accs[(2 * t + 1) & 3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, x[2 * t + 1], accs[(2 * t + 1) & 3], 0, 0, 0);
-      } else {
-        // the line's pieces 2q and 2q + 1 are the 32 K bytes lane (row, q) feeds one 16x16x128 product
-        const v8i wl = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-        const v4i xa = x[2 * t], xb = x[2 * t + 1];
-        const v8i xl8 = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-        accs[t & 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wl, xl8, accs[t & 3], 0, 0, 0, 0, 0, 0);
-      }
+      accs[(2 * t) & 3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, x[2 * t], accs[(2 * t) & 3], 0, 0, 0);
+      accs[(2 * t + 1) & 3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, x[2 * t + 1], accs[(2 * t + 1) & 3], 0, 0, 0);
     }
   };
   for (int l0 = 0; l0 < nline; l0 += 2 * GM_LINES) {
@@ -520,16 +509,16 @@ __global__ __launch_bounds__(GM_MAX_WAVES * 64) void gemv_mfma_kernel(GemvArgs p
     if (l0 + 3 * GM_LINES < nline) wload(l0 + 3 * GM_LINES, wb);
   }
 
-  accv acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
+  v4i acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
   // sum the K parts: all but the first wavefront of each group park their 4 sums in LDS
   __syncthreads();  // everyone is done reading the token codes: the buffer is reused
   int* part = reinterpret_cast<int*>(xs) + grp * (ksplit - 1) * 256;
   if (kh != 0) {
-    *reinterpret_cast<accv*>(part + (kh - 1) * 256 + lane * 4) = acc;
+    *reinterpret_cast<v4i*>(part + (kh - 1) * 256 + lane * 4) = acc;
   }
   __syncthreads();
   if (kh != 0) return;
-  for (int k = 0; k < ksplit - 1; ++k) acc += *reinterpret_cast<const accv*>(part + k * 256 + lane * 4);  // fp32: a fixed order
+  for (int k = 0; k < ksplit - 1; ++k) acc += *reinterpret_cast<const v4i*>(part + k * 256 + lane * 4);
 
   if (tok >= M) return;
   float y[4];
@@ -570,7 +559,7 @@ static bool gemv_mfma_ok(int64_t M, int64_t K) {
   return M > GV_MFMA_MIN_M && (K % 256) == 0 && 16 * (K + 16) + 64 + 16 <= GV_MAX_LDS;
 }
 
-static int launch_gemv_mfma(GemvArgs a, hipStream_t st, bool fp8 = false) {
+static int launch_gemv_mfma(GemvArgs a, hipStream_t st) {
   // 2 row groups x 2 K parts per workgroup by default; with too few rows for that to give every
   // compute unit a workgroup, one row group per workgroup and up to 8 K parts
   a.ksplit = 2;
@@ -588,19 +577,13 @@ static int launch_gemv_mfma(GemvArgs a, hipStream_t st, bool fp8 = false) {
   // one round of token-code loads ahead of the weights covers 8 vectors per thread; longer rows take three
   const bool long_rows = (int64_t)16 * (a.K / 16) > (int64_t)8 * a.ksplit * a.groups * 64;
   using kern_t = void (*)(GemvArgs);
-  static const kern_t table[2][2][2][2] = {
-      {{{gemv_mfma_kernel<0, 0, false, 1>, gemv_mfma_kernel<0, 0, false, 3>},
-        {gemv_mfma_kernel<0, 0, true, 1>, gemv_mfma_kernel<0, 0, true, 3>}},
-       {{gemv_mfma_kernel<2, 2, false, 1>, gemv_mfma_kernel<2, 2, false, 3>},
-        {gemv_mfma_kernel<2, 2, true, 1>, gemv_mfma_kernel<2, 2, true, 3>}}},
-      {{{gemv_mfma_kernel<0, 0, false, 1, true>, gemv_mfma_kernel<0, 0, false, 3, true>},
-        {gemv_mfma_kernel<0, 0, true, 1, true>, gemv_mfma_kernel<0, 0, true, 3, true>}},
-       {{gemv_mfma_kernel<2, 2, false, 1, true>, gemv_mfma_kernel<2, 2, false, 3, true>},
-        {gemv_mfma_kernel<2, 2, true, 1, true>, gemv_mfma_kernel<2, 2, true, 3, true>}}}};
-  const kern_t fn = table[fp8][fixed][res][long_rows];
+  static const kern_t table[2][2][2] = {
+      {{gemv_mfma_kernel<0, 0, false, 1>, gemv_mfma_kernel<0, 0, false, 3>}, {gemv_mfma_kernel<0, 0, true, 1>, gemv_mfma_kernel<0, 0, true, 3>}},
+      {{gemv_mfma_kernel<2, 2, false, 1>, gemv_mfma_kernel<2, 2, false, 3>}, {gemv_mfma_kernel<2, 2, true, 1>, gemv_mfma_kernel<2, 2, true, 3>}}};
+  const kern_t fn = table[fixed][res][long_rows];
   if (lds > 64 * 1024) {
-    static LdsOptIn opted[16];
-    const int e = opted[fp8 * 8 + fixed * 4 + res * 2 + long_rows].ensure(reinterpret_cast<const void*>(fn));
+    static LdsOptIn opted[8];
+    const int e = opted[fixed * 4 + res * 2 + long_rows].ensure(reinterpret_cast<const void*>(fn));
     if (e) return e;
   }
   aq::queue_kernel(fn, dim3(grid), dim3(a.ksplit * a.groups * 64), lds, st, a);
@@ -616,8 +599,8 @@ static bool gemv_swiglu_ok(int64_t M, int64_t F, int64_t K) {
 // 17..32 tokens on codes: the same weight stream (every weight byte HBM -> registers once, operands assembled by
 // one DPP rotation per dword) with TG = 2 groups of 16 tokens multiplied against each weight fragment: a bandwidth-bound
 // launch for matrices of more 32-row blocks than compute units, where the GEMM whose wavefronts share K would take a second
-// round of tiles (its comment has both sides; at one tile per compute unit it is the faster one from the last-level cache
-// and level to 16 % slower from HBM).  Also the decode batch sizes whose rows are too long for the kernels above.  From 33
+// round of tiles (at one tile per compute unit it is the faster one).  Also decode batches of as many outputs whose rows are too long
+// for the kernels above.  From 33
 // tokens on, with a third and fourth token group, it was the slower one (48 rows: 6.1 us, 64 rows: 7.6 us with the weights
 // in the last-level cache, where a 128 x 32 tile took 5.8 us).  Same integer sums, same epilogue: the bits of the tiled GEMM.
 // K is walked in chunks of 1024 bytes per wavefront (KS wavefronts per row group: 1024-, 2048- or 4096-byte chunks
@@ -627,7 +610,7 @@ static bool gemv_swiglu_ok(int64_t M, int64_t F, int64_t K) {
 // the chunk boundaries untouched (two register batches, each reloaded as soon as it has been consumed).  GRP row
 // groups of 16 rows per workgroup (every workgroup copies all token codes from L2: more rows per workgroup for
 // matrices of more 32-row blocks than compute units); rows must be whole 128-byte lines (K % 128 == 0).
-// FP8: e4m3 codes with one scale per tensor and fp32 accumulation, as in gemv_mfma_kernel (chunks and K parts
+// FP8: e4m3 codes with one scale per tensor, v_mfma_f32_16x16x128_f8f6f4 and fp32 accumulation (chunks and K parts
 // summed in a fixed order).
 template <int TG, int KS, bool RES, int GRP = 2, bool FP8 = false>
 __global__ __launch_bounds__(KS * GRP * 64) void gemv_mfma_tokens_kernel(GemvArgs p) {
@@ -1059,8 +1042,7 @@ extern "C" int aq_gemv_w8a8_decode_residual(const void* x, int x_dtype, const in
 }
 
 // ---------------------------------------------------------------------------
-// FP8 decode: the same streaming GEMV on e4m3 codes with per-tensor scales.  Shapes the kernel does not take
-// (K not in whole 256-byte steps, rows too long for the LDS) go to the tiled FP8 GEMM, which takes any M.
+// FP8 decode: rows that gemv_rows.hip casts itself, or codes and tiles whose K is cut among wavefronts (gemm_slices.hip).
 extern "C" size_t aq_gemv_fp8_workspace_bytes(int64_t M, int64_t K) {
   if (M < 0 || K < 0) return 0;
   return aq::align256((size_t)(M * K)) + 256 + AQ_FP8_AMAX_WS_BYTES;  // codes, the scale, the quantiser's partial maxima
@@ -1110,10 +1092,21 @@ extern "C" int aq_gemv_fp8_codes_residual(const uint8_t* xq, const float* sx, co
   if (!xq || !sx) return AQ_E_NULL;
   if (aq::check_ptr16(xq) || aq::check_ptr(sx, 4)) return AQ_E_ALIGN;
   if (!gemv_fp8_ok(K)) return aq_linear_fp8_residual(xq, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, stream);
-  aq::GemvArgs a = gemv_fp8_args(wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K);
-  a.xq = reinterpret_cast<const int8_t*>(xq);
+  aq::GemmArgs a{};
+  a.A = xq;
+  a.B = wq;
+  a.C = y;
+  a.M = (int)M;
+  a.N = (int)N;
+  a.K = a.lda = (int)K;
   a.sx = sx;
-  return aq::launch_gemv_mfma(a, static_cast<hipStream_t>(stream), true);
+  a.sw = sw;
+  a.bias = bias;
+  a.bias_dtype = bias_dtype;
+  a.res = residual;
+  const int tile = aq::gemm_slices_tile(M, N, K, aq::device_cus());
+  return y_dtype == AQ_BF16 ? aq::gemm_slices_launch<true, aq::OUT_BF16>(a, tile, static_cast<hipStream_t>(stream))
+                            : aq::gemm_slices_launch<true, aq::OUT_F32>(a, tile, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int aq_gemv_fp8_decode_residual(const void* x, int x_dtype, const uint8_t* wq, const float* sw,

@@ -486,8 +486,10 @@ template <int KS, int R, bool TILED>
 static int launch_shape(const GemvArgs& a, RowsKind kind, hipStream_t st) {
 #define AQ_GX(BF16, RPW, VPL, NORM, FP8) gemv_rows_kernel<KS, R, BF16, RPW, VPL, NORM, FP8, false, 0, TILED>
   static const rows_kernel_t i8[2][4] = {
-      {AQ_GX(true, 1, 2, false, false), AQ_GX(true, 1, 4, false, false), AQ_GX(true, 1, 8, false, false), AQ_GX(true, 1, 16, false, false)},
-      {AQ_GX(true, 2, 2, false, false), AQ_GX(true, 2, 4, false, false), AQ_GX(true, 2, 8, false, false), AQ_GX(true, 2, 16, false, false)}};
+      {AQ_GX(true, 1, 2, false, false), AQ_GX(true, 1, 4, false, false), AQ_GX(true, 1, 8, false, false),
+       TILED ? nullptr : gemv_rows_kernel<KS, R, true, 1, 16, false, false>},
+      {AQ_GX(true, 2, 2, false, false), AQ_GX(true, 2, 4, false, false), AQ_GX(true, 2, 8, false, false),
+       TILED ? nullptr : gemv_rows_kernel<KS, R, true, 2, 16, false, false>}};  // (tiles: up to 4096)
   // (16 rows of more than 4096 cannot stay in registers between the tensor's maximum and the cast: gemv_rows_ok)
   static const rows_kernel_t f8[2][4] = {
       {AQ_GX(true, 1, 2, false, true), AQ_GX(true, 1, 4, false, true), AQ_GX(true, 1, 8, false, true),
@@ -535,16 +537,17 @@ static bool rounds_merge(const GemvArgs& a, bool norm) {
 // length class, whose vectors are requested whether the row has them or not):
 //   tiles      start + rounds over the compute units x (row x tile rows x length + weight x weight rows x K + all x M x K)
 //   launches   two[0] + two[1] K + two[2] M N K / 10^6 + (more than one tile of 32 x 32 per unit: two[3]) + two[4] N K / 10^4
-// Taken where the tiles are 10 % ahead by that: two sizes in five, at 0.77 of the time in the mean, one in 60 of them slower (by 1 to 8 %, three
-// by more); the choice is 1 % from the faster way in the mean.  us, launches -> tiles: bf16 32 x 2048 -> 2048 6.8 -> 4.7, 64 x 1024 -> 3072 6.4 ->
-// 5.1, 32 x 512 -> 8192 5.9 -> 4.8, fp32 64 x 512 -> 2048 5.7 -> 4.2, norm 48 x 1024 -> 2048 6.6 -> 4.3, FP8 35 x 1456 -> 944 8.5 -> 6.3; not 64 x 2048 ->
-// 3072 (6.9, tiles 8.1) nor fp32 64 x 2048 -> 2048 (7.2, 7.6).
+// Taken where the tiles are 5 % ahead by that: one size in three, at 0.84 of the time in the mean, one in fifteen of them slower; the choice is
+// 0.7 % from the faster way in the mean (1 % at 10 % ahead, 0.8 % at level).  us from a graph, launches -> tiles, weights in the last-level cache | from
+// HBM: bf16 32 x 2048 -> 2048 5.7 -> 4.8 | 6.7 -> 5.1, 64 x 1024 -> 3072 6.1 -> 4.7 | 6.9 -> 5.0, 32 x 512 -> 8192 5.5 -> 4.6 | 6.4 -> 4.8, fp32 64 x 512 -> 2048 5.2 -> 4.2 |
+// 5.8 -> 4.6; furthest off fp32 64 x 2048 -> 2048 6.5 -> 7.5 | 7.3 -> 7.4.  Calls that are not captured gain the host's 2.4 us of a launch besides (that
+// one 8.1 -> 7.1).
 struct TiledCost {
   double start, row, weight, all, two[5];
 };
 static const TiledCost& tiled_cost(RowsKind kind) {
-  static const TiledCost i8 = {3.07, 0.038, 0.038, 0, {5.5, 0.77, 2.32, 0.91, 0.47}}, norm = {3.24, 0.083, 0.033, 0, {5.79, 0.95, 1.8, 0.86, 0.98}},
-                         f32 = {3.26, 0.041, 0.042, 0, {5.0, 1.3, 2.06, 0.82, 0.58}}, f8 = {3.81, 0.054, 0.047, 0.018, {7.53, 0.82, 3.34, 0.67, 0.38}};
+  static const TiledCost i8 = {3.07, 0.038, 0.038, 0, {5.27, 0.27, 4.1, 0.47, 0.79}}, norm = {3.24, 0.083, 0.033, 0, {5.49, 0.44, 4.78, 0.35, 1.38}},
+                         f32 = {3.26, 0.041, 0.042, 0, {4.74, 0.79, 4.33, 0.47, 0.92}}, f8 = {3.81, 0.054, 0.047, 0.018, {7.43, 0.32, 6.0, 0.38, 0.84}};
   return kind == ROWS_I8 ? i8 : kind == ROWS_I8_NORM ? norm : kind == ROWS_I8_F32 ? f32 : f8;
 }
 struct Tiled {
@@ -553,7 +556,7 @@ struct Tiled {
 };
 static Tiled tiled_best(RowsKind kind, int64_t M, int64_t N, int64_t K) {
   const TiledCost& c = tiled_cost(kind);
-  const double k = (double)K / 1024, length = K <= 1024 ? 1 : K <= 2048 ? 2 : kind == ROWS_I8_F32 ? 11.2 : K <= 4096 ? 4 : 8;
+  const double k = (double)K / 1024, length = K <= 1024 ? 1 : K <= 2048 ? 2 : kind == ROWS_I8_F32 ? 11.2 : 4;
   const int64_t cus = device_cus();
   Tiled best = {0, 0, 1e30};
   for (int most = 8; most <= 16; most += 8) {
@@ -566,12 +569,13 @@ static Tiled tiled_best(RowsKind kind, int64_t M, int64_t N, int64_t K) {
   return best;
 }
 bool gemv_rows_tiled_ok(RowsKind kind, int64_t M, int64_t N, int64_t K) {
-  // Tiles of more outputs than 80 to a compute unit never gained (64 x 512 -> 8192: 6.3 | 6.6).
-  if (M <= 16 || (M + 15) / 16 * N > 80 * device_cus() || K > (kind == ROWS_I8_NORM ? 2048 : kind == ROWS_FP8 ? 4096 : GX_MAX_K)) return false;
+  // Tiles of more outputs than 80 to a compute unit never gained (64 x 512 -> 8192: 6.3 | 6.6), nor longer bf16 rows than 4096.
+  const int64_t most = kind == ROWS_I8_NORM ? 2048 : kind == ROWS_I8_F32 ? GX_MAX_K : 4096;
+  if (M <= 16 || (M + 15) / 16 * N > 80 * device_cus() || K > most) return false;
   const double* two = tiled_cost(kind).two;
   const double k = (double)K / 1024, nk = (double)N * k;
   const bool rounds = (M + 31) / 32 * ((N + 31) / 32) > device_cus();
-  return tiled_best(kind, M, N, K).us < 0.9 * (two[0] + two[1] * k + two[2] * M * nk / 1e6 + (rounds ? two[3] : 0) + two[4] * nk / 1e4);
+  return tiled_best(kind, M, N, K).us < 0.95 * (two[0] + two[1] * k + two[2] * M * nk / 1e6 + (rounds ? two[3] : 0) + two[4] * nk / 1e4);
 }
 
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {

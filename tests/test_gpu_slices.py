@@ -18,9 +18,9 @@ def to_np(t):
     return t.detach().cpu().numpy()
 
 
-# 48 x 32, 32 x 48, 32 x 64, 48 x 48: fewer K steps than wavefronts, K that ends in a step and at one's end, ragged rows and outputs, odd N
-@pytest.mark.parametrize("kind", [36, 37, 38, 39])
-@pytest.mark.parametrize("M,N,K", [(17, 33, 16), (33, 97, 400), (97, 130, 1040), (65, 1001, 2064), (49, 64, 2048), (200, 512, 1936)])
+# 48 x 32, 32 x 48, 32 x 64, 48 x 48, 16 x 16, 16 x 32, 32 x 16, 16 x 64: fewer K steps than wavefronts, K that ends in a step and at one's end, ragged rows and outputs, odd N
+@pytest.mark.parametrize("kind", [36, 37, 38, 39, 40, 41, 42, 43])
+@pytest.mark.parametrize("M,N,K", [(1, 40, 16), (17, 33, 16), (33, 97, 400), (97, 130, 1040), (65, 1001, 2064), (49, 64, 2048), (200, 512, 1936)])
 def test_tiles_of_sixteens(oracle, M, N, K, kind):
     rng = np.random.default_rng(M + N + K)
     xq, wq = (rng.integers(-128, 128, (n, K), dtype=np.int8) for n in (M, N))
@@ -49,7 +49,8 @@ def test_tiles_of_sixteens(oracle, M, N, K, kind):
 # Both sides of the rule's lines on 256 compute units: 256 tiles of a shape and a few more, K 512 and 3072, 64 rows
 @pytest.mark.parametrize("M,N,K,tile", [(64, 4096, 528, 34), (96, 4096, 528, 36), (97, 2752, 528, 37), (64, 4097, 528, 37), (64, 8192, 528, 33),
                                         (65, 4100, 512, 38), (65, 4100, 496, 65), (32, 12288, 272, 37), (333, 1536, 3072, None),
-                                        (333, 1536, 3056, None), (336, 1776, 3088, None), (336, 1777, 3088, None), (64, 6145, 3088, 35)])
+                                        (333, 1536, 3056, None), (336, 1776, 3088, None), (336, 1777, 3088, None), (64, 6145, 3088, 35), (16, 4096, 528, 34), (16, 4097, 528, 34),
+                                        (33, 1360, 528, 34), (9, 8193, 528, 43), (3, 16385, 272, 34), (32, 2048, 1040, 34), (17, 4097, 1040, 34)])
 def test_the_rule_for_tiles_of_sixteens(M, N, K, tile):
     """Whichever tile the rule takes, int8 sums are the bits of the 64 x 64 tile; FP8 sums differ by their order alone: fp32 sums of K
     products by at most 2 K 2^-24 of the sum of their magnitudes, bf16 results by a rounding more."""
@@ -69,3 +70,17 @@ def test_the_rule_for_tiles_of_sixteens(M, N, K, tile):
     sums = (x8.float().abs() @ w8.float().abs().T) * (sx[0] * sw[0])
     diff = (got[1].float() - want[1].float()).abs()
     assert (diff <= 2.0 ** -7 * want[1].float().abs() + 2 * K * 2.0 ** -24 * sums).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 300, 256), (9, 4100, 512), (12, 816, 6416), (16, 8200, 4352), (5, 16400, 272), (9, 130, 8448)])
+def test_up_to_sixteen_rows_of_codes(M, N, K):
+    """FP8 rows that are cast by a launch of their own (K in whole 256-byte steps and not): against fp64 sums, with a bias and a residual."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x8, w8 = (torch.randn(n, K, generator=g).to(torch.float8_e4m3fn) for n in (M, N))
+    bias, res = torch.randn(N, generator=g), torch.randn(M, N, generator=g)
+    one = torch.ones(1, device=DEV)
+    y = ops.gemv_fp8_codes(x8.view(torch.uint8).to(DEV), one, w8.view(torch.uint8).to(DEV), one, bias.to(DEV), out_dtype=torch.float32, residual=res.to(DEV))
+    a, c = x8.double(), w8.double()
+    want = a @ c.T + bias.double() + res.double()
+    bound = (6e-5 + (K + 4) * 2.0 ** -24) * (a.abs() @ c.abs().T) + 2.0 ** -22 * (want.abs() + bias.abs() + res.abs())  # as above, and two additions
+    assert ((y.cpu().double() - want).abs() <= bound).all()
