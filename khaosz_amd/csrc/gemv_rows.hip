@@ -490,11 +490,11 @@ static int launch_shape(const GemvArgs& a, RowsKind kind, hipStream_t st) {
        TILED ? nullptr : gemv_rows_kernel<KS, R, true, 1, 16, false, false>},
       {AQ_GX(true, 2, 2, false, false), AQ_GX(true, 2, 4, false, false), AQ_GX(true, 2, 8, false, false),
        TILED ? nullptr : gemv_rows_kernel<KS, R, true, 2, 16, false, false>}};  // (tiles: up to 4096)
-  // (16 rows of more than 4096 cannot stay in registers between the tensor's maximum and the cast: gemv_rows_ok)
+  // (16 rows of more than 4096 cannot stay in registers between the tensor's maximum and the cast: gemv_rows_ok; tiles: up to 2048)
   static const rows_kernel_t f8[2][4] = {
-      {AQ_GX(true, 1, 2, false, true), AQ_GX(true, 1, 4, false, true), AQ_GX(true, 1, 8, false, true),
+      {AQ_GX(true, 1, 2, false, true), AQ_GX(true, 1, 4, false, true), TILED ? nullptr : gemv_rows_kernel<KS, R, true, 1, 8, false, true>,
        TILED ? nullptr : gemv_rows_kernel<KS, R, true, 1, 16, false, true>},
-      {AQ_GX(true, 2, 2, false, true), AQ_GX(true, 2, 4, false, true), AQ_GX(true, 2, 8, false, true), nullptr}};
+      {AQ_GX(true, 2, 2, false, true), AQ_GX(true, 2, 4, false, true), TILED ? nullptr : gemv_rows_kernel<KS, R, true, 2, 8, false, true>, nullptr}};
   static const rows_kernel_t norm[2][2] = {{AQ_GX(true, 1, 2, true, false), AQ_GX(true, 1, 4, true, false)},
                                            {AQ_GX(true, 2, 2, true, false), AQ_GX(true, 2, 4, true, false)}};
   static const rows_kernel_t f32[3] = {AQ_GX(false, 1, 4, false, false), AQ_GX(false, 1, 8, false, false), AQ_GX(false, 1, 32, false, false)};
@@ -533,21 +533,21 @@ static bool rounds_merge(const GemvArgs& a, bool norm) {
 // More than 16 rows: tiles of 9..16 or of up to 8 rows, each with its own workgroups over the weight rows.  Every tile reads the
 // weights and every workgroup rounds its tile's rows again, so it is the faster form while tiles x outputs x row length is small:
 // one launch then stands for the quantiser's and the GEMM's (FP8: the maximum's, the cast's and the GEMM's), 3.3 to 5 us of which are
-// launches and first requests.  Both ways as fitted to 4265 random sizes of 17 to 200 rows, us (K in units of 1024; `length`: the row
+// launches and first requests.  Both ways as fitted to 4093 random sizes of 17 to 200 rows, us (K in units of 1024; `length`: the row
 // length class, whose vectors are requested whether the row has them or not):
 //   tiles      start + rounds over the compute units x (row x tile rows x length + weight x weight rows x K + all x M x K)
-//   launches   two[0] + two[1] K + two[2] M N K / 10^6 + (more than one tile of 32 x 32 per unit: two[3]) + two[4] N K / 10^4
-// Taken where the tiles are 5 % ahead by that: one size in three, at 0.84 of the time in the mean, one in fifteen of them slower; the choice is
-// 0.7 % from the faster way in the mean (1 % at 10 % ahead, 0.8 % at level).  us from a graph, launches -> tiles, weights in the last-level cache | from
-// HBM: bf16 32 x 2048 -> 2048 5.7 -> 4.8 | 6.7 -> 5.1, 64 x 1024 -> 3072 6.1 -> 4.7 | 6.9 -> 5.0, 32 x 512 -> 8192 5.5 -> 4.6 | 6.4 -> 4.8, fp32 64 x 512 -> 2048 5.2 -> 4.2 |
-// 5.8 -> 4.6; furthest off fp32 64 x 2048 -> 2048 6.5 -> 7.5 | 7.3 -> 7.4.  Calls that are not captured gain the host's 2.4 us of a launch besides (that
-// one 8.1 -> 7.1).
+//   launches   two[0] + two[1] K + two[2] M N K / 10^6 + (more than one tile of 32 x 32 per unit: two[3]) + two[4] N K / 10^4, FP8 + 1.5 M K / 65536
+// From a graph the choice would be best with the line where the tiles are 5 % ahead by that: one size in three, at 0.84 of the time in the mean; 0.7 % from
+// the faster way in the mean (1 % at 10 % ahead, 0.8 % at level).  A call that is not captured pays 2.4 us of the host's time for a launch, 7.5 us in all for
+// two: tiles of less than that are taken up to 5 % behind.  us from a graph, launches -> tiles, weights in the last-level cache | from HBM: bf16 32 x 2048 ->
+// 2048 5.7 -> 4.8 | 6.7 -> 5.1, 64 x 1024 -> 3072 6.1 -> 4.7 | 6.9 -> 5.0, 32 x 512 -> 8192 5.5 -> 4.6 | 6.4 -> 4.8, fp32 64 x 512 -> 2048 5.2 -> 4.2 | 5.8 -> 4.6; furthest off
+// fp32 64 x 2048 -> 2048 6.5 -> 7.5 | 7.3 -> 7.4 (not captured 8.1 -> 7.1); FP8 19 x 720 -> 6000, not captured, 8.9 -> 6.7.
 struct TiledCost {
   double start, row, weight, all, two[5];
 };
 static const TiledCost& tiled_cost(RowsKind kind) {
   static const TiledCost i8 = {3.07, 0.038, 0.038, 0, {5.27, 0.27, 4.1, 0.47, 0.79}}, norm = {3.24, 0.083, 0.033, 0, {5.49, 0.44, 4.78, 0.35, 1.38}},
-                         f32 = {3.26, 0.041, 0.042, 0, {4.74, 0.79, 4.33, 0.47, 0.92}}, f8 = {3.81, 0.054, 0.047, 0.018, {7.43, 0.32, 6.0, 0.38, 0.84}};
+                         f32 = {3.26, 0.041, 0.042, 0, {4.74, 0.79, 4.33, 0.47, 0.92}}, f8 = {3.81, 0.054, 0.047, 0.018, {5.35, 0.23, 4.11, 0.4, 1.14}};
   return kind == ROWS_I8 ? i8 : kind == ROWS_I8_NORM ? norm : kind == ROWS_I8_F32 ? f32 : f8;
 }
 struct Tiled {
@@ -569,13 +569,15 @@ static Tiled tiled_best(RowsKind kind, int64_t M, int64_t N, int64_t K) {
   return best;
 }
 bool gemv_rows_tiled_ok(RowsKind kind, int64_t M, int64_t N, int64_t K) {
-  // Tiles of more outputs than 80 to a compute unit never gained (64 x 512 -> 8192: 6.3 | 6.6), nor longer bf16 rows than 4096.
-  const int64_t most = kind == ROWS_I8_NORM ? 2048 : kind == ROWS_I8_F32 ? GX_MAX_K : 4096;
+  // Tiles of more outputs than 80 to a compute unit never gained (64 x 512 -> 8192: 6.3 | 6.6), nor longer bf16 rows than 4096 (FP8: 2048).
+  const int64_t most = kind == ROWS_I8_NORM || kind == ROWS_FP8 ? 2048 : kind == ROWS_I8_F32 ? GX_MAX_K : 4096;
   if (M <= 16 || (M + 15) / 16 * N > 80 * device_cus() || K > most) return false;
   const double* two = tiled_cost(kind).two;
   const double k = (double)K / 1024, nk = (double)N * k;
   const bool rounds = (M + 31) / 32 * ((N + 31) / 32) > device_cus();
-  return tiled_best(kind, M, N, K).us < 0.95 * (two[0] + two[1] * k + two[2] * M * nk / 1e6 + (rounds ? two[3] : 0) + two[4] * nk / 1e4);
+  const double cast = kind == ROWS_FP8 ? 1.5 * (double)(M * K < 98304 ? M * K : 98304) / 65536 : 0;  // by the tensor's size, up to where it takes two launches
+  const double us = tiled_best(kind, M, N, K).us, by_two = two[0] + cast + two[1] * k + two[2] * M * nk / 1e6 + (rounds ? two[3] : 0) + two[4] * nk / 1e4;
+  return us < (us < 7.5 ? 1.05 : 0.95) * by_two;
 }
 
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {
