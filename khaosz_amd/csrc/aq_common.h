@@ -463,10 +463,23 @@ inline int per_device(int (&cached)[64], int otherwise, F&& ask) {
 }
 
 // Compute units of the current device (launch shapes are sized by it: a partition mode that exposes fewer compute units
-// per device gets fewer workgroups).
+// per device gets fewer workgroups).  Where all devices of the process have as many, which one is current need not be asked: 55 ns
+// of the host's time, two to eight times a call.
 inline int device_cus() {
+  auto ask = [](int* v, int dev) { return hipDeviceGetAttribute(v, hipDeviceAttributeMultiprocessorCount, dev); };
+  static const int common = [&] {
+    int n = 0, all = 0;
+    if (hipGetDeviceCount(&n) != hipSuccess) return 0;
+    for (int dev = 0; dev < n; ++dev) {
+      int v = 0;
+      if (ask(&v, dev) != hipSuccess || v <= 0 || (all && v != all)) return 0;
+      all = v;
+    }
+    return all;
+  }();
+  if (common) return common;
   static int cached[64] = {};
-  return per_device(cached, 256, [](int* v, int dev) { return hipDeviceGetAttribute(v, hipDeviceAttributeMultiprocessorCount, dev); });
+  return per_device(cached, 256, ask);
 }
 
 }  // namespace aq
