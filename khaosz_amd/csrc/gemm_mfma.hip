@@ -18,8 +18,8 @@
 // workgroup barrier per K step.  The epilogue is fused and runs straight from
 // the accumulator registers: int32 store, or dequantise (+bias) and cast.
 // Two other kernels take calls from here: gemm_walk.hip the 256 x 128 and
-// 256 x 192 tiles of K from 512 (even N), gemm_slices.hip a few dozen to a few
-// hundred rows.
+// 256 x 192 tiles of K from 512 (even N), gemm_slices.hip up to a few hundred
+// rows.
 #include "aq_gemm.h"
 
 namespace aq {
