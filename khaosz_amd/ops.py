@@ -796,7 +796,7 @@ def linear_fp8(xq, sx, wq, sw, bias=None, out_dtype=torch.bfloat16, residual=Non
     if out_dtype not in _DT:
         raise ValueError(f"out_dtype {out_dtype} is not supported")
     wq, ld = wq.contiguous(), xq.stride(0)
-    if xq.stride(1) != 1 or ld < K or ld % 16 or M < 2 or xq.data_ptr() % 16:
+    if xq.stride(1) != 1 or ld < K or ld % 16 or ld > 1 << 22 or M < 2 or xq.data_ptr() % 16:  # 2^22: the kernels' 32-bit offsets
         xq, ld = xq.contiguous(), K
     b, bdt = _bias_args(bias, N)
     r = _residual_arg(residual, M, N, out_dtype, xq.device)

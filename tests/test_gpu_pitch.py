@@ -124,6 +124,18 @@ def test_distances_that_are_refused():
         ops.quant_tensor_fp8(x.view(-1), pitch=128)
 
 
+@pytest.mark.parametrize("M,N,K,step", [(3, 48, 64, 1 << 23), (3, 48, 64, (1 << 22) + 16), (3, 48, 64, 1 << 22), (40, 300, 1040, 4176), (40, 300, 1040, 1048)])
+def test_codes_whose_rows_lie_anywhere(M, N, K, step):
+    """Rows up to and beyond the distance that the entry point takes, and rows that are no multiple of 16 bytes apart: codes that the kernels
+    cannot read in place are copied, as they always were."""
+    a, w = _codes(M, K, True, 9), _codes(N, K, True, 10)
+    rows = torch.empty((M - 1) * step + K, dtype=torch.uint8, device=DEV).as_strided((M, K), (step, 1))
+    rows.copy_(a)
+    one = torch.full((1,), 0.01, device=DEV)
+    for out in (BF16, F32):
+        assert torch.equal(ops.linear_fp8(rows, one, w, one, None, out_dtype=out), ops.linear_fp8(a, one, w, one, None, out_dtype=out))
+
+
 @pytest.mark.parametrize("M,N,K", [(40, 6000, 1040), (300, 1601, 2064), (2100, 1040, 4016), (1500, 2048, 1024)])
 def test_layers_give_the_bits_of_their_operators(M, N, K):
     """(2100 x 4016 bf16 values: the FP8 quantiser's one-launch form)"""
