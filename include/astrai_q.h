@@ -223,9 +223,9 @@ int aq_gemv_fp8_decode_residual(const void *x, int x_dtype, const uint8_t *wq, c
 /* Codes in rows that begin ldx (ldq) bytes apart, at least K and a multiple of 16: the quantisers that write them and
  * the Linears that take them (otherwise aq_quant_rowwise_i8, aq_quant_tensor_fp8(_onepass) of M * K elements,
  * aq_linear_w8a8_residual and aq_linear_fp8_residual).  With rows that begin on 128-byte lines the tiled kernels bring in
- * half as many lines of them: aq_linear_codes_pitch is the distance to take for a Linear of M > 16 rows, K or the next
- * multiple of 128. */
-int64_t aq_linear_codes_pitch(int fp8, int64_t M, int64_t N, int64_t K);
+ * half as many lines of them: aq_linear_codes_pitch is the distance to take for a Linear of M > 16 rows, with a residual or
+ * without, K or the next multiple of 128. */
+int64_t aq_linear_codes_pitch(int fp8, int residual, int64_t M, int64_t N, int64_t K);
 int aq_quant_rowwise_i8_strided(const void *x, int x_dtype, int64_t M, int64_t K, int64_t ldx, int8_t *q, int64_t ldq,
                                 float *scale, void *stream);
 int aq_quant_tensor_fp8_strided(const void *x, int x_dtype, int64_t M, int64_t K, uint8_t *q, int64_t ldq,

@@ -71,7 +71,7 @@ SYMBOLS = {
                                      _i64, _i64, _vp]),
     "aq_gemv_w8a8_decode_one_launch": (_int, [_int, _int, _i64, _i64, _i64]),
     "aq_gemv_fp8_decode_one_launch": (_int, [_int, _i64, _i64]),
-    "aq_linear_codes_pitch": (_i64, [_int, _i64, _i64, _i64]),
+    "aq_linear_codes_pitch": (_i64, [_int, _int, _i64, _i64, _i64]),
     "aq_quant_rowwise_i8_strided": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _vp]),
     "aq_quant_tensor_fp8_strided": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _vp, _vp, _sz, _vp]),
     "aq_quant_tensor_fp8_onepass_strided": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _vp, _vp, _sz, _vp]),

@@ -1230,10 +1230,13 @@ extern "C" int aq_linear_fp8_strided(const uint8_t* xq, int64_t ldx, const float
 // of the activations are written here, to rows that begin on lines.  us, K apart -> whole lines (all rows on lines, weights too): 798 x 4704 -> 1648 19.4 -> 16.2
 // (13.9), 333 x 6896 -> 1536 18.5 -> 14.9 (12.6), 2048 x 6896 -> 1536 35.3 -> 30.0 (25.0), 4096 x 2032 -> 11264 108 -> 92.5 (89.4), 7601 x 4272 -> 1096 47.7 ->
 // 44.9 (40.5), FP8 4958 x 1264 -> 6288 51.2 -> 43.2, 952 x 3392 -> 1392 13.2 -> 11.8 (10.8); level with few rows (64 x 2032 -> 2048 4.2).  Not where the
-// 256 x 256 FP8 tile serves, whose 64-byte steps halve no line, nor the weight-streaming kernel, which takes rows as they are.
-extern "C" int64_t aq_linear_codes_pitch(int fp8, int64_t M, int64_t N, int64_t K) {
-  if (M <= 16 || N < 1 || K < 1 || K % 16 || K % 128 == 0 || K > (1 << 22) - 128 || M > (1 << 30) || M * K / 8 > (int64_t)0x7fffffff) return K;
-  if (aq::streams_weights(M, N, K)) return K;
+// 256 x 256 FP8 tile serves, whose 64-byte steps halve no line (with a residual it does not: 4864 x 3264 -> 8640 148.7 -> 132.8, 8192 x 8128 -> 8192 583 -> 486),
+// nor the weight-streaming kernel, which takes rows as they are.  Nor what the quantisers do not write in rows: more than 2^31 vectors of 16 bytes,
+// of which fp32 rows have K / 4.  Nor where the gaps alone take the codes past the 31-bit offsets of the kernel that walks tiles.
+extern "C" int64_t aq_linear_codes_pitch(int fp8, int residual, int64_t M, int64_t N, int64_t K) {
+  if (M <= 16 || N < 1 || K < 1 || K % 16 || K % 128 == 0 || K > (1 << 22) - 128 || M > (1 << 30) || M * K / 4 > (int64_t)0x7fffffff) return K;
+  const int64_t pitch = (K + 127) / 128 * 128, reach = aq::OOB_OFFSET;
+  if (aq::streams_weights(M, N, K) || (M * pitch > reach && M * K <= reach)) return K;
   aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
-  return fp8 && aq::huge_fp8_ok(a, aq::device_cus()) ? K : (K + 127) / 128 * 128;
+  return fp8 && !residual && aq::huge_fp8_ok(a, aq::device_cus()) ? K : pitch;
 }

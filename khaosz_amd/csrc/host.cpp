@@ -623,7 +623,7 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   shape.back() = N;
   Tensor y = c.empty(shape, type);
   // codes and scales of the tokens (and, for FP8, the partial maxima); the codes of a tile's rows begin on lines
-  const int64_t pitch = few || gain ? r.K : lib.aq_linear_codes_pitch(fp8, r.M, N, r.K);
+  const int64_t pitch = few || gain ? r.K : lib.aq_linear_codes_pitch(fp8, res != nullptr, r.M, N, r.K);
   const int64_t codes = !few  ? (r.M * pitch + 255) & ~int64_t(255)
                         : fp8 ? static_cast<int64_t>(lib.aq_gemv_fp8_workspace_bytes(r.M, r.K))
                               : static_cast<int64_t>(lib.aq_gemv_w8a8_workspace_bytes(r.M, r.K));

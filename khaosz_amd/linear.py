@@ -380,7 +380,7 @@ class Fp8Linear(_NativeCall):
             if x2.numel() * x2.element_size() >= ops.FP8_ONEPASS_MIN_BYTES:  # quantised in one launch
                 ops._need_gpu(x, wq)
                 state = self._quant_states.get(x.device, lambda: ops.fp8_onepass_state(x.device))
-                pitch = ops.codes_pitch(x2.size(0), n, k, True)
+                pitch = ops.codes_pitch(x2.size(0), n, k, True, residual is not None)
                 if pitch != k:
                     rows = {"pitch": pitch}
             xq, sx = ops.quant_tensor_fp8(x2, state=state, **rows)

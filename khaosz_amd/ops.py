@@ -182,9 +182,9 @@ def fp8_onepass_state(device) -> torch.Tensor:
     return torch.zeros((_abi.AQ_FP8_ONEPASS_WS_BYTES // 8,), dtype=torch.int64, device=device)
 
 
-def codes_pitch(M: int, N: int, K: int, fp8: bool) -> int:
-    """Bytes between the rows of the codes that a Linear ``[M, K] -> [M, N]`` reads fastest: K, or the next multiple of 128."""
-    return _abi.load().aq_linear_codes_pitch(int(fp8), M, N, K)
+def codes_pitch(M: int, N: int, K: int, fp8: bool, residual: bool = False) -> int:
+    """Bytes between the rows of the codes that a Linear ``[M, K] -> [M, N]`` reads fastest, K or the next multiple of 128."""
+    return _abi.load().aq_linear_codes_pitch(int(fp8), int(residual), M, N, K)
 
 
 def quant_tensor_fp8(x: torch.Tensor, state: Optional[torch.Tensor] = None,

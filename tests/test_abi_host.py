@@ -315,6 +315,23 @@ def test_gemm_tile_choice_where_tiles_are_walked_or_k_is_cut():
     assert pick(333, 1536, 6912, res=1) == 65
 
 
+def test_the_distance_between_rows_of_codes_is_one_that_their_quantiser_writes():
+    """Rows on 128-byte lines where the quantisers write them (fewer than 2^31 vectors of four fp32 values) and the kernels take them as
+    well as rows without a gap (31-bit offsets of the walked tiles); the 256 x 256 FP8 tile, which no residual takes, reads them as they are."""
+    pitch = lambda M, N, K, fp8=1, res=0: _abi.load().aq_linear_codes_pitch(fp8, res, M, N, K)
+    assert pitch(300, 1500, 1040) == 1152 and pitch(300, 1500, 1040, fp8=0) == 1152
+    assert pitch(300, 1500, 1024) == 1024 and pitch(16, 1500, 1040) == 1040 and pitch(20, 1500, 0) == 0
+    most = (1 << 33) // 8176  # rows of 8176 with fewer than 2^31 vectors of fp32
+    for fp8 in (0, 1):
+        assert pitch(most, 2048, 8176, fp8) == 8192 and pitch(most + 1, 2048, 8176, fp8) == 8176 and pitch(1100000, 2048, 8176, fp8) == 8176
+    reach = 0x7ffffff0
+    for M, want in ((reach // 7168, 7168), (reach // 7168 + 1, 7152), (reach // 7152, 7152), (reach // 7152 + 1, 7168)):
+        assert pitch(M, 2048, 7152) == want and pitch(M, 2048, 7152, fp8=0) == want
+    assert pitch(4864, 8640, 3264) == 3264 and pitch(4864, 8640, 3264, res=1) == 3328 and pitch(4864, 8640, 3264, fp8=0) == 3328
+    for M in (0, -1, 1 << 31):
+        assert pitch(M, 2048, 1040) == 1040
+
+
 def test_quant_tensor_fp8_refuses_a_workspace_smaller_than_its_slots():
     """aq_quant_tensor_fp8 writes AQ_FP8_AMAX_WS_BYTES of partial maxima: a smaller workspace is refused before
     anything is launched (argument checks only: runs without a GPU)."""
