@@ -96,7 +96,11 @@ __device__ __forceinline__ typename Acc<FP8>::type mma(const typename Frag<FP8>:
 }
 
 // gemm_slices.hip: small tiles, K cut among a workgroup's wavefronts
-enum SlicesTile { SLICES_16X16 = 1, SLICES_16X32, SLICES_16X64, SLICES_32X16, SLICES_32X32, SLICES_48X32, SLICES_32X48, SLICES_64X32, SLICES_32X64, SLICES_48X48 };
+// (numbered on from gemm_mfma.hip's TileKind)
+enum SlicesTile {
+  SLICES_FIRST = 34, SLICES_32X32 = SLICES_FIRST, SLICES_64X32, SLICES_48X32, SLICES_32X48, SLICES_32X64, SLICES_48X48, SLICES_16X16, SLICES_16X32,
+  SLICES_32X16, SLICES_16X64, SLICES_LAST = SLICES_16X64
+};
 int gemm_slices_tile(int64_t M, int64_t N, int64_t K, int64_t cus);
 template <bool FP8, int OUT>
 int gemm_slices_launch(GemmArgs& a, int tile, hipStream_t st);

@@ -15,15 +15,15 @@ extern "C" {
 
 /* Forces the GEMM workgroup tile for every later GEMM call of this process through the lab
  * library: 32 (128 x 32), 33 (64 x 32), 64 (128 x 64), 65 (64 x 64), 128 (128 x 128), 129 (128 x 128 on
- * wavefront pairs that split every K step: lab build only), 256 (256 x 128), 258 and 192 (256 x 128 and 256 x 192 of the kernel that walks its tiles,
- * where it can take the call), 0 = by shape.  Process-wide and
- * unsynchronised -- which is why it does not exist in the product library. */
+ * wavefront pairs that split every K step: lab build only), 34 to 43 (K cut among the wavefronts: 32 x 32,
+ * 64 x 32, 48 x 32, 32 x 48, 32 x 64, 48 x 48, 16 x 16, 16 x 32, 32 x 16, 16 x 64), 256 (256 x 128), 258 and 192
+ * (256 x 128 and 256 x 192 of the kernel that walks its tiles, where it can take the call), 0 = by shape.
+ * Process-wide and unsynchronised -- which is why it does not exist in the product library. */
 int aq_lab_set_gemm_tile(int rows);
 
 /* The tile with which the library multiplies M x K by N x K codes (y_dtype AQ_F32, AQ_BF16, or -1 for int32 sums; residual: whether
- * there is one) on a device of `compute_units` compute units, in the numbering above, with 34 and 35 (32 x 32 and 64 x 32, K cut
- * among the wavefronts) and 512 (256 x 256).  A pure function of its arguments: no device is touched.  (Calls of few rows that
- * a weight-streaming kernel takes do not get here.) */
+ * there is one) on a device of `compute_units` compute units, in the numbering above and 512 (256 x 256).  A pure function of its
+ * arguments: no device is touched.  (Calls of few rows that a weight-streaming kernel takes do not get here.) */
 int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8, int y_dtype, int residual, int compute_units);
 
 /* Clock counters the lab build's tiled GEMM leaves behind (wavefront 0 of workgroup 0 of the LAST GEMM launch that

@@ -922,9 +922,7 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
 // 6 % of it.  The small tiles are for launches of a few rounds only.
 enum TileKind {
   TILE_AUTO = 0, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129, TILE_WIDE = 192,
-  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258,
-  TILE_SLICES32 = 34, TILE_SLICES64 = 35, TILE_SLICES48X32 = 36, TILE_SLICES32X48 = 37, TILE_SLICES32X64 = 38, TILE_SLICES48 = 39,
-  TILE_SLICES16 = 40, TILE_SLICES16X32 = 41, TILE_SLICES32X16 = 42, TILE_SLICES16X64 = 43
+  TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258  // and SlicesTile's
 };
 #ifdef AQ_LAB
 static int g_forced_tile = 0;  // lab build only: TILE_AUTO = by shape, otherwise forced (tuning and tests)
@@ -1023,7 +1021,7 @@ static bool huge_fp8_ok(const GemmArgs& a, int64_t cus) {
   return tiles >= 2 * cus && (tiles % cus == 0 || 2 * (tiles % cus) > cus);
 }
 
-// The tile that takes a call on a device of `cus` compute units.  TILE_WALK and TILE_WIDE: of gemm_walk_kernel, TILE_SLICES..: of
+// The tile that takes a call on a device of `cus` compute units.  TILE_WALK and TILE_WIDE: of gemm_walk_kernel, a SlicesTile: of
 // gemm_slices_kernel.
 static int choose_tile(const GemmArgs& a, bool fp8, int out, int64_t cus) {
   if (fp8 && out != OUT_I32 && huge_fp8_ok(a, cus)) return TILE_HUGE;
@@ -1031,19 +1029,8 @@ static int choose_tile(const GemmArgs& a, bool fp8, int out, int64_t cus) {
   const int tile = choose_tile_for(a.M, a.N, cus, walk, a.res != nullptr);
   if (walk && tile == TILE_LARGE) return TILE_WALK;
   if (tile == TILE_WIDE || out == OUT_I32) return tile;
-  switch (gemm_slices_tile(a.M, a.N, a.K, cus)) {
-    case SLICES_16X16: return TILE_SLICES16;
-    case SLICES_16X32: return TILE_SLICES16X32;
-    case SLICES_16X64: return TILE_SLICES16X64;
-    case SLICES_32X16: return TILE_SLICES32X16;
-    case SLICES_32X32: return TILE_SLICES32;
-    case SLICES_48X32: return TILE_SLICES48X32;
-    case SLICES_32X48: return TILE_SLICES32X48;
-    case SLICES_64X32: return TILE_SLICES64;
-    case SLICES_32X64: return TILE_SLICES32X64;
-    case SLICES_48X48: return TILE_SLICES48;
-  }
-  return tile;
+  const int slices = gemm_slices_tile(a.M, a.N, a.K, cus);
+  return slices ? slices : tile;
 }
 
 template <bool FP8, int OUT>
@@ -1060,17 +1047,8 @@ static int launch(GemmArgs& a, hipStream_t st) {
     switch (tile) {
       case TILE_WALK: return gemm_walk_launch<FP8, OUT>(a, st, 128);
       case TILE_WIDE: return gemm_walk_launch<FP8, OUT>(a, st, 192);
-      case TILE_SLICES16: return gemm_slices_launch<FP8, OUT>(a, SLICES_16X16, st);
-      case TILE_SLICES16X32: return gemm_slices_launch<FP8, OUT>(a, SLICES_16X32, st);
-      case TILE_SLICES16X64: return gemm_slices_launch<FP8, OUT>(a, SLICES_16X64, st);
-      case TILE_SLICES32X16: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X16, st);
-      case TILE_SLICES32: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X32, st);
-      case TILE_SLICES48X32: return gemm_slices_launch<FP8, OUT>(a, SLICES_48X32, st);
-      case TILE_SLICES32X48: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X48, st);
-      case TILE_SLICES64: return gemm_slices_launch<FP8, OUT>(a, SLICES_64X32, st);
-      case TILE_SLICES32X64: return gemm_slices_launch<FP8, OUT>(a, SLICES_32X64, st);
-      case TILE_SLICES48: return gemm_slices_launch<FP8, OUT>(a, SLICES_48X48, st);
     }
+    if (tile >= SLICES_FIRST && tile <= SLICES_LAST) return gemm_slices_launch<FP8, OUT>(a, tile, st);
     if constexpr (FP8)
       if (tile == TILE_HUGE) return launch_shape<FP8, OUT, ShapeHuge>(a, st);
   }
@@ -1120,7 +1098,7 @@ extern "C" int aq_lab_read_clock(long long* host2) {
   return (int)hipMemcpyFromSymbol(host2, HIP_SYMBOL(aq::aq_lab_clock), 64);
 }
 extern "C" int aq_lab_set_gemm_tile(int rows) {
-  if (rows != 192 && rows != 258 && (rows < 34 || rows > 43) && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
+  if (rows != 192 && rows != 258 && (rows < aq::SLICES_FIRST || rows > aq::SLICES_LAST) && rows != 0 && rows != 129 && rows != 33 && rows != 65 && rows != 64 && rows != 32 && rows != 128 && rows != 256 && rows != 257 && rows != 512 && rows != 513) return AQ_E_SHAPE;
   aq::g_forced_tile = rows;
   return AQ_OK;
 }
@@ -1130,10 +1108,7 @@ extern "C" int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8,
   static const char some = 0;
   aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
   a.res = residual ? &some : nullptr;  // only whether there is one
-  const int tile = aq::choose_tile(a, fp8 != 0, y_dtype < 0 ? aq::OUT_I32 : y_dtype == AQ_BF16 ? aq::OUT_BF16 : aq::OUT_F32, compute_units);
-  // tiles with K cut: 32 x 32 stands for the smaller ones too, the larger tile whose place 48 x 48 take for both
-  if (tile == aq::TILE_SLICES16 || tile == aq::TILE_SLICES16X32 || tile == aq::TILE_SLICES32X16) return aq::TILE_SLICES32;
-  return tile == aq::TILE_SLICES48 ? aq::choose_tile_for(M, N, compute_units) : tile;
+  return aq::choose_tile(a, fp8 != 0, y_dtype < 0 ? aq::OUT_I32 : y_dtype == AQ_BF16 ? aq::OUT_BF16 : aq::OUT_F32, compute_units);
 }
 #endif
 

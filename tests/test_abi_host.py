@@ -292,7 +292,7 @@ def test_gemm_tile_choice_for_the_benchmark_shapes_and_a_few_hundred_rows():
 
 def test_gemm_tile_choice_where_tiles_are_walked_or_k_is_cut():
     """What a Linear's launch takes on 256 compute units: walked tiles of 256 x 128 (258) or 256 x 192 (192) with K from 512 and an even
-    N, tiles with K cut among the wavefronts (34, 35) for few rows, 256 x 256 (512) for some FP8 launches, else the tile above."""
+    N, tiles with K cut among the wavefronts (34 to 43) for few rows, 256 x 256 (512) for some FP8 launches, else the tile above."""
     lab = _abi.load_lab()
     f32, bf16 = _abi.AQ_F32, _abi.AQ_BF16
     pick = lambda M, N, K, fp8=0, out=bf16, res=0: lab.aq_lab_choose_gemm_tile(M, N, K, fp8, out, res, 256)
@@ -311,8 +311,12 @@ def test_gemm_tile_choice_where_tiles_are_walked_or_k_is_cut():
                          (8192, 8192, 8192, 0)):
         assert pick(M, N, K, fp8=1, res=res) in (192, 258)
     # K cut among the wavefronts; a tile too many for that
-    assert pick(64, 2048, 2048, out=f32) == 34 and pick(200, 2048, 6912) == 35 and pick(200, 2048, 1520) == 33
-    assert pick(333, 1536, 6912, res=1) == 65
+    assert pick(64, 2048, 2048, out=f32) == 41 and pick(200, 2048, 6912) == 35 and pick(200, 2048, 1520) == 33
+    assert pick(333, 1536, 6912, res=1) == 39
+    # the smallest of which 256 are enough: 16 x 16, 16 x 32, 16 x 64 (up to 16 rows; then 16 x 32 in rounds), 32 x 16, 32 x 32
+    for M, N, tile in ((16, 4096, 40), (16, 4097, 41), (16, 8192, 41), (16, 8193, 43), (16, 16384, 43), (16, 16385, 41), (17, 2048, 40), (17, 2049, 41),
+                       (32, 4096, 41), (32, 4097, 34), (2100, 48, 42), (33, 1360, 40), (33, 1361, 41), (64, 4096, 34), (64, 4097, 37)):
+        assert pick(M, N, 1040) == pick(M, N, 1040, fp8=1, out=f32, res=1) == tile
 
 
 def test_the_distance_between_rows_of_codes_is_one_that_their_quantiser_writes():

@@ -21,7 +21,7 @@ def _codes(rows, K, fp8, seed):
 
 
 # tile by tile (lab numbering) as the library picks them on 256 compute units: K of no whole number of 128-byte lines, ragged M and N
-TILES = [(34, 40, 130, 1040), (36, 200, 1500, 1616), (37, 60, 6000, 272), (38, 70, 5000, 1040), (35, 200, 2048, 1616), (33, 200, 2048, 272), (65, 330, 1536, 1040), (64, 700, 1600, 2064),
+TILES = [(40, 40, 130, 1040), (41, 60, 1800, 1040), (42, 2100, 48, 1040), (43, 9, 12000, 1040), (34, 100, 2000, 1040), (39, 330, 1600, 3088), (36, 200, 1500, 1616), (37, 60, 6000, 272), (38, 70, 5000, 1040), (35, 200, 2048, 1616), (33, 200, 2048, 272), (65, 330, 1536, 1040), (64, 700, 1600, 2064),
          (128, 1500, 1537, 336), (258, 2000, 2050, 1040), (192, 4000, 3070, 528), (256, 4097, 2049, 624), (258, 6000, 8186, 1008)]
 
 

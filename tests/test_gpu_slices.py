@@ -48,14 +48,14 @@ def test_tiles_of_sixteens(oracle, M, N, K, kind):
 
 # Both sides of the rule's lines on 256 compute units: 256 tiles of a shape and a few more, K 512 and 3072, 64 rows
 @pytest.mark.parametrize("M,N,K,tile", [(64, 4096, 528, 34), (96, 4096, 528, 36), (97, 2752, 528, 37), (64, 4097, 528, 37), (64, 8192, 528, 33),
-                                        (65, 4100, 512, 38), (65, 4100, 496, 65), (32, 12288, 272, 37), (333, 1536, 3072, None),
-                                        (333, 1536, 3056, None), (336, 1776, 3088, None), (336, 1777, 3088, None), (64, 6145, 3088, 35), (16, 4096, 528, 34), (16, 4097, 528, 34),
-                                        (33, 1360, 528, 34), (9, 8193, 528, 43), (3, 16385, 272, 34), (32, 2048, 1040, 34), (17, 4097, 1040, 34)])
+                                        (65, 4100, 512, 38), (65, 4100, 496, 65), (32, 12288, 272, 37), (333, 1536, 3072, 39),
+                                        (333, 1536, 3056, 65), (336, 1728, 3088, 39), (336, 1729, 3088, 65), (64, 6145, 3088, 35), (16, 4096, 528, 40),
+                                        (16, 4097, 528, 41), (33, 1360, 528, 40), (33, 1361, 528, 41), (9, 8193, 528, 43), (3, 16385, 272, 41),
+                                        (32, 2048, 1040, 40), (32, 2049, 1040, 41), (17, 4097, 1040, 34), (2100, 48, 528, 42)])
 def test_the_rule_for_tiles_of_sixteens(M, N, K, tile):
     """Whichever tile the rule takes, int8 sums are the bits of the 64 x 64 tile; FP8 sums differ by their order alone: fp32 sums of K
     products by at most 2 K 2^-24 of the sum of their magnitudes, bf16 results by a rounding more."""
-    if tile is not None:
-        assert _abi.load_lab().aq_lab_choose_gemm_tile(M, N, K, 0, _abi.AQ_BF16, 0, 256) == tile
+    assert _abi.load_lab().aq_lab_choose_gemm_tile(M, N, K, 0, _abi.AQ_BF16, 0, 256) == tile
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     xq, wq = (torch.randint(-128, 128, (n, K), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
     sx, sw = (torch.rand(n, generator=g, device=DEV) * 0.01 + 1e-4 for n in (M, N))
