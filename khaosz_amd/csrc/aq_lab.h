@@ -22,8 +22,8 @@ extern "C" {
 int aq_lab_set_gemm_tile(int rows);
 
 /* The tile with which the library multiplies M x K by N x K codes (y_dtype AQ_F32, AQ_BF16, or -1 for int32 sums; residual: whether
- * there is one) on a device of `compute_units` compute units, in the numbering above and 512 (256 x 256).  A pure function of its
- * arguments: no device is touched.  (Calls of few rows that a weight-streaming kernel takes do not get here.) */
+ * there is one) on a device of `compute_units` compute units, in the numbering above, 512 (256 x 256) and 31 (the weight-streaming
+ * kernel for 17 to 32 rows).  A pure function of its arguments: no device is touched. */
 int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8, int y_dtype, int residual, int compute_units);
 
 /* Clock counters the lab build's tiled GEMM leaves behind (wavefront 0 of workgroup 0 of the LAST GEMM launch that

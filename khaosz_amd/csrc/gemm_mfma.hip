@@ -921,7 +921,7 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
 // 33..2048 rows against N = 1024..16384 and K = 1024..5632, where the rule picks the fastest shape or one within
 // 6 % of it.  The small tiles are for launches of a few rounds only.
 enum TileKind {
-  TILE_AUTO = 0, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129, TILE_WIDE = 192,
+  TILE_AUTO = 0, TILE_STREAMS = 31 /* no tile: gemv.hip's */, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129, TILE_WIDE = 192,
   TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258  // and SlicesTile's
 };
 #ifdef AQ_LAB
@@ -1080,6 +1080,14 @@ static int check_gemm(const void* A, const void* B, const void* C, int64_t M, in
   return AQ_OK;
 }
 
+// 17..32 rows, in whole lines, of more outputs than tiles cut among wavefronts serve: the weight-streaming kernel takes them.  Not 16 rows and fewer, however long: us, weights in the last-level cache | from HBM, the weight-streaming
+// kernel -> tiles of 16 x 64 or 16 x 32: 16 x 11008 -> 8200 29.5 -> 20.6 | 29.2 -> 26.5, -> 12288 35.0 -> 26.6 | 34.8 -> 35.6, -> 20000 62.8 -> 36.8 | 63.3 ->
+// 49.5, -> 32000 73.4 -> 65.9 | 74.7 -> 67.8; 8 x 20480 -> 8200 50.6 -> 29.1 | 49.7 -> 42.6; of 119 sizes the slowest 16 x 14336 -> 32000 74.3 -> 79.6 and,
+// from HBM, 9 x 16384 -> 16384 49.7 -> 53.7.
+static bool streams_weights(int64_t M, int64_t N, int64_t K, int64_t cus) {
+  return M > 16 && M <= 32 && K % 128 == 0 && !gemm_slices_tile(M, N, K, cus);
+}
+
 static GemmArgs make_args(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K) {
   GemmArgs a{};
   a.A = static_cast<const uint8_t*>(A);
@@ -1105,6 +1113,7 @@ extern "C" int aq_lab_set_gemm_tile(int rows) {
 extern "C" int aq_lab_choose_gemm_tile(int64_t M, int64_t N, int64_t K, int fp8, int y_dtype, int residual, int compute_units) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 16 || M > (1 << 30) || N > (1 << 20) || K > (1 << 22) || compute_units <= 0) return AQ_E_SHAPE;
   if ((fp8 && y_dtype < 0) || (y_dtype >= 0 && y_dtype != AQ_F32 && y_dtype != AQ_BF16) || (y_dtype < 0 && residual)) return AQ_E_DTYPE;
+  if (y_dtype >= 0 && aq::streams_weights(M, N, K, compute_units)) return aq::TILE_STREAMS;
   static const char some = 0;
   aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
   a.res = residual ? &some : nullptr;  // only whether there is one
@@ -1128,20 +1137,10 @@ extern "C" int aq_linear_w8a8(const int8_t* xq, const float* sx, const int8_t* w
 
 namespace aq {
 // gemv.hip: the weight-streaming kernel for 17..32 rows (same sums, same epilogue: same bits)
-bool gemv_tokens_ok(int64_t M, int64_t N, int64_t K);
 int gemv_tokens_launch(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw, const void* bias,
                        int bias_dtype, const void* residual, void* y, int y_dtype, int64_t M, int64_t N, int64_t K,
                        hipStream_t st, bool fp8);
 
-// 17..32 rows of more outputs than tiles cut among wavefronts serve (and decode batches of as many whose rows are too long for the GEMV
-// kernels): the weight-streaming kernel takes them (not when a test has forced a tile shape)
-static bool streams_weights(int64_t M, int64_t N, int64_t K) {
-#ifdef AQ_LAB
-  if (g_forced_tile) return false;
-#endif
-  const int64_t cus = device_cus();
-  return (M <= 16 ? (N + 31) / 32 > cus : !gemm_slices_tile(M, N, K, cus)) && gemv_tokens_ok(M, N, K);
-}
 }  // namespace aq
 
 namespace aq {
@@ -1156,7 +1155,11 @@ static int linear_codes(bool fp8, const void* xq, int64_t ldx, const float* sx, 
   if (!sx || !sw) return AQ_E_NULL;
   if (check_ptr(sx, 4) || check_ptr(sw, 4) || check_ptr(bias, bias_dtype == AQ_BF16 ? 2 : 4) || check_ptr(residual, 4)) return AQ_E_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (ldx == K && streams_weights(M, N, K) && check_ptr16(residual) == 0)
+  bool streams = ldx == K && streams_weights(M, N, K, device_cus()) && check_ptr16(residual) == 0;
+#ifdef AQ_LAB
+  streams = streams && !g_forced_tile;
+#endif
+  if (streams)
     return gemv_tokens_launch(static_cast<const int8_t*>(xq), sx, static_cast<const int8_t*>(wq), sw, bias, bias_dtype, residual, y, y_dtype, M, N, K,
                               st, fp8);
   GemmArgs a = make_args(xq, wq, y, M, N, K);
@@ -1211,7 +1214,7 @@ extern "C" int aq_linear_fp8_strided(const uint8_t* xq, int64_t ldx, const float
 extern "C" int64_t aq_linear_codes_pitch(int fp8, int residual, int64_t M, int64_t N, int64_t K) {
   if (M <= 16 || N < 1 || K < 1 || K % 16 || K % 128 == 0 || K > (1 << 22) - 128 || M > (1 << 30) || M * K / 4 > (int64_t)0x7fffffff) return K;
   const int64_t pitch = (K + 127) / 128 * 128, reach = aq::OOB_OFFSET;
-  if (aq::streams_weights(M, N, K) || (M * pitch > reach && M * K <= reach)) return K;
+  if (aq::streams_weights(M, N, K, aq::device_cus()) || (M * pitch > reach && M * K <= reach)) return K;
   aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
   return fp8 && !residual && aq::huge_fp8_ok(a, aq::device_cus()) ? K : pitch;
 }

@@ -598,18 +598,17 @@ static bool gemv_swiglu_ok(int64_t M, int64_t F, int64_t K) {
 // ---------------------------------------------------------------------------
 // 17..32 tokens on codes: the same weight stream (every weight byte HBM -> registers once, operands assembled by
 // one DPP rotation per dword) with TG = 2 groups of 16 tokens multiplied against each weight fragment: a bandwidth-bound
-// launch for matrices of more 32-row blocks than compute units, where the GEMM whose wavefronts share K would take a second
-// round of tiles (at one tile per compute unit it is the faster one).  Also decode batches of as many outputs whose rows are too long
-// for the kernels above.  From 33
+// launch for matrices of more than 48 outputs to a compute unit, where the GEMM whose wavefronts share K would take a second
+// round of tiles (at one tile per compute unit it is the faster one).  From 33
 // tokens on, with a third and fourth token group, it was the slower one (48 rows: 6.1 us, 64 rows: 7.6 us with the weights
 // in the last-level cache, where a 128 x 32 tile took 5.8 us).  Same integer sums, same epilogue: the bits of the tiled GEMM.
-// K is walked in chunks of 1024 bytes per wavefront (KS wavefronts per row group: 1024-, 2048- or 4096-byte chunks
+// K is walked in chunks of 1024 bytes per wavefront (KS wavefronts per row group: 1024- or 2048-byte chunks
 // per workgroup), the token codes of one chunk at a time in LDS, so that rows of any length are taken (an MLP's
 // down projection) and the LDS of a compute unit holds several workgroups.  A chunk's codes are requested into
 // registers while the chunk before is multiplied and stored between two barriers; the weight stream runs through
 // the chunk boundaries untouched (two register batches, each reloaded as soon as it has been consumed).  GRP row
-// groups of 16 rows per workgroup (every workgroup copies all token codes from L2: more rows per workgroup for
-// matrices of more 32-row blocks than compute units); rows must be whole 128-byte lines (K % 128 == 0).
+// groups of 16 rows per workgroup (every workgroup copies all token codes from L2); rows must be whole 128-byte lines
+// (K % 128 == 0).
 // FP8: e4m3 codes with one scale per tensor, v_mfma_f32_16x16x128_f8f6f4 and fp32 accumulation (chunks and K parts
 // summed in a fixed order).
 template <int TG, int KS, bool RES, int GRP = 2, bool FP8 = false>
@@ -798,21 +797,11 @@ __global__ __launch_bounds__(KS * GRP * 64) void gemv_mfma_tokens_kernel(GemvArg
   }
 }
 
-// Shapes the token-group kernel takes: 17..32 rows of whole 128-byte lines, and the decode batch sizes whose rows
-// are too long for the GEMV kernels' own LDS budget (9..16 rows beyond 10 096 bytes, 5..8 beyond 20 208, ...),
-// where the tiles were the only path (12 x 4096 x 11008: 41 us against 19 us).  int8 and FP8 codes alike.
-bool gemv_tokens_ok(int64_t M, int64_t N, int64_t K) {
-  if (M < 1 || M > 32 || N <= 0 || (K % 128) != 0 || K > (1 << 22)) return false;
-  if (M <= 16) {
-    const int64_t mt = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
-    return mt * K + 64 + 2048 > GV_MAX_LDS;  // the GEMV kernels' own limit (gemv_check)
-  }
-  return true;
-}
-
-template <int KS, int GRP>
+// A launch of the token-group kernel: 64 weight rows per workgroup, half the copies of the token codes (32 x 16384 x 2048: 7.0 us
+// against 7.4 us with 32), in chunks no longer than the rows, 1024 or 2048 bytes.
+template <int KS>
 static int launch_gemv_tokens_shape(const GemvArgs& a, hipStream_t st, bool fp8) {
-  constexpr int TG = 2;
+  constexpr int TG = 2, GRP = 4;
   const unsigned grid = (unsigned)((a.N + GRP * GM_ROWS - 1) / (GRP * GM_ROWS));
   const size_t lds = (size_t)16 * TG * (1024 * KS + 16) + 16;
   using kern_t = void (*)(GemvArgs);
@@ -825,18 +814,7 @@ static int launch_gemv_tokens_shape(const GemvArgs& a, hipStream_t st, bool fp8)
   return (int)hipGetLastError();
 }
 
-// Chunk and workgroup shapes.  Two kinds of call come here: 17..32 rows of more 32-row blocks than compute units (fewer take
-// the GEMM whose wavefronts share K), and 16 rows or fewer whose rows are too long for the GEMV kernels, 9.9 KB and more.
-//   * more 32-row blocks than compute units: 64 rows per workgroup, half the copies of the token codes (32 x 16384 x 2048:
-//     7.0 us against 7.4 us with 32), in chunks no longer than the rows, 1024 or 2048 bytes;
-//   * else 4096-byte chunks over 4 or 8 wavefronts, 16 rows per workgroup while that gives no compute unit a second one.
-// (gemv_tokens_ok and gemv_tokens_launch are not static: the tiled GEMM's entry points in gemm_mfma.hip hand these
-// shapes over)
-int launch_gemv_tokens(const GemvArgs& a, hipStream_t st, bool fp8) {
-  if ((a.N + 31) / 32 > device_cus()) return a.K <= 1024 ? launch_gemv_tokens_shape<1, 4>(a, st, fp8) : launch_gemv_tokens_shape<2, 4>(a, st, fp8);
-  return (a.N + 15) / 16 <= device_cus() ? launch_gemv_tokens_shape<4, 1>(a, st, fp8) : launch_gemv_tokens_shape<4, 2>(a, st, fp8);
-}
-
+// (not static: the tiled GEMM's entry points in gemm_mfma.hip hand over what streams_weights says)
 int gemv_tokens_launch(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw, const void* bias,
                        int bias_dtype, const void* residual, void* y, int y_dtype, int64_t M, int64_t N, int64_t K,
                        hipStream_t st, bool fp8) {
@@ -854,7 +832,7 @@ int gemv_tokens_launch(const int8_t* xq, const float* sx, const int8_t* wq, cons
   a.K = (int)K;
   a.bias_dtype = bias_dtype;
   a.y_dtype = y_dtype;
-  return launch_gemv_tokens(a, st, fp8);
+  return K <= 1024 ? launch_gemv_tokens_shape<1>(a, st, fp8) : launch_gemv_tokens_shape<2>(a, st, fp8);
 }
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -1082,8 +1060,6 @@ static aq::GemvArgs gemv_fp8_args(const uint8_t* wq, const float* sw, const void
   return a;
 }
 
-static bool gemv_fp8_ok(int64_t K) { return (K % 256) == 0 && 16 * (K + 16) + 64 + 16 <= aq::GV_MAX_LDS; }
-
 extern "C" int aq_gemv_fp8_codes_residual(const uint8_t* xq, const float* sx, const uint8_t* wq, const float* sw,
                                           const void* bias, int bias_dtype, const void* residual, void* y, int y_dtype,
                                           int64_t M, int64_t N, int64_t K, void* stream) {
@@ -1091,8 +1067,8 @@ extern "C" int aq_gemv_fp8_codes_residual(const uint8_t* xq, const float* sx, co
   if (rc || M == 0 || N == 0) return rc;
   if (!xq || !sx) return AQ_E_NULL;
   if (aq::check_ptr16(xq) || aq::check_ptr(sx, 4)) return AQ_E_ALIGN;
-  if (!gemv_fp8_ok(K)) return aq_linear_fp8_residual(xq, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, stream);
-  aq::GemmArgs a{};
+  if (N <= (1 << 20)) return aq_linear_fp8_residual(xq, sx, wq, sw, bias, bias_dtype, residual, y, y_dtype, M, N, K, stream);
+  aq::GemmArgs a{};  // more outputs than its other tiles index
   a.A = xq;
   a.B = wq;
   a.C = y;

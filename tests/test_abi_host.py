@@ -315,8 +315,12 @@ def test_gemm_tile_choice_where_tiles_are_walked_or_k_is_cut():
     assert pick(333, 1536, 6912, res=1) == 39
     # the smallest of which 256 are enough: 16 x 16, 16 x 32, 16 x 64 (up to 16 rows; then 16 x 32 in rounds), 32 x 16, 32 x 32
     for M, N, tile in ((16, 4096, 40), (16, 4097, 41), (16, 8192, 41), (16, 8193, 43), (16, 16384, 43), (16, 16385, 41), (17, 2048, 40), (17, 2049, 41),
-                       (32, 4096, 41), (32, 4097, 34), (2100, 48, 42), (33, 1360, 40), (33, 1361, 41), (64, 4096, 34), (64, 4097, 37)):
+                       (16, 1 << 20, 41), (32, 4096, 41), (32, 4097, 34), (2100, 48, 42), (33, 1360, 40), (33, 1361, 41), (64, 4096, 34), (64, 4097, 37)):
         assert pick(M, N, 1040) == pick(M, N, 1040, fp8=1, out=f32, res=1) == tile
+    # 17 to 32 rows in whole lines of more outputs than those: weights streamed (31); no fewer rows, however long
+    for M, N, K, tile in ((32, 12288, 1024, 37), (32, 12289, 1024, 31), (17, 12289, 11008, 31), (32, 12289, 1040, 65), (16, 12289, 11008, 43),
+                          (9, 8193, 10240, 43), (8, 40000, 20480, 41), (33, 16384, 1024, 65)):
+        assert pick(M, N, K) == pick(M, N, K, fp8=1, out=f32, res=1) == tile
 
 
 def test_the_distance_between_rows_of_codes_is_one_that_their_quantiser_writes():

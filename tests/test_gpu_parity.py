@@ -707,9 +707,9 @@ def test_up_gate_gemv_with_the_activation_refuses_what_it_does_not_serve():
 @pytest.mark.parametrize("M", [17, 31, 32, 33, 48, 50, 64])
 @pytest.mark.parametrize("N,K", [(8192, 2048), (200, 256), (77, 1536), (2048, 2304), (3072, 4096), (130, 9984),
                                  (2048, 5632), (8200, 6912), (77, 11008), (40, 128), (12000, 4224), (8400, 1024),
-                                 (4200, 4224)])
+                                 (4200, 4224), (12289, 4224), (12300, 1024), (12352, 128)])
 def test_a_few_dozen_rows_same_bits_as_the_oracle(oracle, M, N, K):
-    """17..64 rows: the GEMM whose wavefronts share K while there is at most one of its 32-column tiles per compute unit; with
+    """17..64 rows: the GEMM whose wavefronts share K while there is at most one of its tiles per compute unit (12 288 outputs); with
     more, 17..32 rows of whole 128-byte lines go to the weight-streaming matrix-core kernel with 2 groups of 16 tokens,
     which walks rows of any length in chunks of 1024 or 2048 bytes (ragged last chunks, rows shorter than a chunk), and
     33..64 rows to the narrow tiles.  int32 sums and the frozen epilogue: bit for bit against the oracle, bf16 and fp32
@@ -738,14 +738,12 @@ def test_a_few_dozen_rows_same_bits_as_the_oracle(oracle, M, N, K):
     assert torch.equal(ops.linear_w8a8(xqd, sxd, wqd, swd, b.to(DEV), out_dtype=torch.float32, residual=rf), yf + rf)
 
 
-@pytest.mark.parametrize("M,K", [(12, 11008), (16, 14336), (7, 22016), (9, 10160)])
-def test_decode_rows_too_long_for_the_gemv_take_the_kernel_that_walks_k_in_chunks(oracle, M, K):
+@pytest.mark.parametrize("M,K,N", [(12, 11008, 200), (16, 14336, 200), (7, 22016, 200), (9, 10160, 200), (12, 11008, 8200)])
+def test_decode_rows_too_long_for_the_gemv(oracle, M, K, N):
     """Activation codes of 9..16 tokens fit a compute unit's LDS up to K = 10 096 (5..8 tokens: 20 208).
     Longer rows (FFN down projections of 11 008 or 14 336) must still work at decode batch sizes:
-    the decode entry points hand them on to the Linear on codes, whose weight-streaming kernel walks such
-    rows in chunks (rows that are not whole 128-byte lines would take the tiles).  Same bits as the oracle,
-    with bias and residual, through the drop-in module as well."""
-    N = 200
+    the decode entry points hand them on to the Linear on codes, whose tiles with K cut among wavefronts take
+    rows of any length.  Same bits as the oracle, with bias and residual, through the drop-in module as well."""
     _say("gemv long K", M, N, K)
     x = make_x(M, K, 41 + M).to(torch.bfloat16)
     w = make_x(N, K, 42) * 0.02
@@ -985,9 +983,9 @@ def test_linear_fp8_within_tolerance(oracle, tile, M, N, K):
 
 @pytest.mark.parametrize("M", [17, 32, 33, 50, 64])
 @pytest.mark.parametrize("N,K", [(8192, 2048), (77, 512), (3072, 1536), (200, 256), (8400, 2304), (130, 4096),
-                                 (8400, 1024), (300, 5632), (4200, 4224)])
+                                 (8400, 1024), (300, 5632), (4200, 4224), (12289, 2304), (12300, 1024)])
 def test_linear_fp8_a_few_dozen_rows(oracle, M, N, K):
-    """17..64 rows of FP8 codes: the GEMM whose wavefronts share K, or, with more 32-column tiles than compute units, the
+    """17..64 rows of FP8 codes: the GEMM whose wavefronts share K, or, with more of its tiles than compute units, the
     weight-streaming kernel for 17..32 rows (one 16x16x128 product per 128-byte line and token group, fp32 sums, chunks and
     K parts added in a fixed order) and the narrow tiles.  Against the float64 sum of the oracle's codes inside the stated
     tolerance, against the tiled GEMM on the same codes (a forced tile shape keeps it on the tiles) within the

@@ -72,7 +72,7 @@ def test_the_rule_for_tiles_of_sixteens(M, N, K, tile):
     assert (diff <= 2.0 ** -7 * want[1].float().abs() + 2 * K * 2.0 ** -24 * sums).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 300, 256), (9, 4100, 512), (12, 816, 6416), (16, 8200, 4352), (5, 16400, 272), (9, 130, 8448)])
+@pytest.mark.parametrize("M,N,K", [(1, 300, 256), (9, 4100, 512), (12, 816, 6416), (16, 8200, 4352), (5, 16400, 272), (9, 130, 8448), (12, 8200, 11008), (16, 200, 10240)])
 def test_up_to_sixteen_rows_of_codes(M, N, K):
     """FP8 rows that are cast by a launch of their own (K in whole 256-byte steps and not): against fp64 sums, with a bias and a residual."""
     g = torch.Generator().manual_seed(M + N + K)

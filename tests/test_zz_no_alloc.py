@@ -71,8 +71,8 @@ def test_no_alloc_decode_matches_the_workspace_entry_point_twice_in_a_row():
     # fp32 rows take the array at every row count; then a one-launch shape (rows quantised inside the GEMV)
     case(3, 300, 2048, torch.float32, torch.float32, True, False)
     case(4, 300, 2048, torch.bfloat16, torch.bfloat16, False, False)
-    # rows too long for the GEMV kernels' LDS (16 x 16384): row quantiser into the array, then the token-group
-    # kernel of the tiled path reads the codes from it
+    # rows too long for the GEMV kernels' LDS (16 x 16384): row quantiser into the array, then tiles with K
+    # cut among wavefronts read the codes from it
     case(16, 136, 16384, torch.bfloat16, torch.bfloat16, True, True)
     case(9, 72, 16384, torch.float32, torch.float32, False, False)
 
