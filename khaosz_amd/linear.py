@@ -160,7 +160,7 @@ _OPERATORS = {name: getattr(ops, name) for name in (
 
 class _NativeCall(Linear):
     """A quantized Linear's call: natively in one step where nothing observes it (no hooks, plain tensors), through
-    ``nn.Module.__call__`` and ``forward`` otherwise -- the same launches and bits."""
+    ``nn.Module.__call__`` and ``forward`` otherwise -- the same bits."""
 
     def __call__(self, *args, **kwargs):
         # Calls come to native code first (``serve_calls``), once a layer has been called; what it leaves comes here, and
@@ -376,15 +376,20 @@ class Fp8Linear(_NativeCall):
         if x2.size(0) <= self.DECODE_MAX_ROWS:  # decode step: the weight-streaming GEMV
             y = ops.gemv_fp8_decode(x2, wq, sw, bias, out_dtype=x.dtype, residual=residual)
         else:
-            state, rows = None, {}
+            # operators that a program has put in the place of these two are called as they always were: for all rows, on dense codes
+            own = ops.quant_tensor_fp8 is _OPERATORS["quant_tensor_fp8"] and ops.linear_fp8 is _OPERATORS["linear_fp8"]
+            state, rows, y = None, {}, None
             if x2.numel() * x2.element_size() >= ops.FP8_ONEPASS_MIN_BYTES:  # quantised in one launch
                 ops._need_gpu(x, wq)
                 state = self._quant_states.get(x.device, lambda: ops.fp8_onepass_state(x.device))
-                pitch = ops.codes_pitch(x2.size(0), n, k, True, residual is not None)
+            elif own:
+                y = ops.linear_fp8_few_rows(x2, wq, sw, bias, residual)
+            if y is None:
+                pitch = ops.codes_pitch(x2.size(0), n, k, True, residual is not None) if own else k
                 if pitch != k:
                     rows = {"pitch": pitch}
-            xq, sx = ops.quant_tensor_fp8(x2, state=state, **rows)
-            y = ops.linear_fp8(xq, sx, wq, sw, bias, out_dtype=x.dtype, residual=residual)
+                xq, sx = ops.quant_tensor_fp8(x2, state=state, **rows)
+                y = ops.linear_fp8(xq, sx, wq, sw, bias, out_dtype=x.dtype, residual=residual)
         return y if x2 is x else y.view(x.shape[:-1] + (n,))
 
 

@@ -886,3 +886,25 @@ def gemv_fp8_decode(x, wq, sw, bias=None, out_dtype=None, workspace: Optional[to
     elif r is not None:
         y.copy_(r.view(M, N))
     return y
+
+
+def linear_fp8_few_rows(x, wq, sw, bias=None, residual=None) -> Optional[torch.Tensor]:
+    """``linear_fp8`` of ``quant_tensor_fp8(x)`` in one launch, fp32 sums in an order of its own; None where two launches are the
+    faster form of the shape (``aq_linear_few_rows_ok``) or take the type, and so decide what is wrong with it."""
+    if x.dtype is not torch.bfloat16 or x.dim() != 2 or wq.dim() != 2 or wq.shape[1] != x.shape[1]:
+        return None
+    (M, K), N, lib = x.shape, wq.shape[0], _abi.load()
+    if not lib.aq_linear_few_rows_ok(_abi.AQ_BF16, 0, 1, M, N, K):
+        return None
+    _need_gpu(x, wq, sw, bias, residual)
+    if wq.dtype != torch.uint8 or sw.dtype != torch.float32 or sw.numel() != 1:
+        raise ValueError("linear_fp8_few_rows takes e4m3fn codes as uint8 and a float32 device scalar")
+    x, wq = x.contiguous(), wq.contiguous()
+    b, bdt = _bias_args(bias, N)
+    r = _residual_arg(residual, M, N, x.dtype, x.device)
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    with _OnDevice(x.device):
+        rc = lib.aq_linear_few_rows(x.data_ptr(), _abi.AQ_BF16, None, 0.0, wq.data_ptr(), 1, sw.data_ptr(), b.data_ptr() if b is not None else None,
+                                    bdt, r.data_ptr() if r is not None else None, y.data_ptr(), _abi.AQ_BF16, M, N, K, _stream(x))
+    _abi.check(rc, "aq_linear_few_rows")
+    return y

@@ -230,6 +230,55 @@ def test_what_the_native_functions_do_not_take_goes_the_general_way(rows):
             q(wide[:, :256].cpu())
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 513, 528), (40, 1024, 1024), (64, 2048, 512), (100, 300, 1040), (300, 1601, 2064)])
+def test_an_fp8_layer_gives_the_same_bits_however_it_is_called(monkeypatch, M, N, K):
+    """Rows that one launch casts and multiplies, in an order of sums of its own, and rows that take two: called natively, by its forward,
+    with a hook, compiled, with rows that are not contiguous.  Two large products cancel, so that another order shows in the result."""
+    g = torch.Generator().manual_seed(M)
+    base = torch.nn.Linear(K, N)
+    x, res = torch.randn(M, K, generator=g).to(DT).to(DEV), torch.randn(M, N, generator=g).to(DT).to(DEV)
+    with torch.no_grad():
+        base.weight[:, 0], base.weight[:, K - 1], x[:, 0], x[:, K - 1] = 2.0, -2.0, 100.0, 100.0
+    layer = Fp8Linear.from_linear(base.to(DEV).to(DT))
+    wide = torch.zeros(M, K + 16, device=DEV, dtype=DT)
+    wide[:, :K] = x
+    with torch.inference_mode():
+        for kw in ({}, {"residual": res}):
+            layer(x, **kw)
+            y, seen = _frames(lambda: layer(x, **kw))
+            assert "forward" not in seen
+            assert torch.equal(layer.forward(x, **kw), y) and torch.equal(layer(wide[:, :K], **kw), y)
+            handle = layer.register_forward_hook(lambda m, a, y: None)
+            assert torch.equal(layer(x, **kw), y)
+            handle.remove()
+            torch._dynamo.reset()
+            assert torch.equal(torch.compile(lambda x: layer(x, **kw), backend="eager")(x), y)
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 1024, 1024), (300, 160, 2064), (2100, 160, 4016)])
+def test_replaced_fp8_operators_are_called_as_ever(monkeypatch, M, N, K):
+    """With dense codes and without a keyword that they do not know."""
+    layer = Fp8Linear.from_linear(torch.nn.Linear(K, N).to(DEV).to(DT))
+    x, real, seen = torch.randn(M, K, device=DEV).to(DT), (ops.quant_tensor_fp8, ops.linear_fp8), []
+
+    def quant(x, state=None, onepass=None):
+        return real[0](x, state=state, onepass=onepass)
+
+    def linear(xq, sx, wq, sw, bias=None, out_dtype=DT, residual=None):
+        seen.append(xq.is_contiguous())
+        return real[1](xq, sx, wq, sw, bias, out_dtype=out_dtype, residual=residual)
+
+    with torch.inference_mode():
+        want = real[1](*real[0](x), layer.qweight, layer.w_scale, layer.bias)
+        monkeypatch.setattr(ops, "linear_fp8", linear)
+        assert torch.equal(layer(x), want)
+        monkeypatch.setattr(ops, "quant_tensor_fp8", quant)
+        assert torch.equal(layer(x), want)
+        monkeypatch.setattr(ops, "linear_fp8", real[1])
+        assert torch.equal(layer(x), want)
+    assert seen == [True, True]
+
+
 class _Sub(QuantLinear):
     pass
 
