@@ -239,10 +239,12 @@ int aq_linear_fp8_strided(const uint8_t *xq, int64_t ldx, const float *sx, const
 
 /* A Linear of 17 rows and more in one launch that quantises them itself (normalises them first, with gamma), for small
  * ones: aq_linear_few_rows_ok tells whether that is the faster form of a shape, for rows of x_dtype (norm and fp8: bf16, and not
- * both), and aq_linear_few_rows takes no other (AQ_E_RANGE).  The bits of aq_quant_rowwise_i8 (aq_rmsnorm_quant_rowwise_i8) +
+ * both), and aq_linear_few_rows takes no other (AQ_E_RANGE); aq_linear_few_rows_queued_ok whether it is so too in a graph or
+ * behind other launches, where the host's time for a second launch does not count.  The bits of aq_quant_rowwise_i8 (aq_rmsnorm_quant_rowwise_i8) +
  * aq_linear_w8a8_residual; fp8: the codes of aq_quant_tensor_fp8, fp32 sums in an order of its own.  wq: int8 or e4m3 codes [N, K];
  * sw: [N], or one scale for fp8.  Replaces F.linear (linear.py:21). */
 int aq_linear_few_rows_ok(int x_dtype, int norm, int fp8, int64_t M, int64_t N, int64_t K);
+int aq_linear_few_rows_queued_ok(int x_dtype, int norm, int fp8, int64_t M, int64_t N, int64_t K);
 int aq_linear_few_rows(const void *x, int x_dtype, const void *gamma, float eps, const void *wq, int fp8, const float *sw,
                        const void *bias, int bias_dtype, const void *residual, void *y, int y_dtype, int64_t M,
                        int64_t N, int64_t K, void *stream);

@@ -78,6 +78,7 @@ SYMBOLS = {
     "aq_linear_w8a8_strided": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "aq_linear_fp8_strided": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "aq_linear_few_rows_ok": (_int, [_int, _int, _int, _i64, _i64, _i64]),
+    "aq_linear_few_rows_queued_ok": (_int, [_int, _int, _int, _i64, _i64, _i64]),
     "aq_linear_few_rows": (_int, [_vp, _int, _vp, ctypes.c_float, _vp, _int, _vp, _vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "aq_prefill_attn_causal_ahead": (_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, ctypes.c_float, _i64, _i64, _i64, _i64, _i64,
                                             _vp, _int, _vp]),

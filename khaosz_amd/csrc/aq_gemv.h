@@ -99,8 +99,9 @@ constexpr int64_t GV_MAX_LDS = 160 * 1024;  // LDS of one gfx950 CU
 // rows; launch only what gemv_rows_ok admits.
 enum RowsKind { ROWS_I8, ROWS_I8_NORM, ROWS_I8_F32, ROWS_FP8 };
 bool gemv_rows_ok(RowsKind kind, int64_t M, int64_t K);
-int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st);  // a.M above 16: in tiles (gemv_rows_tiled_ok)
-bool gemv_rows_tiled_ok(RowsKind kind, int64_t M, int64_t N, int64_t K);
+int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st);  // a.M above 16: in tiles (gemv_rows_tiled)
+enum Tiling { TILED_NOT, TILED, TILED_ALONE };  // ALONE: the faster form only where the host's time for a launch counts
+Tiling gemv_rows_tiled(RowsKind kind, int64_t M, int64_t N, int64_t K);
 int launch_gemv_rows_swiglu(const GemvArgs& a, hipStream_t st);
 int launch_gemv_rows_attn(const GemvArgs& a, hipStream_t st);  // rows from a.parts; M <= 8, K <= 2048
 

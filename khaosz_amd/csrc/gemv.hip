@@ -1262,10 +1262,18 @@ extern "C" int aq_gemv_w8a8_decode(const void* x, int x_dtype, const int8_t* wq,
 
 // ---------------------------------------------------------------------------
 // 17 rows and more, quantised in the launch that multiplies them: the decode kernel on tiles of up to 16 rows (gemv_rows.hip).
+static aq::Tiling few_rows(int x_dtype, int norm, int fp8, int64_t M, int64_t N, int64_t K) {
+  if ((x_dtype != AQ_F32 && x_dtype != AQ_BF16) || M <= 16 || N < 1 || K < 1 || K % 16) return aq::TILED_NOT;
+  if ((fp8 || norm) && (x_dtype != AQ_BF16 || (fp8 && norm))) return aq::TILED_NOT;
+  return aq::gemv_rows_tiled(fp8 ? aq::ROWS_FP8 : fused_kind(norm != 0, x_dtype == AQ_BF16), M, N, K);
+}
+
 extern "C" int aq_linear_few_rows_ok(int x_dtype, int norm, int fp8, int64_t M, int64_t N, int64_t K) {
-  if ((x_dtype != AQ_F32 && x_dtype != AQ_BF16) || M <= 16 || N < 1 || K < 1 || K % 16) return 0;
-  if ((fp8 || norm) && (x_dtype != AQ_BF16 || (fp8 && norm))) return 0;
-  return aq::gemv_rows_tiled_ok(fp8 ? aq::ROWS_FP8 : fused_kind(norm != 0, x_dtype == AQ_BF16), M, N, K) ? 1 : 0;
+  return few_rows(x_dtype, norm, fp8, M, N, K) != aq::TILED_NOT;
+}
+
+extern "C" int aq_linear_few_rows_queued_ok(int x_dtype, int norm, int fp8, int64_t M, int64_t N, int64_t K) {
+  return few_rows(x_dtype, norm, fp8, M, N, K) == aq::TILED;
 }
 
 extern "C" int aq_linear_few_rows(const void* x, int x_dtype, const void* gamma, float eps, const void* wq, int fp8, const float* sw,

@@ -537,11 +537,16 @@ static bool rounds_merge(const GemvArgs& a, bool norm) {
 // length class, whose vectors are requested whether the row has them or not):
 //   tiles      start + rounds over the compute units x (row x tile rows x length + weight x weight rows x K + all x M x K)
 //   launches   two[0] + two[1] K + two[2] M N K / 10^6 + (more than one tile of 32 x 32 per unit: two[3]) + two[4] N K / 10^4, FP8 + 1.5 M K / 65536
-// From a graph the choice would be best with the line where the tiles are 5 % ahead by that: one size in three, at 0.84 of the time in the mean; 0.7 % from
-// the faster way in the mean (1 % at 10 % ahead, 0.8 % at level).  A call that is not captured pays 2.4 us of the host's time for a launch, 7.5 us in all for
-// two: tiles of less than that are taken up to 5 % behind.  us from a graph, launches -> tiles, weights in the last-level cache | from HBM: bf16 32 x 2048 ->
-// 2048 5.7 -> 4.8 | 6.7 -> 5.1, 64 x 1024 -> 3072 6.1 -> 4.7 | 6.9 -> 5.0, 32 x 512 -> 8192 5.5 -> 4.6 | 6.4 -> 4.8, fp32 64 x 512 -> 2048 5.2 -> 4.2 | 5.8 -> 4.6; furthest off
-// fp32 64 x 2048 -> 2048 6.5 -> 7.5 | 7.3 -> 7.4 (not captured 8.1 -> 7.1); FP8 19 x 720 -> 6000, not captured, 8.9 -> 6.7.
+// us from a graph, launches -> tiles, weights in the last-level cache | from HBM: bf16 32 x 2048 -> 2048 5.7 -> 4.8 | 6.7 -> 5.1, 64 x 1024 -> 3072 6.1 -> 4.7 |
+// 6.9 -> 5.0, 32 x 512 -> 8192 5.5 -> 4.6 | 6.4 -> 4.8, fp32 64 x 512 -> 2048 5.2 -> 4.2 | 5.8 -> 4.6.
+//
+// A call on its own pays 2.4 us of the host's time for a launch, 8 us in all for two: tiles of less than that (7.5) are taken up to 5 % behind (TILED_ALONE):
+// fp32 64 x 2048 -> 2048 8.1 -> 7.1, int8 181 x 1360 -> 416 8.4 -> 6.0, FP8 19 x 720 -> 6000 8.9 -> 6.7.  In a graph, or among a block's launches, the host's time is
+// not what counts, and there the tiles have to be ahead by 5 %, fp32 rows, whose cost the fit misses by most, by 8 % (TILED).  1380 sizes drawn from 17..200 rows, the
+// times of both from a graph, cache and HBM in the mean: at the line for a call on its own int8 rows are slower than by two launches by more than 3 % at 4 sizes of 220
+// (at worst 1.25 | 1.26: 125 x 1216 -> 1824), with the norm at 3 of 220 (1.33 | 1.21), fp32 rows at 16 of 720 (1.25 | 1.19; 64 x 2048 -> 2048 6.4 -> 6.9 | 8.1 -> 7.8); at these none,
+// none and one.  FP8, whose two launches are three where the tensor is not small, at none of 220 with either (1.05 | 1.03), and so its line, on which the order of its
+// sums depends, is one for all calls.
 struct TiledCost {
   double start, row, weight, all, two[5];
 };
@@ -568,16 +573,17 @@ static Tiled tiled_best(RowsKind kind, int64_t M, int64_t N, int64_t K) {
   }
   return best;
 }
-bool gemv_rows_tiled_ok(RowsKind kind, int64_t M, int64_t N, int64_t K) {
+Tiling gemv_rows_tiled(RowsKind kind, int64_t M, int64_t N, int64_t K) {
   // Tiles of more outputs than 80 to a compute unit never gained (64 x 512 -> 8192: 6.3 | 6.6), nor longer bf16 rows than 4096 (FP8: 2048).
   const int64_t most = kind == ROWS_I8_NORM || kind == ROWS_FP8 ? 2048 : kind == ROWS_I8_F32 ? GX_MAX_K : 4096;
-  if (M <= 16 || (M + 15) / 16 * N > 80 * device_cus() || K > most) return false;
+  if (M <= 16 || (M + 15) / 16 * N > 80 * device_cus() || K > most) return TILED_NOT;
   const double* two = tiled_cost(kind).two;
   const double k = (double)K / 1024, nk = (double)N * k;
   const bool rounds = (M + 31) / 32 * ((N + 31) / 32) > device_cus();
   const double cast = kind == ROWS_FP8 ? 1.5 * (double)(M * K < 98304 ? M * K : 98304) / 65536 : 0;  // by the tensor's size, up to where it takes two launches
   const double us = tiled_best(kind, M, N, K).us, by_two = two[0] + cast + two[1] * k + two[2] * M * nk / 1e6 + (rounds ? two[3] : 0) + two[4] * nk / 1e4;
-  return us < (us < 7.5 ? 1.05 : 0.95) * by_two;
+  const double ahead = kind == ROWS_FP8 ? (us < 7.5 ? 1.05 : 0.95) : kind == ROWS_I8_F32 ? 0.92 : 0.95;
+  return us < ahead * by_two ? TILED : us < (us < 7.5 ? 1.05 : 0.95) * by_two ? TILED_ALONE : TILED_NOT;
 }
 
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {

@@ -48,6 +48,7 @@ namespace {
   X(aq_linear_w8a8_strided)                                                                                      \
   X(aq_linear_fp8_strided)                                                                                       \
   X(aq_linear_few_rows_ok)                                                                                       \
+  X(aq_linear_few_rows_queued_ok)                                                                                \
   X(aq_linear_few_rows)                                                                                          \
   X(aq_gemv_w8a8_decode_residual)                                                                                \
   X(aq_gemv_w8a8_decode_rmsnorm)                                                                                 \
@@ -121,6 +122,11 @@ struct Call {  // the device and stream of one call
     return dev == c10::hip::current_device();
   }
   void current_stream() { stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream(); }
+  bool captured() const {  // (the null stream cannot be)
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (stream && hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) (void)hipGetLastError();
+    return status != hipStreamCaptureStatusNone;
+  }
   Tensor empty(at::IntArrayRef size, ScalarType type) const {
     return at::detail::empty_cuda(size, type, c10::Device(c10::kCUDA, static_cast<c10::DeviceIndex>(dev)), std::nullopt);
   }
@@ -630,7 +636,8 @@ PyObject* linear_native(PyObject* layer, PyObject* const* args, Py_ssize_t nargs
   const int64_t room = codes + (!few ? (fp8 ? 256 + AQ_FP8_AMAX_WS_BYTES : 4 * r.M) : 0);
   void* yp = y.mutable_data_ptr();
   // a launch that quantises its rows itself touches no workspace: an allocation is 0.4 us of a 5 us call
-  const bool tiles = !few && lib.aq_linear_few_rows_ok(r.code, gain != nullptr, fp8, r.M, N, r.K);
+  const bool tiles = !few && lib.aq_linear_few_rows_ok(r.code, gain != nullptr, fp8, r.M, N, r.K) &&
+                     (!c.captured() || lib.aq_linear_few_rows_queued_ok(r.code, gain != nullptr, fp8, r.M, N, r.K));
   const bool alone = tiles || (few && (fp8 ? lib.aq_gemv_fp8_decode_one_launch(r.code, r.M, r.K)
                                  : lib.aq_gemv_w8a8_decode_one_launch(r.code, gain != nullptr, r.M, N, r.K)));
   Tensor ws;
@@ -916,7 +923,7 @@ int Block::queue(const void* in, void* out, char* base, const char** what) const
       return lib.aq_gemv_w8a8_decode_rmsnorm(x, AQ_BF16, g.p, g.eps, p.w, p.s, p.b.p, p.b.code, nullptr, y, AQ_BF16, M, p.N, p.K, room,
                                              lib.aq_gemv_w8a8_workspace_bytes(M, p.K), c.stream);
     }
-    if (lib.aq_linear_few_rows_ok(AQ_BF16, 1, 0, M, p.N, p.K)) {
+    if (lib.aq_linear_few_rows_queued_ok(AQ_BF16, 1, 0, M, p.N, p.K)) {
       *what = "aq_linear_few_rows";
       return lib.aq_linear_few_rows(x, AQ_BF16, g.p, g.eps, p.w, 0, p.s, p.b.p, p.b.code, nullptr, y, AQ_BF16, M, p.N, p.K, c.stream);
     }
@@ -934,7 +941,7 @@ int Block::queue(const void* in, void* out, char* base, const char** what) const
       return lib.aq_gemv_w8a8_decode_residual(x, AQ_BF16, p.w, p.s, p.b.p, p.b.code, res, y, AQ_BF16, M, p.N, p.K, room,
                                               lib.aq_gemv_w8a8_workspace_bytes(M, p.K), c.stream);
     }
-    if (lib.aq_linear_few_rows_ok(AQ_BF16, 0, 0, M, p.N, p.K)) {
+    if (lib.aq_linear_few_rows_queued_ok(AQ_BF16, 0, 0, M, p.N, p.K)) {
       *what = "aq_linear_few_rows";
       return lib.aq_linear_few_rows(x, AQ_BF16, nullptr, 0.f, p.w, 0, p.s, p.b.p, p.b.code, res, y, AQ_BF16, M, p.N, p.K, c.stream);
     }

@@ -340,6 +340,24 @@ def test_the_distance_between_rows_of_codes_is_one_that_their_quantiser_writes()
         assert pitch(M, 2048, 1040) == 1040
 
 
+def test_one_launch_for_few_rows_where_the_host_pays_for_launches_and_in_a_graph():
+    """Taken for less in a call on its own (int8 rows), where a launch saved is the host's time; FP8, whose bits depend on it, for the same."""
+    lib = _abi.load()
+    f32, bf16 = _abi.AQ_F32, _abi.AQ_BF16
+    both = lambda dt, norm, fp8, M, N, K: (lib.aq_linear_few_rows_ok(dt, norm, fp8, M, N, K), lib.aq_linear_few_rows_queued_ok(dt, norm, fp8, M, N, K))
+    assert both(f32, 0, 0, 64, 2048, 2048) == both(bf16, 0, 0, 125, 1824, 1216) == both(bf16, 1, 0, 93, 1184, 1072) == (1, 0)
+    assert both(f32, 0, 0, 64, 2048, 512) == both(bf16, 0, 0, 32, 2048, 2048) == both(bf16, 1, 0, 32, 1024, 1024) == (1, 1)
+    assert both(f32, 0, 0, 64, 2048, 4096) == both(bf16, 0, 0, 16, 512, 512) == both(bf16, 0, 0, 64, 8192, 2048) == (0, 0)
+    for M in range(17, 200, 7):
+        for N in (300, 1100, 2048, 5000):
+            for K in range(16, 2064, 80):
+                ok, queued = both(bf16, 0, 1, M, N, K)
+                assert ok == queued
+                for case in ((f32, 0, 0, M, N, K), (bf16, 0, 0, M, N, K), (bf16, 1, 0, M, N, K)):
+                    ok, queued = both(*case)
+                    assert ok >= queued
+
+
 def test_quant_tensor_fp8_refuses_a_workspace_smaller_than_its_slots():
     """aq_quant_tensor_fp8 writes AQ_FP8_AMAX_WS_BYTES of partial maxima: a smaller workspace is refused before
     anything is launched (argument checks only: runs without a GPU)."""

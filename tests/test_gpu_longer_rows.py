@@ -1,5 +1,7 @@
 """Rows at the ends of the classes by which a launch takes them, against the CPU oracle: the row quantiser's (csrc/quant.hip), and the
 tiles of up to 16 rows of a launch that quantises more than 16 itself (csrc/gemv_rows.hip)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -115,6 +117,34 @@ def test_shapes_that_take_two_launches_are_refused():
     p = x.data_ptr()
     assert lib.aq_linear_few_rows(p, _abi.AQ_BF16, None, 0.0, p, 0, p, None, 0, None, p, _abi.AQ_BF16, 64, 8192, 2048, None) == -6  # AQ_E_RANGE
     assert lib.aq_linear_few_rows(p, _abi.AQ_BF16, p, -1.0, p, 0, p, None, 0, None, p, _abi.AQ_BF16, 32, 512, 512, None) == -2  # AQ_E_SHAPE
+
+
+def _kernel_launches(graph):
+    hip = ctypes.CDLL(next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l))
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("M,N,K,dtype,norm,launches", [(64, 2048, 2048, F32, False, 2), (125, 1824, 1216, BF16, False, 2), (93, 1184, 1072, BF16, True, 2),
+                                                       (64, 2048, 512, F32, False, 1), (32, 2048, 2048, BF16, False, 1), (32, 1024, 1024, BF16, True, 1)])
+def test_a_captured_layer_takes_the_launches_that_are_faster_in_a_graph(M, N, K, dtype, norm, launches):
+    """Where one launch only saves the host's time for a second (the first three), a graph has the two; the same bits on every replay."""
+    layer = QuantLinear.from_linear(torch.nn.Linear(K, N).to(DEV).to(dtype))
+    kw = {"norm": (torch.ones(K, device=DEV, dtype=dtype), 1e-5)} if norm else {}
+    x = _rows(M, K, M).to(dtype).to(DEV)
+    with torch.inference_mode():
+        for _ in range(2):
+            layer(x, **kw)
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            y = layer(x, **kw)
+        assert _kernel_launches(graph) == launches
+        for i in range(3):
+            x.copy_(_rows(M, K, 100 + i).to(dtype))
+            want = layer(x, **kw)
+            graph.replay()
+            assert torch.equal(y, want)
 
 
 # vectors of 16 bytes around the sizes that one launch covers with 1, 4, 8 and 12 (fp32: 16) per thread, and beyond
