@@ -921,7 +921,8 @@ __global__ __launch_bounds__(S::NTHREADS) void gemm_kernel(GemmArgs p) {
 // 33..2048 rows against N = 1024..16384 and K = 1024..5632, where the rule picks the fastest shape or one within
 // 6 % of it.  The small tiles are for launches of a few rounds only.
 enum TileKind {
-  TILE_AUTO = 0, TILE_STREAMS = 31 /* no tile: gemv.hip's */, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128, TILE_PAIR = 129, TILE_WIDE = 192,
+  TILE_AUTO = 0, TILE_STREAMS = 31 /* no tile: gemv.hip's */, TILE_N32 = 32, TILE_M64N32 = 33, TILE_N64 = 64, TILE_M64N64 = 65, TILE_SMALL = 128,
+  TILE_PAIR = 129, TILE_WIDE = 192,
   TILE_LARGE = 256, TILE_TALL = 257, TILE_HUGE = 512, TILE_HUGE8 = 513, TILE_WALK = 258  // and SlicesTile's
 };
 #ifdef AQ_LAB
@@ -1080,10 +1081,11 @@ static int check_gemm(const void* A, const void* B, const void* C, int64_t M, in
   return AQ_OK;
 }
 
-// 17..32 rows, in whole lines, of more outputs than tiles cut among wavefronts serve: the weight-streaming kernel takes them.  Not 16 rows and fewer, however long: us, weights in the last-level cache | from HBM, the weight-streaming
-// kernel -> tiles of 16 x 64 or 16 x 32: 16 x 11008 -> 8200 29.5 -> 20.6 | 29.2 -> 26.5, -> 12288 35.0 -> 26.6 | 34.8 -> 35.6, -> 20000 62.8 -> 36.8 | 63.3 ->
-// 49.5, -> 32000 73.4 -> 65.9 | 74.7 -> 67.8; 8 x 20480 -> 8200 50.6 -> 29.1 | 49.7 -> 42.6; of 119 sizes the slowest 16 x 14336 -> 32000 74.3 -> 79.6 and,
-// from HBM, 9 x 16384 -> 16384 49.7 -> 53.7.
+// 17..32 rows, in whole lines, of more outputs than tiles cut among wavefronts serve: the weight-streaming kernel takes them.  Not 16 rows
+// and fewer, however long: us, weights in the last-level cache | from HBM, the weight-streaming kernel -> tiles of 16 x 64 or 16 x 32: 16 x
+// 11008 -> 8200 29.5 -> 20.6 | 29.2 -> 26.5, -> 12288 35.0 -> 26.6 | 34.8 -> 35.6, -> 20000 62.8 -> 36.8 | 63.3 -> 49.5, -> 32000 73.4 -> 65.9 |
+// 74.7 -> 67.8; 8 x 20480 -> 8200 50.6 -> 29.1 | 49.7 -> 42.6; of 119 sizes the slowest 16 x 14336 -> 32000 74.3 -> 79.6 and, from HBM, 9 x
+// 16384 -> 16384 49.7 -> 53.7.
 static bool streams_weights(int64_t M, int64_t N, int64_t K, int64_t cus) {
   return M > 16 && M <= 32 && K % 128 == 0 && !gemm_slices_tile(M, N, K, cus);
 }

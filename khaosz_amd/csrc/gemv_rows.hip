@@ -524,12 +524,6 @@ static bool rounds_merge(const GemvArgs& a, bool norm) {
   return a.K <= 2048 && a.N > (a.K > 1024 ? 64 : 128) * device_cus() && !(a.M > 8 && (norm || a.K <= 1024));
 }
 
-// Two exceptions, 2200 sizes with weights from HBM:
-// * 1 to 4 bf16 rows of 3073 to 4096, where 64-row workgroups would be a round of which at most 5/8 of the units have one: five rounds
-//   of 8-row workgroups overlap enough.  us, 64 -> 8: FP8 2 x 3824 -> 8896 14.6 -> 12.7, 1 x 3440 -> 8864 13.4 -> 12.0, int8 1 x 3440 -> 10128 12.9
-//   -> 11.4; not 1 x 2864 -> 10160 (11.2 | 11.5), nor with six rounds (FP8 3 x 3504 -> 11000 13.1 | 14.0).
-// * 1 to 4 fp32 rows of 1025 to 2048, whose rounds overlap the less the larger they are: 16 at most, 1 x 1424 -> 4128 4.7 -> 4.2 (in the
-//   mean 1.6 % from the best of the four, so 0.8 %).
 // More than 16 rows: tiles of 9..16 or of up to 8 rows, each with its own workgroups over the weight rows.  Every tile reads the
 // weights and every workgroup rounds its tile's rows again, so it is the faster form while tiles x outputs x row length is small:
 // one launch then stands for the quantiser's and the GEMM's (FP8: the maximum's, the cast's and the GEMM's), 3.3 to 5 us of which are
@@ -540,13 +534,13 @@ static bool rounds_merge(const GemvArgs& a, bool norm) {
 // us from a graph, launches -> tiles, weights in the last-level cache | from HBM: bf16 32 x 2048 -> 2048 5.7 -> 4.8 | 6.7 -> 5.1, 64 x 1024 -> 3072 6.1 -> 4.7 |
 // 6.9 -> 5.0, 32 x 512 -> 8192 5.5 -> 4.6 | 6.4 -> 4.8, fp32 64 x 512 -> 2048 5.2 -> 4.2 | 5.8 -> 4.6.
 //
-// A call on its own pays 2.4 us of the host's time for a launch, 8 us in all for two: tiles of less than that (7.5) are taken up to 5 % behind (TILED_ALONE):
-// fp32 64 x 2048 -> 2048 8.1 -> 7.1, int8 181 x 1360 -> 416 8.4 -> 6.0, FP8 19 x 720 -> 6000 8.9 -> 6.7.  In a graph, or among a block's launches, the host's time is
-// not what counts, and there the tiles have to be ahead by 5 %, fp32 rows, whose cost the fit misses by most, by 8 % (TILED).  1380 sizes drawn from 17..200 rows, the
-// times of both from a graph, cache and HBM in the mean: at the line for a call on its own int8 rows are slower than by two launches by more than 3 % at 4 sizes of 220
-// (at worst 1.25 | 1.26: 125 x 1216 -> 1824), with the norm at 3 of 220 (1.33 | 1.21), fp32 rows at 16 of 720 (1.25 | 1.19; 64 x 2048 -> 2048 6.4 -> 6.9 | 8.1 -> 7.8); at these none,
-// none and one.  FP8, whose two launches are three where the tensor is not small, at none of 220 with either (1.05 | 1.03), and so its line, on which the order of its
-// sums depends, is one for all calls.
+// A call on its own pays 2.4 us of the host's time for a launch, 8 us in all for two: tiles of less than that (7.5) are taken up to 5 %
+// behind (TILED_ALONE): fp32 64 x 2048 -> 2048 8.1 -> 7.1, int8 181 x 1360 -> 416 8.4 -> 6.0, FP8 19 x 720 -> 6000 8.9 -> 6.7.  In a graph, or
+// among a block's launches, the host's time is not what counts, and there the tiles have to be ahead by 5 %, fp32 rows, whose cost the fit
+// misses by most, by 8 % (TILED).  1380 sizes drawn from 17..200 rows, both ways from a graph, slower by more than 3 % with the tiles, cache and
+// HBM together: by the line for a call on its own int8 rows at 4 of 220 (at worst 1.25 | 1.26: 125 x 1216 -> 1824), with the norm 3 of 220 (1.33 |
+// 1.21), fp32 rows 16 of 720 (1.25 | 1.19; 64 x 2048 -> 2048 6.4 -> 6.9 | 8.1 -> 7.8); by these none, none and one (1.05).  FP8 at none of 220 (at
+// worst 1.05 | 1.03), and so its line, on which the order of its sums depends, is one for all calls.
 struct TiledCost {
   double start, row, weight, all, two[5];
 };
@@ -586,6 +580,12 @@ Tiling gemv_rows_tiled(RowsKind kind, int64_t M, int64_t N, int64_t K) {
   return us < ahead * by_two ? TILED : us < (us < 7.5 ? 1.05 : 0.95) * by_two ? TILED_ALONE : TILED_NOT;
 }
 
+// Two exceptions, 2200 sizes with weights from HBM:
+// * 1 to 4 bf16 rows of 3073 to 4096, where 64-row workgroups would be a round of which at most 5/8 of the units have one: five rounds
+//   of 8-row workgroups overlap enough.  us, 64 -> 8: FP8 2 x 3824 -> 8896 14.6 -> 12.7, 1 x 3440 -> 8864 13.4 -> 12.0, int8 1 x 3440 -> 10128 12.9
+//   -> 11.4; not 1 x 2864 -> 10160 (11.2 | 11.5), nor with six rounds (FP8 3 x 3504 -> 11000 13.1 | 14.0).
+// * 1 to 4 fp32 rows of 1025 to 2048, whose rounds overlap the less the larger they are: 16 at most, 1 x 1424 -> 4128 4.7 -> 4.2 (in the
+//   mean 1.6 % from the best of the four, so 0.8 %).
 int launch_gemv_rows(const GemvArgs& a, RowsKind kind, hipStream_t st) {
   const bool few = a.M <= 4, f32 = kind == ROWS_I8_F32, norm = kind == ROWS_I8_NORM;
   if (a.M > 16) {

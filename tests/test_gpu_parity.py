@@ -1022,12 +1022,10 @@ def test_linear_fp8_a_few_dozen_rows(oracle, M, N, K):
 @pytest.mark.parametrize("M", [1, 3, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [(8192, 2048), (77, 512), (11264, 1024), (300, 4096), (130, 1040), (200, 11008)])
 def test_gemv_fp8_decode_within_tolerance(oracle, M, N, K):
-    """The FP8 Linear at decode sizes: (8192, 2048), (77, 512) and (11264, 1024) cast their bf16 rows inside the
-    GEMV kernel (32- and 64-row workgroups, a ragged single workgroup); (300, 4096) goes through the workspace
-    (quantiser + GEMV on codes); (130, 1040) is handed to the tiled GEMM; rows of 11008 codes are too long for the
-    GEMV's LDS and go to the Linear on codes (its weight-streaming kernel from 9 rows on).  All against the float64 sum of the
-    oracle's codes, and the fused cast against the codes path (a wrong code would move an output by far more
-    than a change of summation order)."""
+    """The FP8 Linear at decode sizes: rows of up to 4096 are cast inside the GEMV kernel (32- and 64-row workgroups, a
+    ragged single workgroup), rows of 11008 by a launch of their own in front of tiles with K cut among wavefronts.  All against
+    the float64 sum of the oracle's codes, and the fused cast against the codes path and a tile of the other GEMM (a wrong code
+    would move an output by far more than a change of summation order)."""
     _say("gemv_fp8", M, N, K)
     g = torch.Generator().manual_seed(M * 13 + N)
     x = (torch.randn(M, K, generator=g) * (0.2 + 3 * torch.rand(M, 1, generator=g))).to(torch.bfloat16)
@@ -1042,13 +1040,15 @@ def test_gemv_fp8_decode_within_tolerance(oracle, M, N, K):
     assert np.max(np.abs(to_np(y32) - exact)) <= 1e-3 * rms
     yb = ops.gemv_fp8_decode(x.to(DEV), wqd, swd, bias.to(DEV), out_dtype=torch.bfloat16)
     np.testing.assert_allclose(to_np(yb.float()), exact, rtol=1e-2, atol=1e-2 * rms)   # stated tolerance
-    # the library's own quantiser gives the oracle's codes; the GEMV on them agrees with the fused launch
+    # the library's own quantiser gives the oracle's codes; the tiles with K cut on them agree with the fused launch
     xqd, sxd = ops.quant_tensor_fp8(x.to(DEV))
     assert np.array_equal(to_np(xqd), xq) and float(sxd.item()) == float(sx)
     yc = ops.gemv_fp8_codes(xqd, sxd, wqd, swd, bias.to(DEV), out_dtype=torch.float32)
     assert np.max(np.abs(to_np(yc) - to_np(y32))) <= 2e-5 * rms
-    # and with the tiled GEMM on the same codes
-    yg = ops.linear_fp8(xqd, sxd, wqd, swd, bias.to(DEV), out_dtype=torch.float32)
+    # and with a tile whose wavefronts share the K steps, on the same codes
+    with _abi.lab_library() as lab:
+        assert lab.aq_lab_set_gemm_tile(33) == 0
+        yg = ops.linear_fp8(xqd, sxd, wqd, swd, bias.to(DEV), out_dtype=torch.float32)
     assert np.max(np.abs(to_np(yg) - to_np(y32))) <= 2e-5 * rms
     r = torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV)
     assert torch.equal(ops.gemv_fp8_decode(x.to(DEV), wqd, swd, bias.to(DEV), out_dtype=torch.bfloat16, residual=r), yb + r)
@@ -1061,7 +1061,7 @@ def test_fp8_linear_module_decode_rows_take_the_gemv_and_match_the_prefill_path(
     f = Fp8Linear.from_linear(lin.to(DEV))
     x = torch.randn(40, 2048, device=DEV, dtype=torch.bfloat16)
     with torch.inference_mode():
-        big = f(x)                                   # 40 rows: quantiser + tiled GEMM, one scale for all 40
+        big = f(x)                                   # 40 rows: quantiser + GEMM, one scale for all 40
         small = f(x[:16])                            # 16 rows: the GEMV, one scale for these 16
     ref = torch.nn.functional.linear(x.float(), lin.weight)
     assert ((big.float() - ref).norm() / ref.norm()).item() < 0.08
