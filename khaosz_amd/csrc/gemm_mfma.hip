@@ -1213,10 +1213,18 @@ extern "C" int aq_linear_fp8_strided(const uint8_t* xq, int64_t ldx, const float
 // 256 x 256 FP8 tile serves, whose 64-byte steps halve no line (with a residual it does not: 4864 x 3264 -> 8640 148.7 -> 132.8, 8192 x 8128 -> 8192 583 -> 486),
 // nor the weight-streaming kernel, which takes rows as they are.  Nor what the quantisers do not write in rows: more than 2^31 vectors of 16 bytes,
 // of which fp32 rows have K / 4.  Nor where the gaps alone take the codes past the 31-bit offsets of the kernel that walks tiles.
+// Nor short rows of that kernel: in some processes, on most cards, it reads codes that have just been written at a half to three quarters of its
+// rate if they begin on lines, with no more requests, misses or bytes than in others.  us of quantiser and GEMM, K apart -> whole lines, where
+// that happens | where it does not: 6181 x 720 -> 1096 18.8 -> 22.9 | 18.8 -> 17.9, 6020 x 880 -> 4400 47 -> 62 | 45 -> 40.5, 7182 x 1088 -> 4192
+// 52 -> 74.  1018 sizes of it by K, in the mean (slowest): 512 to 1151 0.999 (1.40) | 0.955 (1.09), to 1663 0.961 (1.16) | 0.928, to 2047 0.957 (1.20) |
+// 0.916, from 2048 on 0.901 (1.02) | 0.897.  The other tiles gain where it happens too (132 sizes, 0.947, slowest 1.01).
 extern "C" int64_t aq_linear_codes_pitch(int fp8, int residual, int64_t M, int64_t N, int64_t K) {
   if (M <= 16 || N < 1 || K < 1 || K % 16 || K % 128 == 0 || K > (1 << 22) - 128 || M > (1 << 30) || M * K / 4 > (int64_t)0x7fffffff) return K;
   const int64_t pitch = (K + 127) / 128 * 128, reach = aq::OOB_OFFSET;
   if (aq::streams_weights(M, N, K, aq::device_cus()) || (M * pitch > reach && M * K <= reach)) return K;
+  static const char some = 0;
   aq::GemmArgs a = aq::make_args(nullptr, nullptr, nullptr, M, N, K);
-  return fp8 && !residual && aq::huge_fp8_ok(a, aq::device_cus()) ? K : pitch;
+  a.res = residual ? &some : nullptr;  // only whether there is one
+  const int tile = aq::choose_tile(a, fp8 != 0, aq::OUT_BF16, aq::device_cus());
+  return tile == aq::TILE_HUGE || ((tile == aq::TILE_WALK || tile == aq::TILE_WIDE) && K < 2048) ? K : pitch;
 }

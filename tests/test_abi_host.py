@@ -338,6 +338,13 @@ def test_the_distance_between_rows_of_codes_is_one_that_their_quantiser_writes()
     assert pitch(4864, 8640, 3264) == 3264 and pitch(4864, 8640, 3264, res=1) == 3328 and pitch(4864, 8640, 3264, fp8=0) == 3328
     for M in (0, -1, 1 << 31):
         assert pitch(M, 2048, 1040) == 1040
+    # walked tiles (258, 192) read short rows as they are; the other tiles do not
+    for M, N, K in ((6181, 1096, 720), (6020, 4400, 880), (7182, 4192, 1088), (8000, 8186, 1200), (4097, 2048, 2032)):
+        assert _abi.load_lab().aq_lab_choose_gemm_tile(M, N, K, 0, _abi.AQ_BF16, 0, 256) in (258, 192)
+        for fp8 in (0, 1):
+            assert pitch(M, N, K, fp8) == pitch(M, N, K, fp8, res=1) == K
+    for fp8 in (0, 1):
+        assert pitch(4097, 2048, 2064, fp8) == 2176 and pitch(6181, 1095, 720, fp8) == 768 and pitch(700, 1600, 1040, fp8) == 1152
 
 
 def test_one_launch_for_few_rows_where_the_host_pays_for_launches_and_in_a_graph():
